@@ -1,14 +1,28 @@
 // out[M, N] = x[M, K] . W[N, K]^T (+ bias) with 32-bit operands on the matrix units: the product of
-// the float32 mode.  v_mfma_f32_32x32x2_f32 multiplies 32-bit numbers and accumulates in 32-bit
-// (no reduced-precision matrix mode), about ten times the rate of the vector units' multiply-adds.
+// the float32 mode.  v_mfma_f32_32x32x2_f32 and v_mfma_f32_16x16x4_f32 multiply 32-bit numbers and
+// accumulate in 32-bit (no reduced-precision matrix mode), about ten times the rate of the vector
+// units' multiply-adds.  Both are chains of fused multiply-adds in the order of k, bit for bit.
 //
-// A block of four waves owns a 64 x 64 tile of the output, a wave a 32 x 32 quarter.  K goes in steps
-// of 16 through shared memory; the next step's operands are asked for from global memory before
-// the current step is computed.  For a step, lane (h, r), h = lane / 32, r = lane % 32, reads
-// x[row r][8 h .. 8 h + 8] and W[row r][8 h .. 8 h + 8] as two 16-byte pieces each, and the j-th
-// MFMA of the step takes element j of both (which k stands at which place of an MFMA's sum does
-// not matter, as long as both operands have it at the same).  Every output is summed in the same
-// order whatever M is, so a row's result does not depend on what else is in the batch.
+// Every output is summed in one order whatever M is and whichever kernel takes the rows, so a row's
+// result does not depend on what else is in the batch.  K is cut into 16 chunks of chunk_len(K) (a
+// multiple of 16; the last ones may be short or empty).  Inside a chunk one chain runs over steps of 16,
+// in a step over k = 0, 4, 8, 12, 1, 5, 9, 13, 2, ... (which is what lets a lane bring four neighbouring
+// k by one load and use them in four instructions).  The chunks of a quarter are added in order, then
+// the quarters in order.
+//
+// Two kernels share that order:
+//   few rows: a block owns 16 outputs (or 32) and has a wave per chunk, so that the weights are asked for
+//     by 16 waves a block at once and the sums meet in shared memory.  Bound by the stream of the weights and
+//     a kernel's fixed cost.  Two rows (as 64 x 64 tiles before): 4096 x 1024 7.1 us (42), 6144 x 1024 10.6 (42),
+//     1024 x 3072 11.6 (117), 151936 x 1024 137 (215; 4.5 TB/s).  At most 64 registers a lane, so that two
+//     blocks of 16 waves fit a compute unit (four steps at a time instead of two: 10.0, 17.7, 14.5 and 294 us).
+//   more rows: tiles of 64 x 64, a wave a 32 x 32 quarter, K in steps of 16 through two buffers of shared
+//     memory.  With fewer than TILES_FOR_FOUR tiles four groups of four waves share a tile's K, one
+//     quarter each (a compute unit with one tile would else have a wave a SIMD and wait for every step's
+//     loads).
+// Loads stand under no condition where K is a multiple of 16 and both operands are aligned: rows beyond
+// the matrix read the last row again and are not stored.  (Behind a conditional load the compiler waits
+// for all loads in flight.)
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(4))) float floatx4;
@@ -17,85 +31,236 @@ typedef __attribute__((ext_vector_type(16))) float floatx16;
 #define FT 64         // tile rows and columns
 #define FK 16         // k step
 #define FROW (FK + 4) // floats of a staged row: padded, so that the 32 rows a wave reads lie in different banks
+#define CHUNKS 16
+#define TILES_FOR_FOUR 512
 
-__global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w,
-                                                       const float* __restrict__ bias, float* __restrict__ out,
-                                                       int M, int N, int K) {
-    __shared__ __attribute__((aligned(16))) float xs[2][FT][FROW];
-    __shared__ __attribute__((aligned(16))) float ws[2][FT][FROW];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+__host__ __device__ __forceinline__ int chunk_len(int K) { return (K + CHUNKS * FK - 1) / (CHUNKS * FK) * FK; }
+
+// four consecutive elements of a row from k on; without FULL the row may end inside them
+template <bool FULL>
+__device__ __forceinline__ floatx4 four_of_row(const float* __restrict__ row, int k, int K) {
+    if (FULL) return *(const floatx4*)(row + k);
+    floatx4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = k + e < K ? row[k + e] : 0.f;
+    return v;
+}
+
+// 16 MT rows a block (blockIdx.y: which).  Lane (g, r), g = lane / 16, r = lane % 16, brings W[n0 + r][k + 4 g .. + 4] and the same of x's row r.
+// BATCH steps are asked for at once, the next batch before the current one is multiplied.
+template <int MT, int NT, int BATCH, bool FULL>
+__global__ __launch_bounds__(64 * CHUNKS) void gemm_f32_rows_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                                    const float* __restrict__ bias, float* __restrict__ out,
+                                                                    int M, int N, int K, int chunk) {
+    __shared__ float part[CHUNKS][MT * NT][4][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, r = lane & 15;
+    const int n0 = blockIdx.x * (16 * NT), m0 = blockIdx.y * (16 * MT);
+    const int k_lo = wave * chunk, k_hi = k_lo + chunk < K ? k_lo + chunk : K;   // (a block has a wave per chunk that holds some of K)
+    const float* wrow[NT];
+    const float* xrow[MT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const int n = n0 + 16 * j + r;
+        wrow[j] = w + (long)(n < N ? n : N - 1) * K + 4 * g;
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        const int m = m0 + 16 * i + r;
+        xrow[i] = x + (long)(m < M ? m : M - 1) * K + 4 * g;
+    }
+    floatx4 acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    floatx4 wv[2][BATCH][NT], xv[2][BATCH][MT];
+    const int last = k_lo + (k_hi - k_lo - 1) / FK * FK;          // the chunk's last step (read again where a batch passes it)
+    auto ask = [&](int buf, int k0) {
+#pragma unroll
+        for (int b = 0; b < BATCH; ++b) {
+            const int k = k0 + b * FK < last ? k0 + b * FK : last;
+#pragma unroll
+            for (int j = 0; j < NT; ++j) wv[buf][b][j] = four_of_row<FULL>(wrow[j], k, K - 4 * g);
+#pragma unroll
+            for (int i = 0; i < MT; ++i) xv[buf][b][i] = four_of_row<FULL>(xrow[i], k, K - 4 * g);
+        }
+    };
+    auto multiply = [&](int buf, int k0) {
+#pragma unroll
+        for (int b = 0; b < BATCH; ++b) {
+            if (k0 + b * FK > last) break;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[buf][b][i][e], wv[buf][b][j][e], acc[i][j], 0, 0, 0);
+        }
+    };
+    ask(0, k_lo);
+    for (int k0 = k_lo; k0 <= last; k0 += 2 * BATCH * FK) {
+        ask(1, k0 + BATCH * FK);
+        multiply(0, k0);
+        ask(0, k0 + 2 * BATCH * FK);
+        multiply(1, k0 + BATCH * FK);
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) part[wave][i * NT + j][e][lane] = acc[i][j][e];
+    __syncthreads();
+    const int waves = blockDim.x >> 6;
+    for (int at = threadIdx.x; at < MT * NT * 256; at += blockDim.x) {
+        const int l = at & 63, e = (at >> 6) & 3, tile = at >> 8;
+        float total = 0.f;
+        for (int q = 0; 4 * q < waves; ++q) {
+            float quarter = part[4 * q][tile][e][l];
+            for (int c = 4 * q + 1; c < 4 * q + 4 && c < waves; ++c) quarter += part[c][tile][e][l];
+            total = q ? total + quarter : quarter;
+        }
+        const int m = m0 + (tile / NT) * 16 + 4 * (l >> 4) + e, n = n0 + (tile % NT) * 16 + (l & 15);
+        if (m < M && n < N) out[(long)m * N + n] = bias ? total + bias[n] : total;
+    }
+}
+
+// Tiles of 64 x 64, GROUPS (1 or 4) groups of four waves.  For a step, lane (h, r), h = lane / 32, r = lane % 32, reads
+// x[row r][4 h .. + 4] and [8 + 4 h .. + 4], and the same of W: with the instructions taking element j of the first and of
+// the second piece in turn, the order is the one above.
+template <int GROUPS, bool FULL>
+__global__ __launch_bounds__(256 * GROUPS) void gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                                const float* __restrict__ bias, float* __restrict__ out,
+                                                                int M, int N, int K, int chunk) {
+    // (the groups' sums take the place of the staged steps at the end)
+    constexpr int STAGE = 2 * FT * FROW, ALL = GROUPS * 2 * STAGE, SUMS = GROUPS > 1 ? GROUPS * 16 * 256 : 0;
+    __shared__ __attribute__((aligned(16))) float lds[ALL > SUMS ? ALL : SUMS];
+    const int group = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     const int h = lane >> 5, r = lane & 31;
     const int m0 = blockIdx.y * FT, n0 = blockIdx.x * FT;
+    float* xs = lds + group * 2 * STAGE;              // [2 buffers][FT][FROW], then the same for w
+    float* ws = xs + STAGE;
     // staging: thread tid brings four consecutive k of one row of each operand
     const int srow = tid >> 2, sk = (tid & 3) * 4;
-    const bool xrow_ok = m0 + srow < M, wrow_ok = n0 + srow < N;
-    const float* xsrc = x + (long)(xrow_ok ? m0 + srow : 0) * K + sk;
-    const float* wsrc = w + (long)(wrow_ok ? n0 + srow : 0) * K + sk;
-    const bool vec = (K & 3) == 0;
+    const float* xsrc = x + (long)(m0 + srow < M ? m0 + srow : M - 1) * K + sk;
+    const float* wsrc = w + (long)(n0 + srow < N ? n0 + srow : N - 1) * K + sk;
+    const int sat = srow * FROW + sk;
 
-    auto fetch = [&](const float* src, bool row_ok, int k0, floatx4& v) {
-        v = floatx4{0.f, 0.f, 0.f, 0.f};
-        if (!row_ok) return;
-        if (vec && k0 + sk + 3 < K) {
-            v = *(const floatx4*)(src + k0);
-        } else {
+    const int quarters = GROUPS > 1 ? 1 : 4;          // quarters of K that this group walks
+    const int k_begin = group * 4 * chunk;
+    const int steps_chunk = chunk / FK, steps = quarters * 4 * steps_chunk;
+    const int last = (K - 1) / FK * FK;               // K's last step
+    // (steps behind the end of K are walked for the barriers' sake, their loads repeat the last step and nothing is multiplied)
+    auto k_of = [&](int s) { const int k = k_begin + s * FK; return k < last ? k : last; };
+    floatx16 acc, quarter, total;
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (k0 + sk + e < K) v[e] = src[k0 + e];
-        }
-    };
-
-    floatx16 acc;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) acc[e] = 0.f;
-    floatx4 xv, wv;
-    fetch(xsrc, xrow_ok, 0, xv);
-    fetch(wsrc, wrow_ok, 0, wv);
-    *(floatx4*)&xs[0][srow][sk] = xv;
-    *(floatx4*)&ws[0][srow][sk] = wv;
+    for (int e = 0; e < 16; ++e) acc[e] = quarter[e] = total[e] = 0.f;
+    floatx4 xv = four_of_row<FULL>(xsrc, k_of(0), K - sk), wv = four_of_row<FULL>(wsrc, k_of(0), K - sk);
+    *(floatx4*)&xs[sat] = xv;
+    *(floatx4*)&ws[sat] = wv;
+    xv = four_of_row<FULL>(xsrc, k_of(1), K - sk);
+    wv = four_of_row<FULL>(wsrc, k_of(1), K - sk);
     __syncthreads();
-    int buf = 0;
-    for (int k0 = 0; k0 < K; k0 += FK) {
-        const bool more = k0 + FK < K;
-        if (more) {
-            fetch(xsrc, xrow_ok, k0 + FK, xv);
-            fetch(wsrc, wrow_ok, k0 + FK, wv);
-        }
-        const float* xa = &xs[buf][wm * 32 + r][h * 8];
-        const float* wa = &ws[buf][wn * 32 + r][h * 8];
-        const floatx4 a0 = *(const floatx4*)xa, a1 = *(const floatx4*)(xa + 4);
-        const floatx4 b0 = *(const floatx4*)wa, b1 = *(const floatx4*)(wa + 4);
+    int buf = 0, in_chunk = 0, chunk_no = 0;
+    const int busy = k_begin >= K ? 0 : (K - k_begin + FK - 1) / FK < steps ? (K - k_begin + FK - 1) / FK : steps;
+    const int walk = GROUPS > 1 ? (steps < (K + FK - 1) / FK ? steps : (K + FK - 1) / FK) : busy;   // (the first group's busy steps)
+    for (int s = 0; s < walk; ++s) {
+        const float* xa = &xs[(buf * FT + wm * 32 + r) * FROW + h * 4];
+        const float* wa = &ws[(buf * FT + wn * 32 + r) * FROW + h * 4];
+        const floatx4 a0 = *(const floatx4*)xa, a1 = *(const floatx4*)(xa + 8);
+        const floatx4 b0 = *(const floatx4*)wa, b1 = *(const floatx4*)(wa + 8);
+        // the next step, asked for a step ago, goes to the other buffer (its readers passed the last barrier); the step
+        // after it is asked for
+        *(floatx4*)&xs[(buf ^ 1) * FT * FROW + sat] = xv;
+        *(floatx4*)&ws[(buf ^ 1) * FT * FROW + sat] = wv;
+        xv = four_of_row<FULL>(xsrc, k_of(s + 2), K - sk);
+        wv = four_of_row<FULL>(wsrc, k_of(s + 2), K - sk);
+        if (s < busy) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[j], b0[j], acc, 0, 0, 0);
+            for (int j = 0; j < 4; ++j) {
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[j], b0[j], acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[j], b1[j], acc, 0, 0, 0);
+            }
+            if (++in_chunk == steps_chunk || s + 1 == busy) {     // the end of a chunk, perhaps of a quarter
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[j], b1[j], acc, 0, 0, 0);
-        if (more) {
-            *(floatx4*)&xs[buf ^ 1][srow][sk] = xv;     // (that buffer's readers passed the last barrier)
-            *(floatx4*)&ws[buf ^ 1][srow][sk] = wv;
+                for (int e = 0; e < 16; ++e) quarter[e] = (chunk_no & 3) ? quarter[e] + acc[e] : acc[e];
+                if ((chunk_no & 3) == 3 || s + 1 == busy) {
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) total[e] = chunk_no >= 4 ? total[e] + quarter[e] : quarter[e];
+                }
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+                in_chunk = 0;
+                ++chunk_no;
+            }
         }
         __syncthreads();
         buf ^= 1;
     }
     // lane (h, r) holds out[m0 + 32 wm + 8 b + 4 h + i][n0 + 32 wn + r] as element 4 b + i
     const int n = n0 + wn * 32 + r;
-    if (n < N) {
-        const float bv = bias ? bias[n] : 0.f;
+    const float bv = bias && n < N ? bias[n] : 0.f;
+    auto put = [&](int e, float v) {
+        const int m = m0 + wm * 32 + 8 * (e >> 2) + 4 * h + (e & 3);
+        if (m < M && n < N) out[(long)m * N + n] = bias ? v + bv : v;
+    };
+    if (GROUPS == 1) {
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
+        for (int e = 0; e < 16; ++e) put(e, total[e]);
+    } else {
+        // the groups' quarters meet in shared memory; every group adds and stores four of a lane's 16 outputs
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int m = m0 + wm * 32 + 8 * b + 4 * h + i;
-                if (m < M) out[(long)m * N + n] = bias ? acc[4 * b + i] + bv : acc[4 * b + i];
-            }
+        for (int e = 0; e < 16; ++e) lds[(group * 16 + e) * 256 + tid] = total[e];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int e = group * 4 + i;
+            float v = lds[e * 256 + tid];
+#pragma unroll
+            for (int q = 1; q < 4; ++q)
+                if (q * 4 * chunk < K) v += lds[(q * 16 + e) * 256 + tid];
+            put(e, v);
+        }
     }
+}
+
+template <int MT, int NT, int BATCH>
+static void launch_rows(const float* x, const float* w, const float* bias, float* out, int M, int N, int K, bool full,
+                        hipStream_t stream) {
+    const int chunk = chunk_len(K), waves = qe_cdiv(K, chunk);
+    const dim3 grid(qe_cdiv(N, 16 * NT), qe_cdiv(M, 16 * MT));
+    if (full) gemm_f32_rows_kernel<MT, NT, BATCH, true><<<grid, 64 * waves, 0, stream>>>(x, w, bias, out, M, N, K, chunk);
+    else gemm_f32_rows_kernel<MT, NT, BATCH, false><<<grid, 64 * waves, 0, stream>>>(x, w, bias, out, M, N, K, chunk);
 }
 
 int qe_gemm_f32(const float* x, const float* w, const float* bias, float* out, int M, int N, int K,
                 hipStream_t stream) {
+    const bool full = K % FK == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0;
+    // More than 16 rows against a very wide matrix (logits): every block would read all rows again, and the tiles are
+    // enough to fill the chip (33 rows, 151936 x 1024: 467 us by rows, 235 by tiles).  Up to 128 tiles leave half of the
+    // compute units idle; blocks of 64 rows and 16 outputs do not (100 rows, 1024 x 3072: 73.5 us by tiles, 33.4 by rows).
+    const long tiles = (long)qe_cdiv(N, FT) * qe_cdiv(M, FT);
+    if (M <= 16 || (M <= 64 && N < 16384) || tiles <= 128) {
+        // 32 outputs a block halve the reads of x; they pay where the rows are some and the blocks enough (16 rows,
+        // 6144 x 1024: 12.0 us against 14.3, 151936 x 1024: 183 against 213; 2 rows: 10.3 against 10.6, 148 against 137;
+        // 16 rows, 4096 x 1024: 11.5 against 9.5)
+        if (M > 4 && M <= 16 && N >= 6144) launch_rows<1, 2, 1>(x, w, bias, out, M, N, K, full, stream);
+        else if (M <= 16) launch_rows<1, 1, 2>(x, w, bias, out, M, N, K, full, stream);
+        else if (M <= 32) launch_rows<2, 1, 2>(x, w, bias, out, M, N, K, full, stream);
+        else launch_rows<4, 1, 1>(x, w, bias, out, M, N, K, full, stream);
+        QE_LAUNCH_CHECK();
+        return 0;
+    }
     QE_REQUIRE(qe_cdiv(M, FT) <= 65535, "gemm (32-bit): M=%d is too large for one launch", M);
     dim3 grid(qe_cdiv(N, FT), qe_cdiv(M, FT));
-    gemm_f32_kernel<<<grid, 256, 0, stream>>>(x, w, bias, out, M, N, K);
+    const int chunk = chunk_len(K);
+    const bool four = tiles < TILES_FOR_FOUR;
+    if (four && full) gemm_f32_kernel<4, true><<<grid, 1024, 0, stream>>>(x, w, bias, out, M, N, K, chunk);
+    else if (four) gemm_f32_kernel<4, false><<<grid, 1024, 0, stream>>>(x, w, bias, out, M, N, K, chunk);
+    else if (full) gemm_f32_kernel<1, true><<<grid, 256, 0, stream>>>(x, w, bias, out, M, N, K, chunk);
+    else gemm_f32_kernel<1, false><<<grid, 256, 0, stream>>>(x, w, bias, out, M, N, K, chunk);
     QE_LAUNCH_CHECK();
     return 0;
 }
