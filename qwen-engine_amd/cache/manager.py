@@ -154,14 +154,20 @@ class StateSlots:
         self.free.append(slot)
 
 
+def packed_tokens(tokens: Sequence[int]) -> bytes:
+    """The tokens as 8 bytes each: what is hashed and compared, a slice a page (an object per token and a call
+    of the hash for each took two thirds of an admission with 64 shared pages)."""
+    return np.asarray(tokens, dtype="<i8").tobytes()
+
+
+def _chained(parent: bytes, page: bytes) -> bytes:
+    return hashlib.blake2b(parent + page, digest_size=8).digest()
+
+
 def chain_hash(parent: int, tokens: Sequence[int]) -> int:
     """64-bit hash of a page's tokens chained to the hash of the page before it
     (the construction of src/engine/kvcache.py:81-86)."""
-    h = hashlib.blake2b(digest_size=8)
-    h.update(int(parent).to_bytes(8, "little", signed=False))
-    for tok in tokens:
-        h.update(int(tok).to_bytes(8, "little", signed=True))
-    return int.from_bytes(h.digest(), "little", signed=False)
+    return int.from_bytes(_chained(int(parent).to_bytes(8, "little"), packed_tokens(tokens)), "little")
 
 
 @dataclass
@@ -182,7 +188,7 @@ class RequestCache:
 @dataclass
 class _SharedEntry:
     pages: Tuple[int, ...]   # one page id per group
-    tokens: Tuple[int, ...]
+    tokens: bytes            # packed_tokens of the page
 
 
 class CacheManager:
@@ -241,10 +247,18 @@ class CacheManager:
         if self.keep_freed:
             # registered pages go index by index, the pages of all groups together: an entry that
             # nobody holds any more is kept instead of freed
-            for i, page0 in enumerate(rc.tables[0]):
-                h = self._page_hash.get(page0) if page0 >= 0 else None
+            first = rc.tables[0]
+            for i, page0 in enumerate(first):
+                h = self._page_hash.get(page0)             # (-1, no page, is never registered)
                 entry = self._shared.get(h) if h is not None else None
-                if entry is None or any(i >= len(t) or t[i] != entry.pages[g] for g, t in enumerate(rc.tables)):
+                if entry is None:
+                    continue
+                if len(rc.tables) == 1:
+                    if self.pools[0].release(page0, to_free_list=False):
+                        kept.append(h)
+                    first[i] = -1
+                    continue
+                if any(i >= len(t) or t[i] != entry.pages[g] for g, t in enumerate(rc.tables)):
                     continue
                 unheld = [self.pools[g].release(p, to_free_list=False) for g, p in enumerate(entry.pages)]
                 if all(unheld):
@@ -432,33 +446,31 @@ class CacheManager:
         if not self.prefix_sharing:
             return 0
         P = self.page_size
-        max_pages = (len(prompt) - 1) // P if prompt else 0
-        parent = 0
+        max_pages = (len(prompt) - 1) // P if prompt is not None and len(prompt) else 0
+        packed = packed_tokens(prompt[:max_pages * P] if max_pages else ())
+        parent = bytes(8)
         taken: List[_SharedEntry] = []
         hashes = []
         for i in range(max_pages):
-            toks = tuple(int(t) for t in prompt[i * P:(i + 1) * P])
-            h = chain_hash(parent, toks)
+            page = packed[8 * P * i:8 * P * (i + 1)]
+            parent = _chained(parent, page)
+            h = int.from_bytes(parent, "little")
             entry = self._shared.get(h)
-            if entry is None or entry.tokens != toks:   # the token test guards against collisions
+            if entry is None or entry.tokens != page:   # the token test guards against collisions
                 break
             taken.append(entry)
             hashes.append(h)
-            parent = h
-        for h, entry in zip(hashes, taken):
-            was_kept = self._kept.pop(h, None) is not None    # held by nobody until now
-            self.stats["kept_page_hits"] += int(was_kept)
-            for g, page in enumerate(entry.pages):
-                if was_kept:
-                    self.pools[g].revive(page)
-                else:
-                    self.pools[g].retain(page)
-                rc.dirty[g].append(len(rc.tables[g]))
-                rc.tables[g].append(page)
+        was_kept = [self._kept.pop(h, None) is not None for h in hashes]    # held by nobody until now
+        self.stats["kept_page_hits"] += sum(was_kept)
+        for g, pool in enumerate(self.pools):
+            for entry, kept in zip(taken, was_kept):
+                (pool.revive if kept else pool.retain)(entry.pages[g])
+            rc.dirty[g].extend(range(len(taken)))
+            rc.tables[g].extend(entry.pages[g] for entry in taken)
         n = len(taken) * P
         rc.num_tokens = n
         rc.shared_len = n
-        rc.tokens = [int(t) for t in prompt[:n]]
+        rc.tokens = np.frombuffer(packed, dtype="<i8", count=n).tolist()
         rc.hashes = hashes
         self.stats["shared_page_hits"] += len(taken)
         return n
@@ -468,9 +480,9 @@ class CacheManager:
         full = rc.num_tokens // P
         while len(rc.hashes) < full:
             i = len(rc.hashes)
-            toks = tuple(rc.tokens[i * P:(i + 1) * P])
+            toks = packed_tokens(rc.tokens[i * P:(i + 1) * P])
             parent = rc.hashes[-1] if rc.hashes else 0
-            h = chain_hash(parent, toks)
+            h = int.from_bytes(_chained(parent.to_bytes(8, "little"), toks), "little")
             rc.hashes.append(h)
             pages = tuple(rc.tables[g][i] for g in range(len(self.groups)))
             if h not in self._shared and pages[0] not in self._page_hash:
