@@ -125,10 +125,11 @@ extern "C" int qe_latent_kv_store(const float* kv, const float* weight, float ep
 }
 
 // q [T, H, Dn + Dr] -> qp[T, H, R + Dr]: the last Dr of each head, rotated, to the last Dr of the
-// packed query (its first R come from the product with the folded key map).
+// packed query (its first R come from the product with the folded key map).  qp may be q itself (R = Dn): a thread
+// reads its pair and writes it back.
 template <typename TA>
-__global__ void latent_q_rotate_kernel(const TA* __restrict__ q, const int* __restrict__ positions,
-                                       const float* __restrict__ inv_freq, int rot_dims, TA* __restrict__ qp,
+__global__ void latent_q_rotate_kernel(const TA* q, const int* __restrict__ positions,
+                                       const float* __restrict__ inv_freq, int rot_dims, TA* qp,
                                        long n_heads_total, int H, int Dn, int Dr, int R, int half_split) {
     const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;      // (token * H + head) * ceil(Dr / 2) + pair
     const int pairs = (Dr + 1) / 2;

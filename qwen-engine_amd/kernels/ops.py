@@ -114,6 +114,9 @@ def load_library():
         "qe_scaled_sum": [vp, f32, vp, f32, i32, vp, i64, vp],
         "qe_polynorm": [vp, vp, f32, vp, i32, i32, i32, vp],
         "qe_short_conv": [vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, vp],
+        "qe_latent_prefill_supported": [i32, i32, i32, i32],
+        "qe_latent_gather": [vp, vp, vp, vp, i32, vp, vp, vp, vp, i64, i32, i32, i32, i32, vp],
+        "qe_latent_prefill": [vp, vp, vp, vp, i64, vp, vp, vp, i32, vp, vp, i32, i32, i32, i32, f32, i32, vp, vp, i64, i32, i32, vp],
         "qe_latent_kv_store": [vp, vp, f32, vp, vp, i32, vp, vp, i32, i32, i32, i32, vp, vp, i32, i32, i32, vp],
         "qe_latent_q_rotate": [vp, vp, vp, i32, vp, i32, i32, i32, i32, i32, i32, i32, vp],
         "qe_latent_attention": [vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, f32, i32, vp, i32, vp],
@@ -1208,6 +1211,80 @@ def latent_attention(qp: torch.Tensor, cache: torch.Tensor, positions: torch.Ten
     return out
 
 
+def latent_prefill_supported(latent: int, dim: int, rot_dim: int, v_dim: int, dtype: torch.dtype) -> bool:
+    """True if latent_gather and latent_prefill take heads of these sizes."""
+    return dtype == torch.bfloat16 and bool(load_library().qe_latent_prefill_supported(int(latent), int(dim), int(rot_dim), int(v_dim)))
+
+
+def latent_gather(cache: torch.Tensor, positions: torch.Tensor, tok_seq: torch.Tensor, block_table: torch.Tensor,
+                  portions: torch.Tensor, owner: torch.Tensor, latent: int, window: int = 0):
+    """The cache rows that portions of prompts see, side by side: (latents [keys, R], shared rotated parts [keys, Dr]) for keys =
+    64 owner.shape[0].  portions int32 [n, 3] = (first row, rows, place of its first key, a multiple of 64), owner int32: the
+    portion of every 64 places.  A portion's keys are those at positions 0 (with ``window``: of the first key that its first row
+    sees) .. of its last row; zeros behind them.  The caller guarantees that they fit and have pages."""
+    lib = load_library()
+    _need(cache, "cache", torch.bfloat16, (None, 1, 1, None, None))
+    dev, D, R = cache.device, cache.shape[4], int(latent)
+    _need(positions, "positions", torch.int32, (None,), dev)
+    _need(tok_seq, "tok_seq", torch.int32, (positions.shape[0],), dev)
+    _need(block_table, "block_table", torch.int32, (None, None), dev)
+    _need(portions, "portions", torch.int32, (None, 3), dev)
+    _need(owner, "owner", torch.int32, (None,), dev)
+    keys = 64 * owner.shape[0]
+    ck = torch.empty((keys, R), dtype=cache.dtype, device=dev)
+    kr = torch.empty((keys, D - R), dtype=cache.dtype, device=dev)
+    _check(lib.qe_latent_gather(cache.data_ptr(), positions.data_ptr(), tok_seq.data_ptr(), block_table.data_ptr(),
+                                block_table.shape[1], portions.data_ptr(), owner.data_ptr(), ck.data_ptr(), kr.data_ptr(), keys,
+                                R, D - R, cache.shape[3], int(window), _stream()), "latent_gather")
+    return ck, kr
+
+
+def latent_prefill(q: torch.Tensor, kx: torch.Tensor, kr: torch.Tensor, vt: torch.Tensor, out: torch.Tensor,
+                   tiles: torch.Tensor, group_portion: torch.Tensor, portions: torch.Tensor, positions: torch.Tensor,
+                   scale: float, window: int = 0, sink: Optional[torch.Tensor] = None,
+                   gate: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """Attention of the rows of portions over expanded keys: q [T, H, Dn + Dr] (its last Dr rotated), kx [keys, H Dn] and kr
+    [keys, Dr] the heads' own and the shared part of the keys, vt [H Dv, keys] the values transposed, out [T, H, Dv].  tiles int32
+    [4 n, 2] = (first row, rows <= 32) in groups of four of one portion in ascending rows (filled up with 0 rows), group_portion
+    int32 [n]; portions as for latent_gather.  window, sink: as for latent_attention; gate: as for gemm_heads."""
+    lib = load_library()
+    _need(q, "q", torch.bfloat16, (None, None, None))
+    T, H, Dq = q.shape
+    dev, Dr = q.device, kr.shape[1]
+    Dn, keys = Dq - Dr, kx.shape[0]
+    _need(kx, "kx", q.dtype, (keys, H * Dn), dev)
+    _need(kr, "kr", q.dtype, (keys, Dr), dev)
+    _need(out, "out", q.dtype, (T, H, None), dev)
+    Dv = out.shape[2]
+    _need(vt, "vt", q.dtype, (H * Dv, keys), dev)
+    _need(tiles, "tiles", torch.int32, (None, 2), dev)
+    n = tiles.shape[0] // 4
+    _need(group_portion, "group_portion", torch.int32, (n,), dev)
+    _need(portions, "portions", torch.int32, (None, 3), dev)
+    _need(positions, "positions", torch.int32, (T,), dev)
+    if tiles.shape[0] % 4:
+        raise KernelError("latent_prefill: tiles come in groups of four")
+    if sink is not None:
+        _need(sink, "sink", torch.float32, (H,), dev)
+    gs = _gate_strides(gate, q, T, H, Dv) if gate is not None else (0, 0, 0)
+    _check(lib.qe_latent_prefill(q.data_ptr(), kx.data_ptr(), kr.data_ptr(), vt.data_ptr(), keys, out.data_ptr(),
+                                 tiles.data_ptr(), group_portion.data_ptr(), n, portions.data_ptr(), positions.data_ptr(), H,
+                                 Dn, Dr, Dv, float(scale), int(window or 0), _ptr(sink), _ptr(gate), gs[0], gs[1], gs[2],
+                                 _stream()), "latent_prefill")
+    return out
+
+
+def _gate_strides(gate: torch.Tensor, x: torch.Tensor, T: int, H: int, N: int):
+    """The strides (row, head, number) of a gate [T, H * N], or [T, H] with one number a head (or a view of H columns of wider
+    rows)."""
+    if gate.dim() == 2 and gate.shape == (T, H) and gate.stride(1) == 1 and H * N != H:
+        if not gate.is_cuda or gate.dtype != x.dtype or gate.device != x.device:
+            raise KernelError("the gate is not where and what the rows are")
+        return gate.stride(0), 1, 0
+    _need(gate, "gate", x.dtype, (T, H * N), x.device)
+    return H * N, N, 1
+
+
 def gemm_heads(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gate: Optional[torch.Tensor] = None,
                algo: int = ALGO_AUTO) -> torch.Tensor:
     """out[t, h, :N] = w[h] x[t, h, :K] for w [H, N, K]; x [T, H, >= K] and out [T, H, >= N] (the product reads
@@ -1223,15 +1300,7 @@ def gemm_heads(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gate: Option
         raise KernelError("gemm_heads: heads narrower than the product")
     if x.dtype == torch.float32 and w.dtype != torch.float32:
         raise KernelError("gemm_heads: 32-bit activations need 32-bit weights")
-    gs = (0, 0, 0)
-    if gate is not None:
-        if gate.dim() == 2 and gate.shape == (T, H) and gate.stride(1) == 1 and H * N != H:
-            if not gate.is_cuda or gate.dtype != x.dtype or gate.device != x.device:
-                raise KernelError("gemm_heads: the gate is not where and what the rows are")
-            gs = (gate.stride(0), 1, 0)
-        else:
-            _need(gate, "gate", x.dtype, (T, H * N), x.device)
-            gs = (H * N, N, 1)
+    gs = _gate_strides(gate, x, T, H, N) if gate is not None else (0, 0, 0)
     if (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and algo != ALGO_GENERIC and
             lib.qe_gemm_heads_mfma_supported(K, H * x.shape[2], x.shape[2])):
         _check(lib.qe_gemm_heads_mfma(x.data_ptr(), H * x.shape[2], x.shape[2], w.data_ptr(), out.data_ptr(),

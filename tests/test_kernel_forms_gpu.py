@@ -34,3 +34,83 @@ def test_float32_gemm_sums_in_one_order(ops, M, N, K):
         assert torch.equal(ops.gemm(x[m:m + 1].to(DEV), w.to(DEV))[0], got[m])
     odd = torch.empty(M * K + 1, device=DEV)[1:].view(M, K).copy_(x)
     assert torch.equal(ops.gemm(odd, w.to(DEV)), got)
+
+
+def latent_rows(before, rows, R, dr, page, seed):
+    """Requests with ``before`` cached tokens and ``rows`` new ones over scattered pages: (cache, table, positions, tok_seq, the
+    requests' rows [keys, R + dr])."""
+    keys = [b + n for b, n in zip(before, rows)]
+    pages = [-(-k // page) for k in keys]
+    order = torch.randperm(sum(pages), generator=torch.Generator().manual_seed(seed))
+    cache = torch.full((sum(pages), 1, 1, page, R + dr), float("nan"))       # (what was never written must not be used)
+    table = torch.full((len(keys), max(pages)), -1, dtype=torch.int32)
+    own, at = [], 0
+    for i, k in enumerate(keys):
+        c = rand(k, R + dr, seed=seed + 1 + i).bfloat16().float()
+        ids = order[at:at + pages[i]]
+        at += pages[i]
+        table[i, :pages[i]] = ids.int()
+        flat = torch.full((pages[i] * page, R + dr), float("nan"))
+        flat[:k] = c
+        cache[ids, 0, 0] = flat.view(pages[i], page, R + dr)
+        own.append(c.double())
+    pos = torch.cat([torch.arange(b, b + n) for b, n in zip(before, rows)]).int()
+    seq = torch.cat([torch.full((n,), i) for i, n in enumerate(rows)]).int()
+    return cache.bfloat16().to(DEV), table.to(DEV), pos.to(DEV), seq.to(DEV), own
+
+
+@pytest.mark.parametrize("R,dn,dr,dv", [(512, 128, 64, 128), (128, 64, 32, 64), (64, 128, 0, 128), (72, 64, 0, 64), (256, 96, 32, 64)])
+@pytest.mark.parametrize("before,rows", [((0,), (1,)), ((0, 0), (33, 130)), ((70, 0, 5), (31, 128, 64)), ((300,), (257,)), ((1000, 3), (5, 700))])
+@pytest.mark.parametrize("window,sink,gated", [(0, False, 0), (40, True, 1), (64, False, 2)])
+def test_latent_attention_of_portions_with_expanded_keys(ops, R, dn, dr, dv, before, rows, window, sink, gated):
+    """Every size of head that the kernel takes, portions that end inside a tile of rows, of keys and of 64 places, windows that
+    begin anywhere, against 64-bit attention; the kernel with folded maps beside it."""
+    from qwen_engine_amd.parts.attention import prefill_tiles
+    H, page, scale, T = 3, 16, 0.11, sum(rows)
+    cache, table, pos, seq, own = latent_rows(before, rows, R, dr, page, 17)
+    uk, uv = rand(H * dn, R, seed=3, scale=R ** -0.5).bfloat16(), rand(H * dv, R, seed=4, scale=R ** -0.5).bfloat16()
+    q = rand(T, H, dn + dr, seed=5, scale=1.5).bfloat16()
+    sinks = rand(H, seed=6).to(DEV) if sink else None
+    gate = rand(T, H * dv if gated == 1 else H, seed=7).bfloat16().to(DEV) if gated else None
+    portions, owner, tiles, group, at = [], [], [], [], 0
+    for i, (b, n) in enumerate(zip(before, rows)):
+        keys = b + n - (max(0, b - window + 1) if window else 0)
+        portions += [at, n, 64 * len(owner)]
+        owner += [i] * -(-keys // 64)
+        mine = prefill_tiles([(at, n)], 32)
+        tiles += mine
+        group += [i] * (len(mine) // 8)
+        at += n
+    i32 = lambda v, *shape: torch.tensor(v, dtype=torch.int32, device=DEV).view(*shape)
+    portions = i32(portions, -1, 3)
+    ck, kr = ops.latent_gather(cache, pos, seq, table, portions, i32(owner, -1), R, window=window)
+    out = torch.full((T, H, dv), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.latent_prefill(q.to(DEV), ops.gemm(ck, uk.to(DEV)), kr, ops.gemm(uv.to(DEV), ck), out, i32(tiles, -1, 2), i32(group, -1),
+                       portions, pos, scale, window=window, sink=sinks, gate=gate)
+    qp = torch.empty(T, H, R + dr, dtype=torch.bfloat16, device=DEV)
+    qp[..., R:] = q.to(DEV)[..., dn:]
+    ops.gemm_heads(q.to(DEV), uk.view(H, dn, R).transpose(1, 2).contiguous().to(DEV), qp)
+    folded = torch.empty_like(out)
+    ops.gemm_heads(ops.latent_attention(qp, cache, pos, seq, table, R, scale, window=window, sink=sinks),
+                   uv.view(H, dv, R).to(DEV), folded, gate)
+    want, at = [], 0
+    for i, (b, n) in enumerate(zip(before, rows)):
+        c = own[i]
+        k = torch.cat([(c[:, :R] @ uk.double().t()).view(-1, H, dn), c[:, None, R:].expand(-1, H, dr)], dim=2)
+        v = (c[:, :R] @ uv.double().t()).view(-1, H, dv)
+        s = torch.einsum("thd,khd->htk", q[at:at + n].double(), k) * scale
+        d = torch.arange(b, b + n)[:, None] - torch.arange(b + n)[None, :]
+        s = s.masked_fill((d < 0) | ((d >= window) if window else False), float("-inf"))
+        if sink:
+            s = torch.cat([s, sinks.cpu().double().view(H, 1, 1).expand(H, n, 1)], dim=2)
+        p = torch.softmax(s, dim=-1)[..., :b + n]
+        want.append(torch.einsum("htk,khd->thd", p, v))
+        at += n
+    want = torch.cat(want)
+    if gated:
+        want = want * torch.sigmoid(gate.cpu().double().view(T, H, -1))
+    off = lambda t: float((t.cpu().double() - want).norm() / want.norm())
+    # keys, values, weights and the result are rounded to bfloat16 once each: 2^-9 / sqrt(3) of the size apiece, the keys'
+    # by way of scores of a few units (the folded maps round queries, weights, latent sums and the result)
+    print(f"expanded {off(out):.2e} folded {off(folded):.2e}")
+    assert off(out) < 5e-3, (off(out), off(folded))
