@@ -89,20 +89,36 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // Consecutive blocks go to the eight XCDs in turn, and each XCD has an L2 of its own: the blocks
     // of one XCD take a compact part of the tiles, xcd_m parts down by xcd_n across (the host picks
-    // the cut that makes the XCDs read the fewest rows of x and W altogether; 0: no cut fits), so
-    // that they share what they read through that L2.
+    // the cut that makes the XCDs read the fewest rows of x and W altogether; 0: no cut into equal parts), so
+    // that they share what they read through that L2.  (A single row of tiles shares nothing of W and goes as the blocks
+    // come; so do grouped rows.)
     int tile_m, tile_n;
-    if (xcd_m > 0) {
-        const int xcd = blockIdx.x % 8, local = blockIdx.x / 8;
-        const int per_m = tiles_m / xcd_m, per_n = tiles_n / xcd_n;
-        // Inside the part the tiles go in bands of up to 8 tile rows, across the band column by
-        // column: the 32 or 64 blocks that an XCD runs at a time are then a patch of 8 by 4 or 8
+    if (!tail.tiles && tiles_m > 1) {
+        int local, part_m = 0, part_n = 0, per_m = tiles_m, per_n = tiles_n;
+        const int xcd = blockIdx.x % 8;
+        local = blockIdx.x / 8;
+        if (xcd_m > 0) {
+            per_m /= xcd_m;
+            per_n /= xcd_n;
+            part_m = (xcd / xcd_n) * per_m;
+            part_n = (xcd % xcd_n) * per_n;
+        } else {
+            // no cut into equal parts: each XCD takes an eighth of the walk below through all tiles (dealt out block by
+            // block, every XCD read nearly all of W: 1600 rows against 5120 x 25600 in three cuts, 7 by 20 tiles of
+            // 256 x 256: 455 us, now 435)
+            const int all = gridDim.x, each = all / 8, over = all % 8;
+            local += xcd * each + min(xcd, over);
+        }
+        // Inside the part the tiles go in bands of 8 tile rows (the last band has what is left), across the band
+        // column by column: the 32 or 64 blocks that an XCD runs at a time are then a patch of 8 by 4 or 8
         // tiles, which reads 12 or 16 tiles' worth of rows where a column of 32 reads 33 (what
-        // the XCDs fetch through the fabric is what bounds a large product).
-        const int gm = per_m % 8 == 0 ? 8 : (per_m % 4 == 0 ? 4 : (per_m % 2 == 0 ? 2 : 1));
-        const int band = local / (gm * per_n), within = local % (gm * per_n);
-        tile_m = (xcd / xcd_n) * per_m + band * gm + within % gm;
-        tile_n = (xcd % xcd_n) * per_n + within / gm;
+        // the XCDs fetch through the fabric is what bounds a large product).  With bands of a divisor of the tile rows
+        // instead, five tile rows went one after the other, each through all of W: 272 rows
+        // against 51200 x 5120 in tiles of 64 rows 470 us, now 266; 528 rows in tiles of 128 rows 476, now 337.
+        const int band = local / (8 * per_n), within = local - band * 8 * per_n;
+        const int rows = min(8, per_m - band * 8);
+        tile_m = part_m + band * 8 + within % rows;
+        tile_n = part_n + within / rows;
     } else {
         tile_m = blockIdx.x % tiles_m;
         tile_n = blockIdx.x / tiles_m;

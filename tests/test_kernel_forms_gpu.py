@@ -36,6 +36,23 @@ def test_float32_gemm_sums_in_one_order(ops, M, N, K):
     assert torch.equal(ops.gemm(odd, w.to(DEV)), got)
 
 
+@pytest.mark.parametrize("tile", [64, 128, 256, 512])
+@pytest.mark.parametrize("M,N", [(64 * 5, 128 * 13), (64 * 9 + 1, 128 * 7 + 64), (128 * 11 - 3, 128 * 5), (2300, 640), (130, 128 * 257 + 8)])
+def test_tiled_gemm_covers_every_tile(ops, tile, M, N):
+    """The walk through the tiles: numbers of tile rows and columns that are no multiples of eight, one band of tile rows and
+    several, a last band of one tile row; every sum is a whole number far below 2^24, so the results are exact."""
+    if tile >= 256 and M <= 128:
+        pytest.skip("no such tile for so few rows")
+    g = torch.Generator().manual_seed(M + N)
+    K = 192
+    x = torch.randint(-3, 4, (M, K), generator=g).bfloat16()
+    w = torch.randint(-3, 4, (N, K), generator=g).bfloat16()
+    want = (x.float() @ w.float().t()).to(DEV)
+    assert torch.equal(ops.gemm(x.to(DEV), w.to(DEV), out_dtype=torch.float32, algo=ops.ALGO_TILE + tile), want)
+    parts = ops.gemm(x.to(DEV), w.to(DEV), epilogue=ops.EPI_PARTIAL, splits=3, algo=ops.ALGO_TILE + tile)
+    assert torch.equal(parts[0] + parts[1] + parts[2], want)
+
+
 def latent_rows(before, rows, R, dr, page, seed):
     """Requests with ``before`` cached tokens and ``rows`` new ones over scattered pages: (cache, table, positions, tok_seq, the
     requests' rows [keys, R + dr])."""
