@@ -10,6 +10,7 @@ int qe_gemm_skinny(const void* x, const void* w, const float* bias, void* out, i
 bool qe_gemm_skinny_norm_ok(int M, int N, int K);
 int qe_gemm_skinny_splits(int N, int K);
 bool qe_gemm_mfma_ok(int M, int N, int K, int dt_a, int dt_w);
+float qe_gemm_mfma_shape(int M, int N, int K, int splits, int* tile);
 int qe_gemm_mfma(const void* x, const void* w, const float* bias, void* out, int M, int N, int K, int dt_o,
                  int tile, bool silu, int splits, hipStream_t stream);
 
@@ -83,10 +84,12 @@ extern "C" int qe_gemm_partial_splits(int M, int N, int K) {
 
 // How the product of a layer's branch (its output goes to the norm that adds it to the stream)
 // should be asked for: 0 = as a plain product; S >= 1 = as S partial products (epilogue 3), which
-// that norm adds up.  Few rows: always, the cut fills the chip.  Many rows against a narrow matrix
-// with a long K (at most one 64 x 128 tile a compute unit: a block then spends its time on the
-// trips of its K loop): two to four cuts give every unit blocks to overlap (2048 x 1024 x 3072
-// with the norm behind it: 27.7 us in two cuts against 30.8; 512 rows: 15.7 against 24.7).
+// that norm adds up.  Few rows: always, the cut fills the chip.  More rows: what the product (qe_gemm_mfma_shape) and the
+// parts, stored and read by the norm at 4 TB/s (8 bytes a number, a plain product 4), take together, for each number of
+// cuts that leaves 512 of K to a part; the cuts give every compute unit as many tiles as the others (800 rows against 5120 x 25600 with the norm
+// behind it: 232 us in three cuts of 256 x 256, 347 as a plain product; 528 rows against 4096 x 12288: 81 in three
+// of 128 x 128, 139 plain; 8192 rows against 5120 x 25600: 1851 in two, 2082 plain; 1300 rows against 4096 x 4096 stay plain:
+// 65, in two cuts 74).  Parts beyond 2^28 numbers (1 GiB) are not asked for.
 extern "C" int qe_gemm_branch_splits(int M, int N, int K, int dt_a, int dt_w) {
     if (qe_gemm_skinny_ok(M, N, K, dt_a, dt_w) || (M <= 64 && tiled_for_few_rows(M, N, K, dt_a, dt_w))) {
         const int s = qe_gemm_partial_splits(M, N, K);
@@ -94,13 +97,17 @@ extern "C" int qe_gemm_branch_splits(int M, int N, int K, int dt_a, int dt_w) {
         // product reads all of them for all rows, so at most four)
         return (M <= qe_gemm_norm_max_rows() && s > 4) ? 4 : s;
     }
-    if (!qe_gemm_mfma_ok(M, N, K, dt_a, dt_w) || K < 2048) return 0;
-    const long tiles = (long)qe_cdiv(M, 64) * qe_cdiv(N, 128);
-    if (tiles > 256) return 0;
-    int s = (int)qe_cdiv(512, tiles);
-    s = s < 2 ? 2 : (s > 4 ? 4 : s);
-    while (s > 1 && (long)(s - 1) * (qe_cdiv(qe_cdiv(K, s), 64) * 64) >= K) --s;   // every cut has some of K
-    return s > 1 ? s : 0;
+    if (!qe_gemm_mfma_ok(M, N, K, dt_a, dt_w)) return 0;
+    int best_s = 1;
+    float best = 0.f;
+    for (int s = 1; s <= 6; ++s) {
+        if (s > 1 && (K < 512 * s || (long)s * M * N > (1L << 28))) break;
+        if ((long)(s - 1) * (qe_cdiv(qe_cdiv(K, s), 64) * 64) >= K) continue;   // every cut has some of K
+        int tile;
+        const float t = qe_gemm_mfma_shape(M, N, K, s, &tile) + (s == 1 ? 4.f : 8.f * (float)s) * (float)M * (float)N / 4e6f;
+        if (s == 1 || t < best) { best_s = s; best = t; }
+    }
+    return best_s > 1 ? best_s : 0;
 }
 
 // out[M, N] = x[M, K] . w[N, K]^T (+ bias).  epilogue 0: store in dt_o.  1: add into out, the

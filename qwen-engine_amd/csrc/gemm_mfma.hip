@@ -682,29 +682,42 @@ extern "C" int qe_gemm_mfma_grouped(const void* x, const void* w, void* out, con
 }
 extern "C" int qe_gemm_mfma_grouped_tile_rows() { return 128; }
 
-static int choose_tile(int M, int N, int splits, bool with_256x256 = true) {
-    // The shape is chosen by what the busiest compute unit gets: its number of tiles (they are dealt
-    // out in turn) times a tile's area, over how well the shape uses the unit (measured on large
-    // products: 256 x 256 reaches 1.30, 256 x 128 1.16, 128 x 128 1.07, 64 x 128 0.80 PFLOP/s).
-    // A shape is never taller than the rows need.
-    // The two smaller shapes reach their rate with two blocks on a compute unit: where the busiest
-    // unit gets an odd number of them, three or more, the last runs alone at 0.7 of the rate
-    // (5120 columns against 2048 rows: 640 tiles of 128 x 128 took 632 us where 160 of 256 x 256 took 513).
+// The tile shape for a product in S cuts of K, and the microseconds it is taken to need (what the caller then does with
+// partial products left out).
+float qe_gemm_mfma_shape(int M, int N, int K, int splits, int* tile) {
+    // The busiest compute unit decides: its number of tiles (they are dealt out in turn) times what a tile costs, its
+    // operations at the rate that the shape reaches on large products (256 x 256: 1.30 PFLOP/s over the chip, 256 x 128
+    // 1.16, 128 x 128 1.07, 64 x 128 0.65) and a microsecond for the trip through an empty pipeline.
+    // 128 x 128 reaches its rate with two blocks on a compute unit: where the busiest unit gets an odd number of
+    // them, the last runs alone at 0.7 of the rate; so does 64 x 128 where every unit has one.  A chip with idle
+    // units runs the others faster (a third, were nearly all idle).  A shape is never taller than the rows need.
+    // Against the best of all shapes (and, for a branch's last product, cuts) in products of 1024 to 25600 by 1024 to
+    // 51200 with 80 to 2048 rows, measured one by one, what this picks is 1 % slower in the mean and 9 % at the
+    // most; a rule without the cuts of K for many rows and the factors for idle and odd units was 13 % and, with 400
+    // rows against 5120 x 25600, twice as slow (277 us in 128 x 128, 134 in three cuts of 256 x 128).
     const long cus = 256;
-    struct Shape { int tile, bm, bn; float rate; bool pairs; };
-    const Shape shapes[4] = {{64, 64, 128, 0.80f, true}, {128, 128, 128, 1.07f, true}, {256, 256, 128, 1.16f, false},
-                             {512, 256, 256, 1.30f, false}};
-    int tile = 0;
+    struct Shape { int tile, bm, bn; float rate, alone_first, alone_later; };
+    const Shape shapes[4] = {{64, 64, 128, 0.65f, 0.43f, 0.f}, {128, 128, 128, 1.07f, 0.43f, 0.43f},
+                             {256, 256, 128, 1.16f, 0.f, 0.f}, {512, 256, 256, 1.30f, 0.f, 0.f}};
+    const long cut = (long)qe_cdiv(qe_cdiv(K, splits), 64) * 64;
     float best = 0.f;
+    *tile = 0;
     for (const Shape& sh : shapes) {
         if (sh.tile != 64 && M <= sh.bm / 2) continue;
-        if (sh.tile == 512 && !with_256x256) continue;
         const long blocks = (long)qe_cdiv(M, sh.bm) * qe_cdiv(N, sh.bn) * splits;
         const long turns = qe_cdiv(blocks, cus);
-        const float alone = sh.pairs && turns >= 3 && turns % 2 ? 1.f / 0.7f - 1.f : 0.f;
-        const float cost = ((float)turns + alone) * sh.bm * sh.bn / sh.rate;
-        if (tile == 0 || cost < best) { tile = sh.tile; best = cost; }
+        const float alone = turns == 1 ? sh.alone_first : (turns % 2 ? sh.alone_later : 0.f);
+        const float busy = (float)blocks / (float)(turns * cus);
+        const float one = (float)(cut * sh.bm * sh.bn) * (2e-9f * (float)cus) / sh.rate;
+        const float cost = ((float)turns + alone) * (one * (0.65f + 0.35f * busy) + 1.f);
+        if (*tile == 0 || cost < best) { *tile = sh.tile; best = cost; }
     }
+    return best;
+}
+
+static int choose_tile(int M, int N, int K, int splits) {
+    int tile;
+    qe_gemm_mfma_shape(M, N, K, splits, &tile);
     return tile;
 }
 
@@ -716,7 +729,7 @@ static int pick_mfma(const void* x, const void* w, const float* bias, void* out,
     // 128 doubles that (24576 x 4096 against 64 rows: 44.4 us against 49.2; with two blocks a unit, 51200 x
     // 5120, it gains nothing).
     if (tile == 0 && SILU && M <= 64 && qe_cdiv(N, 128) <= 256) tile = 65;
-    if (tile == 0) tile = choose_tile(M, N, splits);
+    if (tile == 0) tile = choose_tile(M, N, K, splits);
     if (tile == 65) return launch_mfma<TO, 64, 128, 128, 4, 1, SILU>(x, w, bias, out, M, N, K, splits, stream);
     if (tile == 512) return launch_mfma<TO, 256, 256, 64, 4, 1, SILU>(x, w, bias, out, M, N, K, splits, stream);
     if (tile == 256) return launch_mfma<TO, 256, 128, 64, 8, 1, SILU>(x, w, bias, out, M, N, K, splits, stream);
@@ -761,8 +774,7 @@ int qe_gemm_qkv(const void* x, const void* w, const float* bias, int M, int K, i
     int lp = 0;
     while ((1 << lp) < P) ++lp;
     QkvTail tail{positions, slots, q_w, k_w, table, (bf16_t*)q_out, (bf16_t*)cache, eps, Hq, Hkv, P, lp};
-    // (the 256 x 256 shape has four waves for an epilogue over 65536 values: the others finish it sooner)
-    if (tile == 0) tile = choose_tile(M, N, 1, false);
+    if (tile == 0) tile = choose_tile(M, N, K, 1);
     if (tile == 512) return launch_mfma<bf16_t, 256, 256, 64, 4, 1, 0, true>(x, w, bias, nullptr, M, N, K, 1, stream, tail);
     if (tile == 256) return launch_mfma<bf16_t, 256, 128, 64, 8, 1, 0, true>(x, w, bias, nullptr, M, N, K, 1, stream, tail);
     if (tile == 128) return launch_mfma<bf16_t, 128, 128, 64, 4, 2, 0, true>(x, w, bias, nullptr, M, N, K, 1, stream, tail);

@@ -53,6 +53,20 @@ def test_tiled_gemm_covers_every_tile(ops, tile, M, N):
     assert torch.equal(parts[0] + parts[1] + parts[2], want)
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 1024, 1024), (80, 5120, 6400), (144, 256, 4096), (272, 640, 12288), (400, 1024, 2048), (528, 136, 3080),
+                                   (1300, 512, 2048), (2049, 1024, 1032)])
+def test_branch_products_in_as_many_cuts_as_asked_for(ops, M, N, K):
+    """The number of cuts that is asked for leaves every part some of K, is one the product takes, and its parts add up to
+    it, whole numbers far below 2^24 exactly."""
+    g = torch.Generator().manual_seed(M)
+    x = torch.randint(-3, 4, (M, K), generator=g).bfloat16().to(DEV)
+    w = torch.randint(-3, 4, (N, K), generator=g).bfloat16().to(DEV)
+    splits = ops.gemm_branch_splits(x, w)
+    got = ops.gemm(x, w, epilogue=ops.EPI_PARTIAL, splits=splits) if splits else ops.gemm(x, w, out_dtype=torch.float32)[None]
+    assert splits in range(7) and len(got) == max(splits, 1)
+    assert torch.equal(got.sum(0), x.float() @ w.float().t())
+
+
 def latent_rows(before, rows, R, dr, page, seed):
     """Requests with ``before`` cached tokens and ``rows`` new ones over scattered pages: (cache, table, positions, tok_seq, the
     requests' rows [keys, R + dr])."""
