@@ -91,10 +91,11 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
     // of one XCD take a compact part of the tiles, xcd_m parts down by xcd_n across (the host picks
     // the cut that makes the XCDs read the fewest rows of x and W altogether; 0: no cut into equal parts), so
     // that they share what they read through that L2.  (A single row of tiles shares nothing of W and goes as the blocks
-    // come; so do grouped rows.)
+    // come.)
     int tile_m, tile_n;
-    if (!tail.tiles && tiles_m > 1) {
-        int local, part_m = 0, part_n = 0, per_m = tiles_m, per_n = tiles_n;
+    const int rows_m = tail.tiles ? tail.n_tiles[0] : tiles_m;       // (grouped rows: the grid has blocks for the most tiles there can be)
+    if (rows_m > 1) {
+        int local, part_m = 0, part_n = 0, per_m = rows_m, per_n = tiles_n;
         const int xcd = blockIdx.x % 8;
         local = blockIdx.x / 8;
         if (xcd_m > 0) {
@@ -105,8 +106,9 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
         } else {
             // no cut into equal parts: each XCD takes an eighth of the walk below through all tiles (dealt out block by
             // block, every XCD read nearly all of W: 1600 rows against 5120 x 25600 in three cuts, 7 by 20 tiles of
-            // 256 x 256: 455 us, now 435)
-            const int all = gridDim.x, each = all / 8, over = all % 8;
+            // 256 x 256: 455 us, now 435; 8192 rows of 32 experts of 2048 x 2048: 137 us, now 122)
+            const int all = rows_m * tiles_n, each = all / 8, over = all % 8;
+            if (local >= each + (xcd < over)) return;
             local += xcd * each + min(xcd, over);
         }
         // Inside the part the tiles go in bands of 8 tile rows (the last band has what is left), across the band
@@ -120,11 +122,11 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
         tile_m = part_m + band * 8 + within % rows;
         tile_n = part_n + within / rows;
     } else {
-        tile_m = blockIdx.x % tiles_m;
-        tile_n = blockIdx.x / tiles_m;
+        tile_m = 0;
+        tile_n = blockIdx.x;
+        if (tile_n >= rows_m * tiles_n) return;
     }
     if (tail.tiles) {
-        if (tile_m >= tail.n_tiles[0]) return;
         const int expert = tail.tiles[3 * tile_m], first = tail.tiles[3 * tile_m + 1];
         if (SILU && tail.row_w) tail.perm += first;        // (from here on by the tile's own rows)
         M = tail.tiles[3 * tile_m + 2];
