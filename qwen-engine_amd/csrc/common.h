@@ -86,6 +86,9 @@ template <> struct Vec4<bf16_t> {
     }
 };
 
+// the exact gelu
+__device__ __forceinline__ float gelu_of(float v) { return 0.5f * v * (1.f + erff(v * 0.70710678118654752440f)); }
+
 // What the attention kernels do with a head's result o[0 .. D) before they store it: only the first dv numbers are
 // stored (a value head smaller than the common head size of the cache), head h of row t at out + t * out_stride +
 // h * dv; with a gate they are multiplied by sigmoid(gate[t * gate_stride + h * dv + d]) first, in 32-bit.  sink: per query

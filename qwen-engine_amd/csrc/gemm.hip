@@ -10,16 +10,16 @@ int qe_gemm_skinny(const void* x, const void* w, const float* bias, void* out, i
 bool qe_gemm_skinny_norm_ok(int M, int N, int K);
 int qe_gemm_skinny_splits(int N, int K);
 bool qe_gemm_mfma_ok(int M, int N, int K, int dt_a, int dt_w);
-float qe_gemm_mfma_shape(int M, int N, int K, int splits, int* tile);
+float qe_gemm_mfma_shape(int M, int N, int K, int splits, int* tile, bool largest = true);
 int qe_gemm_mfma(const void* x, const void* w, const float* bias, void* out, int M, int N, int K, int dt_o,
-                 int tile, bool silu, int splits, hipStream_t stream);
+                 int tile, bool silu, int splits, hipStream_t stream, bool gelu = false);
 
 int qe_gemm_qkv(const void* x, const void* w, const float* bias, int M, int K, int Hq, int Hkv, int P,
                 const int* positions, const int* slots, const float* q_w, const float* k_w, float eps,
                 const float* table, void* q_out, void* cache, int tile, hipStream_t stream);
 
 enum { ALGO_AUTO = 0, ALGO_GENERIC = 1, ALGO_MFMA = 2, ALGO_TILE = 1000 };   // ALGO_TILE + rows: the tiled kernel with that tile
-enum { EPI_STORE = 0, EPI_RESIDUAL = 1, EPI_SILU_MUL = 2, EPI_PARTIAL = 3, EPI_SILU_MUL_IL = 4 };
+enum { EPI_STORE = 0, EPI_RESIDUAL = 1, EPI_SILU_MUL = 2, EPI_PARTIAL = 3, EPI_SILU_MUL_IL = 4, EPI_GELU = 5 };
 
 // 1 if the fused epilogues (add into the 32-bit residual stream; silu(gate) * up) can be used
 extern "C" int qe_gemm_fused_supported(int M, int N, int K, int dt_a, int dt_w) {
@@ -50,6 +50,11 @@ extern "C" int qe_gemm_norm_preferred(int M, int N, int K, int dt_w, int n_delta
 // 1 if epilogue 4 (silu-mul over interleaved gate|up rows) can be used: N counts the outputs
 extern "C" int qe_gemm_silu_supported(int M, int N, int K, int dt_a, int dt_w) {
     return (N % 32 == 0 && (qe_gemm_skinny_ok(M, N, K, dt_a, dt_w) || qe_gemm_mfma_ok(M, 2 * N, K, dt_a, dt_w))) ? 1 : 0;
+}
+
+// 1 if epilogue 5 (the exact gelu) can be used
+extern "C" int qe_gemm_gelu_supported(int M, int N, int K, int dt_a, int dt_w) {
+    return (qe_gemm_skinny_ok(M, N, K, dt_a, dt_w) || qe_gemm_mfma_ok(M, N, K, dt_a, dt_w)) ? 1 : 0;
 }
 
 // More than 16 rows against a large matrix: the kernel for few rows, in which every wave reads the
@@ -116,6 +121,7 @@ extern "C" int qe_gemm_branch_splits(int M, int N, int K, int dt_a, int dt_w) {
 // 3: out is float [splits, M, N], partial products along K to be summed over the first index.
 // 4: as 2 with the gate and up rows of w interleaved in blocks of 32 (gate 0..31, up 0..31, ...);
 //    taken by the kernel for few rows and by the tiled one.
+// 5: out = gelu(product) in bfloat16, no bias; where qe_gemm_gelu_supported.
 // norm_w (or null): the weight of an RMSNorm (eps norm_eps) that stands before the product: x is then the
 // 32-bit stream [M, K]; needs qe_gemm_norm_supported and epilogue 0, 2 or 4.  With it, delta (or null):
 // n_delta float tensors [M, K] one after the other that are added to the stream's rows, in order, before
@@ -145,6 +151,11 @@ extern "C" int qe_gemm(const void* x, const void* w, const float* bias, void* ou
         QE_REQUIRE(N % 32 == 0 && qe_gemm_mfma_ok(M, 2 * N, K, dt_a, dt_w),
                    "gemm: M=%d N=%d K=%d is not taken by a silu-mul kernel", M, N, K);
         return qe_gemm_mfma(x, w, bias, out, M, 2 * N, K, dt_o, algo > ALGO_TILE ? algo - ALGO_TILE : 0, true, 1, stream);
+    }
+    if (epilogue == EPI_GELU) {
+        QE_REQUIRE(!bias && dt_o == QE_BF16 && (skinny || tiled), "gemm: M=%d N=%d K=%d is not taken by a gelu kernel", M, N, K);
+        if (!skinny || tiled_for_few_rows(M, N, K, dt_a, dt_w))
+            return qe_gemm_mfma(x, w, bias, out, M, N, K, dt_o, algo > ALGO_TILE ? algo - ALGO_TILE : 0, false, 1, stream, true);
     }
     if (epilogue == EPI_PARTIAL && (tiled_for_few_rows(M, N, K, dt_a, dt_w) || (!skinny && tiled))) {
         QE_REQUIRE(dt_o == QE_F32, "gemm: partial products are 32-bit");

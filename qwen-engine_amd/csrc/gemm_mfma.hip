@@ -75,6 +75,7 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const float* __restrict__ bias,
     TO* __restrict__ out, int M, int N, int K, int tiles_m, int tiles_n, int k_per_split, int xcd_m, int xcd_n,
     int rotate, QkvTail tail) {
+    constexpr bool PAIR = SILU > 0;
     constexpr int ROWB = BK * 2 + 16;       // bytes of a staged row
     constexpr int PPR = BK / 8;             // 16-byte pieces per row
     constexpr int RPI = 64 * NW / PPR;      // rows the block stages with one piece per thread
@@ -128,11 +129,11 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
     }
     if (tail.tiles) {
         const int expert = tail.tiles[3 * tile_m], first = tail.tiles[3 * tile_m + 1];
-        if (SILU && tail.row_w) tail.perm += first;        // (from here on by the tile's own rows)
+        if (PAIR && tail.row_w) tail.perm += first;        // (from here on by the tile's own rows)
         M = tail.tiles[3 * tile_m + 2];
         x += (long)first * K;
         w += (long)expert * N * K;
-        out += (long)first * (SILU ? N / 2 : N);
+        out += (long)first * (PAIR ? N / 2 : N);
         tile_m = 0;
     }
     const int m0 = tile_m * BM, n0 = tile_n * BN;
@@ -516,29 +517,29 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
         }
         return;
     }
-    const int NO = SILU ? N / 2 : N;                       // width of the output
-    constexpr int WNO = SILU ? WN / 2 : WN;                // output columns of a wave's strip
+    const int NO = PAIR ? N / 2 : N;                       // width of the output
+    constexpr int WNO = PAIR ? WN / 2 : WN;                // output columns of a wave's strip
     constexpr int ESZ = (int)sizeof(TO);
     constexpr int CH = 16 / ESZ;                           // outputs in 16 bytes
     constexpr int CPR = WNO / CH;                          // 16-byte chunks in a row of the strip
     constexpr int SROW = WNO * ESZ + 16;                   // bytes of a staged row
     static_assert(NW * 32 * SROW <= 2 * BUF, "the strips of the waves must fit the staging buffers");
     unsigned char* strip = smem + wave * 32 * SROW;
-    const int no0 = SILU ? (n0 + wn) / 2 : n0 + wn;        // first output column of the wave's strip
+    const int no0 = PAIR ? (n0 + wn) / 2 : n0 + wn;        // first output column of the wave's strip
     const bool vec_ok = (NO % CH) == 0 && (((unsigned long)out) & 15) == 0;
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
         __builtin_amdgcn_sched_barrier(0);   // one strip after the other: nothing of the next is computed early
         float row_w = 1.f;
-        if (SILU && tail.row_w) {
+        if (PAIR && tail.row_w) {
             const int m = wm + i * 32 + (lane & 31);       // (a grouped tile starts at row 0 of its rows)
             row_w = tail.row_w[tail.perm[m < M ? m : M - 1]];
         }
 #pragma unroll
-        for (int j = 0; j < NJ; j += (SILU ? 2 : 1))
+        for (int j = 0; j < NJ; j += (PAIR ? 2 : 1))
 #pragma unroll
             for (int bq = 0; bq < 4; ++bq) {
-                const int nl = (SILU ? j * 16 : j * 32) + 8 * bq + 4 * (lane >> 5);   // column within the strip
+                const int nl = (PAIR ? j * 16 : j * 32) + 8 * bq + 4 * (lane >> 5);   // column within the strip
                 float v[4], bg[4], bu[4];
                 if (SILU == 2) {                           // (columns beyond the output are never stored: any bias does)
                     const int ng = min(n0 + wn + j * 32 + 8 * bq + 4 * (lane >> 5), N - 36);
@@ -547,8 +548,8 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
                 }
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    if (SILU) {
-                        float gt = acc[i][j][4 * bq + r], up = acc[i][j + (SILU ? 1 : 0)][4 * bq + r];
+                    if (PAIR) {
+                        float gt = acc[i][j][4 * bq + r], up = acc[i][j + (PAIR ? 1 : 0)][4 * bq + r];
                         float slope = 1.f;
                         if (SILU == 2) { gt += bg[r]; up += bu[r]; }
                         if (tail.row_w) { gt *= row_w; up *= row_w; }
@@ -561,9 +562,10 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
                     } else {
                         v[r] = acc[i][j][4 * bq + r];
                         if (tail.relu_sq) { const float z = fmaxf(v[r], 0.f); v[r] = z * z; }
+                        if (SILU < 0) v[r] = gelu_of(v[r]);
                     }
                 }
-                if (!SILU && bias && blockIdx.y == 0) {                       // (a column beyond the output is never stored: any bias does)
+                if (!PAIR && bias && blockIdx.y == 0) {                       // (a column beyond the output is never stored: any bias does)
 #pragma unroll
                     for (int r = 0; r < 4; ++r) v[r] += bias[no0 + nl + r < NO ? no0 + nl + r : NO - 1];
                 }
@@ -686,7 +688,7 @@ extern "C" int qe_gemm_mfma_grouped_tile_rows() { return 128; }
 
 // The tile shape for a product in S cuts of K, and the microseconds it is taken to need (what the caller then does with
 // partial products left out).
-float qe_gemm_mfma_shape(int M, int N, int K, int splits, int* tile) {
+float qe_gemm_mfma_shape(int M, int N, int K, int splits, int* tile, bool largest = true) {
     // The busiest compute unit decides: its number of tiles (they are dealt out in turn) times what a tile costs, its
     // operations at the rate that the shape reaches on large products (256 x 256: 1.30 PFLOP/s over the chip, 256 x 128
     // 1.16, 128 x 128 1.07, 64 x 128 0.65) and a microsecond for the trip through an empty pipeline.
@@ -706,6 +708,7 @@ float qe_gemm_mfma_shape(int M, int N, int K, int splits, int* tile) {
     *tile = 0;
     for (const Shape& sh : shapes) {
         if (sh.tile != 64 && M <= sh.bm / 2) continue;
+        if (sh.tile == 512 && !largest) continue;
         const long blocks = (long)qe_cdiv(M, sh.bm) * qe_cdiv(N, sh.bn) * splits;
         const long turns = qe_cdiv(blocks, cus);
         const float alone = turns == 1 ? sh.alone_first : (turns % 2 ? sh.alone_later : 0.f);
@@ -717,9 +720,9 @@ float qe_gemm_mfma_shape(int M, int N, int K, int splits, int* tile) {
     return best;
 }
 
-static int choose_tile(int M, int N, int K, int splits) {
+static int choose_tile(int M, int N, int K, int splits, bool largest = true) {
     int tile;
-    qe_gemm_mfma_shape(M, N, K, splits, &tile);
+    qe_gemm_mfma_shape(M, N, K, splits, &tile, largest);
     return tile;
 }
 
@@ -730,8 +733,10 @@ static int pick_mfma(const void* x, const void* w, const float* bias, void* out,
     // cut): a block streams its weights alone on its unit, and what it has in flight bounds it.  A k step of
     // 128 doubles that (24576 x 4096 against 64 rows: 44.4 us against 49.2; with two blocks a unit, 51200 x
     // 5120, it gains nothing).
-    if (tile == 0 && SILU && M <= 64 && qe_cdiv(N, 128) <= 256) tile = 65;
-    if (tile == 0) tile = choose_tile(M, N, K, splits);
+    if (tile == 0 && SILU > 0 && M <= 64 && qe_cdiv(N, 128) <= 256) tile = 65;
+    // (the gelu of 65536 values is 35 us in which nothing else runs on the unit: 256 x 256 is never its shape; 3000 rows against
+    // 4096 x 1024: 65 us in it, 52 in 256 x 128, 47 in 128 x 128)
+    if (tile == 0) tile = choose_tile(M, N, K, splits, SILU >= 0);
     if (tile == 65) return launch_mfma<TO, 64, 128, 128, 4, 1, SILU>(x, w, bias, out, M, N, K, splits, stream);
     if (tile == 512) return launch_mfma<TO, 256, 256, 64, 4, 1, SILU>(x, w, bias, out, M, N, K, splits, stream);
     if (tile == 256) return launch_mfma<TO, 256, 128, 64, 8, 1, SILU>(x, w, bias, out, M, N, K, splits, stream);
@@ -743,8 +748,9 @@ static int pick_mfma(const void* x, const void* w, const float* bias, void* out,
 // by the shape.  silu: w is [N, K] with
 // gate and up rows interleaved in blocks of 32, out is [M, N / 2] = silu(gate) * up.
 // splits > 1: out is float [splits, M, N], partial products along K (no silu then).
+// gelu (without a bias, in bfloat16): out = gelu(product).
 int qe_gemm_mfma(const void* x, const void* w, const float* bias, void* out, int M, int N, int K, int dt_o,
-                 int tile, bool silu, int splits, hipStream_t stream) {
+                 int tile, bool silu, int splits, hipStream_t stream, bool gelu) {
     QE_REQUIRE(splits >= 1 && (splits == 1 || (!silu && dt_o == QE_F32)), "mfma gemm: partial products are 32-bit and plain");
     QE_REQUIRE(K % 8 == 0 && K >= 64 && K < (1 << 22), "mfma gemm: K=%d is no multiple of 8 in [64, 2^22)", K);
     QE_REQUIRE(tile == 0 || tile == 512 || tile == 256 || tile == 128 || tile == 64 || tile == 65, "mfma gemm: tile of %d rows", tile);
@@ -756,6 +762,10 @@ int qe_gemm_mfma(const void* x, const void* w, const float* bias, void* out, int
                         : pick_mfma<bf16_t, 1>(x, w, bias, out, M, N, K, tile, splits, stream);
         return bias ? pick_mfma<float, 2>(x, w, bias, out, M, N, K, tile, splits, stream)
                     : pick_mfma<float, 1>(x, w, bias, out, M, N, K, tile, splits, stream);
+    }
+    if (gelu) {
+        QE_REQUIRE(dt_o == QE_BF16 && !bias && splits == 1, "mfma gemm: gelu is stored in bfloat16, without a bias");
+        return pick_mfma<bf16_t, -1>(x, w, bias, out, M, N, K, tile, splits, stream);
     }
     if (dt_o == QE_BF16) return pick_mfma<bf16_t, 0>(x, w, bias, out, M, N, K, tile, splits, stream);
     return pick_mfma<float, 0>(x, w, bias, out, M, N, K, tile, splits, stream);

@@ -34,7 +34,7 @@
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float floatx4;
 
-enum { EPI_STORE = 0, EPI_RESIDUAL = 1, EPI_SILU_MUL = 2, EPI_PARTIAL = 3, EPI_SILU_MUL_IL = 4 };
+enum { EPI_STORE = 0, EPI_RESIDUAL = 1, EPI_SILU_MUL = 2, EPI_PARTIAL = 3, EPI_SILU_MUL_IL = 4, EPI_GELU = 5 };
 
 // The prologue of a product of few rows (M <= 16): the rows of the 32-bit stream hs [M][K], with the
 // n_delta partial products delta[s][M][K] of the branch before added in the order of s (the residual
@@ -490,6 +490,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(
             } else if (bias && blockIdx.y == 0) {
                 y += bias[n];
             }
+            if (EPI == EPI_GELU) y = gelu_of(y);
             if (EPI == EPI_PARTIAL) {
                 ((float*)out)[((long)blockIdx.y * M + t) * N + n] = y;
             } else if (EPI == EPI_RESIDUAL) {
@@ -618,6 +619,7 @@ int qe_gemm_skinny_splits(int N, int K) {
 // EPI_SILU_MUL: w is [2 N, K] (gate rows, then up rows), out [M, N] in dt_o.
 // EPI_SILU_MUL_IL: the same with gate and up rows interleaved in blocks of 32.
 // EPI_PARTIAL: out is float [splits, M, N]; the product is the sum over the first index.
+// EPI_GELU: out [M, N] = gelu(product), the exact gelu on the 32-bit sums, in bfloat16.
 // norm_w (or null): the weight of an RMSNorm that stands before the product; x is then the 32-bit
 // stream [M, K] and the rows are normed (eps norm_eps) before they are multiplied.  delta (or null):
 // n_delta partial products [n_delta][M][K] of the branch before, added to the stream's rows in
@@ -647,6 +649,10 @@ int qe_gemm_skinny(const void* x, const void* w, const float* bias, void* out, i
         QE_REQUIRE(N % 32 == 0, "skinny gemm: interleaved silu-mul takes N in blocks of 32");
         if (dt_o == QE_BF16) return launch_skinny<EPI_SILU_MUL_IL, bf16_t>(x, w, bias, out, M, N, K, 1, norm_w, norm_eps, delta, n_delta, h_out, stream);
         return launch_skinny<EPI_SILU_MUL_IL, float>(x, w, bias, out, M, N, K, 1, norm_w, norm_eps, delta, n_delta, h_out, stream);
+    }
+    if (epilogue == EPI_GELU) {
+        QE_REQUIRE(dt_o == QE_BF16 && !norm_w, "skinny gemm: gelu is stored in bfloat16, without a norm before");
+        return launch_skinny<EPI_GELU, bf16_t>(x, w, bias, out, M, N, K, 1, norm_w, norm_eps, delta, n_delta, h_out, stream);
     }
     QE_REQUIRE(epilogue == EPI_STORE, "skinny gemm: unknown epilogue %d", epilogue);
     if (dt_o == QE_BF16) return launch_skinny<EPI_STORE, bf16_t>(x, w, bias, out, M, N, K, 1, norm_w, norm_eps, delta, n_delta, h_out, stream);

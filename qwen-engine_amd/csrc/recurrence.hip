@@ -490,7 +490,7 @@ __global__ void unary_kernel(const TI* __restrict__ z, TO* __restrict__ y, long 
     if (i >= n) return;
     const float v = Elem<TI>::load(z + i);
     float r;
-    if (kind == 0) r = 0.5f * v * (1.f + erff(v * 0.70710678118654752440f));
+    if (kind == 0) r = gelu_of(v);
     else if (kind == 1) r = tanhf(v);
     else r = cap * tanhf(v / cap);
     Elem<TO>::store(y + i, r);

@@ -19,7 +19,7 @@ _DT = {torch.float32: F32, torch.bfloat16: BF16}
 
 ALGO_AUTO, ALGO_GENERIC, ALGO_FAST = 0, 1, 2
 ALGO_TILE = 1000   # ALGO_TILE + 256, 128 or 64: the tiled MFMA gemm with tiles of that many rows (+ 512: 256 x 256; + 65: 64 rows, k step 128)
-EPI_STORE, EPI_RESIDUAL, EPI_SILU_MUL, EPI_PARTIAL, EPI_SILU_MUL_IL = 0, 1, 2, 3, 4
+EPI_STORE, EPI_RESIDUAL, EPI_SILU_MUL, EPI_PARTIAL, EPI_SILU_MUL_IL, EPI_GELU = 0, 1, 2, 3, 4, 5
 DECODE_SPLIT_KEYS = 128   # keys per split of the decode attention kernel
 
 
@@ -78,6 +78,7 @@ def load_library():
         "qe_qk_rope_store_parts_supported": [i32, i32],
         "qe_gemm_partial_preferred": [i32, i32, i32, i32, i32],
         "qe_gemm_branch_splits": [i32, i32, i32, i32, i32],
+        "qe_gemm_gelu_supported": [i32, i32, i32, i32, i32],
         "qe_attention": [vp, vp, vp, vp, vp, vp, i32, vp, i32, i32, i32, i32, i32, f32, i32, i32, i32, f32, i32, vp],
         "qe_attention_tail": [vp, vp, vp, vp, vp, vp, i32, vp, i32, i32, i32, i32, i32, f32, i32, i32, i32, f32, i32,
                               i64, i32, vp, vp, i64, i32, vp],
@@ -481,6 +482,7 @@ def gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
     epilogue EPI_PARTIAL: the product is cut along K into ``splits`` (0: chosen for the shape)
     partial products, returned as float32 [splits, M, N]; their sum over the first index, taken
     in order, is the product.  All three need gemm_fused_supported(x, w).
+    epilogue EPI_GELU: the exact gelu of the 32-bit sums, in bfloat16, without a bias; needs gemm_gelu_supported(x, w).
 
     norm_weight (float32 [K]) with norm_eps: x is the 32-bit stream and the RMSNorm of its rows, rounded
     to bfloat16 as the norm kernel rounds it, is what is multiplied (out_dtype defaults to bfloat16);
@@ -642,6 +644,12 @@ def qk_rope_store(qkv: torch.Tensor, num_heads: int, num_kv_heads: int, head_dim
     return packed_out if packed else q_out
 
 
+def gemm_gelu_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """True if gemm(epilogue=EPI_GELU) takes these operands."""
+    lib = load_library()
+    return x.dtype in _DT and w.dtype in _DT and bool(lib.qe_gemm_gelu_supported(x.shape[0], w.shape[0], x.shape[1], _DT[x.dtype], _DT[w.dtype]))
+
+
 def gemm_branch_splits(x: torch.Tensor, w: torch.Tensor) -> int:
     """How a product whose result goes to a norm that adds it to the stream should be asked for:
     0 = plain, S >= 1 = gemm(..., epilogue=EPI_PARTIAL, splits=S), the S partial products being
@@ -650,6 +658,15 @@ def gemm_branch_splits(x: torch.Tensor, w: torch.Tensor) -> int:
     if x.dtype not in _DT or w.dtype not in _DT:
         return 0
     return int(lib.qe_gemm_branch_splits(x.shape[0], w.shape[0], x.shape[1], _DT[x.dtype], _DT[w.dtype]))
+
+
+def gemm_branch(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """A product that goes, in 32-bit, to a norm that adds it to the stream: float32 [S, T, N] partial products where that is
+    quicker (gemm_branch_splits), else float32 [T, N]."""
+    splits = gemm_branch_splits(x, w)
+    if splits:
+        return gemm(x, w, bias, epilogue=EPI_PARTIAL, splits=splits)
+    return gemm(x, w, bias, out_dtype=torch.float32)
 
 
 def gemm_splits_supported(x: torch.Tensor, w: torch.Tensor) -> bool:

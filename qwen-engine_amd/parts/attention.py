@@ -455,6 +455,7 @@ class ChunkAttention(PagedAttention):
     """
     takes_stream = False
     graph_safe = True        # every launch's grid follows the rows alone
+    hands_on_parts = True    # the output may be partial products (a mixer beside this one must then do the same)
 
     def __init__(self, spec, hidden_size: int):
         self.spec = spec
@@ -622,7 +623,7 @@ class ChunkAttention(PagedAttention):
                       v_dim=self.dv, gate=y[:, y.shape[1] - n:] if self.spec.output_gate else None, out=out)
 
     def forward(self, x: torch.Tensor, ctx, binding: CacheBinding) -> torch.Tensor:
-        """x [T, H] in the activation type.  Returns the mixer's output, float32 [T, H]."""
+        """x [T, H] in the activation type.  Returns the mixer's output, float32 [T, H] or partial products [S, T, H]."""
         if binding.kv is None:
             raise RuntimeError("attention was given no cache")
         y = ops.gemm(x, self.w_qkv, self.b_qkv)
@@ -633,7 +634,7 @@ class ChunkAttention(PagedAttention):
         else:
             o = torch.empty((x.shape[0], self.hq * self.dv), dtype=x.dtype, device=x.device)
             self.mix(y, None, ctx, binding, o)
-        return ops.gemm(o, self.w_o, self.b_o, out_dtype=torch.float32)
+        return ops.gemm_branch(o, self.w_o, self.b_o) if self.hands_on_parts else ops.gemm(o, self.w_o, self.b_o, out_dtype=torch.float32)
 
 
 register_part("paged_attention", PagedAttention)

@@ -82,7 +82,8 @@ class SwiGLU:
 
 class GeluMLP:
     """down(gelu(up x)), the exact gelu; the up product's result stays 32-bit until the activation has been applied
-    (one rounding), and the output is handed on in 32-bit for the residual sum."""
+    (one rounding; in the product's epilogue where its kernel has one), and the output is handed on in 32-bit for the
+    residual sum."""
 
     def __init__(self, spec, hidden_size: int):
         self.spec = spec
@@ -101,9 +102,11 @@ class GeluMLP:
         self.w_down = rt.place_matrix(tensors[down])
 
     def forward(self, x: torch.Tensor, ctx) -> torch.Tensor:
-        z = ops.gemm(x, self.w_up, out_dtype=torch.float32)
-        a = ops.unary(z, ops.UNARY_GELU, out_dtype=ctx.rt.dtype)
-        return ops.gemm(a, self.w_down, out_dtype=torch.float32)
+        if ops.gemm_gelu_supported(x, self.w_up):
+            a = ops.gemm(x, self.w_up, epilogue=ops.EPI_GELU)
+        else:
+            a = ops.unary(ops.gemm(x, self.w_up, out_dtype=torch.float32), ops.UNARY_GELU, out_dtype=ctx.rt.dtype)
+        return ops.gemm_branch(a, self.w_down)
 
 
 register_part("swiglu", SwiGLU)

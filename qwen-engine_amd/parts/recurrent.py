@@ -98,6 +98,7 @@ class DecayedLinearMixer:
     """``DecayedLinearSpec``: one product for q | k | v | gate, the recurrence with one decay per head (silu on q, k
     and v as they are read), all heads normed together, the sigmoid gate, the output projection."""
     graph_safe = True
+    hands_on_parts = True           # the output may be partial products (a mixer beside this one must then do the same)
 
     def __init__(self, spec, hidden_size: int):
         self.spec = spec
@@ -138,10 +139,10 @@ class DecayedLinearMixer:
         nk, nv = self.h * self.d, self.h * self.dv
         y = ops.gemm(x, self.w_in)
         o = ops.linear_recurrence(y[:, :nk], y[:, nk:2 * nk], y[:, 2 * nk:2 * nk + nv], binding.state, ctx.tok_seq,
-                                  self.h, decay=self.decay, silu=True, chunks=_chunks(ctx, self.h))
+                                  self.h, decay=self.decay, silu=True, chunks=_chunks(ctx, self.h), single_rows=ctx.single_rows)
         z = ops.gated_norm(o.view(T, nv), self.norm, self.eps, 1, ctx.rt.dtype, gate=y[:, 2 * nk + nv:],
                            gate_act=ops.GATE_SIGMOID)
-        return ops.gemm(z, self.w_o, out_dtype=torch.float32)
+        return ops.gemm_branch(z, self.w_o) if self.hands_on_parts else ops.gemm(z, self.w_o, out_dtype=torch.float32)
 
 
 class ForgetGateLinearMixer:
@@ -447,6 +448,11 @@ class SideBySideMixer:
         if not self.joint:
             for part, t in both:
                 part.load(t, rt)
+            # (partial products are added part by part: both mixers' output products must be cut alike, and products of one shape are)
+            alike = all(getattr(part, "hands_on_parts", False) for part, _ in both) and self.left.w_o.shape == self.right.w_o.shape
+            for part, _ in both:
+                if hasattr(part, "hands_on_parts"):
+                    part.hands_on_parts = alike
             return
         for part, t in both:
             part.load_own(t, rt)

@@ -145,3 +145,18 @@ def test_latent_attention_of_portions_with_expanded_keys(ops, R, dn, dr, dv, bef
     # by way of scores of a few units (the folded maps round queries, weights, latent sums and the result)
     print(f"expanded {off(out):.2e} folded {off(folded):.2e}")
     assert off(out) < 5e-3, (off(out), off(folded))
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 24, 128), (8, 4096, 1024), (16, 1000, 512), (17, 256, 64), (65, 192, 136), (300, 1160, 256),
+                                   (1100, 2304, 128)])
+def test_gelu_in_the_product(ops, M, N, K):
+    """The gelu on a product's 32-bit sums, by the kernel for few rows and in every tile shape."""
+    x, w = rand(M, K, seed=M).bfloat16(), rand(N, K, seed=N, scale=K ** -0.5).bfloat16()
+    assert ops.gemm_gelu_supported(x.to(DEV), w.to(DEV))
+    want = torch.nn.functional.gelu(x.double() @ w.double().t())
+    algos = [0] + ([ops.ALGO_TILE + t for t in (64, 128, 256, 512) if t < 256 or M > 128] if M > 64 else [])
+    for algo in algos:
+        got = ops.gemm(x.to(DEV), w.to(DEV), epilogue=ops.EPI_GELU, algo=algo)
+        assert got.dtype == torch.bfloat16
+        # (a bfloat16 rounding of the result, and sqrt(K) roundings of 2^-24 of sums of size one to three before it)
+        assert ((got.cpu().double() - want).abs() <= want.abs() * 2.0 ** -8 + 2.0 ** -22 * K ** 0.5).all(), algo
