@@ -42,13 +42,55 @@ __global__ void token_shift_kernel(const TA* __restrict__ x, const float* __rest
     }
 }
 
+// The same, four columns a thread and TS_COLS a block: everything a thread needs is asked for before the first of it is used
+// and before the state is written (few rows: a launch of T blocks that walked their rows two bytes at a time, waiting for the
+// state at every turn, took 19.8 us for eight rows of 2048; 5.2 us so).
+#define TS_COLS 256
+#define TS_BLENDS 8
+template <typename TA>
+__global__ __launch_bounds__(TS_COLS / 4) void token_shift_vec_kernel(const TA* __restrict__ x, const float* __restrict__ mu, int n,
+                                                                      float* __restrict__ state, long state_stride,
+                                                                      const int* __restrict__ tok_seq, TA* __restrict__ y, int T,
+                                                                      int W, int mode) {
+    const long t = blockIdx.x;
+    const int c = blockIdx.y * TS_COLS + threadIdx.x * 4;
+    if (c >= W) return;
+    const int seq = tok_seq[t];
+    float* st = state + (long)seq * state_stride + c;
+    float h[4], hp[4], m[TS_BLENDS][4];
+    Vec4<TA>::load(x + t * W + c, h);
+    if (mode == 2 || t == 0 || tok_seq[t - 1] != seq) Vec4<float>::load(st, hp);
+    else Vec4<TA>::load(x + (t - 1) * W + c, hp);
+#pragma unroll
+    for (int s = 0; s < TS_BLENDS; ++s) Vec4<float>::load(mu + (long)(s < n ? s : 0) * W + c, m[s]);
+#pragma unroll
+    for (int s = 0; s < TS_BLENDS; ++s) {
+        if (s >= n) break;
+        float o[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = fmaf(hp[e] - h[e], m[s][e], h[e]);
+        Vec4<TA>::store(y + ((long)s * T + t) * W + c, o);
+    }
+    if (mode == 2) Vec4<float>::store(st, h);
+}
+
 extern "C" int qe_token_shift(const void* x, const float* mu, int n, float* state, long state_stride,
                               const int* tok_seq, void* y, int T, int W, int single_rows, int dt_a,
                               hipStream_t stream) {
     QE_REQUIRE(T >= 0 && W > 0 && n > 0 && state_stride >= W, "token_shift: bad sizes");
     if (T == 0) return 0;
     const int threads = W >= 1024 ? 256 : (W >= 256 ? 128 : 64);
-#define QE_TS(TA_, mode_) token_shift_kernel<TA_><<<T, threads, 0, stream>>>((const TA_*)x, mu, n, state, state_stride, tok_seq, (TA_*)y, T, W, mode_)
+    // whole pieces of four everywhere, and blends that fit a thread's registers (mode 1 only copies a few rows)
+    const bool vec = W % 4 == 0 && state_stride % 4 == 0 && n <= TS_BLENDS && qe_cdiv(W, TS_COLS) <= 65535 &&
+                     (((uintptr_t)x | (uintptr_t)mu | (uintptr_t)state | (uintptr_t)y) & 15) == 0;
+#define QE_TS(TA_, mode_)                                                                                                 \
+    do {                                                                                                                  \
+        if (vec && mode_ != 1)                                                                                            \
+            token_shift_vec_kernel<TA_><<<dim3(T, qe_cdiv(W, TS_COLS)), TS_COLS / 4, 0, stream>>>(                        \
+                (const TA_*)x, mu, n, state, state_stride, tok_seq, (TA_*)y, T, W, mode_);                                \
+        else                                                                                                              \
+            token_shift_kernel<TA_><<<T, threads, 0, stream>>>((const TA_*)x, mu, n, state, state_stride, tok_seq, (TA_*)y, T, W, mode_); \
+    } while (0)
     if (dt_a == QE_F32) { if (single_rows) QE_TS(float, 2); else { QE_TS(float, 0); QE_TS(float, 1); } }
     else if (dt_a == QE_BF16) { if (single_rows) QE_TS(bf16_t, 2); else { QE_TS(bf16_t, 0); QE_TS(bf16_t, 1); } }
     else QE_REQUIRE(false, "token_shift: unknown element type %d", dt_a);
@@ -464,6 +506,60 @@ __global__ void gated_norm_kernel(const float* __restrict__ o, const float* __re
     }
 }
 
+// The same with the row in registers, NV pieces of four a thread of a block of 256, all asked for at once: one group a row, or
+// groups of 4 GL numbers that lie in GL neighbouring lanes (GL a power of two up to 64).  Eight rows of 2048: 9.9 us with the
+// kernel above, two walks of single numbers; 4.8 us so.
+template <typename TG, typename TO, int NV>
+__global__ __launch_bounds__(256) void gated_norm_regs_kernel(const float* __restrict__ o, const float* __restrict__ weight,
+                                                              const TG* __restrict__ gate, long gate_stride, int gate_act, float eps,
+                                                              float scale, TO* __restrict__ y, long y_stride, int N, int GL) {
+    __shared__ float red[16];
+    const long t = blockIdx.x;
+    float v[NV][4], w[NV][4], z[NV][4];
+    int at[NV];
+    bool ok[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int c = (threadIdx.x + i * 256) * 4;
+        ok[i] = c < N;
+        at[i] = ok[i] ? c : 0;
+        Vec4<float>::load(o + t * N + at[i], v[i]);
+        Vec4<float>::load(weight + at[i], w[i]);
+        if (gate) Vec4<TG>::load(gate + t * gate_stride + at[i], z[i]);
+    }
+    float all = 0.f, f[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        float a = 0.f;
+        if (ok[i]) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a = fmaf(v[i][e], v[i][e], a);
+        }
+        all += a;
+        if (GL > 0) {
+            for (int d = GL >> 1; d > 0; d >>= 1) a += __shfl_xor(a, d, 64);
+            f[i] = rsqrtf(a / (float)(4 * GL) + eps);
+        }
+    }
+    if (GL == 0) {
+        const float g = rsqrtf(block_sum(all, red) / (float)N + eps);
+#pragma unroll
+        for (int i = 0; i < NV; ++i) f[i] = g;
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        if (!ok[i]) continue;
+        float r[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            r[e] = v[i][e] * f[i] * w[i][e];
+            if (gate) r[e] *= gate_act == 1 ? silu_f(z[i][e]) : (gate_act == 2 ? sigmoid_f(z[i][e]) : z[i][e]);
+            r[e] *= scale;
+        }
+        Vec4<TO>::store(y + t * y_stride + at[i], r);
+    }
+}
+
 extern "C" int qe_gated_norm(const float* o, const float* weight, const void* gate, long gate_stride, int dt_g,
                              int gate_act, float eps, float scale, void* y, long y_stride, int dt_y, int T, int N,
                              int groups, hipStream_t stream) {
@@ -471,13 +567,24 @@ extern "C" int qe_gated_norm(const float* o, const float* weight, const void* ga
     QE_REQUIRE(y_stride >= N && (!gate || gate_stride >= N), "gated_norm: rows overlap");
     if (T == 0) return 0;
     const int threads = (groups >= 4 || N / groups >= 512) ? 256 : 64 * groups;   // (long groups: four waves share each)
-#define QE_GN(TG_, TO_) gated_norm_kernel<TG_, TO_><<<T, threads, 0, stream>>>(o, weight, (const TG_*)gate, gate_stride, gate_act, eps, scale, (TO_*)y, y_stride, N, groups)
+    const int GL = groups == 1 ? 0 : N / groups / 4;
+    const bool vec = N % (4 * groups) == 0 && N <= 8192 && (groups == 1 || (GL >= 1 && GL <= 64 && (GL & (GL - 1)) == 0)) &&
+                     y_stride % 4 == 0 && (!gate || gate_stride % 4 == 0) &&
+                     (((uintptr_t)o | (uintptr_t)weight | (uintptr_t)gate | (uintptr_t)y) & 15) == 0;
+#define QE_GN_ARGS(TG_, TO_) o, weight, (const TG_*)gate, gate_stride, gate_act, eps, scale, (TO_*)y, y_stride, N
+#define QE_GN(TG_, TO_)                                                                                          \
+    do {                                                                                                         \
+        if (vec && N <= 2048) gated_norm_regs_kernel<TG_, TO_, 2><<<T, 256, 0, stream>>>(QE_GN_ARGS(TG_, TO_), GL); \
+        else if (vec) gated_norm_regs_kernel<TG_, TO_, 8><<<T, 256, 0, stream>>>(QE_GN_ARGS(TG_, TO_), GL);      \
+        else gated_norm_kernel<TG_, TO_><<<T, threads, 0, stream>>>(QE_GN_ARGS(TG_, TO_), groups);               \
+    } while (0)
     const int dg = gate ? dt_g : dt_y;
     if (dg == QE_F32 && dt_y == QE_F32) QE_GN(float, float);
     else if (dg == QE_BF16 && dt_y == QE_BF16) QE_GN(bf16_t, bf16_t);
     else if (dg == QE_F32 && dt_y == QE_BF16) QE_GN(float, bf16_t);
     else QE_REQUIRE(false, "gated_norm: no kernel for gate type %d with output type %d", dt_g, dt_y);
 #undef QE_GN
+#undef QE_GN_ARGS
     QE_LAUNCH_CHECK();
     return 0;
 }

@@ -87,11 +87,10 @@ class ShiftedDecayMixer:
         r, k, v, gate = (ops.gemm(m[i], w) for i, w in enumerate((self.w_r, self.w_k, self.w_v, self.w_g)))
         low = ops.unary(ops.gemm(m[4], self.w_1, out_dtype=torch.float32), ops.UNARY_TANH, out_dtype=ctx.rt.dtype)
         decay_x = ops.gemm(low, self.w_2, out_dtype=torch.float32)      # (exponentials of the decay: in the recurrence, 32-bit)
-        o = ops.linear_recurrence(r, k, v, st[:, W:], ctx.tok_seq, self.h, decay_x=decay_x, decay_bias=self.w0,
-                                  bonus=self.u, chunks=_chunks(ctx, self.h))
-        y = ops.gated_norm(o.view(T, self.h * self.d), self.norm, self.eps, self.h, ctx.rt.dtype, gate=gate,
-                           gate_act=ops.GATE_SILU)
-        return ops.gemm(y, self.w_o, out_dtype=torch.float32)
+        y = ops.linear_recurrence(r, k, v, st[:, W:], ctx.tok_seq, self.h, decay_x=decay_x, decay_bias=self.w0,
+                                  bonus=self.u, chunks=_chunks(ctx, self.h), norm_weight=self.norm, norm_eps=self.eps,
+                                  norm_dtype=ctx.rt.dtype, single_rows=ctx.single_rows, gate=gate, gate_act=ops.GATE_SILU)
+        return ops.gemm_branch(y, self.w_o)
 
 
 class DecayedLinearMixer:

@@ -147,6 +147,10 @@ def test_latent_attention_of_portions_with_expanded_keys(ops, R, dn, dr, dv, bef
     assert off(out) < 5e-3, (off(out), off(folded))
 
 
+def rms_of(x):
+    return x / (x.square().mean(-1, keepdim=True) + 1e-5).sqrt()
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 24, 128), (8, 4096, 1024), (16, 1000, 512), (17, 256, 64), (65, 192, 136), (300, 1160, 256),
                                    (1100, 2304, 128)])
 def test_gelu_in_the_product(ops, M, N, K):
@@ -160,3 +164,39 @@ def test_gelu_in_the_product(ops, M, N, K):
         assert got.dtype == torch.bfloat16
         # (a bfloat16 rounding of the result, and sqrt(K) roundings of 2^-24 of sums of size one to three before it)
         assert ((got.cpu().double() - want).abs() <= want.abs() * 2.0 ** -8 + 2.0 ** -22 * K ** 0.5).all(), algo
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-6), (torch.bfloat16, 2.0 ** -8)])
+@pytest.mark.parametrize("W,n", [(4, 1), (20, 8), (256, 5), (260, 6), (1028, 9)])
+def test_token_shift_in_whole_pieces(ops, dtype, tol, W, n):
+    """Four columns a thread: columns that end inside a block's, one to nine blends (eight fit the registers), portions and
+    single rows, states that are not touched."""
+    mu = torch.rand(n, W, generator=torch.Generator().manual_seed(W))
+    state = torch.full((3, W + 4), 7.0, device=DEV)
+    first = rand(3, W, seed=n)
+    state[:, :W] = first.to(DEV)
+    prev = {s: first[s].double() for s in range(3)}
+    for lens, single in (((5, 0, 2), False), ((1, 0, 1), True), ((1, 0, 300), False)):
+        seq = sum(([s] * k for s, k in enumerate(lens)), [])
+        x = rand(len(seq), W, seed=len(seq)).to(dtype)
+        y = ops.token_shift(x.to(DEV), mu.to(DEV), state, torch.tensor(seq, dtype=torch.int32, device=DEV), single_rows=single)
+        for t, s in enumerate(seq):
+            h = x[t].double()
+            want = h + (prev[s] - h) * mu.double()
+            assert ((y[:, t].cpu().double() - want).abs() <= tol * (h.abs() + prev[s].abs()) + 1e-30).all(), (lens, t)
+            prev[s] = h
+    for s in range(3):
+        assert torch.equal(state[s, :W].cpu().double(), prev[s])
+    assert float(state[:, W:].min()) == 7.0
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.float32, 2e-6), (torch.bfloat16, 2.0 ** -8)])
+@pytest.mark.parametrize("N,groups", [(4, 1), (2048, 1), (2052, 1), (8192, 1), (8, 2), (96, 3), (2048, 16), (8192, 32), (2560, 10), (8196, 1)])
+def test_gated_norm_in_registers(ops, dtype, tol, N, groups):
+    """A row in registers: one group, groups of one to 64 lanes, rows that end inside a thread's pieces, the longest and one more."""
+    x, w, gate = rand(3, N, seed=N) * 3, 1 + 0.3 * rand(N, seed=1), rand(3, 2 * N + 8, seed=2).to(dtype)
+    off = -N % 8 + N                                       # (whole 16-byte pieces from the row's start)
+    gate = gate[:, off:off + N]
+    want = rms_of(x.double().view(3, groups, -1)).view(3, N) * w.double() * torch.nn.functional.silu(gate.double()) * 0.5
+    got = ops.gated_norm(x.to(DEV), w.to(DEV), 1e-5, groups, dtype, gate=gate.to(DEV), gate_act=ops.GATE_SILU, scale=0.5)
+    assert got.dtype == dtype and ((got.cpu().double() - want).abs() <= tol * want.abs() + 1e-7).all()
