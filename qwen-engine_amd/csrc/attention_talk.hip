@@ -319,6 +319,253 @@ __global__ __launch_bounds__(TALK_THREADS) void attention_talk_kernel(
     }
 }
 
+// ---- bfloat16 heads of up to 128 numbers -----------------------------------------------------------------------
+// What bounds a token here is the chain of a tile's steps, not what they read (64 keys of 4 heads of 128: 128 KB).  The
+// kernel above brings a tile through shared memory in stages, one after the other, each a trip to memory long (eight
+// stages there: 42 us a token and tile).  Here 16 waves hold a whole tile in registers: a wave takes one key/value head and
+// 16, 32 or 64 of the tile's keys, 16 at a time, LPK lanes a key with 16 bytes each, for the keys and later, with the same
+// lanes, for the values; the values and the next tile's keys are
+// on their way before the softmax.  A key row in registers serves all its query heads; the lanes of a key add up by halving.  Each lane keeps its
+// sums over its keys, for eight columns of every query head, to the end; there the lanes, then the waves add theirs
+// in a fixed order.  8 tokens over up to 250 keys, 16 heads of 128 on 4 (a tile a block): 15 us against 43; 1826 rows of
+// prompts of 235 keys: 174 us against 474 of the kernel with four rows a block.
+struct TalkWideLayout { int sc, pm, small, tk, part, total; };
+
+__host__ __device__ __forceinline__ TalkWideLayout talk_wide_layout(int Hq, int DP, int wph) {
+    TalkWideLayout L;
+    L.sc = Hq * DP;                                        // (the queries come first)
+    L.pm = L.sc + Hq * 64;
+    L.part = L.pm + Hq * 64;
+    L.small = L.part + wph * Hq * DP;
+    L.tk = L.small + 3 * Hq;
+    L.total = L.tk + Hq * Hq;
+    return L;
+}
+
+template <int LPK, int GM, int SHIFT>
+__global__ __launch_bounds__(1024) void attention_talk_wide_kernel(
+    const bf16_t* __restrict__ q, bf16_t* __restrict__ out, long out_stride, float out_scale, const bf16_t* __restrict__ cache,
+    const int* __restrict__ positions, const int* __restrict__ tok_seq, const int* __restrict__ block_table,
+    int max_blocks, const int* __restrict__ tokens, const float* __restrict__ bias, int bias_rows,
+    const float* __restrict__ talk, int Hq, int Hkv, int Dk, int Dv, int Dc, int P, float scale, int window,
+    int KS, float* __restrict__ ws) {
+    constexpr int DP = LPK * 8, NK = 64 / LPK, I = 16 / NK;      // keys a load of the wave, loads for 16 keys
+    extern __shared__ __align__(16) float sm[];
+    constexpr int wph = 1 << SHIFT, passes = 4 >> SHIFT;         // waves a key/value head, and sixteens of keys a wave
+    const TalkWideLayout L = talk_wide_layout(Hq, DP, wph);
+    float* qs = sm;
+    float* sc = sm + L.sc;
+    float* pm = sm + L.pm;
+    float* part = sm + L.part;
+    float* ml = sm + L.small;
+    float* al = ml + 2 * Hq;
+    float* tk = sm + L.tk;
+    const long t = tokens ? tokens[blockIdx.x] : blockIdx.x;
+    const int split = blockIdx.y;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int G = Hq / Hkv;
+    const int p = positions[t];
+    const int lo = first_seen_key(p, window);
+    const int* bt = block_table + (long)tok_seq[t] * max_blocks;
+    const long page_stride = 2L * Hkv * P * Dc, plane = (long)Hkv * P * Dc;
+    const int kvh = wave >> SHIFT, sub = wave & (wph - 1);
+    const bool works = kvh < Hkv;                          // (a wave beyond the heads helps with the softmax alone)
+    const int col = (lane & (LPK - 1)) * 8, lg = lane / LPK;
+    const int k_first = sub * (64 >> SHIFT);           // the wave's first key of a tile
+    // the key whose score this lane holds after the lanes of a key have added up
+    const int own = (I == 4 ? (lane & 1) * 2 + (lane >> 1 & 1) : (lane & 1)) * NK + lg;
+    const bool writes = (lane & (LPK - 1)) < I;
+    const bf16_t* mine = cache + (long)kvh * P * Dc + col;
+
+    long off[I];
+    uint4 kr[I], vr[I];
+    float bb[GM];
+    // where the 16 keys from j on lie (-1: not seen, or a column beyond the row)
+    auto locate = [&](int j) {
+#pragma unroll
+        for (int i = 0; i < I; ++i) {
+            const int jj = j + i * NK + lg;
+            off[i] = works && jj <= p && col < Dc ? (long)bt[jj / P] * page_stride + (long)(jj % P) * Dc : -1L;
+        }
+    };
+    auto load = [&](uint4 (&r)[I], long from) {
+#pragma unroll
+        for (int i = 0; i < I; ++i) r[i] = off[i] >= 0 ? *(const uint4*)(mine + off[i] + from) : make_uint4(0u, 0u, 0u, 0u);
+    };
+    // (a key's numbers count in whole fours up to Dk: what lies in its row beyond them does not)
+    const unsigned keep_lo = col < Dk ? ~0u : 0u, keep_hi = col + 4 < Dk ? ~0u : 0u;
+    auto load_bias = [&](int j) {
+        const int n = p - (j + own);
+#pragma unroll
+        for (int g = 0; g < GM; ++g)
+            bb[g] = bias && works && writes && n >= 0 && g < G ? bias[(long)(n < bias_rows ? n : bias_rows - 1) * Hq + kvh * G + g] : 0.f;
+    };
+
+    int j0 = lo + 64 * split;
+    if (j0 <= p) {
+        locate(j0 + k_first);
+        load(kr, 0);
+        load_bias(j0 + k_first);
+    }
+    for (int i = tid; i < Hq * DP; i += 1024) {
+        const int h = i / DP, d = i % DP;
+        qs[i] = d < Dk ? bf16_to_float(q[(t * Hq + h) * Dc + d]) : 0.f;
+    }
+    if (talk) for (int i = tid; i < Hq * Hq; i += 1024) tk[i] = talk[i];
+    for (int h = tid; h < Hq; h += 1024) { ml[2 * h] = -INFINITY; ml[2 * h + 1] = 0.f; }
+    float acc[GM][8];
+#pragma unroll
+    for (int g = 0; g < GM; ++g)
+#pragma unroll
+        for (int c = 0; c < 8; ++c) acc[g][c] = 0.f;
+    __syncthreads();
+
+    for (; j0 <= p; j0 += 64 * KS) {
+        const int jn = j0 + 64 * KS;
+        // ---- scores
+        for (int ps = 0; ps < passes; ++ps) {
+            const int at = k_first + ps * 16;
+            if (ps > 0) {
+                locate(j0 + at);
+                load(kr, 0);
+                load_bias(j0 + at);
+            }
+#pragma unroll
+            for (int i = 0; i < I; ++i) kr[i] = make_uint4(kr[i].x & keep_lo, kr[i].y & keep_lo, kr[i].z & keep_hi, kr[i].w & keep_hi);
+            if (works) {
+#pragma unroll
+                for (int g = 0; g < GM; ++g) {
+                    if (g >= G) continue;
+                    const float4 qa = *(const float4*)(qs + (kvh * G + g) * DP + col), qb = *(const float4*)(qs + (kvh * G + g) * DP + col + 4);
+                    float d[I];
+#pragma unroll
+                    for (int i = 0; i < I; ++i) {
+                        float x = qa.x * bf16_bits_to_float(kr[i].x & 0xffffu);
+                        x = fmaf(qa.y, bf16_bits_to_float(kr[i].x >> 16), x);
+                        x = fmaf(qa.z, bf16_bits_to_float(kr[i].y & 0xffffu), x);
+                        x = fmaf(qa.w, bf16_bits_to_float(kr[i].y >> 16), x);
+                        x = fmaf(qb.x, bf16_bits_to_float(kr[i].z & 0xffffu), x);
+                        x = fmaf(qb.y, bf16_bits_to_float(kr[i].z >> 16), x);
+                        x = fmaf(qb.z, bf16_bits_to_float(kr[i].w & 0xffffu), x);
+                        d[i] = fmaf(qb.w, bf16_bits_to_float(kr[i].w >> 16), x);
+                    }
+                    float r;
+                    const bool b0 = lane & 1, b1 = lane & 2;
+                    if (I == 4) {
+                        const float r0 = (b0 ? d[I - 2] : d[0]) + __shfl_xor(b0 ? d[0] : d[I - 2], 1);
+                        const float r1 = (b0 ? d[I - 1] : d[1]) + __shfl_xor(b0 ? d[1] : d[I - 1], 1);
+                        r = (b1 ? r1 : r0) + __shfl_xor(b1 ? r0 : r1, 2);
+                    } else {
+                        r = (b0 ? d[1] : d[0]) + __shfl_xor(b0 ? d[0] : d[1], 1);
+                        r += __shfl_xor(r, 2);
+                    }
+                    r += __shfl_xor(r, 4);
+                    if (LPK == 16) r += __shfl_xor(r, 8);
+                    if (writes) sc[(kvh * G + g) * 64 + at + own] = r * scale + bb[g];
+                    __builtin_amdgcn_sched_barrier(0);       // (a head after the other: together they want more registers than there are)
+                }
+            }
+        }
+        if (passes == 1) {
+            load(vr, plane);
+            if (jn <= p) {
+                locate(jn + k_first);
+                load(kr, 0);
+                load_bias(jn + k_first);
+            }
+        }
+        __syncthreads();
+        // ---- the heads' scores mixed, then the tile joins each head's running softmax
+        const bool seen = j0 + lane <= p;
+        for (int h = wave; h < Hq; h += 16) {
+            float sv;
+            if (talk) {
+                sv = 0.f;
+#pragma unroll 4
+                for (int g = 0; g < Hq; ++g) sv = fmaf(tk[h * Hq + g], sc[g * 64 + lane], sv);
+            } else {
+                sv = sc[h * 64 + lane];
+            }
+            if (!seen) sv = -INFINITY;
+            const float m_old = ml[2 * h], l_old = ml[2 * h + 1];
+            const float m_new = fmaxf(m_old, wave_max(sv));          // finite: key j0 is always seen
+            const float a = expf(m_old - m_new);                     // exp(-inf) = 0 on the first tile
+            const float pj = seen ? expf(sv - m_new) : 0.f;
+            const float l_new = l_old * a + wave_sum(pj);
+            pm[h * 64 + lane] = pj;
+            if (lane == 0) { ml[2 * h] = m_new; ml[2 * h + 1] = l_new; al[h] = a; }
+        }
+        __syncthreads();
+        // ---- the values (unseen keys: zeros with weight zero)
+        for (int ps = 0; ps < passes; ++ps) {
+            const int at = k_first + ps * 16;
+            if (passes > 1) {
+                locate(j0 + at);
+                load(vr, plane);
+            }
+            if (works) {
+#pragma unroll
+                for (int g = 0; g < GM; ++g) {
+                    if (g >= G) continue;
+                    const int h = kvh * G + g;
+                    const float f = ps == 0 ? al[h] : 1.f;
+#pragma unroll
+                    for (int c = 0; c < 8; ++c) acc[g][c] *= f;
+#pragma unroll
+                    for (int i = 0; i < I; ++i) {
+                        const float w = pm[h * 64 + at + i * NK + lg];
+                        acc[g][0] = fmaf(w, bf16_bits_to_float(vr[i].x & 0xffffu), acc[g][0]);
+                        acc[g][1] = fmaf(w, bf16_bits_to_float(vr[i].x >> 16), acc[g][1]);
+                        acc[g][2] = fmaf(w, bf16_bits_to_float(vr[i].y & 0xffffu), acc[g][2]);
+                        acc[g][3] = fmaf(w, bf16_bits_to_float(vr[i].y >> 16), acc[g][3]);
+                        acc[g][4] = fmaf(w, bf16_bits_to_float(vr[i].z & 0xffffu), acc[g][4]);
+                        acc[g][5] = fmaf(w, bf16_bits_to_float(vr[i].z >> 16), acc[g][5]);
+                        acc[g][6] = fmaf(w, bf16_bits_to_float(vr[i].w & 0xffffu), acc[g][6]);
+                        acc[g][7] = fmaf(w, bf16_bits_to_float(vr[i].w >> 16), acc[g][7]);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+        }
+        if (passes > 1 && jn <= p) {
+            locate(jn + k_first);
+            load(kr, 0);
+            load_bias(jn + k_first);
+        }
+    }
+    // ---- the lanes of a column, then the waves of a head
+    if (works) {
+#pragma unroll
+        for (int g = 0; g < GM; ++g) {
+            if (g >= G) continue;
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                float a = acc[g][c];
+#pragma unroll
+                for (int x = LPK; x < 64; x *= 2) a += __shfl_xor(a, x);
+                acc[g][c] = a;
+            }
+            if (lg == 0) {
+                float* o = part + ((long)sub * Hq + kvh * G + g) * DP + col;
+                *(float4*)o = make_float4(acc[g][0], acc[g][1], acc[g][2], acc[g][3]);
+                *(float4*)(o + 4) = make_float4(acc[g][4], acc[g][5], acc[g][6], acc[g][7]);
+            }
+        }
+    }
+    __syncthreads();
+    const int n_out = Hq * Dv;
+    float* w = KS > 1 ? ws + ((long)blockIdx.x * KS + split) * (2 * Hq + n_out) : nullptr;
+    if (KS > 1) for (int i = tid; i < 2 * Hq; i += 1024) w[i] = ml[i];
+    for (int i = tid; i < Hq * DP; i += 1024) {
+        const int h = i / DP, d = i % DP;
+        if (d >= Dv) continue;
+        float a = part[i];
+        for (int s = 1; s < wph; ++s) a += part[s * Hq * DP + i];
+        if (KS > 1) w[2 * Hq + h * Dv + d] = a;
+        else Elem<bf16_t>::store(out + t * out_stride + h * Dv + d, a * (out_scale / ml[2 * h + 1]));
+    }
+}
+
 // ---- several rows a block ------------------------------------------------------------------------------------
 // For portions of prompts: a block takes R neighbouring rows of the flat batch.  Rows of one request whose first seen
 // key is the same (one chunk, or no window) are walked together over the keys up to the last row's position, so that
@@ -574,7 +821,9 @@ __global__ __launch_bounds__(TALK_THREADS) void attention_talk_rows_kernel(
     }
 }
 
-// grid (tokens): the splits' partial results weighed by exp(m_s - max m) and added in the order of the splits
+// grid (tokens, 256 outputs each): the splits' partial results weighed by exp(m_s - max m) and added in the order of the
+// splits.  Bound by its one trip to memory: a thread an output, with all its splits' numbers asked for together (8 tokens of
+// 2048 numbers in 8 splits: 4.6 us against 28 with a block a token, each thread going through eight outputs split by split).
 template <typename TA>
 __global__ __launch_bounds__(TALK_THREADS) void attention_talk_merge_kernel(
     const float* __restrict__ ws, TA* __restrict__ out, long out_stride, float out_scale,
@@ -582,18 +831,30 @@ __global__ __launch_bounds__(TALK_THREADS) void attention_talk_merge_kernel(
     const long t = tokens ? tokens[blockIdx.x] : blockIdx.x;
     const int n_out = Hq * Dv, rec = 2 * Hq + n_out;
     const float* w = ws + (long)blockIdx.x * KS * rec;
-    for (int o = threadIdx.x; o < n_out; o += TALK_THREADS) {
-        const int h = o / Dv;
-        float m = -INFINITY;
-        for (int s = 0; s < KS; ++s) m = fmaxf(m, w[(long)s * rec + 2 * h]);
-        float l = 0.f, a = 0.f;
-        for (int s = 0; s < KS; ++s) {
-            const float f = expf(w[(long)s * rec + 2 * h] - m);          // (a split without keys: exp(-inf) = 0)
-            l = fmaf(w[(long)s * rec + 2 * h + 1], f, l);
-            a = fmaf(w[(long)s * rec + 2 * Hq + o], f, a);
-        }
-        Elem<TA>::store(out + t * out_stride + o, a / l * out_scale);
+    const int o = blockIdx.y * TALK_THREADS + threadIdx.x;
+    if (o >= n_out) return;
+    const int h = o / Dv;
+    float ms[TALK_MAX_SPLITS], ls[TALK_MAX_SPLITS], as[TALK_MAX_SPLITS];
+    float m = -INFINITY;
+#pragma unroll
+    for (int s = 0; s < TALK_MAX_SPLITS; ++s) {
+        const float* r = w + (long)min(s, KS - 1) * rec;
+        ms[s] = r[2 * h];
+        ls[s] = r[2 * h + 1];
+        as[s] = r[2 * Hq + o];
     }
+#pragma unroll
+    for (int s = 0; s < TALK_MAX_SPLITS; ++s) m = fmaxf(m, ms[s]);
+    float l = 0.f, a = 0.f;
+#pragma unroll
+    for (int s = 0; s < TALK_MAX_SPLITS; ++s) {
+        if (s < KS) {
+            const float f = expf(ms[s] - m);                         // (a split without keys: exp(-inf) = 0)
+            l = fmaf(ls[s], f, l);
+            a = fmaf(as[s], f, a);
+        }
+    }
+    Elem<TA>::store(out + t * out_stride + o, a / l * out_scale);
 }
 
 // Into how many blocks a token's key tiles are dealt: none while the tokens alone fill the machine, else a split for
@@ -640,6 +901,34 @@ extern "C" int qe_attention_talk(const void* q, void* out, long out_stride, floa
     const size_t shmem = (size_t)L.total * sizeof(float);
     QE_REQUIRE(shmem <= 150 * 1024, "talking attention: %zu bytes of shared memory", shmem);
     dim3 grid(n_tokens, splits);
+    // bfloat16 heads of up to 128 numbers in rows of whole 16-byte pieces, up to 16 key/value heads of up to 8 queries
+    // each: a tile in registers
+    {
+        const int d = Dk > Dv ? Dk : Dv, G = Hq / Hkv;
+        const int wph_shift = Hkv <= 4 ? 2 : (Hkv <= 8 ? 1 : 0);
+        const int DP = d <= 64 ? 64 : 128;
+        const size_t bytes = (size_t)talk_wide_layout(Hq, DP, 1 << wph_shift).total * sizeof(float);
+        if (dt_a == QE_BF16 && d <= 128 && Dc % 8 == 0 && ((unsigned long)cache & 15) == 0 && Hkv <= 16 && G <= 8 && bytes <= 150 * 1024) {
+#define QE_TALK_WIDE3(LPK_, GM_, SH_)                                                                                      \
+    do {                                                                                                             \
+        if (bytes > 48 * 1024)                                                                                       \
+            (void)hipFuncSetAttribute((const void*)attention_talk_wide_kernel<LPK_, GM_, SH_>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes); \
+        attention_talk_wide_kernel<LPK_, GM_, SH_><<<grid, 1024, bytes, stream>>>(                                        \
+            (const bf16_t*)q, (bf16_t*)out, out_stride, out_scale, (const bf16_t*)cache, positions, tok_seq, block_table, \
+            max_blocks, tokens, bias, bias_rows, talk, Hq, Hkv, Dk, Dv, Dc, P, scale, window, splits, ws); \
+    } while (0)
+#define QE_TALK_WIDE(LPK_, GM_) do { if (wph_shift == 2) QE_TALK_WIDE3(LPK_, GM_, 2); else if (wph_shift == 1) QE_TALK_WIDE3(LPK_, GM_, 1); else QE_TALK_WIDE3(LPK_, GM_, 0); } while (0)
+            if (DP == 64) { if (G <= 4) QE_TALK_WIDE(8, 4); else QE_TALK_WIDE(8, 8); }
+            else { if (G <= 4) QE_TALK_WIDE(16, 4); else QE_TALK_WIDE(16, 8); }
+#undef QE_TALK_WIDE
+#undef QE_TALK_WIDE3
+            if (splits > 1)
+                attention_talk_merge_kernel<bf16_t><<<dim3(n_tokens, qe_cdiv(Hq * Dv, TALK_THREADS)), TALK_THREADS, 0, stream>>>(
+                    ws, (bf16_t*)out, out_stride, out_scale, tokens, Hq, Dv, splits);
+            QE_LAUNCH_CHECK();
+            return 0;
+        }
+    }
     // many rows (portions of prompts): several neighbouring rows a block, where shared memory holds their scores
     const int R = TALK_ROWS;
     const TalkRowsLayout LR = talk_rows_layout(L, R, Hq);
@@ -654,7 +943,7 @@ extern "C" int qe_attention_talk(const void* q, void* out, long out_stride, floa
             (const TA_*)q, (TA_*)out, out_stride, out_scale, (const TA_*)cache, positions, tok_seq, block_table,     \
             max_blocks, n_tokens, bias, bias_rows, talk, Hq, Hkv, Dk, Dv, Dc, P, scale, window, splits, hgk, kps_shift, ws); \
         if (splits > 1)                                                                                              \
-            attention_talk_merge_kernel<TA_><<<n_tokens, TALK_THREADS, 0, stream>>>(ws, (TA_*)out, out_stride,       \
+            attention_talk_merge_kernel<TA_><<<dim3(n_tokens, qe_cdiv(Hq * Dv, TALK_THREADS)), TALK_THREADS, 0, stream>>>(ws, (TA_*)out, out_stride,       \
                                                                                     out_scale, tokens, Hq, Dv, splits); \
     } while (0)
 #define QE_TALK2(TA_, NV_)                                                                                           \
@@ -665,7 +954,7 @@ extern "C" int qe_attention_talk(const void* q, void* out, long out_stride, floa
             (const TA_*)q, (TA_*)out, out_stride, out_scale, (const TA_*)cache, positions, tok_seq, block_table,     \
             max_blocks, tokens, bias, bias_rows, talk, Hq, Hkv, Dk, Dv, Dc, P, scale, window, splits, hgk, kps_shift, ws); \
         if (splits > 1)                                                                                              \
-            attention_talk_merge_kernel<TA_><<<n_tokens, TALK_THREADS, 0, stream>>>(ws, (TA_*)out, out_stride,       \
+            attention_talk_merge_kernel<TA_><<<dim3(n_tokens, qe_cdiv(Hq * Dv, TALK_THREADS)), TALK_THREADS, 0, stream>>>(ws, (TA_*)out, out_stride,       \
                                                                                     out_scale, tokens, Hq, Dv, splits); \
     } while (0)
 #define QE_TALK(TA_) do { if (rows) QE_TALK_ROWS(TA_); else if (nv == 8) QE_TALK2(TA_, 8); else QE_TALK2(TA_, 16); } while (0)

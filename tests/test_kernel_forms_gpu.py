@@ -200,3 +200,40 @@ def test_gated_norm_in_registers(ops, dtype, tol, N, groups):
     want = rms_of(x.double().view(3, groups, -1)).view(3, N) * w.double() * torch.nn.functional.silu(gate.double()) * 0.5
     got = ops.gated_norm(x.to(DEV), w.to(DEV), 1e-5, groups, dtype, gate=gate.to(DEV), gate_act=ops.GATE_SILU, scale=0.5)
     assert got.dtype == dtype and ((got.cpu().double() - want).abs() <= tol * want.abs() + 1e-7).all()
+
+
+@pytest.mark.parametrize("hkv,G,dk,dv,dc,window", [(1, 1, 8, 8, 8, -100), (1, 8, 64, 64, 64, 0), (3, 2, 12, 20, 24, -1024), (4, 4, 128, 128, 128, -600),
+                                                   (5, 3, 100, 128, 128, 70), (8, 8, 128, 64, 128, -300), (16, 1, 72, 4, 80, 0),
+                                                   (16, 2, 64, 64, 64, -200)])
+def test_talking_heads_in_registers(ops, hkv, G, dk, dv, dc, window):
+    """A tile of keys in registers: one to sixteen key/value heads (four, two or one wave each) of one to eight queries, heads
+    that end inside a lane's piece, windows, chunks and neither, tokens with keys in one tile and in several splits.  What
+    lies behind a token's keys or beyond a row's numbers is not a number and must not be used."""
+    hq, P, L = hkv * G, 16, 700
+    q = rand(L, hq, dc, seed=hq).bfloat16()
+    k, v = rand(L, hkv, dc, seed=dk).bfloat16(), rand(L, hkv, dc, seed=dv + 1).bfloat16()
+    talk, bias = torch.eye(hq) + 0.3 * rand(hq, hq, seed=3) / hq ** 0.5, rand(40, hq, seed=4)
+    pages = -(-L // P)
+    order = torch.randperm(pages + 3, generator=torch.Generator().manual_seed(5))[:pages]
+    cache = torch.full((pages + 3, 2, hkv, P, dc), float("nan"), dtype=torch.bfloat16)
+    last = 650
+    kk = k.clone()
+    kk[:, :, (dk + 3) // 4 * 4:] = float("nan")
+    kk[:, :, dk:(dk + 3) // 4 * 4] = 0
+    for j in range(last + 1):
+        cache[order[j // P], 0, :, j % P] = kk[j]
+        cache[order[j // P], 1, :, j % P, :dv] = v[j, :, :dv]
+    pos = [0, 1, 15, 63, 64, 65, 199, 200, 299, 511, 599, 600, last]
+    kw = dict(window=window) if window >= 0 else dict(chunk=-window)
+    got = ops.attention_talk(q[pos].to(DEV), cache.to(DEV), torch.tensor(pos, dtype=torch.int32, device=DEV),
+                             torch.zeros(len(pos), dtype=torch.int32, device=DEV), order.int()[None].to(DEV), dk ** -0.5, dk, dv,
+                             bias=bias.to(DEV), talk=talk.to(DEV), **kw).cpu().double().view(len(pos), hq, dv)
+    for i, p in enumerate(pos):
+        lo = max(0, p - window + 1) if window > 0 else (p // -window * -window if window < 0 else 0)
+        kd, vd = k[lo:p + 1, :, :dk].double(), v[lo:p + 1, :, :dv].double()
+        s = torch.stack([kd[:, h // G] @ q[p, h, :dk].double() for h in range(hq)]) * dk ** -0.5
+        s = talk.double() @ (s + bias.double()[(p - torch.arange(lo, p + 1)).clamp(max=39)].t())
+        w = torch.softmax(s, -1)
+        want = torch.stack([w[h] @ vd[:, h // G] for h in range(hq)])
+        # (a bfloat16 rounding of each result; the scores' own errors, some 2^-20, move the weights by as much)
+        assert ((got[i] - want).abs() <= want.abs() * 2.0 ** -8 + 2.0 ** -17 * vd.abs().max()).all(), p
