@@ -3,25 +3,68 @@
 // of one wave (see attention_tile.h), so the cache is read from HBM once; this kernel is bound
 // by that read.  Heads beyond the group size (lanes n >= G) compute on zeros and are not stored.
 //
-// One wave per (split of the keys, key/value head, token).  The splits are cut at absolute key
-// positions (multiples of SPLIT), so a token's result does not depend on what else is in the
-// batch.  A second kernel merges the splits.
+// W waves per (split of the keys, key/value head, token): one where the step has waves enough, four where it has few; wave w
+// takes the split's tiles w, w + W, ... and the four states are put together at the end.  The splits are cut at absolute
+// key positions (multiples of SPLIT), so a token's result does not depend on what else is in the
+// batch but for W.  A second kernel merges the splits.
+//
+// What bounds a step of few tokens is a wave's chain: some 0.7 us of memory and some 0.4 of arithmetic for each of its tiles,
+// eight of them in a split of 128 keys, whatever the other units do.  With four waves the chain is two tiles, both on their
+// way from the start (with the merge behind it, one token of 16 heads on 4 over
+// 1000 keys: 8.7 us against 11.4 with one wave; with the step before folded in 10.3 against 12.5).
 #include "attention_tile.h"
+
+// The states of a block's W waves put together in the order of the waves: results as of one wave that has them all, in wave
+// 0 .. W - 1 by rows of acc: wave w ends with the rows db = w D / 16 / W ... of all columns.  lds: W (D / 16) 64 float4
+// and W 32 floats.
+template <int D, int W>
+struct WaveStates {
+    floatx4 acc[W][D / 16][64];
+    float m[W][16], l[W][16];
+};
+
+template <int D, int W>
+__device__ __forceinline__ void join_waves(WaveStates<D, W>& ws, const AttnState<D>& st, float l, int wave, int lane,
+                                           floatx4 (&out)[D / 16 / W], float& m_all, float& l_all) {
+    const int g = lane >> 4, n = lane & 15;
+#pragma unroll
+    for (int db = 0; db < D / 16; ++db) ws.acc[wave][db][lane] = st.acc[db];
+    if (g == 0) { ws.m[wave][n] = st.m; ws.l[wave][n] = l; }
+    __syncthreads();
+    float f[W];
+    m_all = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < W; ++w) m_all = fmaxf(m_all, ws.m[w][n]);
+    l_all = 0.f;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+        const float mw = ws.m[w][n];
+        f[w] = mw == -INFINITY ? 0.f : __expf(mw - m_all);
+        l_all += ws.l[w][n] * f[w];
+    }
+#pragma unroll
+    for (int i = 0; i < D / 16 / W; ++i) {
+        floatx4 a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < W; ++w) a += ws.acc[w][wave * (D / 16 / W) + i][lane] * f[w];
+        out[i] = a;
+    }
+}
 
 // SPLIT: keys per split (a multiple of 16, at most 64 tiles).  The next tile is loaded while the
 // current one is computed, and the split's page ids are read before the loop.
 // (Merging the splits in this same kernel, by the wave that finishes last, was tried: the
 // device-wide fences it needs cost several times what the separate merge kernel costs.)
 // CAP: a soft cap on the scores (scale then holds 2 log2(e) / cap, see attn_tile_step).
-template <int D, int SPLIT, bool CAP>
-__global__ __launch_bounds__(64) void attention_decode_split_kernel(
+template <int D, int SPLIT, bool CAP, int W>
+__global__ __launch_bounds__(64 * W) void attention_decode_split_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ cache,
     const int* __restrict__ dec_tokens, const int* __restrict__ positions, const int* __restrict__ tok_seq,
     const int* __restrict__ block_table, int max_blocks, const int* __restrict__ shared_keys,
     float* __restrict__ part_acc, float* __restrict__ part_ml,
     int Hq, int Hkv, int P, float scale, int window, int keep_first, int num_splits, float cap) {
-    constexpr int TILES = SPLIT / 16;
-    const int lane = threadIdx.x, g = lane >> 4, n = lane & 15;
+    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
+    const int wave = W > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
     const int split = blockIdx.x, kvh = blockIdx.y, di = blockIdx.z;
     const int G = Hq / Hkv;
     const int t = dec_tokens ? dec_tokens[di] : di;       // (no list: every row, in order)
@@ -37,7 +80,7 @@ __global__ __launch_bounds__(64) void attention_decode_split_kernel(
     float* pacc = part_acc + (((long)di * Hq + head) * num_splits + split) * D;
     float* pml = part_ml + (((long)di * Hq + head) * num_splits + split) * 2;
     if (k_begin >= k_end && first_tiles == 0) {   // nothing of this split is seen by the token
-        if (head_ok && g == 0) { pml[0] = -INFINITY; pml[1] = 0.f; }
+        if (head_ok && g == 0 && wave == 0) { pml[0] = -INFINITY; pml[1] = 0.f; }
         return;
     }
     const int row = tok_seq[t];
@@ -73,16 +116,18 @@ __global__ __launch_bounds__(64) void attention_decode_split_kernel(
                                     (split * SPLIT + TILE_OF(i_) * 16) % P, g, n, stream)
 #define STEP(buf_, i_) attn_tile_step<D, CAP>(st, buf_, qreg, scale, split * SPLIT + TILE_OF(i_) * 16, g, k_begin, k_end, k_begin, k_end, kf, cap)
     KVTile<D> ta, tb;
-    int i = walk0;
+    int i = walk0 + wave;
     const int walk1 = tile1 - gap;
-    LOAD(ta, i);
-    while (true) {
-        if (i + 1 < walk1) LOAD(tb, i + 1);
-        STEP(ta, i);
-        if (++i >= walk1) break;
-        if (i + 1 < walk1) LOAD(ta, i + 1);
-        STEP(tb, i);
-        if (++i >= walk1) break;
+    if (W == 1 || i < walk1) {
+        LOAD(ta, i);
+        while (true) {
+            if (i + W < walk1) LOAD(tb, i + W);
+            STEP(ta, i);
+            if ((i += W) >= walk1) break;
+            if (i + W < walk1) LOAD(ta, i + W);
+            STEP(tb, i);
+            if ((i += W) >= walk1) break;
+        }
     }
 #undef LOAD
 #undef STEP
@@ -91,6 +136,18 @@ __global__ __launch_bounds__(64) void attention_decode_split_kernel(
     const float m = st.m;
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
+    if constexpr (W > 1) {
+        __shared__ WaveStates<D, W> ws;
+        floatx4 o[D / 16 / W];
+        float m_all, l_all;
+        join_waves<D, W>(ws, st, l, wave, lane, o, m_all, l_all);
+        if (head_ok) {
+#pragma unroll
+            for (int i = 0; i < D / 16 / W; ++i) *(floatx4*)(pacc + (wave * (D / 16 / W) + i) * 16 + g * 4) = o[i];
+            if (g == 0 && wave == 0) { pml[0] = m_all; pml[1] = l_all; }
+        }
+        return;
+    }
     if (head_ok) {
 #pragma unroll
         for (int db = 0; db < D / 16; ++db)
@@ -189,8 +246,10 @@ struct NormRotate {
 // token's 256 waves.  With 3 the code of a whole split is straight-line (waits are then exact) and
 // takes 64 registers more, which with many waves costs more than it brings.  The order of the
 // arithmetic is the same either way.
-template <int D, int SPLIT, int AHEAD>
-__global__ __launch_bounds__(64) void attention_decode_fused_split_kernel(
+// W: the waves of a block, as above (with AHEAD 1).  A wave's first two tiles travel while it prepares q, which every wave does for
+// itself; the last one takes the token's own key and value too (it has the fewest tiles).
+template <int D, int SPLIT, int AHEAD, int W>
+__global__ __launch_bounds__(64 * W) void attention_decode_fused_split_kernel(
     const bf16_t* __restrict__ qkv, bf16_t* cache,
     const int* __restrict__ dec_tokens, const int* __restrict__ positions, const int* __restrict__ tok_seq,
     const int* __restrict__ block_table, int max_blocks, const int* __restrict__ shared_keys,
@@ -198,21 +257,23 @@ __global__ __launch_bounds__(64) void attention_decode_fused_split_kernel(
     float* __restrict__ part_acc, float* __restrict__ part_ml,
     int Hq, int Hkv, int P, float scale, int window, int num_splits) {
     constexpr int TILES = SPLIT / 16;
-    const int lane = threadIdx.x, g = lane >> 4, n = lane & 15;
+    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
+    const int wave = W > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
     const int split = blockIdx.x, kvh = blockIdx.y, di = blockIdx.z;
     const int G = Hq / Hkv;
     const int t = dec_tokens ? dec_tokens[di] : di;       // (no list: every row, in order)
     const int p = positions[t];
     const int lo = first_seen_key(p, window);
-    const bool own = split == p / SPLIT;                   // this wave takes the token's own key and value
+    const bool owns = split == p / SPLIT;                  // this block takes the token's own key and value
+    const bool own = owns && wave == W - 1;
     const int k_begin = max(split * SPLIT, lo);
     const int k_end = min((split + 1) * SPLIT, p);         // cached keys: the token's own is not among them
     const int head = kvh * G + n;
     const bool head_ok = n < G;
     float* pacc = part_acc + (((long)di * Hq + head) * num_splits + split) * D;
     float* pml = part_ml + (((long)di * Hq + head) * num_splits + split) * 2;
-    if (k_begin >= k_end && !own) {   // nothing of this split is seen by the token
-        if (head_ok && g == 0) { pml[0] = -INFINITY; pml[1] = 0.f; }
+    if (k_begin >= k_end && !owns) {   // nothing of this split is seen by the token
+        if (head_ok && g == 0 && wave == 0) { pml[0] = -INFINITY; pml[1] = 0.f; }
         return;
     }
     const long width = (long)(Hq + 2 * Hkv) * D;
@@ -222,7 +283,8 @@ __global__ __launch_bounds__(64) void attention_decode_fused_split_kernel(
     AttnState<D> st;
     st.init();
     bf16x8 qreg[D / 32];
-    if (k_begin < k_end) {
+    // (the wave's tiles: those of the split from the first that is seen on, W apart)
+    if (k_begin < k_end && (W == 1 || (k_begin - split * SPLIT) / 16 + wave < (k_end - split * SPLIT + 15) / 16)) {
         const int row = tok_seq[t];
         const int* bt = block_table + (long)row * max_blocks;
         const bool stream = !(shared_keys && split * SPLIT < shared_keys[row]);
@@ -249,22 +311,22 @@ __global__ __launch_bounds__(64) void attention_decode_fused_split_kernel(
             }
         } else {
             KVTile<D> ta, tb;
-            int i = tile0;
+            int i = tile0 + wave;
             LOAD(ta, i);                                   // the first tiles travel while q is prepared
-            if (i + 1 < tile1) LOAD(tb, i + 1);
+            if (i + W < tile1) LOAD(tb, i + W);
             nq.finish(qreg, q_w != nullptr, eps, cs != nullptr);
             while (true) {
                 STEP(ta, i);
-                if (++i >= tile1) break;
-                if (i + 1 < tile1) LOAD(ta, i + 1);
+                if ((i += W) >= tile1) break;
+                if (i + W < tile1) LOAD(ta, i + W);
                 STEP(tb, i);
-                if (++i >= tile1) break;
-                if (i + 1 < tile1) LOAD(tb, i + 1);
+                if ((i += W) >= tile1) break;
+                if (i + W < tile1) LOAD(tb, i + W);
             }
         }
 #undef LOAD
 #undef STEP
-    } else {
+    } else if (W == 1 || own) {
         NormRotate<D> nq;
         nq.fetch(qkv + t * width + (long)head * D, head_ok, q_w, cs, g);
         nq.finish(qreg, q_w != nullptr, eps, cs != nullptr);
@@ -319,6 +381,18 @@ __global__ __launch_bounds__(64) void attention_decode_fused_split_kernel(
     const float m = st.m;
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
+    if constexpr (W > 1) {
+        __shared__ WaveStates<D, W> ws;
+        floatx4 o[D / 16 / W];
+        float m_all, l_all;
+        join_waves<D, W>(ws, st, l, wave, lane, o, m_all, l_all);
+        if (head_ok) {
+#pragma unroll
+            for (int i = 0; i < D / 16 / W; ++i) *(floatx4*)(pacc + (wave * (D / 16 / W) + i) * 16 + g * 4) = o[i];
+            if (g == 0 && wave == 0) { pml[0] = m_all; pml[1] = l_all; }
+        }
+        return;
+    }
     if (head_ok) {
 #pragma unroll
         for (int db = 0; db < D / 16; ++db)
@@ -433,11 +507,19 @@ int qe_attention_decode(const void* q, void* out, const void* cache, const int* 
     (void)qe_cdiv;
     dim3 grid(num_splits, Hkv, n_dec);
     dim3 mgrid(n_dec, Hq);
+    // (with 512 waves of one tile after the other the units have two each: 14.4 us with one wave a split, 12.9 with four; with
+    // 1024 19.2 and 20.9)
+    const bool four = (long)num_splits * Hkv * n_dec <= 512;
     if (softcap > 0.f) scale = scale * 2.f * 1.4426950408889634f / softcap;
-#define QE_DECODE_SPLIT(D_, S_, CAP_)                                                                   \
-        attention_decode_split_kernel<D_, S_, CAP_><<<grid, 64, 0, stream>>>(                           \
+#define QE_DECODE_SPLIT2(D_, S_, CAP_, W_)                                                              \
+        attention_decode_split_kernel<D_, S_, CAP_, W_><<<grid, 64 * W_, 0, stream>>>(                  \
             (const bf16_t*)q, (const bf16_t*)cache, dec_tokens, positions, tok_seq, block_table,        \
             max_blocks, shared_keys, part_acc, part_ml, Hq, Hkv, P, scale, window, keep_first, num_splits, softcap)
+#define QE_DECODE_SPLIT(D_, S_, CAP_)                                                                   \
+    do {                                                                                                \
+        if (four) QE_DECODE_SPLIT2(D_, S_, CAP_, 4);                                                   \
+        else QE_DECODE_SPLIT2(D_, S_, CAP_, 1);                                                         \
+    } while (0)
 #define QE_DECODE(D_, S_)                                                                               \
     do {                                                                                                \
         if (softcap > 0.f) QE_DECODE_SPLIT(D_, S_, true);                                               \
@@ -451,6 +533,7 @@ int qe_attention_decode(const void* q, void* out, const void* cache, const int* 
     else QE_DECODE(64, 256);
 #undef QE_DECODE
 #undef QE_DECODE_SPLIT
+#undef QE_DECODE_SPLIT2
     QE_LAUNCH_CHECK();
     return 0;
 }
@@ -478,19 +561,18 @@ int qe_attention_decode_fused(const void* qkv, void* out, void* cache, const int
     AttnTail tail{};
     tail.out_stride = (long)Hq * D;
     tail.dv = D;
-    const bool few = (long)num_splits * Hkv * n_dec <= 1024;   // at most a wave per SIMD: loads further ahead
+    const long waves = (long)num_splits * Hkv * n_dec;
+    const bool few = waves <= 1024;                            // at most a wave per SIMD: loads further ahead
+    // (every wave prepares q: 192 waves of one request each take 11.4 us, four times as many 10.1; 384 take 12.0, and 14.8)
+    const bool four = waves <= 256;
+#define QE_DECODE_FUSED_ARGS(D_)                                                                        \
+            (const bf16_t*)qkv, (bf16_t*)cache, dec_tokens, positions, tok_seq, block_table, max_blocks, \
+            shared_keys, slots, q_w, k_w, eps, table, part_acc, part_ml, Hq, Hkv, P, scale, window, num_splits
 #define QE_DECODE_FUSED(D_, S_)                                                                         \
     do {                                                                                                \
-        if (few)                                                                                        \
-            attention_decode_fused_split_kernel<D_, S_, 3><<<grid, 64, 0, stream>>>(                    \
-                (const bf16_t*)qkv, (bf16_t*)cache, dec_tokens, positions, tok_seq, block_table, max_blocks, \
-                shared_keys, slots, q_w, k_w, eps, table, part_acc, part_ml, Hq, Hkv, P, scale, window, \
-                num_splits);                                                                            \
-        else                                                                                            \
-        attention_decode_fused_split_kernel<D_, S_, 1><<<grid, 64, 0, stream>>>(                        \
-            (const bf16_t*)qkv, (bf16_t*)cache, dec_tokens, positions, tok_seq, block_table, max_blocks, \
-            shared_keys, slots, q_w, k_w, eps, table, part_acc, part_ml, Hq, Hkv, P, scale, window,     \
-            num_splits);                                                                                \
+        if (four) attention_decode_fused_split_kernel<D_, S_, 1, 4><<<grid, 256, 0, stream>>>(QE_DECODE_FUSED_ARGS(D_)); \
+        else if (few) attention_decode_fused_split_kernel<D_, S_, 3, 1><<<grid, 64, 0, stream>>>(QE_DECODE_FUSED_ARGS(D_)); \
+        else attention_decode_fused_split_kernel<D_, S_, 1, 1><<<grid, 64, 0, stream>>>(QE_DECODE_FUSED_ARGS(D_)); \
         attention_decode_merge_kernel<D_><<<mgrid, 256, 0, stream>>>(part_acc, part_ml, dec_tokens,     \
                                                                      (bf16_t*)out, Hq, num_splits, 0, tail); \
     } while (0)
@@ -499,6 +581,7 @@ int qe_attention_decode_fused(const void* qkv, void* out, void* cache, const int
     else if (split_keys == 128) QE_DECODE_FUSED(64, 128);
     else QE_DECODE_FUSED(64, 256);
 #undef QE_DECODE_FUSED
+#undef QE_DECODE_FUSED_ARGS
     QE_LAUNCH_CHECK();
     return 0;
 }

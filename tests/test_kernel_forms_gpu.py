@@ -237,3 +237,48 @@ def test_talking_heads_in_registers(ops, hkv, G, dk, dv, dc, window):
         want = torch.stack([w[h] @ vd[:, h // G] for h in range(hq)])
         # (a bfloat16 rounding of each result; the scores' own errors, some 2^-20, move the weights by as much)
         assert ((got[i] - want).abs() <= want.abs() * 2.0 ** -8 + 2.0 ** -17 * vd.abs().max()).all(), p
+
+
+@pytest.mark.parametrize("hq,hkv,D,window", [(4, 4, 128, 0), (16, 2, 64, 0), (6, 2, 128, 40), (8, 8, 64, 200), (16, 1, 128, 130)])
+@pytest.mark.parametrize("copies", [1, 40])
+def test_decode_attention_by_one_wave_and_by_four(ops, hq, hkv, D, window, copies):
+    """Single new tokens with a split's tiles dealt to four waves (few tokens) and to one (many), with the step before folded in and
+    without: positions at the edges of tiles and splits, a wave without a tile, the token's own key alone in its split."""
+    P, pos = 16, [0, 1, 15, 16, 17, 48, 63, 64, 127, 128, 129, 255, 256, 300]
+    n = len(pos)
+    pages = [p // P + 1 for p in pos]
+    order = torch.randperm(sum(pages), generator=torch.Generator().manual_seed(7)).int()
+    table, at = torch.full((n, max(pages)), -1, dtype=torch.int32), 0
+    cache = torch.full((sum(pages), 2, hkv, P * D), float("nan"), dtype=torch.bfloat16)     # (a key tile [P][D], a value tile [D][P])
+    q, ks, vs = rand(n, hq, D, seed=hq).bfloat16(), [], []
+    for i, p in enumerate(pos):
+        k, v = rand(p + 1, hkv, D, seed=20 + i).bfloat16(), rand(p + 1, hkv, D, seed=60 + i).bfloat16()
+        ids = order[at:at + pages[i]]
+        at += pages[i]
+        table[i, :pages[i]] = ids
+        for j in range(p + 1):
+            page = cache[ids[j // P]]
+            page[0].view(hkv, P, D)[:, j % P] = k[j]
+            page[1].view(hkv, D, P)[:, :, j % P] = v[j]
+        ks.append(k)
+        vs.append(v)
+    cache = cache.view(-1, 2, hkv, P, D).to(DEV)
+    rows = torch.arange(n).repeat(copies)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    positions, seq = i32(pos)[rows.to(DEV)], rows.int().to(DEV)
+    scale = 1.5 / D ** 0.5
+    out = ops.attention(q[rows].to(DEV), cache, positions, seq, table.to(DEV), scale, window, dec_tokens=i32(range(len(rows))),
+                        max_dec_position=max(pos)).cpu()
+    qkv = torch.stack([torch.cat([q[i].flatten(), ks[i][-1].flatten(), vs[i][-1].flatten()]) for i in range(n)])
+    fused = ops.attention_decode_fused(qkv[rows].to(DEV), hq, cache, positions, seq, table.to(DEV), scale, window, None, max(pos),
+                                       None, None, 1e-6, None, None).cpu()
+    for i, p in enumerate(pos):
+        lo = max(0, p - window + 1) if window else 0
+        k, v = ks[i][lo:].double(), vs[i][lo:].double()
+        w = torch.softmax(torch.stack([k[:, h * hkv // hq] @ q[i, h].double() for h in range(hq)]) * scale, -1)
+        want = torch.stack([w[h] @ v[:, h * hkv // hq] for h in range(hq)])
+        # (the weights and the result are rounded to bfloat16: 2^-9 of each weight times its value, and of the result)
+        bound = 2.0 ** -8 * (torch.stack([w[h] @ v[:, h * hkv // hq].abs() for h in range(hq)]) + want.abs())
+        for got in (out, fused):
+            for c in (0, copies - 1):
+                assert ((got.view(len(rows), hq, D)[c * n + i].double() - want).abs() <= bound).all(), (p, c)
