@@ -35,7 +35,11 @@
 #define LAT_VT_PITCH 36
 #define LAT_CHUNK 512         // keys whose places in the cache are looked up at a time
 
-template <int RB, int DKC>
+// WS: the waves that share a token's group of 16 heads, four where a block has one such group (few rows, up to 16 heads; the other three
+// waves of the block helped with the tiles and then waited): each takes every fourth piece of the scores' contraction, whose parts
+// meet in shared memory, and every fourth 16 rows of the output (one token of 16 heads over 2048 rows of 512 + 64 numbers: 15.2 us
+// with the merge, 22.0 with one working wave; 4 tokens 17.7, and 24.0).
+template <int RB, int DKC, int WS>
 __global__ __launch_bounds__(256) void latent_attention_mfma_kernel(
     const bf16_t* __restrict__ qp, bf16_t* __restrict__ out, float* __restrict__ part_acc, float* __restrict__ part_ml,
     const bf16_t* __restrict__ cache, const int* __restrict__ positions, const int* __restrict__ tok_seq,
@@ -52,7 +56,9 @@ __global__ __launch_bounds__(256) void latent_attention_mfma_kernel(
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4, n = lane & 15;
     const int split = blockIdx.y;
     const int HG = (H + 15) / 16;
-    const int wt = wave / HGB, whg = wave % HGB;
+    __shared__ floatx4 part_s[WS > 1 ? WS : 1][2][WS > 1 ? 64 : 1];
+    const int ws = WS > 1 ? wave : 0;              // this wave's place among those that share its heads
+    const int wt = WS > 1 ? 0 : wave / HGB, whg = WS > 1 ? 0 : wave % HGB;
     // (the step's last rows see the most keys: their blocks start first, so that no compute unit is left with a
     // long block at the end)
     const int t0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * TOK;
@@ -62,17 +68,18 @@ __global__ __launch_bounds__(256) void latent_attention_mfma_kernel(
     const int head = hg * 16 + n;
     const bool head_ok = unit_ok && head < H;
 
-    bf16x8 q[DKC];
+    constexpr int QC = (DKC + WS - 1) / WS;        // this wave's pieces of the contraction
+    bf16x8 q[QC];
     const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-    for (int c = 0; c < DKC; ++c) {
-        const int d = c * 32 + g * 8;
+    for (int c = 0; c < QC; ++c) {
+        const int d = (c * WS + ws) * 32 + g * 8;
         q[c] = (head_ok && d < Dk) ? *(const bf16x8*)(qp + ((long)t * H + head) * Dk + d) : zero8;
     }
     float m = -INFINITY, l = 0.f;
-    floatx4 acc[RB];
+    floatx4 acc[RB / WS];
 #pragma unroll
-    for (int db = 0; db < RB; ++db) acc[db] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int db = 0; db < RB / WS; ++db) acc[db] = floatx4{0.f, 0.f, 0.f, 0.f};
 
     int seg = 0;
     while (seg < TOK && t0 + seg < T) {
@@ -144,13 +151,23 @@ __global__ __launch_bounds__(256) void latent_attention_mfma_kernel(
             if (!mine) continue;
             floatx4 s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int c = 0; c < DKC; ++c) {
-                if (c < dkc) {
-                    const bf16x8 a0 = *(const bf16x8*)(Ck + n * kpitch + c * 32 + g * 8);
-                    const bf16x8 a1 = *(const bf16x8*)(Ck + (16 + n) * kpitch + c * 32 + g * 8);
+            for (int c = 0; c < QC; ++c) {
+                const int cc = c * WS + ws;
+                if (cc < dkc) {
+                    const bf16x8 a0 = *(const bf16x8*)(Ck + n * kpitch + cc * 32 + g * 8);
+                    const bf16x8 a1 = *(const bf16x8*)(Ck + (16 + n) * kpitch + cc * 32 + g * 8);
                     s0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, q[c], s0, 0, 0, 0);
                     s1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, q[c], s1, 0, 0, 0);
                 }
+            }
+            if constexpr (WS > 1) {                    // (all waves of the block are here or none is; the next tile's barriers
+                part_s[ws][0][lane] = s0;              // come before this is written again)
+                part_s[ws][1][lane] = s1;
+                __syncthreads();
+                s0 = part_s[0][0][lane];
+                s1 = part_s[0][1][lane];
+#pragma unroll
+                for (int w = 1; w < WS; ++w) { s0 += part_s[w][0][lane]; s1 += part_s[w][1][lane]; }
             }
             float sv[8];
             float tmax = -INFINITY;
@@ -176,15 +193,16 @@ __global__ __launch_bounds__(256) void latent_attention_mfma_kernel(
             l = l * alpha + psum;
             m = mn;
 #pragma unroll
-            for (int db = 0; db < RB; ++db) {
+            for (int k = 0; k < RB / WS; ++k) {
+                const int db = k * WS + ws;
                 if (db < rb) {
                     union { bf16x8 v; uint2 h[2]; } au;
                     const bf16_t* ap = VT + (db * 16 + n) * LAT_VT_PITCH + g * 8;
                     au.h[0] = *(const uint2*)ap;
                     au.h[1] = *(const uint2*)(ap + 4);
                     const bf16x8 a = au.v;
-                    acc[db] *= alpha;
-                    acc[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pb, acc[db], 0, 0, 0);
+                    acc[k] *= alpha;
+                    acc[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, pb, acc[k], 0, 0, 0);
                 }
             }
         }
@@ -203,10 +221,10 @@ __global__ __launch_bounds__(256) void latent_attention_mfma_kernel(
                     }
                     bf16_t* o = out + ((long)t * H + head) * R;
 #pragma unroll
-                    for (int db = 0; db < RB; ++db) {
-                        const int d = db * 16 + g * 4;
+                    for (int k = 0; k < RB / WS; ++k) {
+                        const int d = (k * WS + ws) * 16 + g * 4;
                         if (d < R) {                       // (R is a multiple of 8: four numbers lie inside or outside together)
-                            const float v[4] = {acc[db][0] * inv, acc[db][1] * inv, acc[db][2] * inv, acc[db][3] * inv};
+                            const float v[4] = {acc[k][0] * inv, acc[k][1] * inv, acc[k][2] * inv, acc[k][3] * inv};
                             Vec4<bf16_t>::store(o + d, v);
                         }
                     }
@@ -214,9 +232,9 @@ __global__ __launch_bounds__(256) void latent_attention_mfma_kernel(
                     const int RP = rb * 16;
                     float* pa = part_acc + (((long)t * H + head) * NS + split) * RP;
 #pragma unroll
-                    for (int db = 0; db < RB; ++db)
-                        if (db < rb) *(floatx4*)(pa + db * 16 + g * 4) = acc[db];
-                    if (g == 0) {
+                    for (int k = 0; k < RB / WS; ++k)
+                        if (k * WS + ws < rb) *(floatx4*)(pa + (k * WS + ws) * 16 + g * 4) = acc[k];
+                    if (g == 0 && ws == 0) {
                         float* pm = part_ml + (((long)t * H + head) * NS + split) * 2;
                         pm[0] = m;
                         pm[1] = ls;
@@ -228,46 +246,54 @@ __global__ __launch_bounds__(256) void latent_attention_mfma_kernel(
     }
 }
 
-// One block per (token, head): the splits' partial results, in the order of the splits.  Lane s of the first
-// wave fetches split s's maximum and sum, so that the weights are there after one trip to memory; then every
-// thread adds up its output numbers, eight splits' loads at a time.
+// A block per (token, head) and 256 / SG numbers of the output: the splits' partial results.  Lane s of every wave fetches split s's
+// maximum and sum; the splits are cut into SG parts, each summed by a part of the threads, eight asked for at a time and before the
+// weights are there, and the parts' sums are added in their order.  Few heads are bound by the trips to memory: SG = 4, one
+// trip for 32 splits (16 heads of 512 numbers: 4.6 us, 6.7 with a block a head that fetched the weights first and went
+// through its numbers twice).
+template <int SG>
 __global__ __launch_bounds__(256) void latent_attention_merge_kernel(const float* __restrict__ part_acc,
                                                                      const float* __restrict__ part_ml,
                                                                      bf16_t* __restrict__ out, int NS, int R, int RP,
                                                                      const float* __restrict__ sink, int H) {
-    __shared__ float wgt[64];
-    __shared__ float inv_l;
+    constexpr int COLS = 256 / SG;
+    __shared__ float red[SG][COLS];
     const long th = blockIdx.x;
-    const int tid = threadIdx.x;
-    if (tid < 64) {
-        const float* pm = part_ml + th * NS * 2;
-        const float ms = tid < NS ? pm[2 * tid] : -INFINITY;
-        const float ls = tid < NS ? pm[2 * tid + 1] : 0.f;
-        float M = wave_max(ms);
-        const float sk = sink ? sink[th % H] : -INFINITY;
-        M = fmaxf(M, sk);
-        const float w = ms == -INFINITY ? 0.f : __expf(ms - M);
-        wgt[tid] = w;
-        float L = sink ? __expf(sk - M) : 0.f;
-        for (int s = 0; s < NS; ++s) L = fmaf(__shfl(w, s, 64), __shfl(ls, s, 64), L);      // in the order of the splits
-        if (tid == 0) inv_l = 1.f / L;
-    }
-    __syncthreads();
-    const float inv = inv_l;
-    for (int d = tid; d < R; d += blockDim.x) {
-        const float* pa = part_acc + th * NS * RP + d;
-        float a = 0.f;
-        int s = 0;
-        for (; s + 8 <= NS; s += 8) {
-            float v[8];
+    const int lane = threadIdx.x & 63, at = threadIdx.x % COLS;
+    const int part = SG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / COLS) : 0;      // (COLS is a multiple of 64)
+    const int d = blockIdx.y * COLS + at;
+    const float* pm = part_ml + th * NS * 2;
+    const float ms = lane < NS ? pm[2 * lane] : -INFINITY;
+    const float ls = lane < NS ? pm[2 * lane + 1] : 0.f;
+    const float sk = sink ? sink[th % H] : -INFINITY;
+    const float* pa = part_acc + th * NS * RP + (d < R ? d : 0);
+    const int per = (NS + SG - 1) / SG, s_begin = part * per, s_end = min(NS, s_begin + per);
+    float w = 0.f, M = 0.f, a = 0.f;
+    for (int s0 = s_begin; s0 < s_end || s0 == s_begin; s0 += 8) {
+        float v[8];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) v[u] = pa[(long)(s + u) * RP];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) a = fmaf(wgt[s + u], v[u], a);
+        for (int u = 0; u < 8; ++u) v[u] = pa[(long)min(s0 + u, NS - 1) * RP];
+        if (s0 == s_begin) {
+            M = fmaxf(wave_max(ms), sk);
+            w = ms == -INFINITY ? 0.f : __expf(ms - M);
         }
-        for (; s < NS; ++s) a = fmaf(wgt[s], pa[(long)s * RP], a);
-        Elem<bf16_t>::store(out + th * R + d, a * inv);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const float f = __shfl(w, s0 + u, 64);
+            // (a split without keys left no numbers: whatever lies there does not count)
+            if (s0 + u < s_end && f != 0.f) a = fmaf(f, v[u], a);
+        }
     }
+    float L = sink ? __expf(sk - M) : 0.f;
+    for (int s = 0; s < NS; ++s) L = fmaf(__shfl(w, s, 64), __shfl(ls, s, 64), L);      // in the order of the splits
+    if (SG > 1) {
+        red[part][at] = a;
+        __syncthreads();
+        if (part > 0) return;
+#pragma unroll
+        for (int k = 1; k < SG; ++k) a += red[k][at];
+    }
+    if (d < R) Elem<bf16_t>::store(out + th * R + d, a / L);
 }
 
 static bool latent_mfma_fits(int R, int Dk, int& rbc, int& dkc) {
@@ -335,17 +361,18 @@ extern "C" int qe_latent_attention_mfma(const void* qp, void* out, const void* c
     const int dkc = (Dk + 31) / 32, rb = (R + 15) / 16;
     const size_t shmem = ((size_t)32 * (dkc * 32 + 8) + (size_t)rb * 16 * LAT_VT_PITCH) * sizeof(bf16_t);
     dim3 grid(qe_cdiv(T, TOK), NS, qe_cdiv(HG, HGB));
-#define QE_LA(RB_, DKC_)                                                                                              \
+#define QE_LA(RB_, DKC_) do { if (HGB * TOK == 1) QE_LA2(RB_, DKC_, 4); else QE_LA2(RB_, DKC_, 1); } while (0)
+#define QE_LA2(RB_, DKC_, WS_)                                                                                        \
     do {                                                                                                              \
         static size_t attr_bytes = 48 * 1024;          /* (what a kernel may take without asking) */                 \
         if (shmem > attr_bytes) {                                                                                     \
-            hipError_t e_ = hipFuncSetAttribute((const void*)latent_attention_mfma_kernel<RB_, DKC_>,                 \
+            hipError_t e_ = hipFuncSetAttribute((const void*)latent_attention_mfma_kernel<RB_, DKC_, WS_>,                 \
                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);              \
             QE_REQUIRE(e_ == hipSuccess, "latent_attention (mfma): %zu bytes of shared memory: %s", shmem,             \
                        hipGetErrorString(e_));                                                                        \
             attr_bytes = shmem;                                                                                       \
         }                                                                                                             \
-        latent_attention_mfma_kernel<RB_, DKC_><<<grid, 256, shmem, stream>>>(                                        \
+        latent_attention_mfma_kernel<RB_, DKC_, WS_><<<grid, 256, shmem, stream>>>(                                        \
             (const bf16_t*)qp, (bf16_t*)out, part_acc, part_ml, (const bf16_t*)cache, positions, tok_seq, block_table, \
             max_blocks, T, H, R, Dk, P, scale, TOK, HGB, NS, window, sink);                                                       \
     } while (0)
@@ -354,9 +381,14 @@ extern "C" int qe_latent_attention_mfma(const void* qp, void* out, const void* c
     else if (rbc == 16) QE_LA(16, 10);
     else QE_LA(32, 20);
 #undef QE_LA
+#undef QE_LA2
     QE_LAUNCH_CHECK();
     if (NS > 1) {
-        latent_attention_merge_kernel<<<T * H, R >= 256 ? 256 : (R >= 128 ? 128 : 64), 0, stream>>>(part_acc, part_ml, (bf16_t*)out, NS, R, (int)RP, sink, H);
+        // (four parts while the blocks fit the chip at once; 64 rows of 32 heads, 16384 blocks of 64 numbers: 12 us more than
+        // 4096 of 256)
+        const bool few = (long)T * H * qe_cdiv(R, 64) <= 1024;
+        if (few) latent_attention_merge_kernel<4><<<dim3(T * H, qe_cdiv(R, 64)), 256, 0, stream>>>(part_acc, part_ml, (bf16_t*)out, NS, R, (int)RP, sink, H);
+        else latent_attention_merge_kernel<1><<<dim3(T * H, qe_cdiv(R, 256)), 256, 0, stream>>>(part_acc, part_ml, (bf16_t*)out, NS, R, (int)RP, sink, H);
         QE_LAUNCH_CHECK();
     }
     return 0;

@@ -282,3 +282,32 @@ def test_decode_attention_by_one_wave_and_by_four(ops, hq, hkv, D, window, copie
         for got in (out, fused):
             for c in (0, copies - 1):
                 assert ((got.view(len(rows), hq, D)[c * n + i].double() - want).abs() <= bound).all(), (p, c)
+
+
+@pytest.mark.parametrize("T,H,N,K", [(1, 16, 128, 512), (1, 3, 20, 8), (2, 2, 64, 40), (17, 5, 130, 256), (32, 1, 16, 264), (33, 2, 128, 520), (70, 3, 40, 72)])
+def test_products_of_heads_in_steps_of_k(ops, T, H, N, K):
+    """Eight steps of K asked for together (few rows) and two (many): sums of whole numbers far below 2^24, rounded once."""
+    g = torch.Generator().manual_seed(K)
+    x, w = torch.randint(-3, 4, (T, H, K), generator=g).bfloat16(), torch.randint(-3, 4, (H, N, K), generator=g).bfloat16()
+    out = torch.empty(T, H, N, dtype=torch.bfloat16, device=DEV)
+    ops.gemm_heads(x.to(DEV), w.to(DEV), out)
+    want = torch.stack([x[:, h].float() @ w[h].float().t() for h in range(H)], 1).bfloat16()
+    assert torch.equal(out.cpu(), want)
+
+
+@pytest.mark.parametrize("H,R,dr", [(16, 512, 64), (5, 8, 8), (16, 64, 64), (3, 120, 72), (16, 256, 64), (16, 200, 48), (17, 128, 64), (48, 64, 32)])
+@pytest.mark.parametrize("window", [0, 50])
+def test_latent_attention_of_single_tokens(ops, H, R, dr, window):
+    """Four waves share a token's heads (up to 16 of them) or take a group each: latents of every size class, one key, tiles' edges,
+    many splits and splits without keys."""
+    before = [0, 30, 31, 32, 200, 1100]
+    cache, table, pos, seq, own = latent_rows(before, [1] * len(before), R, dr, 16, 50)
+    q = rand(len(before), H, R + dr, seed=9).bfloat16()
+    scale = (R + dr) ** -0.5
+    for rows in (list(range(len(before))), [5], list(range(len(before))) * 12):
+        got = ops.latent_attention(q[rows].to(DEV), cache, pos[rows], seq[rows], table, R, scale, window=window).cpu().double()
+        for j, i in enumerate(rows[:len(before)]):
+            c = own[i][max(0, len(own[i]) - window) if window else 0:]
+            w = torch.softmax(q[i].double() @ c.t() * scale, -1)
+            want = w @ c[:, :R]
+            assert ((got[j] - want).abs() <= 2.0 ** -8 * (w @ c[:, :R].abs() + want.abs())).all(), (i, rows[:2])
