@@ -311,3 +311,28 @@ def test_latent_attention_of_single_tokens(ops, H, R, dr, window):
             w = torch.softmax(q[i].double() @ c.t() * scale, -1)
             want = w @ c[:, :R]
             assert ((got[j] - want).abs() <= 2.0 ** -8 * (w @ c[:, :R].abs() + want.abs())).all(), (i, rows[:2])
+
+
+@pytest.mark.parametrize("tile", [64, 128, 256, 512])
+@pytest.mark.parametrize("page", [16, 64])
+def test_qkv_product_stores_values_behind_other_rows(ops, tile, page):
+    """Values go to the cache in pieces of eight tokens wherever eight slots lie side by side from a multiple of eight on: rows whose
+    slots are scattered, absent, in runs that begin in the middle of a piece and of a tile, whole pages and runs in descending
+    order.  Sums of whole numbers, rounded once; what is not named stays as it was."""
+    hq, hkv, K, M = 2, 3, 64, 410
+    slots = [5, 900, 17, -1, 40] + list(range(61, 150)) + [-1] * 3 + list(range(200, 233)) + list(range(448, 256, -1)) + list(range(512, 600))
+    assert len(slots) == M
+    g = torch.Generator().manual_seed(page)
+    x = torch.randint(-3, 4, (M, K), generator=g).bfloat16()
+    w = torch.randint(-3, 4, ((hq + 2 * hkv) * 128, K), generator=g).bfloat16()
+    cache = torch.full((1024 // page, 2, hkv, page * 128), -0.5, dtype=torch.bfloat16)
+    want, y = cache.clone(), (x.float() @ w.float().t()).bfloat16()
+    for m, s in enumerate(slots):
+        if s >= 0:
+            want[s // page, 0].view(hkv, page, 128)[:, s % page] = y[m, hq * 128:(hq + hkv) * 128].view(hkv, 128)
+            want[s // page, 1].view(hkv, 128, page)[:, :, s % page] = y[m, (hq + hkv) * 128:].view(hkv, 128)
+    got = cache.view(-1, 2, hkv, page, 128).to(DEV)
+    q = ops.gemm_qkv(x.to(DEV), w.to(DEV), None, hq, got, torch.zeros(M, dtype=torch.int32, device=DEV), None, None, 1e-6, None,
+                     torch.tensor(slots, dtype=torch.int32, device=DEV), tile=tile)
+    assert torch.equal(q.cpu().view(M, -1), y[:, :hq * 128])
+    assert torch.equal(got.cpu().view(want.shape), want)
