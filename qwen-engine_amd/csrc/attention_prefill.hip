@@ -635,9 +635,10 @@ int qe_attention_prefill(const void* q, void* out, const void* cache, const int*
     dim3 mgrid(Hkv * waves_per_kv, D / 32, num_tiles / 4);
     const float scale_log2 = softcap > 0.f ? 1.f : scale * 1.4426950408889634f;
     const float cap_in = softcap > 0.f ? scale * 2.f * 1.4426950408889634f / softcap : 0.f, cap_out = softcap * 1.4426950408889634f;
-    // two groups a block where the blocks do not fill the compute units twice anyway
-    // (groups: 0 = choose, 1 or 2)
-    if (groups == 0) groups = (long)grid.x * grid.z <= qe_compute_units() ? 2 : 1;
+    // two groups a block where the blocks do not fill the compute units more than twice anyway: the longest walk decides
+    // (whole prompts of 2048 tokens, 32 heads: 512 blocks, 69 us with one group, 61 with two; 3000 tokens, 16 heads, 376
+    // blocks: 92 and 67; 3000 tokens, 32 heads, 752 blocks: 100 and 119).  (groups: 0 = choose, 1 or 2)
+    if (groups == 0) groups = (long)grid.x * grid.z <= 2 * qe_compute_units() ? 2 : 1;
     QE_REQUIRE(groups == 1 || groups == 2, "prefill attention: %d groups a block", groups);
 #define QE_PREFILL_CAP(D_, NG_, CAP_)                                                               \
     attention_prefill_kernel<D_, NG_, CAP_><<<grid, 256 * NG_, 0, stream>>>(                        \
