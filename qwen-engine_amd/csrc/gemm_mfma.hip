@@ -61,6 +61,8 @@ struct QkvTail {
     float act_limit, act_slope;
     // Without SILU: the result is relu(.)^2 instead of the product itself.
     int relu_sq;
+    // The first column of the product that this launch computes (a multiple of 256).
+    int n_first;
     // With SILU over grouped rows: sorted row i is row_w[perm[i]] times its row of x (null: that row itself); the
     // factor meets gate and up in 32-bit.
     const float* row_w;
@@ -136,7 +138,7 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
         out += (long)first * (PAIR ? N / 2 : N);
         tile_m = 0;
     }
-    const int m0 = tile_m * BM, n0 = tile_n * BN;
+    const int m0 = tile_m * BM, n0 = tail.n_first + tile_n * BN;
     const int wm = (wave >> 1) * WM, wn = (wave & 1) * WN;
     // (QKV: thread i fetches the position and the slot of the tile's row i now, for the end)
     int my_pos = 0, my_slot = -1;
@@ -623,10 +625,11 @@ bool qe_gemm_mfma_ok(int M, int N, int K, int dt_a, int dt_w) {
     return dt_a == QE_BF16 && dt_w == QE_BF16 && M > 16 && K % 8 == 0 && K >= 64;
 }
 
+// The columns tail.n_first .. tail.n_first + n_cols - 1 of the product (rounded up to whole tiles).
 template <typename TO, int BM, int BN, int BK, int NW, int MINB, int SILU, bool QKV = false>
 static int launch_mfma(const void* x, const void* w, const float* bias, void* out, int M, int N, int K,
-                       int splits, hipStream_t stream, const QkvTail& tail = QkvTail{}) {
-    const int tiles_m = qe_cdiv(M, BM), tiles_n = qe_cdiv(N, BN);
+                       int n_cols, int splits, hipStream_t stream, const QkvTail& tail) {
+    const int tiles_m = qe_cdiv(M, BM), tiles_n = qe_cdiv(n_cols, BN);
     const long blocks = (long)tiles_m * tiles_n;
     QE_REQUIRE(blocks <= 2147483647L, "mfma gemm: too many tiles");
     const size_t shmem = 2 * (BM + BN) * (BK * 2 + 16);
@@ -647,7 +650,7 @@ static int launch_mfma(const void* x, const void* w, const float* bias, void* ou
     for (int a = 1; a <= 8; a *= 2) {
         const int b = 8 / a;
         if (tiles_m % a || tiles_n % b) continue;
-        const long rows = (long)b * M + (long)a * N;
+        const long rows = (long)b * M + (long)a * n_cols;
         if (xcd_m == 0 || rows < fewest) { xcd_m = a; xcd_n = b; fewest = rows; }
     }
     gemm_mfma_kernel<TO, BM, BN, BK, NW, MINB, SILU, QKV><<<dim3((unsigned)blocks, (unsigned)splits), 64 * NW, shmem, stream>>>(
@@ -750,9 +753,40 @@ static int choose_tile(int M, int N, int K, int splits, bool largest = true) {
     return tile;
 }
 
+// Where the last turn of a product's tiles would leave most units idle, the columns that fill the turns before it go first, and the
+// rest in a launch and a shape of its own: the number of the first columns, a multiple of 256, or 0.  Three microseconds for the
+// second launch; less than 3 % is not worth it.  (1972 rows against gate and up of 51200 x 5120, 1600 tiles of 256 x 256: 923 us,
+// now 884; 656 rows 434, now 342;
+// 1300 rows against 24576 x 4096 299, now 269; q, k and v of 10240 x 5120 with 1600 rows 254, now 193.)
+static int first_columns(int M, int N, int K, bool largest = true) {
+    int tile;
+    const float whole = qe_gemm_mfma_shape(M, N, K, 1, &tile, largest);
+    float best = 0.97f * whole;
+    int cut = 0;
+    const int bms[4] = {64, 128, 256, 256}, bns[4] = {128, 128, 128, 256};
+    for (int i = 0; i < 4; ++i) {
+        const long tiles_m = qe_cdiv(M, bms[i]), turns = tiles_m * qe_cdiv(N, bns[i]) / 256;
+        const long n1 = turns * 256 / tiles_m * bns[i] / 256 * 256;
+        if (n1 <= 0 || n1 >= N) continue;
+        const float t = qe_gemm_mfma_shape(M, (int)n1, K, 1, &tile, largest) + qe_gemm_mfma_shape(M, N - (int)n1, K, 1, &tile, largest) + 3.f;
+        if (t < best) { best = t; cut = (int)n1; }
+    }
+    return cut;
+}
+
 template <typename TO, int SILU>
 static int pick_mfma(const void* x, const void* w, const float* bias, void* out, int M, int N, int K,
-                     int tile, int splits, hipStream_t stream) {
+                     int tile, int splits, hipStream_t stream, int n_first = 0, int n_cols = 0) {
+    if (tile == 0 && splits == 1 && n_cols == 0 && M > 64) {
+        const int n1 = first_columns(M, N, K, SILU >= 0);
+        if (n1 > 0) {
+            const int rc = pick_mfma<TO, SILU>(x, w, bias, out, M, N, K, choose_tile(M, n1, K, 1, SILU >= 0), 1, stream, 0, n1);
+            return rc ? rc : pick_mfma<TO, SILU>(x, w, bias, out, M, N, K, choose_tile(M, N - n1, K, 1, SILU >= 0), 1, stream, n1, N - n1);
+        }
+    }
+    if (n_cols == 0) n_cols = N;
+    QkvTail tail{};
+    tail.n_first = n_first;
     // Up to 64 rows against a gate|up matrix of at most one tile column a compute unit (its K cannot be
     // cut): a block streams its weights alone on its unit, and what it has in flight bounds it.  A k step of
     // 128 doubles that (24576 x 4096 against 64 rows: 44.4 us against 49.2; with two blocks a unit, 51200 x
@@ -761,11 +795,11 @@ static int pick_mfma(const void* x, const void* w, const float* bias, void* out,
     // (the gelu of 65536 values is 35 us in which nothing else runs on the unit: 256 x 256 is never its shape; 3000 rows against
     // 4096 x 1024: 65 us in it, 52 in 256 x 128, 47 in 128 x 128)
     if (tile == 0) tile = choose_tile(M, N, K, splits, SILU >= 0);
-    if (tile == 65) return launch_mfma<TO, 64, 128, 128, 4, 1, SILU>(x, w, bias, out, M, N, K, splits, stream);
-    if (tile == 512) return launch_mfma<TO, 256, 256, 64, 4, 1, SILU>(x, w, bias, out, M, N, K, splits, stream);
-    if (tile == 256) return launch_mfma<TO, 256, 128, 64, 8, 1, SILU>(x, w, bias, out, M, N, K, splits, stream);
-    if (tile == 128) return launch_mfma<TO, 128, 128, 64, 4, 2, SILU>(x, w, bias, out, M, N, K, splits, stream);
-    return launch_mfma<TO, 64, 128, 64, 4, 2, SILU>(x, w, bias, out, M, N, K, splits, stream);
+    if (tile == 65) return launch_mfma<TO, 64, 128, 128, 4, 1, SILU>(x, w, bias, out, M, N, K, n_cols, splits, stream, tail);
+    if (tile == 512) return launch_mfma<TO, 256, 256, 64, 4, 1, SILU>(x, w, bias, out, M, N, K, n_cols, splits, stream, tail);
+    if (tile == 256) return launch_mfma<TO, 256, 128, 64, 8, 1, SILU>(x, w, bias, out, M, N, K, n_cols, splits, stream, tail);
+    if (tile == 128) return launch_mfma<TO, 128, 128, 64, 4, 2, SILU>(x, w, bias, out, M, N, K, n_cols, splits, stream, tail);
+    return launch_mfma<TO, 64, 128, 64, 4, 2, SILU>(x, w, bias, out, M, N, K, n_cols, splits, stream, tail);
 }
 
 // tile: rows of the output tile (256, 128 or 64; 512 stands for 256 x 256, 65 for 64 x 128 with a k step of 128), 0 to choose
@@ -810,9 +844,16 @@ int qe_gemm_qkv(const void* x, const void* w, const float* bias, int M, int K, i
     int lp = 0;
     while ((1 << lp) < P) ++lp;
     QkvTail tail{positions, slots, q_w, k_w, table, (bf16_t*)q_out, (bf16_t*)cache, eps, Hq, Hkv, P, lp};
-    if (tile == 0) tile = choose_tile(M, N, K, 1);
-    if (tile == 512) return launch_mfma<bf16_t, 256, 256, 64, 4, 1, 0, true>(x, w, bias, nullptr, M, N, K, 1, stream, tail);
-    if (tile == 256) return launch_mfma<bf16_t, 256, 128, 64, 8, 1, 0, true>(x, w, bias, nullptr, M, N, K, 1, stream, tail);
-    if (tile == 128) return launch_mfma<bf16_t, 128, 128, 64, 4, 2, 0, true>(x, w, bias, nullptr, M, N, K, 1, stream, tail);
-    return launch_mfma<bf16_t, 64, 128, 64, 4, 2, 0, true>(x, w, bias, nullptr, M, N, K, 1, stream, tail);
+    const int n1 = tile == 0 ? first_columns(M, N, K) : 0;
+    for (int part = 0; part < (n1 > 0 ? 2 : 1); ++part) {
+        tail.n_first = part ? n1 : 0;
+        const int n_cols = n1 == 0 ? N : (part ? N - n1 : n1), t = tile ? tile : choose_tile(M, n_cols, K, 1);
+        int rc;
+        if (t == 512) rc = launch_mfma<bf16_t, 256, 256, 64, 4, 1, 0, true>(x, w, bias, nullptr, M, N, K, n_cols, 1, stream, tail);
+        else if (t == 256) rc = launch_mfma<bf16_t, 256, 128, 64, 8, 1, 0, true>(x, w, bias, nullptr, M, N, K, n_cols, 1, stream, tail);
+        else if (t == 128) rc = launch_mfma<bf16_t, 128, 128, 64, 4, 2, 0, true>(x, w, bias, nullptr, M, N, K, n_cols, 1, stream, tail);
+        else rc = launch_mfma<bf16_t, 64, 128, 64, 4, 2, 0, true>(x, w, bias, nullptr, M, N, K, n_cols, 1, stream, tail);
+        if (rc) return rc;
+    }
+    return 0;
 }

@@ -336,3 +336,28 @@ def test_qkv_product_stores_values_behind_other_rows(ops, tile, page):
                      torch.tensor(slots, dtype=torch.int32, device=DEV), tile=tile)
     assert torch.equal(q.cpu().view(M, -1), y[:, :hq * 128])
     assert torch.equal(got.cpu().view(want.shape), want)
+
+
+@pytest.mark.parametrize("M,N", [(656, 24576), (1600, 10240), (700, 6144 * 3), (2048, 10240)])
+def test_products_in_two_launches(ops, M, N):
+    """Products whose last turn of tiles is thin go in two launches over the columns: gate and up with silu, the product itself with a
+    bias, and q|k|v, against the same in one launch of one shape.  Whole numbers where nothing is computed on the sums."""
+    g = torch.Generator().manual_seed(N)
+    K = 512
+    x = torch.randint(-2, 3, (M, K), generator=g).bfloat16().to(DEV)
+    w = torch.randint(-2, 3, (N, K), generator=g).bfloat16().to(DEV)
+    bias = torch.randint(-9, 9, (N,), generator=g).float().to(DEV)
+    want = x.float() @ w.float().t()
+    assert torch.equal(ops.gemm(x, w, bias, out_dtype=torch.float32), want + bias)
+    gate_up = (x.double() @ w.double().t()).view(M, N // 64, 2, 32) * 2.0 ** -6
+    small = (w.float() * 2.0 ** -6).bfloat16()
+    act = (torch.nn.functional.silu(gate_up[:, :, 0]) * gate_up[:, :, 1]).reshape(M, N // 2)
+    got = ops.gemm(x, small, epilogue=ops.EPI_SILU_MUL_IL).double()
+    assert ((got - act).abs() <= act.abs() * 2.0 ** -8 + 2.0 ** -20).all()
+    hkv = 2 if N % 256 == 0 else 1
+    hq = N // 128 - 2 * hkv
+    cache = [torch.zeros(M // 16 + 1, 2, hkv, 16, 128, dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+    at = torch.arange(M, dtype=torch.int32, device=DEV)
+    q = [ops.gemm_qkv(x, w, None, hq, c, at, None, None, 1e-6, None, at, tile=t) for c, t in zip(cache, (0, 128))]
+    assert torch.equal(q[0], q[1]) and torch.equal(cache[0], cache[1])
+    assert torch.equal(q[0].view(M, -1).float(), want[:, :hq * 128].bfloat16().float())
