@@ -361,3 +361,34 @@ def test_products_in_two_launches(ops, M, N):
     q = [ops.gemm_qkv(x, w, None, hq, c, at, None, None, 1e-6, None, at, tile=t) for c, t in zip(cache, (0, 128))]
     assert torch.equal(q[0], q[1]) and torch.equal(cache[0], cache[1])
     assert torch.equal(q[0].view(M, -1).float(), want[:, :hq * 128].bfloat16().float())
+
+
+@pytest.mark.parametrize("hq,hkv,D,window", [(4, 2, 128, 0), (3, 1, 16, 0), (6, 2, 48, 100), (2, 2, 256, 0), (20, 1, 64, 37), (4, 4, 144, 0)])
+def test_float32_attention_in_eight_walks(ops, hq, hkv, D, window):
+    """Few tokens (eight waves, a walk each) and many (four waves, two walks each): against 64 bits, and the same bits."""
+    P, L = 16, 430
+    k, v, q = rand(L, hkv, D, seed=1), rand(L, hkv, D, seed=2), rand(L, hq, D, seed=3)
+    pages = -(-L // P)
+    order = torch.randperm(pages + 2, generator=torch.Generator().manual_seed(4))[:pages].int()
+    cache = torch.full((pages + 2, 2, hkv, P * D), float("nan"))
+    for j in range(L):
+        page = cache[order[j // P]]
+        page[0].view(hkv, P, D)[:, j % P] = k[j]
+        page[1].view(hkv, D, P)[:, :, j % P] = v[j]
+    cache, table = cache.view(-1, 2, hkv, P, D).to(DEV), order[None].to(DEV)
+    scale = D ** -0.5
+
+    def run(rows):
+        r = torch.tensor(rows, dtype=torch.int32, device=DEV)
+        return ops.attention(q[rows].to(DEV), cache, r, torch.zeros_like(r), table, scale, window).cpu()
+
+    every = run(list(range(L)))
+    for p in (0, 1, 15, 16, 63, 64, 127, 128, 200, 255, 429):
+        got = run([p])[0]
+        lo = max(0, p - window + 1) if window else 0
+        w = torch.softmax(torch.stack([k[lo:p + 1, h * hkv // hq].double() @ q[p, h].double() for h in range(hq)]) * scale, -1)
+        want = torch.stack([w[h] @ v[lo:p + 1, h * hkv // hq].double() for h in range(hq)])
+        size = torch.stack([w[h] @ v[lo:p + 1, h * hkv // hq].double().abs() for h in range(hq)])
+        # (scores of a few units and the sums: some sqrt(keys + D) roundings of 2^-24 each)
+        assert ((got.double() - want).abs() <= 2.0 ** -24 * 4 * (p + 1 + D) ** 0.5 * size + 1e-30).all(), p
+        assert torch.equal(got, every[p]), p
