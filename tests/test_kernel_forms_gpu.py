@@ -392,3 +392,30 @@ def test_float32_attention_in_eight_walks(ops, hq, hkv, D, window):
         # (scores of a few units and the sums: some sqrt(keys + D) roundings of 2^-24 each)
         assert ((got.double() - want).abs() <= 2.0 ** -24 * 4 * (p + 1 + D) ** 0.5 * size + 1e-30).all(), p
         assert torch.equal(got, every[p]), p
+
+
+@pytest.mark.parametrize("taps", [2, 3, 4, 8])
+@pytest.mark.parametrize("H", [4, 260, 1028])
+def test_short_convolution_by_eight_rows(ops, taps, H):
+    """Four channels of eight rows a thread: portions that begin and end anywhere in a block's rows, shorter than the taps and longer
+    than blocks, continued from step to step; what no row names stays as it was."""
+    w = rand(H, taps, seed=taps)
+    state = torch.full((5, taps - 1, H), 7.0, device=DEV)
+    state[:4] = 0
+    past = {s: torch.zeros(0, H) for s in range(4)}
+    for step, lens in enumerate(([5, 0, 1, 12], [1, 3, 0, 8], [9, 2, 30, 1], [2, 1, 1, 1])):
+        rows = {s: rand(n, H, seed=10 * step + s) for s, n in enumerate(lens) if n}
+        seq = torch.tensor(sum(([s] * lens[s] for s in rows), []), dtype=torch.int32, device=DEV)
+        got = ops.short_conv(torch.cat(list(rows.values())).to(DEV), w.to(DEV), state, seq, torch.float32).cpu()
+        want, size = [], []
+        for s, x in rows.items():
+            full = torch.cat([torch.zeros(taps - 1, H), past[s], x]).double()
+            past[s] = torch.cat([past[s], x])
+            n0 = len(full) - len(x)
+            for to, f, wd in ((want, full, w.double()), (size, full.abs(), w.double().abs())):
+                to.append(torch.stack([f[n0 + i] + sum(wd[:, taps - 1 - k] * f[n0 + i - k] for k in range(taps)) for i in range(len(x))]))
+            last = torch.cat([torch.zeros(taps - 1, H), past[s]])[-(taps - 1):]
+            assert torch.equal(state[s].cpu(), last), (step, s)
+        # (a multiply-add a tap, each rounded by 2^-24 of a partial sum, which is at most the sum of the sizes of its terms)
+        assert ((got.double() - torch.cat(want)).abs() <= 2.0 ** -24 * taps * torch.cat(size)).all(), step
+    assert float(state[4].min()) == 7.0
