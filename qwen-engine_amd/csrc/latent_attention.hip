@@ -49,7 +49,9 @@ __device__ __forceinline__ void pair_place(int i, int rot_dims, int half_split, 
 }
 
 // q (may be null) [T, H, Dn + Dr] -> qp [T, H, R + Dr]: in the same launch, the rotated parts of the token's
-// queries go to the packed queries (what qe_latent_q_rotate does), so that a step of few rows has a kernel less.
+// queries go to the packed queries (what qe_latent_q_rotate does), by a block of their own beside the token's (one token of 16
+// heads, 64 numbers rotated, a latent of 512: 4.0 us, 6.4 with one block for both), so
+// that a step of few rows has a kernel less.
 template <typename TC>
 __global__ void latent_kv_store_kernel(const float* __restrict__ kv, const float* __restrict__ weight, float eps,
                                        const int* __restrict__ positions, const float* __restrict__ inv_freq,
@@ -58,7 +60,8 @@ __global__ void latent_kv_store_kernel(const float* __restrict__ kv, const float
                                        int half_split) {
     __shared__ float red[16];
     const long t = blockIdx.x;
-    if (q) {
+    const int slot = slots ? slots[t] : -1;
+    if (blockIdx.y == 1) {
         const float pq = (float)positions[t];
         const int pairs = (Dr + 1) / 2;
         for (int idx = threadIdx.x; idx < H * pairs; idx += blockDim.x) {
@@ -77,12 +80,12 @@ __global__ void latent_kv_store_kernel(const float* __restrict__ kv, const float
             Elem<TC>::store(dst + a, u);
             Elem<TC>::store(dst + b, v);
         }
+        return;
     }
     const float* row = kv + t * (R + Dr);
     float ss = 0.f;
     for (int i = threadIdx.x; i < R; i += blockDim.x) ss += row[i] * row[i];
     ss = block_sum(ss, red);
-    const int slot = slots ? slots[t] : -1;
     if (slot < 0) return;
     const float f = rsqrtf(ss / (float)R + eps);
     TC* dst = cache + (long)slot * (R + Dr);
@@ -112,11 +115,12 @@ extern "C" int qe_latent_kv_store(const float* kv, const float* weight, float ep
     QE_REQUIRE(rot_dims >= 0 && rot_dims <= Dr && rot_dims % 2 == 0, "latent_kv_store: %d rotated of %d", rot_dims, Dr);
     if (T == 0) return 0;
     const int threads = R >= 512 ? 256 : 64;
+    const dim3 grid(T, q ? 2 : 1);
     if (dt_c == QE_F32)
-        latent_kv_store_kernel<float><<<T, threads, 0, stream>>>(kv, weight, eps, positions, inv_freq, rot_dims, slots,
+        latent_kv_store_kernel<float><<<grid, threads, 0, stream>>>(kv, weight, eps, positions, inv_freq, rot_dims, slots,
                                                                   (float*)cache, R, Dr, (const float*)q, (float*)qp, H, Dn, half_split);
     else if (dt_c == QE_BF16)
-        latent_kv_store_kernel<bf16_t><<<T, threads, 0, stream>>>(kv, weight, eps, positions, inv_freq, rot_dims, slots,
+        latent_kv_store_kernel<bf16_t><<<grid, threads, 0, stream>>>(kv, weight, eps, positions, inv_freq, rot_dims, slots,
                                                                    (bf16_t*)cache, R, Dr, (const bf16_t*)q, (bf16_t*)qp, H, Dn, half_split);
     else
         QE_REQUIRE(false, "latent_kv_store: unknown cache type %d", dt_c);
