@@ -3,53 +3,124 @@
 // of one wave (see attention_tile.h), so the cache is read from HBM once; this kernel is bound
 // by that read.  Heads beyond the group size (lanes n >= G) compute on zeros and are not stored.
 //
-// W waves per (split of the keys, key/value head, token): one where the step has waves enough, four where it has few; wave w
-// takes the split's tiles w, w + W, ... and the four states are put together at the end.  The splits are cut at absolute
-// key positions (multiples of SPLIT), so a token's result does not depend on what else is in the
-// batch but for W.  A second kernel merges the splits.
+// W waves per (split of the keys, key/value head, token): one where the step has waves enough, four where it has few.  The
+// splits are cut at absolute key positions (multiples of SPLIT), and four waves do the arithmetic of one in its order, so a
+// token's result does not depend on what else is in the batch.  A second kernel merges the splits.
 //
 // What bounds a step of few tokens is a wave's chain: some 0.7 us of memory and some 0.4 of arithmetic for each of its tiles,
-// eight of them in a split of 128 keys, whatever the other units do.  With four waves the chain is two tiles, both on their
-// way from the start (with the merge behind it, one token of 16 heads on 4 over
-// 1000 keys: 8.7 us against 11.4 with one wave; with the step before folded in 10.3 against 12.5).
+// eight of them in a split of 128 keys, whatever the other units do.  Of four waves each takes the scores and then the weights of
+// every fourth tile, which meet in shared memory, and multiplies its quarter of the value rows by the weights of all tiles, in
+// the order of the keys; everything a wave needs is asked for at its start.  (With the merge behind it, one token of 16 heads of
+// 128 on 8 over 1000 keys: 8.6 us against 11.3 with one wave, over 40 keys 7.2 against 7.4; with the step before folded in
+// 10.1 against 12.2, and 8.8 against 9.6.  With a softmax of its own for every wave, joined at the end, the sums had another
+// order than one wave's and took 8.7 and 7.1, and 10.2 and 8.5.)
 #include "attention_tile.h"
+#include <type_traits>
 
-// The states of a block's W waves put together in the order of the waves: results as of one wave that has them all, in wave
-// 0 .. W - 1 by rows of acc: wave w ends with the rows db = w D / 16 / W ... of all columns.  lds: W (D / 16) 64 float4
-// and W 32 floats.
-template <int D, int W>
-struct WaveStates {
-    floatx4 acc[W][D / 16][64];
-    float m[W][16], l[W][16];
+// What the waves of a block leave for each other about a split's tiles.
+template <int TILES>
+struct WaveShared {
+    float tmax[16][TILES];
+    short4_t weights[TILES][64];
+    float sums[TILES][64];
 };
 
-template <int D, int W>
-__device__ __forceinline__ void join_waves(WaveStates<D, W>& ws, const AttnState<D>& st, float l, int wave, int lane,
-                                           floatx4 (&out)[D / 16 / W], float& m_all, float& l_all) {
-    const int g = lane >> 4, n = lane & 15;
+// What wave ``wave`` of W asks for of the n tiles of a walk (1 <= n <= TILES): the key rows of the tiles wave, wave + W, ..., and of
+// every tile its part of the value rows.  Beyond the last tile the last is asked for again: without a branch the waits are exact
+// (for the same reason all loads are plain: so few splits, 16 MB at most, leave room in the caches).
+// place(i, page, o): the i-th tile's page, and the place of its first key in it.
+template <int D, int TILES, int W>
+struct WaveTiles {
+    static constexpr int NV = D / 16 / W;
+    bf16x8 k[TILES / W][D / 32];
+    short4_t v[TILES][NV];
+    template <typename Place>
+    __device__ __forceinline__ void ask(const bf16_t* cache, long page_stride, int kvh, int Hkv, int P, int n, int wave, int g, int lane_n,
+                                        Place place) {
+        int page, o;
 #pragma unroll
-    for (int db = 0; db < D / 16; ++db) ws.acc[wave][db][lane] = st.acc[db];
-    if (g == 0) { ws.m[wave][n] = st.m; ws.l[wave][n] = l; }
-    __syncthreads();
-    float f[W];
-    m_all = -INFINITY;
+        for (int j = 0; j < TILES / W; ++j) {
+            place(min(j * W + wave, n - 1), page, o);
+            const bf16_t* kbase = cache + page * page_stride + ((long)kvh * P + o) * D + (long)lane_n * D + g * 8;
 #pragma unroll
-    for (int w = 0; w < W; ++w) m_all = fmaxf(m_all, ws.m[w][n]);
-    l_all = 0.f;
+            for (int c = 0; c < D / 32; ++c) k[j][c] = *(const bf16x8*)(kbase + c * 32);
+        }
+        __builtin_amdgcn_sched_barrier(0);                 // (the keys are wanted first)
 #pragma unroll
-    for (int w = 0; w < W; ++w) {
-        const float mw = ws.m[w][n];
-        f[w] = mw == -INFINITY ? 0.f : __expf(mw - m_all);
-        l_all += ws.l[w][n] * f[w];
+        for (int i = 0; i < TILES; ++i) {
+            place(min(i, n - 1), page, o);
+            const bf16_t* vbase = cache + page * page_stride + ((long)(Hkv + kvh) * P) * D + o + (long)lane_n * P + g * 4;
+#pragma unroll
+            for (int b = 0; b < NV; ++b) v[i][b] = *(const short4_t*)(vbase + (long)(wave * NV + b) * 16 * P);
+        }
     }
+    floatx4 s[TILES / W];
+    // The scores of the wave's tiles, and their maxima for the others; kk(i): the i-th tile's first key.  What stands for a tile behind
+    // the last has no key that is seen: a maximum of minus infinity, a factor of 1 and weights of 0 below.
+    template <bool CAP, int ALL, typename FirstKey>
+    __device__ __forceinline__ void score(WaveShared<ALL>& sh, const bf16x8 (&qreg)[D / 32], float scale, int wave, int g, int lane_n, int lo, int hi,
+                                          int kf, float cap, FirstKey kk) {
 #pragma unroll
-    for (int i = 0; i < D / 16 / W; ++i) {
-        floatx4 a = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int w = 0; w < W; ++w) a += ws.acc[w][wave * (D / 16 / W) + i][lane] * f[w];
-        out[i] = a;
+        for (int j = 0; j < TILES / W; ++j) {
+            s[j] = attn_tile_scores<D, CAP>(k[j], qreg, scale, kk(j * W + wave), g, lo, hi, kf, cap);
+            const float t = attn_tile_max(s[j]);
+            if (g == 0) sh.tmax[lane_n][j * W + wave] = t;
+        }
     }
-}
+    // Behind a barrier: the running maxima, the weights of the wave's tiles for the others, and, behind another, the walk with
+    // all weights through the wave's value rows.  l: only the first wave's.
+    template <int ALL, typename FirstKey>
+    __device__ __forceinline__ void walk(WaveShared<ALL>& sh, int n, int wave, int g, int lane, int vlo, int vhi, int kf, FirstKey kk, float& m,
+                                         float& l, floatx4 (&acc)[NV]) const {
+        float tmax[TILES], ref[TILES], alpha[TILES];
+#pragma unroll
+        for (int i = 0; i < TILES; i += 4) Vec4<float>::load(&sh.tmax[lane & 15][i], *(float(*)[4])(tmax + i));
+        m = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < TILES; ++i) {
+            const float mn = fmaxf(m, tmax[i]);
+            ref[i] = attn_reference(mn);
+            alpha[i] = __expf(m - ref[i]);
+            m = mn;
+        }
+#pragma unroll
+        for (int j = 0; j < TILES / W; ++j) {
+            float mine = ref[j * W];
+#pragma unroll
+            for (int w = 1; w < W; ++w) mine = wave == w ? ref[j * W + w] : mine;
+            float psum;
+            sh.weights[j * W + wave][lane] = attn_tile_weights(s[j], mine, psum);
+            sh.sums[j * W + wave][lane] = psum;
+        }
+        __syncthreads();
+        l = 0.f;
+#pragma unroll
+        for (int b = 0; b < NV; ++b) acc[b] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i0 = 0; i0 < TILES; i0 += 4) {
+            if (i0 >= n) break;
+            short4_t pb[4];
+            float psum[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) pb[u] = sh.weights[i0 + u][lane];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) psum[u] = sh.sums[i0 + u][lane];
+            // (value rows of tiles that lie wholly among the keys seen need no mask)
+            const bool inside = i0 + 4 <= n && kk(i0) >= vlo && kk(i0 + 3) + 16 <= vhi && kk(i0 + 3) - kk(i0) == 48;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                l = l * alpha[i0 + u] + psum[u];
+                short4_t vmask = {-1, -1, -1, -1};
+                if (!inside) vmask = attn_value_mask(kk(i0 + u), g, vlo, vhi, kf);
+#pragma unroll
+                for (int b = 0; b < NV; ++b) {
+                    acc[b] *= alpha[i0 + u];
+                    acc[b] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(v[i0 + u][b] & vmask, pb[u], acc[b], 0, 0, 0);
+                }
+            }
+        }
+    }
+};
 
 // SPLIT: keys per split (a multiple of 16, at most 64 tiles).  The next tile is loaded while the
 // current one is computed, and the split's page ids are read before the loop.
@@ -58,7 +129,7 @@ __device__ __forceinline__ void join_waves(WaveStates<D, W>& ws, const AttnState
 // CAP: a soft cap on the scores (scale then holds 2 log2(e) / cap, see attn_tile_step).
 template <int D, int SPLIT, bool CAP, int W>
 __global__ __launch_bounds__(64 * W) void attention_decode_split_kernel(
-    const bf16_t* __restrict__ q, const bf16_t* __restrict__ cache,
+    const bf16_t* __restrict__ q, const bf16_t* cache,           // (not restrict: loads of a tile then stay where they are asked for)
     const int* __restrict__ dec_tokens, const int* __restrict__ positions, const int* __restrict__ tok_seq,
     const int* __restrict__ block_table, int max_blocks, const int* __restrict__ shared_keys,
     float* __restrict__ part_acc, float* __restrict__ part_ml,
@@ -98,15 +169,13 @@ __global__ __launch_bounds__(64 * W) void attention_decode_split_kernel(
     // then read from that lane
     int my_page = 0;
     if ((lane >= tile0 && lane < tile1) || lane < first_tiles) my_page = bt[(split * SPLIT + lane * 16) / P];
+    const int my_place = (split * SPLIT + lane * 16) % P;             // (and the place of its first key in the page)
 
     bf16x8 qreg[D / 32];
     const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
     for (int c = 0; c < D / 32; ++c)
         qreg[c] = head_ok ? *(const bf16x8*)(q + ((long)t * Hq + head) * D + c * 32 + g * 8) : zero8;
-
-    AttnState<D> st;
-    st.init();
 
     // Two tile buffers used in turn: the loads of the next tile are issued before the current
     // one is computed, and nothing is copied from one buffer to the other.
@@ -115,19 +184,47 @@ __global__ __launch_bounds__(64 * W) void attention_decode_split_kernel(
 #define LOAD(buf_, i_) load_tile<D>(buf_, cache, __builtin_amdgcn_readlane(my_page, TILE_OF(i_)), page_stride, kvh, Hkv, P, \
                                     (split * SPLIT + TILE_OF(i_) * 16) % P, g, n, stream)
 #define STEP(buf_, i_) attn_tile_step<D, CAP>(st, buf_, qreg, scale, split * SPLIT + TILE_OF(i_) * 16, g, k_begin, k_end, k_begin, k_end, kf, cap)
-    KVTile<D> ta, tb;
-    int i = walk0 + wave;
     const int walk1 = tile1 - gap;
-    if (W == 1 || i < walk1) {
-        LOAD(ta, i);
-        while (true) {
-            if (i + W < walk1) LOAD(tb, i + W);
-            STEP(ta, i);
-            if ((i += W) >= walk1) break;
-            if (i + W < walk1) LOAD(ta, i + W);
-            STEP(tb, i);
-            if ((i += W) >= walk1) break;
-        }
+    if constexpr (W > 1) {
+        constexpr int TILES = SPLIT / 16, NV = D / 16 / W;
+        __shared__ WaveShared<TILES> shared;
+        const int tiles = walk1 - walk0;
+        const auto first_key = [&](int i) { return split * SPLIT + TILE_OF(walk0 + i) * 16; };
+        const auto by_waves = [&](auto most) {             // (half of the loads where half of the tiles are all there are)
+            WaveTiles<D, decltype(most)::value, W> wt;
+            wt.ask(cache, page_stride, kvh, Hkv, P, tiles, wave, g, n, [&](int i, int& page, int& o) {
+                page = __builtin_amdgcn_readlane(my_page, TILE_OF(walk0 + i));
+                o = __builtin_amdgcn_readlane(my_place, TILE_OF(walk0 + i));
+            });
+            wt.template score<CAP>(shared, qreg, scale, wave, g, n, k_begin, k_end, kf, cap, first_key);
+            __syncthreads();
+            float m, l;
+            floatx4 acc[NV];
+            wt.walk(shared, tiles, wave, g, lane, k_begin, k_end, kf, first_key, m, l, acc);
+            l += __shfl_xor(l, 16, 64);
+            l += __shfl_xor(l, 32, 64);
+            if (head_ok) {
+#pragma unroll
+                for (int b = 0; b < NV; ++b) *(floatx4*)(pacc + (wave * NV + b) * 16 + g * 4) = acc[b];
+                if (g == 0 && wave == 0) { pml[0] = m; pml[1] = l; }
+            }
+        };
+        if (tiles > TILES / 2) by_waves(std::integral_constant<int, TILES>{});
+        else by_waves(std::integral_constant<int, TILES / 2>{});
+        return;
+    }
+    AttnState<D> st;
+    st.init();
+    KVTile<D> ta, tb;
+    int i = walk0;
+    LOAD(ta, i);
+    while (true) {
+        if (i + 1 < walk1) LOAD(tb, i + 1);
+        STEP(ta, i);
+        if (++i >= walk1) break;
+        if (i + 1 < walk1) LOAD(ta, i + 1);
+        STEP(tb, i);
+        if (++i >= walk1) break;
     }
 #undef LOAD
 #undef STEP
@@ -136,18 +233,6 @@ __global__ __launch_bounds__(64 * W) void attention_decode_split_kernel(
     const float m = st.m;
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
-    if constexpr (W > 1) {
-        __shared__ WaveStates<D, W> ws;
-        floatx4 o[D / 16 / W];
-        float m_all, l_all;
-        join_waves<D, W>(ws, st, l, wave, lane, o, m_all, l_all);
-        if (head_ok) {
-#pragma unroll
-            for (int i = 0; i < D / 16 / W; ++i) *(floatx4*)(pacc + (wave * (D / 16 / W) + i) * 16 + g * 4) = o[i];
-            if (g == 0 && wave == 0) { pml[0] = m_all; pml[1] = l_all; }
-        }
-        return;
-    }
     if (head_ok) {
 #pragma unroll
         for (int db = 0; db < D / 16; ++db)
@@ -246,10 +331,10 @@ struct NormRotate {
 // token's 256 waves.  With 3 the code of a whole split is straight-line (waits are then exact) and
 // takes 64 registers more, which with many waves costs more than it brings.  The order of the
 // arithmetic is the same either way.
-// W: the waves of a block, as above (with AHEAD 1).  A wave's first two tiles travel while it prepares q, which every wave does for
-// itself; the last one takes the token's own key and value too (it has the fewest tiles).
+// W: the waves that share a split, as above (AHEAD then means nothing).  Every wave prepares q for itself while its keys and values
+// travel; one more wave prepares the token's own key, whose score it leaves for the others, and writes key and value to the cache.
 template <int D, int SPLIT, int AHEAD, int W>
-__global__ __launch_bounds__(64 * W) void attention_decode_fused_split_kernel(
+__global__ __launch_bounds__(64 * (W > 1 ? W + 1 : 1)) void attention_decode_fused_split_kernel(
     const bf16_t* __restrict__ qkv, bf16_t* cache,
     const int* __restrict__ dec_tokens, const int* __restrict__ positions, const int* __restrict__ tok_seq,
     const int* __restrict__ block_table, int max_blocks, const int* __restrict__ shared_keys,
@@ -265,7 +350,6 @@ __global__ __launch_bounds__(64 * W) void attention_decode_fused_split_kernel(
     const int p = positions[t];
     const int lo = first_seen_key(p, window);
     const bool owns = split == p / SPLIT;                  // this block takes the token's own key and value
-    const bool own = owns && wave == W - 1;
     const int k_begin = max(split * SPLIT, lo);
     const int k_end = min((split + 1) * SPLIT, p);         // cached keys: the token's own is not among them
     const int head = kvh * G + n;
@@ -279,19 +363,137 @@ __global__ __launch_bounds__(64 * W) void attention_decode_fused_split_kernel(
     const long width = (long)(Hq + 2 * Hkv) * D;
     const float* cs = table ? table + (long)p * D : nullptr;
     const long page_stride = 2L * Hkv * P * D;
+    const bf16_t* vsrc = qkv + t * width + (long)(Hq + Hkv + kvh) * D;
 
-    AttnState<D> st;
-    st.init();
     bf16x8 qreg[D / 32];
-    // (the wave's tiles: those of the split from the first that is seen on, W apart)
-    if (k_begin < k_end && (W == 1 || (k_begin - split * SPLIT) / 16 + wave < (k_end - split * SPLIT + 15) / 16)) {
+    bf16x8 kreg[D / 32];                                   // the token's own key, normed and turned
+    // its score
+    const auto own_score = [&]() {
+        float dot = 0.f;
+#pragma unroll
+        for (int c = 0; c < D / 32; ++c)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) dot += (float)qreg[c][e] * (float)kreg[c][e];
+        dot += __shfl_xor(dot, 16, 64);
+        dot += __shfl_xor(dot, 32, 64);
+        return dot;
+    };
+    // the key and the value to the cache
+    const auto store_own = [&]() {
+        const int slot = slots ? slots[t] : -1;
+        if (slot < 0) return;
+        const long page = slot / P;
+        const int off = slot % P;
+        if (n == 0) {
+#pragma unroll
+            for (int c = 0; c < D / 32; ++c)
+                *(bf16x8*)(cache + page * page_stride + ((long)kvh * P + off) * D + c * 32 + g * 8) = kreg[c];
+        }
+        if (n < D / 16) {                                  // the value tile is [D][P]: a column of single elements
+            bf16_t* vt = cache + page * page_stride + ((long)(Hkv + kvh) * P) * D + off;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int d = n * 16 + g * 4 + j;
+                vt[(long)d * P] = vsrc[d];
+            }
+        }
+    };
+    // the own key's score joins a running maximum and sum: its weight, rounded, and the factor for what was summed before it
+    // (the roundings are written out: one wave and four do the same)
+    const auto own_weight = [&](float dot, float& m, float& l, float& alpha) {
+        const float mn = fmaxf(m, dot * scale);
+        alpha = __expf(m - mn);                            // 0 when no cached key was seen
+        const float pn = __expf(__builtin_fmaf(dot, scale, -mn));
+        l = __builtin_fmaf(l, alpha, g == 0 ? pn : 0.f);   // (a lane's share of the sum: once per column)
+        m = mn;
+        return (float)(__bf16)pn;
+    };
+    const auto add_own = [&](floatx4& acc, float alpha, float weight, const short4_t& vv) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[j] = __builtin_fmaf(weight, bf16_bits_to_float((unsigned short)vv[j]), acc[j] * alpha);
+    };
+    const int tile0 = (k_begin - split * SPLIT) / 16;
+    const int tile1 = k_begin < k_end ? (k_end - split * SPLIT + 15) / 16 : tile0;
+    int my_page = 0;
+    bool stream = false;
+    if (k_begin < k_end) {
         const int row = tok_seq[t];
         const int* bt = block_table + (long)row * max_blocks;
-        const bool stream = !(shared_keys && split * SPLIT < shared_keys[row]);
-        const int tile0 = (k_begin - split * SPLIT) / 16;
-        const int tile1 = (k_end - split * SPLIT + 15) / 16;
-        int my_page = 0;
+        stream = !(shared_keys && split * SPLIT < shared_keys[row]);
         if (lane >= tile0 && lane < tile1) my_page = bt[(split * SPLIT + lane * 16) / P];
+    }
+    if constexpr (W > 1) {
+        constexpr int NV = D / 16 / W;
+        __shared__ WaveShared<TILES> shared;
+        __shared__ float own_dot[16];
+        const int tiles = tile1 - tile0;
+        if (wave == W) {                                   // the token's own key
+            NormRotate<D> nq, nk;
+            if (owns) {
+                nk.fetch(qkv + t * width + (long)(Hq + kvh) * D, true, k_w, cs, g);
+                nq.fetch(qkv + t * width + (long)head * D, head_ok, q_w, cs, g);
+                nk.finish(kreg, k_w != nullptr, eps, cs != nullptr);
+                nq.finish(qreg, q_w != nullptr, eps, cs != nullptr);
+            }
+            __syncthreads();
+            if (owns) {
+                const float dot = own_score();
+                if (g == 0) own_dot[n] = dot;
+            }
+            __syncthreads();
+            if (owns) store_own();
+            return;
+        }
+        const auto first_key = [&](int i) { return split * SPLIT + (tile0 + i) * 16; };
+        const auto by_waves = [&](auto most) {
+            constexpr int MOST = decltype(most)::value;    // tiles there can be; 0: none, the own key alone
+            float m = -INFINITY, l = 0.f;
+            floatx4 acc[NV];
+#pragma unroll
+            for (int b = 0; b < NV; ++b) acc[b] = floatx4{0.f, 0.f, 0.f, 0.f};
+            short4_t vv[NV];
+#pragma unroll
+            for (int b = 0; b < NV; ++b) vv[b] = *(const short4_t*)(vsrc + (wave * NV + b) * 16 + g * 4);
+            if constexpr (MOST > 0) {
+                NormRotate<D> nq;
+                nq.fetch(qkv + t * width + (long)head * D, head_ok, q_w, cs, g);
+                const int my_place = (split * SPLIT + lane * 16) % P;
+                WaveTiles<D, MOST, W> wt;
+                wt.ask(cache, page_stride, kvh, Hkv, P, tiles, wave, g, n, [&](int i, int& page, int& o) {
+                    page = __builtin_amdgcn_readlane(my_page, tile0 + i);
+                    o = __builtin_amdgcn_readlane(my_place, tile0 + i);
+                });
+                __builtin_amdgcn_sched_barrier(0);         // (the tiles are asked for before anything waits for q)
+                nq.finish(qreg, q_w != nullptr, eps, cs != nullptr);
+                wt.template score<false>(shared, qreg, scale, wave, g, n, k_begin, k_end, 0, 0.f, first_key);
+                __syncthreads();
+                wt.walk(shared, tiles, wave, g, lane, k_begin, k_end, 0, first_key, m, l, acc);
+            } else {
+                __syncthreads();
+                __syncthreads();
+            }
+            if (owns) {
+                float alpha;
+                const float weight = own_weight(own_dot[n], m, l, alpha);
+#pragma unroll
+                for (int b = 0; b < NV; ++b) add_own(acc[b], alpha, weight, vv[b]);
+            }
+            l += __shfl_xor(l, 16, 64);
+            l += __shfl_xor(l, 32, 64);
+            if (head_ok) {
+#pragma unroll
+                for (int b = 0; b < NV; ++b) *(floatx4*)(pacc + (wave * NV + b) * 16 + g * 4) = acc[b];
+                if (g == 0 && wave == 0) { pml[0] = m; pml[1] = l; }
+            }
+        };
+        if (tiles > TILES / 2) by_waves(std::integral_constant<int, TILES>{});
+        else if (tiles > 0) by_waves(std::integral_constant<int, TILES / 2>{});
+        else by_waves(std::integral_constant<int, 0>{});
+        return;
+    }
+    AttnState<D> st;
+    st.init();
+    if (k_begin < k_end) {
 #define LOAD(buf_, i_) load_tile<D>(buf_, cache, __builtin_amdgcn_readlane(my_page, (i_)), page_stride, kvh, Hkv, P, \
                                     (split * SPLIT + (i_) * 16) % P, g, n, stream)
 #define STEP(buf_, i_) attn_tile_step<D>(st, buf_, qreg, scale, split * SPLIT + (i_) * 16, g, k_begin, k_end, k_begin, k_end)
@@ -311,88 +513,41 @@ __global__ __launch_bounds__(64 * W) void attention_decode_fused_split_kernel(
             }
         } else {
             KVTile<D> ta, tb;
-            int i = tile0 + wave;
+            int i = tile0;
             LOAD(ta, i);                                   // the first tiles travel while q is prepared
-            if (i + W < tile1) LOAD(tb, i + W);
+            if (i + 1 < tile1) LOAD(tb, i + 1);
             nq.finish(qreg, q_w != nullptr, eps, cs != nullptr);
             while (true) {
                 STEP(ta, i);
-                if ((i += W) >= tile1) break;
-                if (i + W < tile1) LOAD(ta, i + W);
+                if (++i >= tile1) break;
+                if (i + 1 < tile1) LOAD(ta, i + 1);
                 STEP(tb, i);
-                if ((i += W) >= tile1) break;
-                if (i + W < tile1) LOAD(tb, i + W);
+                if (++i >= tile1) break;
+                if (i + 1 < tile1) LOAD(tb, i + 1);
             }
         }
 #undef LOAD
 #undef STEP
-    } else if (W == 1 || own) {
+    } else {
         NormRotate<D> nq;
         nq.fetch(qkv + t * width + (long)head * D, head_ok, q_w, cs, g);
         nq.finish(qreg, q_w != nullptr, eps, cs != nullptr);
     }
-    if (own) {
-        bf16x8 kreg[D / 32];
+    if (owns) {
         NormRotate<D> nk;
         nk.fetch(qkv + t * width + (long)(Hq + kvh) * D, true, k_w, cs, g);
         nk.finish(kreg, k_w != nullptr, eps, cs != nullptr);
-        float dot = 0.f;
+        const float dot = own_score();
+        float alpha;
+        const float weight = own_weight(dot, st.m, st.l, alpha);
 #pragma unroll
-        for (int c = 0; c < D / 32; ++c)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) dot += (float)qreg[c][e] * (float)kreg[c][e];
-        dot += __shfl_xor(dot, 16, 64);
-        dot += __shfl_xor(dot, 32, 64);
-        const float s_new = dot * scale;
-        const float mn = fmaxf(st.m, s_new);
-        const float alpha = __expf(st.m - mn);             // 0 when no cached key was seen
-        const float pn = __expf(s_new - mn);
-        const float pn_b = (float)(__bf16)pn;
-        st.l = st.l * alpha + (g == 0 ? pn : 0.f);         // (a lane's share of the sum: once per column)
-        st.m = mn;
-        const bf16_t* vsrc = qkv + t * width + (long)(Hq + Hkv + kvh) * D;
-#pragma unroll
-        for (int db = 0; db < D / 16; ++db) {
-            const short4_t vv = *(const short4_t*)(vsrc + db * 16 + g * 4);
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                st.acc[db][j] = st.acc[db][j] * alpha + pn_b * bf16_bits_to_float((unsigned short)vv[j]);
-        }
-        const int slot = slots ? slots[t] : -1;
-        if (slot >= 0) {
-            const long page = slot / P;
-            const int off = slot % P;
-            if (n == 0) {
-#pragma unroll
-                for (int c = 0; c < D / 32; ++c)
-                    *(bf16x8*)(cache + page * page_stride + ((long)kvh * P + off) * D + c * 32 + g * 8) = kreg[c];
-            }
-            if (n < D / 16) {                              // the value tile is [D][P]: a column of single elements
-                bf16_t* vt = cache + page * page_stride + ((long)(Hkv + kvh) * P) * D + off;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int d = n * 16 + g * 4 + j;
-                    vt[(long)d * P] = vsrc[d];
-                }
-            }
-        }
+        for (int db = 0; db < D / 16; ++db) add_own(st.acc[db], alpha, weight, *(const short4_t*)(vsrc + db * 16 + g * 4));
+        store_own();
     }
     float l = st.l;
     const float m = st.m;
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
-    if constexpr (W > 1) {
-        __shared__ WaveStates<D, W> ws;
-        floatx4 o[D / 16 / W];
-        float m_all, l_all;
-        join_waves<D, W>(ws, st, l, wave, lane, o, m_all, l_all);
-        if (head_ok) {
-#pragma unroll
-            for (int i = 0; i < D / 16 / W; ++i) *(floatx4*)(pacc + (wave * (D / 16 / W) + i) * 16 + g * 4) = o[i];
-            if (g == 0 && wave == 0) { pml[0] = m_all; pml[1] = l_all; }
-        }
-        return;
-    }
     if (head_ok) {
 #pragma unroll
         for (int db = 0; db < D / 16; ++db)
@@ -507,8 +662,8 @@ int qe_attention_decode(const void* q, void* out, const void* cache, const int* 
     (void)qe_cdiv;
     dim3 grid(num_splits, Hkv, n_dec);
     dim3 mgrid(n_dec, Hq);
-    // (with 512 waves of one tile after the other the units have two each: 14.4 us with one wave a split, 12.9 with four; with
-    // 1024 19.2 and 20.9)
+    // (512 splits of 8 tokens over 1000 keys: 14.0 us with one wave a split, 12.6 with four; from 576 on the two are within 3 %
+    // of each other: 14.2 and 14.4, 1024 17.6 and 17.4)
     const bool four = (long)num_splits * Hkv * n_dec <= 512;
     if (softcap > 0.f) scale = scale * 2.f * 1.4426950408889634f / softcap;
 #define QE_DECODE_SPLIT2(D_, S_, CAP_, W_)                                                              \
@@ -563,14 +718,14 @@ int qe_attention_decode_fused(const void* qkv, void* out, void* cache, const int
     tail.dv = D;
     const long waves = (long)num_splits * Hkv * n_dec;
     const bool few = waves <= 1024;                            // at most a wave per SIMD: loads further ahead
-    // (every wave prepares q: 192 waves of one request each take 11.4 us, four times as many 10.1; 384 take 12.0, and 14.8)
+    // (every wave prepares q: 256 splits of one request each take 11.4 us with four, 12.6 with one; 384 13.2 with one, 17.1 with four)
     const bool four = waves <= 256;
 #define QE_DECODE_FUSED_ARGS(D_)                                                                        \
             (const bf16_t*)qkv, (bf16_t*)cache, dec_tokens, positions, tok_seq, block_table, max_blocks, \
             shared_keys, slots, q_w, k_w, eps, table, part_acc, part_ml, Hq, Hkv, P, scale, window, num_splits
 #define QE_DECODE_FUSED(D_, S_)                                                                         \
     do {                                                                                                \
-        if (four) attention_decode_fused_split_kernel<D_, S_, 1, 4><<<grid, 256, 0, stream>>>(QE_DECODE_FUSED_ARGS(D_)); \
+        if (four) attention_decode_fused_split_kernel<D_, S_, 1, 4><<<grid, 320, 0, stream>>>(QE_DECODE_FUSED_ARGS(D_)); \
         else if (few) attention_decode_fused_split_kernel<D_, S_, 3, 1><<<grid, 64, 0, stream>>>(QE_DECODE_FUSED_ARGS(D_)); \
         else attention_decode_fused_split_kernel<D_, S_, 1, 1><<<grid, 64, 0, stream>>>(QE_DECODE_FUSED_ARGS(D_)); \
         attention_decode_merge_kernel<D_><<<mgrid, 256, 0, stream>>>(part_acc, part_ml, dec_tokens,     \

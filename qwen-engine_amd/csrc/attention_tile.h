@@ -81,45 +81,70 @@ struct AttnState {
 // the range that any column of the wave sees (keys outside it may be unwritten memory).  Keys below
 // kf are seen as well, by every column (a request's kept first keys, where a window is given).
 // CAP: the scaled scores pass cap * tanh(. / cap); scale is then the scores' scale times 2 log2(e) / cap.
+// The step is cut in parts, so that waves which share a tile do the same arithmetic on it as one that has it alone.
+
+// The column's scores of the keys kk + 4 g .. + 3, minus infinity for those it does not see.
 template <int D, bool CAP = false>
-__device__ __forceinline__ void attn_tile_step(AttnState<D>& st, const KVTile<D>& tile, const bf16x8 (&qreg)[D / 32],
-                                               float scale, int kk, int g, int lo, int hi, int vlo, int vhi, int kf = 0,
-                                               float cap = 0.f) {
+__device__ __forceinline__ floatx4 attn_tile_scores(const bf16x8 (&k)[D / 32], const bf16x8 (&qreg)[D / 32], float scale,
+                                                    int kk, int g, int lo, int hi, int kf = 0, float cap = 0.f) {
     floatx4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int c = 0; c < D / 32; ++c) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tile.k[c], qreg[c], s, 0, 0, 0);
-    float tmax = -INFINITY;
-    bool ok[4];
+    for (int c = 0; c < D / 32; ++c) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[c], qreg[c], s, 0, 0, 0);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int key = kk + g * 4 + j;
-        ok[j] = (key >= lo && key < hi) || key < kf;
-        s[j] = ok[j] ? (CAP ? soft_capped(s[j] * scale, cap) : s[j] * scale) : -INFINITY;
-        tmax = fmaxf(tmax, s[j]);
+        const bool ok = (key >= lo && key < hi) || key < kf;
+        s[j] = ok ? (CAP ? soft_capped(s[j] * scale, cap) : s[j] * scale) : -INFINITY;
     }
-    tmax = max_over_lane_rows(tmax);
-    const float mn = fmaxf(st.m, tmax);
-    const float ref = (mn == -INFINITY) ? 0.f : mn;   // a column that has seen no key yet: all weights 0
-    const float alpha = __expf(st.m - ref);
+    return s;
+}
+
+// the column's largest score in the tile
+__device__ __forceinline__ float attn_tile_max(const floatx4& s) {
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) tmax = fmaxf(tmax, s[j]);
+    return max_over_lane_rows(tmax);
+}
+// what the weights are relative to, from the running maximum with the tile in it
+__device__ __forceinline__ float attn_reference(float m) { return (m == -INFINITY) ? 0.f : m; }   // (a column that has seen no key yet: all weights 0)
+// the tile's weights, rounded, and the lane's share of their sum
+__device__ __forceinline__ short4_t attn_tile_weights(const floatx4& s, float ref, float& psum) {
     short4_t pb;
-    float psum = 0.f;
+    psum = 0.f;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const float pj = __expf(s[j] - ref);           // 0 for keys that are not seen
         psum += pj;
         pb[j] = bf16_bits(pj);
     }
-    st.l = st.l * alpha + psum;
-    st.m = mn;
-    // The value rows a lane holds serve every column, so they are masked by the wave's range only
-    // (a key outside it may be an unwritten part of a page: anything, times a weight of 0);
-    // what a single column does not see has weight 0 already.
+    return pb;
+}
+
+// The value rows a lane holds serve every column, so they are masked by the wave's range only
+// (a key outside it may be an unwritten part of a page: anything, times a weight of 0);
+// what a single column does not see has weight 0 already.
+__device__ __forceinline__ short4_t attn_value_mask(int kk, int g, int vlo, int vhi, int kf) {
     short4_t vmask;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int key = kk + g * 4 + j;
         vmask[j] = (short)(((key >= vlo && key < vhi) || key < kf) ? -1 : 0);
     }
+    return vmask;
+}
+
+template <int D, bool CAP = false>
+__device__ __forceinline__ void attn_tile_step(AttnState<D>& st, const KVTile<D>& tile, const bf16x8 (&qreg)[D / 32],
+                                               float scale, int kk, int g, int lo, int hi, int vlo, int vhi, int kf = 0,
+                                               float cap = 0.f) {
+    const floatx4 s = attn_tile_scores<D, CAP>(tile.k, qreg, scale, kk, g, lo, hi, kf, cap);
+    const float mn = fmaxf(st.m, attn_tile_max(s)), ref = attn_reference(mn), alpha = __expf(st.m - ref);
+    float psum;
+    const short4_t pb = attn_tile_weights(s, ref, psum);
+    st.l = st.l * alpha + psum;
+    st.m = mn;
+    const short4_t vmask = attn_value_mask(kk, g, vlo, vhi, kf);
 #pragma unroll
     for (int db = 0; db < D / 16; ++db) {
         st.acc[db] *= alpha;

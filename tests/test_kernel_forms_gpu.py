@@ -284,6 +284,53 @@ def test_decode_attention_by_one_wave_and_by_four(ops, hq, hkv, D, window, copie
                 assert ((got.view(len(rows), hq, D)[c * n + i].double() - want).abs() <= bound).all(), (p, c)
 
 
+@pytest.mark.parametrize("hq,hkv,D,page", [(4, 4, 128, 16), (16, 2, 64, 48), (6, 2, 128, 32), (16, 1, 64, 16)])
+@pytest.mark.parametrize("window,keep_first,softcap", [(0, 0, 0.0), (70, 0, 0.0), (150, 20, 0.0), (33, 300, 25.0), (0, 0, 30.0)])
+def test_decode_attention_of_a_token_alone_and_in_company(ops, hq, hkv, D, page, window, keep_first, softcap):
+    """Few tokens' splits are shared by four waves, many tokens' have one each: a token gets the same bits either way, with
+    the step before folded in (the new key and value in the cache too) and without.  What lies behind a request's keys or is
+    not seen may be anything."""
+    pos = [0, 1, 15, 16, 17, 48, 63, 64, 127, 128, 129, 143, 255, 256, 300, 383, 384, 640]
+    n, copies, most = len(pos), 30, max(pos)
+    pages = [p // page + 1 for p in pos]
+    order = torch.randperm(sum(pages), generator=torch.Generator().manual_seed(7)).int()
+    table, at = torch.full((n, max(pages)), -1, dtype=torch.int32), 0
+    cache = torch.full((sum(pages), 2, hkv, page * D), float("nan"), dtype=torch.bfloat16)
+    for i, p in enumerate(pos):
+        table[i, :pages[i]] = order[at:at + pages[i]]
+        at += pages[i]
+        k, v = rand(p + 1, hkv, D, seed=20 + i, scale=2.0).bfloat16(), rand(p + 1, hkv, D, seed=60 + i).bfloat16()
+        for j in range(p + 1):
+            here = cache[table[i, j // page]]
+            here[0].view(hkv, page, D)[:, j % page] = k[j]
+            here[1].view(hkv, D, page)[:, :, j % page] = v[j]
+    cache, table = cache.view(-1, 2, hkv, page, D).to(DEV), table.to(DEV)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    rows = list(range(n)) * copies
+    positions = i32([pos[i] for i in rows])
+    q = rand(n, hq, D, seed=hq).bfloat16()[rows].to(DEV)
+    seen = dict(window=window, keep_first=keep_first, softcap=softcap, max_dec_position=most)
+    every = ops.attention(q, cache, positions, i32(rows), table, 0.15, dec_tokens=i32(range(len(rows))), **seen)
+    assert len(rows) * hkv * (most // 128 + 1) > 512 >= hkv * (most // 128 + 1)
+    for i in range(n):
+        alone = ops.attention(q, cache, positions, i32(rows), table, 0.15, dec_tokens=i32([i]), **seen)
+        assert torch.equal(alone[i], every[i]) and torch.equal(every[i], every[i + n]), pos[i]
+    if keep_first or softcap:
+        return
+    qkv = rand(n, (hq + 2 * hkv) * D, seed=8).bfloat16()[rows].to(DEV)
+    qw, kw, turn = 1 + rand(D, seed=1).to(DEV) / 4, 1 + rand(D, seed=2).to(DEV) / 4, torch.rand(most + 1, D, device=DEV)
+    slots = [-1 if i == 3 else int(table[i, p // page]) * page + p % page for i, p in enumerate(pos)]
+    fused = lambda c, which: ops.attention_decode_fused(qkv, hq, c, positions, i32(rows), table, 0.15, window, i32(which), most, qw, kw, 1e-6,
+                                                        turn, i32(slots + [-1] * (len(rows) - n)))
+    together = cache.clone()
+    every = fused(together, range(len(rows)))
+    one_by_one = cache.clone()
+    for i in range(n):
+        assert torch.equal(fused(one_by_one, [i])[i], every[i]), pos[i]
+    assert torch.equal(torch.nan_to_num(one_by_one.float()), torch.nan_to_num(together.float()))
+    assert not torch.isnan(every).any()
+
+
 @pytest.mark.parametrize("T,H,N,K", [(1, 16, 128, 512), (1, 3, 20, 8), (2, 2, 64, 40), (17, 5, 130, 256), (32, 1, 16, 264), (33, 2, 128, 520), (70, 3, 40, 72)])
 def test_products_of_heads_in_steps_of_k(ops, T, H, N, K):
     """Eight steps of K asked for together (few rows) and two (many): sums of whole numbers far below 2^24, rounded once."""
