@@ -20,9 +20,9 @@
 //     memory.  With fewer than TILES_FOR_FOUR tiles four groups of four waves share a tile's K, one
 //     quarter each (a compute unit with one tile would else have a wave a SIMD and wait for every step's
 //     loads).
-// Loads stand under no condition where K is a multiple of 16 and both operands are aligned: rows beyond
-// the matrix read the last row again and are not stored.  (Behind a conditional load the compiler waits
-// for all loads in flight.)
+// Loads stand under no condition: rows beyond the matrix read the last row again and are not stored, elements
+// beyond a row its last ones and count as zeros.  (Behind a conditional load the compiler waits for all loads in flight: with
+// such loads where K was no multiple of 16, 333 rows of 1024 x 1000 took 87.7 us.)
 #include "common.h"
 
 typedef __attribute__((ext_vector_type(4))) float floatx4;
@@ -36,19 +36,33 @@ typedef __attribute__((ext_vector_type(16))) float floatx16;
 
 __host__ __device__ __forceinline__ int chunk_len(int K) { return (K + CHUNKS * FK - 1) / (CHUNKS * FK) * FK; }
 
-// four consecutive elements of a row from k on; without FULL the row may end inside them
-template <bool FULL>
+// How the rows of x and W lie: rows of whole steps, of whole fours (a four lies inside a row or behind its end), or any.
+enum { ROWS_ANY = 0, ROWS_FOURS = 1, ROWS_STEPS = 2 };
+
+// Four consecutive elements of a row from k on, zeros behind its end (row may point behind the row's start: K is what is left of it
+// from there on, perhaps less than nothing).  No load stands under a condition: one that would lie behind the end reads the row's last
+// elements instead.  (A float is aligned to its own size and no more.)
+typedef float floatx4_any __attribute__((ext_vector_type(4), aligned(4)));
+template <int ROWS>
 __device__ __forceinline__ floatx4 four_of_row(const float* __restrict__ row, int k, int K) {
-    if (FULL) return *(const floatx4*)(row + k);
+    if (ROWS == ROWS_STEPS) return *(const floatx4_any*)(row + k);
     floatx4 v;
+    if (ROWS == ROWS_FOURS) {
+        v = *(const floatx4_any*)(row + min(k, K - 4));
+        if (k >= K) v = floatx4{0.f, 0.f, 0.f, 0.f};
+        return v;
+    }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = k + e < K ? row[k + e] : 0.f;
+    for (int e = 0; e < 4; ++e) {
+        v[e] = row[min(k + e, K - 1)];
+        if (k + e >= K) v[e] = 0.f;
+    }
     return v;
 }
 
 // 16 MT rows a block (blockIdx.y: which).  Lane (g, r), g = lane / 16, r = lane % 16, brings W[n0 + r][k + 4 g .. + 4] and the same of x's row r.
 // BATCH steps are asked for at once, the next batch before the current one is multiplied.
-template <int MT, int NT, int BATCH, bool FULL>
+template <int MT, int NT, int BATCH, int ROWS>
 __global__ __launch_bounds__(64 * CHUNKS) void gemm_f32_rows_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                     const float* __restrict__ bias, float* __restrict__ out,
                                                                     int M, int N, int K, int chunk) {
@@ -80,9 +94,9 @@ __global__ __launch_bounds__(64 * CHUNKS) void gemm_f32_rows_kernel(const float*
         for (int b = 0; b < BATCH; ++b) {
             const int k = k0 + b * FK < last ? k0 + b * FK : last;
 #pragma unroll
-            for (int j = 0; j < NT; ++j) wv[buf][b][j] = four_of_row<FULL>(wrow[j], k, K - 4 * g);
+            for (int j = 0; j < NT; ++j) wv[buf][b][j] = four_of_row<ROWS>(wrow[j], k, K - 4 * g);
 #pragma unroll
-            for (int i = 0; i < MT; ++i) xv[buf][b][i] = four_of_row<FULL>(xrow[i], k, K - 4 * g);
+            for (int i = 0; i < MT; ++i) xv[buf][b][i] = four_of_row<ROWS>(xrow[i], k, K - 4 * g);
         }
     };
     auto multiply = [&](int buf, int k0) {
@@ -129,7 +143,7 @@ __global__ __launch_bounds__(64 * CHUNKS) void gemm_f32_rows_kernel(const float*
 // Tiles of 64 x 64, GROUPS (1 or 4) groups of four waves.  For a step, lane (h, r), h = lane / 32, r = lane % 32, reads
 // x[row r][4 h .. + 4] and [8 + 4 h .. + 4], and the same of W: with the instructions taking element j of the first and of
 // the second piece in turn, the order is the one above.
-template <int GROUPS, bool FULL>
+template <int GROUPS, int ROWS>
 __global__ __launch_bounds__(256 * GROUPS) void gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                 const float* __restrict__ bias, float* __restrict__ out,
                                                                 int M, int N, int K, int chunk) {
@@ -157,11 +171,11 @@ __global__ __launch_bounds__(256 * GROUPS) void gemm_f32_kernel(const float* __r
     floatx16 acc, quarter, total;
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[e] = quarter[e] = total[e] = 0.f;
-    floatx4 xv = four_of_row<FULL>(xsrc, k_of(0), K - sk), wv = four_of_row<FULL>(wsrc, k_of(0), K - sk);
+    floatx4 xv = four_of_row<ROWS>(xsrc, k_of(0), K - sk), wv = four_of_row<ROWS>(wsrc, k_of(0), K - sk);
     *(floatx4*)&xs[sat] = xv;
     *(floatx4*)&ws[sat] = wv;
-    xv = four_of_row<FULL>(xsrc, k_of(1), K - sk);
-    wv = four_of_row<FULL>(wsrc, k_of(1), K - sk);
+    xv = four_of_row<ROWS>(xsrc, k_of(1), K - sk);
+    wv = four_of_row<ROWS>(wsrc, k_of(1), K - sk);
     __syncthreads();
     int buf = 0, in_chunk = 0, chunk_no = 0;
     const int busy = k_begin >= K ? 0 : (K - k_begin + FK - 1) / FK < steps ? (K - k_begin + FK - 1) / FK : steps;
@@ -175,8 +189,8 @@ __global__ __launch_bounds__(256 * GROUPS) void gemm_f32_kernel(const float* __r
         // after it is asked for
         *(floatx4*)&xs[(buf ^ 1) * FT * FROW + sat] = xv;
         *(floatx4*)&ws[(buf ^ 1) * FT * FROW + sat] = wv;
-        xv = four_of_row<FULL>(xsrc, k_of(s + 2), K - sk);
-        wv = four_of_row<FULL>(wsrc, k_of(s + 2), K - sk);
+        xv = four_of_row<ROWS>(xsrc, k_of(s + 2), K - sk);
+        wv = four_of_row<ROWS>(wsrc, k_of(s + 2), K - sk);
         if (s < busy) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -227,29 +241,33 @@ __global__ __launch_bounds__(256 * GROUPS) void gemm_f32_kernel(const float* __r
 }
 
 template <int MT, int NT, int BATCH>
-static void launch_rows(const float* x, const float* w, const float* bias, float* out, int M, int N, int K, bool full,
+static void launch_rows(const float* x, const float* w, const float* bias, float* out, int M, int N, int K, int rows,
                         hipStream_t stream) {
     const int chunk = chunk_len(K), waves = qe_cdiv(K, chunk);
     const dim3 grid(qe_cdiv(N, 16 * NT), qe_cdiv(M, 16 * MT));
-    if (full) gemm_f32_rows_kernel<MT, NT, BATCH, true><<<grid, 64 * waves, 0, stream>>>(x, w, bias, out, M, N, K, chunk);
-    else gemm_f32_rows_kernel<MT, NT, BATCH, false><<<grid, 64 * waves, 0, stream>>>(x, w, bias, out, M, N, K, chunk);
+#define QE_F32_ROWS(R_) gemm_f32_rows_kernel<MT, NT, BATCH, R_><<<grid, 64 * waves, 0, stream>>>(x, w, bias, out, M, N, K, chunk)
+    if (rows == ROWS_STEPS) QE_F32_ROWS(ROWS_STEPS);
+    else if (rows == ROWS_FOURS) QE_F32_ROWS(ROWS_FOURS);
+    else QE_F32_ROWS(ROWS_ANY);
+#undef QE_F32_ROWS
 }
 
 int qe_gemm_f32(const float* x, const float* w, const float* bias, float* out, int M, int N, int K,
                 hipStream_t stream) {
-    const bool full = K % FK == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0;
+    const int rows = K % FK == 0 ? ROWS_STEPS : (K % 4 == 0 ? ROWS_FOURS : ROWS_ANY);
     // More than 16 rows against a very wide matrix (logits): every block would read all rows again, and the tiles are
     // enough to fill the chip (33 rows, 151936 x 1024: 467 us by rows, 235 by tiles).  Up to 128 tiles leave half of the
-    // compute units idle; blocks of 64 rows and 16 outputs do not (100 rows, 1024 x 3072: 73.5 us by tiles, 33.4 by rows).
+    // compute units idle; blocks of 64 rows and 16 outputs do not (100 rows, 1024 x 3072: 73.5 us by tiles, 33.4 by rows).  Rows that are
+    // read number by number cost a block of 64 rows more (1023 x 1001: 200 rows 33.7 us by rows, 50 by tiles, 333 65 and 51).
     const long tiles = (long)qe_cdiv(N, FT) * qe_cdiv(M, FT);
-    if (M <= 16 || (M <= 64 && N < 16384) || tiles <= 128) {
+    if (M <= 16 || (M <= 64 && N < 16384) || tiles <= (rows == ROWS_ANY ? 80 : 128)) {
         // 32 outputs a block halve the reads of x; they pay where the rows are some and the blocks enough (16 rows,
         // 6144 x 1024: 12.0 us against 14.3, 151936 x 1024: 183 against 213; 2 rows: 10.3 against 10.6, 148 against 137;
         // 16 rows, 4096 x 1024: 11.5 against 9.5)
-        if (M > 4 && M <= 16 && N >= 6144) launch_rows<1, 2, 1>(x, w, bias, out, M, N, K, full, stream);
-        else if (M <= 16) launch_rows<1, 1, 2>(x, w, bias, out, M, N, K, full, stream);
-        else if (M <= 32) launch_rows<2, 1, 2>(x, w, bias, out, M, N, K, full, stream);
-        else launch_rows<4, 1, 1>(x, w, bias, out, M, N, K, full, stream);
+        if (M > 4 && M <= 16 && N >= 6144) launch_rows<1, 2, 1>(x, w, bias, out, M, N, K, rows, stream);
+        else if (M <= 16) launch_rows<1, 1, 2>(x, w, bias, out, M, N, K, rows, stream);
+        else if (M <= 32) launch_rows<2, 1, 2>(x, w, bias, out, M, N, K, rows, stream);
+        else launch_rows<4, 1, 1>(x, w, bias, out, M, N, K, rows, stream);
         QE_LAUNCH_CHECK();
         return 0;
     }
@@ -257,10 +275,13 @@ int qe_gemm_f32(const float* x, const float* w, const float* bias, float* out, i
     dim3 grid(qe_cdiv(N, FT), qe_cdiv(M, FT));
     const int chunk = chunk_len(K);
     const bool four = tiles < TILES_FOR_FOUR;
-    if (four && full) gemm_f32_kernel<4, true><<<grid, 1024, 0, stream>>>(x, w, bias, out, M, N, K, chunk);
-    else if (four) gemm_f32_kernel<4, false><<<grid, 1024, 0, stream>>>(x, w, bias, out, M, N, K, chunk);
-    else if (full) gemm_f32_kernel<1, true><<<grid, 256, 0, stream>>>(x, w, bias, out, M, N, K, chunk);
-    else gemm_f32_kernel<1, false><<<grid, 256, 0, stream>>>(x, w, bias, out, M, N, K, chunk);
+#define QE_F32_TILES(G_, R_) gemm_f32_kernel<G_, R_><<<grid, 256 * G_, 0, stream>>>(x, w, bias, out, M, N, K, chunk)
+#define QE_F32_TILES2(R_) do { if (four) QE_F32_TILES(4, R_); else QE_F32_TILES(1, R_); } while (0)
+    if (rows == ROWS_STEPS) QE_F32_TILES2(ROWS_STEPS);
+    else if (rows == ROWS_FOURS) QE_F32_TILES2(ROWS_FOURS);
+    else QE_F32_TILES2(ROWS_ANY);
+#undef QE_F32_TILES2
+#undef QE_F32_TILES
     QE_LAUNCH_CHECK();
     return 0;
 }

@@ -36,6 +36,24 @@ def test_float32_gemm_sums_in_one_order(ops, M, N, K):
     assert torch.equal(ops.gemm(odd, w.to(DEV)), got)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 24, 4), (70, 300, 77), (333, 1023, 1001), (5, 6160, 1020), (20, 40, 36), (64, 1040, 100), (333, 1024, 1000),
+                                   (744, 640, 20), (2049, 1024, 44)])
+def test_float32_gemm_of_rows_that_end_inside_a_step(ops, M, N, K):
+    """K a multiple of 4 and no multiple of 16, and neither: by rows and by tiles, one and four groups; what lies behind a row
+    (the next one, or nothing) has no part in it, and a view that begins anywhere gives the same bits."""
+    x, w = rand(M, K, seed=K), rand(N, K, seed=K + 1)
+    want = x.double() @ w.double().t()
+    got = ops.gemm(x.to(DEV), w.to(DEV))
+    bound = 2.0 ** -24 * 2 * K ** 0.5 * (x.double().abs() @ w.double().abs().t())      # (K products, rounded K times)
+    assert ((got.cpu().double() - want).abs() <= bound + 1e-30).all()
+    wide = torch.full((M * K + 7,), float("nan"), device=DEV)
+    wide[3:3 + M * K] = x.flatten().to(DEV)
+    wide_w = torch.full((N * K + 7,), float("nan"), device=DEV)
+    wide_w[1:1 + N * K] = w.flatten().to(DEV)
+    assert torch.equal(ops.gemm(wide[3:3 + M * K].view(M, K), wide_w[1:1 + N * K].view(N, K)), got)
+    assert torch.equal(ops.gemm(x[M // 2:M // 2 + 1].to(DEV), w.to(DEV))[0], got[M // 2])
+
+
 @pytest.mark.parametrize("tile", [64, 128, 256, 512])
 @pytest.mark.parametrize("M,N", [(64 * 5, 128 * 13), (64 * 9 + 1, 128 * 7 + 64), (128 * 11 - 3, 128 * 5), (2300, 640), (130, 128 * 257 + 8)])
 def test_tiled_gemm_covers_every_tile(ops, tile, M, N):
@@ -191,7 +209,8 @@ def test_token_shift_in_whole_pieces(ops, dtype, tol, W, n):
 
 
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 2e-6), (torch.bfloat16, 2.0 ** -8)])
-@pytest.mark.parametrize("N,groups", [(4, 1), (2048, 1), (2052, 1), (8192, 1), (8, 2), (96, 3), (2048, 16), (8192, 32), (2560, 10), (8196, 1)])
+@pytest.mark.parametrize("N,groups", [(4, 1), (2048, 1), (2052, 1), (8192, 1), (8, 2), (96, 3), (2048, 16), (4096, 16), (4100, 1), (4096, 64),
+                                      (8192, 32), (2560, 10), (8196, 1)])
 def test_gated_norm_in_registers(ops, dtype, tol, N, groups):
     """A row in registers: one group, groups of one to 64 lanes, rows that end inside a thread's pieces, the longest and one more."""
     x, w, gate = rand(3, N, seed=N) * 3, 1 + 0.3 * rand(N, seed=1), rand(3, 2 * N + 8, seed=2).to(dtype)
