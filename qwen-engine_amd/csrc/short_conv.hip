@@ -189,8 +189,10 @@ extern "C" int qe_short_conv(const float* x, const float* w, float* state, const
         QE_LAUNCH_CHECK();
         return 0;
     }
-    // (whole fours everywhere; the out rows of four numbers are 8 bytes in bfloat16)
-    const bool fours = H % 4 == 0 && taps >= 2 && taps <= 8 && (((uintptr_t)x | (uintptr_t)state | (uintptr_t)out) & 15) == 0;
+    // (whole fours everywhere; the out rows of four numbers are 8 bytes in bfloat16).  Eight rows a thread are worth it where a thread a
+    // number fills the chip more than once; the sums are the same.  (Both launches, a thread a number and eight rows a thread: 64 rows
+    // of 2048 4.9 us and 9.9, 300 9.0 and 10.0, 400 10.6 and 10.2, 700 of 1024 9.7 and 9.9, 200 of 4096 10.6 and 10.1.)
+    const bool fours = (long)T * H >= 3L << 18 && H % 4 == 0 && taps >= 2 && taps <= 8 && (((uintptr_t)x | (uintptr_t)state | (uintptr_t)out) & 15) == 0;
     if (fours) {
         dim3 rgrid(qe_cdiv(H, 1024), qe_cdiv(T, CV_ROWS));
         const int rthreads = H >= 1024 ? 256 : (qe_cdiv(H / 4, 64) * 64);

@@ -485,3 +485,22 @@ def test_short_convolution_by_eight_rows(ops, taps, H):
         # (a multiply-add a tap, each rounded by 2^-24 of a partial sum, which is at most the sum of the sizes of its terms)
         assert ((got.double() - torch.cat(want)).abs() <= 2.0 ** -24 * taps * torch.cat(size)).all(), step
     assert float(state[4].min()) == 7.0
+
+
+@pytest.mark.parametrize("taps", [2, 4, 8])
+@pytest.mark.parametrize("H,lens", [(260, (1500, 0, 8, 1700)), (1028, (5, 401, 1, 377)), (157292, (2, 0, 1, 2))])
+def test_short_convolution_of_many_rows_as_of_few(ops, taps, H, lens):
+    """Steps with rows and channels enough for eight rows a thread, and the same rows a few at a time (a thread a number): the same
+    bits, in the results and in the state, over three steps of portions that end anywhere."""
+    w = rand(H, taps, seed=taps).to(DEV)
+    many = torch.zeros(5, taps - 1, H, device=DEV)
+    few = many.clone()
+    for step in range(3):
+        n = [max(0, k - step * (k > 4)) for k in lens]
+        assert sum(n) * H >= 3 << 18
+        x = torch.randn(sum(n), H, device=DEV, generator=torch.Generator(DEV).manual_seed(step))
+        seq = torch.repeat_interleave(torch.arange(4), torch.tensor(n)).int().to(DEV)
+        got = ops.short_conv(x, w, many, seq, torch.float32)
+        piece = max(1, (3 << 18) // H - 1)
+        parts = [ops.short_conv(x[a:a + piece], w, few, seq[a:a + piece], torch.float32) for a in range(0, len(x), piece)]
+        assert torch.equal(got, torch.cat(parts)) and torch.equal(many, few), step
