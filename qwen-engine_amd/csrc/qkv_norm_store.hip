@@ -19,6 +19,30 @@
 
 enum { QKN_NONE = 0, QKN_HEAD = 1, QKN_WHOLE = 2 };
 
+// The sum of v[0 .. n)'s squares by 256 threads in the order in which 1024 add them up: a thread's four sums are those of the
+// threads tid, tid + 256, ... of the larger block, each wave's four those of its waves wave, wave + 4, ...
+__device__ __forceinline__ float wide_sum(const float* v, int n, float* red) {
+    float a[4] = {0.f, 0.f, 0.f, 0.f};
+    const int tid = threadIdx.x;
+    for (int c = tid; c < n; c += 1024)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (c + 256 * j < n) a[j] += v[c + 256 * j] * v[c + 256 * j];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) a[j] = wave_sum(a[j]);
+    __syncthreads();
+    if ((tid & 63) == 0) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) red[(tid >> 6) + 4 * j] = a[j];
+    }
+    __syncthreads();
+    float r = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) r += red[i];
+    return r;
+}
+
+// wide: a norm over the whole projection adds up in the order of a block of 1024 threads
 template <typename TI, typename TA>
 __global__ __launch_bounds__(1024) void qkv_norm_store_kernel(
     const TI* __restrict__ qkv, int row_stride, const float* __restrict__ q_w, const float* __restrict__ k_w,
@@ -26,7 +50,7 @@ __global__ __launch_bounds__(1024) void qkv_norm_store_kernel(
     const float* __restrict__ v_blend, float* __restrict__ v_first, int v_first_write,
     const int* __restrict__ positions, const float* __restrict__ inv_freq, int rot_dims,
     int rot_pairs, float rot_gain, const int* __restrict__ slots, TA* __restrict__ q_out, TA* __restrict__ cache,
-    int HqT, int HkvT, int Dk, int Dv, int Dc, int P, int v_rows) {
+    int HqT, int HkvT, int Dk, int Dv, int Dc, int P, int v_rows, int wide) {
     extern __shared__ float sm[];
     __shared__ float red[16];
     const long t = blockIdx.x;
@@ -60,11 +84,17 @@ __global__ __launch_bounds__(1024) void qkv_norm_store_kernel(
     }
     // ---- q and k norm ------------------------------------------------------------------------
     if (qk_mode == QKN_WHOLE) {
-        float a = 0.f, b = 0.f;
-        for (int c = tid; c < Nq; c += nt) a += sq[c] * sq[c];
-        for (int c = tid; c < Nk; c += nt) b += sk[c] * sk[c];
-        a = block_sum(a, red);
-        b = block_sum(b, red);
+        float a, b;
+        if (nt == 1024 || !wide) {
+            a = b = 0.f;
+            for (int c = tid; c < Nq; c += nt) a += sq[c] * sq[c];
+            for (int c = tid; c < Nk; c += nt) b += sk[c] * sk[c];
+            a = block_sum(a, red);
+            b = block_sum(b, red);
+        } else {                                           // (a thread adds as four of a block of 1024 do)
+            a = wide_sum(sq, Nq, red);
+            b = wide_sum(sk, Nk, red);
+        }
         const float fq = rsqrtf(a / (float)Nq + qk_eps), fk = rsqrtf(b / (float)Nk + qk_eps);
         for (int c = tid; c < Nq; c += nt) sq[c] = sq[c] * fq * q_w[c];
         for (int c = tid; c < Nk; c += nt) sk[c] = sk[c] * fk * k_w[c];
@@ -165,8 +195,9 @@ extern "C" int qe_qkv_norm_store(const void* qkv, int row_stride, const float* q
     QE_REQUIRE(shmem <= 150 * 1024, "qkv_norm_store: a row of %zu bytes does not fit shared memory", shmem);
     const dim3 grid(T, groups);
     // A norm over the whole projection keeps a row in one block: with 1024 threads its walks through the row are a quarter as
-    // long (eight rows of 3072: 9.0 us, 14.0 with 256).  The same for many rows, so that a row's sums have one order.
-    const int threads = qk_mode == QKN_WHOLE && need >= 2048 ? 1024 : 256;
+    // long (eight rows of 3072: 5.9 us, 8.6 with 256), with many rows the blocks are what counts (2048 rows of 3072 20.5 us with 256, 29.8 with 1024; 400 9.2 with 1024, 9.8 with 256).
+    // A row's sums have one order, that of 1024 threads, either way.
+    const int wide = qk_mode == QKN_WHOLE && need >= 2048, threads = wide && T <= 512 ? 1024 : 256;
 #define QE_QNS(TI_, TA_)                                                                                                  \
     do {                                                                                                             \
         if (shmem > 48 * 1024)                                                                                       \
@@ -174,7 +205,7 @@ extern "C" int qe_qkv_norm_store(const void* qkv, int row_stride, const float* q
         qkv_norm_store_kernel<TI_, TA_><<<grid, threads, shmem, stream>>>(                                                  \
             (const TI_*)qkv, row_stride, q_w, k_w, qk_mode, qk_eps, values_from_keys, v_eps, v_norm, v_blend, v_first, \
             v_first_write, positions, inv_freq, rot_dims, rot_pairs, rot_gain, slots, (TA_*)q_out, (TA_*)cache, Hq, Hkv, Dk, Dv, \
-            Dc, P, v_rows);                                                                                          \
+            Dc, P, v_rows, wide);                                                                                    \
     } while (0)
     if (dt_i == QE_F32 && dt_a == QE_F32) QE_QNS(float, float);
     else if (dt_i == QE_BF16 && dt_a == QE_BF16) QE_QNS(bf16_t, bf16_t);

@@ -504,3 +504,26 @@ def test_short_convolution_of_many_rows_as_of_few(ops, taps, H, lens):
         piece = max(1, (3 << 18) // H - 1)
         parts = [ops.short_conv(x[a:a + piece], w, few, seq[a:a + piece], torch.float32) for a in range(0, len(x), piece)]
         assert torch.equal(got, torch.cat(parts)) and torch.equal(many, few), step
+
+
+@pytest.mark.parametrize("hq,hkv,D", [(16, 4, 128), (30, 6, 72), (24, 8, 96)])
+def test_whole_norms_in_one_order(ops, hq, hkv, D):
+    """The norm over a whole projection by 1024 threads (few rows) and by 256 (many): a row gets the same bits."""
+    T = 700
+    y = rand(T, (hq + 2 * hkv) * D, seed=D).bfloat16().to(DEV)
+    wq, wk = 1 + rand(hq * D, seed=1).to(DEV) / 4, 1 + rand(hkv * D, seed=2).to(DEV) / 4
+    at = torch.arange(T, dtype=torch.int32, device=DEV)
+
+    def run(rows):
+        cache = torch.zeros(T // 16 + 1, 2, hkv, 16, D, dtype=torch.bfloat16, device=DEV)
+        q = ops.qkv_norm_store(y[rows], hq, hkv, D, D, cache, at[rows], qk_norm=ops.QK_NORM_WHOLE, q_weight=wq, k_weight=wk, qk_eps=1e-5)
+        return q, cache
+
+    q, cache = run(slice(0, T))
+    some = slice(130, 140)
+    q_some, cache_some = run(some)
+    assert torch.equal(q_some, q[some])
+    here = cache_some.abs().sum((0, 1, 2, 4)) > 0
+    assert here.any()
+    for t in range(130, 140):
+        assert torch.equal(cache_some[t // 16, :, :, :, :][0][:, t % 16], cache[t // 16][0][:, t % 16]), t
