@@ -575,6 +575,7 @@ extern "C" int qe_gated_norm(const float* o, const float* weight, const void* ga
 #define QE_GN(TG_, TO_)                                                                                          \
     do {                                                                                                         \
         if (vec && N <= 2048) gated_norm_regs_kernel<TG_, TO_, 2><<<T, 256, 0, stream>>>(QE_GN_ARGS(TG_, TO_), GL); \
+        else if (vec && N <= 4096) gated_norm_regs_kernel<TG_, TO_, 4><<<T, 256, 0, stream>>>(QE_GN_ARGS(TG_, TO_), GL); \
         else if (vec) gated_norm_regs_kernel<TG_, TO_, 8><<<T, 256, 0, stream>>>(QE_GN_ARGS(TG_, TO_), GL);      \
         else gated_norm_kernel<TG_, TO_><<<T, threads, 0, stream>>>(QE_GN_ARGS(TG_, TO_), groups);               \
     } while (0)
