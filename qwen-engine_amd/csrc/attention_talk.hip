@@ -908,7 +908,11 @@ extern "C" int qe_attention_talk(const void* q, void* out, long out_stride, floa
         const int wph_shift = Hkv <= 4 ? 2 : (Hkv <= 8 ? 1 : 0);
         const int DP = d <= 64 ? 64 : 128;
         const size_t bytes = (size_t)talk_wide_layout(Hq, DP, 1 << wph_shift).total * sizeof(float);
-        if (dt_a == QE_BF16 && d <= 128 && Dc % 8 == 0 && ((unsigned long)cache & 15) == 0 && Hkv <= 16 && G <= 8 && bytes <= 150 * 1024) {
+        // (with one key/value head four of the sixteen waves work: for more than four queries many rows are better off in the kernel
+        // with several rows a block, which reads the keys once for them: 8 heads of 128 on 1, 235 rows 66 us here and 45 there, 1000 402
+        // and 326, 2000 without chunks 1361 and 946; heads of 64, 235 rows 43 and 35, but 400 54 and 81, 1000 180 and 274)
+        const bool one = Hkv == 1 && G > 4 && !tokens && n_tokens >= 192 && (DP == 128 || n_tokens < 256);
+        if (dt_a == QE_BF16 && !one && d <= 128 && Dc % 8 == 0 && ((unsigned long)cache & 15) == 0 && Hkv <= 16 && G <= 8 && bytes <= 150 * 1024) {
 #define QE_TALK_WIDE3(LPK_, GM_, SH_)                                                                                      \
     do {                                                                                                             \
         if (bytes > 48 * 1024)                                                                                       \

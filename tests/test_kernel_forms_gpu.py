@@ -527,3 +527,30 @@ def test_whole_norms_in_one_order(ops, hq, hkv, D):
     assert here.any()
     for t in range(130, 140):
         assert torch.equal(cache_some[t // 16, :, :, :, :][0][:, t % 16], cache[t // 16][0][:, t % 16]), t
+
+
+@pytest.mark.parametrize("D,T", [(128, 200), (128, 700), (64, 200), (64, 300)])
+def test_talking_heads_of_one_key_value_head(ops, D, T):
+    """Eight queries on one key/value head: many rows go several a block, few a block each; both against 64 bits."""
+    hq, P = 8, 16
+    q, k, v = rand(T, hq, D, seed=1).bfloat16().to(DEV), rand(T, D, seed=2).bfloat16().to(DEV), rand(T, D, seed=3).bfloat16().to(DEV)
+    talk, bias = (torch.eye(hq) + 0.1 * rand(hq, hq, seed=4)).to(DEV), rand(40, hq, seed=5).to(DEV)
+    cache = torch.full((T // P + 1, 2, 1, P, D), float("nan"), dtype=torch.bfloat16, device=DEV)
+    cache[torch.arange(T) // P, 0, 0, torch.arange(T) % P] = k
+    cache[torch.arange(T) // P, 1, 0, torch.arange(T) % P] = v
+    pos = torch.arange(T, dtype=torch.int32, device=DEV)
+    seq, table = torch.zeros_like(pos), torch.arange(T // P + 1, dtype=torch.int32, device=DEV)[None]
+    kw = dict(chunk=1024, bias=bias, talk=talk)
+    every = ops.attention_talk(q, cache, pos, seq, table, D ** -0.5, D, D, **kw)
+    few = torch.zeros_like(every)
+    some = pos[T - 20:].contiguous()
+    ops.attention_talk(q, cache, pos, seq, table, D ** -0.5, D, D, out=few, tokens=some, **kw)
+    d = (pos[:, None] - pos[None]).long()
+    s = (q.double().transpose(0, 1) @ k.double().t()) * D ** -0.5 + bias.double()[d.clamp(0, 39)].permute(2, 0, 1)
+    s = (talk.double() @ s.reshape(hq, -1)).view(hq, T, T).masked_fill(d < 0, float("-inf"))
+    w = torch.softmax(s, -1)
+    want = (w @ v.double()).transpose(0, 1).reshape(T, -1)
+    # (a bfloat16 rounding of each result; the scores' own errors, some 2^-20, move the weights by as much)
+    bound = want.abs() * 2.0 ** -8 + 2.0 ** -17 * v.double().abs().max()
+    assert ((every.double() - want).abs() <= bound).all()
+    assert ((few.double() - want).abs() <= bound)[T - 20:].all()
