@@ -42,6 +42,7 @@ static AttnTail make_tail(int Hq, int D, const void* out, long out_stride, int d
 
 int qe_attention_prefill_segment_keys(long blocks, int max_keys);
 int qe_attention_prefill_segments(long blocks);
+int qe_attention_prefill_choose_groups(long blocks, long rows, int window, int max_keys);
 int qe_attention_prefill_uncut_keys();
 size_t qe_attention_prefill_workspace(int num_tiles, int Hq, int Hkv, int D, int segments);
 
@@ -76,6 +77,13 @@ extern "C" int qe_attention_prefill_plan_segments(int num_tiles, int Hq, int Hkv
     if (num_tiles <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv) return 1;
     const int R = qe_attention_prefill_tile_rows(Hq, Hkv);
     return qe_attention_prefill_segments((long)(num_tiles / 4) * Hkv * ((Hq / Hkv) / (32 / R)));
+}
+
+// The wave groups a block that the prefill kernel chooses for num_tiles tiles whose rows see at most max_keys keys (0: not known).
+extern "C" int qe_attention_prefill_plan_groups(int num_tiles, int Hq, int Hkv, int window, int max_keys) {
+    if (num_tiles <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv) return 1;
+    const int R = qe_attention_prefill_tile_rows(Hq, Hkv);
+    return qe_attention_prefill_choose_groups((long)(num_tiles / 4) * Hkv * ((Hq / Hkv) / (32 / R)), (long)num_tiles * R, window, max_keys);
 }
 
 // up to this many keys the plan is never to cut

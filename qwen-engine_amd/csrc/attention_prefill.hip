@@ -587,6 +587,17 @@ int qe_attention_prefill_segment_keys(long blocks, int max_keys) {
     return seg >= max_keys ? 0 : seg;
 }
 
+// Wave groups a block: two where the blocks do not fill the compute units anyway, and up to twice as many blocks as units where the
+// longest walk decides: one prompt from its start, or several beside one that is as long as they together.  (rows: 32 a tile, those
+// that fill a tile up among them.  One group and two, 32 heads of 128 on 8: 2048 rows from the start 64 and 58 us, 16 prompts of 128 rows
+// 18 and 25, four of 512 31 and 36, 512 rows each behind 4096 keys 185 and 189; 16 heads on 8, 4096 rows 134 and 109, eight prompts of
+// 256 beside one of 2000 63 and 52, the same behind 4096 keys 195 and 215; 64 heads, 1000 rows 37 and 39.)
+int qe_attention_prefill_choose_groups(long blocks, long rows, int window, int max_keys) {
+    const int units = qe_compute_units();
+    if (blocks <= units) return 2;
+    return blocks <= 2L * units && window == 0 && max_keys >= 1536 && 5L * max_keys >= 2 * rows && 4L * max_keys <= 5 * rows ? 2 : 1;
+}
+
 size_t qe_attention_prefill_workspace(int num_tiles, int Hq, int Hkv, int D, int segments) {
     const int R = qe_attention_prefill_tile_rows(Hq, Hkv);
     const long blocks = (long)(num_tiles / 4) * Hkv * ((Hq / Hkv) / (32 / R));
@@ -635,10 +646,7 @@ int qe_attention_prefill(const void* q, void* out, const void* cache, const int*
     dim3 mgrid(Hkv * waves_per_kv, D / 32, num_tiles / 4);
     const float scale_log2 = softcap > 0.f ? 1.f : scale * 1.4426950408889634f;
     const float cap_in = softcap > 0.f ? scale * 2.f * 1.4426950408889634f / softcap : 0.f, cap_out = softcap * 1.4426950408889634f;
-    // two groups a block where the blocks do not fill the compute units more than twice anyway: the longest walk decides
-    // (whole prompts of 2048 tokens, 32 heads: 512 blocks, 69 us with one group, 61 with two; 3000 tokens, 16 heads, 376
-    // blocks: 92 and 67; 3000 tokens, 32 heads, 752 blocks: 100 and 119).  (groups: 0 = choose, 1 or 2)
-    if (groups == 0) groups = (long)grid.x * grid.z <= 2 * qe_compute_units() ? 2 : 1;
+    if (groups == 0) groups = qe_attention_prefill_choose_groups((long)grid.x * grid.z, (long)num_tiles * R, window, max_keys);
     QE_REQUIRE(groups == 1 || groups == 2, "prefill attention: %d groups a block", groups);
 #define QE_PREFILL_CAP(D_, NG_, CAP_)                                                               \
     attention_prefill_kernel<D_, NG_, CAP_><<<grid, 256 * NG_, 0, stream>>>(                        \

@@ -68,6 +68,7 @@ def load_library():
         "qe_attention_prefill_workspace_bytes_for": [i32, i32, i32, i32, i32],
         "qe_attention_prefill_plan": [i32, i32, i32, i32],
         "qe_attention_prefill_plan_uncut_keys": [],
+        "qe_attention_prefill_plan_groups": [i32, i32, i32, i32, i32],
         "qe_attention_prefill_workspace_bytes": [i32, i32, i32, i32, i32, i32],
         "qe_attention_decode_run": [vp, vp, vp, vp, i32, vp, vp, vp, i32, vp, i32, i32, i32, i32, f32, i32, i32, i32, f32, i32, i32, vp, i64,
                                     i64, i32, vp, vp, i64, i32, vp],
@@ -781,6 +782,12 @@ def prefill_uncut_keys() -> int:
     """Up to this many keys a row sees, the prefill attention kernel never cuts its walks into
     segments of keys."""
     return load_library().qe_attention_prefill_plan_uncut_keys()
+
+
+def prefill_groups_of(num_tiles: int, num_heads: int, num_kv_heads: int, window: int, max_keys: int) -> int:
+    """The wave groups a block (1 or 2) that the prefill attention kernel chooses for ``num_tiles`` tiles whose rows see at most
+    ``max_keys`` keys (0: not known)."""
+    return load_library().qe_attention_prefill_plan_groups(num_tiles, num_heads, num_kv_heads, window, max_keys)
 
 
 def attention(q: torch.Tensor, cache: torch.Tensor, positions: torch.Tensor, tok_seq: torch.Tensor,

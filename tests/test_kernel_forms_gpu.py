@@ -554,3 +554,17 @@ def test_talking_heads_of_one_key_value_head(ops, D, T):
     bound = want.abs() * 2.0 ** -8 + 2.0 ** -17 * v.double().abs().max()
     assert ((every.double() - want).abs() <= bound).all()
     assert ((few.double() - want).abs() <= bound)[T - 20:].all()
+
+
+def test_prefill_attention_takes_two_groups_where_one_walk_decides(ops):
+    """Blocks once to twice the compute units: two wave groups for one prompt from its start or beside short ones, one for walks of
+    one length, whether short or deep in a context, for windows and where the keys are not known; two for few blocks."""
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    rows = ops.prefill_tile_rows(32, 8)
+    tiles = lambda n: -(-n // (4 * rows)) * 4
+    blocks = lambda n: tiles(n) // 4 * 8 * (4 // (32 // rows))
+    assert units < blocks(2048) <= 2 * units and blocks(1000) <= units < 2 * units < blocks(3000)
+    groups = lambda n, keys, window=0: ops.prefill_groups_of(tiles(n), 32, 8, window, keys)
+    assert groups(2048, 2048) == 2 and groups(2048, 1600) == 2
+    assert groups(2048, 128) == groups(2048, 512) == groups(2048, 8192) == groups(2048, 0) == groups(2048, 2048, 512) == 1
+    assert groups(1000, 100) == groups(1000, 30000) == 2 and groups(3000, 3000) == 1
