@@ -249,9 +249,9 @@ __global__ __launch_bounds__(256) void latent_attention_mfma_kernel(
 // A block per (token, head) and 256 / SG numbers of the output: the splits' partial results.  Lane s of every wave fetches split s's
 // maximum and sum; the splits are cut into SG parts, each summed by a part of the threads, eight asked for at a time and before the
 // weights are there, and the parts' sums are added in their order.  Few heads are bound by the trips to memory: SG = 4, one
-// trip for 32 splits (16 heads of 512 numbers: 4.6 us, 6.7 with a block a head that fetched the weights first and went
-// through its numbers twice).
-template <int SG>
+// trip for 32 splits (16 heads of 512 numbers: 3.9 us, 6.7 with a block a head that fetched the weights first and went
+// through its numbers twice).  SG = 1, many heads: a thread adds up the four parts one after the other, to the same bits.
+template <int SG>     // 4 or 1
 __global__ __launch_bounds__(256) void latent_attention_merge_kernel(const float* __restrict__ part_acc,
                                                                      const float* __restrict__ part_ml,
                                                                      bf16_t* __restrict__ out, int NS, int R, int RP,
@@ -267,25 +267,39 @@ __global__ __launch_bounds__(256) void latent_attention_merge_kernel(const float
     const float ls = lane < NS ? pm[2 * lane + 1] : 0.f;
     const float sk = sink ? sink[th % H] : -INFINITY;
     const float* pa = part_acc + th * NS * RP + (d < R ? d : 0);
-    const int per = (NS + SG - 1) / SG, s_begin = part * per, s_end = min(NS, s_begin + per);
-    float w = 0.f, M = 0.f, a = 0.f;
+    const auto weight_of = [](float v, int split) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), split)); };
+    const int per = (NS + 3) / 4, s_begin = SG > 1 ? part * per : 0, s_end = SG > 1 ? min(NS, s_begin + per) : NS;
+    int next = per;                                        // (SG = 1: the first split of the next part)
+    float w = 0.f, M = 0.f, a = 0.f, before = 0.f;
     for (int s0 = s_begin; s0 < s_end || s0 == s_begin; s0 += 8) {
         float v[8];
+        if (s0 + 8 <= s_end || SG > 1) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = pa[(long)min(s0 + u, NS - 1) * RP];
+            for (int u = 0; u < 8; ++u) v[u] = pa[(long)min(s0 + u, NS - 1) * RP];
+        } else {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = s0 + u < s_end ? pa[(long)(s0 + u) * RP] : 0.f;
+        }
         if (s0 == s_begin) {
             M = fmaxf(wave_max(ms), sk);
             w = ms == -INFINITY ? 0.f : __expf(ms - M);
         }
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-            const float f = __shfl(w, s0 + u, 64);
+            if (s0 + u >= s_end) break;                    // (all this is the same for the whole wave)
+            const float f = weight_of(w, s0 + u);
+            if (SG == 1 && s0 + u == next) {
+                before += a;
+                a = 0.f;
+                next += per;
+            }
             // (a split without keys left no numbers: whatever lies there does not count)
-            if (s0 + u < s_end && f != 0.f) a = fmaf(f, v[u], a);
+            if (f != 0.f) a = fmaf(f, v[u], a);
         }
     }
+    if (SG == 1) a += before;
     float L = sink ? __expf(sk - M) : 0.f;
-    for (int s = 0; s < NS; ++s) L = fmaf(__shfl(w, s, 64), __shfl(ls, s, 64), L);      // in the order of the splits
+    for (int s = 0; s < NS; ++s) L = fmaf(weight_of(w, s), weight_of(ls, s), L);        // in the order of the splits
     if (SG > 1) {
         red[part][at] = a;
         __syncthreads();

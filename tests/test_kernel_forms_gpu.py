@@ -379,6 +379,20 @@ def test_latent_attention_of_single_tokens(ops, H, R, dr, window):
             assert ((got[j] - want).abs() <= 2.0 ** -8 * (w @ c[:, :R].abs() + want.abs())).all(), (i, rows[:2])
 
 
+@pytest.mark.parametrize("H,R,dr", [(32, 512, 64), (48, 256, 64), (16, 512, 64)])
+@pytest.mark.parametrize("window", [0, 700])
+def test_latent_splits_are_merged_in_one_order(ops, H, R, dr, window):
+    """Up to eight single tokens have as many splits each as one; the merge by four parts a thread group (few heads) and by one thread
+    (many) adds them up in the same order: a token gets the same bits alone and with seven others."""
+    before = [0, 30, 200, 640, 900, 1100, 1500, 77]
+    cache, table, pos, seq, own = latent_rows(before, [1] * len(before), R, dr, 16, 50)
+    q = rand(len(before), H, R + dr, seed=9).bfloat16().to(DEV)
+    scale = (R + dr) ** -0.5
+    every = ops.latent_attention(q, cache, pos, seq, table, R, scale, window=window)
+    for i in range(len(before)):
+        assert torch.equal(ops.latent_attention(q[i:i + 1], cache, pos[i:i + 1], seq[i:i + 1], table, R, scale, window=window)[0], every[i]), i
+
+
 @pytest.mark.parametrize("tile", [64, 128, 256, 512])
 @pytest.mark.parametrize("page", [16, 64])
 def test_qkv_product_stores_values_behind_other_rows(ops, tile, page):
