@@ -29,7 +29,8 @@ from .attention import prefill_tiles
 from .base import CacheBinding, Runtime, TensorInfo
 from .registry import build_part, register_part
 
-# Bytes that the expanded keys and values of a step may take (they are gone when the layer is done)
+# Bytes that the gathered cache rows and the expanded keys and values of a step may take, all its portions together (they are gone
+# when the layer is done)
 EXPAND_MAX_BYTES = 1 << 30
 
 
@@ -70,18 +71,22 @@ class LatentAttention:
     def mixed_graph_extras(rows: int, tokens: int, key, device, dynamic: torch.Tensor) -> dict:
         return {}
 
+    def _seen(self, rows: int, keys: int) -> int:
+        """How many of ``keys`` positions the last ``rows`` of them see."""
+        return min(keys, self.window + rows - 1) if self.window else keys
+
+    def _expanded_bytes(self, keys: int) -> int:
+        return 2 * (-(-keys // 64) * 64) * (self.h * (self.dn + self.dv) + self.r + self.dr)
+
     def _pays(self, rows: int, keys: int) -> bool:
         """True if rows that are the last of ``keys`` positions are better off with expanded keys: every key costs R (Dn + Dv)
         multiply-adds a head at some 500 TFLOP/s, which every pair of a row and a key pays back with the difference of
         2 R + Dr at 200 and Dn + Dr + Dv at 350 (the rates of the kernels; half as much again asked for, the launches being more)."""
-        if self.window:
-            keys = min(keys, self.window + rows - 1)
-            pairs = rows * min(self.window, keys - rows / 2.0)
-        else:
-            pairs = rows * (keys - rows / 2.0)
+        seen = self._seen(rows, keys)
+        pairs = rows * min(self.window, seen - rows / 2.0) if self.window else rows * (seen - rows / 2.0)
         a_key = self.r * (self.dn + self.dv) / 500.0
         a_pair = (2 * self.r + self.dr) / 200.0 - (self.dn + self.dr + self.dv) / 350.0
-        return a_pair > 0 and pairs * a_pair > 1.5 * keys * a_key and 2 * keys * self.h * (self.dn + self.dv) <= EXPAND_MAX_BYTES
+        return a_pair > 0 and pairs * a_pair > 1.5 * seen * a_key
 
     def _expansion(self, ctx) -> Optional[dict]:
         """Which of the step's rows see expanded keys, made once per step for all layers of the same sizes: the rows' ranges, the
@@ -91,16 +96,20 @@ class LatentAttention:
         key = ("latent_attention.expansion", self.r, self.dn, self.dr, self.dv, self.h, self.window)
         if key not in ctx.memo:
             ex = next((ctx.extras[cls] for cls in type(self).__mro__ if cls in ctx.extras), {})
-            portions: List[Tuple[int, int, int]] = []                # (first row, rows, keys)
+            wanted: List[Tuple[int, int, int]] = []                  # (first row, rows, keys)
             if "keys" in ex:                                         # a recorded portion
                 n, k = ctx.num_tokens, ex["keys"]
                 if self._pays(n, k):
-                    portions = [(0, n, min(k, self.window + n - 1) if self.window else k)]
+                    wanted.append((0, n, self._seen(n, k)))
             elif "eager" in ex:
                 for s in ctx.seqs:
-                    k = s.kv_before + s.q_len
-                    if s.q_len > 1 and self._pays(s.q_len, k):
-                        portions.append((s.q_start, s.q_len, k - (max(0, s.kv_before - self.window + 1) if self.window else 0)))
+                    if s.q_len > 1 and self._pays(s.q_len, s.kv_before + s.q_len):
+                        wanted.append((s.q_start, s.q_len, self._seen(s.q_len, s.kv_before + s.q_len)))
+            portions, room = [], EXPAND_MAX_BYTES
+            for first, rows, keys in wanted:
+                if self._expanded_bytes(keys) <= room:
+                    room -= self._expanded_bytes(keys)
+                    portions.append((first, rows, keys))
             ctx.memo[key] = self._lists(ctx, portions) if portions else None
         return ctx.memo[key]
 
