@@ -47,7 +47,8 @@ class LatentAttention:
 
     @staticmethod
     def portion_graph_key(tokens: int, keys: int) -> int:
-        """The portion's keys rounded up to its rows times a power of two: few recorded steps for a prompt in many portions."""
+        """The portion's keys rounded up to its rows times a power of two: few recorded steps for a prompt in many portions (each
+        serves the places of more than half as many keys)."""
         n = int(tokens)
         while n < keys:
             n *= 2
@@ -78,15 +79,16 @@ class LatentAttention:
     def _expanded_bytes(self, keys: int) -> int:
         return 2 * (-(-keys // 64) * 64) * (self.h * (self.dn + self.dv) + self.r + self.dr)
 
-    def _pays(self, rows: int, keys: int) -> bool:
-        """True if rows that are the last of ``keys`` positions are better off with expanded keys: every key costs R (Dn + Dv)
-        multiply-adds a head at some 500 TFLOP/s, which every pair of a row and a key pays back with the difference of
-        2 R + Dr at 200 and Dn + Dr + Dv at 350 (the rates of the kernels; half as much again asked for, the launches being more)."""
+    def _pays(self, rows: int, keys: int, expanded: int = 0) -> bool:
+        """True if rows that are the last of ``keys`` positions are better off with expanded keys: every key (``expanded`` of them,
+        if those are more than the rows see) costs R (Dn + Dv) multiply-adds a head at some 500 TFLOP/s, which every pair of a
+        row and a key pays back with the difference of 2 R + Dr at 200 and Dn + Dr + Dv at 350 (the rates of the kernels; half as
+        much again asked for, the launches being more)."""
         seen = self._seen(rows, keys)
         pairs = rows * min(self.window, seen - rows / 2.0) if self.window else rows * (seen - rows / 2.0)
         a_key = self.r * (self.dn + self.dv) / 500.0
         a_pair = (2 * self.r + self.dr) / 200.0 - (self.dn + self.dr + self.dv) / 350.0
-        return a_pair > 0 and pairs * a_pair > 1.5 * seen * a_key
+        return a_pair > 0 and pairs * a_pair > 1.5 * max(seen, expanded) * a_key
 
     def _expansion(self, ctx) -> Optional[dict]:
         """Which of the step's rows see expanded keys, made once per step for all layers of the same sizes: the rows' ranges, the
@@ -97,9 +99,9 @@ class LatentAttention:
         if key not in ctx.memo:
             ex = next((ctx.extras[cls] for cls in type(self).__mro__ if cls in ctx.extras), {})
             wanted: List[Tuple[int, int, int]] = []                  # (first row, rows, keys)
-            if "keys" in ex:                                         # a recorded portion
+            if "keys" in ex:                                         # a recorded portion: for all the places that replay it
                 n, k = ctx.num_tokens, ex["keys"]
-                if self._pays(n, k):
+                if self._pays(n, k if k == n else k // 2 + 1, self._seen(n, k)):
                     wanted.append((0, n, self._seen(n, k)))
             elif "eager" in ex:
                 for s in ctx.seqs:

@@ -57,3 +57,23 @@ def test_few_rows_and_single_tokens_stay_folded(part, window):
     assert plan(part(window), [(0, 2048), (10, 1)])["others"] == [(2048, 2049)]
     seen = 64 * plan(part(window), [(4000, 512)])["owner"].shape[0]
     assert seen == (64 * -(-4512 // 64) if not window else 64 * -(-811 // 64))
+
+
+@pytest.mark.parametrize("window", [None, 300, 5000])
+@pytest.mark.parametrize("rows", [64, 96, 120, 128, 160, 256, 512, 2048])
+def test_a_recorded_portion_pays_at_every_place_it_serves(part, rows, window):
+    """Recorded for its rows times a power of two, it expands that many keys wherever it is replayed: with half as many keys seen it
+    must still be worth it."""
+    p = part(window)
+    for doublings in range(7):
+        keys = rows << doublings
+        got = plan(p, recorded=(rows, keys))
+        served = [n for n in range(rows, keys + 1) if p.portion_graph_key(rows, n) == keys]
+        assert served[-1] == keys and len(served) == (1 if doublings == 0 else keys // 2)
+        for n in (served[0], served[-1]):
+            seen, expanded = p._seen(rows, n), p._seen(rows, keys)
+            pairs = sum(min(i + 1, window or i + 1) for i in range(n - rows, n))
+            gain = pairs * ((2 * 512 + 64) / 200 - 320 / 350)        # (microseconds' worth of folded minus expanded pairs, and of keys)
+            assert got is None or gain > expanded * 512 * 256 / 500
+            assert got is None or 64 * got["owner"].shape[0] >= seen
+    assert plan(p, recorded=(512, 2048)) is not None
