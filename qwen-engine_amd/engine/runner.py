@@ -224,12 +224,23 @@ class ModelRunner:
                 self._graph_seen.pop(key, None)
             before = torch.cuda.memory_allocated(self.rt.device)
             rec = record()
-            rec["bytes"] = max(0, torch.cuda.memory_allocated(self.rt.device) - before)
+            rec["bytes"] = max(rec.pop("held"), torch.cuda.memory_allocated(self.rt.device) - before)
             self.graphs_recorded += 1
         self._graphs[key] = rec                                # dicts keep insertion order: the oldest use comes first
         while len(self._graphs) > 1 and (len(self._graphs) > self.MAX_GRAPHS or self.graph_bytes() > self.graph_memory_bytes):
             self._graphs.pop(next(iter(self._graphs)))
         return rec
+
+    def _capture(self, run, stream):
+        """Records ``run`` on ``stream``: the graph, its results, and the device memory that the recording keeps for its
+        replays, what was given back while it ran included."""
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            before = torch.cuda.memory_reserved(self.rt.device)
+            out = run()
+            held = torch.cuda.memory_reserved(self.rt.device) - before
+        torch.cuda.synchronize()
+        return graph, out, max(0, held)
 
     def graph_bytes(self) -> int:
         """Device memory that the recorded steps hold (their buffers, activations and workspaces)."""
@@ -706,13 +717,10 @@ class ModelRunner:
             run()
         stream.synchronize()
         ctx.memo.clear()                          # (what the parts made for the first run is made again inside the graph)
-        graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph, stream=stream):
-            logits, tokens = run()
-        torch.cuda.synchronize()
+        graph, (logits, tokens), held = self._capture(run, stream)
         event = torch.cuda.Event()
         event.record()
-        return {"graph": graph, "ctx": ctx, "host": host, "host_np": host.numpy(), "meta": meta, "logits": logits, "tokens": tokens,
+        return {"graph": graph, "held": held, "ctx": ctx, "host": host, "host_np": host.numpy(), "meta": meta, "logits": logits, "tokens": tokens,
                 "event": event, "none": np.full(cap, -1, dtype=np.int32), "zero": np.zeros(cap, dtype=np.int32)}
 
     # ---- one prompt portion through a recorded graph ----------------------------------------
@@ -801,13 +809,10 @@ class ModelRunner:
         with torch.cuda.stream(stream):
             run()                                 # (what the parts keep for the step, ctx.memo, is made here)
         stream.synchronize()
-        graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph, stream=stream):
-            logits, tokens = run()
-        torch.cuda.synchronize()
+        graph, (logits, tokens), held = self._capture(run, stream)
         event = torch.cuda.Event()
         event.record()
-        return {"graph": graph, "ctx": ctx, "host": host, "host_np": host.numpy(), "meta": meta, "logits": logits, "tokens": tokens,
+        return {"graph": graph, "held": held, "ctx": ctx, "host": host, "host_np": host.numpy(), "meta": meta, "logits": logits, "tokens": tokens,
                 "event": event, "none": np.full(cap, -1, dtype=np.int32), "zero": np.zeros(cap, dtype=np.int32)}
 
     def _record_decode_graph(self, B: int, part_keys: tuple, cap: int):
@@ -857,14 +862,11 @@ class ModelRunner:
         with torch.cuda.stream(stream):
             run()
         stream.synchronize()
-        graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph, stream=stream):
-            logits, tokens = run()
-        torch.cuda.synchronize()
+        graph, (logits, tokens), held = self._capture(run, stream)
         event = torch.cuda.Event()
         event.record()
         # (the context is kept with the graph: what the parts made for the recorded step, their
         # graph_extras, is read by every replay)
-        return {"graph": graph, "ctx": ctx, "host": host, "host_np": host.numpy(), "meta": meta, "logits": logits, "tokens": tokens,
+        return {"graph": graph, "held": held, "ctx": ctx, "host": host, "host_np": host.numpy(), "meta": meta, "logits": logits, "tokens": tokens,
                 "event": event, "iota": np.arange(B, dtype=np.int32), "none": np.full(cap, -1, dtype=np.int32),
                 "zero": np.zeros(cap, dtype=np.int32)}

@@ -30,7 +30,7 @@ from .base import CacheBinding, Runtime, TensorInfo
 from .registry import build_part, register_part
 
 # Bytes that the gathered cache rows and the expanded keys and values of a step may take, all its portions together (they are gone
-# when the layer is done)
+# when the layer is done; a recorded step keeps them for its replays, and they count among what it holds)
 EXPAND_MAX_BYTES = 1 << 30
 
 
