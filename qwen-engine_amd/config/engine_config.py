@@ -25,7 +25,8 @@ class EngineConfig:
     graph_record_after: int = 2      # a step with prompt tokens is recorded when its shape is met for this many times
     graph_memory_bytes: int = 8 << 30  # recorded steps may hold this much device memory; the least recently used go first
     # num_blocks None and this set: the pool takes this fraction of the device memory that is free once
-    # the weights are loaded, less graph_memory_bytes (the reference has the fixed formula only, main.py:23)
+    # the weights are loaded, less graph_memory_bytes (the reference has the fixed formula only, main.py:23).  The rest is what a
+    # step's own tensors have: its activations, partial products up to 512 MiB, expanded latent keys up to 1 GiB
     gpu_memory_fraction: Optional[float] = None
 
     def pages_per_group(self, free_bytes: Optional[int] = None, bytes_per_page: int = 0) -> int:

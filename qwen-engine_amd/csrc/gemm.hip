@@ -94,7 +94,8 @@ extern "C" int qe_gemm_partial_splits(int M, int N, int K) {
 // cuts that leaves 512 of K to a part; the cuts give every compute unit as many tiles as the others (800 rows against 5120 x 25600 with the norm
 // behind it: 232 us in three cuts of 256 x 256, 347 as a plain product; 528 rows against 4096 x 12288: 81 in three
 // of 128 x 128, 139 plain; 8192 rows against 5120 x 25600: 1851 in two, 2082 plain; 1300 rows against 4096 x 4096 stay plain:
-// 65, in two cuts 74).  Parts beyond 2^28 numbers (1 GiB) are not asked for.
+// 65, in two cuts 74).  Parts beyond 2^27 numbers (512 MiB, what a pool of pages that takes nearly all memory should leave a step) are
+// not asked for.
 extern "C" int qe_gemm_branch_splits(int M, int N, int K, int dt_a, int dt_w) {
     if (qe_gemm_skinny_ok(M, N, K, dt_a, dt_w) || (M <= 64 && tiled_for_few_rows(M, N, K, dt_a, dt_w))) {
         const int s = qe_gemm_partial_splits(M, N, K);
@@ -106,7 +107,7 @@ extern "C" int qe_gemm_branch_splits(int M, int N, int K, int dt_a, int dt_w) {
     int best_s = 1;
     float best = 0.f;
     for (int s = 1; s <= 6; ++s) {
-        if (s > 1 && (K < 512 * s || (long)s * M * N > (1L << 28))) break;
+        if (s > 1 && (K < 512 * s || (long)s * M * N > (1L << 27))) break;
         if ((long)(s - 1) * (qe_cdiv(qe_cdiv(K, s), 64) * 64) >= K) continue;   // every cut has some of K
         int tile;
         const float t = qe_gemm_mfma_shape(M, N, K, s, &tile) + (s == 1 ? 4.f : 8.f * (float)s) * (float)M * (float)N / 4e6f;

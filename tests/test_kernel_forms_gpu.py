@@ -582,3 +582,12 @@ def test_prefill_attention_takes_two_groups_where_one_walk_decides(ops):
     assert groups(2048, 2048) == 2 and groups(2048, 1600) == 2
     assert groups(2048, 128) == groups(2048, 512) == groups(2048, 8192) == groups(2048, 0) == groups(2048, 2048, 512) == 1
     assert groups(1000, 100) == groups(1000, 30000) == 2 and groups(3000, 3000) == 1
+
+
+def test_parts_of_a_product_stay_within_their_bytes(ops):
+    """However many rows a step has, the partial products that are asked for take 512 MiB at the most."""
+    for n, k in ((5120, 25600), (4096, 12288), (5120, 8192), (1024, 3072)):
+        w = torch.empty(n, k, dtype=torch.bfloat16, device=DEV)
+        for rows in (1, 64, 512, 2048, 8192, 12288, 16384, 32768, 65536):
+            splits = ops.gemm_branch_splits_for(rows, w, torch.bfloat16)
+            assert splits * rows * n * 4 <= 512 << 20, (rows, n, k, splits)
