@@ -774,6 +774,12 @@ static int first_columns(int M, int N, int K, bool largest = true) {
     return cut;
 }
 
+// The same for a caller that wants to know: the number of columns that a product of more than 64 rows gives a launch of their own, or 0
+// (gelu: of one with that epilogue).
+extern "C" int qe_gemm_first_columns(int M, int N, int K, int gelu) {
+    return M > 64 && N > 0 && K >= 64 ? first_columns(M, N, K, !gelu) : 0;
+}
+
 template <typename TO, int SILU>
 static int pick_mfma(const void* x, const void* w, const float* bias, void* out, int M, int N, int K,
                      int tile, int splits, hipStream_t stream, int n_first = 0, int n_cols = 0) {

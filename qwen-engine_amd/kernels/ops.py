@@ -80,6 +80,7 @@ def load_library():
         "qe_gemm_partial_preferred": [i32, i32, i32, i32, i32],
         "qe_gemm_branch_splits": [i32, i32, i32, i32, i32],
         "qe_gemm_gelu_supported": [i32, i32, i32, i32, i32],
+        "qe_gemm_first_columns": [i32, i32, i32, i32],
         "qe_attention": [vp, vp, vp, vp, vp, vp, i32, vp, i32, i32, i32, i32, i32, f32, i32, i32, i32, f32, i32, vp],
         "qe_attention_tail": [vp, vp, vp, vp, vp, vp, i32, vp, i32, i32, i32, i32, i32, f32, i32, i32, i32, f32, i32,
                               i64, i32, vp, vp, i64, i32, vp],
@@ -649,6 +650,12 @@ def gemm_gelu_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
     """True if gemm(epilogue=EPI_GELU) takes these operands."""
     lib = load_library()
     return x.dtype in _DT and w.dtype in _DT and bool(lib.qe_gemm_gelu_supported(x.shape[0], w.shape[0], x.shape[1], _DT[x.dtype], _DT[w.dtype]))
+
+
+def gemm_first_columns(rows: int, columns: int, k: int, gelu: bool = False) -> int:
+    """How many first columns of a product of ``rows`` rows by the tiled kernel go in a launch of their own (0: all in one), see
+    gemm_mfma.hip."""
+    return load_library().qe_gemm_first_columns(int(rows), int(columns), int(k), int(gelu))
 
 
 def gemm_branch_splits(x: torch.Tensor, w: torch.Tensor) -> int:

@@ -418,12 +418,15 @@ def test_qkv_product_stores_values_behind_other_rows(ops, tile, page):
     assert torch.equal(got.cpu().view(want.shape), want)
 
 
-@pytest.mark.parametrize("M,N", [(656, 24576), (1600, 10240), (700, 6144 * 3), (2048, 10240)])
+@pytest.mark.parametrize("M,N", [(656, 24576), (1601, 10368), (2048, 10240)])
 def test_products_in_two_launches(ops, M, N):
     """Products whose last turn of tiles is thin go in two launches over the columns: gate and up with silu, the product itself with a
-    bias, and q|k|v, against the same in one launch of one shape.  Whole numbers where nothing is computed on the sums."""
+    bias, and q|k|v (with the cut among the queries and among the values), against the same in one launch of one shape.  Whole
+    numbers where nothing is computed on the sums."""
     g = torch.Generator().manual_seed(N)
-    K = 512
+    K = 2048
+    first = ops.gemm_first_columns(M, N, K)
+    assert 0 < first < N and first % 256 == 0
     x = torch.randint(-2, 3, (M, K), generator=g).bfloat16().to(DEV)
     w = torch.randint(-2, 3, (N, K), generator=g).bfloat16().to(DEV)
     bias = torch.randint(-9, 9, (N,), generator=g).float().to(DEV)
@@ -434,13 +437,29 @@ def test_products_in_two_launches(ops, M, N):
     act = (torch.nn.functional.silu(gate_up[:, :, 0]) * gate_up[:, :, 1]).reshape(M, N // 2)
     got = ops.gemm(x, small, epilogue=ops.EPI_SILU_MUL_IL).double()
     assert ((got - act).abs() <= act.abs() * 2.0 ** -8 + 2.0 ** -20).all()
-    hkv = 2 if N % 256 == 0 else 1
-    hq = N // 128 - 2 * hkv
-    cache = [torch.zeros(M // 16 + 1, 2, hkv, 16, 128, dtype=torch.bfloat16, device=DEV) for _ in range(2)]
-    at = torch.arange(M, dtype=torch.int32, device=DEV)
-    q = [ops.gemm_qkv(x, w, None, hq, c, at, None, None, 1e-6, None, at, tile=t) for c, t in zip(cache, (0, 128))]
-    assert torch.equal(q[0], q[1]) and torch.equal(cache[0], cache[1])
-    assert torch.equal(q[0].view(M, -1).float(), want[:, :hq * 128].bfloat16().float())
+    heads, at = N // 128, torch.arange(M, dtype=torch.int32, device=DEV)
+    most = max(d for d in range(1, heads // 3 + 1) if heads % d == 0)
+    assert (heads - most) * 128 < first < N - 256                        # (among the values of most heads, among the queries of one)
+    for hkv in (1, most):
+        hq = heads - 2 * hkv
+        cache = [torch.zeros(M // 16 + 1, 2, hkv, 16, 128, dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+        q = [ops.gemm_qkv(x, w, None, hq, c, at, None, None, 1e-6, None, at, tile=t) for c, t in zip(cache, (0, 128))]
+        assert torch.equal(q[0], q[1]) and torch.equal(cache[0], cache[1])
+        assert torch.equal(q[0].view(M, -1).float(), want[:, :hq * 128].bfloat16().float())
+
+
+@pytest.mark.parametrize("M,N", [(1600, 5120), (1601, 5176)])
+def test_gelu_products_in_two_launches(ops, M, N):
+    """The gelu's product where its last turn of tiles is thin, against one launch of one shape and 64 bits."""
+    K = 2048
+    first = ops.gemm_first_columns(M, N, K, gelu=True)
+    assert 0 < first < N and first % 256 == 0
+    x, w = rand(M, K, seed=M).bfloat16().to(DEV), rand(N, K, seed=N, scale=K ** -0.5).bfloat16().to(DEV)
+    got = ops.gemm(x, w, epilogue=ops.EPI_GELU)
+    assert torch.equal(got, ops.gemm(x, w, epilogue=ops.EPI_GELU, algo=ops.ALGO_TILE + 128))
+    want = torch.nn.functional.gelu(x.double() @ w.double().t())
+    # (a bfloat16 rounding of the result, and sqrt(K) roundings of 2^-24 of sums of size one to three before it)
+    assert ((got.double() - want).abs() <= want.abs() * 2.0 ** -8 + 2.0 ** -22 * K ** 0.5).all()
 
 
 @pytest.mark.parametrize("hq,hkv,D,window", [(4, 2, 128, 0), (3, 1, 16, 0), (6, 2, 48, 100), (2, 2, 256, 0), (20, 1, 64, 37), (4, 4, 144, 0)])
@@ -475,9 +494,9 @@ def test_float32_attention_in_eight_walks(ops, hq, hkv, D, window):
 
 
 @pytest.mark.parametrize("taps", [2, 3, 4, 8])
-@pytest.mark.parametrize("H", [4, 260, 1028])
+@pytest.mark.parametrize("H", [4, 260, 1028, 157292])
 def test_short_convolution_by_eight_rows(ops, taps, H):
-    """Four channels of eight rows a thread: portions that begin and end anywhere in a block's rows, shorter than the taps and longer
+    """Four channels of eight rows a thread (the most channels) and a thread a number: portions that begin and end anywhere in a block's rows, shorter than the taps and longer
     than blocks, continued from step to step; what no row names stays as it was."""
     w = rand(H, taps, seed=taps)
     state = torch.full((5, taps - 1, H), 7.0, device=DEV)
