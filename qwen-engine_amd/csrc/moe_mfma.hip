@@ -13,7 +13,8 @@
 // KSPLIT (with MT == 1, few rows): the block's four waves take the same 16 features and a quarter of K each
 // (steps of 32 in turn), and wave 0 adds the four parts in the order of the waves: four times the blocks, for
 // a product that is bound by streaming the weights of the few experts that a handful of tokens choose.
-template <int MT, int MODE, bool KSPLIT = false>     // MODE 0: second product, weighted; 1: gate and up; 2: one matrix, squared relu
+// AHEAD: the steps of K whose operands are asked for together.  The order of the sums does not depend on it.
+template <int MT, int MODE, bool KSPLIT, int AHEAD>     // MODE 0: second product, weighted; 1: gate and up; 2: one matrix, squared relu
 __global__ __launch_bounds__(256) void moe_gemm_mfma_kernel(
     const bf16_t* __restrict__ x, const int* __restrict__ perm, int top, const bf16_t* __restrict__ w,
     void* __restrict__ out_, const float* __restrict__ weights, const int* __restrict__ tiles,
@@ -41,10 +42,11 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_kernel(
 #pragma unroll
     for (int i = 0; i < MT; ++i) ag[i] = au[i] = floatx4{0.f, 0.f, 0.f, 0.f};
     const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
-    // Few rows are bound by the trips to memory one after the other: the operands of eight steps are asked for together, the
-    // weights first, whose places do not wait for the rows' numbers (one token, 4 of 32 experts of 2 x 1024 x 2048: 11.5 us, 15.9
-    // with two steps at a time; their second product 6.3, and 8.4).  64 rows take their time for the arithmetic.
-    constexpr int AHEAD = MT == 1 ? 8 : 2, STEP = KSPLIT ? 128 : 32;
+    // Few rows are bound by the trips to memory one after the other: where the blocks are few the operands of eight steps are asked for
+    // together, the weights first, whose places do not wait for the rows' numbers (one token, 4 of 32 experts of 2 x 1024 x 2048: 11.5
+    // us, 15.9 with two steps at a time; their second product 6.3, and 8.4).  More blocks fetch enough between them with four
+    // steps and have the registers for it.  64 rows take their time for the arithmetic.
+    constexpr int STEP = KSPLIT ? 128 : 32;
     for (int k0 = KSPLIT ? wave * 32 : 0; k0 < K; k0 += STEP * AHEAD) {
         bf16x8 a[AHEAD], b[DUAL ? AHEAD : 1], xb[AHEAD][MT];
 #pragma unroll
@@ -53,13 +55,19 @@ __global__ __launch_bounds__(256) void moe_gemm_mfma_kernel(
             const bool kin = k + g * 8 < K;
             a[u] = kin ? *(const bf16x8*)(wg + k) : zero8;
             if (DUAL) b[u] = kin ? *(const bf16x8*)(wu + k) : zero8;
+            if (AHEAD < 8) {
+#pragma unroll
+                for (int i = 0; i < MT; ++i) xb[u][i] = kin ? *(const bf16x8*)(xr[i] + k) : zero8;
+            }
         }
+        if (AHEAD == 8) {
 #pragma unroll
-        for (int u = 0; u < AHEAD; ++u) {
-            const int k = k0 + u * STEP;
-            const bool kin = k + g * 8 < K;
+            for (int u = 0; u < AHEAD; ++u) {
+                const int k = k0 + u * STEP;
+                const bool kin = k + g * 8 < K;
 #pragma unroll
-            for (int i = 0; i < MT; ++i) xb[u][i] = kin ? *(const bf16x8*)(xr[i] + k) : zero8;
+                for (int i = 0; i < MT; ++i) xb[u][i] = kin ? *(const bf16x8*)(xr[i] + k) : zero8;
+            }
         }
 #pragma unroll
         for (int u = 0; u < AHEAD; ++u)
@@ -141,10 +149,16 @@ extern "C" int qe_moe_gemm_mfma(const void* x, const int* perm, int top, const v
     // few tiles of 16 rows (single new tokens): K is shared out over a block's waves
     const bool ksplit = tile_rows == 16 && max_tiles <= 64 && K >= 256;
     dim3 grid(qe_cdiv(N, ksplit ? 16 : 64), max_tiles);
-#define QE_MM(MT_, DUAL_, KS_) moe_gemm_mfma_kernel<MT_, DUAL_, KS_><<<grid, 256, 0, stream>>>((const bf16_t*)x, perm, top, (const bf16_t*)w, out, weights, tiles, n_tiles, T, N, K, limit, slope, interleaved)
-    if (ksplit) { if (dual == 2) QE_MM(1, 2, true); else if (dual) QE_MM(1, 1, true); else QE_MM(1, 0, true); }
-    else if (tile_rows == 16) { if (dual == 2) QE_MM(1, 2, false); else if (dual) QE_MM(1, 1, false); else QE_MM(1, 0, false); }
-    else { if (dual == 2) QE_MM(4, 2, false); else if (dual) QE_MM(4, 1, false); else QE_MM(4, 0, false); }
+#define QE_MM(MT_, DUAL_, KS_, A_) moe_gemm_mfma_kernel<MT_, DUAL_, KS_, A_><<<grid, 256, 0, stream>>>((const bf16_t*)x, perm, top, (const bf16_t*)w, out, weights, tiles, n_tiles, T, N, K, limit, slope, interleaved)
+#define QE_MMS(MT_, KS_, A_) do { if (dual == 2) QE_MM(MT_, 2, KS_, A_); else if (dual) QE_MM(MT_, 1, KS_, A_); else QE_MM(MT_, 0, KS_, A_); } while (0)
+    // (both products, the weights from memory: 16 experts of 3 x 1024 x 2048, 2 chosen, 2 tokens 16.4 us, 18.8 with two steps and
+    // 20.6 with one after the other; 8 of 3 x 2048 x 4096, 3 tokens 62.9 with four steps, 64.4 with eight, 64.1 with one after the
+    // other, 12 tokens 94.9, 94.9, 100.3.  With weights that the caches hold eight steps were up to 20 % slower than four.)
+    if (ksplit && (long)grid.x * max_tiles <= 400) QE_MMS(1, true, 8);
+    else if (ksplit) QE_MMS(1, true, 4);
+    else if (tile_rows == 16) QE_MMS(1, false, 2);
+    else QE_MMS(4, false, 2);
+#undef QE_MMS
 #undef QE_MM
     QE_LAUNCH_CHECK();
     return 0;

@@ -350,6 +350,29 @@ def test_decode_attention_of_a_token_alone_and_in_company(ops, hq, hkv, D, page,
     assert not torch.isnan(every).any()
 
 
+@pytest.mark.parametrize("E,K,F", [(16, 264, 192), (6, 2048, 544), (40, 512, 96)])
+@pytest.mark.parametrize("T", [2, 9, 48])
+def test_experts_of_few_rows_in_steps_of_k(ops, E, K, F, T):
+    """The experts' products with eight steps of K in flight (few blocks) and with four: against the 64-bit products, and a token the
+    same bits alone and in company."""
+    top = 2
+    x, wg, wd = rand(T, K, seed=1).bfloat16(), rand(E, 2 * F, K, seed=2, scale=K ** -0.5).bfloat16(), rand(E, K, F, seed=3, scale=F ** -0.5).bfloat16()
+    ids = torch.stack([torch.randperm(E, generator=torch.Generator().manual_seed(t))[:top] for t in range(T)]).int()
+    weights = torch.rand(T, top, generator=torch.Generator().manual_seed(9)) + 0.1
+    run = lambda n: ops.moe_experts(x[:n].to(DEV), ids[:n].to(DEV), weights[:n].to(DEV), wg.to(DEV), wd.to(DEV)).cpu()
+    got, alone = run(T), run(1)
+    assert got.shape == (top, T, K) and torch.equal(alone[:, 0], got[:, 0])
+    for t in range(T):
+        for j in range(top):
+            gate, up = (wg[ids[t, j]].double() @ x[t].double()).split(F)
+            mid = torch.nn.functional.silu(gate) * up
+            down = wd[ids[t, j]].double()
+            want = weights[t, j].double() * (down @ mid)
+            # (the middle rounded to bfloat16, 2^-9 of each; the 32-bit sums far below)
+            bound = weights[t, j].double() * (2.0 ** -8 * (down.abs() @ mid.abs()) + 1e-4)
+            assert ((got[j, t].double() - want).abs() <= bound).all(), (t, j)
+
+
 @pytest.mark.parametrize("T,H,N,K", [(1, 16, 128, 512), (1, 3, 20, 8), (2, 2, 64, 40), (17, 5, 130, 256), (32, 1, 16, 264), (33, 2, 128, 520), (70, 3, 40, 72)])
 def test_products_of_heads_in_steps_of_k(ops, T, H, N, K):
     """Eight steps of K asked for together (few rows) and two (many): sums of whole numbers far below 2^24, rounded once."""
