@@ -4,22 +4,25 @@
 // units' multiply-adds.  Both are chains of fused multiply-adds in the order of k, bit for bit.
 //
 // Every output is summed in one order whatever M is and whichever kernel takes the rows, so a row's
-// result does not depend on what else is in the batch.  K is cut into 16 chunks of chunk_len(K) (a
-// multiple of 16; the last ones may be short or empty).  Inside a chunk one chain runs over steps of 16,
+// result does not depend on what else is in the batch.  K is cut into at most 16 chunks of chunk_len(K) (a
+// multiple of 16, at least 64: with a chunk a step, 2000 rows of 3072 x 256 took 47 us, 40 now, 41 as one
+// chain; the last one may be short).  Inside a chunk one chain runs over steps of 16,
 // in a step over k = 0, 4, 8, 12, 1, 5, 9, 13, 2, ... (which is what lets a lane bring four neighbouring
 // k by one load and use them in four instructions).  The chunks of a quarter are added in order, then
 // the quarters in order.
 //
 // Two kernels share that order:
-//   few rows: a block owns 16 outputs (or 32) and has a wave per chunk, so that the weights are asked for
-//     by 16 waves a block at once and the sums meet in shared memory.  Bound by the stream of the weights and
+//   few rows: a block owns 16 outputs (or 32) and has a wave per chunk (16 from K = 1024 on), so that the weights are asked for
+//     by all its waves at once and the sums meet in shared memory.  Bound by the stream of the weights and
 //     a kernel's fixed cost.  Two rows (as 64 x 64 tiles before): 4096 x 1024 7.1 us (42), 6144 x 1024 10.6 (42),
 //     1024 x 3072 11.6 (117), 151936 x 1024 137 (215; 4.5 TB/s).  At most 64 registers a lane, so that two
 //     blocks of 16 waves fit a compute unit (four steps at a time instead of two: 10.0, 17.7, 14.5 and 294 us).
 //   more rows: tiles of 64 x 64, a wave a 32 x 32 quarter, K in steps of 16 through two buffers of shared
-//     memory.  With fewer than TILES_FOR_FOUR tiles four groups of four waves share a tile's K, one
-//     quarter each (a compute unit with one tile would else have a wave a SIMD and wait for every step's
-//     loads).
+//     memory.  With fewer than TILES_FOR_FOUR tiles and a K that gives each something four groups of four
+//     waves share a tile's K, one quarter each (a compute unit with one tile would else have a wave a SIMD and
+//     wait for every step's loads: 235 rows of 3072 x 1024 took 38 us, now 28; with two tiles on some units one
+//     group is the better one: 300 rows of 4096 x 512 33 us with four, 24 with one; a K of a chunk or two leaves
+//     three groups idle: 744 rows of 2048 x 77 30 us, now 9).
 // Loads stand under no condition: rows beyond the matrix read the last row again and are not stored, elements
 // beyond a row its last ones and count as zeros.  (Behind a conditional load the compiler waits for all loads in flight: with
 // such loads where K was no multiple of 16, 333 rows of 1024 x 1000 took 87.7 us.)
@@ -32,12 +35,16 @@ typedef __attribute__((ext_vector_type(16))) float floatx16;
 #define FK 16         // k step
 #define FROW (FK + 4) // floats of a staged row: padded, so that the 32 rows a wave reads lie in different banks
 #define CHUNKS 16
-#define TILES_FOR_FOUR 512
+#define TILES_FOR_FOUR 257
 
-__host__ __device__ __forceinline__ int chunk_len(int K) { return (K + CHUNKS * FK - 1) / (CHUNKS * FK) * FK; }
+__host__ __device__ __forceinline__ int chunk_len(int K) {
+    const int even = (K + CHUNKS * FK - 1) / (CHUNKS * FK) * FK;
+    return even < 4 * FK ? 4 * FK : even;
+}
 
-// How the rows of x and W lie: rows of whole steps, of whole fours (a four lies inside a row or behind its end), or any.
-enum { ROWS_ANY = 0, ROWS_FOURS = 1, ROWS_STEPS = 2 };
+// How the rows of x and W lie: rows of whole steps, of whole fours (a four lies inside a row or behind its end), any of at least four
+// numbers (the row's last four, moved up, stand for a four that passes its end), or shorter ones.
+enum { ROWS_SHORT = 0, ROWS_ANY = 1, ROWS_FOURS = 2, ROWS_STEPS = 3 };
 
 // Four consecutive elements of a row from k on, zeros behind its end (row may point behind the row's start: K is what is left of it
 // from there on, perhaps less than nothing).  No load stands under a condition: one that would lie behind the end reads the row's last
@@ -50,6 +57,18 @@ __device__ __forceinline__ floatx4 four_of_row(const float* __restrict__ row, in
     if (ROWS == ROWS_FOURS) {
         v = *(const floatx4_any*)(row + min(k, K - 4));
         if (k >= K) v = floatx4{0.f, 0.f, 0.f, 0.f};
+        return v;
+    }
+    if (ROWS == ROWS_ANY) {
+        v = *(const floatx4_any*)(row + min(k, K - 4));
+        const int past = k - (K - 4);
+        if (past > 0) {
+            const floatx4 u = v;
+            v[0] = past == 1 ? u[1] : past == 2 ? u[2] : past == 3 ? u[3] : 0.f;
+            v[1] = past == 1 ? u[2] : past == 2 ? u[3] : 0.f;
+            v[2] = past == 1 ? u[3] : 0.f;
+            v[3] = 0.f;
+        }
         return v;
     }
 #pragma unroll
@@ -168,9 +187,12 @@ __global__ __launch_bounds__(256 * GROUPS) void gemm_f32_kernel(const float* __r
     const int last = (K - 1) / FK * FK;               // K's last step
     // (steps behind the end of K are walked for the barriers' sake, their loads repeat the last step and nothing is multiplied)
     auto k_of = [&](int s) { const int k = k_begin + s * FK; return k < last ? k : last; };
-    floatx16 acc, quarter, total;
+    floatx16 acc, quarter, total;                     // (-0 is what leaves the first summand as it is)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) acc[e] = quarter[e] = total[e] = 0.f;
+    for (int e = 0; e < 16; ++e) {
+        acc[e] = 0.f;
+        quarter[e] = total[e] = -0.f;
+    }
     floatx4 xv = four_of_row<ROWS>(xsrc, k_of(0), K - sk), wv = four_of_row<ROWS>(wsrc, k_of(0), K - sk);
     *(floatx4*)&xs[sat] = xv;
     *(floatx4*)&ws[sat] = wv;
@@ -199,13 +221,17 @@ __global__ __launch_bounds__(256 * GROUPS) void gemm_f32_kernel(const float* __r
             }
             if (++in_chunk == steps_chunk || s + 1 == busy) {     // the end of a chunk, perhaps of a quarter
 #pragma unroll
-                for (int e = 0; e < 16; ++e) quarter[e] = (chunk_no & 3) ? quarter[e] + acc[e] : acc[e];
+                for (int e = 0; e < 16; ++e) {
+                    quarter[e] += acc[e];
+                    acc[e] = 0.f;
+                }
                 if ((chunk_no & 3) == 3 || s + 1 == busy) {
 #pragma unroll
-                    for (int e = 0; e < 16; ++e) total[e] = chunk_no >= 4 ? total[e] + quarter[e] : quarter[e];
+                    for (int e = 0; e < 16; ++e) {
+                        total[e] += quarter[e];
+                        quarter[e] = -0.f;
+                    }
                 }
-#pragma unroll
-                for (int e = 0; e < 16; ++e) acc[e] = 0.f;
                 in_chunk = 0;
                 ++chunk_no;
             }
@@ -248,19 +274,20 @@ static void launch_rows(const float* x, const float* w, const float* bias, float
 #define QE_F32_ROWS(R_) gemm_f32_rows_kernel<MT, NT, BATCH, R_><<<grid, 64 * waves, 0, stream>>>(x, w, bias, out, M, N, K, chunk)
     if (rows == ROWS_STEPS) QE_F32_ROWS(ROWS_STEPS);
     else if (rows == ROWS_FOURS) QE_F32_ROWS(ROWS_FOURS);
-    else QE_F32_ROWS(ROWS_ANY);
+    else if (rows == ROWS_ANY) QE_F32_ROWS(ROWS_ANY);
+    else QE_F32_ROWS(ROWS_SHORT);
 #undef QE_F32_ROWS
 }
 
 int qe_gemm_f32(const float* x, const float* w, const float* bias, float* out, int M, int N, int K,
                 hipStream_t stream) {
-    const int rows = K % FK == 0 ? ROWS_STEPS : (K % 4 == 0 ? ROWS_FOURS : ROWS_ANY);
+    const int rows = K % FK == 0 ? ROWS_STEPS : (K % 4 == 0 ? ROWS_FOURS : (K > 4 ? ROWS_ANY : ROWS_SHORT));
     // More than 16 rows against a very wide matrix (logits): every block would read all rows again, and the tiles are
-    // enough to fill the chip (33 rows, 151936 x 1024: 467 us by rows, 235 by tiles).  Up to 128 tiles leave half of the
-    // compute units idle; blocks of 64 rows and 16 outputs do not (100 rows, 1024 x 3072: 73.5 us by tiles, 33.4 by rows).  Rows that are
-    // read number by number cost a block of 64 rows more (1023 x 1001: 200 rows 33.7 us by rows, 50 by tiles, 333 65 and 51).
+    // enough to fill the chip (33 rows, 151936 x 1024: 467 us by rows, 235 by tiles).  More than 32 rows with a single chunk of K
+    // are one wave's work a block of rows (235 rows of 2048 x 64: 9.4 us by rows, 6.3 by tiles).  Up to 128 tiles leave half of the
+    // compute units idle; blocks of 64 rows and 16 outputs do not (100 rows, 1024 x 3072: 73.5 us by tiles, 33.4 by rows).
     const long tiles = (long)qe_cdiv(N, FT) * qe_cdiv(M, FT);
-    if (M <= 16 || (M <= 64 && N < 16384) || tiles <= (rows == ROWS_ANY ? 80 : 128)) {
+    if (M <= 16 || ((K > 64 || M <= 32) && ((M <= 64 && N < 16384) || tiles <= 128))) {
         // 32 outputs a block halve the reads of x; they pay where the rows are some and the blocks enough (16 rows,
         // 6144 x 1024: 12.0 us against 14.3, 151936 x 1024: 183 against 213; 2 rows: 10.3 against 10.6, 148 against 137;
         // 16 rows, 4096 x 1024: 11.5 against 9.5)
@@ -274,12 +301,13 @@ int qe_gemm_f32(const float* x, const float* w, const float* bias, float* out, i
     QE_REQUIRE(qe_cdiv(M, FT) <= 65535, "gemm (32-bit): M=%d is too large for one launch", M);
     dim3 grid(qe_cdiv(N, FT), qe_cdiv(M, FT));
     const int chunk = chunk_len(K);
-    const bool four = tiles < TILES_FOR_FOUR;
+    const bool four = tiles < TILES_FOR_FOUR && K >= 512;
 #define QE_F32_TILES(G_, R_) gemm_f32_kernel<G_, R_><<<grid, 256 * G_, 0, stream>>>(x, w, bias, out, M, N, K, chunk)
 #define QE_F32_TILES2(R_) do { if (four) QE_F32_TILES(4, R_); else QE_F32_TILES(1, R_); } while (0)
     if (rows == ROWS_STEPS) QE_F32_TILES2(ROWS_STEPS);
     else if (rows == ROWS_FOURS) QE_F32_TILES2(ROWS_FOURS);
-    else QE_F32_TILES2(ROWS_ANY);
+    else if (rows == ROWS_ANY) QE_F32_TILES2(ROWS_ANY);
+    else QE_F32_TILES2(ROWS_SHORT);
 #undef QE_F32_TILES2
 #undef QE_F32_TILES
     QE_LAUNCH_CHECK();

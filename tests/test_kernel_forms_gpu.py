@@ -37,6 +37,7 @@ def test_float32_gemm_sums_in_one_order(ops, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 24, 4), (70, 300, 77), (333, 1023, 1001), (5, 6160, 1020), (20, 40, 36), (64, 1040, 100), (333, 1024, 1000),
+                                   (40, 130, 5), (3, 20, 6), (200, 70, 7), (33, 1000, 63), (33, 1000, 65), (520, 2048, 511), (520, 1024, 515),
                                    (744, 640, 20), (2049, 1024, 44)])
 def test_float32_gemm_of_rows_that_end_inside_a_step(ops, M, N, K):
     """K a multiple of 4 and no multiple of 16, and neither: by rows and by tiles, one and four groups; what lies behind a row
