@@ -17,6 +17,11 @@
 #include "attention_tile.h"
 #include <type_traits>
 
+// A split of so many tiles is the first wave's alone: what the waves would tell each other takes longer than a second tile (one token of
+// 32 heads on 8 over 16 keys: 7.2 us with four waves at work, 6.2 so; where the host knows that there are no more, one wave is launched:
+// 6.0).
+#define ALONE 2
+
 // What the waves of a block leave for each other about a split's tiles.
 template <int TILES>
 struct WaveShared {
@@ -185,7 +190,9 @@ __global__ __launch_bounds__(64 * W) void attention_decode_split_kernel(
                                     (split * SPLIT + TILE_OF(i_) * 16) % P, g, n, stream)
 #define STEP(buf_, i_) attn_tile_step<D, CAP>(st, buf_, qreg, scale, split * SPLIT + TILE_OF(i_) * 16, g, k_begin, k_end, k_begin, k_end, kf, cap)
     const int walk1 = tile1 - gap;
-    if constexpr (W > 1) {
+    const bool alone = W > 1 && walk1 - walk0 <= ALONE;
+    if (alone && wave > 0) return;
+    if constexpr (W > 1) if (!alone) {
         constexpr int TILES = SPLIT / 16, NV = D / 16 / W;
         __shared__ WaveShared<TILES> shared;
         const int tiles = walk1 - walk0;
@@ -422,7 +429,9 @@ __global__ __launch_bounds__(64 * (W > 1 ? W + 1 : 1)) void attention_decode_fus
         stream = !(shared_keys && split * SPLIT < shared_keys[row]);
         if (lane >= tile0 && lane < tile1) my_page = bt[(split * SPLIT + lane * 16) / P];
     }
-    if constexpr (W > 1) {
+    const bool alone = W > 1 && tile1 - tile0 <= ALONE;
+    if (alone && wave > 0) return;
+    if constexpr (W > 1) if (!alone) {
         constexpr int NV = D / 16 / W;
         __shared__ WaveShared<TILES> shared;
         __shared__ float own_dot[16];
@@ -664,7 +673,7 @@ int qe_attention_decode(const void* q, void* out, const void* cache, const int* 
     dim3 mgrid(n_dec, Hq);
     // (512 splits of 8 tokens over 1000 keys: 14.0 us with one wave a split, 12.6 with four; from 576 on the two are within 3 %
     // of each other: 14.2 and 14.4, 1024 17.6 and 17.4)
-    const bool four = (long)num_splits * Hkv * n_dec <= 512;
+    const bool four = (long)num_splits * Hkv * n_dec <= 512 && max_position >= 16 * ALONE;
     if (softcap > 0.f) scale = scale * 2.f * 1.4426950408889634f / softcap;
 #define QE_DECODE_SPLIT2(D_, S_, CAP_, W_)                                                              \
         attention_decode_split_kernel<D_, S_, CAP_, W_><<<grid, 64 * W_, 0, stream>>>(                  \
@@ -719,7 +728,7 @@ int qe_attention_decode_fused(const void* qkv, void* out, void* cache, const int
     const long waves = (long)num_splits * Hkv * n_dec;
     const bool few = waves <= 1024;                            // at most a wave per SIMD: loads further ahead
     // (every wave prepares q: 256 splits of one request each take 11.4 us with four, 12.6 with one; 384 13.2 with one, 17.1 with four)
-    const bool four = waves <= 256;
+    const bool four = waves <= 256 && max_position > 16 * ALONE;
 #define QE_DECODE_FUSED_ARGS(D_)                                                                        \
             (const bf16_t*)qkv, (bf16_t*)cache, dec_tokens, positions, tok_seq, block_table, max_blocks, \
             shared_keys, slots, q_w, k_w, eps, table, part_acc, part_ml, Hq, Hkv, P, scale, window, num_splits
