@@ -147,7 +147,10 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? 3 : 1) void a
                 acc[db][i] = own_first ? fmaf(o, b, acc[db][i] * a) : fmaf(acc[db][i], a, o * b);
             }
     };
-    for (int walk = wave; walk < F32_WALKS; walk += NW) {
+    // (a walk without a tile changes nothing where it is joined: where a wave's second walk, or every walk from the fifth on, has none,
+    // there is nothing to join)
+    const bool second = wave + F32_SLOTS < n_tiles, joins = F32_SLOTS < n_tiles;
+    for (int walk = wave; walk < F32_WALKS && (walk == wave || second); walk += NW) {
         m = -INFINITY;
         l = 0.f;                                           // this lane's share of the column's sum
 #pragma unroll
@@ -224,13 +227,17 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? 3 : 1) void a
     }
     // walks w and w + 4
     if (NW == F32_SLOTS) {
-        join(false);
-        leave();
+        if (second) {
+            join(false);
+            leave();
+        }
     } else {
-        if (wave >= F32_SLOTS) leave();
-        __syncthreads();
+        if (joins) {
+            if (wave >= F32_SLOTS) leave();
+            __syncthreads();
+        }
         if (wave < F32_SLOTS) {
-            join(true);
+            if (joins) join(true);
             leave();
         }
     }
