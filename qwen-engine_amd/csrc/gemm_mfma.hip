@@ -723,8 +723,8 @@ float qe_gemm_mfma_shape(int M, int N, int K, int splits, int* tile, bool larges
     // them, the last runs alone at 0.7 of the rate; so does 64 x 128 where every unit has one.  A chip with idle
     // units runs the others faster (a third, were nearly all idle).  A shape is never taller than the rows need.
     // Against the best of all shapes (and, for a branch's last product, cuts) in products of 1024 to 25600 by 1024 to
-    // 51200 with 80 to 2048 rows, measured one by one, what this picks is 1 % slower in the mean and 9 % at the
-    // most; a rule without the cuts of K for many rows and the factors for idle and odd units was 13 % and, with 400
+    // 51200 with 80 to 2048 rows, measured one by one, what this picks is 1 % slower in the mean and 11 % at the
+    // most (shapes alone 0.1 % and 9 %); a rule without the cuts of K for many rows and the factors for idle and odd units was 13 % and, with 400
     // rows against 5120 x 25600, twice as slow (277 us in 128 x 128, 134 in three cuts of 256 x 128).
     const long cus = 256;
     struct Shape { int tile, bm, bn; float rate, alone_first, alone_later; };

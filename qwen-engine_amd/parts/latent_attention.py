@@ -1,13 +1,13 @@
 """Attention over one cached latent per token.
 
 Per token the cache holds c = norm(W_dkv x)[:R] (R = kv_rank) and one rotated key part of Dr numbers that
-all heads share; a head's key is [Uk_h c | rotated part], its value Uv_h c.  The engine never expands keys
-or values: with q'_h = Uk_h^T q_h the score of head h against token j is q'_h . c_j + q_rot_h . k_rot_j, one
-dot product against the cached row, and the head's output is Uv_h (sum_j p_j c_j).  So the attention
-kernel sees one key/value head of R + Dr numbers whose first R are also the value, read by all query heads,
-and the two maps are products per head before and after it (``ops.gemm_heads``).
+all heads share; a head's key is [Uk_h c | rotated part], its value Uv_h c.  The cache never holds expanded keys
+or values, and single tokens need none: with q'_h = Uk_h^T q_h the score of head h against token j is
+q'_h . c_j + q_rot_h . k_rot_j, one dot product against the cached row, and the head's output is
+Uv_h (sum_j p_j c_j).  So the attention kernel sees one key/value head of R + Dr numbers whose first R are also
+the value, read by all query heads, and the two maps are products per head before and after it (``ops.gemm_heads``).
 
-Portions of prompts are the exception: rows that share their keys with some dozens of others cost less with the keys
+Portions of prompts may do otherwise: rows that share their keys with some dozens of others cost less with the keys
 and values expanded once for all of them (``ops.latent_prefill``).  Which rows go that way follows from the number of
 (row, key) pairs a key has part in.
 
@@ -40,7 +40,8 @@ class LatentAttention:
     # ---- what the step function prepares for this part (parts.base) --------------------------
     # A step run as it comes knows its portions (ctx.seqs); a recorded portion is recorded for the number of keys that its
     # buffers hold, and where the keys lie the kernels read from the positions; single tokens beside a portion in a recorded
-    # step go with the folded maps, all rows alike.
+    # step go with the folded maps, all rows alike (its portion's first row and number of rows, which the lists of expanded keys
+    # name, differ from replay to replay; unrecorded, a long portion beside single tokens is expanded).
     @staticmethod
     def step_extras(seqs) -> dict:
         return {"eager": 1}
