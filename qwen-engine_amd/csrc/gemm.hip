@@ -90,12 +90,12 @@ extern "C" int qe_gemm_partial_splits(int M, int N, int K) {
 // How the product of a layer's branch (its output goes to the norm that adds it to the stream)
 // should be asked for: 0 = as a plain product; S >= 1 = as S partial products (epilogue 3), which
 // that norm adds up.  Few rows: always, the cut fills the chip.  More rows: what the product (qe_gemm_mfma_shape) and the
-// parts, stored and read by the norm at 4 TB/s (8 bytes a number, a plain product 4), take together, for each number of
+// parts' way into the norm (4 bytes a number at 6 TB/s, a plain product's 2) take together, for each number of
 // cuts that leaves 512 of K to a part; the cuts give every compute unit as many tiles as the others (800 rows against 5120 x 25600 with the norm
-// behind it: 232 us in three cuts of 256 x 256, 347 as a plain product; 528 rows against 4096 x 12288: 81 in three
-// of 128 x 128, 139 plain; 8192 rows against 5120 x 25600: 1851 in two, 2082 plain; 1300 rows against 4096 x 4096 stay plain:
-// 65, in two cuts 74).  Parts beyond 2^27 numbers (512 MiB, what a pool of pages that takes nearly all memory should leave a step) are
-// not asked for.
+// behind it: 232 us in three cuts of 256 x 256, 347 as a plain product).  Parts beyond 2^27 numbers (512 MiB, what a pool of pages that takes
+// nearly all memory should leave a step) are not asked for.  A plain product's numbers are rounded to 16 bits on their way to the norm,
+// which only many rows against a K that needs no cut pay for (those bytes are then a twentieth of the time); elsewhere a product that
+// is quickest without a cut is one 32-bit part.
 extern "C" int qe_gemm_branch_splits(int M, int N, int K, int dt_a, int dt_w) {
     if (qe_gemm_skinny_ok(M, N, K, dt_a, dt_w) || (M <= 64 && tiled_for_few_rows(M, N, K, dt_a, dt_w))) {
         const int s = qe_gemm_partial_splits(M, N, K);
@@ -104,16 +104,19 @@ extern "C" int qe_gemm_branch_splits(int M, int N, int K, int dt_a, int dt_w) {
         return (M <= qe_gemm_norm_max_rows() && s > 4) ? 4 : s;
     }
     if (!qe_gemm_mfma_ok(M, N, K, dt_a, dt_w)) return 0;
+    const long large = (long)qe_cdiv(M, 256) * qe_cdiv(N, 256), turns = (large + 255) / 256;
+    const bool plain = K < 1024 || (long)M * N > (1L << 26) ||
+                       (K <= 4096 ? (long)qe_cdiv(M, 128) * qe_cdiv(N, 128) > 256 : large > 256 && large * 10 >= turns * 256 * 9);
     int best_s = 1;
     float best = 0.f;
     for (int s = 1; s <= 6; ++s) {
         if (s > 1 && (K < 512 * s || (long)s * M * N > (1L << 27))) break;
         if ((long)(s - 1) * (qe_cdiv(qe_cdiv(K, s), 64) * 64) >= K) continue;   // every cut has some of K
         int tile;
-        const float t = qe_gemm_mfma_shape(M, N, K, s, &tile) + (s == 1 ? 4.f : 8.f * (float)s) * (float)M * (float)N / 4e6f;
+        const float t = qe_gemm_mfma_shape(M, N, K, s, &tile) + (s == 1 && plain ? 2.f : 4.f * (float)s) * (float)M * (float)N / 6e6f;
         if (s == 1 || t < best) { best_s = s; best = t; }
     }
-    return best_s > 1 ? best_s : 0;
+    return best_s > 1 || !plain ? best_s : 0;
 }
 
 // out[M, N] = x[M, K] . w[N, K]^T (+ bias).  epilogue 0: store in dt_o.  1: add into out, the

@@ -2,23 +2,23 @@
 // bfloat16 in, 32-bit accumulation with v_mfma_f32_32x32x16_bf16, output bfloat16 or float32.
 //
 // A block of NW waves (NW / 2 down, 2 across) computes a BM x BN tile of the output; each wave its
-// part as MFMA tiles of 32 x 32.  K is walked in steps of BK through shared memory with two
-// buffers.  Both operands are K-contiguous in memory, so they are staged alike: a row of BK
-// bfloat16 is padded by 16 bytes, which makes the 16-byte fragment reads of the 32 rows of an
-// MFMA operand fall into distinct banks.
+// part as MFMA tiles of 32 x 32.  K is walked in stages of 64 through shared memory.  Both operands are
+// K-contiguous in memory, so they are staged alike, by loads that write to shared memory directly.
 //
-// What the time of such a block goes to, as measured on this chip (cycle counters in a copy of
-// the kernel, hardware counters): not to the MFMA units alone.  A compute unit takes 64 bytes a
-// cycle from its L1, so a 128 x 128 x 64 step (32 KB) costs as many cycles to load as its MFMAs
-// take; loads have to be in flight two steps ahead to arrive in time; and the result has to be
-// stored as whole rows.  128 x 128 tiles (four waves, two blocks a compute unit) are the default,
-// 64 x 128 where there would be too few blocks otherwise, 256 x 128 (eight waves) where even
-// those give every compute unit two blocks, 256 x 256 (four waves, a wave's part 128 x 128) where
-// even that shape gives every compute unit two blocks in turn: it reads half the bytes per MFMA
-// from the L1 and from shared memory.
+// What the time of such a block goes to: a compute unit takes 64 bytes a cycle from its L1 and 128 from its shared
+// memory, a wave issues in order, and a load needs up to two microseconds to arrive.  So whatever is not an MFMA stands between
+// MFMAs, fragments are read a good part of a stage before they are wanted, and a stage's loads are issued one and a half to
+// two stages ahead.  (With the loads in registers first, stored to shared memory a stage later, and all fragments of a k
+// step read in a row behind each stage's barrier: 8192 x 8192 x 8192 took 829 us, now 769; 8192 rows against gate and up of 24576 x 4096
+// 1316, now 1220; 512 rows against 6144 x 1024 12.2, now 10.7; 512 against q, k and v of 4096 x 1024 11.8, now 9.9.  Stages of 32 of K,
+// half lines of 64 bytes a row, are 5 to 25 % slower than the whole lines of 64.)
+//
+// 128 x 128 by four waves (two blocks a compute unit), 64 x 128 where there would be too few blocks otherwise, 256 x 128
+// (eight waves) and 256 x 256 (four waves, a wave's part 128 x 128, which reads half the bytes per MFMA
+// from the L1 and from shared memory) where there are many: see qe_gemm_mfma_shape.
 //
 // Rows of x beyond M and rows of W beyond N are read as zero and never stored; K must be a
-// multiple of 8 (16-byte loads), a tail shorter than BK is filled with zeros.
+// multiple of 8 (16-byte loads), a tail shorter than 64 is filled with zeros.
 // The blocks of one XCD (every eighth block) take a compact part of the tiles, see the kernel.
 #include "common.h"
 
@@ -69,25 +69,28 @@ struct QkvTail {
     const int* perm;
 };
 
-// BIG (256 x 256 by four waves, one wave a SIMD, a wave's part 128 x 128): the accumulators fill the
-// 256 AGPRs, so the staging registers are VGPRs.  Per MFMA this shape reads half the bytes from
-// the L1 and from shared memory that 128 x 128 by four waves reads.
-template <typename TO, int BM, int BN, int BK, int NW, int MINB, int SILU, bool QKV = false>
+// Bytes of shared memory: the ring, or the tile of results with the rows' positions, slots and lists where that takes more.
+constexpr int gemm_mfma_shared_bytes(int BM, int BN, int RING, bool QKV) {
+    const int ring = RING * (BM + BN) * 128, tile = BM * (BN * 2 + 16) + 2 * BM * 4 + (BM + BM / 8 + 8) * 4;
+    return QKV && tile > ring ? tile : ring;
+}
+
+// DIRECT: x and w begin at a whole 16-byte piece.  Loads that write to shared memory themselves want that; operands that lie elsewhere are
+// copied by their elements, in one shape and at a fraction of the speed.
+template <typename TO, int BM, int BN, int RING, int NW, int MINB, int SILU, bool QKV = false, bool DIRECT = true>
 __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const float* __restrict__ bias,
     TO* __restrict__ out, int M, int N, int K, int tiles_m, int tiles_n, int k_per_split, int xcd_m, int xcd_n,
     int rotate, QkvTail tail) {
     constexpr bool PAIR = SILU > 0;
-    constexpr int ROWB = BK * 2 + 16;       // bytes of a staged row
-    constexpr int PPR = BK / 8;             // 16-byte pieces per row
-    constexpr int RPI = 64 * NW / PPR;      // rows the block stages with one piece per thread
     constexpr int WM = BM / (NW / 2), WN = BN / 2;   // a wave's part: NW / 2 waves down, 2 across
     constexpr int MI = WM / 32, NJ = WN / 32;
-    constexpr int LDA = BM / RPI, LD = (BM + BN) / RPI;   // pieces a thread stages per step: LDA of x, then of W
-    constexpr bool BIG = BM == 256 && BN == 256 && NW == 4;
-    static_assert((LD == 16 || LD == 12 || LD == 8 || LD == 6) && (LD == 16) == BIG && BM % RPI == 0 && BN % RPI == 0,
-                  "tile rows must be a multiple of the rows staged at once");
-    constexpr int BUF = (BM + BN) * ROWB;   // bytes of one buffer: the x rows, then the W rows
+    constexpr int LDA = BM / (8 * NW), LD = (BM + BN) / (8 * NW);   // a wave's loads of a stage: LDA of x, then of W
+    static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0 && LD >= 2 && (RING - 2) * LD + (LD + 1) / 2 < 64 && RING >= 2,
+                  "the rows of a stage must be whole loads of every wave, the loads in flight no more than can be counted");
+    constexpr bool BIG = BM == 256 && BN == 256 && NW == 4, TWO = BM == 128 && BN == 128 && RING == 2;
+    constexpr int STAGE = (BM + BN) * 128;   // bytes of a stage: the x rows, then the W rows
+    [[maybe_unused]] constexpr int SMEM = gemm_mfma_shared_bytes(BM, BN, RING, QKV);
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     // Consecutive blocks go to the eight XCDs in turn, and each XCD has an L2 of its own: the blocks
@@ -154,7 +157,7 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
     // number blockIdx.y (out is then [splits][M][N]); without a cut k_per_split = K
     const int k0 = blockIdx.y * k_per_split;
     const int klen = K - k0 < k_per_split ? K - k0 : k_per_split;
-    const int nk = (klen + BK - 1) / BK;
+    const int nk = (klen + 63) / 64;
     // rotate: the block walks its k steps from another start than its neighbours (and wraps round).  Few rows
     // of x against a large matrix: the blocks stream their rows of W in step, and with a row stride that is a
     // power of two all their loads of a moment have the same address bits below the stride, which land on the
@@ -164,22 +167,22 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
     // the batch.
     const int rot = rotate ? (tile_n * 5 + (int)blockIdx.y * 3) % nk : 0;
 #define QE_KK(kt_) ((kt_) < nk ? ((kt_) + rot < nk ? (kt_) + rot : (kt_) + rot - nk) : (kt_))
-    // Two sets of staging registers in turn: a step's loads are issued two steps ahead and go to
-    // shared memory one step ahead, so a load has a whole step of MFMAs to arrive.
-    uint4_t stage[2][LD];
-
-    // Piece i of a thread is row (tid / PPR) of the i-th group of RPI rows, 16 bytes at k = 8 (tid % PPR).
+    // A stage is 64 values of K of all the tile's rows, 128 bytes a row (a line of the caches) without padding.  The loads
+    // go to shared memory directly (no registers, no stores of the waves' own): one instruction
+    // brings 8 rows, 16 bytes a lane, side by side.  The eight pieces of a row are exchanged by the row's number
+    // (piece p of row r lies at place p ^ (r / 2 % 8)), so that the fragment reads of 16 rows fall into distinct banks;
+    // the exchange is made by the addresses that the lanes ask for.
+    //
     // The loads are buffer loads: one descriptor for the tile's rows of x and one for its rows of W,
     // each ending with the last row that exists, so that a row beyond the matrix is "out of range"
-    // and reads as zeros by itself.  The thread's byte offset never changes and the step's k offset
-    // is a scalar.  A thread whose piece lies beyond K (in a last step shorter than BK) picks an
+    // and arrives as zeros by itself.  The thread's byte offset never changes and the stage's k offset
+    // is a scalar.  A thread whose piece lies beyond K (in a last stage shorter than 64) picks an
     // offset that is out of range.
     //
-    // The loads and the waits for them are written as instructions: the compiler's own placing of
-    // waits joins what it knows at the loop's top and so waits for the youngest loads as well,
-    // which would undo the two steps of distance.  A set's registers pass through the wait
-    // statement as operands, so nothing that uses them can move ahead of it.
-    const int lrow = tid / PPR, pc = tid % PPR;
+    // The loads and the waits for them are written as instructions: the compiler would wait for every load in flight
+    // before it reads shared memory.
+    const int wave_s = __builtin_amdgcn_readfirstlane(wave);
+    const int pc = (lane & 7) ^ ((wave & 1) * 4 + (lane >> 4));            // the lane's piece of its row (of the 8 of an instruction)
     const int a_rows = M - m0 < BM ? M - m0 : BM, b_rows = N - n0 < BN ? N - n0 : BN;
     const unsigned long a_addr = (unsigned long)(x + (long)m0 * K + k0), b_addr = (unsigned long)(w + (long)n0 * K + k0);
     uint4_t rsrc_a, rsrc_b;   // base, base high 16 bits (stride 0), bytes, format: 32-bit raw buffer
@@ -192,63 +195,14 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
         rsrc_a[c] = __builtin_amdgcn_readfirstlane(rsrc_a[c]);
         rsrc_b[c] = __builtin_amdgcn_readfirstlane(rsrc_b[c]);
     }
-    int voff[LD];
-#pragma unroll
-    for (int i = 0; i < LD; ++i)
-        voff[i] = ((i < LDA ? RPI * i : RPI * (i - LDA)) + lrow) * K * 2 + pc * 16;
-    const int dst = lrow * ROWB + pc * 16;                 // where piece 0 goes in a buffer; piece i: + i RPI ROWB
-#define LOAD_GLOBAL(set_, kt_)                                                           \
-    {                                                                                    \
-        const int kk = QE_KK(kt_);                                                       \
-        const bool k_ok = kk * BK + pc * 8 < klen;                                       \
-        const int soff = kk * BK * 2;                                                    \
-        _Pragma("unroll") for (int i = 0; i < LD; ++i) {                                 \
-            const int vo = k_ok ? voff[i] : 0x7fffffff;                                  \
-            if constexpr (BIG) {                                                         \
-                if (i < LDA)                                                             \
-                    asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen"              \
-                                 : "=&v"(stage[set_][i]) : "v"(vo), "s"(rsrc_a), "s"(soff) : "memory"); \
-                else                                                                     \
-                    asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen"              \
-                                 : "=&v"(stage[set_][i]) : "v"(vo), "s"(rsrc_b), "s"(soff) : "memory"); \
-            } else if (i < LDA)                                                          \
-                asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen"                  \
-                             : "=&a"(stage[set_][i]) : "v"(vo), "s"(rsrc_a), "s"(soff) : "memory"); \
-            else                                                                         \
-                asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen"                  \
-                             : "=&a"(stage[set_][i]) : "v"(vo), "s"(rsrc_b), "s"(soff) : "memory"); \
-        }                                                                                \
-    }
-    // waits until at most `younger_` loads are in flight; the set's registers are valid afterwards
-#define WAIT_LOADS(set_, younger_)                                                       \
-    if constexpr (LD == 16)                                                              \
-        asm volatile("s_waitcnt vmcnt(%16)"                                              \
-                     : "+v"(stage[set_][0]), "+v"(stage[set_][1]), "+v"(stage[set_][2]), "+v"(stage[set_][3]), \
-                       "+v"(stage[set_][4]), "+v"(stage[set_][5]), "+v"(stage[set_][6 % LD]), "+v"(stage[set_][7 % LD]), \
-                       "+v"(stage[set_][8 % LD]), "+v"(stage[set_][9 % LD]), "+v"(stage[set_][10 % LD]),       \
-                       "+v"(stage[set_][11 % LD]), "+v"(stage[set_][12 % LD]), "+v"(stage[set_][13 % LD]),     \
-                       "+v"(stage[set_][14 % LD]), "+v"(stage[set_][15 % LD])                                  \
-                     : "n"(younger_) : "memory");                                        \
-    else if constexpr (LD == 12)                                                         \
-        asm volatile("s_waitcnt vmcnt(%12)"                                              \
-                     : "+a"(stage[set_][0]), "+a"(stage[set_][1]), "+a"(stage[set_][2]), "+a"(stage[set_][3]), \
-                       "+a"(stage[set_][4]), "+a"(stage[set_][5]), "+a"(stage[set_][6]), "+a"(stage[set_][7]), \
-                       "+a"(stage[set_][8 % LD]), "+a"(stage[set_][9 % LD]), "+a"(stage[set_][10 % LD]),       \
-                       "+a"(stage[set_][11 % LD])                                        \
-                     : "n"(younger_) : "memory");                                        \
-    else if constexpr (LD == 8)                                                          \
-        asm volatile("s_waitcnt vmcnt(%8)"                                               \
-                     : "+a"(stage[set_][0]), "+a"(stage[set_][1]), "+a"(stage[set_][2]), "+a"(stage[set_][3]), \
-                       "+a"(stage[set_][4]), "+a"(stage[set_][5]), "+a"(stage[set_][6 % LD]), "+a"(stage[set_][7 % LD]) \
-                     : "n"(younger_) : "memory");                                        \
-    else                                                                                 \
-        asm volatile("s_waitcnt vmcnt(%6)"                                               \
-                     : "+a"(stage[set_][0]), "+a"(stage[set_][1]), "+a"(stage[set_][2]), "+a"(stage[set_][3]), \
-                       "+a"(stage[set_][4]), "+a"(stage[set_][5])                        \
-                     : "n"(younger_) : "memory");
-#define STORE_SHARED(buf_)                                                               \
-    _Pragma("unroll") for (int i = 0; i < LD; ++i)                                       \
-        *(uint4_t*)(smem + (buf_) * BUF + dst + i * RPI * ROWB) = stage[buf_][i];
+    const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) unsigned char*)smem + wave_s * 1024;
+#define LOAD_LDS(to_, vo_, rsrc_, soff_)                                                 \
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" \
+                 : : "s"(to_), "v"(vo_), "s"(rsrc_), "s"(soff_) : "memory");
+    // waits until at most younger_ loads of the wave are in flight and its reads of shared memory are done, then for
+    // the other waves
+#define MEET(younger_)                                                                   \
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(younger_) : "memory");
 
     floatx16 acc[MI][NJ];
 #pragma unroll
@@ -258,107 +212,237 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
-    const int fr = lane & 31;          // row of the fragment this lane holds
-    const int fk = (lane >> 5) * 16;   // byte offset of its 8 k values within a 16-wide k step
-    const unsigned char* a_frag = smem + (wm + fr) * ROWB + fk;
-    const unsigned char* b_frag = smem + (BM + wn + fr) * ROWB + fk;
-    // One step on buffer buf_ (a constant, so every shared-memory address is base + immediate).
-    // A wave issues in order, so whatever is not an MFMA stands between the MFMAs: the fragments of
-    // k step ks + 1 are read before the MFMAs of ks; the loads of the step after the next go with
-    // the MFMAs of the first k steps, the stores to shared memory of the next step's tile, loaded
-    // a step ago, with those of the last.  Tiles of 128 rows or more spread the loads over all k
-    // steps but the last and the stores over all but the first (the compute unit's L1 takes 64
-    // bytes a cycle: the 64 KB a step of a 256 x 256 tile are half of the step's time, and as
-    // much for the LDS; issued in a row they hold up the MFMAs behind them, which cost that
-    // shape a third of the step).  The 64-row tile, whose steps are short, keeps the loads in
-    // the first k step and the stores in the last: a load then has the longest time to arrive
-    // (spread, its loads from HBM came late: 27 us against 24 for the o and down products of the
-    // small model, though it was the faster on operands that lie in the L2).
-    // (Passing the barrier before the last MFMAs and reading the next step's first fragments
-    // under them was tried: 3 % faster with one wave a SIMD, 10 % slower with two.)
-#define READ_FRAGS(buf_, ks_, a_, b_)                                                    \
-    _Pragma("unroll") for (int i = 0; i < MI; ++i)                                       \
-        a_[i] = *(const bf16x8*)(a_frag + (buf_) * BUF + i * 32 * ROWB + (ks_) * 32);    \
-    _Pragma("unroll") for (int j = 0; j < NJ; ++j)                                       \
-        b_[j] = *(const bf16x8*)(b_frag + (buf_) * BUF + j * 32 * ROWB + (ks_) * 32);
-#define LOAD_PIECE(set_, kt_, i_)                                                        \
-    {                                                                                    \
-        const int kk = QE_KK(kt_);                                                       \
-        const int vo = kk * BK + pc * 8 < klen ? voff[i_] : 0x7fffffff;                  \
-        const int soff = kk * BK * 2;                                                    \
-        if constexpr (BIG) {                                                             \
-            if ((i_) < LDA)                                                              \
-                asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen"                  \
-                             : "=&v"(stage[set_][i_]) : "v"(vo), "s"(rsrc_a), "s"(soff) : "memory"); \
-            else                                                                         \
-                asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen"                  \
-                             : "=&v"(stage[set_][i_]) : "v"(vo), "s"(rsrc_b), "s"(soff) : "memory"); \
-        } else if ((i_) < LDA)                                                           \
-            asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen"                      \
-                         : "=&a"(stage[set_][i_]) : "v"(vo), "s"(rsrc_a), "s"(soff) : "memory"); \
-        else                                                                             \
-            asm volatile("buffer_load_dwordx4 %0, %1, %2, %3 offen"                      \
-                         : "=&a"(stage[set_][i_]) : "v"(vo), "s"(rsrc_b), "s"(soff) : "memory"); \
-    }
-    constexpr int NS = BK / 16, PER = MI * NJ;            // k steps; MFMAs of one
-    constexpr bool SPREAD = BM >= 128;
-    constexpr int LE = SPREAD ? NS - 1 : 1, SB = SPREAD ? 1 : NS - 1;   // loads go with the k steps [0, LE), stores with [SB, NS)
-    constexpr int LSLOTS = LE * PER, SSLOTS = (NS - SB) * PER;    // places (MFMAs) for a load, for a store
-    constexpr int EARLY = SB * PER * LD / LSLOTS < LD ? SB * PER * LD / LSLOTS : LD;   // this step's loads issued before k step SB
-    static_assert(NS >= 2, "a step has two k steps or more");
-    // the pieces that go with place s of n: [s LD / n, (s + 1) LD / n)
-#define K_STEP(buf_, kt_)                                                                \
-    {                                                                                    \
-        bf16x8 fa[2][MI], fb[2][NJ];                                                     \
-        READ_FRAGS(buf_, 0, fa[0], fb[0])                                                \
-        _Pragma("unroll") for (int ks = 0; ks < NS; ++ks) {                              \
-            if (ks + 1 < NS) { READ_FRAGS(buf_, ks + 1, fa[(ks + 1) & 1], fb[(ks + 1) & 1]) } \
-            /* the other set, loaded a step ago; this step's own loads, issued so far, may stay in flight */ \
-            if (ks == SB) { WAIT_LOADS((buf_) ^ 1, EARLY) }                              \
+    // A lane's fragment: row lane % 32, of its 16-wide k step ks the 8 values from 8 (lane / 32) on; that of k step 0, the
+    // others: ^ 32 ks
+    const int fr = lane & 31;
+    const int f0 = fr * 128 + (((lane >> 5) ^ ((fr >> 1) & 7)) * 16);
+    if constexpr (BIG) {
+        // 256 x 256 by four waves, one wave a SIMD, its accumulators in the 256 AGPRs.  The halves of a wave's rows of x and of W
+        // are four regions of a stage, each read once into registers and kept there: a stage is four quarters (a half of x with a
+        // half of W, 16 MFMAs), in an order in which one quarter's last operands are no operands of the next, so that
+        // each quarter reads the region that is first wanted in the next one or the one after it.  Behind the barrier at its end that
+        // region's memory takes the same rows two stages later: seven quarters, over two microseconds, for a load to
+        // arrive, and 24 loads of a wave always in flight.  The order alternates: even stages x0 w0, x0 w1, x1 w1, x1 w0,
+        // odd ones x0 w1, x0 w0, x1 w0, x1 w1.
+        int voff[2][4];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                voff[h][i] = ((i / 2) * 128 + h * 64 + (i % 2) * 32 + wave * 8 + (lane >> 3)) * K * 2 + pc * 16;
+        bf16x8 fa[2][2][4], fb[2][2][4];
+        const unsigned char* const fa0 = smem + (wave >> 1) * 8192;
+        const unsigned char* const fb0 = smem + (wave & 1) * 8192;
+        // region rg_: 0, 1: the halves of x; 2, 3: of W; its place for a stage of parity st_
+#define REGION_AT(rg_, st_) ((((st_) & 1) * 4 + (rg_)) * 16384)
+#define LOAD_REGION(rg_, st_, par_, i_)                                                  \
+        {                                                                                \
+            const int kk = QE_KK(st_);                                                   \
+            const int vo = kk * 64 + pc * 8 < klen ? voff[(rg_) & 1][i_] : 0x7fffffff;   \
+            const int soff = kk * 128;                                                   \
+            const unsigned to = lds0 + REGION_AT(rg_, par_) + (i_) * 4096;               \
+            if ((rg_) < 2) LOAD_LDS(to, vo, rsrc_a, soff) else LOAD_LDS(to, vo, rsrc_b, soff) \
+        }
+#define READ_REGION(rg_, par_, p_)                                                       \
+        {                                                                                \
+            if ((rg_) < 2) fa[(rg_) & 1][(p_) & 1][(p_) >> 1] = *(const bf16x8*)(fa0 + REGION_AT(rg_, par_) + ((p_) & 1) * 4096 + (f0 ^ (((p_) >> 1) * 32))); \
+            else fb[(rg_) & 1][(p_) & 1][(p_) >> 1] = *(const bf16x8*)(fb0 + REGION_AT(rg_, par_) + ((p_) & 1) * 4096 + (f0 ^ (((p_) >> 1) * 32))); \
+        }
+        // half ha_ of x with half hb_ of W; meanwhile region rrg_ of a stage of parity rpar_ is read and region lrg_ of stage lst_ (parity
+        // lpar_) asked for
+#define QUAD(ha_, hb_, rrg_, rpar_, lrg_, lst_, lpar_)                                   \
+        _Pragma("unroll") for (int sl = 0; sl < 16; ++sl) {                              \
+            if (sl < 8) READ_REGION(rrg_, rpar_, sl)                                     \
+            acc[(ha_) * 2 + (sl / 2) % 2][(hb_) * 2 + sl % 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16( \
+                fb[hb_][sl % 2][sl / 4], fa[ha_][(sl / 2) % 2][sl / 4], acc[(ha_) * 2 + (sl / 2) % 2][(hb_) * 2 + sl % 2], 0, 0, 0); \
+            if (sl % 4 == 1) LOAD_REGION(lrg_, lst_, lpar_, sl / 4)                      \
             __builtin_amdgcn_sched_barrier(0);                                           \
-            _Pragma("unroll") for (int i = 0; i < MI; ++i)                               \
-                _Pragma("unroll") for (int j = 0; j < NJ; ++j) {                         \
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[ks & 1][j], fa[ks & 1][i], acc[i][j], 0, 0, 0); \
-                    _Pragma("unroll") for (int p = 0; p < LD; ++p) {                     \
-                        const int sl = ks * PER + i * NJ + j, ss = sl - SB * PER;   /* place of a load, of a store */ \
-                        if (ks < LE && p >= sl * LD / LSLOTS && p < (sl + 1) * LD / LSLOTS) \
-                            LOAD_PIECE(buf_, (kt_) + 2, p)   /* this set went to shared memory a step ago */ \
-                        /* the other buffer: its readers finished before the last barrier (after the  \
-                           last step this stores a step that does not exist, which nobody reads) */ \
-                        if (ks >= SB && p >= ss * LD / SSLOTS && p < (ss + 1) * LD / SSLOTS) \
-                            *(uint4_t*)(smem + ((buf_) ^ 1) * BUF + dst + p * RPI * ROWB) = stage[(buf_) ^ 1][p]; \
-                    }                                                                    \
-                    __builtin_amdgcn_sched_barrier(0);                                   \
-                }                                                                        \
         }                                                                                \
-        __syncthreads();                                                                 \
+        MEET(24)
+#define EVEN(st_)                                                                        \
+        QUAD(0, 0, 3, 0, 2, (st_) + 2, 0)                                                \
+        QUAD(0, 1, 1, 0, 3, (st_) + 2, 0)                                                \
+        QUAD(1, 1, 0, 1, 1, (st_) + 2, 0)                                                \
+        QUAD(1, 0, 3, 1, 0, (st_) + 3, 1)
+#define ODD(st_)                                                                         \
+        QUAD(0, 1, 2, 1, 3, (st_) + 2, 1)                                                \
+        QUAD(0, 0, 1, 1, 2, (st_) + 2, 1)                                                \
+        QUAD(1, 0, 0, 0, 1, (st_) + 2, 1)                                                \
+        QUAD(1, 1, 2, 0, 0, (st_) + 3, 0)
+        constexpr int first[8] = {0, 2, 3, 1, 0 + 4, 3 + 4, 2 + 4, 1 + 4};      // in the order in which they are read (4: of the second stage)
+#pragma unroll
+        for (int r = 0; r < 8; ++r)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) LOAD_REGION(first[r] & 3, first[r] >> 2, first[r] >> 2, i)
+        MEET(24)
+#pragma unroll
+        for (int p = 0; p < 8; ++p) READ_REGION(0, 0, p)
+#pragma unroll
+        for (int p = 0; p < 8; ++p) READ_REGION(2, 0, p)
+        MEET(24)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) LOAD_REGION(0, 2, 0, i)
+        MEET(24)
+        int st = 0;
+        for (; st + 1 < nk; st += 2) {
+            EVEN(st)
+            ODD(st + 1)
+        }
+        if (st < nk) { EVEN(st) }
+#undef EVEN
+#undef ODD
+#undef QUAD
+#undef READ_REGION
+#undef LOAD_REGION
+#undef REGION_AT
+    } else if constexpr (TWO) {
+        // 128 x 128 by four waves in the same way, with room for two blocks a compute unit (64 KB each): half stages (a half of x with
+        // all of W, 8 MFMAs), the next stage's W in registers of its own, and three half stages for a load to arrive.  (As a
+        // ring of whole stages as below, which leaves one stage: 512 rows against 4096 x 4096 54 us, now 37; 2048 against
+        // 6144 x 2048 57, now 51.)
+        int voff[2][2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) voff[h][i] = (i * 64 + h * 32 + wave * 8 + (lane >> 3)) * K * 2 + pc * 16;
+        bf16x8 fa[2][4], fb[2][2][4];
+        const unsigned char* const fa0 = smem + (wave >> 1) * 4096;
+        const unsigned char* const fb0 = smem + (wave & 1) * 4096;
+#define REGION_AT(rg_, st_) ((((st_) & 1) * 4 + (rg_)) * 8192)
+#define LOAD_REGION(rg_, st_, par_, i_)                                                  \
+        {                                                                                \
+            const int kk = QE_KK(st_);                                                   \
+            const int vo = kk * 64 + pc * 8 < klen ? voff[(rg_) & 1][i_] : 0x7fffffff;   \
+            const int soff = kk * 128;                                                   \
+            const unsigned to = lds0 + REGION_AT(rg_, par_) + (i_) * 4096;               \
+            if ((rg_) < 2) LOAD_LDS(to, vo, rsrc_a, soff) else LOAD_LDS(to, vo, rsrc_b, soff) \
+        }
+#define READ_A(h_, par_, ks_) fa[h_][ks_] = *(const bf16x8*)(fa0 + REGION_AT(h_, par_) + (f0 ^ ((ks_) * 32)));
+#define READ_B(h_, par_, ks_) fb[par_][h_][ks_] = *(const bf16x8*)(fb0 + REGION_AT(2 + (h_), par_) + (f0 ^ ((ks_) * 32)));
+#define HALF_STAGE(ha_, par_, st_)                                                       \
+        _Pragma("unroll") for (int sl = 0; sl < 8; ++sl) {                               \
+            if (sl % 2 == 0) { READ_A((ha_) ^ 1, (ha_) ? (par_) ^ 1 : (par_), sl / 2) }  \
+            else { READ_B(ha_, (par_) ^ 1, sl / 2) }                                     \
+            acc[ha_][sl % 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[par_][sl % 2][sl / 2], fa[ha_][sl / 2], acc[ha_][sl % 2], 0, 0, 0); \
+            if (sl == 1) LOAD_REGION(ha_, (st_) + 2, par_, 0)                            \
+            if (sl == 3) LOAD_REGION(ha_, (st_) + 2, par_, 1)                            \
+            if (sl == 5) LOAD_REGION(3 - (ha_), (st_) + 2 + (ha_), (par_) ^ (ha_), 0)    \
+            if (sl == 7) LOAD_REGION(3 - (ha_), (st_) + 2 + (ha_), (par_) ^ (ha_), 1)    \
+            __builtin_amdgcn_sched_barrier(0);                                           \
+        }                                                                                \
+        MEET(8)
+        constexpr int first[8] = {0, 2, 3, 1, 2 + 4, 0 + 4, 3 + 4, 1 + 4};
+#pragma unroll
+        for (int r = 0; r < 8; ++r)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) LOAD_REGION(first[r] & 3, first[r] >> 2, first[r] >> 2, i)
+        MEET(10)
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            READ_A(0, 0, ks)
+            READ_B(0, 0, ks)
+            READ_B(1, 0, ks)
+        }
+        MEET(10)
+        LOAD_REGION(2, 2, 0, 0)
+        LOAD_REGION(2, 2, 0, 1)
+        MEET(8)
+        int st = 0;
+        for (; st + 1 < nk; st += 2) {
+            HALF_STAGE(0, 0, st)
+            HALF_STAGE(1, 0, st)
+            HALF_STAGE(0, 1, st + 1)
+            HALF_STAGE(1, 1, st + 1)
+        }
+        if (st < nk) {
+            HALF_STAGE(0, 0, st)
+            HALF_STAGE(1, 0, st)
+        }
+#undef HALF_STAGE
+#undef READ_A
+#undef READ_B
+#undef LOAD_REGION
+#undef REGION_AT
+    } else {
+    // The other shapes: a ring of RING stages, three where two blocks of 64 x 128 share a unit and for 256 x 128.
+    int voff[LD];                                          // of the wave's instructions of a stage: LDA for x, then for W
+#pragma unroll
+    for (int i = 0; i < LD; ++i)
+        voff[i] = (((i < LDA ? i : i - LDA) * NW + wave) * 8 + (lane >> 3)) * K * 2 + pc * 16;
+    // the wave's i_-th load of stage st_, into the ring's place that begins at byte at_
+#define LOAD_PIECE(st_, at_, i_)                                                         \
+    {                                                                                    \
+        const int kk = QE_KK(st_);                                                       \
+        const int vo = kk * 64 + pc * 8 < klen ? voff[i_] : 0x7fffffff;                  \
+        const int soff = kk * 128;                                                       \
+        const unsigned place = (at_) + ((i_) < LDA ? (i_) * NW * 1024 : BM * 128 + ((i_) - LDA) * NW * 1024); \
+        if constexpr (!DIRECT) {                                                         \
+            const int row = (((i_) < LDA ? (i_) : (i_) - LDA) * NW + wave) * 8 + (lane >> 3); \
+            const bf16_t* const from = ((i_) < LDA ? x + (long)m0 * K : w + (long)n0 * K) + (long)row * K + k0 + kk * 64 + pc * 8; \
+            const bool there = row < ((i_) < LDA ? a_rows : b_rows) && kk * 64 + pc * 8 < klen; \
+            Piece16 piece;                                                               \
+            _Pragma("unroll") for (int e = 0; e < 8; ++e) piece.e[e] = there ? from[e].bits : (unsigned short)0; \
+            *(uint4_t*)(smem + place + wave * 1024 + lane * 16) = piece.q;               \
+        } else if ((i_) < LDA) LOAD_LDS(lds0 + place, vo, rsrc_a, soff) else LOAD_LDS(lds0 + place, vo, rsrc_b, soff) \
     }
-
-    // step kt uses buffer and register set kt % 2
-    LOAD_GLOBAL(0, 0)
-    LOAD_GLOBAL(1, 1)
-    WAIT_LOADS(0, LD)
-    STORE_SHARED(0)
-    __syncthreads();
-    // (two steps in a body without branches, and an odd last step after the loop)
-    int kt = 0;
-    for (; kt + 1 < nk; kt += 2) {
-        K_STEP(0, kt)
-        K_STEP(1, kt + 1)
+    const unsigned char *a_frag[4], *b_frag[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+        a_frag[ks] = smem + wm * 128 + (f0 ^ (32 * ks));
+        b_frag[ks] = smem + (BM + wn) * 128 + (f0 ^ (32 * ks));
     }
-    if (kt < nk) K_STEP(0, kt)
-    // The loads past the end are still in flight and the compiler does not know of them: their
-    // registers pass through a last wait, so that they stay reserved until the loads have landed
-    // (a register whose value nobody uses would be handed out again at once).
-    WAIT_LOADS(0, 0)
-    WAIT_LOADS(1, 0)
+    bf16x8 fa[2][MI], fb[2][NJ];
+    constexpr int R = MI + NJ;                             // fragments of a k step: of W and of x in turn
+#define READ_FRAG(ks_, at_, p_)                                                          \
+    {                                                                                    \
+        const bool of_a = (p_) < 2 * MI && (p_) < 2 * NJ ? (p_) % 2 : MI > NJ;           \
+        const int i_ = (p_) < 2 * MI && (p_) < 2 * NJ ? (p_) / 2 : (p_) - (MI > NJ ? NJ : MI); \
+        if (of_a) fa[(ks_) & 1][i_ < MI ? i_ : 0] = *(const bf16x8*)(a_frag[ks_] + (at_) + i_ * 4096); \
+        else fb[(ks_) & 1][i_ < NJ ? i_ : 0] = *(const bf16x8*)(b_frag[ks_] + (at_) + i_ * 4096); \
+    }
+    // The MFMAs of k step ks_ of a stage, and between them (a wave issues in order) what is wanted next: the fragments of
+    // the k step behind it, from place rd_, and the wave's loads [l0_, l1_) of stage st_ to place ld_.
+    constexpr int PER = MI * NJ, RSLOTS = PER >= 2 * R ? R : (PER + 1) / 2;
+#define K_STEP(ks_, rd_, st_, ld_, l0_, l1_)                                             \
+    _Pragma("unroll") for (int sl = 0; sl < PER; ++sl) {                                 \
+        _Pragma("unroll") for (int p = 0; p < R; ++p)                                    \
+            if (p * RSLOTS / R == sl) READ_FRAG(((ks_) + 1) & 3, rd_, p)                 \
+        acc[sl / NJ][sl % NJ] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[(ks_) & 1][sl % NJ], fa[(ks_) & 1][sl / NJ], acc[sl / NJ][sl % NJ], 0, 0, 0); \
+        _Pragma("unroll") for (int p = (l0_); p < (l1_); ++p)                            \
+            if ((p - (l0_)) * PER / ((l1_) > (l0_) ? (l1_) - (l0_) : 1) == sl) LOAD_PIECE(st_, ld_, p)       \
+        __builtin_amdgcn_sched_barrier(0);                                               \
+    }
+    // A place of the ring is read for the last time in the third k step of its stage (by then the last k step's fragments are
+    // in registers); behind the barrier there it takes the stage RING later: half of that stage's loads go with
+    // the last k step, half with the first of the next stage.
+    constexpr int HALF = (LD + 1) / 2;
+#pragma unroll
+    for (int st = 0; st < RING; ++st)
+#pragma unroll
+        for (int i = 0; i < LD; ++i)
+            if (st + 1 < RING || i < HALF) LOAD_PIECE(st, st * STAGE, i)
+    MEET((RING - 2) * LD + HALF)
+#pragma unroll
+    for (int p = 0; p < R; ++p) READ_FRAG(0, 0, p)
+    int at = 0, before = (RING - 1) * STAGE;               // this stage's place, and that of the stage before
+    for (int st = 0; st < nk; ++st) {
+        const int next = at + STAGE == RING * STAGE ? 0 : at + STAGE;
+        K_STEP(0, at, st + RING - 1, before, HALF, LD)
+        K_STEP(1, at, 0, 0, 0, 0)
+        K_STEP(2, at, 0, 0, 0, 0)
+        MEET((RING - 2) * LD)
+        K_STEP(3, next, st + RING, at, 0, HALF)
+        before = at;
+        at = next;
+    }
 #undef K_STEP
-#undef QE_KK
 #undef LOAD_PIECE
-#undef READ_FRAGS
-#undef LOAD_GLOBAL
-#undef WAIT_LOADS
-#undef STORE_SHARED
+#undef READ_FRAG
+    }
+    MEET(0)                                                // (what was asked for beyond the end arrives too, before the memory is used again)
+#undef QE_KK
+#undef LOAD_LDS
+#undef MEET
 
     // The MFMA is given the W rows as its first operand and the x rows as its second, so its
     // result is the tile transposed: a lane holds, for the token row m = lane % 32, the outputs
@@ -372,11 +456,11 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
         // 16 lanes take a row of a head each, as in qk_rope_store_vec_kernel: lane j has the features
         // 4 j .. 4 j + 3 and 64 + 4 j .. 64 + 4 j + 3, the two halves that rotate together.
         constexpr int TROW = BN * 2 + 16;                  // bytes of a row of the tile
-        static_assert(BM * TROW <= 2 * BUF && BN % 128 == 0, "the tile must fit the staging buffers, in whole heads");
+        static_assert(BM * TROW <= SMEM && BN % 128 == 0, "the tile must fit the staging buffers, in whole heads");
         // positions and slots of the tile's rows, once, into shared memory behind the tile
         int* pos_sh = (int*)(smem + BM * TROW);
         int* slot_sh = pos_sh + BM;
-        static_assert(BM * TROW + 2 * BM * 4 <= 2 * BUF, "the rows' positions and slots must fit too");
+        static_assert(BM * TROW + 2 * BM * 4 <= SMEM, "the rows' positions and slots must fit too");
         if (tid < BM) { pos_sh[tid] = my_pos; slot_sh[tid] = my_slot; }
         __syncthreads();
         const int D = 128, half = 64;
@@ -478,7 +562,7 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
         int* pieces = slot_sh + BM;
         int* singles = pieces + BM / 8;
         int* counts = singles + BM;                       // of the pieces, then of the single rows, found by each wave
-        static_assert(BM * TROW + 2 * BM * 4 + (BM + BM / 8 + 8) * 4 <= 2 * BUF && BM <= 256, "the lists must fit too");
+        static_assert(BM * TROW + 2 * BM * 4 + (BM + BM / 8 + 8) * 4 <= SMEM && BM <= 256, "the lists must fit too");
         const bool has_values = tail.slots && n0 / 128 + BN / 128 > tail.Hq + tail.Hkv;   // the same for the whole block
         int n_pieces = 0, n_singles = 0;
         if (has_values) {
@@ -549,7 +633,7 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
     constexpr int CH = 16 / ESZ;                           // outputs in 16 bytes
     constexpr int CPR = WNO / CH;                          // 16-byte chunks in a row of the strip
     constexpr int SROW = WNO * ESZ + 16;                   // bytes of a staged row
-    static_assert(NW * 32 * SROW <= 2 * BUF, "the strips of the waves must fit the staging buffers");
+    static_assert(NW * 32 * SROW <= SMEM, "the strips of the waves must fit the staging buffers");
     unsigned char* strip = smem + wave * 32 * SROW;
     const int no0 = PAIR ? (n0 + wn) / 2 : n0 + wn;        // first output column of the wave's strip
     const bool vec_ok = (NO % CH) == 0 && (((unsigned long)out) & 15) == 0;
@@ -626,21 +710,25 @@ bool qe_gemm_mfma_ok(int M, int N, int K, int dt_a, int dt_w) {
 }
 
 // The columns tail.n_first .. tail.n_first + n_cols - 1 of the product (rounded up to whole tiles).
-template <typename TO, int BM, int BN, int BK, int NW, int MINB, int SILU, bool QKV = false>
+template <typename TO, int BM, int BN, int RING, int NW, int MINB, int SILU, bool QKV = false, bool DIRECT = true>
 static int launch_mfma(const void* x, const void* w, const float* bias, void* out, int M, int N, int K,
                        int n_cols, int splits, hipStream_t stream, const QkvTail& tail) {
+    if constexpr (DIRECT) {
+        if (((unsigned long)x | (unsigned long)w) & 15)
+            return launch_mfma<TO, 128, 128, 3, 4, 1, SILU, QKV, false>(x, w, bias, out, M, N, K, n_cols, splits, stream, tail);
+    }
     const int tiles_m = qe_cdiv(M, BM), tiles_n = qe_cdiv(n_cols, BN);
     const long blocks = (long)tiles_m * tiles_n;
     QE_REQUIRE(blocks <= 2147483647L, "mfma gemm: too many tiles");
-    const size_t shmem = 2 * (BM + BN) * (BK * 2 + 16);
+    const size_t shmem = gemm_mfma_shared_bytes(BM, BN, RING, QKV);
     static bool attr_set = false;   // one flag per instantiation
     if (!attr_set) {
-        (void)hipFuncSetAttribute((const void*)gemm_mfma_kernel<TO, BM, BN, BK, NW, MINB, SILU, QKV>,
+        (void)hipFuncSetAttribute((const void*)gemm_mfma_kernel<TO, BM, BN, RING, NW, MINB, SILU, QKV, DIRECT>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
         attr_set = true;
     }
-    // a cut of K is a multiple of BK long (the last may be shorter)
-    const int k_per_split = splits > 1 ? qe_cdiv(qe_cdiv(K, splits), BK) * BK : K;
+    // a cut of K is a multiple of 64 long (the last may be shorter)
+    const int k_per_split = splits > 1 ? qe_cdiv(qe_cdiv(K, splits), 64) * 64 : K;
     QE_REQUIRE(splits >= 1 && splits <= 65535 && (long)(splits - 1) * k_per_split < K,
                "mfma gemm: K=%d cannot be cut into %d parts", K, splits);
     // the eight XCDs as a by b parts of the tiles (a b = 8): every XCD reads M / a rows of x and
@@ -653,7 +741,7 @@ static int launch_mfma(const void* x, const void* w, const float* bias, void* ou
         const long rows = (long)b * M + (long)a * n_cols;
         if (xcd_m == 0 || rows < fewest) { xcd_m = a; xcd_n = b; fewest = rows; }
     }
-    gemm_mfma_kernel<TO, BM, BN, BK, NW, MINB, SILU, QKV><<<dim3((unsigned)blocks, (unsigned)splits), 64 * NW, shmem, stream>>>(
+    gemm_mfma_kernel<TO, BM, BN, RING, NW, MINB, SILU, QKV, DIRECT><<<dim3((unsigned)blocks, (unsigned)splits), 64 * NW, shmem, stream>>>(
         (const bf16_t*)x, (const bf16_t*)w, bias, (TO*)out, M, N, K, tiles_m, tiles_n, k_per_split, xcd_m, xcd_n,
         (!QKV && M <= 64 && (K * 2) % 8192 == 0) ? 1 : 0, tail);
     QE_LAUNCH_CHECK();
@@ -661,18 +749,22 @@ static int launch_mfma(const void* x, const void* w, const float* bias, void* ou
 }
 
 // Rows grouped by expert against one matrix per expert (see QkvTail): tiles of 128 x 128.
-template <typename TO, int SILU>
+template <typename TO, int SILU, bool DIRECT = true>
 static int launch_grouped(const void* x, const void* w, void* out, const int* tiles, const int* n_tiles,
                           int max_tiles, int N, int K, float limit, float slope, hipStream_t stream, int relu_sq = 0,
                           const float* row_w = nullptr, const int* perm = nullptr) {
-    constexpr int BM = 128, BN = 128, BK = 64, NW = 4;
+    constexpr int BM = 128, BN = 128, RING = DIRECT ? 2 : 3, NW = 4, MINB = DIRECT ? 2 : 1;
+    if constexpr (DIRECT) {
+        if (((unsigned long)x | (unsigned long)w) & 15)
+            return launch_grouped<TO, SILU, false>(x, w, out, tiles, n_tiles, max_tiles, N, K, limit, slope, stream, relu_sq, row_w, perm);
+    }
     const int tiles_n = qe_cdiv(N, BN);
     const long blocks = (long)max_tiles * tiles_n;
     QE_REQUIRE(blocks > 0 && blocks <= 2147483647L, "mfma gemm (grouped): too many tiles");
-    const size_t shmem = 2 * (BM + BN) * (BK * 2 + 16);
+    const size_t shmem = gemm_mfma_shared_bytes(BM, BN, RING, false);
     static bool attr_set = false;
     if (!attr_set) {
-        (void)hipFuncSetAttribute((const void*)gemm_mfma_kernel<TO, BM, BN, BK, NW, 2, SILU, false>,
+        (void)hipFuncSetAttribute((const void*)gemm_mfma_kernel<TO, BM, BN, RING, NW, MINB, SILU, false, DIRECT>,
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
         attr_set = true;
     }
@@ -684,7 +776,7 @@ static int launch_grouped(const void* x, const void* w, void* out, const int* ti
     tail.relu_sq = relu_sq;
     tail.row_w = row_w;
     tail.perm = perm;
-    gemm_mfma_kernel<TO, BM, BN, BK, NW, 2, SILU, false><<<dim3((unsigned)blocks, 1), 64 * NW, shmem, stream>>>(
+    gemm_mfma_kernel<TO, BM, BN, RING, NW, MINB, SILU, false, DIRECT><<<dim3((unsigned)blocks, 1), 64 * NW, shmem, stream>>>(
         (const bf16_t*)x, (const bf16_t*)w, nullptr, (TO*)out, 0, N, K, max_tiles, tiles_n, K, 0, 0, 0, tail);
     QE_LAUNCH_CHECK();
     return 0;
@@ -717,19 +809,18 @@ extern "C" int qe_gemm_mfma_grouped_tile_rows() { return 128; }
 // partial products left out).
 float qe_gemm_mfma_shape(int M, int N, int K, int splits, int* tile, bool largest = true) {
     // The busiest compute unit decides: its number of tiles (they are dealt out in turn) times what a tile costs, its
-    // operations at the rate that the shape reaches on large products (256 x 256: 1.30 PFLOP/s over the chip, 256 x 128
-    // 1.16, 128 x 128 1.07, 64 x 128 0.65) and a microsecond for the trip through an empty pipeline.
-    // 128 x 128 reaches its rate with two blocks on a compute unit: where the busiest unit gets an odd number of
-    // them, the last runs alone at 0.7 of the rate; so does 64 x 128 where every unit has one.  A chip with idle
-    // units runs the others faster (a third, were nearly all idle).  A shape is never taller than the rows need.
-    // Against the best of all shapes (and, for a branch's last product, cuts) in products of 1024 to 25600 by 1024 to
-    // 51200 with 80 to 2048 rows, measured one by one, what this picks is 1 % slower in the mean and 11 % at the
-    // most (shapes alone 0.1 % and 9 %); a rule without the cuts of K for many rows and the factors for idle and odd units was 13 % and, with 400
-    // rows against 5120 x 25600, twice as slow (277 us in 128 x 128, 134 in three cuts of 256 x 128).
+    // operations at the rate that the shape reaches in long products (256 x 256: 1.27 PFLOP/s over the chip, 256 x 128
+    // 1.18, 128 x 128 1.07, 64 x 128 0.78) and 2.6 microseconds for the first trip to memory and the result's way out.
+    // 128 x 128 and 64 x 128 reach their rates with two blocks on a compute unit: where the busiest unit gets an odd number of
+    // them, the last runs alone and takes longer.  A chip with idle
+    // units runs the others faster (two and a half times, were nearly all idle).  A shape is never taller than the rows need.
+    // Against the best of all shapes (and, for a branch's last product, cuts) in products of 1024 to 51200 by 1024 to
+    // 25600 with 80 to 3300 rows, 2900 measured one by one on rows that are in no L2 and weights that are in no cache, what this picks is
+    // 0.3 % slower in the mean (of a branch's product with what its norm reads 0.6 %), 12 % at the most (3300 rows against 6144 x 1024).
     const long cus = 256;
     struct Shape { int tile, bm, bn; float rate, alone_first, alone_later; };
-    const Shape shapes[4] = {{64, 64, 128, 0.65f, 0.43f, 0.f}, {128, 128, 128, 1.07f, 0.43f, 0.43f},
-                             {256, 256, 128, 1.16f, 0.f, 0.f}, {512, 256, 256, 1.30f, 0.f, 0.f}};
+    const Shape shapes[4] = {{64, 64, 128, 0.78f, 0.f, 0.15f}, {128, 128, 128, 1.07f, 0.05f, 0.41f},
+                             {256, 256, 128, 1.18f, 0.f, 0.f}, {512, 256, 256, 1.27f, 0.f, 0.f}};
     const long cut = (long)qe_cdiv(qe_cdiv(K, splits), 64) * 64;
     float best = 0.f;
     *tile = 0;
@@ -741,7 +832,7 @@ float qe_gemm_mfma_shape(int M, int N, int K, int splits, int* tile, bool larges
         const float alone = turns == 1 ? sh.alone_first : (turns % 2 ? sh.alone_later : 0.f);
         const float busy = (float)blocks / (float)(turns * cus);
         const float one = (float)(cut * sh.bm * sh.bn) * (2e-9f * (float)cus) / sh.rate;
-        const float cost = ((float)turns + alone) * (one * (0.65f + 0.35f * busy) + 1.f);
+        const float cost = ((float)turns + alone) * (one * (0.4f + 0.6f * busy) + 2.6f);
         if (*tile == 0 || cost < best) { *tile = sh.tile; best = cost; }
     }
     return best;
@@ -801,11 +892,11 @@ static int pick_mfma(const void* x, const void* w, const float* bias, void* out,
     // (the gelu of 65536 values is 35 us in which nothing else runs on the unit: 256 x 256 is never its shape; 3000 rows against
     // 4096 x 1024: 65 us in it, 52 in 256 x 128, 47 in 128 x 128)
     if (tile == 0) tile = choose_tile(M, N, K, splits, SILU >= 0);
-    if (tile == 65) return launch_mfma<TO, 64, 128, 128, 4, 1, SILU>(x, w, bias, out, M, N, K, n_cols, splits, stream, tail);
-    if (tile == 512) return launch_mfma<TO, 256, 256, 64, 4, 1, SILU>(x, w, bias, out, M, N, K, n_cols, splits, stream, tail);
-    if (tile == 256) return launch_mfma<TO, 256, 128, 64, 8, 1, SILU>(x, w, bias, out, M, N, K, n_cols, splits, stream, tail);
-    if (tile == 128) return launch_mfma<TO, 128, 128, 64, 4, 2, SILU>(x, w, bias, out, M, N, K, n_cols, splits, stream, tail);
-    return launch_mfma<TO, 64, 128, 64, 4, 2, SILU>(x, w, bias, out, M, N, K, n_cols, splits, stream, tail);
+    if (tile == 65) return launch_mfma<TO, 64, 128, 6, 4, 1, SILU>(x, w, bias, out, M, N, K, n_cols, splits, stream, tail);
+    if (tile == 512) return launch_mfma<TO, 256, 256, 2, 4, 1, SILU>(x, w, bias, out, M, N, K, n_cols, splits, stream, tail);
+    if (tile == 256) return launch_mfma<TO, 256, 128, 3, 8, 1, SILU>(x, w, bias, out, M, N, K, n_cols, splits, stream, tail);
+    if (tile == 128) return launch_mfma<TO, 128, 128, 2, 4, 2, SILU>(x, w, bias, out, M, N, K, n_cols, splits, stream, tail);
+    return launch_mfma<TO, 64, 128, 3, 4, 2, SILU>(x, w, bias, out, M, N, K, n_cols, splits, stream, tail);
 }
 
 // tile: rows of the output tile (256, 128 or 64; 512 stands for 256 x 256, 65 for 64 x 128 with a k step of 128), 0 to choose
@@ -855,10 +946,10 @@ int qe_gemm_qkv(const void* x, const void* w, const float* bias, int M, int K, i
         tail.n_first = part ? n1 : 0;
         const int n_cols = n1 == 0 ? N : (part ? N - n1 : n1), t = tile ? tile : choose_tile(M, n_cols, K, 1);
         int rc;
-        if (t == 512) rc = launch_mfma<bf16_t, 256, 256, 64, 4, 1, 0, true>(x, w, bias, nullptr, M, N, K, n_cols, 1, stream, tail);
-        else if (t == 256) rc = launch_mfma<bf16_t, 256, 128, 64, 8, 1, 0, true>(x, w, bias, nullptr, M, N, K, n_cols, 1, stream, tail);
-        else if (t == 128) rc = launch_mfma<bf16_t, 128, 128, 64, 4, 2, 0, true>(x, w, bias, nullptr, M, N, K, n_cols, 1, stream, tail);
-        else rc = launch_mfma<bf16_t, 64, 128, 64, 4, 2, 0, true>(x, w, bias, nullptr, M, N, K, n_cols, 1, stream, tail);
+        if (t == 512) rc = launch_mfma<bf16_t, 256, 256, 2, 4, 1, 0, true>(x, w, bias, nullptr, M, N, K, n_cols, 1, stream, tail);
+        else if (t == 256) rc = launch_mfma<bf16_t, 256, 128, 3, 8, 1, 0, true>(x, w, bias, nullptr, M, N, K, n_cols, 1, stream, tail);
+        else if (t == 128) rc = launch_mfma<bf16_t, 128, 128, 2, 4, 2, 0, true>(x, w, bias, nullptr, M, N, K, n_cols, 1, stream, tail);
+        else rc = launch_mfma<bf16_t, 64, 128, 3, 4, 2, 0, true>(x, w, bias, nullptr, M, N, K, n_cols, 1, stream, tail);
         if (rc) return rc;
     }
     return 0;

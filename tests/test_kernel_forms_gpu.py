@@ -634,3 +634,46 @@ def test_parts_of_a_product_stay_within_their_bytes(ops):
         for rows in (1, 64, 512, 2048, 8192, 12288, 16384, 32768, 65536):
             splits = ops.gemm_branch_splits_for(rows, w, torch.bfloat16)
             assert splits * rows * n * 4 <= 512 << 20, (rows, n, k, splits)
+
+
+@pytest.mark.parametrize("K", [64, 72, 128, 200, 320, 1096])
+def test_tiled_products_at_the_ends_of_their_stages(ops, K):
+    """One stage of 64 of K and several, odd and even numbers, whole and not, in every tile shape, rows and columns just beyond and
+    short of a tile, and two cuts of K; NaN and infinities beside the operands change nothing."""
+    for M, N in ((65, 136), (129, 120), (257, 264), (255, 256)):
+        xs, ws = (torch.full((r + 2, K), float("nan"), dtype=torch.bfloat16) for r in (M, N))
+        xs[0], ws[0] = float("inf"), float("-inf")
+        xs[1:-1], ws[1:-1] = rand(M, K, seed=M + K, dtype=torch.bfloat16), rand(N, K, seed=N + K, dtype=torch.bfloat16)
+        x, w = xs.to(DEV)[1:-1], ws.to(DEV)[1:-1]
+        want = xs[1:-1].double() @ ws[1:-1].double().t()
+        # (K products summed in 32-bit: some sqrt(K) units of 2^-24 of the sum of their sizes; 2^-20 bounds it)
+        bound = 2.0 ** -20 * (xs[1:-1].double().abs() @ ws[1:-1].double().abs().t())
+        for rows in (64, 65, 128, 256, 512):
+            got = ops.gemm(x, w, out_dtype=torch.float32, algo=ops.ALGO_TILE + rows)
+            assert ((got.cpu().double() - want).abs() <= bound).all(), (M, N, K, rows)
+        if K > 64:
+            parts = ops.gemm(x, w, epilogue=ops.EPI_PARTIAL, splits=2) if M > 64 else None
+            assert parts is None or ((parts.cpu().double().sum(0) - want).abs() <= bound).all(), (M, N, K)
+
+
+def test_tiled_products_of_operands_at_any_address(ops):
+    """Operands that begin at an odd element: the bits of aligned ones, in a plain product, gate and up, and grouped rows."""
+    odd = lambda t: torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(t.shape)
+    M, N, K = 200, 192, 328
+    x, w = rand(M, K, seed=1, dtype=torch.bfloat16).to(DEV), rand(N, K, seed=2, dtype=torch.bfloat16).to(DEV)
+    ox, ow = odd(x), odd(w)
+    assert ox.data_ptr() % 4 == 2 and ow.data_ptr() % 4 == 2
+    for a, b in ((ox, w), (x, ow), (ox, ow)):
+        assert torch.equal(ops.gemm(a, b), ops.gemm(x, w))
+        assert torch.equal(ops.gemm(a, b, epilogue=ops.EPI_SILU_MUL_IL), ops.gemm(x, w, epilogue=ops.EPI_SILU_MUL_IL))
+
+
+@pytest.mark.parametrize("K", [1016, 1024, 2048, 4096, 4160, 12288])
+def test_products_whose_parts_are_rounded_are_large(ops, K):
+    """A branch's product is handed on in 16 bits only where its rows are many (or K is short); else in 32-bit parts."""
+    for N in (1024, 2048, 4096, 5120):
+        w = torch.empty(N, K, dtype=torch.bfloat16, device=DEV)
+        for M in (65, 300, 512, 1000, 2048, 8192):
+            splits = ops.gemm_branch_splits_for(M, w, torch.bfloat16)
+            tiles = -(-M // 128) * -(-N // 128)
+            assert (splits == 0) == (K < 1024) or (splits == 0 and tiles > 256), (M, N, K, splits)
