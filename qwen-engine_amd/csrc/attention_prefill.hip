@@ -5,21 +5,24 @@
 // heads that share one key/value head (GH = the group size when that is a power of two up to 32,
 // else 1), so one pass over the keys serves the whole group.  A block is four waves with four
 // neighbouring row tiles of one request.  It walks the keys its rows see, 32 at a time, from the
-// cache pages (keys written by this same step included): the 256 threads bring the next key
-// tile and value tile into shared memory with contiguous 16-byte loads while the waves compute
-// on the current one (two buffers, one barrier per tile); every wave then reads its MFMA
-// operands from shared memory, whose rows are padded so that those reads do not collide.
+// cache pages (keys written by this same step included): a block's loads write key and value tiles to shared memory
+// directly, a ring of four tiles ahead, one barrier per tile; every wave reads its MFMA
+// operands from shared memory, whose pieces are exchanged so that those reads do not collide.
 //   S^T[key, col] = K[key, :] . Q[col, :]         v_mfma_f32_32x32x16_bf16, D / 16 of them;
-//       lane (g, r), g = lane / 32, r = lane % 32, takes K[key r][ks * 16 + g * 8 .. + 8]
-//       and ends up with 16 scores: keys 8 b + 4 g + j (b, j < 4) of column r
+//       lane (g, r), g = lane / 32, r = lane % 32, takes K[key r'][ks * 16 + g * 8 .. + 8], r' being r with its bits 2
+//       and 3 exchanged, and ends up with 16 scores: keys 16 h + 8 g + j (h < 2, j < 8) of column r
 //   online softmax per column in 32-bit, in the base-2 domain (scores are scaled by
 //       scale * log2 e once); the accumulator is rescaled only when a score exceeds the column's
 //       reference by more than 8
 //   O^T[d, col] += V^T[d, key] . P^T[key, col]    v_mfma_f32_32x32x16_bf16, 2 * D / 32 of them;
 //       the 8 probabilities of a half tile that a lane holds are its B operand as they lie, and
 //       because value tiles are stored transposed ([D][P]) the A operand is the same 8 keys of
-//       one row of V^T: the staged rows hold the keys in the order 0-3, 8-11, 4-7, 12-15, so that
-//       it is one 16-byte read
+//       one row of V^T, one 16-byte read
+// What bounds it: the vector units' 560 cycles and the matrix units' 512 of a wave's tile, which overlap only between the two waves of
+// a SIMD.  (With tiles through registers, a barrier behind every tile's arrival and the scores of a tile right before its weights:
+// 8192 tokens of 32 heads of 128 on 8, 626 us, now 573; 512 rows each behind 4096 keys, four requests, 197, now 166; 2048 tokens of
+// 16 heads 48.5, now 46; 512 rows behind 7680 keys 61, now 58.  The two groups of a block half a round apart, a barrier for each phase,
+// took 48 and 60.5 there.)
 // The causal and window limits are applied per column, so the order of the sums for a row
 // depends on its position and the window only.
 //
@@ -68,7 +71,10 @@ __device__ __forceinline__ float sum_of_both_halves(float v) {
 
 #define QE_PREFILL_UNCUT_KEYS 1024
 #define QE_PREFILL_MIN_SEGMENT 512
-#define VROW 48   // bytes of a staged value row: 16 keys = 32 bytes of data + 16 of padding
+
+// Tiles of keys and values in a group's shared memory: 64 KB for heads of 128, for two groups a compute unit (eight tiles of heads of 64
+// are no quicker).
+#define RING 4
 
 // The keys of a segment when ``keys`` keys are cut into ks segments: a multiple of 64, at least
 // QE_PREFILL_MIN_SEGMENT; 0 (no cut) up to QE_PREFILL_UNCUT_KEYS keys.  One formula for the host's plan
@@ -144,17 +150,15 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
     const int* __restrict__ block_table, int max_blocks,
     int Hq, int Hkv, int P, int log2P, float scale_log2, int window, int R, int seg_param, int keys_row,
     float* __restrict__ part, int keep_first, int sink, float cap_in, float cap_out, AttnTail tail) {
-    constexpr int KROW = D * 2 + 16;                 // bytes of a staged key row
-    constexpr int KBYTES = 32 * KROW, VBYTES = 2 * D * VROW, BUF = KBYTES + VBYTES;
-    constexpr int KP = 32 * (D / 8) / 256;           // 16-byte key pieces per thread (2 for D = 128)
-    constexpr int VP = 2 * D * 2 / 256;              // 16-byte value pieces per thread
-    __shared__ __attribute__((aligned(16))) unsigned char smem_all[NG * 2 * BUF];
+    constexpr int KROW = D * 2, KBYTES = 32 * KROW, BUF = 2 * KBYTES;    // bytes of a key row, of a tile's keys, of a tile
+    constexpr int LP = D / 64;                       // loads of a wave for a tile's keys, and for its values
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];      // NG rings of RING tiles
 
     // (group and wave are the same for all lanes of a wave: kept in scalar registers, so that what
     // follows from them — tile keys, pages, addresses — is scalar arithmetic)
     const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x / 256);   // which half of the key tiles (NG = 2)
     const int tid = threadIdx.x % 256, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    unsigned char* smem = smem_all + grp * 2 * BUF;
+    unsigned char* smem = smem_all + grp * RING * BUF;
     const int g = lane >> 5, r = lane & 31;
     const int G = Hq / Hkv;
     const int GH = 32 / R;                                 // heads per wave
@@ -210,15 +214,6 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
     const int all_hi = p_first + 1;
     const int all_lo = first_seen_key(p_last, window);
 
-    bf16x8 qreg[D / 16];
-#pragma unroll
-    for (int ks = 0; ks < D / 16; ++ks)
-        qreg[ks] = *(const bf16x8*)(q + ((long)row * Hq + head) * D + ks * 16 + g * 8);
-    // Wait for q here, with an instruction the compiler sees: else it waits for these loads where q
-    // is first used, inside the loop, where its count of loads in flight includes the loop's own,
-    // and every round would end up waiting for the loads it has just issued.
-    __builtin_amdgcn_s_waitcnt(0x0f70);                    // vmcnt(0)
-
     float m = -INFINITY, l = 0.f;
     floatx16 acc[D / 32];
 #pragma unroll
@@ -226,138 +221,140 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[db][e] = 0.f;
 
-    // ---- staging: global -> registers -> shared ------------------------------------------------
-    // A 32-key tile has two halves of 16 keys with pages and offsets of their own.  A half that no
+    // ---- staging: global -> shared -------------------------------------------------------------
+    // A 32-key tile has two halves of 16 keys with pages and offsets of their own; half of the waves bring one, half the
+    // other.  A half that no
     // row of the block sees (beyond the request's keys, or wholly behind the window, where the page
-    // may have been given back) reads the other half's memory again; what lies outside
-    // [kmin, kmax) is zeroed in the value tile (it may be unwritten memory, and anything times a
-    // weight of 0 must still be 0) and masked in the scores.
-    // Two sets of staging registers in turn: the loads of a tile are issued two tiles ahead and
-    // stored to shared memory one tile ahead, so a load has a whole tile's computation to arrive
-    // (one tile of arithmetic is shorter than a trip to memory).
-    // The loads are buffer loads: the page's address and the offset of the 16 keys in it are
-    // scalar, and a thread adds bytes that are constant over the loop.  Which half of the tile a
-    // piece belongs to is the same for a whole wave (256 pieces are 2 D / 8 rows of 8 pieces).
-    Piece kst[2][KP], vst[2][VP];
-    int kconst[KP], vconst[VP];                           // bytes from the page's start, without the keys' offset
-    bool khalf[KP], vhalf[VP];
+    // may have been given back) is asked for with a descriptor of no bytes and arrives as zeros; what else lies outside
+    // [kmin, kmax) is masked in the scores and zeroed in the value fragments (it may be unwritten memory, and anything times a
+    // weight of 0 must still be 0).
+    // The loads are buffer loads that write to shared memory directly, 64 pieces of 16 bytes side by side an instruction: the
+    // page's address and the offset of the 16 keys in it are scalar, and a lane adds bytes that are constant over the
+    // loop.  A ring of RING tiles, each tile's loads issued RING - 1 rounds or more ahead; the next tile's page
+    // id is asked for a round before it is used.  Pieces are exchanged so that the fragment reads fall into distinct
+    // banks: piece p of key row r lies at place p ^ (r % 16) (D = 64: p ^ (r / 2 % 8)), of value row d at p ^ (d / 8 % 2).
+    // (So is a tile that does not exist: the number of loads in flight is always known.)  The loads and the waits for them are written as instructions: the compiler would wait for every
+    // load in flight before it reads shared memory.
+    int kconst[LP], vconst[LP];                            // bytes from the page's start, without the keys' offset
+    const int half = wave >> 1;                            // of the tile, that this wave brings
 #pragma unroll
-    for (int i = 0; i < KP; ++i) {
-        const int id = tid + 256 * i;
-        const int krow = id / (D / 8), col = id % (D / 8);
-        khalf[i] = __builtin_amdgcn_readfirstlane(krow >= 16);
-        kconst[i] = ((kvh * P + (krow & 15)) * D + col * 8) * 2;
-    }
-#pragma unroll
-    for (int i = 0; i < VP; ++i) {
-        const int id = tid + 256 * i;
-        const int rem = id % (2 * D);
-        vhalf[i] = __builtin_amdgcn_readfirstlane(id >= 2 * D);
-        vconst[i] = (((Hkv + kvh) * P) * D + (rem >> 1) * P + (rem & 1) * 8) * 2;
+    for (int i = 0; i < LP; ++i) {
+        const int krow = (wave & 1) * 8 + (D == 128 ? i * 4 + (lane >> 4) : lane >> 3);
+        const int piece = D == 128 ? (lane & 15) ^ krow : (lane & 7) ^ (((half * 16 + krow) >> 1) & 7);
+        kconst[i] = ((kvh * P + krow) * D) * 2 + piece * 16;
+        const int d = (wave & 1) * (D / 2) + i * 32 + (lane >> 1);
+        vconst[i] = (((Hkv + kvh) * P) * D + d * P) * 2 + ((lane & 1) ^ ((d >> 3) & 1)) * 16;
     }
     const int pmask = P - 1;
     const int page_bytes = (int)page_stride * 2;
-#define STAGE_LOAD(set_, kk_)                                                                       \
+    const unsigned lds_k = (unsigned)(unsigned long)(__attribute__((address_space(3))) unsigned char*)smem + wave * (LP * 1024);
+    const unsigned lds_v = lds_k + KBYTES;                 // (as many bytes of a tile's values before a wave's as of its keys)
+    // (a tile's place, and the page of this wave's half of it; no more than the last key's page is ever asked for)
+#define PAGE_OF(kk_) bt[min((kk_) + 16 * half, kmax - 1) >> log2P]
+#define LOAD_TILE(kk_, page_, at_)                                                                  \
     {                                                                                               \
-        const bool first_ = (kk_) + 16 > kmin || (kk_) < kfb;                                       \
-        const bool second_ = ((kk_) + 16 < kmax && (kk_) + 32 > kmin) || (kk_) + 16 < kfb;          \
-        const int ka_ = first_ ? (kk_) : (kk_) + 16;                                                \
-        const int kb_ = second_ ? (kk_) + 16 : (kk_);                                               \
-        const __amdgpu_buffer_rsrc_t ra_ = __builtin_amdgcn_make_buffer_rsrc(                       \
-            (void*)(cache + (long)bt[ka_ >> log2P] * page_stride), 0, page_bytes, 0x00020000);      \
-        const __amdgpu_buffer_rsrc_t rb_ = __builtin_amdgcn_make_buffer_rsrc(                       \
-            (void*)(cache + (long)bt[kb_ >> log2P] * page_stride), 0, page_bytes, 0x00020000);      \
-        const int oa_ = (ka_ & pmask) * 2, ob_ = (kb_ & pmask) * 2;   /* bytes in a row of V^T */   \
-        _Pragma("unroll") for (int i = 0; i < KP; ++i)                                              \
-            kst[set_][i].q = __builtin_amdgcn_raw_buffer_load_b128(khalf[i] ? rb_ : ra_, kconst[i], \
-                                                                   (khalf[i] ? ob_ : oa_) * D, 0);  \
-        _Pragma("unroll") for (int i = 0; i < VP; ++i)                                              \
-            vst[set_][i].q = __builtin_amdgcn_raw_buffer_load_b128(vhalf[i] ? rb_ : ra_, vconst[i], \
-                                                                   vhalf[i] ? ob_ : oa_, 0);        \
+        const unsigned long base_ = (unsigned long)(cache + (long)(page_) * page_stride);           \
+        const int key_ = (kk_) + 16 * half, off_ = key_ & pmask;                                    \
+        const bool there_ = key_ < kmax && (key_ + 16 > kmin || key_ < kfb);                        \
+        const uint4_t rsrc_ = {(unsigned)base_, (unsigned)(base_ >> 32) & 0xffffu, there_ ? (unsigned)page_bytes : 0u, 0x00020000u}; \
+        _Pragma("unroll") for (int i_ = 0; i_ < LP; ++i_) {                                         \
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"  \
+                         : : "s"(lds_k + (at_) + i_ * 1024), "v"(kconst[i_]), "s"(rsrc_), "s"(off_ * (D * 2)) : "memory"); \
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"  \
+                         : : "s"(lds_v + (at_) + i_ * 1024), "v"(vconst[i_]), "s"(rsrc_), "s"(off_ * 2) : "memory"); \
+        }                                                                                           \
     }
-#define STAGE_STORE(buf_, set_, kk_)                                                                \
+    // waits until at most younger_ loads of the wave are in flight and its reads of shared memory are done, then for the other
+    // waves; nothing is moved across
+#define MEET(younger_)                                                                              \
     {                                                                                               \
-        if ((kk_) + 32 > kmax || (kk_) < kmin) {                                                    \
-            _Pragma("unroll") for (int i = 0; i < VP; ++i) {                                        \
-                const int id = tid + 256 * i;                                                       \
-                const int half = id / (2 * D), part = id & 1;                                       \
-                _Pragma("unroll") for (int e = 0; e < 8; ++e) {                                     \
-                    const int key = (kk_) + 16 * half + 8 * part + e;                               \
-                    if ((key < kmin && key >= kfb) || key >= kmax) vst[set_][i].e[e] = 0;           \
-                }                                                                                   \
-            }                                                                                       \
-        }                                                                                           \
-        unsigned char* ks_ = smem + (buf_) * BUF;                                                   \
-        unsigned char* vs_ = ks_ + KBYTES;                                                          \
-        _Pragma("unroll") for (int i = 0; i < KP; ++i) {                                            \
-            const int id = tid + 256 * i;                                                           \
-            *(uint4_t*)(ks_ + (id / (D / 8)) * KROW + (id % (D / 8)) * 16) = kst[set_][i].q;        \
-        }                                                                                           \
-        _Pragma("unroll") for (int i = 0; i < VP; ++i) {                                            \
-            const int id = tid + 256 * i;                                                           \
-            unsigned char* dst = vs_ + (id >> 1) * VROW + (id & 1) * 8;                             \
-            *(uint2*)dst = vst[set_][i].u[0];                                                       \
-            *(uint2*)(dst + 16) = vst[set_][i].u[1];                                                \
-        }                                                                                           \
+        __builtin_amdgcn_sched_barrier(0);                                                          \
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(younger_) : "memory");   \
+        __builtin_amdgcn_sched_barrier(0);                                                          \
     }
 
-    // The group's i-th tile holds the keys from kk0 + 32 (NG i + grp) on and uses register set and
-    // shared buffer i % 2.  All groups make the same number of rounds (the barriers are the
+    // The group's i-th tile holds the keys from kk0 + 32 (NG i + grp) on and uses place i % RING.
+    // All groups make the same number of rounds (the barriers are the
     // block's); a round whose tile lies beyond the keys brings and computes nothing.
     // The walk's tiles: those of the kept first keys that lie wholly before the window's first tile, then
     // the tiles from the window's first on.
     const int kk0 = (kmin / 32) * 32;
     const int n_first = (kfb + 31) / 32 < kk0 / 32 ? (kfb + 31) / 32 : kk0 / 32;
     const int rounds = (n_first + (kmax - kk0 + 31) / 32 + NG - 1) / NG;
-#define TILE_KEY(i_) (NG * (i_) + grp < n_first ? 32 * (NG * (i_) + grp) : kk0 + 32 * (NG * (i_) + grp - n_first))
-    const int kk_first = TILE_KEY(0), kk_second = TILE_KEY(1);
-    if (kk_first < kmax) {
-        STAGE_LOAD(0, kk_first)
-        STAGE_STORE(0, 0, kk_first)
+    const int gap = kk0 - 32 * n_first;
+#define TILE_KEY(i_) (32 * (NG * (i_) + grp) + (NG * (i_) + grp < n_first ? 0 : gap))
+    // some row of the wave sees some key of the tile, and it is a tile of this block's keys
+    const int see_from = k_start - 32, see_to = wave_on ? min(k_stop, kmax) : 0;
+#define SEEN(kk_) ((kk_) < see_to && ((kk_) > see_from || (kk_) < keep_first))
+    bf16x8 qreg[D / 16];
+    int kk_r = TILE_KEY(RING), page;                       // the tile that is asked for next, and its page
+    {
+        int pages[RING];
+#pragma unroll
+        for (int t = 0; t < RING; ++t) pages[t] = PAGE_OF(TILE_KEY(t));
+        page = PAGE_OF(kk_r);
+#pragma unroll
+        for (int ks = 0; ks < D / 16; ++ks)
+            qreg[ks] = *(const bf16x8*)(q + ((long)row * Hq + head) * D + ks * 16 + g * 8);
+        __builtin_amdgcn_sched_barrier(0);
+        LOAD_TILE(TILE_KEY(0), pages[0], 0)
+        LOAD_TILE(TILE_KEY(1), pages[1], BUF)
+        // Wait for q here, with an instruction the compiler sees: else it waits for these loads where q
+        // is first used, inside the loop, where its count of loads in flight knows nothing of the loop's own,
+        // and every round would end up waiting for the loads it has just issued.
+        __builtin_amdgcn_s_waitcnt(0x0f70);                // vmcnt(0)
+#pragma unroll
+        for (int t = 2; t < RING; ++t) LOAD_TILE(TILE_KEY(t), pages[t], t * BUF)
     }
-    // (From here on the loads are issued whether their tile exists or not, one that does not
-    // exist reads the first tile again and is never stored: with loads under a condition the
-    // compiler cannot count how many are in flight and waits for all of them before every store
-    // to shared memory, the ones just issued included.)
-#define EXISTING(kk_) ((kk_) < kmax ? (kk_) : kk0)
-    STAGE_LOAD(1, EXISTING(kk_second))
-    __syncthreads();
-    for (int i2 = 0; i2 < rounds; i2 += 2) {
+    // The rows of the MFMA's first operand are the tile's keys in an order in which the eight weights of a half tile that a
+    // lane ends up with belong to eight neighbouring keys, 16 h + 8 g + 0 .. 7: row r is key r with its bits 2 and 3
+    // exchanged.  A value fragment is then one piece of a row of V^T.
+    const int kr = (r & 19) | ((r & 4) << 1) | ((r & 8) >> 1);
+    const unsigned char* const k_frag = smem + kr * KROW;
+    const int kx = D == 128 ? (kr & 15) : ((kr >> 1) & 7);
+    const unsigned char* const v_frag = smem + KBYTES + r * 32 + ((g ^ ((r >> 3) & 1)) * 16);
+    bf16x8 kf[D / 16];
+    PackV vf[D / 32][2];
+    floatx16 s;
 #pragma unroll
-      for (int buf = 0; buf < 2; ++buf) {
-        const int i = i2 + buf;
-        if (i >= rounds) break;                           // the same for all threads of the block
-        const int kk = TILE_KEY(i);
-        const int kk_1 = TILE_KEY(i + 1), kk_2 = TILE_KEY(i + 2);   // (values, not expressions in i: the macros have loops over i)
-        STAGE_LOAD(buf, EXISTING(kk_2))                   // this set's tile went to shared memory a round ago
-        __builtin_amdgcn_sched_barrier(0);                // keep the loads ahead of the computation
-        if (wave_on && kk < k_stop && (kk + 32 > k_start || kk < keep_first) && kk < kmax) {   // some row of the wave sees some key of the tile, and it is a tile of this block's keys
-            const unsigned char* ks_ = smem + buf * BUF + r * KROW + g * 16;
-            const unsigned char* vs_ = smem + buf * BUF + KBYTES + r * VROW + g * 16;
-            // all key fragments are read before the first MFMA, all value fragments before the
-            // softmax: shared-memory latency then passes under the arithmetic instead of before it
-            bf16x8 kf[D / 16];
+    for (int e = 0; e < 16; ++e) s[e] = 0.f;
+#define READ_KEYS(at_)                                                                              \
+    _Pragma("unroll") for (int ks = 0; ks < D / 16; ++ks) kf[ks] = *(const bf16x8*)(k_frag + (at_) + (((ks * 2 + g) ^ kx) * 16));
+    // A round: the weights of tile i from its scores, on the vector units, while the fragments of its values and of
+    // the next tile's keys come from shared memory; then the products of the weights and the values, and the scores of tile i + 1, in
+    // turn on the matrix units (an MFMA that adds to the one before it waits for it).  So nothing waits for shared memory, one
+    // barrier a round is enough, and two blocks on a unit fill each other's phases.  Tiles the wave sees nothing of are multiplied like the
+    // others, as zeros: with branches around the MFMAs the accumulators are copied.
+    constexpr int LT = 2 * LP;                             // loads of a wave for a tile
+    int at = 0, kk = TILE_KEY(0);
+    bool seen = SEEN(kk);
+    MEET((RING - 2) * LT)
+    READ_KEYS(0)
 #pragma unroll
-            for (int ks = 0; ks < D / 16; ++ks) kf[ks] = *(const bf16x8*)(ks_ + ks * 32);
+    for (int ks = 0; ks < D / 16; ++ks) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ks], qreg[ks], s, 0, 0, 0);
+    for (int i = 0; i < rounds; ++i) {
+        const int next = at + BUF == RING * BUF ? 0 : at + BUF;
+        const int kk_1 = TILE_KEY(i + 1);
+        const bool seen_1 = SEEN(kk_1);
+        PackV pb[2];
+        READ_KEYS(next)
+        if (!seen) {                                       // (a tile that the wave sees nothing of adds nothing; without a branch around the MFMAs)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                pb[h].v = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+                for (int db = 0; db < D / 32; ++db) vf[db][h].v = pb[h].v;
+            }
+        } else {
+#pragma unroll
+            for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) vf[db][h].v = *(const bf16x8*)(v_frag + at + (h * D + db * 32) * 32);
             __builtin_amdgcn_sched_barrier(0);
-            floatx16 s;
-#pragma unroll
-            for (int e = 0; e < 16; ++e) s[e] = 0.f;
-#pragma unroll
-            for (int ks = 0; ks < D / 16; ++ks)
-                s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ks], qreg[ks], s, 0, 0, 0);
             if (CAP) {
 #pragma unroll
                 for (int e = 0; e < 16; ++e) s[e] = soft_capped(s[e] * cap_in, cap_out);
             }
-            PackV vf[D / 32][2];
-#pragma unroll
-            for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    vf[db][h].v = *(const bf16x8*)(vs_ + (h * D + db * 32) * VROW);
-                }
-
             // (the scores stay unscaled: the scale is positive, so it is applied to the maximum, and
             // to each score by the multiply-add that also subtracts the maximum)
             float tmax = -INFINITY;
@@ -367,7 +364,7 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
             } else {
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
-                    const int key = kk + 8 * (e >> 2) + 4 * g + (e & 3);
+                    const int key = kk + 16 * (e >> 3) + 8 * g + (e & 7);
                     s[e] = ((key >= lo || key < keep_first) && key < hi) ? s[e] : -INFINITY;
                     tmax = fmaxf(tmax, s[e]);
                 }
@@ -386,7 +383,6 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
                 for (int db = 0; db < D / 32; ++db) acc[db] *= alpha;
             }
             const float ref = (m == -INFINITY) ? 0.f : m;      // a column that has seen no key yet: all weights 0
-            PackV pb[2];
             float psum = 0.f;
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
@@ -395,21 +391,50 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
                 pb[e >> 3].v[e & 7] = (__bf16)pe;
             }
             l += psum;
+            if (kk < kmin || kk + 32 > kmax) {
 #pragma unroll
-            for (int db = 0; db < D / 32; ++db)
+                for (int h = 0; h < 2; ++h) {
+                    unsigned keep[4];
 #pragma unroll
-                for (int h = 0; h < 2; ++h)
-                    acc[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[db][h].v, pb[h].v, acc[db], 0, 0, 0);
+                    for (int e = 0; e < 8; ++e) {
+                        const int key = kk + 16 * h + 8 * g + e;
+                        const unsigned on = (key >= kmin || key < kfb) && key < kmax ? 0xffffu : 0u;
+                        keep[e / 2] = e % 2 ? keep[e / 2] | on << 16 : on;
+                    }
+#pragma unroll
+                    for (int db = 0; db < D / 32; ++db) {
+                        Piece pv = __builtin_bit_cast(Piece, vf[db][h]);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) pv.q[e] &= keep[e];
+                        vf[db][h] = __builtin_bit_cast(PackV, pv);
+                    }
+                }
+            }
         }
-        __builtin_amdgcn_sched_barrier(0);
-        if (kk_1 < kmax) STAGE_STORE(buf ^ 1, buf ^ 1, kk_1)   // that buffer's readers finished before the last barrier
-        __syncthreads();
-      }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s[e] = 0.f;
+#pragma unroll
+        for (int u = 0; u < D / 16; ++u) {
+            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[u], qreg[u], s, 0, 0, 0);
+            acc[u % (D / 32)] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[u % (D / 32)][u / (D / 32)].v, pb[u / (D / 32)].v,
+                                                                        acc[u % (D / 32)], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        MEET((RING - 3) * LT)
+        LOAD_TILE(kk_r, page, at)                          // the place was read for the last time before the last barrier
+        kk_r = TILE_KEY(i + RING + 1);
+        page = PAGE_OF(kk_r);
+        at = next;
+        kk = kk_1;
+        seen = seen_1;
     }
-#undef STAGE_LOAD
-#undef EXISTING
-#undef STAGE_STORE
+    MEET(0)                                                // (what was asked for beyond the end arrives too, before the memory is used again)
+#undef LOAD_TILE
+#undef PAGE_OF
+#undef MEET
 #undef TILE_KEY
+#undef SEEN
+#undef READ_KEYS
     l = sum_of_both_halves(l);
     if (NG == 2) {
         // group 1 hands its maxima, sums and accumulators to group 0, 16 values of every lane at a
@@ -649,11 +674,19 @@ int qe_attention_prefill(const void* q, void* out, const void* cache, const int*
     if (groups == 0) groups = qe_attention_prefill_choose_groups((long)grid.x * grid.z, (long)num_tiles * R, window, max_keys);
     QE_REQUIRE(groups == 1 || groups == 2, "prefill attention: %d groups a block", groups);
 #define QE_PREFILL_CAP(D_, NG_, CAP_)                                                               \
-    attention_prefill_kernel<D_, NG_, CAP_><<<grid, 256 * NG_, 0, stream>>>(                        \
+    {                                                                                               \
+        constexpr int shmem_ = NG_ * RING * 2 * 32 * D_ * 2;                                       \
+        static bool raised_ = false;   /* (once per kernel: the limit of dynamic shared memory) */  \
+        if (!raised_) {                                                                             \
+            (void)hipFuncSetAttribute((const void*)attention_prefill_kernel<D_, NG_, CAP_>, hipFuncAttributeMaxDynamicSharedMemorySize, shmem_); \
+            raised_ = true;                                                                         \
+        }                                                                                           \
+        attention_prefill_kernel<D_, NG_, CAP_><<<grid, 256 * NG_, shmem_, stream>>>(               \
         (const bf16_t*)q, (bf16_t*)out, (const bf16_t*)cache, tiles, positions, tok_seq, block_table, \
         max_blocks, Hq, Hkv, P, log2P, scale_log2, window, R, seg_keys, keys_row, (float*)workspace, keep_first, sink, \
-        cap_in, cap_out, tail)
-#define QE_PREFILL(D_, NG_) do { if (softcap > 0.f) QE_PREFILL_CAP(D_, NG_, true); else QE_PREFILL_CAP(D_, NG_, false); } while (0)
+        cap_in, cap_out, tail);                                                                     \
+    }
+#define QE_PREFILL(D_, NG_) do { if (softcap > 0.f) QE_PREFILL_CAP(D_, NG_, true) else QE_PREFILL_CAP(D_, NG_, false) } while (0)
     if (D == 128) { if (groups == 2) QE_PREFILL(128, 2); else QE_PREFILL(128, 1); }
     else          { if (groups == 2) QE_PREFILL(64, 2); else QE_PREFILL(64, 1); }
 #undef QE_PREFILL

@@ -677,3 +677,35 @@ def test_products_whose_parts_are_rounded_are_large(ops, K):
             splits = ops.gemm_branch_splits_for(M, w, torch.bfloat16)
             tiles = -(-M // 128) * -(-N // 128)
             assert (splits == 0) == (K < 1024) or (splits == 0 and tiles > 256), (M, N, K, splits)
+
+
+@pytest.mark.parametrize("D,P", [(128, 16), (128, 64), (64, 16), (64, 32)])
+@pytest.mark.parametrize("groups", [1, 2])
+def test_prefill_attention_over_few_and_many_tiles(ops, D, P, groups):
+    """Prompts that end inside, at and behind tiles of 32 keys, with fewer tiles than shared memory takes and with more, alone and
+    behind keys of an earlier step, with and without a window; what the pages hold beside the keys is NaN."""
+    from qwen_engine_amd.parts.attention import prefill_tiles
+    hq, hkv = 4, 2
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    for n, before, window in ((1, 0, 0), (15, 0, 0), (33, 0, 0), (64, 0, 0), (97, 31, 0), (128, 0, 0), (129, 16, 0), (160, 0, 40),
+                              (161, 100, 33), (290, 7, 0), (300, 0, 128)):
+        L = before + n
+        k, v, q = (rand(L, h, D, seed=s + L, dtype=torch.bfloat16) for s, h in ((1, hkv), (2, hkv), (3, hq)))
+        pages = -(-L // P)
+        cache = torch.full((pages + 1, 2, hkv, P, D), float("nan"), dtype=torch.bfloat16)
+        order = torch.randperm(pages, generator=torch.Generator().manual_seed(L)) + 1
+        vt = cache[:, 1].view(-1, hkv, D, P)
+        for t in range(L):
+            cache[order[t // P], 0, :, t % P] = k[t]
+            vt[order[t // P], :, :, t % P] = v[t]
+        tiles = i32(prefill_tiles([(0, n)], ops.prefill_tile_rows(hq, hkv))).view(-1, 2)
+        got = ops.attention(q[before:].contiguous().to(DEV), cache.to(DEV), i32(list(range(before, L))), i32([0] * n), order.int()[None].to(DEV), D ** -0.5, window=window,
+                            other_tokens=i32(list(range(n))), other_tiles=tiles, prefill_groups=groups).view(n, hq, D).cpu().double()
+        pos, key = torch.arange(before, L)[:, None], torch.arange(L)[None]
+        hidden = (key > pos) | ((key <= pos - window) if window else torch.zeros_like(key, dtype=torch.bool))
+        for h in range(hq):
+            s = (q[before:, h].double() @ k[:, h // 2].double().t() * D ** -0.5).masked_fill(hidden, float("-inf"))
+            w = torch.softmax(s, -1)
+            want, size = w @ v[:, h // 2].double(), w @ v[:, h // 2].double().abs()
+            # (each weight and the result rounded to 8 bits of mantissa: 2^-8 of the sum of the sizes, 2^-8 of the result)
+            assert ((got[:, h] - want).abs() <= 2.0 ** -8 * (size + want.abs()) + 1e-6).all(), (n, before, window, h)
