@@ -11,11 +11,11 @@
 // k by one load and use them in four instructions).  The chunks of a quarter are added in order, then
 // the quarters in order.
 //
-// Two kernels share that order:
+// Three kernels share that order (the third, for the logits, beside itself):
 //   few rows: a block owns 16 outputs (or 32) and has a wave per chunk (16 from K = 1024 on), so that the weights are asked for
 //     by all its waves at once and the sums meet in shared memory.  Bound by the stream of the weights and
 //     a kernel's fixed cost.  Two rows (as 64 x 64 tiles before): 4096 x 1024 7.1 us (42), 6144 x 1024 10.6 (42),
-//     1024 x 3072 11.6 (117), 151936 x 1024 137 (215; 4.5 TB/s).  At most 64 registers a lane, so that two
+//     1024 x 3072 11.6 (117), 151936 x 1024 137 (215).  At most 64 registers a lane, so that two
 //     blocks of 16 waves fit a compute unit (four steps at a time instead of two: 10.0, 17.7, 14.5 and 294 us).
 //   more rows: tiles of 64 x 64, a wave a 32 x 32 quarter, K in steps of 16 through two buffers of shared
 //     memory.  With fewer than TILES_FOR_FOUR tiles and a K that gives each something four groups of four
@@ -159,6 +159,74 @@ __global__ __launch_bounds__(64 * CHUNKS) void gemm_f32_rows_kernel(const float*
     }
 }
 
+// The same for up to 16 rows against a matrix of very many rows (the logits'), K up to 1024 in whole lines of 32 numbers: blocks of 16
+// outputs and four waves, a wave a quarter of K, its (up to) four chunks of 64 one after the other.  A chunk's 16 x 64 weights come as whole lines of 128
+// bytes, 8 lanes a row, straight to shared memory, two chunks of a wave on their way; the row's pieces are exchanged there (piece p of row r at
+// place p ^ (r / 2 % 8)) so that the reads in the operands' layout fall into distinct banks.  Five such blocks share a unit, and the
+// end of one is hidden by the others (two rows against 151936 x 1024: 135 us with sixteen waves a block, now 100; one block's lines of all
+// sixteen chunks at once, two blocks a unit, took 128; 32768 x 1024 32.0, now 25.0; 16400 x 512 10.9, now 10.5; 20000 x 96 4.7 and 6.9).
+__global__ __launch_bounds__(256, 5) void gemm_f32_lines_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                                const float* __restrict__ bias, float* __restrict__ out,
+                                                                int M, int N, int K) {
+    typedef __attribute__((ext_vector_type(4))) unsigned int uint4_t;
+    constexpr int CHUNK = 4 * FK, QUARTER = 4 * CHUNK;
+    __shared__ __attribute__((aligned(16))) float lines[4][2][1024];       // a wave's two chunks
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, r = lane & 15;
+    const int n0 = blockIdx.x * 16, k_lo = wave * QUARTER, left = K - k_lo;        // (a block has a wave per quarter that holds some of K)
+    const float* xrow = x + (long)min(r, M - 1) * K + 4 * g + k_lo;
+    floatx4 xv[16];
+#pragma unroll
+    for (int s = 0; s < 16; ++s) xv[s] = *(const floatx4_any*)(xrow + min(s * FK, left - FK));
+    __builtin_amdgcn_sched_barrier(0);
+    // (rows beyond the matrix are out of the descriptor's range and arrive as zeros, as does what lies beyond the last row's end; what lies
+    // beyond another row's end is the next row's and is not multiplied)
+    const unsigned long base = (unsigned long)(w + (long)n0 * K);
+    const uint4_t rsrc = {(unsigned)base, (unsigned)(base >> 32) & 0xffffu, (unsigned)(min(16, N - n0) * K) * 4u, 0x00020000u};
+    const unsigned to = (unsigned)(unsigned long)(__attribute__((address_space(3))) float*)lines + wave * 8192;
+    int off[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) off[i] = ((8 * i + (lane >> 3)) * K + ((lane & 7) ^ (4 * i + (lane >> 4))) * 4) * 4;
+    auto ask = [&](int c) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
+                         : : "s"(to + (c & 1) * 4096 + i * 1024), "v"(off[i & 1]), "s"(rsrc), "s"((k_lo + c * CHUNK + (i >> 1) * 32) * 4) : "memory");
+    };
+    ask(0);
+    ask(1);
+    floatx4 quarter;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        if (c < 3) asm volatile("s_waitcnt vmcnt(4)" : : : "memory");      // (the wave's own lines: no barrier)
+        else asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+        floatx4 wv[4], acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) wv[s] = *(const floatx4*)(&lines[wave][c & 1][(s >> 1) * 512 + r * 32 + ((((s & 1) * 4 + g) ^ (r >> 1)) * 4)]);
+        if (c < 2) {
+            asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(wv[0]), "+v"(wv[1]), "+v"(wv[2]), "+v"(wv[3]) : : "memory");
+            ask(c + 2);
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            if (c * CHUNK + s * FK >= left) break;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[c * 4 + s][e], wv[s][e], acc, 0, 0, 0);
+        }
+        if (c == 0) quarter = acc;
+        else if (c * CHUNK < left) quarter += acc;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) lines[wave][0][e * 64 + lane] = quarter[e];
+    __syncthreads();
+    const int waves = blockDim.x >> 6;
+    for (int at = threadIdx.x; at < 256; at += blockDim.x) {
+        float total = lines[0][0][at];
+        for (int q = 1; q < waves; ++q) total += lines[q][0][at];
+        const int m = 4 * ((at & 63) >> 4) + (at >> 6), n = n0 + (at & 15);
+        if (m < M && n < N) out[(long)m * N + n] = bias ? total + bias[n] : total;
+    }
+}
+
 // Tiles of 64 x 64, GROUPS (1 or 4) groups of four waves.  For a step, lane (h, r), h = lane / 32, r = lane % 32, reads
 // x[row r][4 h .. + 4] and [8 + 4 h .. + 4], and the same of W: with the instructions taking element j of the first and of
 // the second piece in turn, the order is the one above.
@@ -291,7 +359,10 @@ int qe_gemm_f32(const float* x, const float* w, const float* bias, float* out, i
         // 32 outputs a block halve the reads of x; they pay where the rows are some and the blocks enough (16 rows,
         // 6144 x 1024: 12.0 us against 14.3, 151936 x 1024: 183 against 213; 2 rows: 10.3 against 10.6, 148 against 137;
         // 16 rows, 4096 x 1024: 11.5 against 9.5)
-        if (M > 4 && M <= 16 && N >= 6144) launch_rows<1, 2, 1>(x, w, bias, out, M, N, K, rows, stream);
+        // (the logits; with fewer chunks than eight a wave's walk is not worth a block)
+        if (M <= 16 && N >= 16384 && K > 512 && K <= 4 * FK * CHUNKS && K % 32 == 0 && (((unsigned long)w) & 15) == 0)
+            gemm_f32_lines_kernel<<<qe_cdiv(N, 16), 64 * qe_cdiv(K, 16 * FK), 0, stream>>>(x, w, bias, out, M, N, K);
+        else if (M > 4 && M <= 16 && N >= 6144) launch_rows<1, 2, 1>(x, w, bias, out, M, N, K, rows, stream);
         else if (M <= 16) launch_rows<1, 1, 2>(x, w, bias, out, M, N, K, rows, stream);
         else if (M <= 32) launch_rows<2, 1, 2>(x, w, bias, out, M, N, K, rows, stream);
         else launch_rows<4, 1, 1>(x, w, bias, out, M, N, K, rows, stream);

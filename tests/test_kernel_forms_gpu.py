@@ -709,3 +709,19 @@ def test_prefill_attention_over_few_and_many_tiles(ops, D, P, groups):
             want, size = w @ v[:, h // 2].double(), w @ v[:, h // 2].double().abs()
             # (each weight and the result rounded to 8 bits of mantissa: 2^-8 of the sum of the sizes, 2^-8 of the result)
             assert ((got[:, h] - want).abs() <= 2.0 ** -8 * (size + want.abs()) + 1e-6).all(), (n, before, window, h)
+
+
+@pytest.mark.parametrize("N,K", [(16384, 544), (16390, 992), (20001, 1024)])
+def test_float32_logits_sum_in_the_same_order(ops, N, K):
+    """Few rows against a matrix of very many (its last block of 16 outputs whole and not, K whole quarters and not): the bits
+    that the tiles give a row among many, and those of operands at an odd address."""
+    x, w, bias = rand(20, K, seed=K).to(DEV), rand(N, K, seed=N).to(DEV), rand(N, seed=3).to(DEV)
+    every = ops.gemm(x, w, bias)
+    want = x.cpu().double() @ w.cpu().double().t() + bias.cpu().double()
+    bound = 2.0 ** -24 * K ** 0.5 * 4 * (x.cpu().double().abs() @ w.cpu().double().abs().t() + bias.cpu().double().abs())
+    for M in (1, 3, 16):
+        got = ops.gemm(x[:M].contiguous(), w, bias)
+        assert torch.equal(got, every[:M]), M
+        assert ((got.cpu().double() - want[:M]).abs() <= bound[:M]).all(), M
+    odd = torch.cat([w.new_zeros(1), w.reshape(-1)])[1:].view(N, K)
+    assert odd.data_ptr() % 16 == 4 and torch.equal(ops.gemm(x[:2].contiguous(), odd, bias), every[:2])
