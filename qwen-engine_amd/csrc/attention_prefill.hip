@@ -518,19 +518,41 @@ __global__ __launch_bounds__(256) void attention_prefill_merge_kernel(
     const int row = row0 + rr;
     const long zstride = (long)gridDim.x * gridDim.z * 4 * NV * 64;
     const float* src = part + (((long)bhead * gridDim.z + bgroup) * 4 + wave) * NV * 64 + lane;
+    // Four segments are asked for at once, their accumulators without waiting for the maxima (those of a segment of which the column saw
+    // no key were never written and are not used; a segment beyond the last is the last again).  One after the other, with a trip
+    // to memory for each of its loops' rounds, four segments of 512 rows of 16 heads took 8.0 us,
+    // now 6.7.
+    constexpr int AT = 4;
+    float ms[AT], ls[AT], as[AT][16];
+    const auto ask = [&](int z0) {
+#pragma unroll
+        for (int k = 0; k < AT; ++k) {
+            const float* at = src + min(z0 + k, z_hi) * zstride;
+            ms[k] = at[0];
+            ls[k] = at[64];
+#pragma unroll
+            for (int e = 0; e < 16; ++e) as[k][e] = at[(2 + db * 16 + e) * 64];
+        }
+    };
+    ask(z_lo);
     float M = -INFINITY;
-    for (int z = z_lo; z <= z_hi; ++z) M = fmaxf(M, src[z * zstride]);
+#pragma unroll
+    for (int k = 0; k < AT; ++k) M = fmaxf(M, ms[k]);
+    for (int z = z_lo + AT; z <= z_hi; ++z) M = fmaxf(M, src[z * zstride]);
     float l = 0.f;
     floatx16 acc;
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[e] = 0.f;
-    for (int z = z_lo; z <= z_hi; ++z) {
-        const float mz = src[z * zstride];
-        if (mz == -INFINITY) continue;                     // no key of this segment was seen by the column
-        const float wgt = __builtin_amdgcn_exp2f(mz - M);
-        l += wgt * src[z * zstride + 64];
+    for (int z = z_lo; z <= z_hi; z += AT) {
+        if (z > z_lo) ask(z);
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[e] += wgt * src[z * zstride + (2 + db * 16 + e) * 64];
+        for (int k = 0; k < AT; ++k) {
+            if (z + k > z_hi || ms[k] == -INFINITY) continue;
+            const float wgt = __builtin_amdgcn_exp2f(ms[k] - M);
+            l += wgt * ls[k];
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[e] += wgt * as[k][e];
+        }
     }
     const float inv = 1.f / l;
     bf16_t* orow = out + (long)row * tail.out_stride + (long)head * D + 4 * g + db * 32;

@@ -453,8 +453,9 @@ __global__ __launch_bounds__(256) void skip_gate_norm_regs_kernel(SkipGateNorm a
     __shared__ float part[NV * 4];
     const long t = blockIdx.x;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, N = a.N, n = N / a.groups;
-    float v[NV][4], zv[NV][4], xv[NV][4], w[NV][4];
-    int cs[NV];
+    float v[NV][4], zv[NV][4], xv[NV][4], w[NV][4], s0[NV];
+    int cs[NV], h0[NV];
+    const bool whole = a.Dv % 4 == 0;                      // (four numbers side by side are of one head)
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int c = (threadIdx.x + i * 256) * 4;
@@ -465,15 +466,19 @@ __global__ __launch_bounds__(256) void skip_gate_norm_regs_kernel(SkipGateNorm a
         Vec4<float>::load(a.w + cs[i], w[i]);
     }
 #pragma unroll
+    for (int i = 0; i < NV; ++i) {                         // (on the same trip to memory)
+        h0[i] = cs[i] / a.Dv;
+        s0[i] = a.skip[h0[i]];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
     for (int i = 0; i < NV; ++i) {
         const bool ok = (threadIdx.x + i * 256) * 4 < N;
-        const int h0 = cs[i] / a.Dv;
-        const float s0 = a.skip[h0];
         float ss = 0.f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int c = cs[i] + e;
-            const float s = c < (h0 + 1) * a.Dv ? s0 : a.skip[c / a.Dv];
+            const float s = whole || c < (h0[i] + 1) * a.Dv ? s0[i] : a.skip[c / a.Dv];
             const float u = fmaf(s, xv[i][e], v[i][e]);
             v[i][e] = u * silu_f(zv[i][e]);
             ss += v[i][e] * v[i][e];
