@@ -91,8 +91,8 @@ extern "C" int qe_gemm_partial_splits(int M, int N, int K) {
 // should be asked for: 0 = as a plain product; S >= 1 = as S partial products (epilogue 3), which
 // that norm adds up.  Few rows: always, the cut fills the chip.  More rows: what the product (qe_gemm_mfma_shape) and the
 // parts' way into the norm (4 bytes a number at 6 TB/s, a plain product's 2) take together, for each number of
-// cuts that leaves 512 of K to a part; the cuts give every compute unit as many tiles as the others (800 rows against 5120 x 25600 with the norm
-// behind it: 232 us in three cuts of 256 x 256, 347 as a plain product).  Parts beyond 2^27 numbers (512 MiB, what a pool of pages that takes
+// cuts that leaves 512 of K to a part; the cuts give every compute unit as many tiles as the others (800 rows against 5120 x 25600: 200 us in three
+// cuts of 256 x 256, 303 at the best without one; 528 against 4096 x 12288 72 in three of 128 x 128, 107).  Parts beyond 2^27 numbers (512 MiB, what a pool of pages that takes
 // nearly all memory should leave a step) are not asked for.  A plain product's numbers are rounded to 16 bits on their way to the norm,
 // which only many rows against a K that needs no cut pay for (those bytes are then a twentieth of the time); elsewhere a product that
 // is quickest without a cut is one 32-bit part.

@@ -112,7 +112,7 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
         } else {
             // no cut into equal parts: each XCD takes an eighth of the walk below through all tiles (dealt out block by
             // block, every XCD read nearly all of W: 1600 rows against 5120 x 25600 in three cuts, 7 by 20 tiles of
-            // 256 x 256: 455 us, now 435; 8192 rows of 32 experts of 2048 x 2048: 137 us, now 122)
+            // 256 x 256: 455 us, then 435; 8192 rows of 32 experts of 2048 x 2048: 137 us, then 122)
             const int all = rows_m * tiles_n, each = all / 8, over = all % 8;
             if (local >= each + (xcd < over)) return;
             local += xcd * each + min(xcd, over);
@@ -122,7 +122,7 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
         // tiles, which reads 12 or 16 tiles' worth of rows where a column of 32 reads 33 (what
         // the XCDs fetch through the fabric is what bounds a large product).  With bands of a divisor of the tile rows
         // instead, five tile rows went one after the other, each through all of W: 272 rows
-        // against 51200 x 5120 in tiles of 64 rows 470 us, now 266; 528 rows in tiles of 128 rows 476, now 337.
+        // against 51200 x 5120 in tiles of 64 rows 470 us, then 266; 528 rows in tiles of 128 rows 476, then 337.
         const int band = local / (8 * per_n), within = local - band * 8 * per_n;
         const int rows = min(8, per_m - band * 8);
         tile_m = part_m + band * 8 + within % rows;
@@ -846,7 +846,7 @@ static int choose_tile(int M, int N, int K, int splits, bool largest = true) {
 
 // Where the last turn of a product's tiles would leave most units idle, the columns that fill the turns before it go first, and the
 // rest in a launch and a shape of its own: the number of the first columns, a multiple of 256, or 0.  Three microseconds for the
-// second launch; less than 3 % is not worth it.  (1972 rows against gate and up of 51200 x 5120, 1600 tiles of 256 x 256: 923 us,
+// second launch; less than 3 % is not worth it.  (With the rates that the shapes had when loads went through registers: 1972 rows against gate and up of 51200 x 5120, 1600 tiles of 256 x 256: 923 us,
 // now 884; 656 rows 434, now 342;
 // 1300 rows against 24576 x 4096 299, now 269; q, k and v of 10240 x 5120 with 1600 rows 254, now 193.)
 static int first_columns(int M, int N, int K, bool largest = true) {
@@ -885,9 +885,9 @@ static int pick_mfma(const void* x, const void* w, const float* bias, void* out,
     QkvTail tail{};
     tail.n_first = n_first;
     // Up to 64 rows against a gate|up matrix of at most one tile column a compute unit (its K cannot be
-    // cut): a block streams its weights alone on its unit, and what it has in flight bounds it.  A k step of
-    // 128 doubles that (24576 x 4096 against 64 rows: 44.4 us against 49.2; with two blocks a unit, 51200 x
-    // 5120, it gains nothing).
+    // cut): a block streams its weights alone on its unit, and what it has in flight bounds it.  A ring of six stages
+    // doubles that (24576 x 4096 against 64 rows: 37.8 us; through registers 49.2, with k steps of 128 40.2; with two blocks a unit, 51200 x
+    // 5120, a longer ring gains nothing).
     if (tile == 0 && SILU > 0 && M <= 64 && qe_cdiv(N, 128) <= 256) tile = 65;
     // (the gelu of 65536 values is 35 us in which nothing else runs on the unit: 256 x 256 is never its shape; 3000 rows against
     // 4096 x 1024: 65 us in it, 52 in 256 x 128, 47 in 128 x 128)
@@ -899,7 +899,7 @@ static int pick_mfma(const void* x, const void* w, const float* bias, void* out,
     return launch_mfma<TO, 64, 128, 3, 4, 2, SILU>(x, w, bias, out, M, N, K, n_cols, splits, stream, tail);
 }
 
-// tile: rows of the output tile (256, 128 or 64; 512 stands for 256 x 256, 65 for 64 x 128 with a k step of 128), 0 to choose
+// tile: rows of the output tile (256, 128 or 64; 512 stands for 256 x 256, 65 for 64 x 128 with a ring of six stages), 0 to choose
 // by the shape.  silu: w is [N, K] with
 // gate and up rows interleaved in blocks of 32, out is [M, N / 2] = silu(gate) * up.
 // splits > 1: out is float [splits, M, N], partial products along K (no silu then).
