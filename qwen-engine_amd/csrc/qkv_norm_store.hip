@@ -64,44 +64,6 @@ __global__ __launch_bounds__(1024) void qkv_norm_store_kernel(
     float* sc = sv + Nv;         // rot_dims: cosines, then sines
     const TI* row = qkv + t * row_stride;
     const int tid = threadIdx.x, nt = blockDim.x;
-    // A single row's time is its trips to memory: the row's numbers, the norm's weights, the values to blend with and the slot are
-    // asked for together, up to PB of each a thread (eight rows of 3072 normed whole 9.1 us, now 8.4; one row of
-    // 16 heads of 128, by heads, 6.8, now 5.9); longer rows walk as they come.
-    constexpr int PB = 4;
-    const int total = Nq + Nk + (values_from_keys ? 0 : Nv);
-    const bool held = total <= PB * nt;
-    float x[PB], w[PB], vfirst[PB];
-    // (the place of number c of this block's q | k | v in the row)
-    const auto at = [&](int c) { return c < Nq ? q0 * Dk + c : c < Nq + Nk ? HqT * Dk + k0 * Dk + c - Nq : (HqT + HkvT) * Dk + k0 * Dv + c - Nq - Nk; };
-    const bool blend = v_first && !v_first_write;
-    const float* vf_row = v_first ? v_first + t * ((long)HkvT * Dv) + k0 * Dv : nullptr;
-    const int slot = slots ? slots[t] : -1;
-    const float lam = blend ? v_blend[0] : 0.f;
-    float hw[2][2];              // a head's weights, of q and of k: the lane's two numbers of a head of up to 128
-    if (qk_mode == QKN_HEAD) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int d = min((tid & 63) + 64 * j, Dk - 1);
-            hw[0][j] = q_w[d];
-            hw[1][j] = k_w[d];
-        }
-    }
-    if (held) {
-#pragma unroll
-        for (int j = 0; j < PB; ++j) x[j] = Elem<TI>::load(row + at(min(tid + j * nt, total - 1)));
-        if (qk_mode == QKN_WHOLE) {
-#pragma unroll
-            for (int j = 0; j < PB; ++j) {
-                const int c = min(tid + j * nt, Nq + Nk - 1);
-                w[j] = c < Nq ? q_w[c] : k_w[c - Nq];
-            }
-        }
-        if (blend) {
-#pragma unroll
-            for (int j = 0; j < PB; ++j) vfirst[j] = vf_row[min(tid + j * nt, Nv - 1)];
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    }
     if (rot_dims > 0) {          // (one angle for all heads)
         const float pos = (float)positions[t];
         for (int j = tid; j < rot_dims >> 1; j += nt) {
@@ -111,16 +73,10 @@ __global__ __launch_bounds__(1024) void qkv_norm_store_kernel(
             sc[j + (rot_dims >> 1)] = s * rot_gain;
         }
     }
-    if (held) {
-#pragma unroll
-        for (int j = 0; j < PB; ++j)
-            if (tid + j * nt < total) sm[tid + j * nt] = x[j];
-    } else {
-        for (int c = tid; c < Nq; c += nt) sq[c] = Elem<TI>::load(row + q0 * Dk + c);
-        for (int c = tid; c < Nk; c += nt) sk[c] = Elem<TI>::load(row + HqT * Dk + k0 * Dk + c);
-        if (!values_from_keys)
-            for (int c = tid; c < Nv; c += nt) sv[c] = Elem<TI>::load(row + (HqT + HkvT) * Dk + k0 * Dv + c);
-    }
+    for (int c = tid; c < Nq; c += nt) sq[c] = Elem<TI>::load(row + q0 * Dk + c);
+    for (int c = tid; c < Nk; c += nt) sk[c] = Elem<TI>::load(row + HqT * Dk + k0 * Dk + c);
+    if (!values_from_keys)
+        for (int c = tid; c < Nv; c += nt) sv[c] = Elem<TI>::load(row + (HqT + HkvT) * Dk + k0 * Dv + c);
     __syncthreads();
     if (values_from_keys) {      // the keys as projected (Dv == Dk)
         for (int c = tid; c < Nv; c += nt) sv[c] = sk[c];
@@ -140,30 +96,19 @@ __global__ __launch_bounds__(1024) void qkv_norm_store_kernel(
             b = wide_sum(sk, Nk, red);
         }
         const float fq = rsqrtf(a / (float)Nq + qk_eps), fk = rsqrtf(b / (float)Nk + qk_eps);
-        if (held) {
-#pragma unroll
-            for (int j = 0; j < PB; ++j) {
-                const int c = tid + j * nt;
-                if (c < Nq + Nk) sm[c] = x[j] * (c < Nq ? fq : fk) * w[j];
-            }
-        } else {
-            for (int c = tid; c < Nq; c += nt) sq[c] = sq[c] * fq * q_w[c];
-            for (int c = tid; c < Nk; c += nt) sk[c] = sk[c] * fk * k_w[c];
-        }
+        for (int c = tid; c < Nq; c += nt) sq[c] = sq[c] * fq * q_w[c];
+        for (int c = tid; c < Nk; c += nt) sk[c] = sk[c] * fk * k_w[c];
         __syncthreads();
     } else if (qk_mode == QKN_HEAD) {
         const int lane = tid & 63, wave = tid >> 6, nw = nt >> 6;
         for (int h = wave; h < Hq + Hkv; h += nw) {      // (q and k heads lie one after the other in sm)
             float* hp = sm + (long)h * Dk;
             const float* w = h < Hq ? q_w : k_w;
-            const float w0 = h < Hq ? hw[0][0] : hw[1][0], w1 = h < Hq ? hw[0][1] : hw[1][1];
             float a = 0.f;
             for (int d = lane; d < Dk; d += 64) a += hp[d] * hp[d];
             a = wave_sum(a);
             const float f = rsqrtf(a / (float)Dk + qk_eps);
-            if (lane < Dk) hp[lane] = hp[lane] * f * w0;
-            if (lane + 64 < Dk) hp[lane + 64] = hp[lane + 64] * f * w1;
-            for (int d = lane + 128; d < Dk; d += 64) hp[d] = hp[d] * f * w[d];
+            for (int d = lane; d < Dk; d += 64) hp[d] = hp[d] * f * w[d];
         }
         __syncthreads();
     }
@@ -181,19 +126,12 @@ __global__ __launch_bounds__(1024) void qkv_norm_store_kernel(
         __syncthreads();
     }
     if (v_first) {
+        float* vf = v_first + t * ((long)HkvT * Dv) + k0 * Dv;
         if (v_first_write) {
-            float* vf = v_first + t * ((long)HkvT * Dv) + k0 * Dv;
             for (int c = tid; c < Nv; c += nt) vf[c] = sv[c];
         } else {
-            if (held && Nv <= PB * nt) {
-#pragma unroll
-                for (int j = 0; j < PB; ++j) {
-                    const int c = tid + j * nt;
-                    if (c < Nv) sv[c] = (1.f - lam) * sv[c] + lam * vfirst[j];
-                }
-            } else {
-                for (int c = tid; c < Nv; c += nt) sv[c] = (1.f - lam) * sv[c] + lam * vf_row[c];
-            }
+            const float lam = v_blend[0];
+            for (int c = tid; c < Nv; c += nt) sv[c] = (1.f - lam) * sv[c] + lam * vf[c];
             __syncthreads();
         }
     }
@@ -214,6 +152,7 @@ __global__ __launch_bounds__(1024) void qkv_norm_store_kernel(
         const int h = i / Dc, d = i - h * Dc;
         Elem<TA>::store(qo + i, d < Dk ? sq[h * Dk + d] : 0.f);
     }
+    const int slot = slots ? slots[t] : -1;
     if (slot < 0) return;                                  // (a row that writes nowhere)
     const long page = slot / P;
     const int off = slot % P;
