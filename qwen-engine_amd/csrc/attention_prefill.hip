@@ -143,7 +143,10 @@ __device__ __forceinline__ void store_columns(bf16_t* __restrict__ out, const fl
 // two: while one wave waits for its next tile or at its barrier, the other computes.
 // CAP: the scaled scores pass cap * tanh(. / cap): cap_in is the scores' scale times 2 log2(e) / cap, cap_out the cap
 // in the base-2 domain, and scale_log2 is 1.
-template <int D, int NG, bool CAP>
+// DIRECT: the cache begins at a whole 16-byte piece, which loads that write to shared memory themselves want.  Tiles of a cache that lies
+// elsewhere come through registers, asked for a round before they are stored to their place; the same bits (8192 tokens of 32 heads of 128 on 8
+// 546 us and 609, 2048 of 16 heads 45 and 58, 512 rows behind 7680 keys 50 and 61).
+template <int D, int NG, bool CAP, bool DIRECT>
 __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_kernel(
     const bf16_t* __restrict__ q, bf16_t* __restrict__ out, const bf16_t* __restrict__ cache,
     const int* __restrict__ tiles, const int* __restrict__ positions, const int* __restrict__ tok_seq,
@@ -251,11 +254,13 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
     const unsigned lds_v = lds_k + KBYTES;                 // (as many bytes of a tile's values before a wave's as of its keys)
     // (a tile's place, and the page of this wave's half of it; no more than the last key's page is ever asked for)
 #define PAGE_OF(kk_) bt[min((kk_) + 16 * half, kmax - 1) >> log2P]
+#define TILE_HALF(kk_)                                                                              \
+        const int key_ = (kk_) + 16 * half, off_ = key_ & pmask;                                    \
+        const bool there_ = key_ < kmax && (key_ + 16 > kmin || key_ < kfb);
 #define LOAD_TILE(kk_, page_, at_)                                                                  \
     {                                                                                               \
+        TILE_HALF(kk_)                                                                              \
         const unsigned long base_ = (unsigned long)(cache + (long)(page_) * page_stride);           \
-        const int key_ = (kk_) + 16 * half, off_ = key_ & pmask;                                    \
-        const bool there_ = key_ < kmax && (key_ + 16 > kmin || key_ < kfb);                        \
         const uint4_t rsrc_ = {(unsigned)base_, (unsigned)(base_ >> 32) & 0xffffu, there_ ? (unsigned)page_bytes : 0u, 0x00020000u}; \
         _Pragma("unroll") for (int i_ = 0; i_ < LP; ++i_) {                                         \
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"  \
@@ -263,6 +268,24 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"  \
                          : : "s"(lds_v + (at_) + i_ * 1024), "v"(vconst[i_]), "s"(rsrc_), "s"(off_ * 2) : "memory"); \
         }                                                                                           \
+    }
+    // (the two steps of it through registers)
+    [[maybe_unused]] uint4_t kst[LP], vst[LP];
+#define FETCH_TILE(kk_, page_)                                                                      \
+    {                                                                                               \
+        TILE_HALF(kk_)                                                                              \
+        const __amdgpu_buffer_rsrc_t rsrc_ = __builtin_amdgcn_make_buffer_rsrc(                     \
+            (void*)(cache + (long)(page_) * page_stride), 0, there_ ? page_bytes : 0, 0x00020000);  \
+        _Pragma("unroll") for (int i_ = 0; i_ < LP; ++i_) {                                         \
+            kst[i_] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_, kconst[i_], off_ * (D * 2), 0);  \
+            vst[i_] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_, vconst[i_], off_ * 2, 0);        \
+        }                                                                                           \
+    }
+#define PUT_TILE(at_)                                                                               \
+    _Pragma("unroll") for (int i_ = 0; i_ < LP; ++i_) {                                             \
+        unsigned char* const to_ = smem + (at_) + wave * (LP * 1024) + i_ * 1024 + lane * 16;       \
+        *(uint4_t*)to_ = kst[i_];                                                                   \
+        *(uint4_t*)(to_ + KBYTES) = vst[i_];                                                        \
     }
     // waits until at most younger_ loads of the wave are in flight and its reads of shared memory are done, then for the other
     // waves; nothing is moved across
@@ -297,14 +320,25 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
         for (int ks = 0; ks < D / 16; ++ks)
             qreg[ks] = *(const bf16x8*)(q + ((long)row * Hq + head) * D + ks * 16 + g * 8);
         __builtin_amdgcn_sched_barrier(0);
-        LOAD_TILE(TILE_KEY(0), pages[0], 0)
-        LOAD_TILE(TILE_KEY(1), pages[1], BUF)
+        if constexpr (DIRECT) {
+            LOAD_TILE(TILE_KEY(0), pages[0], 0)
+            LOAD_TILE(TILE_KEY(1), pages[1], BUF)
+        }
         // Wait for q here, with an instruction the compiler sees: else it waits for these loads where q
         // is first used, inside the loop, where its count of loads in flight knows nothing of the loop's own,
         // and every round would end up waiting for the loads it has just issued.
         __builtin_amdgcn_s_waitcnt(0x0f70);                // vmcnt(0)
+        if constexpr (DIRECT) {
 #pragma unroll
-        for (int t = 2; t < RING; ++t) LOAD_TILE(TILE_KEY(t), pages[t], t * BUF)
+            for (int t = 2; t < RING; ++t) LOAD_TILE(TILE_KEY(t), pages[t], t * BUF)
+        } else {
+#pragma unroll
+            for (int t = 0; t < RING - 1; ++t) {
+                FETCH_TILE(TILE_KEY(t), pages[t])
+                PUT_TILE(t * BUF)
+            }
+            FETCH_TILE(TILE_KEY(RING - 1), pages[RING - 1])
+        }
     }
     // The rows of the MFMA's first operand are the tile's keys in an order in which the eight weights of a half tile that a
     // lane ends up with belong to eight neighbouring keys, 16 h + 8 g + 0 .. 7: row r is key r with its bits 2 and 3
@@ -411,6 +445,10 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
                 }
             }
         }
+        if constexpr (!DIRECT) {                           // (to the place of the tile before this one)
+            PUT_TILE(at == 0 ? (RING - 1) * BUF : at - BUF)
+            FETCH_TILE(kk_r, page)
+        }
 #pragma unroll
         for (int e = 0; e < 16; ++e) s[e] = 0.f;
 #pragma unroll
@@ -421,7 +459,7 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
             __builtin_amdgcn_sched_barrier(0);
         }
         MEET((RING - 3) * LT)
-        LOAD_TILE(kk_r, page, at)                          // the place was read for the last time before the last barrier
+        if constexpr (DIRECT) LOAD_TILE(kk_r, page, at)    // the place was read for the last time before the last barrier
         kk_r = TILE_KEY(i + RING + 1);
         page = PAGE_OF(kk_r);
         at = next;
@@ -430,6 +468,9 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
     }
     MEET(0)                                                // (what was asked for beyond the end arrives too, before the memory is used again)
 #undef LOAD_TILE
+#undef FETCH_TILE
+#undef PUT_TILE
+#undef TILE_HALF
 #undef PAGE_OF
 #undef MEET
 #undef TILE_KEY
@@ -695,26 +736,30 @@ int qe_attention_prefill(const void* q, void* out, const void* cache, const int*
     const float cap_in = softcap > 0.f ? scale * 2.f * 1.4426950408889634f / softcap : 0.f, cap_out = softcap * 1.4426950408889634f;
     if (groups == 0) groups = qe_attention_prefill_choose_groups((long)grid.x * grid.z, (long)num_tiles * R, window, max_keys);
     QE_REQUIRE(groups == 1 || groups == 2, "prefill attention: %d groups a block", groups);
-#define QE_PREFILL_CAP(D_, NG_, CAP_)                                                               \
+    // (a cache may begin at any element of a larger buffer)
+    const bool direct = ((unsigned long)cache & 15) == 0;
+#define QE_PREFILL_FORM(D_, NG_, CAP_, DIRECT_)                                                               \
     {                                                                                               \
         constexpr int shmem_ = NG_ * RING * 2 * 32 * D_ * 2;                                       \
         static unsigned long raised_ = 0;   /* (once per kernel and device: the limit of dynamic shared memory) */ \
         int device_ = 0;                                                                            \
         (void)hipGetDevice(&device_);                                                               \
         if (!(raised_ >> (device_ & 63) & 1)) {                                                     \
-            (void)hipFuncSetAttribute((const void*)attention_prefill_kernel<D_, NG_, CAP_>, hipFuncAttributeMaxDynamicSharedMemorySize, shmem_); \
+            (void)hipFuncSetAttribute((const void*)attention_prefill_kernel<D_, NG_, CAP_, DIRECT_>, hipFuncAttributeMaxDynamicSharedMemorySize, shmem_); \
             raised_ |= 1ul << (device_ & 63);                                                       \
         }                                                                                           \
-        attention_prefill_kernel<D_, NG_, CAP_><<<grid, 256 * NG_, shmem_, stream>>>(               \
+        attention_prefill_kernel<D_, NG_, CAP_, DIRECT_><<<grid, 256 * NG_, shmem_, stream>>>(               \
         (const bf16_t*)q, (bf16_t*)out, (const bf16_t*)cache, tiles, positions, tok_seq, block_table, \
         max_blocks, Hq, Hkv, P, log2P, scale_log2, window, R, seg_keys, keys_row, (float*)workspace, keep_first, sink, \
         cap_in, cap_out, tail);                                                                     \
     }
+#define QE_PREFILL_CAP(D_, NG_, CAP_) { if (direct) QE_PREFILL_FORM(D_, NG_, CAP_, true) else QE_PREFILL_FORM(D_, NG_, CAP_, false) }
 #define QE_PREFILL(D_, NG_) do { if (softcap > 0.f) QE_PREFILL_CAP(D_, NG_, true) else QE_PREFILL_CAP(D_, NG_, false) } while (0)
     if (D == 128) { if (groups == 2) QE_PREFILL(128, 2); else QE_PREFILL(128, 1); }
     else          { if (groups == 2) QE_PREFILL(64, 2); else QE_PREFILL(64, 1); }
 #undef QE_PREFILL
 #undef QE_PREFILL_CAP
+#undef QE_PREFILL_FORM
     if (seg_keys != 0) {
         if (D == 128)
             attention_prefill_merge_kernel<128><<<mgrid, 256, 0, stream>>>((const float*)workspace, (bf16_t*)out, tiles,

@@ -725,3 +725,27 @@ def test_float32_logits_sum_in_the_same_order(ops, N, K):
         assert ((got.cpu().double() - want[:M]).abs() <= bound[:M]).all(), M
     odd = torch.cat([w.new_zeros(1), w.reshape(-1)])[1:].view(N, K)
     assert odd.data_ptr() % 16 == 4 and torch.equal(ops.gemm(x[:2].contiguous(), odd, bias), every[:2])
+
+
+@pytest.mark.parametrize("D,softcap", [(128, 0.0), (64, 0.0), (128, 20.0), (64, 20.0)])
+@pytest.mark.parametrize("offset", [1, 4])
+def test_prefill_attention_of_a_cache_at_any_address(ops, D, softcap, offset):
+    """A cache that begins at no whole 16-byte piece: the bits of an aligned one, by one wave group a block and by two, with keys in
+    segments, with a window, with fewer tiles than shared memory takes and with more."""
+    from qwen_engine_amd.parts.attention import prefill_tiles
+    hq, hkv, P = 8, 2, 16
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    for n, before, window, segment in ((5, 0, 0, 0), (97, 31, 0, 0), (161, 100, 33, 0), (290, 7, 0, 0), (70, 1100, 0, 512)):
+        L = before + n
+        pages = -(-L // P)
+        cache = rand(pages, 2, hkv, P, D, seed=L, dtype=torch.bfloat16).to(DEV)
+        moved = torch.cat([cache.new_zeros(offset), cache.reshape(-1)])[offset:].view(cache.shape)
+        assert moved.is_contiguous() and moved.data_ptr() % 16 == 2 * offset
+        q = rand(n, hq, D, seed=L + 1, dtype=torch.bfloat16).to(DEV)
+        tiles = i32(prefill_tiles([(0, n)], ops.prefill_tile_rows(hq, hkv))).view(-1, 2)
+        order = torch.randperm(pages, generator=torch.Generator().manual_seed(L)).int()[None].to(DEV)
+        for groups in (1, 2):
+            got = [ops.attention(q, c, i32(list(range(before, L))), i32([0] * n), order, D ** -0.5, window=window, softcap=softcap,
+                                 other_tokens=i32(list(range(n))), other_tiles=tiles, prefill_groups=groups,
+                                 max_other_keys=L if segment else 0, prefill_segment_keys=segment) for c in (cache, moved)]
+            assert torch.isfinite(got[0].float()).all() and torch.equal(got[0], got[1]), (n, before, window, segment, groups)
