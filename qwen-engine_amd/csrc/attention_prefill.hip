@@ -263,10 +263,13 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
         const unsigned long base_ = (unsigned long)(cache + (long)(page_) * page_stride);           \
         const uint4_t rsrc_ = {(unsigned)base_, (unsigned)(base_ >> 32) & 0xffffu, there_ ? (unsigned)page_bytes : 0u, 0x00020000u}; \
         _Pragma("unroll") for (int i_ = 0; i_ < LP; ++i_) {                                         \
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"  \
-                         : : "s"(lds_k + (at_) + i_ * 1024), "v"(kconst[i_]), "s"(rsrc_), "s"(off_ * (D * 2)) : "memory"); \
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"  \
-                         : : "s"(lds_v + (at_) + i_ * 1024), "v"(vconst[i_]), "s"(rsrc_), "s"(off_ * 2) : "memory"); \
+            if constexpr (CAP && D == 64) {   /* (these forms keep more scalars than there are registers) */ \
+                QE_LOAD_TO_SHARED(lds_k + (at_) + i_ * 1024, kconst[i_], rsrc_, off_ * (D * 2), "4", ""); \
+                QE_LOAD_TO_SHARED(lds_v + (at_) + i_ * 1024, vconst[i_], rsrc_, off_ * 2, "4", "");  \
+            } else {                                                                                \
+                QE_LOAD_TO_SHARED(lds_k + (at_) + i_ * 1024, kconst[i_], rsrc_, off_ * (D * 2), "0", ""); \
+                QE_LOAD_TO_SHARED(lds_v + (at_) + i_ * 1024, vconst[i_], rsrc_, off_ * 2, "0", "");  \
+            }                                                                                       \
         }                                                                                           \
     }
     // (the two steps of it through registers)

@@ -217,4 +217,12 @@ extern "C" int qe_compute_units();
         if (e_ != hipSuccess) { qe_set_error("%s: %s", __func__, hipGetErrorString(e_)); return (int)e_; } \
     } while (0)
 
+// 64 pieces of 16 bytes, one a lane, from the buffer's bytes offset_ (a lane's) + soffset_ on to shared memory, side by side from byte to_ on.
+// Written as an instruction: the compiler would wait for every load in flight before it reads shared memory.  It does not look inside
+// either: m0 is an operand, so that it knows who sets it, and wait_ are the wait states (as s_nop counts them) between the write of an operand and the
+// load: 0 for m0; 4 where a vector instruction may just have written a scalar one, as the reload of a spilled register does.  hint_: "" or " nt".
+#define QE_LOAD_TO_SHARED(to_, offset_, rsrc_, soffset_, wait_, hint_)                                               \
+    asm volatile("s_nop " wait_ "\n\tbuffer_load_dwordx4 %1, %2, %3 offen" hint_ " lds"                              \
+                 : : "{m0}"(to_), "v"(offset_), "s"(rsrc_), "s"(soffset_) : "memory")
+
 static inline int qe_cdiv(long a, long b) { return (int)((a + b - 1) / b); }

@@ -189,8 +189,7 @@ __global__ __launch_bounds__(256, 5) void gemm_f32_lines_kernel(const float* __r
     auto ask = [&](int c) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
-                         : : "s"(to + (c & 1) * 4096 + i * 1024), "v"(off[i & 1]), "s"(rsrc), "s"((k_lo + c * CHUNK + (i >> 1) * 32) * 4) : "memory");
+            QE_LOAD_TO_SHARED(to + (c & 1) * 4096 + i * 1024, off[i & 1], rsrc, (k_lo + c * CHUNK + (i >> 1) * 32) * 4, "0", " nt");
     };
     ask(0);
     ask(1);

@@ -196,9 +196,7 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
         rsrc_b[c] = __builtin_amdgcn_readfirstlane(rsrc_b[c]);
     }
     const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) unsigned char*)smem + wave_s * 1024;
-#define LOAD_LDS(to_, vo_, rsrc_, soff_)                                                 \
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" \
-                 : : "s"(to_), "v"(vo_), "s"(rsrc_), "s"(soff_) : "memory");
+#define LOAD_LDS(to_, vo_, rsrc_, soff_) QE_LOAD_TO_SHARED(to_, vo_, rsrc_, soff_, "0", "");
     // waits until at most younger_ loads of the wave are in flight and its reads of shared memory are done, then for
     // the other waves
 #define MEET(younger_)                                                                   \
