@@ -291,15 +291,7 @@ int qe_attention_f32(const float* q, float* out, const float* cache, const int* 
 #define QE_ATTN_F32_RUN(DB_, NW_, AHEAD_)                                                             \
     do {                                                                                              \
         const size_t lds = (size_t)F32_SLOTS * (DB_ * 4 + 2) * 64 * sizeof(float);                    \
-        if (lds > 48 * 1024) {                                                                        \
-            static bool raised = false;                                                               \
-            if (!raised) {                                                                            \
-                hipError_t e_ = hipFuncSetAttribute((const void*)attention_f32_kernel<DB_, NW_, AHEAD_>, \
-                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
-                if (e_ != hipSuccess) { qe_set_error("attention (32-bit): %s", hipGetErrorString(e_)); return (int)e_; } \
-                raised = true;                                                                        \
-            }                                                                                         \
-        }                                                                                             \
+        if (lds > 48 * 1024) QE_RAISE_SHARED((attention_f32_kernel<DB_, NW_, AHEAD_>), lds);          \
         attention_f32_kernel<DB_, NW_, AHEAD_><<<grid, 64 * NW_, lds, stream>>>(q, out, cache, positions, tok_seq, \
                                                     block_table, max_blocks, tokens, Hq, Hkv, P, scale, window, keep_first, sink, softcap, tail); \
     } while (0)

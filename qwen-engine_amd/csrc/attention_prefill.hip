@@ -744,13 +744,7 @@ int qe_attention_prefill(const void* q, void* out, const void* cache, const int*
 #define QE_PREFILL_FORM(D_, NG_, CAP_, DIRECT_)                                                               \
     {                                                                                               \
         constexpr int shmem_ = NG_ * RING * 2 * 32 * D_ * 2;                                       \
-        static unsigned long raised_ = 0;   /* (once per kernel and device: the limit of dynamic shared memory) */ \
-        int device_ = 0;                                                                            \
-        (void)hipGetDevice(&device_);                                                               \
-        if (!(raised_ >> (device_ & 63) & 1)) {                                                     \
-            (void)hipFuncSetAttribute((const void*)attention_prefill_kernel<D_, NG_, CAP_, DIRECT_>, hipFuncAttributeMaxDynamicSharedMemorySize, shmem_); \
-            raised_ |= 1ul << (device_ & 63);                                                       \
-        }                                                                                           \
+        QE_RAISE_SHARED((attention_prefill_kernel<D_, NG_, CAP_, DIRECT_>), shmem_);                \
         attention_prefill_kernel<D_, NG_, CAP_, DIRECT_><<<grid, 256 * NG_, shmem_, stream>>>(               \
         (const bf16_t*)q, (bf16_t*)out, (const bf16_t*)cache, tiles, positions, tok_seq, block_table, \
         max_blocks, Hq, Hkv, P, log2P, scale_log2, window, R, seg_keys, keys_row, (float*)workspace, keep_first, sink, \

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "shared_limit.h"
+
 #define QE_WAVE 64
 
 // Element type codes used across the C ABI.
@@ -215,6 +217,17 @@ extern "C" int qe_compute_units();
     do {                                              \
         hipError_t e_ = hipGetLastError();            \
         if (e_ != hipSuccess) { qe_set_error("%s: %s", __func__, hipGetErrorString(e_)); return (int)e_; } \
+    } while (0)
+
+// Before a launch that needs more dynamic shared memory than every kernel may have; the same bytes at each launch of a kernel.
+#define QE_RAISE_SHARED(kernel_, bytes_)                                                          \
+    do {                                                                                          \
+        static std::atomic<unsigned long> raised_{0};                                             \
+        hipError_t e_ = qe_raise_shared_limit((const void*)(kernel_), bytes_, raised_);           \
+        if (e_ != hipSuccess) {                                                                   \
+            qe_set_error("%s: %zu bytes of shared memory: %s", __func__, (size_t)(bytes_), hipGetErrorString(e_)); \
+            return (int)e_;                                                                       \
+        }                                                                                         \
     } while (0)
 
 // 64 pieces of 16 bytes, one a lane, from the buffer's bytes offset_ (a lane's) + soffset_ on to shared memory, side by side from byte to_ on.

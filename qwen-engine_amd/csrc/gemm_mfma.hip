@@ -719,12 +719,7 @@ static int launch_mfma(const void* x, const void* w, const float* bias, void* ou
     const long blocks = (long)tiles_m * tiles_n;
     QE_REQUIRE(blocks <= 2147483647L, "mfma gemm: too many tiles");
     const size_t shmem = gemm_mfma_shared_bytes(BM, BN, RING, QKV);
-    static bool attr_set = false;   // one flag per instantiation
-    if (!attr_set) {
-        (void)hipFuncSetAttribute((const void*)gemm_mfma_kernel<TO, BM, BN, RING, NW, MINB, SILU, QKV, DIRECT>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
-        attr_set = true;
-    }
+    QE_RAISE_SHARED((gemm_mfma_kernel<TO, BM, BN, RING, NW, MINB, SILU, QKV, DIRECT>), shmem);
     // a cut of K is a multiple of 64 long (the last may be shorter)
     const int k_per_split = splits > 1 ? qe_cdiv(qe_cdiv(K, splits), 64) * 64 : K;
     QE_REQUIRE(splits >= 1 && splits <= 65535 && (long)(splits - 1) * k_per_split < K,
@@ -760,12 +755,7 @@ static int launch_grouped(const void* x, const void* w, void* out, const int* ti
     const long blocks = (long)max_tiles * tiles_n;
     QE_REQUIRE(blocks > 0 && blocks <= 2147483647L, "mfma gemm (grouped): too many tiles");
     const size_t shmem = gemm_mfma_shared_bytes(BM, BN, RING, false);
-    static bool attr_set = false;
-    if (!attr_set) {
-        (void)hipFuncSetAttribute((const void*)gemm_mfma_kernel<TO, BM, BN, RING, NW, MINB, SILU, false, DIRECT>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);
-        attr_set = true;
-    }
+    QE_RAISE_SHARED((gemm_mfma_kernel<TO, BM, BN, RING, NW, MINB, SILU, false, DIRECT>), shmem);
     QkvTail tail{};
     tail.tiles = tiles;
     tail.n_tiles = n_tiles;

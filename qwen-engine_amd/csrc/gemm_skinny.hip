@@ -538,15 +538,7 @@ static int launch_skinny(const void* x, const void* w, const float* bias, void* 
         auto kern = gemm_skinny_kernel<MT_, NT_, EPI, TO, WAVES_, NORM_, LN_, XH_>;                    \
         const size_t dyn = NORM_ ? norm_lds_bytes(M, K)                                                \
                                  : (LN_ ? (size_t)WAVES_ * ((SILU ? 2 : 1) * 2048 + ((XH_) ? 2 : 1) * 1024) : 0); \
-        if (dyn > 32 * 1024) {                                                                         \
-            static bool raised = false;   /* (once per kernel: the limit of dynamic shared memory) */ \
-            if (!raised) {                                                                             \
-                hipError_t e_ = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                                    QE_SKINNY_MAX_NORM_LDS);                           \
-                if (e_ != hipSuccess) { qe_set_error("skinny gemm: %s", hipGetErrorString(e_)); return (int)e_; } \
-                raised = true;                                                                         \
-            }                                                                                          \
-        }                                                                                              \
+        if (dyn > 32 * 1024) QE_RAISE_SHARED(kern, QE_SKINNY_MAX_NORM_LDS);                            \
         kern<<<grid, WAVES_ * 64, dyn, stream>>>(x, (const bf16_t*)w, bias, (TO*)out, M, N, K, cps, norm_w, norm_eps, \
                                                  delta, n_delta, h_out);                               \
     } while (0)

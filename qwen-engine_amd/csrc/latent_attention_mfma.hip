@@ -310,6 +310,11 @@ __global__ __launch_bounds__(256) void latent_attention_merge_kernel(const float
     if (d < R) Elem<bf16_t>::store(out + th * R + d, a / L);
 }
 
+// Bytes of shared memory for latents of 16 rb numbers and keys of 32 dkc.
+static size_t latent_shared_bytes(int rb, int dkc) {
+    return ((size_t)32 * (dkc * 32 + 8) + (size_t)rb * 16 * LAT_VT_PITCH) * sizeof(bf16_t);
+}
+
 static bool latent_mfma_fits(int R, int Dk, int& rbc, int& dkc) {
     if (R <= 0 || Dk < R || R % 8 || Dk % 8) return false;
     const int rb = (R + 15) / 16, dk = (Dk + 31) / 32;
@@ -373,19 +378,13 @@ extern "C" int qe_latent_attention_mfma(const void* qp, void* out, const void* c
     float* part_acc = (float*)workspace;
     float* part_ml = part_acc ? part_acc + (long)T * H * NS * RP : nullptr;
     const int dkc = (Dk + 31) / 32, rb = (R + 15) / 16;
-    const size_t shmem = ((size_t)32 * (dkc * 32 + 8) + (size_t)rb * 16 * LAT_VT_PITCH) * sizeof(bf16_t);
+    const size_t shmem = latent_shared_bytes(rb, dkc);
     dim3 grid(qe_cdiv(T, TOK), NS, qe_cdiv(HG, HGB));
 #define QE_LA(RB_, DKC_) do { if (HGB * TOK == 1) QE_LA2(RB_, DKC_, 4); else QE_LA2(RB_, DKC_, 1); } while (0)
 #define QE_LA2(RB_, DKC_, WS_)                                                                                        \
     do {                                                                                                              \
-        static size_t attr_bytes = 48 * 1024;          /* (what a kernel may take without asking) */                 \
-        if (shmem > attr_bytes) {                                                                                     \
-            hipError_t e_ = hipFuncSetAttribute((const void*)latent_attention_mfma_kernel<RB_, DKC_, WS_>,                 \
-                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)shmem);              \
-            QE_REQUIRE(e_ == hipSuccess, "latent_attention (mfma): %zu bytes of shared memory: %s", shmem,             \
-                       hipGetErrorString(e_));                                                                        \
-            attr_bytes = shmem;                                                                                       \
-        }                                                                                                             \
+        /* (the limit: what the largest sizes of the form need) */                                                    \
+        if (shmem > 48 * 1024) QE_RAISE_SHARED((latent_attention_mfma_kernel<RB_, DKC_, WS_>), latent_shared_bytes(RB_, DKC_));\
         latent_attention_mfma_kernel<RB_, DKC_, WS_><<<grid, 256, shmem, stream>>>(                                        \
             (const bf16_t*)qp, (bf16_t*)out, part_acc, part_ml, (const bf16_t*)cache, positions, tok_seq, block_table, \
             max_blocks, T, H, R, Dk, P, scale, TOK, HGB, NS, window, sink);                                                       \
