@@ -75,8 +75,9 @@ constexpr int gemm_mfma_shared_bytes(int BM, int BN, int RING, bool QKV) {
     return QKV && tile > ring ? tile : ring;
 }
 
-// DIRECT: x and w begin at a whole 16-byte piece.  Loads that write to shared memory themselves want that; operands that lie elsewhere are
-// copied by their elements, in one shape and at a fraction of the speed.
+// DIRECT: x and w begin at a whole 16-byte piece, which loads that write to shared memory themselves want.  Operands that lie elsewhere come
+// through registers, asked for a stage before they are stored; every shape is then a ring (both operands at an odd element: 8192 rows against gate
+// and up of 24576 x 4096 2051 us, 1238 aligned; 512 against 6144 x 1024 22, 11; copied by elements they took 12976 and 69).
 template <typename TO, int BM, int BN, int RING, int NW, int MINB, int SILU, bool QKV = false, bool DIRECT = true>
 __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
     const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const float* __restrict__ bias,
@@ -88,7 +89,7 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
     constexpr int LDA = BM / (8 * NW), LD = (BM + BN) / (8 * NW);   // a wave's loads of a stage: LDA of x, then of W
     static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0 && LD >= 2 && (RING - 2) * LD + (LD + 1) / 2 < 64 && RING >= 2,
                   "the rows of a stage must be whole loads of every wave, the loads in flight no more than can be counted");
-    constexpr bool BIG = BM == 256 && BN == 256 && NW == 4, TWO = BM == 128 && BN == 128 && RING == 2;
+    constexpr bool BIG = DIRECT && BM == 256 && BN == 256 && NW == 4, TWO = DIRECT && BM == 128 && BN == 128 && RING == 2;
     constexpr int STAGE = (BM + BN) * 128;   // bytes of a stage: the x rows, then the W rows
     [[maybe_unused]] constexpr int SMEM = gemm_mfma_shared_bytes(BM, BN, RING, QKV);
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -367,21 +368,29 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
 #pragma unroll
     for (int i = 0; i < LD; ++i)
         voff[i] = (((i < LDA ? i : i - LDA) * NW + wave) * 8 + (lane >> 3)) * K * 2 + pc * 16;
-    // the wave's i_-th load of stage st_, into the ring's place that begins at byte at_
-#define LOAD_PIECE(st_, at_, i_)                                                         \
+    // the wave's i_-th load of stage st_, into the ring's place that begins at byte at_; through registers: the piece that was asked for a
+    // stage ago goes there, and the next stage's is asked for
+    [[maybe_unused]] uint4_t held[LD];
+    [[maybe_unused]] const __amdgpu_buffer_rsrc_t piece_a = __builtin_amdgcn_make_buffer_rsrc((void*)a_addr, 0, rsrc_a[2], 0x00020000);
+    [[maybe_unused]] const __amdgpu_buffer_rsrc_t piece_b = __builtin_amdgcn_make_buffer_rsrc((void*)b_addr, 0, rsrc_b[2], 0x00020000);
+#define PLACE(at_, i_) ((at_) + ((i_) < LDA ? (i_) * NW * 1024 : BM * 128 + ((i_) - LDA) * NW * 1024))
+#define HOLD_PIECE(st_, i_)                                                              \
     {                                                                                    \
         const int kk = QE_KK(st_);                                                       \
         const int vo = kk * 64 + pc * 8 < klen ? voff[i_] : 0x7fffffff;                  \
-        const int soff = kk * 128;                                                       \
-        const unsigned place = (at_) + ((i_) < LDA ? (i_) * NW * 1024 : BM * 128 + ((i_) - LDA) * NW * 1024); \
+        held[i_] = __builtin_amdgcn_raw_buffer_load_b128((i_) < LDA ? piece_a : piece_b, vo, kk * 128, 0); \
+    }
+#define PUT_PIECE(at_, i_) *(uint4_t*)(smem + PLACE(at_, i_) + wave * 1024 + lane * 16) = held[i_];
+#define LOAD_PIECE(st_, at_, i_)                                                         \
+    {                                                                                    \
         if constexpr (!DIRECT) {                                                         \
-            const int row = (((i_) < LDA ? (i_) : (i_) - LDA) * NW + wave) * 8 + (lane >> 3); \
-            const bf16_t* const from = ((i_) < LDA ? x + (long)m0 * K : w + (long)n0 * K) + (long)row * K + k0 + kk * 64 + pc * 8; \
-            const bool there = row < ((i_) < LDA ? a_rows : b_rows) && kk * 64 + pc * 8 < klen; \
-            Piece16 piece;                                                               \
-            _Pragma("unroll") for (int e = 0; e < 8; ++e) piece.e[e] = there ? from[e].bits : (unsigned short)0; \
-            *(uint4_t*)(smem + place + wave * 1024 + lane * 16) = piece.q;               \
-        } else if ((i_) < LDA) LOAD_LDS(lds0 + place, vo, rsrc_a, soff) else LOAD_LDS(lds0 + place, vo, rsrc_b, soff) \
+            PUT_PIECE(at_, i_)                                                           \
+            HOLD_PIECE((st_) + 1, i_)                                                    \
+        } else {                                                                         \
+            const int kk = QE_KK(st_);                                                   \
+            const int vo = kk * 64 + pc * 8 < klen ? voff[i_] : 0x7fffffff;              \
+            if ((i_) < LDA) LOAD_LDS(lds0 + PLACE(at_, i_), vo, rsrc_a, kk * 128) else LOAD_LDS(lds0 + PLACE(at_, i_), vo, rsrc_b, kk * 128) \
+        }                                                                                \
     }
     const unsigned char *a_frag[4], *b_frag[4];
 #pragma unroll
@@ -414,6 +423,10 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
     // in registers); behind the barrier there it takes the stage RING later: half of that stage's loads go with
     // the last k step, half with the first of the next stage.
     constexpr int HALF = (LD + 1) / 2;
+    if constexpr (!DIRECT) {
+#pragma unroll
+        for (int i = 0; i < LD; ++i) HOLD_PIECE(0, i)
+    }
 #pragma unroll
     for (int st = 0; st < RING; ++st)
 #pragma unroll
@@ -435,6 +448,9 @@ __global__ __launch_bounds__(64 * NW, MINB) void gemm_mfma_kernel(
     }
 #undef K_STEP
 #undef LOAD_PIECE
+#undef HOLD_PIECE
+#undef PUT_PIECE
+#undef PLACE
 #undef READ_FRAG
     }
     MEET(0)                                                // (what was asked for beyond the end arrives too, before the memory is used again)
@@ -713,7 +729,8 @@ static int launch_mfma(const void* x, const void* w, const float* bias, void* ou
                        int n_cols, int splits, hipStream_t stream, const QkvTail& tail) {
     if constexpr (DIRECT) {
         if (((unsigned long)x | (unsigned long)w) & 15)
-            return launch_mfma<TO, 128, 128, 3, 4, 1, SILU, QKV, false>(x, w, bias, out, M, N, K, n_cols, splits, stream, tail);
+            return launch_mfma<TO, BM, BN, BM == 64 || BN < BM ? 3 : 2, NW, BM <= 128 ? 2 : 1, SILU, QKV, false>(x, w, bias, out, M, N, K, n_cols, splits,
+                                                                                                      stream, tail);
     }
     const int tiles_m = qe_cdiv(M, BM), tiles_n = qe_cdiv(n_cols, BN);
     const long blocks = (long)tiles_m * tiles_n;
@@ -746,7 +763,7 @@ template <typename TO, int SILU, bool DIRECT = true>
 static int launch_grouped(const void* x, const void* w, void* out, const int* tiles, const int* n_tiles,
                           int max_tiles, int N, int K, float limit, float slope, hipStream_t stream, int relu_sq = 0,
                           const float* row_w = nullptr, const int* perm = nullptr) {
-    constexpr int BM = 128, BN = 128, RING = DIRECT ? 2 : 3, NW = 4, MINB = DIRECT ? 2 : 1;
+    constexpr int BM = 128, BN = 128, RING = 2, NW = 4, MINB = 2;
     if constexpr (DIRECT) {
         if (((unsigned long)x | (unsigned long)w) & 15)
             return launch_grouped<TO, SILU, false>(x, w, out, tiles, n_tiles, max_tiles, N, K, limit, slope, stream, relu_sq, row_w, perm);

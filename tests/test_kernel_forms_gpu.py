@@ -651,21 +651,69 @@ def test_tiled_products_at_the_ends_of_their_stages(ops, K):
         for rows in (64, 65, 128, 256, 512):
             got = ops.gemm(x, w, out_dtype=torch.float32, algo=ops.ALGO_TILE + rows)
             assert ((got.cpu().double() - want).abs() <= bound).all(), (M, N, K, rows)
-        if K > 64:
-            parts = ops.gemm(x, w, epilogue=ops.EPI_PARTIAL, splits=2) if M > 64 else None
-            assert parts is None or ((parts.cpu().double().sum(0) - want).abs() <= bound).all(), (M, N, K)
+            if K > 64:
+                parts = ops.gemm(x, w, epilogue=ops.EPI_PARTIAL, splits=2, algo=ops.ALGO_TILE + rows)
+                assert ((parts.cpu().double().sum(0) - want).abs() <= bound).all(), (M, N, K, rows)
 
 
-def test_tiled_products_of_operands_at_any_address(ops):
-    """Operands that begin at an odd element: the bits of aligned ones, in a plain product, gate and up, and grouped rows."""
-    odd = lambda t: torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(t.shape)
-    M, N, K = 200, 192, 328
+def odd(t):
+    """The same numbers in a tensor that begins at an odd element."""
+    t = torch.cat([t.new_zeros(1), t.reshape(-1)])[1:].view(t.shape)
+    assert t.data_ptr() % 4 == 2
+    return t
+
+
+@pytest.mark.parametrize("M,N,K", [(200, 192, 328), (65, 64, 64), (255, 320, 72), (300, 256, 1160)])
+def test_tiled_products_of_operands_at_any_address(ops, M, N, K):
+    """Operands that begin at an odd element: the bits of aligned ones, in every tile shape, as a plain product, gate and up, gelu and in
+    cuts of K."""
     x, w = rand(M, K, seed=1, dtype=torch.bfloat16).to(DEV), rand(N, K, seed=2, dtype=torch.bfloat16).to(DEV)
-    ox, ow = odd(x), odd(w)
-    assert ox.data_ptr() % 4 == 2 and ow.data_ptr() % 4 == 2
-    for a, b in ((ox, w), (x, ow), (ox, ow)):
-        assert torch.equal(ops.gemm(a, b), ops.gemm(x, w))
-        assert torch.equal(ops.gemm(a, b, epilogue=ops.EPI_SILU_MUL_IL), ops.gemm(x, w, epilogue=ops.EPI_SILU_MUL_IL))
+    bias = rand(N, seed=3).to(DEV)
+    forms = [dict(), dict(out_dtype=torch.float32, bias=bias), dict(epilogue=ops.EPI_SILU_MUL_IL), dict(epilogue=ops.EPI_SILU_MUL_IL, bias=bias),
+             dict(epilogue=ops.EPI_GELU)] + ([dict(epilogue=ops.EPI_PARTIAL, splits=2)] if K > 64 else [])
+    for rows in (0, 64, 65, 128, 256, 512):
+        for form in forms:
+            run = lambda a, b: ops.gemm(a, b, algo=ops.ALGO_TILE + rows if rows else ops.ALGO_AUTO, **form)
+            want = run(x, w)
+            for a, b in ((odd(x), w), (x, odd(w)), (odd(x), odd(w))):
+                assert torch.equal(run(a, b), want), (rows, form)
+
+
+@pytest.mark.parametrize("M", [17, 40, 64])
+def test_few_rows_of_operands_at_any_address_against_a_large_matrix(ops, M):
+    """17 to 64 rows by the tiles: plain, gate and up (a matrix of few tile columns: a longer ring), in cuts of K."""
+    N, K = 4096, 4160
+    x, w = rand(M, K, seed=M, dtype=torch.bfloat16).to(DEV), rand(N, K, seed=2, dtype=torch.bfloat16).to(DEV)
+    assert ops.gemm_partial_preferred(x, w)
+    for form in (dict(), dict(epilogue=ops.EPI_SILU_MUL_IL), dict(epilogue=ops.EPI_PARTIAL, splits=5)):
+        assert torch.equal(ops.gemm(odd(x), odd(w), **form), ops.gemm(x, w, **form)), form
+
+
+@pytest.mark.parametrize("tile", [0, 64, 128, 256, 512])
+def test_query_key_value_products_of_operands_at_any_address(ops, tile):
+    M, K, hq, hkv, P = 150, 200, 4, 2, 16
+    x, w = rand(M, K, seed=1, dtype=torch.bfloat16).to(DEV), rand((hq + 2 * hkv) * 128, K, seed=2, dtype=torch.bfloat16).to(DEV)
+    norms = (1 + 0.1 * rand(2, 128, seed=3)).to(DEV)
+    table, pos = rand(M, 128, seed=4).to(DEV), torch.arange(M, dtype=torch.int32, device=DEV)
+    got = []
+    for a, b in ((x, w), (odd(x), odd(w))):
+        cache = torch.zeros(M // P + 1, 2, hkv, P, 128, dtype=torch.bfloat16, device=DEV)
+        got.append((ops.gemm_qkv(a, b, None, hq, cache, pos, norms[0].contiguous(), norms[1].contiguous(), 1e-6, table, pos, tile=tile), cache))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and got[0][1].any()
+
+
+@pytest.mark.parametrize("act", ["gated", "relu_sq"])
+def test_grouped_products_of_weights_at_any_address(ops, act):
+    """Enough pairs for the grouped rows' tiles."""
+    T, E, F, K, top = 300, 8, 96, 136, 4
+    x = rand(T, K, seed=1, dtype=torch.bfloat16).to(DEV)
+    w_in, w_out = rand(E, (2 if act == "gated" else 1) * F, K, seed=2, dtype=torch.bfloat16).to(DEV), rand(E, K, F, seed=3, dtype=torch.bfloat16).to(DEV)
+    ids = torch.stack([torch.randperm(E, generator=torch.Generator().manual_seed(t))[:top] for t in range(T)]).int().to(DEV)
+    weights = torch.rand(T, top, generator=torch.Generator().manual_seed(5)).to(DEV)
+    for rows in (torch.float32, torch.bfloat16):
+        got = [ops.moe_experts(x, ids, weights, a, b, act=act, interleaved=act == "gated", rows_dtype=rows) for a, b in
+               ((w_in, w_out), (odd(w_in), odd(w_out)))]
+        assert torch.equal(*got) and got[0].any()
 
 
 @pytest.mark.parametrize("K", [1016, 1024, 2048, 4096, 4160, 12288])
