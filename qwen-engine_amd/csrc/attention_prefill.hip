@@ -20,9 +20,8 @@
 //       one row of V^T, one 16-byte read
 // What bounds it: the vector units' 560 cycles and the matrix units' 512 of a wave's tile, which overlap only between the two waves of
 // a SIMD.  (With tiles through registers, a barrier behind every tile's arrival and the scores of a tile right before its weights:
-// 8192 tokens of 32 heads of 128 on 8, 626 us, now 573; 512 rows each behind 4096 keys, four requests, 197, now 166; 2048 tokens of
-// 16 heads 48.5, now 46; 512 rows behind 7680 keys 61, now 58.  The two groups of a block half a round apart, a barrier for each phase,
-// took 48 and 60.5 there.)
+// 8192 tokens of 32 heads of 128 on 8, 637 us, now 588; 512 rows each behind 4096 keys, four requests, 204, now 171; 2048 tokens of
+// 16 heads 49, now 44.7; 512 rows behind 7680 keys, with the merge of their segments, 62, now 56; 3000 tokens of 16 heads of 64 on 4 53, now 50.)
 // The causal and window limits are applied per column, so the order of the sums for a row
 // depends on its position and the window only.
 //
@@ -41,6 +40,8 @@
 // in the order of the segments.  The segment length comes from the host, or, where the host does not
 // know the positions (a recorded step), from the position of the row that sees the most keys.
 #include "common.h"
+
+#include <type_traits>
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
@@ -256,7 +257,7 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
 #define PAGE_OF(kk_) bt[min((kk_) + 16 * half, kmax - 1) >> log2P]
 #define TILE_HALF(kk_)                                                                              \
         const int key_ = (kk_) + 16 * half, off_ = key_ & pmask;                                    \
-        const bool there_ = key_ < kmax && (key_ + 16 > kmin || key_ < kfb);
+        const bool there_ = (key_ < kmax) & ((key_ + 16 > kmin) | (key_ < kfb));
 #define LOAD_TILE(kk_, page_, at_)                                                                  \
     {                                                                                               \
         TILE_HALF(kk_)                                                                              \
@@ -332,8 +333,10 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
         // and every round would end up waiting for the loads it has just issued.
         __builtin_amdgcn_s_waitcnt(0x0f70);                // vmcnt(0)
         if constexpr (DIRECT) {
+            if (rounds > 2) {                              // (else nobody reads them)
 #pragma unroll
-            for (int t = 2; t < RING; ++t) LOAD_TILE(TILE_KEY(t), pages[t], t * BUF)
+                for (int t = 2; t < RING; ++t) LOAD_TILE(TILE_KEY(t), pages[t], t * BUF)
+            }
         } else {
 #pragma unroll
             for (int t = 0; t < RING - 1; ++t) {
@@ -358,10 +361,11 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
 #define READ_KEYS(at_)                                                                              \
     _Pragma("unroll") for (int ks = 0; ks < D / 16; ++ks) kf[ks] = *(const bf16x8*)(k_frag + (at_) + (((ks * 2 + g) ^ kx) * 16));
     // A round: the weights of tile i from its scores, on the vector units, while the fragments of its values and of
-    // the next tile's keys come from shared memory; then the products of the weights and the values, and the scores of tile i + 1, in
-    // turn on the matrix units (an MFMA that adds to the one before it waits for it).  So nothing waits for shared memory, one
-    // barrier a round is enough, and two blocks on a unit fill each other's phases.  Tiles the wave sees nothing of are multiplied like the
-    // others, as zeros: with branches around the MFMAs the accumulators are copied.
+    // the next tile's keys come from shared memory; then the products of the weights and the values; and behind the barrier the scores of
+    // tile i + 1, under which the loads of tile i + RING and their addresses pass.  So nothing waits for shared memory, one
+    // barrier a round is enough, and two blocks on a unit fill each other's phases.  (Products and scores in turn before the barrier, the
+    // loads alone behind it: 2048 tokens of 16 heads 43.2 us, 40.0; 512 rows behind 7680 keys 51.1, 48.9.)  Tiles the wave sees nothing of are
+    // multiplied like the others, as zeros: with branches around the MFMAs the accumulators are copied.
     constexpr int LT = 2 * LP;                             // loads of a wave for a tile
     int at = 0, kk = TILE_KEY(0);
     bool seen = SEEN(kk);
@@ -369,12 +373,15 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
     READ_KEYS(0)
 #pragma unroll
     for (int ks = 0; ks < D / 16; ++ks) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ks], qreg[ks], s, 0, 0, 0);
-    for (int i = 0; i < rounds; ++i) {
+    // The last round (LAST) reads nothing ahead: a walk of one tile or a few would pay for scores that nobody wants and for loads that are only
+    // waited for (8 rows of 16 heads 7.5 us with the same round to the end, 6.8; 300 behind a window of 64 11.5, 10.9).
+    const auto round = [&](int i, auto last) {
+        constexpr bool LAST = decltype(last)::value;
         const int next = at + BUF == RING * BUF ? 0 : at + BUF;
         const int kk_1 = TILE_KEY(i + 1);
         const bool seen_1 = SEEN(kk_1);
         PackV pb[2];
-        READ_KEYS(next)
+        if constexpr (!LAST) { READ_KEYS(next) }
         if (!seen) {                                       // (a tile that the wave sees nothing of adds nothing; without a branch around the MFMAs)
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
@@ -448,27 +455,30 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
                 }
             }
         }
-        if constexpr (!DIRECT) {                           // (to the place of the tile before this one)
+        if constexpr (!DIRECT && !LAST) {                  // (to the place of the tile before this one)
             PUT_TILE(at == 0 ? (RING - 1) * BUF : at - BUF)
             FETCH_TILE(kk_r, page)
         }
 #pragma unroll
-        for (int e = 0; e < 16; ++e) s[e] = 0.f;
-#pragma unroll
-        for (int u = 0; u < D / 16; ++u) {
-            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[u], qreg[u], s, 0, 0, 0);
+        for (int u = 0; u < D / 16; ++u)
             acc[u % (D / 32)] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[u % (D / 32)][u / (D / 32)].v, pb[u / (D / 32)].v,
                                                                         acc[u % (D / 32)], 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
+        if constexpr (!LAST) {
+            MEET((RING - 3) * LT)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) s[e] = 0.f;
+            if constexpr (DIRECT) LOAD_TILE(kk_r, page, at)    // the place was read for the last time before the last barrier
+#pragma unroll
+            for (int ks = 0; ks < D / 16; ++ks) s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[ks], qreg[ks], s, 0, 0, 0);
+            kk_r = TILE_KEY(i + RING + 1);
+            page = PAGE_OF(kk_r);
+            at = next;
+            kk = kk_1;
+            seen = seen_1;
         }
-        MEET((RING - 3) * LT)
-        if constexpr (DIRECT) LOAD_TILE(kk_r, page, at)    // the place was read for the last time before the last barrier
-        kk_r = TILE_KEY(i + RING + 1);
-        page = PAGE_OF(kk_r);
-        at = next;
-        kk = kk_1;
-        seen = seen_1;
-    }
+    };
+    for (int i = 0; i + 1 < rounds; ++i) round(i, std::false_type());
+    round(rounds - 1, std::true_type());
     MEET(0)                                                // (what was asked for beyond the end arrives too, before the memory is used again)
 #undef LOAD_TILE
 #undef FETCH_TILE

@@ -735,7 +735,7 @@ def test_prefill_attention_over_few_and_many_tiles(ops, D, P, groups):
     from qwen_engine_amd.parts.attention import prefill_tiles
     hq, hkv = 4, 2
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
-    for n, before, window in ((1, 0, 0), (15, 0, 0), (33, 0, 0), (64, 0, 0), (97, 31, 0), (128, 0, 0), (129, 16, 0), (160, 0, 40),
+    for n, before, window in ((1, 0, 0), (15, 0, 0), (33, 0, 0), (64, 0, 0), (90, 0, 0), (97, 31, 0), (128, 0, 0), (129, 16, 0), (160, 0, 40),
                               (161, 100, 33), (290, 7, 0), (300, 0, 128)):
         L = before + n
         k, v, q = (rand(L, h, D, seed=s + L, dtype=torch.bfloat16) for s, h in ((1, hkv), (2, hkv), (3, hq)))
@@ -759,7 +759,7 @@ def test_prefill_attention_over_few_and_many_tiles(ops, D, P, groups):
             assert ((got[:, h] - want).abs() <= 2.0 ** -8 * (size + want.abs()) + 1e-6).all(), (n, before, window, h)
 
 
-@pytest.mark.parametrize("N,K", [(16384, 544), (16390, 992), (20001, 1024)])
+@pytest.mark.parametrize("N,K", [(16384, 544), (16384, 640), (16386, 672), (16390, 992), (20001, 1024)])
 def test_float32_logits_sum_in_the_same_order(ops, N, K):
     """Few rows against a matrix of very many (its last block of 16 outputs whole and not, K whole quarters and not): the bits
     that the tiles give a row among many, and those of operands at an odd address."""
