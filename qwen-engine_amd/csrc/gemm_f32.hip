@@ -15,7 +15,7 @@
 //   few rows: a block owns 16 outputs (or 32) and has a wave per chunk (16 from K = 1024 on), so that the weights are asked for
 //     by all its waves at once and the sums meet in shared memory.  Bound by the stream of the weights and
 //     a kernel's fixed cost.  Two rows (as 64 x 64 tiles before): 4096 x 1024 7.1 us (42), 6144 x 1024 10.6 (42),
-//     1024 x 3072 11.6 (117), 151936 x 1024 137 (215).  At most 64 registers a lane, so that two
+//     1024 x 3072 11.6 (117), weights of 151936 x 1024 that begin at no whole 16-byte piece 137 (215).  At most 64 registers a lane, so that two
 //     blocks of 16 waves fit a compute unit (four steps at a time instead of two: 10.0, 17.7, 14.5 and 294 us).
 //   more rows: tiles of 64 x 64, a wave a 32 x 32 quarter, K in steps of 16 through two buffers of shared
 //     memory.  With fewer than TILES_FOR_FOUR tiles and a K that gives each something four groups of four
@@ -164,7 +164,7 @@ __global__ __launch_bounds__(64 * CHUNKS) void gemm_f32_rows_kernel(const float*
 // bytes, 8 lanes a row, straight to shared memory, two chunks of a wave on their way; the row's pieces are exchanged there (piece p of row r at
 // place p ^ (r / 2 % 8)) so that the reads in the operands' layout fall into distinct banks.  Five such blocks share a unit, and the
 // end of one is hidden by the others (two rows against 151936 x 1024: 135 us with sixteen waves a block, now 100; one block's lines of all
-// sixteen chunks at once, two blocks a unit, took 128; 32768 x 1024 32.0, now 25.0; 16400 x 512 10.9, now 10.5; 20000 x 96 4.7 and 6.9).
+// sixteen chunks at once, two blocks a unit, took 128; 32768 x 1024 32.0, now 25.0).
 __global__ __launch_bounds__(256, 5) void gemm_f32_lines_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                 const float* __restrict__ bias, float* __restrict__ out,
                                                                 int M, int N, int K) {
@@ -356,10 +356,11 @@ int qe_gemm_f32(const float* x, const float* w, const float* bias, float* out, i
     const long tiles = (long)qe_cdiv(N, FT) * qe_cdiv(M, FT);
     if (M <= 16 || ((K > 64 || M <= 32) && ((M <= 64 && N < 16384) || tiles <= 128))) {
         // 32 outputs a block halve the reads of x; they pay where the rows are some and the blocks enough (16 rows,
-        // 6144 x 1024: 12.0 us against 14.3, 151936 x 1024: 183 against 213; 2 rows: 10.3 against 10.6, 148 against 137;
-        // 16 rows, 4096 x 1024: 11.5 against 9.5)
-        // (the logits; with fewer chunks than eight a wave's walk is not worth a block)
-        if (M <= 16 && N >= 16384 && K > 512 && K <= 4 * FK * CHUNKS && K % 32 == 0 && (((unsigned long)w) & 15) == 0)
+        // 6144 x 1024: 12.0 us against 14.3; 2 rows: 10.3 against 10.6; 16 rows, 4096 x 1024: 11.5 against 9.5)
+        // Whole lines for the logits, with ten chunks of K or more (1 to 16 rows, by rows and by lines: 16384 x 544 11.6 to 13.0 us and 11.0 to
+        // 13.2, 20001 x 576 13.5 to 18.4 and 15.7 to 16.4, 20001 x 640 15.7 to 21.5 and 15.9 to 17.2, 151936 x 640 84 to 124 and 78 to 104) and
+        // up to sixteen: chunks are longer than a wave's 64 beyond
+        if (M <= 16 && N >= 16384 && K >= 640 && K <= 4 * FK * CHUNKS && K % 32 == 0 && (((unsigned long)w) & 15) == 0)
             gemm_f32_lines_kernel<<<qe_cdiv(N, 16), 64 * qe_cdiv(K, 16 * FK), 0, stream>>>(x, w, bias, out, M, N, K);
         else if (M > 4 && M <= 16 && N >= 6144) launch_rows<1, 2, 1>(x, w, bias, out, M, N, K, rows, stream);
         else if (M <= 16) launch_rows<1, 1, 2>(x, w, bias, out, M, N, K, rows, stream);
