@@ -11,6 +11,7 @@ bool qe_gemm_skinny_norm_ok(int M, int N, int K);
 int qe_gemm_skinny_splits(int N, int K);
 bool qe_gemm_mfma_ok(int M, int N, int K, int dt_a, int dt_w);
 float qe_gemm_mfma_shape(int M, int N, int K, int splits, int* tile, bool largest = true);
+float qe_gemm_mfma_uncut(int M, int N, int K);
 int qe_gemm_mfma(const void* x, const void* w, const float* bias, void* out, int M, int N, int K, int dt_o,
                  int tile, bool silu, int splits, hipStream_t stream, bool gelu = false);
 
@@ -94,8 +95,11 @@ extern "C" int qe_gemm_partial_splits(int M, int N, int K) {
 // cuts that leaves 512 of K to a part; the cuts give every compute unit as many tiles as the others (800 rows against 5120 x 25600: 200 us in three
 // cuts of 256 x 256, 303 at the best without one; 528 against 4096 x 12288 72 in three of 128 x 128, 107).  Parts beyond 2^27 numbers (512 MiB, what a pool of pages that takes
 // nearly all memory should leave a step) are not asked for.  A plain product's numbers are rounded to 16 bits on their way to the norm,
-// which only many rows against a K that needs no cut pay for (those bytes are then a twentieth of the time); elsewhere a product that
-// is quickest without a cut is one 32-bit part.
+// which saves it 2 bytes a number, some 200 / K of the product's time (a fifth at K = 1024, a twentieth at 4096): so are products of a K up to
+// 4096 with more tiles of 128 x 128 than units, of a longer K whose tiles of 256 x 256 fill their turns to nine tenths, of more than 2^26
+// numbers, and of a K below 1024.  Elsewhere a product that is quickest without a cut is one 32-bit part, which may go in two launches
+// (qe_gemm_mfma_uncut; taken for one, 3300 rows against 5120 x 8192 were cut in two: 337 us with the norm, 295 as one part; 8192 rows 689 and 620,
+// 4600 against 4096 x 12288 484 and 457).
 extern "C" int qe_gemm_branch_splits(int M, int N, int K, int dt_a, int dt_w) {
     if (qe_gemm_skinny_ok(M, N, K, dt_a, dt_w) || (M <= 64 && tiled_for_few_rows(M, N, K, dt_a, dt_w))) {
         const int s = qe_gemm_partial_splits(M, N, K);
@@ -113,7 +117,7 @@ extern "C" int qe_gemm_branch_splits(int M, int N, int K, int dt_a, int dt_w) {
         if (s > 1 && (K < 512 * s || (long)s * M * N > (1L << 27))) break;
         if ((long)(s - 1) * (qe_cdiv(qe_cdiv(K, s), 64) * 64) >= K) continue;   // every cut has some of K
         int tile;
-        const float t = qe_gemm_mfma_shape(M, N, K, s, &tile) + (s == 1 && plain ? 2.f : 4.f * (float)s) * (float)M * (float)N / 6e6f;
+        const float t = (s == 1 && !plain ? qe_gemm_mfma_uncut(M, N, K) : qe_gemm_mfma_shape(M, N, K, s, &tile)) + (s == 1 && plain ? 2.f : 4.f * (float)s) * (float)M * (float)N / 6e6f;
         if (s == 1 || t < best) { best_s = s; best = t; }
     }
     return best_s > 1 || !plain ? best_s : 0;

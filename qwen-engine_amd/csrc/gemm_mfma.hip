@@ -850,11 +850,12 @@ static int choose_tile(int M, int N, int K, int splits, bool largest = true) {
 }
 
 // Where the last turn of a product's tiles would leave most units idle, the columns that fill the turns before it go first, and the
-// rest in a launch and a shape of its own: the number of the first columns, a multiple of 256, or 0.  Three microseconds for the
-// second launch; less than 3 % is not worth it.  (With the rates that the shapes had when loads went through registers: 1972 rows against gate and up of 51200 x 5120, 1600 tiles of 256 x 256: 923 us,
-// now 884; 656 rows 434, now 342;
-// 1300 rows against 24576 x 4096 299, now 269; q, k and v of 10240 x 5120 with 1600 rows 254, now 193.)
-static int first_columns(int M, int N, int K, bool largest = true) {
+// rest in a launch and a shape of its own: the number of the first columns, a multiple of 256, or 0; and what all that is taken to need.  Three
+// microseconds for the second launch; less than 3 % is not worth it (4 to 8 us and 3 to 10 % were tried and leave more behind).  Of 639 products
+// of 65 to 8192 rows 61 go in two, 57 of them faster than in one, a tenth in the mean: 4628 rows against 4096 x 1024 55.1 us, in two 47.3; 2048 against
+// 10240 x 5120 225, 187; 1024 against 24576 x 4096 187, 174; 3300 against 5120 x 25600 in one part 1047, 806.  The four others are misjudged: 2600 rows
+// against 6144 x 1024 37.5, 44.8, against 6144 x 4096 131, 139; 300 against 24576 x 4096 89, 100, against 51200 x 5120 224, 240.
+static int first_columns(int M, int N, int K, bool largest = true, float* time = nullptr) {
     int tile;
     const float whole = qe_gemm_mfma_shape(M, N, K, 1, &tile, largest);
     float best = 0.97f * whole;
@@ -867,7 +868,15 @@ static int first_columns(int M, int N, int K, bool largest = true) {
         const float t = qe_gemm_mfma_shape(M, (int)n1, K, 1, &tile, largest) + qe_gemm_mfma_shape(M, N - (int)n1, K, 1, &tile, largest) + 3.f;
         if (t < best) { best = t; cut = (int)n1; }
     }
+    if (time) *time = cut ? best : whole;
     return cut;
+}
+
+// The microseconds that a product without a cut of K is taken to need, in one launch or in two.
+float qe_gemm_mfma_uncut(int M, int N, int K) {
+    float time;
+    first_columns(M, N, K, true, &time);
+    return time;
 }
 
 // The same for a caller that wants to know: the number of columns that a product of more than 64 rows gives a launch of their own, or 0

@@ -727,6 +727,16 @@ def test_products_whose_parts_are_rounded_are_large(ops, K):
             assert (splits == 0) == (K < 1024) or (splits == 0 and tiles > 256), (M, N, K, splits)
 
 
+@pytest.mark.parametrize("M,N,K", [(3300, 5120, 8192), (4600, 4096, 12288), (8192, 5120, 8192)])
+def test_products_that_go_in_two_launches_are_not_cut(ops, M, N, K):
+    """A branch's product whose last turn of tiles gets a launch of its own is quicker as one 32-bit part than in cuts of K; the same
+    bits as in one launch."""
+    x, w = rand(M, K, seed=1, dtype=torch.bfloat16).to(DEV), rand(N, K, seed=2, dtype=torch.bfloat16).to(DEV)
+    assert ops.gemm_first_columns(M, N, K) > 0 and ops.gemm_branch_splits(x, w) == 1
+    parts = ops.gemm(x, w, epilogue=ops.EPI_PARTIAL, splits=1)
+    assert torch.equal(parts, ops.gemm(x, w, epilogue=ops.EPI_PARTIAL, splits=1, algo=ops.ALGO_TILE + 128))
+
+
 @pytest.mark.parametrize("D,P", [(128, 16), (128, 64), (64, 16), (64, 32)])
 @pytest.mark.parametrize("groups", [1, 2])
 def test_prefill_attention_over_few_and_many_tiles(ops, D, P, groups):
