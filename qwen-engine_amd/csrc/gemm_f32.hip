@@ -357,10 +357,11 @@ int qe_gemm_f32(const float* x, const float* w, const float* bias, float* out, i
     if (M <= 16 || ((K > 64 || M <= 32) && ((M <= 64 && N < 16384) || tiles <= 128))) {
         // 32 outputs a block halve the reads of x; they pay where the rows are some and the blocks enough (16 rows,
         // 6144 x 1024: 12.0 us against 14.3; 2 rows: 10.3 against 10.6; 16 rows, 4096 x 1024: 11.5 against 9.5)
-        // Whole lines for the logits, with ten chunks of K or more (1 to 16 rows, by rows and by lines: 16384 x 544 11.6 to 13.0 us and 11.0 to
-        // 13.2, 20001 x 576 13.5 to 18.4 and 15.7 to 16.4, 20001 x 640 15.7 to 21.5 and 15.9 to 17.2, 151936 x 640 84 to 124 and 78 to 104) and
-        // up to sixteen: chunks are longer than a wave's 64 beyond
-        if (M <= 16 && N >= 16384 && K >= 640 && K <= 4 * FK * CHUNKS && K % 32 == 0 && (((unsigned long)w) & 15) == 0)
+        // Whole lines for the logits, with more than eight chunks of K and up to sixteen (chunks are longer than a wave's 64 beyond).  Up to two rows
+        // and nine chunks, a matrix of fewer than 30000 rows goes by a wave a chunk (one row, by rows and by lines: 18000 x 544 12.7 us and
+        // 14.5, 20001 x 576 13.5 and 15.6, 18000 x 608 13.9 and 14.8, 20001 x 608 15.5 and 15.7, 32768 x 544 20.6 and 19.1; eight rows: 20001 x 576 16.8 and
+        // 15.9, 32768 x 608 26.6 and 21.0; with eight chunks or fewer a wave's walk is not worth a block: 20000 x 96 4.7 and 6.9)
+        if (M <= 16 && N >= 16384 && (K >= 608 || (K > 512 && (M > 2 || N >= 30000))) && K <= 4 * FK * CHUNKS && K % 32 == 0 && (((unsigned long)w) & 15) == 0)
             gemm_f32_lines_kernel<<<qe_cdiv(N, 16), 64 * qe_cdiv(K, 16 * FK), 0, stream>>>(x, w, bias, out, M, N, K);
         else if (M > 4 && M <= 16 && N >= 6144) launch_rows<1, 2, 1>(x, w, bias, out, M, N, K, rows, stream);
         else if (M <= 16) launch_rows<1, 1, 2>(x, w, bias, out, M, N, K, rows, stream);
