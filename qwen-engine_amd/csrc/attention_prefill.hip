@@ -48,16 +48,6 @@ typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 typedef __attribute__((ext_vector_type(16))) float floatx16;
 typedef __attribute__((ext_vector_type(4))) unsigned int uint4_t;
 
-union PackV {   // an MFMA operand, also addressable as two 8-byte pieces
-    bf16x8 v;
-    uint2 u[2];
-};
-union Piece {   // a staged 16-byte piece, addressable by element for masking
-    uint4_t q;
-    uint2 u[2];
-    unsigned short e[8];
-};
-
 // Lane i and lane i ^ 32 exchange a value without a trip through shared memory.
 __device__ __forceinline__ float max_of_both_halves(float v) {
     float a, b;
@@ -354,7 +344,7 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
     const int kx = D == 128 ? (kr & 15) : ((kr >> 1) & 7);
     const unsigned char* const v_frag = smem + KBYTES + r * 32 + ((g ^ ((r >> 3) & 1)) * 16);
     bf16x8 kf[D / 16];
-    PackV vf[D / 32][2];
+    bf16x8 vf[D / 32][2];
     floatx16 s;
 #pragma unroll
     for (int e = 0; e < 16; ++e) s[e] = 0.f;
@@ -380,20 +370,20 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
         const int next = at + BUF == RING * BUF ? 0 : at + BUF;
         const int kk_1 = TILE_KEY(i + 1);
         const bool seen_1 = SEEN(kk_1);
-        PackV pb[2];
+        bf16x8 pb[2];
         if constexpr (!LAST) { READ_KEYS(next) }
         if (!seen) {                                       // (a tile that the wave sees nothing of adds nothing; without a branch around the MFMAs)
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
-                pb[h].v = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+                pb[h] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-                for (int db = 0; db < D / 32; ++db) vf[db][h].v = pb[h].v;
+                for (int db = 0; db < D / 32; ++db) vf[db][h] = pb[h];
             }
         } else {
 #pragma unroll
             for (int db = 0; db < D / 32; ++db)
 #pragma unroll
-                for (int h = 0; h < 2; ++h) vf[db][h].v = *(const bf16x8*)(v_frag + at + (h * D + db * 32) * 32);
+                for (int h = 0; h < 2; ++h) vf[db][h] = *(const bf16x8*)(v_frag + at + (h * D + db * 32) * 32);
             __builtin_amdgcn_sched_barrier(0);
             if (CAP) {
 #pragma unroll
@@ -432,7 +422,7 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
             for (int e = 0; e < 16; ++e) {
                 const float pe = __builtin_amdgcn_exp2f(__builtin_fmaf(s[e], scale_log2, -ref));   // 0 for keys that are not seen
                 psum += pe;
-                pb[e >> 3].v[e & 7] = (__bf16)pe;
+                pb[e >> 3][e & 7] = (__bf16)pe;
             }
             l += psum;
             if (kk < kmin || kk + 32 > kmax) {
@@ -447,10 +437,10 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
                     }
 #pragma unroll
                     for (int db = 0; db < D / 32; ++db) {
-                        Piece pv = __builtin_bit_cast(Piece, vf[db][h]);
+                        uint4_t pv = __builtin_bit_cast(uint4_t, vf[db][h]);
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) pv.q[e] &= keep[e];
-                        vf[db][h] = __builtin_bit_cast(PackV, pv);
+                        for (int e = 0; e < 4; ++e) pv[e] &= keep[e];
+                        vf[db][h] = __builtin_bit_cast(bf16x8, pv);
                     }
                 }
             }
@@ -461,7 +451,7 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
         }
 #pragma unroll
         for (int u = 0; u < D / 16; ++u)
-            acc[u % (D / 32)] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[u % (D / 32)][u / (D / 32)].v, pb[u / (D / 32)].v,
+            acc[u % (D / 32)] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[u % (D / 32)][u / (D / 32)], pb[u / (D / 32)],
                                                                         acc[u % (D / 32)], 0, 0, 0);
         if constexpr (!LAST) {
             MEET((RING - 3) * LT)

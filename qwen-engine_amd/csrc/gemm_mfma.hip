@@ -820,8 +820,9 @@ float qe_gemm_mfma_shape(int M, int N, int K, int splits, int* tile, bool larges
     // them, the last runs alone and takes longer.  A chip with idle
     // units runs the others faster (two and a half times, were nearly all idle).  A shape is never taller than the rows need.
     // Against the best of all shapes (and, for a branch's last product, cuts) in products of 1024 to 51200 by 1024 to
-    // 25600 with 80 to 3300 rows, 2900 measured one by one on rows that are in no L2 and weights that are in no cache, what this picks is
-    // 0.3 % slower in the mean (of a branch's product with what its norm reads 0.6 %), 12 % at the most (3300 rows against 6144 x 1024).
+    // 25600 with 80 to 3300 rows, 2900 measured one by one on rows that are in no L2 and weights that are in no cache, what this picks was
+    // 0.3 % slower in the mean; in 639 others with 65 to 8192 rows, back to back and a branch's with its norm, 1.5 %, and a quarter at the most
+    // (3300 to 4700 rows against a K of 1024, which mostly go in two launches: first_columns).
     const long cus = 256;
     struct Shape { int tile, bm, bn; float rate, alone_first, alone_later; };
     const Shape shapes[4] = {{64, 64, 128, 0.78f, 0.f, 0.15f}, {128, 128, 128, 1.07f, 0.05f, 0.41f},
@@ -900,8 +901,8 @@ static int pick_mfma(const void* x, const void* w, const float* bias, void* out,
     tail.n_first = n_first;
     // Up to 64 rows against a gate|up matrix of at most one tile column a compute unit (its K cannot be
     // cut): a block streams its weights alone on its unit, and what it has in flight bounds it.  A ring of six stages
-    // doubles that (24576 x 4096 against 64 rows: 37.8 us; through registers 49.2, with k steps of 128 40.2; with two blocks a unit, 51200 x
-    // 5120, a longer ring gains nothing).
+    // doubles that (24576 x 4096 against 64 rows, its weights in no cache: 38.8 us, 39.6 with three stages, 43.8 through registers with k steps of 128; as a
+    // part of a step of 64 requests 44.7, and 45.9 through registers; with two blocks a unit, 51200 x 5120, a longer ring gains nothing).
     if (tile == 0 && SILU > 0 && M <= 64 && qe_cdiv(N, 128) <= 256) tile = 65;
     // (the gelu of 65536 values is 35 us in which nothing else runs on the unit: 256 x 256 is never its shape; 3000 rows against
     // 4096 x 1024: 65 us in it, 52 in 256 x 128, 47 in 128 x 128)
