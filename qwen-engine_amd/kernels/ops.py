@@ -138,6 +138,10 @@ def load_library():
         "qe_moe_tile_rows": [],
         "qe_moe_gemm_mfma_supported": [i32],
         "qe_moe_gemm_mfma": [vp, vp, i32, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, f32, f32, i32, i32, vp],
+        "qe_decode_chain_supported": [i32, i32, i32, i32, i32, i32, i32],
+        "qe_decode_chain_preferred": [i32, i32, i32, i32, i32, i32, i32],
+        "qe_decode_chain_layers": [],
+        "qe_decode_chain": [vp, vp, vp, i32, vp, vp, vp, i32, vp, vp, vp, f32, f32, i32, i32, i32, i32, i32, i32, i32, i32, vp, i64, vp],
     }
     for name, args in sigs.items():
         fn = getattr(lib, name)
@@ -157,6 +161,8 @@ def load_library():
     lib.qe_latent_attention_mfma_workspace_bytes.argtypes = [i32, i32, i32, i32]
     lib.qe_latent_attention_mfma_workspace_bytes.restype = ctypes.c_long
     lib.qe_attention_prefill_workspace_bytes_for.restype = ctypes.c_long
+    lib.qe_decode_chain_workspace_bytes.argtypes = [i32, i32, i32, i32, i32, i32, i32]
+    lib.qe_decode_chain_workspace_bytes.restype = ctypes.c_long
     _lib = lib
     return lib
 
@@ -1027,6 +1033,68 @@ def attention_decode_fused(qkv: torch.Tensor, num_heads: int, cache: torch.Tenso
                                              int(max_dec_position), DECODE_SPLIT_KEYS, ws.data_ptr(), nbytes,
                                              _stream()), "attention (decode, fused)")
     return out
+
+
+def decode_chain_supported(rows: int, hidden: int, num_heads: int, num_kv_heads: int, head_dim: int, intermediate: int, page_size: int) -> bool:
+    """True if decode_chain takes layers of these sizes for so many rows."""
+    return bool(load_library().qe_decode_chain_supported(rows, hidden, num_heads, num_kv_heads, head_dim, intermediate, page_size))
+
+
+def decode_chain_preferred(rows: int, hidden: int, num_heads: int, num_kv_heads: int, head_dim: int, intermediate: int, page_size: int) -> bool:
+    """True if decode_chain takes such layers and is quicker than their kernels one after the other."""
+    return bool(load_library().qe_decode_chain_preferred(rows, hidden, num_heads, num_kv_heads, head_dim, intermediate, page_size))
+
+
+def decode_chain(h: torch.Tensor, layers, positions: torch.Tensor, tok_seq: torch.Tensor, block_table: torch.Tensor,
+                 slots: Optional[torch.Tensor], num_heads: int, scale: float, max_position: int, qk_eps: float = 0.0,
+                 table: Optional[torch.Tensor] = None, shared_keys: Optional[torch.Tensor] = None, units: int = 0) -> None:
+    """The layers of a step whose rows are single new tokens, on the 32-bit stream h [T, H] in place: for each layer
+      h += (attention over the cache and the token's own key of rotated, normed q and k of x W_qkv) W_o,   x = norm1(h)
+      h += (silu(x W_gate) * x W_up) W_down,                                                               x = norm2(h)
+    layers: dicts of w_qkv [(Hq + 2 Hkv) D, H], w_o [H, Hq D], w_gu (interleave_gate_up) [2 I, H], w_down [H, I], bfloat16; norm1, norm2 [H],
+    q_norm, k_norm [D] or None, float32; eps1, eps2; cache [pages, 2, Hkv, P, D].  The rest as for attention_decode_fused().
+    units: how many blocks share the work (0: one a compute unit)."""
+    lib = load_library()
+    _need(h, "h", torch.float32, (None, None))
+    (T, H), dev = h.shape, h.device
+    first = layers[0]
+    cache = first["cache"]
+    if cache.dim() != 5:
+        raise KernelError("decode_chain: the cache has not five dimensions")
+    Hq, Hkv, P, D = int(num_heads), cache.shape[2], cache.shape[3], cache.shape[4]
+    I = first["w_down"].shape[1]
+    if not decode_chain_supported(T, H, Hq, Hkv, D, I, P):
+        raise KernelError("decode_chain: sizes not taken")
+    _need(positions, "positions", torch.int32, (T,), dev)
+    _need(tok_seq, "tok_seq", torch.int32, (T,), dev)
+    _need(block_table, "block_table", torch.int32, (None, None), dev)
+    if slots is not None:
+        _need(slots, "slots", torch.int32, (T,), dev)
+    if table is not None:
+        _need(table, "table", torch.float32, (None, D), dev)
+    if shared_keys is not None:
+        _need(shared_keys, "shared_keys", torch.int32, (block_table.shape[0],), dev)
+    shapes = (("w_qkv", torch.bfloat16, ((Hq + 2 * Hkv) * D, H)), ("w_o", torch.bfloat16, (H, Hq * D)),
+              ("w_gu", torch.bfloat16, (2 * I, H)), ("w_down", torch.bfloat16, (H, I)), ("norm1", torch.float32, (H,)),
+              ("norm2", torch.float32, (H,)), ("q_norm", torch.float32, (D,)), ("k_norm", torch.float32, (D,)),
+              ("cache", torch.bfloat16, (None, 2, Hkv, P, D)))
+    for layer in layers:
+        for name, dtype, shape in shapes:
+            if layer[name] is not None or name not in ("q_norm", "k_norm"):
+                _need(layer[name], name, dtype, shape, dev)
+    # (as many launches as the arguments of one hold layers, of about as many each)
+    most = lib.qe_decode_chain_layers()
+    launches = -(-len(layers) // most)
+    per = -(-len(layers) // launches)
+    nbytes = lib.qe_decode_chain_workspace_bytes(T, H, Hq, Hkv, I, per, int(max_position))
+    ws = torch.empty((nbytes,), dtype=torch.uint8, device=dev)
+    for at in range(0, len(layers), per):
+        some = layers[at:at + per]
+        ptrs = (ctypes.c_void_p * (9 * len(some)))(*[_ptr(layer[name]) for layer in some for name, _, _ in shapes])
+        eps = (ctypes.c_float * (2 * len(some)))(*[float(layer[name]) for layer in some for name in ("eps1", "eps2")])
+        _check(lib.qe_decode_chain(h.data_ptr(), ptrs, eps, len(some), positions.data_ptr(), tok_seq.data_ptr(), block_table.data_ptr(),
+                                   block_table.shape[1], _ptr(shared_keys), _ptr(slots), _ptr(table), float(qk_eps), float(scale), T, H, Hq, Hkv,
+                                   I, P, int(max_position), int(units), ws.data_ptr(), nbytes, _stream()), "decode_chain")
 
 
 def argmax(logits: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:

@@ -11,6 +11,7 @@ from ..cache.plan import CachePlan, plan_cache
 from ..config.spec import ModelSpec
 from ..kernels import ops
 from .base import CacheBinding, Runtime, Stream, TensorInfo, join_name, named_tensors, sub_tensors
+from .chain import run_as_chain
 from .registry import build_part, part_class
 
 
@@ -145,12 +146,13 @@ class DecoderModel:
                 h = ops.embedding(ctx.token_ids, self.embed)
                 if self.prologue is not None:
                     self.prologue.forward(h, ctx)
-            # (few rows: a second buffer, so that a product can do the residual sum before it, see Stream)
-            stream = Stream(h, torch.empty_like(h) if h.shape[0] <= ops.gemm_norm_max_rows() else None)
             pending = None
-            for i, entry in enumerate(self.spec.schedule):
-                pending = self.blocks[entry.layer].forward(stream, pending, ctx, bindings[i])   # (the entry's users' bindings)
-            h = stream.h
+            if not run_as_chain(self.blocks, self.spec.schedule, h, ctx, bindings):
+                # (few rows: a second buffer, so that a product can do the residual sum before it, see Stream)
+                stream = Stream(h, torch.empty_like(h) if h.shape[0] <= ops.gemm_norm_max_rows() else None)
+                for i, entry in enumerate(self.spec.schedule):
+                    pending = self.blocks[entry.layer].forward(stream, pending, ctx, bindings[i])   # (the entry's users' bindings)
+                h = stream.h
             R = ctx.logit_rows.shape[0]
             if R == 0:
                 return torch.empty((0, self.spec.vocab_size), dtype=torch.float32, device=h.device)
