@@ -13,8 +13,8 @@
 //     publish the products' results.
 //
 // A step of 28 layers (16 heads of 128 on 8, width 1024), logits and all, with six kernels a layer and so, in us: one request at 64 keys
-// 914, 609; at 8192 1088, 784; four at 128 1010, 706; eight at 1024 1250, 1084; eight at 12288 3086, 2926.  Of six layers of width 4096 with
-// 12288 in the middle 853, 710 (one request at 512 keys).  What is left above the bytes is the waiting: of some 21 us a layer of one request
+// 914, 590; at 8192 1088, 785; four at 128 1010, 706; eight at 1024 1250, 1058; eight at 12288 3086, 2861.  Of six layers of width 4096 with
+// 12288 in the middle 853, 711 (one request at 512 keys).  What is left above the bytes is the waiting: of some 20 us a layer of one request
 // 14 are the same without any weights, and a look for numbers stands behind the kilobytes that its compute unit has asked for before.
 //
 // A number that is not there yet is told by its bits: every place of the exchange holds ~0 (a NaN that no result has: a result of these
@@ -39,7 +39,7 @@ constexpr int D = 128;
 constexpr int MAX_LAYERS = 40;         // of one launch: what 4 KB of arguments hold
 constexpr int MAX_ROWS = 8;
 constexpr int MAX_GROUP = 8;
-constexpr int MAX_SEGMENTS = 32;       // a token's keys are cut in, of a multiple of 64 each
+constexpr int MAX_SEGMENTS = 32;       // a token's keys are cut in, of a multiple of 16 each
 constexpr unsigned NONE = ~0u;
 constexpr unsigned A_NAN = 0x7fc07fc0u;                    // as a float and as two bfloat16
 constexpr unsigned CLOSED = 0x80000000u;
@@ -285,7 +285,7 @@ template <int MV, int RING, int NP>
 __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) {
     // (read where they lie: the compiler copies an array of arguments that is indexed by a variable to scratch memory)
     const auto& a = *(const __attribute__((address_space(4))) ChainArgs*)__builtin_amdgcn_kernarg_segment_ptr();
-    constexpr int MT = MV > 4 ? 2 : 1, MR = MV, QR = 8 / MT;                // rows of a tile of results; quads of outputs between two barriers
+    constexpr int MT = MV > 4 ? 2 : 1, MR = MV, QR = 8;                // rows of a tile of results; quads of outputs between two barriers
     extern __shared__ __align__(16) unsigned char shared[];
     __shared__ Rows rows;
     __shared__ Share share;
@@ -340,10 +340,12 @@ __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) 
             rows.table[m] = row;
             rows.shared[m] = a.shared_keys ? a.shared_keys[row] : 0;
         }
-        // The keys are cut in segments of as few (of a multiple of 64) as give every block of the grid a segment of one key/value head
+        // The keys are cut in segments of as few (of a multiple of 16) as give every block of the grid a segment of one key/value head
         // at most, and a token MAX_SEGMENTS at most.
-        int keys = (most / (64 * MAX_SEGMENTS) + 1) * 64;
-        for (;; keys += keys >= 1024 ? 256 : 64) {
+        long keys_all = 0;
+        for (int m = 0; m < M; ++m) keys_all += rows.pos[m] + 1;
+        int keys = max(most / (16 * MAX_SEGMENTS) + 1, (int)(keys_all * Hkv / gridDim.x / 16)) * 16;
+        for (keys = max(keys, 16);; keys += 16 * (1 + keys / 256)) {
             int first = 0;
             for (int m = 0; m < M; ++m) {
                 rows.first[m] = first;
@@ -387,12 +389,19 @@ __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) 
         feed.begin(a, layers, share, rows, held, lane);
         feed.ask(RING, a, layers, share, rows, held, lane);
 
+        // What a product has used up is asked for again behind its barrier, or, with few numbers on the way between the blocks, when the next
+        // operand is there: a compute unit's loads come back in their order, and a look for the next numbers would wait for
+        // the kilobytes before it (width 1024, a layer: one request at 2048 keys 21.0 us and 19.9 so, at 8192 25.6 and 25.0; eight rows
+        // at 4060 53.4 and 56.1, width 4096 79 and 84).
+        constexpr bool LATE = MV <= 2 && NP == 1;
+        int debt = 0;
         int cur = 0;                                       // the ring's oldest kilobyte
         const auto slot_at = [&](int i) __attribute__((always_inline)) { const int s = cur + i; return s >= RING ? s - RING : s; };
         for (int turn = 0; turn < 5 * a.layers; ++turn) {
             const int stage = turn % 5;
             if (stage == 1) {
                 if (unit0 < unit1) BLOCK_BARRIER();
+                if (LATE) { feed.ask(debt, a, layers, share, rows, held, lane); debt = 0; }
                 for (int u = unit0; u < unit1; ++u) {
                     const Unit un = unit_of(rows, M, Hkv, u);
                     const int i = u - unit0;
@@ -454,6 +463,7 @@ __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) 
                 float* const mine = part + (r & 1) * (FEED * QR * MR * 4) + wave * (QR * MR * 4);
                 const int total = min(QR, quads - r * QR) * chunks;
                 int c = 0, q = 0, owed = 0;
+                if (LATE) { feed.ask(debt, a, layers, share, rows, held, lane); debt = 0; }
                 float acc[MT];
 #pragma unroll
                 for (int t = 0; t < MT; ++t) acc[t] = 0.f;
@@ -508,7 +518,7 @@ __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) 
                     for (int k = lane; k < QR * MR * 4; k += 64) mine[k] = 0.f;
                 }
                 BLOCK_BARRIER();
-                feed.ask(owed, a, layers, share, rows, held, lane);
+                if (LATE) debt += owed; else feed.ask(owed, a, layers, share, rows, held, lane);
             }
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (no load may come to shared memory that is another block's by then)
@@ -523,6 +533,9 @@ __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) 
     const auto h_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)a.h, 0, (unsigned)M * H * 4u, 0x00020000);
     // (16: past this compute die's L2, which the others' writes do not reach)
     const auto get4 = [&](unsigned word) __attribute__((always_inline)) { return __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(ex_rsrc, word * 4, 0, 16)); };
+    // Through the L2, where a compute die's blocks find what one of them has fetched.  It may hold a place as it was before it was written: then it
+    // still says ~0, as every place is written once, and get4 has to be asked.  (Not for the attention's parts.)
+    const auto near4 = [&](unsigned word) __attribute__((always_inline)) { return __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(ex_rsrc, word * 4, 0, 0)); };
     const auto get2 = [&](unsigned word) __attribute__((always_inline)) { return __builtin_bit_cast(u2, __builtin_amdgcn_raw_buffer_load_b64(ex_rsrc, word * 4, 0, 16)); };
     const auto get1 = [&](unsigned word) __attribute__((always_inline)) { return (unsigned)__builtin_amdgcn_raw_buffer_load_b32(ex_rsrc, word * 4, 0, 16); };
     const auto put1 = [&](unsigned word, unsigned v) __attribute__((always_inline)) { __builtin_amdgcn_raw_buffer_store_b32(v, ex_rsrc, word * 4, 0, 16); };
@@ -566,12 +579,12 @@ __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) 
 #pragma unroll
                 for (int p = 0; p < NP; ++p) v[m][p] = *(const u4*)(a.h + min(m, M - 1) * H + column(p));
         } else {
-            const auto get = [&]() __attribute__((always_inline)) {
+            const auto get_by = [&](auto load) __attribute__((always_inline)) {
                 bool ok = true;
 #pragma unroll
                 for (int m = 0; m < MV; ++m)
 #pragma unroll
-                    for (int p = 0; p < NP; ++p) v[m][p] = get4(from + min(m, M - 1) * H + column(p));
+                    for (int p = 0; p < NP; ++p) v[m][p] = load(from + min(m, M - 1) * H + column(p));
 #pragma unroll
                 for (int m = 0; m < MV; ++m)
 #pragma unroll
@@ -579,6 +592,7 @@ __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) 
                 return ok;
             };
             // (many rows: asked for again and again is one of them, until it is there; all of them would be some megabytes each time)
+            bool all = false;
             if constexpr (MV > 2) {
                 u4 u[NP];
                 await([&]() __attribute__((always_inline)) {
@@ -589,8 +603,9 @@ __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) 
                     for (int p = 0; p < NP; ++p) ok = ok & there(u[p]);
                     return ok;
                 });
+                all = __all(get_by(near4));
             }
-            if (!await(get)) {
+            if (!all && !await([&]() __attribute__((always_inline)) { return get_by(get4); })) {
 #pragma unroll
                 for (int m = 0; m < MV; ++m)
 #pragma unroll
@@ -656,22 +671,24 @@ __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) 
         constexpr int B = decltype(count)::value;
         const int stride = K * 2 + 64, per = K / 8, all = M * per;
         u4 v[B];
-        const auto get = [&]() __attribute__((always_inline)) {
+        const auto get_by = [&](auto load) __attribute__((always_inline)) {
             bool ok = true;
 #pragma unroll
-            for (int b = 0; b < B; ++b) v[b] = get4(from + min(i0 + b * WAIT * 64 + ht, all - 1) * 4);
+            for (int b = 0; b < B; ++b) v[b] = load(from + min(i0 + b * WAIT * 64 + ht, all - 1) * 4);
 #pragma unroll
             for (int b = 0; b < B; ++b) ok = ok & there(v[b]);
             return ok;
         };
+        bool found = false;
         if constexpr (B > 2) {                             // (one of many first, as above)
             u4 u;
             await([&]() __attribute__((always_inline)) {
                 u = get4(from + min(i0 + (B - 1) * WAIT * 64 + ht, all - 1) * 4);
                 return there(u);
             });
+            found = __all(get_by(near4));
         }
-        if (!await(get)) {
+        if (!found && !await([&]() __attribute__((always_inline)) { return get_by(get4); })) {
 #pragma unroll
             for (int b = 0; b < B; ++b) or_nan(v[b]);
         }
@@ -983,7 +1000,7 @@ __global__ __launch_bounds__(256) void decode_chain_clear_kernel(u4* work, unsig
 }
 
 int chain_segments(int max_position) {
-    const int s = max_position / 64 + 1;
+    const int s = max_position / 16 + 1;
     return s < MAX_SEGMENTS ? s : MAX_SEGMENTS;
 }
 
@@ -994,12 +1011,13 @@ size_t chain_shared(int ring, int M, int H, int Hq, int Hkv, int I) {
     if ((long)Hq * D > K) K = (long)Hq * D;
     const size_t x = (size_t)M * (K * 2 + 64);
     const size_t at = (size_t)4 * (2 * FEED * G * (D + 2) + 3 * (G + 2) * 64);
-    return (size_t)FEED * ring * 1024 + 4ul * 2 * FEED * (rows > 4 ? 4 : 8) * rows * 4 + (x > at ? x : at);
+    return (size_t)FEED * ring * 1024 + 4ul * 2 * FEED * 8 * rows * 4 + (x > at ? x : at);
 }
 constexpr size_t SHARED_LIMIT = 160 * 1024 - 512 - sizeof(ChainLayer) * MAX_LAYERS - sizeof(Tile) * FEED * TILES;         // (the kernel's few words besides)
 
 int chain_ring(int M, int H, int Hq, int Hkv, int I) {
-    if (chain_shared(12, M, H, Hq, Hkv, I) <= SHARED_LIMIT) return 12;
+    const int most = M > 4 ? 10 : 12;
+    if (chain_shared(most, M, H, Hq, Hkv, I) <= SHARED_LIMIT) return most;
     return chain_shared(8, M, H, Hq, Hkv, I) <= SHARED_LIMIT ? 8 : 0;
 }
 
@@ -1070,7 +1088,7 @@ extern "C" int qe_decode_chain(void* h, const void* const* layers, const float* 
     } while (0)
 #define QE_CHAIN2(MV_, NP_)                                                                   \
     do {                                                                                      \
-        if (ring == 12) QE_CHAIN3(MV_, 12, NP_);                                              \
+        if (ring > 8) QE_CHAIN3(MV_, (MV_ > 4 ? 10 : 12), NP_);                               \
         else QE_CHAIN3(MV_, 8, NP_);                                                          \
     } while (0)
 #define QE_CHAIN(MV_)                                                                         \
