@@ -1034,9 +1034,12 @@ extern "C" int qe_decode_chain_supported(int M, int H, int Hq, int Hkv, int head
 
 // Whether the chain is the quicker way: up to some 600 MB of matrices a layer.  Larger ones stream for so long that the kernels' starts count
 // for little, and each product's own kernel streams them faster (width 5120 with 25600 in the middle, 975 MB, one request: 899 us for three layers
-// and the logits with kernels, 935 so; width 4096 with 12288, 386 MB: 853 and 710 for six).
+// and the logits with kernels, 935 so; width 4096 with 12288, 386 MB: 853 and 711 for six).  Of wide layers it takes two rows at most: with
+// more the rows' way to all blocks and back costs what the starts do (width 4096, three requests 850 and 855; width 2560 with 9728, eight
+// layers, three 720 and 707, four 732 and 724; width 2048 with 6144, ten layers, six 657 and 588).
 extern "C" int qe_decode_chain_preferred(int M, int H, int Hq, int Hkv, int head_dim, int I, int P) {
-    return qe_decode_chain_supported(M, H, Hq, Hkv, head_dim, I, P) && 2.0 * H * ((Hq * 2.0 + 2.0 * Hkv) * head_dim + 3.0 * I) <= 600e6;
+    return qe_decode_chain_supported(M, H, Hq, Hkv, head_dim, I, P) && (M <= 2 || H <= 3072) &&
+           2.0 * H * ((Hq * 2.0 + 2.0 * Hkv) * head_dim + 3.0 * I) <= 600e6;
 }
 
 extern "C" int qe_decode_chain_layers() { return MAX_LAYERS; }
@@ -1095,6 +1098,7 @@ extern "C" int qe_decode_chain(void* h, const void* const* layers, const float* 
     do {                                                                                      \
         if (H <= 1024) QE_CHAIN2(MV_, 1);                                                     \
         else if (H <= 2048) QE_CHAIN2(MV_, 2);                                                \
+        else if (H <= 3072) QE_CHAIN2(MV_, 3);                                                \
         else QE_CHAIN2(MV_, 5);                                                               \
     } while (0)
     if (M == 1) QE_CHAIN(1);
