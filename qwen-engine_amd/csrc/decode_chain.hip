@@ -28,7 +28,7 @@
 // work is dealt out among those.  Every wait has an end: after LIMIT a wave takes NaN for what has not come, which makes the rows NaN.
 //
 // The sums of a product have one order, whatever the number of rows and blocks: K goes to the eight waves in chunks of 128 dealt out in turn, whose
-// sums are added in the order of the waves.  A token's keys are cut in segments that follow the step's tokens (rows.keys).
+// sums are added in the order of the waves.  A token's keys are cut in segments that follow its own position (segment_keys).
 #include "attention_tile.h"
 #include <type_traits>
 
@@ -39,7 +39,7 @@ constexpr int D = 128;
 constexpr int MAX_LAYERS = 40;         // of one launch: what 4 KB of arguments hold
 constexpr int MAX_ROWS = 8;
 constexpr int MAX_GROUP = 8;
-constexpr int MAX_SEGMENTS = 32;       // a token's keys are cut in, of a multiple of 16 each
+constexpr int MAX_SEGMENTS = 32;       // a token's keys are cut in
 constexpr unsigned NONE = ~0u;
 constexpr unsigned A_NAN = 0x7fc07fc0u;                    // as a float and as two bfloat16
 constexpr unsigned CLOSED = 0x80000000u;
@@ -86,7 +86,15 @@ struct Exchange {
     }
 };
 
-struct Unit { int m, kvh, seg, lo, hi, tiles, own; };      // cached keys [lo, hi); own: the token's own key belongs to it
+// A token's keys are cut in segments by its own position alone, so that its sums, and its bits, are the same alone and in company: of 128 keys, a
+// tile for each feeding wave, up to 16 of them; from 2048 keys on of 256, up to 32; then of as many 128s as make 32 at most.  More and
+// smaller segments suit one row, which has the chip to itself, fewer and larger ones eight, whose units are several a block (us a layer, width 1024
+// with 8 key/value heads, one row and eight rows of 2000 keys: segments of 128 20.8 and 42.1, of 256 22.6 and 40.2; of 4000: 128 23.2 and 57.7,
+// 256 24.2 and 54.0; of 16000: 512 31.1 and 117, 1024 39 and 116).
+__host__ __device__ constexpr int segment_keys(int p) { return 128 * (p < 2048 ? 1 : p < 8192 ? 2 : p / 4096 + 1); }
+
+// A unit of the attention: the cached keys [lo, hi) of one segment for one row and key/value head; own: the token's own key belongs to it.
+struct Unit { int m, kvh, seg, lo, hi, tiles, own; };
 
 __device__ __forceinline__ u4 rsrc_of(const void* p, unsigned bytes) {
     const unsigned long b = (unsigned long)p;
@@ -107,27 +115,45 @@ __device__ __forceinline__ const T* uniform(const T* p) {
     return (const T*)((unsigned long)(unsigned)uniform((int)(v >> 32)) << 32 | (unsigned)uniform((int)v));
 }
 
+__device__ __forceinline__ Unit uniform(const Unit& r) {
+    return Unit{uniform(r.m), uniform(r.kvh), uniform(r.seg), uniform(r.lo), uniform(r.hi), uniform(r.tiles), uniform(r.own)};
+}
+
 // What every wave knows of the step's rows.
 struct Rows {
     int pos[MAX_ROWS], slot[MAX_ROWS], table[MAX_ROWS], shared[MAX_ROWS];
     int first[MAX_ROWS + 1];           // the row's first unit of the attention
-    int keys;                          // a segment's
+    int keys[MAX_ROWS], segments[MAX_ROWS];                // a segment's keys; how many segments
 };
 
-__device__ __forceinline__ Unit unit_of(const Rows& rows, int M, int Hkv, int u) {
-    int m = 0;
-    while (m + 1 < M && u >= uniform(rows.first[m + 1])) ++m;
-    const int p = uniform(rows.pos[m]), len = uniform(rows.keys);
-    const int at = u - uniform(rows.first[m]);
-    Unit r;
-    r.m = m;
-    r.seg = uniform(at / Hkv);
-    r.kvh = at - r.seg * Hkv;
-    r.lo = r.seg * len;
-    r.hi = min(r.lo + len, p);
+__device__ __forceinline__ void unit_ends(Unit& r, const Rows& rows) {
+    const int pos = uniform(rows.pos[r.m]), keys = uniform(rows.keys[r.m]);
+    r.lo = r.seg * keys;
+    r.hi = min(r.lo + keys, pos);
     r.tiles = (max(0, r.hi - r.lo) + 15) >> 4;
-    r.own = p < r.lo + len;
+    r.own = pos < r.lo + keys;
+}
+// the u-th: row by row, in a row head by head, in a head segment by segment
+__device__ __forceinline__ Unit unit_at(const Rows& rows, int M, int u) {
+    Unit r;
+    r.m = 0;
+    while (r.m + 1 < M && u >= rows.first[r.m + 1]) ++r.m;
+    const int at = u - rows.first[r.m];
+    r.kvh = at / rows.segments[r.m];
+    r.seg = at - r.kvh * rows.segments[r.m];
+    unit_ends(r, rows);
     return r;
+}
+// the one behind it, of which there has to be one
+__device__ __forceinline__ void unit_next(Unit& r, const Rows& rows, int Hkv) {
+    if (++r.seg == uniform(rows.segments[r.m])) {
+        r.seg = 0;
+        if (++r.kvh == Hkv) {
+            r.kvh = 0;
+            ++r.m;
+        }
+    }
+    unit_ends(r, rows);
 }
 
 #define BLOCK_BARRIER()                                    \
@@ -162,10 +188,11 @@ struct Feed {
     int which;
 
     __device__ __forceinline__ static int chunks_of(int K, int wave) { return K / 128 > wave ? (K / 128 - wave + FEED - 1) / FEED : 0; }
+    __device__ __forceinline__ static Tile tile_at(const int* table, int max_blocks, int row, int key, int kvh, bool shared, int logP) {
+        return Tile{table[(long)row * max_blocks + (key >> logP)] | (shared ? (int)0x80000000 : 0), kvh << (logP + 8) | (key & ((1 << logP) - 1))};
+    }
     __device__ __forceinline__ static Tile tile_of(const int* table, int max_blocks, const Rows& rows, const Unit& un, int t, int logP) {
-        const int key = un.lo + t * 16;
-        return Tile{table[(long)rows.table[un.m] * max_blocks + (key >> logP)] | (un.lo < rows.shared[un.m] ? (int)0x80000000 : 0),
-                    un.kvh << (logP + 8) | (key & ((1 << logP) - 1))};
+        return tile_at(table, max_blocks, rows.table[un.m], un.lo + t * 16, un.kvh, un.lo < rows.shared[un.m], logP);
     }
     // how many kilobytes stage s has
     template <typename Args>
@@ -180,15 +207,21 @@ struct Feed {
         if (s == 1) {
             const int t = x >> 3, part = x & 7;
             Tile mine = held[min(max(t, 0), TILES - 1)];
-            if (tiles > TILES) {                           // (more than shared memory holds: found again)
-                int before = 0;
-                const int unit1 = uniform(share.unit1);
-                for (int u = uniform(share.unit0); u < unit1; ++u) {
-                    const Unit un = unit_of(rows, a.M, a.Hkv, u);
+            if (tiles > TILES) {                           // (more than shared memory holds: its unit is found again)
+                int before = 0, key = 0, row = 0, kvh = 0, shared = 0;
+                const int units = uniform(share.unit1) - uniform(share.unit0);
+                Unit un = unit_at(rows, a.M, uniform(share.unit0));
+                for (int i = 0; i < units; ++i) {
+                    if (i > 0) unit_next(un, rows, a.Hkv);
                     const int count = un.tiles > wave ? (un.tiles - wave + FEED - 1) / FEED : 0;
-                    if (t >= before && t < before + count) mine = tile_of(a.table, a.max_blocks, rows, un, wave + (t - before) * FEED, logP);
+                    const bool here = t >= before && t < before + count;
+                    key = here ? un.lo + (wave + (t - before) * FEED) * 16 : key;
+                    row = here ? uniform(rows.table[un.m]) : row;
+                    kvh = here ? un.kvh : kvh;
+                    shared = here ? un.lo < uniform(rows.shared[un.m]) : shared;
                     before += count;
                 }
+                mine = tile_at(a.table, a.max_blocks, row, key, kvh, shared, logP);
             }
             const int inside = mine.place & ((1 << logP) - 1), head = mine.place - inside;
             of_kind = (part < 4 ? (part << 6) << 3 | 1 : 2) | (mine.page < 0 ? 4 : 0);
@@ -289,10 +322,11 @@ __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) 
     extern __shared__ __align__(16) unsigned char shared[];
     __shared__ Rows rows;
     __shared__ Share share;
+    __shared__ Unit s_unit;
     __shared__ Tile tiles[FEED * TILES];
     __shared__ ChainLayer layers[MAX_LAYERS];              // (the arguments may lie in the host's memory)
     __shared__ __align__(16) float squares[MAX_ROWS][WAIT];
-    __shared__ int s_worker, s_workers;
+    __shared__ int s_worker, s_workers, s_units[2];
     __shared__ int s_late;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = lane >> 4, n = lane & 15;
@@ -331,30 +365,33 @@ __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) 
         }
         s_worker = worker;
         s_workers = workers;
-        int most = 0;
+        // The units are dealt out in their order and by what they cost: the tiles a wave has of them, and one more for a unit's joining.
+        int first = 0;
+        long weight = 0;
         for (int m = 0; m < M; ++m) {
             const int p = min(a.positions[m], a.max_position), row = a.tok_seq[m];
-            most = max(most, p);
             rows.pos[m] = p;
             rows.slot[m] = a.slots ? a.slots[m] : -1;
             rows.table[m] = row;
             rows.shared[m] = a.shared_keys ? a.shared_keys[row] : 0;
+            rows.keys[m] = segment_keys(p);
+            rows.segments[m] = p / rows.keys[m] + 1;
+            rows.first[m] = first;
+            first += rows.segments[m] * Hkv;
+            weight += (long)(rows.segments[m] * Hkv) * (rows.keys[m] / 128 + 1);
         }
-        // The keys are cut in segments of as few (of a multiple of 16) as give every block of the grid a segment of one key/value head
-        // at most, and a token MAX_SEGMENTS at most.
-        long keys_all = 0;
-        for (int m = 0; m < M; ++m) keys_all += rows.pos[m] + 1;
-        int keys = max(most / (16 * MAX_SEGMENTS) + 1, (int)(keys_all * Hkv / gridDim.x / 16)) * 16;
-        for (keys = max(keys, 16);; keys += 16 * (1 + keys / 256)) {
-            int first = 0;
+        rows.first[M] = first;
+        const auto share_begins = [&](int w) {
+            long left = weight * w;                        // (in parts of 1 / workers)
             for (int m = 0; m < M; ++m) {
-                rows.first[m] = first;
-                first += (rows.pos[m] / keys + 1) * Hkv;
+                const long one = (long)(rows.keys[m] / 128 + 1) * workers, count = rows.first[m + 1] - rows.first[m];
+                if (left <= one * count) return rows.first[m] + (int)((left + one - 1) / one);
+                left -= one * count;
             }
-            rows.first[M] = first;
-            if (first <= (int)gridDim.x || keys > most) break;
-        }
-        rows.keys = keys;
+            return first;
+        };
+        s_units[0] = worker < 0 ? 0 : share_begins(worker);
+        s_units[1] = worker < 0 ? 0 : share_begins(worker + 1);
     }
     __syncthreads();
     const int worker = uniform(s_worker), workers = uniform(s_workers);
@@ -363,9 +400,9 @@ __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) 
     const int qkv0 = part_of(CQ / 4, worker), qkv1 = part_of(CQ / 4, worker + 1);
     const int out0 = part_of(H / 4, worker), out1 = part_of(H / 4, worker + 1);
     const int act0 = part_of(I / 4, worker), act1 = part_of(I / 4, worker + 1);
-    const int units = uniform(rows.first[M]);
-    const int unit0 = part_of(units, worker), unit1 = part_of(units, worker + 1);
+    const int unit0 = uniform(s_units[0]), unit1 = uniform(s_units[1]);
     if (threadIdx.x == 0) share = Share{qkv0, qkv1, out0, out1, act0, act1, unit0, unit1};
+    if (threadIdx.x == 64) s_unit = unit0 < unit1 ? unit_at(rows, M, unit0) : Unit{};
     __syncthreads();
 
     if (wave < FEED) {
@@ -379,8 +416,10 @@ __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) 
         feed.keys = (lane >> 4) * 256 + (((lane & 15) ^ (lane >> 4)) << 4); feed.values = (lane >> 1) * P * 2 + (lane & 1) * 16;
         feed.to = (unsigned)(unsigned long)(__attribute__((address_space(3))) unsigned char*)shared + wave * RING * 1024;
         int count = 0;
+        Unit of = uniform(s_unit);
         for (int u = unit0; u < unit1; ++u) {
-            const Unit un = unit_of(rows, M, Hkv, u);
+            if (u > unit0) unit_next(of, rows, Hkv);
+            const Unit& un = of;
             for (int t = wave; t < un.tiles; t += FEED, ++count)
                 if (count < TILES && lane == 0) held[count] = Feed<RING, QR / 2>::tile_of(a.table, a.max_blocks, rows, un, t, a.logP);
         }
@@ -402,14 +441,19 @@ __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) 
             if (stage == 1) {
                 if (unit0 < unit1) BLOCK_BARRIER();
                 if (LATE) { feed.ask(debt, a, layers, share, rows, held, lane); debt = 0; }
+                Unit un = uniform(s_unit);
+                int turns = 0;
                 for (int u = unit0; u < unit1; ++u) {
-                    const Unit un = unit_of(rows, M, Hkv, u);
                     const int i = u - unit0;
+                    if (i > 0) {
+                        unit_next(un, rows, Hkv);
+                        turns += un.seg == 0;              // (another head's)
+                    }
                     if (wave < un.tiles) {
                         AttnState<D> st;
                         st.init();
                         bf16x8 qreg[D / 32];
-                        const unsigned* qrow = qbuf + (i % 3 * G + min(n, G - 1)) * 64;
+                        const unsigned* qrow = qbuf + (turns % 3 * G + min(n, G - 1)) * 64;
 #pragma unroll
                         for (int c = 0; c < D / 32; ++c) qreg[c] = *(const bf16x8*)(qrow + c * 16 + g * 4);
                         for (int t = wave; t < un.tiles; t += FEED) {
@@ -711,8 +755,8 @@ __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) 
         }
     };
     // q's heads of a unit (and the token's own key and value), normed and rotated, to shared memory; key and value to the cache
-    const auto prepare = [&](const Unit& un, int i, unsigned qkv, const float* q_norm, const float* k_norm, bf16_t* cache) __attribute__((always_inline)) {
-        const int tasks = un.own ? G + 2 : G;
+    const auto prepare = [&](const Unit& un, int i, bool with_q, unsigned qkv, const float* q_norm, const float* k_norm, bf16_t* cache) __attribute__((always_inline)) {
+        const int tasks = un.own ? G + 2 : G, task0 = with_q ? hw : G + hw;
         const int p = uniform(rows.pos[un.m]), slot = uniform(rows.slot[un.m]);
         constexpr int MOST = (MAX_GROUP + 2 + WAIT - 1) / WAIT;
         unsigned v[MOST];
@@ -721,7 +765,7 @@ __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) 
             cs = *(const float2*)(a.rope + (long)p * D + (lane & 31) * 2);
             sn = *(const float2*)(a.rope + (long)p * D + D / 2 + (lane & 31) * 2);
         }
-        const auto task = [&](int t) __attribute__((always_inline)) { return min(hw + t * WAIT, tasks - 1); };
+        const auto task = [&](int t) __attribute__((always_inline)) { return min(task0 + t * WAIT, tasks - 1); };
         float2 w[MOST];
 #pragma unroll
         for (int t = 0; t < MOST; ++t) w[t] = float2{1.f, 1.f};
@@ -750,7 +794,7 @@ __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) 
         const int in = slot & (P - 1);
 #pragma unroll
         for (int t = 0; t < MOST; ++t) {
-            const int j = hw + t * WAIT;
+            const int j = task0 + t * WAIT;
             if (j >= tasks) break;
             if (j == G + 1) {                              // the value
                 vbuf[i % 3 * 64 + lane] = v[t];
@@ -897,7 +941,7 @@ __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) 
     };
     const auto join_segments = [&](unsigned parts, unsigned att) __attribute__((always_inline)) {
         for (int t = join0 + hw; t < join1; t += WAIT) {
-            const int m = uniform((t >> 2) / Hq), segments = uniform(rows.pos[m]) / uniform(rows.keys) + 1;
+            const int m = uniform((t >> 2) / Hq), segments = uniform(rows.segments[m]);
             if (segments <= 8) join_some(std::integral_constant<int, 1>{}, t, segments, parts, att);
             else join_some(std::integral_constant<int, MAX_SEGMENTS / 8>{}, t, segments, parts, att);
         }
@@ -917,16 +961,19 @@ __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) 
             const unsigned parts = ex.parts + (l & 1) * ex.set;
             if (unit0 < unit1) {
                 // (a unit is prepared while the feeding waves have the one before)
-                Unit un = unit_of(rows, M, Hkv, unit0);
-                prepare(un, 0, base + ex.qkv, L.q_norm, L.k_norm, L.cache);
+                Unit un = uniform(s_unit);
+                int turns = 0;
+                prepare(un, 0, true, base + ex.qkv, L.q_norm, L.k_norm, L.cache);
                 BLOCK_BARRIER();
                 for (int u = unit0; u < unit1; ++u) {
                     const int i = u - unit0;
                     const Unit now = un;
-                    look_up_own(now, i);
+                    look_up_own(now, turns);
                     if (u + 1 < unit1) {
-                        un = unit_of(rows, M, Hkv, u + 1);
-                        prepare(un, i + 1, base + ex.qkv, L.q_norm, L.k_norm, L.cache);
+                        unit_next(un, rows, Hkv);
+                        const bool another = un.seg == 0;
+                        turns += another;
+                        if (another || un.own) prepare(un, turns, another, base + ex.qkv, L.q_norm, L.k_norm, L.cache);
                     }
                     BLOCK_BARRIER();
                     join_waves(now, i, parts);
@@ -1000,8 +1047,8 @@ __global__ __launch_bounds__(256) void decode_chain_clear_kernel(u4* work, unsig
 }
 
 int chain_segments(int max_position) {
-    const int s = max_position / 16 + 1;
-    return s < MAX_SEGMENTS ? s : MAX_SEGMENTS;
+    const int small = max_position / 128 + 1, large = max_position / 256 + 1;      // (segment_keys() for all positions up to it)
+    return max(min(small, 16), min(large, MAX_SEGMENTS));
 }
 
 // Shared memory for rings of `ring` kilobytes.

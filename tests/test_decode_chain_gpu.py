@@ -178,6 +178,32 @@ def test_the_same_bits_again_recorded_and_on_two_streams(ops):
         torch.ones(1 << 20, device=DEV).sum().item()
 
 
+@pytest.mark.parametrize("H,Hq,Hkv,I", [(256, 4, 2, 384), (1024, 16, 8, 1024)])
+def test_a_token_alone_and_in_company(ops, H, Hq, Hkv, I):
+    """A row's bits, and those of the key and value it writes, follow neither the rows beside it nor the number of blocks: positions at
+    both sides of where the segments' length changes, and rows whose units are dealt to one block and to many."""
+    pos = [2047, 0, 130, 8191, 700, 2048, 8192, 16500]
+    layers, table, bt, slots, perm, h0 = make(ops, 2, H, Hq, Hkv, I, 16, pos, seed=9)
+    fresh = on_device(ops, layers)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    bt, table = bt.to(DEV), table.to(DEV)
+
+    def run(rows, units=0):
+        dev = [dict(d, cache=d["cache"].clone()) for d in fresh]
+        h = h0[rows].to(DEV)
+        ops.decode_chain(h, dev, i32([pos[r] for r in rows]), i32(rows), bt, slots[rows].to(DEV), Hq, D ** -0.5, max(pos[r] for r in rows), 1e-6, table, units=units)
+        new = [torch.stack([d["cache"][int(perm[r, pos[r] // 16]), 0, :, pos[r] % 16] for d in dev]) for r in rows]
+        return h.cpu(), [x.cpu() for x in new]
+
+    want_h, want_k = run(list(range(8)))
+    assert bool(torch.isfinite(want_h).all())
+    for rows in ([0], [1], [3], [7], [6, 2], [5, 0], [4, 1, 7], [2, 3, 5, 6], [7, 6, 5, 4, 3]):
+        for units in (0, 11):
+            h, k = run(rows, units)
+            for i, r in enumerate(rows):
+                assert torch.equal(h[i], want_h[r]) and torch.equal(k[i], want_k[r]), (rows, r, units)
+
+
 def test_refuses_what_it_does_not_take(ops):
     assert not ops.decode_chain_supported(9, 1024, 16, 8, 128, 3072, 16)          # rows
     assert not ops.decode_chain_supported(1, 1024, 16, 8, 64, 3072, 16)           # head size
