@@ -198,6 +198,7 @@ class RequestCache:
     hashes: List[int] = field(default_factory=list)   # chain hashes of the full pages so far
     shared_len: int = 0                # tokens taken over from other requests at admission
     new_request: bool = True           # no step has run yet: fixed-size state must be cleared
+    trusted: bool = True               # its pages may be registered for others
     dirty: List[List[int]] = field(default_factory=list)   # per group: table indices changed since taken
     released: List[int] = field(default_factory=list)      # per group: table entries below this were given back
 
@@ -406,7 +407,7 @@ class CacheManager:
         rc.tokens.extend(int(t) for t in tokens)
         rc.num_tokens = new_len
         rc.new_request = False
-        if self.prefix_sharing:
+        if self.prefix_sharing and rc.trusted:
             self._register_full_pages(rc)
         for g, table in enumerate(rc.tables):
             if self.groups[g].window is None:
@@ -519,13 +520,14 @@ class CacheManager:
                 self._shared[h] = self._behind[parent, toks] = _SharedEntry(pages=pages, tokens=toks, parent=parent, hash=h)
                 self._page_hash[pages[0]] = h
 
-    # ---- whole-manager views -------------------------------------------------------
-    def num_free_pages(self, group: int = 0) -> int:
-        return self.available(group)
+    def distrust(self) -> None:
+        """What the pages hold may be wrong: no registered page stays so, and the live requests register none any more."""
+        for rc in self.requests.values():
+            rc.trusted = False
+        self.stats["pages_freed"] += len(self._kept) * len(self.pools)
+        self._forget()
 
-    def reset(self) -> None:
-        for req_id in list(self.requests):
-            self.free_request(req_id)
+    def _forget(self) -> None:
         for entry in self._kept.values():
             for g, page in enumerate(entry.pages):
                 self.pools[g].give_back(page)
@@ -535,6 +537,15 @@ class CacheManager:
         self._shared.clear()
         self._behind.clear()
         self._page_hash.clear()
+
+    # ---- whole-manager views -------------------------------------------------------
+    def num_free_pages(self, group: int = 0) -> int:
+        return self.available(group)
+
+    def reset(self) -> None:
+        for req_id in list(self.requests):
+            self.free_request(req_id)
+        self._forget()
 
     def check_invariants(self) -> None:
         """No page lost, held twice without a count, or both free and held."""

@@ -25,7 +25,8 @@
 // published, and a reader of it has published there behind its ~0.
 //
 // No block waits for one that is not running: which blocks take part is settled at the start by a roll call, and the
-// work is dealt out among those.  Every wait has an end: after LIMIT a wave takes NaN for what has not come, which makes the rows NaN.
+// work is dealt out among those.  Every wait has an end: at its limit a wave takes NaN for what has not come, which makes the rows NaN, and says so
+// in a word of the host's memory (`late`), which whoever takes the results looks at.
 //
 // The sums of a product have one order, whatever the number of rows and blocks: K goes to the eight waves in chunks of 128 dealt out in turn, whose
 // sums are added in the order of the waves.  A token's keys are cut in segments that follow its own position (segment_keys).
@@ -43,7 +44,7 @@ constexpr int MAX_SEGMENTS = 32;       // a token's keys are cut in
 constexpr unsigned NONE = ~0u;
 constexpr unsigned A_NAN = 0x7fc07fc0u;                    // as a float and as two bfloat16
 constexpr unsigned CLOSED = 0x80000000u;
-constexpr unsigned long LIMIT = 200000000ul;               // two seconds of the 100 MHz clock
+constexpr unsigned GAP = 1000000u;                         // of the 100 MHz clock: 10 ms
 constexpr unsigned long CALL = 20000ul;                    // 200 us
 
 typedef unsigned u4 __attribute__((ext_vector_type(4)));
@@ -64,6 +65,22 @@ struct ChainArgs {
     unsigned* work;
     float scale, qk_eps;
     int layers, M, H, Hq, Hkv, I, logP, max_blocks, segments, max_position;
+    int* late;                         // host memory, or null: 1 once a wait has been given up
+    unsigned limit;                    // of a wait, in ticks of the 100 MHz clock
+    int absent;                        // blocks that the roll call counts beside those that come
+};
+
+// How long something has been waited for.  The clock also runs while the device has set the whole queue aside for another process, so a gap
+// between two looks counts as GAP at most: what is waited for stood still as well.
+struct Waited {
+    unsigned ticks = 0;
+    unsigned long last = 0;
+    __device__ __forceinline__ unsigned look() {
+        const unsigned long t = __builtin_amdgcn_s_memrealtime();
+        if (last) ticks += (unsigned)min(t - last, (unsigned long)GAP);
+        last = t;
+        return ticks;
+    }
 };
 
 // The exchange, in words from its start: the roll call's, the attention's parts (two sets), then a layer's numbers, layer after layer.
@@ -355,13 +372,16 @@ __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) 
             const unsigned long t0 = __builtin_amdgcn_s_memrealtime();
             while (__hip_atomic_load(a.work, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < gridDim.x &&
                    __builtin_amdgcn_s_memrealtime() - t0 < CALL) {}
-            workers = (int)__hip_atomic_fetch_or(a.work, CLOSED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            workers = (int)__hip_atomic_fetch_or(a.work, CLOSED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + a.absent;
             __hip_atomic_store(a.work + 16, (unsigned)workers, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         } else {                                           // (the first comer runs and says so soon)
-            const unsigned long t0 = __builtin_amdgcn_s_memrealtime();
+            Waited waited;
             do workers = (int)__hip_atomic_load(a.work + 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            while (workers == 0 && __builtin_amdgcn_s_memrealtime() - t0 < LIMIT);
-            if (workers == 0) worker = -1;
+            while (workers == 0 && waited.look() < a.limit);
+            if (workers == 0) {
+                worker = -1;
+                if (a.late) __hip_atomic_store(a.late, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
         }
         s_worker = worker;
         s_workers = workers;
@@ -589,20 +609,17 @@ __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) 
     const auto there = [&](const u4& v) __attribute__((always_inline)) {
         return ((v.x != NONE) & (v.y != NONE) & (v.z != NONE) & (v.w != NONE)) != 0;
     };
-    // Asks (get(): false while something is missing) until all lanes have all, or until LIMIT: then false.
+    // Asks (get(): false while something is missing) until all lanes have all, or until the limit of a wait: then false, and the host is told.
     // (No load of a get() stands under a condition: the compiler would wait for it before the next.)
     const auto await = [&](auto get) __attribute__((always_inline)) {
-        unsigned long t0 = 0;
+        Waited waited;
         for (unsigned i = 1;; ++i) {
             if (__all(get())) return true;
-            if (i % 64 == 0) {
-                const unsigned long t = __builtin_amdgcn_s_memrealtime();
-                if (t0 == 0) t0 = t;
-                if (__hip_atomic_load(&s_late, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) || t - t0 > LIMIT) break;
-            }
+            if (i % 64 == 0 && (waited.look() > a.limit || __hip_atomic_load(&s_late, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))) break;
             asm volatile("" ::: "memory");
         }
         __hip_atomic_store(&s_late, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);   // (nobody in this block waits again)
+        if (a.late && lane == 0) __hip_atomic_store(a.late, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         return false;
     };
     const auto or_nan = [&](u4& v) __attribute__((always_inline)) {
@@ -1098,14 +1115,17 @@ extern "C" long qe_decode_chain_workspace_bytes(int M, int H, int Hq, int Hkv, i
 
 // h: float32 [M, H], the stream in front of the first layer, and behind the last one afterwards.  layers: for each nine pointers: q|k|v, output, gate|up
 // (rows of gate and up in alternating blocks of 32) and down matrices, the weights of the two norms and of q's and k's (null: none), the cache.  eps: two a layer.
-// rope: rows [cos | sin] of 128 numbers a position, or null.  units: blocks (0: one a compute unit).  Every row is the one new token of its request, at positions[m] <= max_position.
+// rope: rows [cos | sin] of 128 numbers a position, or null.  units: blocks (0: one a compute unit).  late: a word of pinned host memory that
+// becomes 1 if a block has waited for others for limit_us in vain (the rows are then NaN), or null.  absent: so many blocks more are given work than
+// come, so that what they should do is waited for in vain.  Every row is the one new token of its request, at positions[m] <= max_position.
 extern "C" int qe_decode_chain(void* h, const void* const* layers, const float* eps, int n_layers, const int* positions, const int* tok_seq,
                                const int* block_table, int max_blocks, const int* shared_keys, const int* slots, const float* rope, float qk_eps,
-                               float scale, int M, int H, int Hq, int Hkv, int I, int P, int max_position, int units, void* workspace,
-                               long workspace_bytes, hipStream_t stream) {
+                               float scale, int M, int H, int Hq, int Hkv, int I, int P, int max_position, int units, int* late, int limit_us,
+                               int absent, void* workspace, long workspace_bytes, hipStream_t stream) {
     QE_REQUIRE(qe_decode_chain_supported(M, H, Hq, Hkv, D, I, P), "decode chain: sizes not taken");
     QE_REQUIRE(n_layers >= 1 && n_layers <= MAX_LAYERS, "decode chain: %d layers in a launch", n_layers);
     QE_REQUIRE(max_position >= 0, "decode chain: position %d", max_position);
+    QE_REQUIRE(limit_us > 0 && limit_us <= 10000000 && absent >= 0 && absent <= 1024, "decode chain: a limit of %d us, %d blocks absent", limit_us, absent);
     for (int l = 0; l < n_layers; ++l) QE_REQUIRE(!layers[9 * l + 6] == !layers[9 * l + 7], "decode chain: a norm of q or of k alone");
     QE_REQUIRE(workspace_bytes >= qe_decode_chain_workspace_bytes(M, H, Hq, Hkv, I, n_layers, max_position),
                "decode chain: workspace of %ld bytes is too small", workspace_bytes);
@@ -1124,6 +1144,7 @@ extern "C" int qe_decode_chain(void* h, const void* const* layers, const float* 
     a.scale = scale; a.qk_eps = qk_eps;
     a.layers = n_layers; a.M = M; a.H = H; a.Hq = Hq; a.Hkv = Hkv; a.I = I;
     a.logP = __builtin_ctz(P);
+    a.late = late; a.limit = (unsigned)limit_us * 100u; a.absent = absent;
     a.max_blocks = max_blocks; a.segments = chain_segments(max_position); a.max_position = max_position;
     const Exchange ex(M, H, Hq, Hkv, I, a.segments, n_layers);
     const int ring = chain_ring(M, H, Hq, Hkv, I);

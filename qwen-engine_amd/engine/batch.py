@@ -39,6 +39,9 @@ class StepContext:
     # pages that other requests read as well (a shared prefix).  A hint for kernels that choose between
     # loads that leave a line in the caches and loads that stream past them; no result depends on it.
     shared_keys: Optional[torch.Tensor] = None
+    # int32 [1] in pinned host memory, or None: kernels whose blocks wait for each other write 1 to it when they have given
+    # a wait up, and the step's rows are then NaN (ModelRunner.check looks at it).
+    late: Optional[torch.Tensor] = None
     # What single parts asked to have prepared for this step, by part class (see
     # ``parts.base``: step_extras / graph_extras), and a place where a part may keep what it
     # builds once per step and shares between its layers.

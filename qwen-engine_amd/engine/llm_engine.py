@@ -116,6 +116,7 @@ class LLMEngine:
             logits = self.runner.step(entries)
             us = [uniform_for(r.params.seed, r.req_id, len(r.output)) if t > 0 else 0.0 for r, t in zip(sampling, temps)]
             tokens = self.sampler.sample(logits, temps, us)
+            self.runner.check()                    # (the tokens are there, and so is the word of a step that failed)
         return self.scheduler.update(planned, tokens)
 
     def run(self) -> List[GenerationResult]:

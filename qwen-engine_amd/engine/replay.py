@@ -42,6 +42,7 @@ def replay(model_dir: str, dtype: str, out_dir: str, max_tokens: int, lines: IO[
             logits = runner.step(entries)
             if logits.shape[0]:
                 arr = logits.detach().to("cpu", torch.float32).numpy().astype("<f4", copy=False)
+                runner.check()
                 arr.tofile(os.path.join(out_dir, f"{step}.f32"))
         for req_id in rec.get("end", []):
             if req_id in runner.cache.requests:

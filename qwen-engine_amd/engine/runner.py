@@ -157,6 +157,9 @@ class ModelRunner:
         # per table row: the request's first keys that other requests read too (StepContext.shared_keys)
         self.shared_keys = torch.zeros(max_requests + 1, dtype=torch.int32, device=dev)
         self._shared_keys_host = [0] * (max_requests + 1)
+        # what kernels write to whose blocks waited for each other in vain (StepContext.late)
+        self._late = torch.zeros(1, dtype=torch.int32).pin_memory()
+        self._late_np = self._late.numpy()
         # positions that a row standing on the spare row may have: inside every group's table row, and the model's
         self._spare_positions = min([w * page_size for w in self.table_width] + [model.spec.max_positions])
         # a part with per-request state is recorded into graphs only if it says that it can be
@@ -251,6 +254,8 @@ class ModelRunner:
         return self.cache.add_request(req_id)
 
     def free_request(self, req_id: Hashable) -> None:
+        if self._late_np[0]:                       # (none of its pages stays for others; the next step or check() says so)
+            self.cache.distrust()
         self.cache.free_request(req_id)
         self._poison_pages()
 
@@ -488,7 +493,7 @@ class ModelRunner:
             extras[cls][name] = t
         return StepContext(rt=self.rt, page_size=self.page_size, num_tokens=T, seqs=seqs, token_ids=d_tok,
                            positions=d_pos, tok_seq=d_seq, block_tables=self.tables,
-                           shared_keys=self.shared_keys, slots=d_slots,
+                           shared_keys=self.shared_keys, late=self._late, slots=d_slots,
                            logit_rows=d_rows, state_slots=d_state, max_position=int(positions.max()),
                            extras=extras)
 
@@ -496,7 +501,10 @@ class ModelRunner:
         """Runs the entries' tokens as one batch; returns float32 logits [wanted, vocab] on the
         device, in the order of the entries and of their ``want``.  With ``greedy`` it returns, instead,
         the index of the largest logit of every wanted row (the lowest on ties, src/engine/executor.py:51-54)
-        as a list of integers: a recorded step picks them inside its graph, and no logits travel."""
+        as a list of integers: a recorded step picks them inside its graph, and no logits travel.
+        Raises KernelError if a step since the last look has failed on the device: this one where it waits for its results
+        (nothing is committed then), else an earlier one (see check)."""
+        self.check()
         logits = None
         if self.use_graphs and all(len(e.tokens) == 1 and list(e.want) == [0] for e in entries) and entries:
             logits = self._decode_step_with_graph(entries, greedy)
@@ -511,11 +519,23 @@ class ModelRunner:
             logits = self.model.forward(ctx, self.bindings)
             if greedy:
                 logits = ops.argmax(logits).tolist() if logits.shape[0] else []
+        if greedy:                                 # (the results are there, and so is the word of a step that failed)
+            self.check()
         for e in entries:
             self.cache.commit(e.req_id, e.tokens)
         self._poison_pages()                       # (pages that a window has passed went back)
         self.steps_run += 1
         return logits
+
+    def check(self) -> None:
+        """Raises KernelError if a step that has run since the last look has failed on the device (blocks that waited for each other's
+        numbers in vain): its logits are NaN, and so is what it left in the cache of its requests.  No page that is
+        registered now or belongs to a live request is shared from then on; the caller frees the requests.  To be called when the
+        results of a step are there; step() looks by itself before it runs anything."""
+        if self._late_np[0]:
+            self._late_np[0] = 0
+            self.cache.distrust()
+            raise ops.KernelError("a step failed: blocks of a kernel waited for each other in vain; the requests that ran have to be freed")
 
     # ---- decoding through a recorded graph ------------------------------------------------
     def _recorded_argmax(self, logits: torch.Tensor) -> Optional[torch.Tensor]:
@@ -699,7 +719,7 @@ class ModelRunner:
             [SeqInfo(None, B, T, 0, self.spare_row, False)]
         ctx = StepContext(rt=self.rt, page_size=self.page_size, num_tokens=B + T, seqs=seqs, token_ids=d_tok,
                           positions=d_pos, tok_seq=d_seq, block_tables=self.tables,
-                          shared_keys=self.shared_keys, slots=d_slots,
+                          shared_keys=self.shared_keys, late=self._late, slots=d_slots,
                           logit_rows=d_rows, state_slots=d_state, max_position=0,
                           extras={cls: dict(cls.mixed_graph_extras(B, T, k, dev, dyn))
                                   for cls, k, dyn in zip(self._step_classes, part_keys, d_dyn)})
@@ -791,7 +811,7 @@ class ModelRunner:
         seqs = [SeqInfo(None, 0, T, 0, self.spare_row, False)]
         ctx = StepContext(rt=self.rt, page_size=self.page_size, num_tokens=T, seqs=seqs, token_ids=d_tok,
                           positions=d_pos, tok_seq=d_seq, block_tables=self.tables,
-                          shared_keys=self.shared_keys, slots=d_slots,
+                          shared_keys=self.shared_keys, late=self._late, slots=d_slots,
                           logit_rows=d_rows, state_slots=d_state, max_position=0,
                           extras={cls: dict(cls.portion_graph_extras(T, dev) if k is None
                                             else cls.portion_graph_extras(T, dev, k))
@@ -845,7 +865,7 @@ class ModelRunner:
         seqs = [SeqInfo(None, i, 1, 0, 0, False) for i in range(B)]
         ctx = StepContext(rt=self.rt, page_size=self.page_size, num_tokens=B, seqs=seqs, token_ids=d_tok,
                           positions=d_pos, tok_seq=d_seq, block_tables=self.tables,
-                          shared_keys=self.shared_keys, slots=d_slots,
+                          shared_keys=self.shared_keys, late=self._late, slots=d_slots,
                           logit_rows=d_rows, state_slots=d_state, max_position=0,
                           extras={cls: dict(cls.graph_extras(B, k, dev)) if hasattr(cls, "graph_extras") else {}
                                   for cls, k in zip(self._step_classes, part_keys)})

@@ -141,7 +141,7 @@ def load_library():
         "qe_decode_chain_supported": [i32, i32, i32, i32, i32, i32, i32],
         "qe_decode_chain_preferred": [i32, i32, i32, i32, i32, i32, i32],
         "qe_decode_chain_layers": [],
-        "qe_decode_chain": [vp, vp, vp, i32, vp, vp, vp, i32, vp, vp, vp, f32, f32, i32, i32, i32, i32, i32, i32, i32, i32, vp, i64, vp],
+        "qe_decode_chain": [vp, vp, vp, i32, vp, vp, vp, i32, vp, vp, vp, f32, f32, i32, i32, i32, i32, i32, i32, i32, i32, vp, i32, i32, vp, i64, vp],
     }
     for name, args in sigs.items():
         fn = getattr(lib, name)
@@ -1047,15 +1047,20 @@ def decode_chain_preferred(rows: int, hidden: int, num_heads: int, num_kv_heads:
 
 def decode_chain(h: torch.Tensor, layers, positions: torch.Tensor, tok_seq: torch.Tensor, block_table: torch.Tensor,
                  slots: Optional[torch.Tensor], num_heads: int, scale: float, max_position: int, qk_eps: float = 0.0,
-                 table: Optional[torch.Tensor] = None, shared_keys: Optional[torch.Tensor] = None, units: int = 0) -> None:
+                 table: Optional[torch.Tensor] = None, shared_keys: Optional[torch.Tensor] = None, units: int = 0,
+                 late: Optional[torch.Tensor] = None, limit_us: int = 2000000, absent: int = 0) -> None:
     """The layers of a step whose rows are single new tokens, on the 32-bit stream h [T, H] in place: for each layer
       h += (attention over the cache and the token's own key of rotated, normed q and k of x W_qkv) W_o,   x = norm1(h)
       h += (silu(x W_gate) * x W_up) W_down,                                                               x = norm2(h)
     layers: dicts of w_qkv [(Hq + 2 Hkv) D, H], w_o [H, Hq D], w_gu (interleave_gate_up) [2 I, H], w_down [H, I], bfloat16; norm1, norm2 [H],
     q_norm, k_norm [D] or None, float32; eps1, eps2; cache [pages, 2, Hkv, P, D].  The rest as for attention_decode_fused().
-    units: how many blocks share the work (0: one a compute unit)."""
+    units: how many blocks share the work (0: one a compute unit).  The blocks wait for each other's numbers: a block that has waited
+    for limit_us in vain goes on with NaN and writes 1 to ``late`` (int32 [1] in pinned host memory), to be looked at when the results are
+    there.  absent: so many blocks more are given work than there are (for a test of that)."""
     lib = load_library()
     _need(h, "h", torch.float32, (None, None))
+    if late is not None and not (late.dtype == torch.int32 and late.shape == (1,) and late.is_pinned()):
+        raise KernelError("decode_chain: late is no word of pinned host memory")
     (T, H), dev = h.shape, h.device
     first = layers[0]
     cache = first["cache"]
@@ -1094,7 +1099,8 @@ def decode_chain(h: torch.Tensor, layers, positions: torch.Tensor, tok_seq: torc
         eps = (ctypes.c_float * (2 * len(some)))(*[float(layer[name]) for layer in some for name in ("eps1", "eps2")])
         _check(lib.qe_decode_chain(h.data_ptr(), ptrs, eps, len(some), positions.data_ptr(), tok_seq.data_ptr(), block_table.data_ptr(),
                                    block_table.shape[1], _ptr(shared_keys), _ptr(slots), _ptr(table), float(qk_eps), float(scale), T, H, Hq, Hkv,
-                                   I, P, int(max_position), int(units), ws.data_ptr(), nbytes, _stream()), "decode_chain")
+                                   I, P, int(max_position), int(units), _ptr(late), int(limit_us), int(absent), ws.data_ptr(), nbytes, _stream()),
+               "decode_chain")
 
 
 def argmax(logits: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:

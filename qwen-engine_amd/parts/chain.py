@@ -68,5 +68,5 @@ def run_as_chain(blocks, schedule, h: torch.Tensor, ctx, bindings: List[CacheBin
                        "norm2": b.ffn_norm.weight, "q_norm": m.q_norm, "k_norm": m.k_norm, "cache": c.kv,
                        "eps1": b.mixer_norm.eps, "eps2": b.ffn_norm.eps})
     ops.decode_chain(h, layers, ctx.positions, ctx.tok_seq, ctx.block_tables[g], ctx.slots[g], mix.hq, mix.scale, ex["max_dec_position"],
-                     mix.qk_eps if mix.qk_eps is not None else 0.0, table, ctx.shared_keys)
+                     mix.qk_eps if mix.qk_eps is not None else 0.0, table, ctx.shared_keys, late=ctx.late)
     return True

@@ -325,3 +325,35 @@ def test_plan_with_blocks_of_several_cache_users_and_of_none():
     assert plan.user_state == [None, StateNeed((3,)), None, None, None]
     with pytest.raises(ValueError):
         plan_cache([([(full, None), (win, None)], None), ([(full, None)], 0)])   # one user cannot pair with two
+
+
+@pytest.mark.parametrize("groups", [1, 2])
+def test_what_is_distrusted_is_not_shared(groups):
+    P = 4
+    m = CacheManager([GroupSpec()] * groups, 12, page_size=P, max_requests=3, prefix_sharing=True, keep_freed_prefixes=True)
+
+    def run(rid, tokens):
+        m.add_request(rid)
+        at = m.match_prefix(rid, tokens)
+        m.reserve(rid, len(tokens))
+        m.commit(rid, tokens[at:])
+        return at
+
+    prompt = list(range(9))
+    assert run("old", prompt) == 0
+    m.free_request("old")
+    assert m.num_kept == 2 and run("live", prompt) == 8
+    m.distrust()
+    m.check_invariants()
+    assert m.num_kept == 0 and run("other", prompt) == 0          # nothing that was registered is found
+    m.reserve("live", 16)
+    m.commit("live", list(range(9, 16)))                          # nor what a request goes on with that was live then
+    m.free_request("live")
+    m.check_invariants()
+    assert m.num_kept == 0 and run("again", prompt) == 8          # ("other" came afterwards)
+    assert m.block_table("again", 0)[:2] == m.block_table("other", 0)[:2]
+    m.free_request("other")
+    m.free_request("again")
+    m.check_invariants()
+    assert m.num_kept == 2 and all(p.num_free == 10 for p in m.pools)
+    assert m.stats["pages_allocated"] - m.stats["pages_freed"] == 2 * groups

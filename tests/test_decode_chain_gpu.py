@@ -82,7 +82,7 @@ def plain(layers, table, perm, h, pos, Hq, Hkv, P):
     return h, new
 
 
-def check(ops, n, H, Hq, Hkv, I, P, pos, units=0, seed=1, write=True, shared=None, **kw):
+def check(ops, n, H, Hq, Hkv, I, P, pos, units=0, seed=1, write=True, shared=None, late=None, **kw):
     layers, table, bt, slots, perm, h0 = make(ops, n, H, Hq, Hkv, I, P, pos, seed, **kw)
     want, new = plain(layers, table, perm, h0, pos, Hq, Hkv, P)
     dev = on_device(ops, layers)
@@ -90,7 +90,7 @@ def check(ops, n, H, Hq, Hkv, I, P, pos, units=0, seed=1, write=True, shared=Non
     args = (i32(pos), i32(list(range(len(pos)))), bt.to(DEV), slots.to(DEV) if write else None, Hq, D ** -0.5, max(pos), 1e-6,
             None if table is None else table.to(DEV), None if shared is None else i32(shared))
     h = h0.to(DEV)
-    ops.decode_chain(h, dev, *args, units=units)
+    ops.decode_chain(h, dev, *args, units=units, late=late)
     torch.cuda.synchronize()
     # what the layers add, of which each of some ten roundings to bfloat16 a layer leaves 2^-9 at the most, 2^-10 in the mean square
     err = float((h.cpu().double() - want).norm() / (want - h0.double()).norm())
@@ -202,6 +202,27 @@ def test_a_token_alone_and_in_company(ops, H, Hq, Hkv, I):
             h, k = run(rows, units)
             for i, r in enumerate(rows):
                 assert torch.equal(h[i], want_h[r]) and torch.equal(k[i], want_k[r]), (rows, r, units)
+
+
+@pytest.mark.parametrize("rows", [1, 3, 8])
+def test_a_wait_in_vain_ends_and_is_told(ops, rows):
+    """Blocks that have work and do not come: every wait ends, the rows are NaN, the word is set; the next launch knows nothing of it."""
+    pos = [40 + 150 * i for i in range(rows)]
+    late = torch.zeros(1, dtype=torch.int32).pin_memory()
+    h, dev, args, h0 = check(ops, 2, 512, 4, 2, 768, 16, pos, late=late)
+    assert int(late) == 0
+    x = h0.to(DEV)
+    ops.decode_chain(x, [dict(d, cache=d["cache"].clone()) for d in dev], *args, late=late, limit_us=3000, absent=2)
+    torch.cuda.synchronize()
+    assert int(late) == 1 and bool(torch.isnan(x).any(1).all())
+    late.zero_()
+    y = h0.to(DEV)
+    dev = on_device(ops, make(ops, 2, 512, 4, 2, 768, 16, pos)[0])
+    ops.decode_chain(y, dev, *args, late=late, limit_us=3000)
+    torch.cuda.synchronize()
+    assert int(late) == 0 and torch.equal(y, h)
+    with pytest.raises(ops.KernelError):
+        ops.decode_chain(y, dev, *args, late=torch.zeros(1, dtype=torch.int32))
 
 
 def test_refuses_what_it_does_not_take(ops):

@@ -41,8 +41,14 @@ TINY_E = dict(
     num_hidden_layers=2, num_attention_heads=4, num_key_value_heads=2, head_dim=128,
     max_position_embeddings=1024, rms_norm_eps=1e-6, rope_theta=1000000.0, tie_word_embeddings=False)
 
+# F: as E, with widths in multiples of 128: in bfloat16 the layers of up to eight single tokens are one launch.
+TINY_F = dict(
+    architectures=["Qwen3ForCausalLM"], vocab_size=400, hidden_size=256, intermediate_size=384,
+    num_hidden_layers=3, num_attention_heads=4, num_key_value_heads=2, head_dim=128,
+    max_position_embeddings=4096, rms_norm_eps=1e-6, rope_theta=1000000.0, tie_word_embeddings=False)
+
 TINY = {"A": (TINY_A, 0, 4), "B": (TINY_B, 1, 8), "C": (TINY_C, 2, 16), "D": (TINY_D, 3, 16),
-        "E": (TINY_E, 4, 16)}   # config, seed, page size
+        "E": (TINY_E, 4, 16), "F": (TINY_F, 5, 16)}   # config, seed, page size
 
 
 def make_folder(tmp, which: str, dtype=torch.bfloat16, norm_std=0.01, std=0.02, scale_qk=None):
