@@ -45,7 +45,8 @@ constexpr unsigned NONE = ~0u;
 constexpr unsigned A_NAN = 0x7fc07fc0u;                    // as a float and as two bfloat16
 constexpr unsigned CLOSED = 0x80000000u;
 constexpr unsigned GAP = 1000000u;                         // of the 100 MHz clock: 10 ms
-constexpr unsigned long CALL = 20000ul;                    // 200 us
+constexpr unsigned long CALL = 5000ul;                     // 50 us
+constexpr unsigned long KILOBYTE = 5ul;                    // 50 ns: what a block takes for one by itself (10 to 29 GB/s a block with 1 to 32 blocks)
 
 typedef unsigned u4 __attribute__((ext_vector_type(4)));
 typedef unsigned u2 __attribute__((ext_vector_type(2)));
@@ -67,6 +68,7 @@ struct ChainArgs {
     int layers, M, H, Hq, Hkv, I, logP, max_blocks, segments, max_position;
     int* late;                         // host memory, or null: 1 once a wait has been given up
     unsigned limit;                    // of a wait, in ticks of the 100 MHz clock
+    long layer_bytes;                  // of a layer's matrices
     int absent;                        // blocks that the roll call counts beside those that come
 };
 
@@ -368,10 +370,21 @@ __global__ __launch_bounds__(THREADS) void decode_chain_kernel(const ChainArgs) 
         int worker = (int)id, workers = 0;
         if (id & CLOSED) {
             worker = -1;
-        } else if (id == 0) {                              // the first comer waits for the others, for a while
-            const unsigned long t0 = __builtin_amdgcn_s_memrealtime();
-            while (__hip_atomic_load(a.work, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < gridDim.x &&
-                   __builtin_amdgcn_s_memrealtime() - t0 < CALL) {}
+        } else if (id == 0) {                              // the first comer waits for the others ...
+            // ... for as long as the step would take longer with those that are there than with all, as which blocks take part is settled for
+            // the whole step.  (Begun after 200 us whoever was there, a step beside a product that leaves 120 of 256 units free for 0.73 ms took
+            // until 4.0 ms, 28 layers of width 1024 and one request, and 5.5, 12 layers and eight requests of 2000 keys; so until 1.25 and 1.2.  Between
+            // products of 7 ms each: 2.3 ms a step, the longest 2.8, 3.0 and 4.8 before; the kernels one after the other wait until the
+            // products are done.)
+            long bytes = a.layer_bytes;
+            for (int m = 0; m < M; ++m) bytes += (long)min(a.positions[m], a.max_position) * (4 * Hkv * D);
+            const unsigned long alone = (unsigned long)a.layers * (bytes >> 10) * KILOBYTE, t0 = __builtin_amdgcn_s_memrealtime();
+            const unsigned grid = gridDim.x;
+            for (;;) {
+                const unsigned come = min(__hip_atomic_load(a.work, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), grid);
+                const unsigned long wait = min(max(CALL, alone / come - alone / grid), (unsigned long)a.limit / 4);
+                if (come == grid || __builtin_amdgcn_s_memrealtime() - t0 >= wait) break;
+            }
             workers = (int)__hip_atomic_fetch_or(a.work, CLOSED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + a.absent;
             __hip_atomic_store(a.work + 16, (unsigned)workers, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         } else {                                           // (the first comer runs and says so soon)
@@ -1145,6 +1158,7 @@ extern "C" int qe_decode_chain(void* h, const void* const* layers, const float* 
     a.layers = n_layers; a.M = M; a.H = H; a.Hq = Hq; a.Hkv = Hkv; a.I = I;
     a.logP = __builtin_ctz(P);
     a.late = late; a.limit = (unsigned)limit_us * 100u; a.absent = absent;
+    a.layer_bytes = 2l * H * ((2l * Hq + 2l * Hkv) * D + 3l * I);
     a.max_blocks = max_blocks; a.segments = chain_segments(max_position); a.max_position = max_position;
     const Exchange ex(M, H, Hq, Hkv, I, a.segments, n_layers);
     const int ring = chain_ring(M, H, Hq, Hkv, I);

@@ -225,6 +225,40 @@ def test_a_wait_in_vain_ends_and_is_told(ops, rows):
         ops.decode_chain(y, dev, *args, late=torch.zeros(1, dtype=torch.int32))
 
 
+def test_beside_a_product_that_holds_half_of_the_chip(ops):
+    """Which blocks take part is settled for the whole step: one that begins while others hold the units waits for them instead of going
+    through all its layers with the few that are free (which took seven times as long as all)."""
+    pos = [2000] * 8
+    layers, table, bt, slots, perm, h0 = make(ops, 1, 1024, 16, 8, 3072, 16, pos)
+    dev = on_device(ops, layers) * 12
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    args = (i32(pos), i32(list(range(8))), bt.to(DEV), slots.to(DEV), 16, D ** -0.5, 2000, 1e-6, table.to(DEV))
+    x, w = torch.ones(1280, 49152, dtype=torch.bfloat16, device=DEV), torch.ones(6144, 49152, dtype=torch.bfloat16, device=DEV)
+    y, h = torch.empty(1280, 6144, dtype=torch.bfloat16, device=DEV), h0.to(DEV)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+
+    def timed(stream, f):
+        begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        with torch.cuda.stream(stream):
+            begin.record()
+            f()
+            end.record()
+        return begin, end
+
+    beside, alone, product = [], [], []
+    for _ in range(4):
+        torch.cuda.synchronize()
+        a = timed(streams[0], lambda: ops.decode_chain(h, dev, *args))
+        torch.cuda.synchronize()
+        b = timed(streams[1], lambda: ops.gemm(x, w, out=y))
+        c = timed(streams[0], lambda: ops.decode_chain(h, dev, *args))
+        torch.cuda.synchronize()
+        for times, (begin, end) in zip((alone, product, beside), (a, b, c)):
+            times.append(begin.elapsed_time(end))
+    # (as soon as the product is done, and then as long as alone: 0.73, 0.55 and 1.2 ms)
+    assert min(beside) < min(product) + 3 * min(alone), (beside, product, alone)
+
+
 def test_refuses_what_it_does_not_take(ops):
     assert not ops.decode_chain_supported(9, 1024, 16, 8, 128, 3072, 16)          # rows
     assert not ops.decode_chain_supported(1, 1024, 16, 8, 64, 3072, 16)           # head size
