@@ -51,11 +51,11 @@ def run_as_chain(blocks, schedule, h: torch.Tensor, ctx, bindings: List[CacheBin
         return False                       # (a position beyond the table: the layers say so)
     layers = []
     for entry, users in zip(schedule, bindings):
-        b, c = blocks[entry.layer], users[0]
+        b = blocks[entry.layer]
         if not (_is(b, PreNormBlock) and _is(b.mixer, PagedAttention) and _is(b.ffn, SwiGLU) and
                 _is(b.mixer_norm, RMSNorm) and _is(b.ffn_norm, RMSNorm)):
             return False
-        m, f = b.mixer, b.ffn
+        m, f, c = b.mixer, b.ffn, users[0]
         if (c.kv is None or not c.write or c.group != g or m.window or m.b_qkv is not None or m.b_o is not None or f.b_gu is not None or
                 not f.interleaved):
             return False
