@@ -2,6 +2,7 @@
 a plain pre-norm block: norm, attention over its own cache, norm, gated feed-forward, without biases or a window."""
 from __future__ import annotations
 
+from types import FunctionType
 from typing import List
 
 import torch
@@ -15,9 +16,22 @@ from .norm import RMSNorm
 from .rope import RotaryHalf
 
 
+def _methods(cls) -> dict:
+    return {name: v for name, v in vars(cls).items() if isinstance(v, (FunctionType, staticmethod, classmethod, property))}
+
+
+# What the chain knows the layers to do is what these classes do as they are written.  Where a program has put something else in the place of
+# one of their methods (a trace, a change of its own), the layers run one by one and call it.
+_WRITTEN = {cls: _methods(cls) for cls in (PreNormBlock, PagedAttention, SwiGLU, RMSNorm, RotaryHalf)}
+
+
+def _as_written() -> bool:
+    return all(_methods(cls) == methods for cls, methods in _WRITTEN.items())
+
+
 def _is(part, cls) -> bool:
-    """A part of this very class, whose forward is the class's."""
-    return type(part) is cls and "forward" not in vars(part)
+    """A part of this very class, with the class's methods."""
+    return type(part) is cls and _WRITTEN[cls].keys().isdisjoint(vars(part))
 
 
 def _of_all_layers(mixer, ffn):
@@ -49,6 +63,8 @@ def run_as_chain(blocks, schedule, h: torch.Tensor, ctx, bindings: List[CacheBin
     table = mix.position.table() if mix.position is not None and same else None
     if same is None or (table is not None and (table.shape[1] != mix.d or ctx.max_position >= table.shape[0])):
         return False                       # (a position beyond the table: the layers say so)
+    if not _as_written():
+        return False
     layers = []
     for entry, users in zip(schedule, bindings):
         b = blocks[entry.layer]

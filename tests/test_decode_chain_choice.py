@@ -11,7 +11,11 @@ from qwen_engine_amd.kernels import ops
 from qwen_engine_amd.parts import DecoderModel, Runtime, expected_tensors
 from qwen_engine_amd.parts.attention import PagedAttention
 from qwen_engine_amd.parts.base import CacheBinding
+from qwen_engine_amd.parts.block import PreNormBlock
 from qwen_engine_amd.parts.chain import run_as_chain
+from qwen_engine_amd.parts.mlp import SwiGLU
+from qwen_engine_amd.parts.norm import RMSNorm
+from qwen_engine_amd.parts.rope import RotaryHalf
 from tiny import TINY_F
 
 CPU = torch.device("cpu")
@@ -42,3 +46,19 @@ def test_a_later_layer_that_keeps_nothing(step):
         pass
     step.blocks[2], step.bindings[2] = Other(), []
     assert not step.run(step) and not step.given
+
+
+@pytest.mark.parametrize("cls,name", [(PagedAttention, "forward"), (PagedAttention, "_project_out"), (SwiGLU, "forward"), (SwiGLU, "activation"),
+                                      (RMSNorm, "forward"), (PreNormBlock, "forward"), (RotaryHalf, "table")])
+@pytest.mark.parametrize("whole_class", [True, False])
+def test_methods_that_a_program_has_replaced(step, monkeypatch, cls, name, whole_class):
+    """A trace put around a method, of all parts of a class or of one, is called: the layers run one by one."""
+    assert step.run(step) and len(step.given) == 1
+    real = getattr(cls, name)
+    if whole_class:
+        monkeypatch.setattr(cls, name, lambda *a, **kw: real(*a, **kw))
+    else:
+        b = step.blocks[1]
+        part = {PagedAttention: b.mixer, SwiGLU: b.ffn, RMSNorm: b.ffn_norm, PreNormBlock: b, RotaryHalf: b.mixer.position}[cls]
+        setattr(part, name, lambda *a, **kw: real(part, *a, **kw))
+    assert not step.run(step) and len(step.given) == 1
