@@ -91,10 +91,7 @@ class PagePool:
         return page
 
     def retain(self, page: int) -> None:
-        self._check_id(page)
-        if self.refcount[page] <= 0:
-            raise CacheError(f"cannot retain page {page}: it is free")
-        self.refcount[page] += 1
+        self.take_over((page,), (False,))
 
     def release(self, page: int, to_free_list: bool = True) -> bool:
         """Drop one reference; True if nobody holds the page any more (it then goes to the free
@@ -110,7 +107,7 @@ class PagePool:
         return False
 
     def take_over(self, pages: Sequence[int], kept: Sequence[bool]) -> None:
-        """``revive`` (for a page that was kept aside) or ``retain`` of many pages."""
+        """One holder more for each of the pages: the first for one that was kept aside, a further one for one that is held."""
         counts = self.refcount
         for page, was_kept in zip(pages, kept):
             if not 0 <= page < self.num_pages:
@@ -118,13 +115,6 @@ class PagePool:
             if (counts[page] != 0) if was_kept else (counts[page] <= 0):
                 raise CacheError(f"page {page} is held: it cannot be revived" if was_kept else f"cannot retain page {page}: it is free")
             counts[page] += 1
-
-    def revive(self, page: int) -> None:
-        """A page that was kept aside with no holder gets its first holder again."""
-        self._check_id(page)
-        if self.refcount[page] != 0:
-            raise CacheError(f"page {page} is held: it cannot be revived")
-        self.refcount[page] = 1
 
     def give_back(self, page: int) -> None:
         """A page that was kept aside with no holder goes to the free list."""

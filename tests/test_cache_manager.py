@@ -61,6 +61,20 @@ def test_reference_counts_refuse_misuse():
         pool.retain(7)
 
 
+def test_pages_taken_over():
+    """Of one admission: pages that others hold, and pages that were kept aside with no holder."""
+    pool = PagePool(4)
+    held, kept, aside = (pool.allocate() for _ in range(3))
+    for page in (kept, aside):
+        assert pool.release(page, to_free_list=False)
+    pool.take_over([held, kept], [False, True])
+    assert [pool.refcount[p] for p in (held, kept, aside)] == [2, 1, 0] and pool.num_free == 1
+    for page, was_kept in ((aside, False), (held, True), (4, True), (-1, False)):
+        with pytest.raises(CacheError):                  # nobody holds it, somebody does, there is no such page
+            pool.take_over([page], [was_kept])
+    assert [pool.refcount[p] for p in (held, kept, aside)] == [2, 1, 0]
+
+
 def test_state_slots():
     s = StateSlots(2)
     a, b = s.take("a"), s.take("b")
