@@ -139,7 +139,7 @@ def load_library():
         "qe_moe_gemm_mfma_supported": [i32],
         "qe_moe_gemm_mfma": [vp, vp, i32, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, f32, f32, i32, i32, vp],
         "qe_decode_chain_supported": [i32, i32, i32, i32, i32, i32, i32],
-        "qe_decode_chain_preferred": [i32, i32, i32, i32, i32, i32, i32],
+        "qe_decode_chain_preferred": [i32, i32, i32, i32, i32, i32, i32, i32],
         "qe_decode_chain_layers": [],
         "qe_decode_chain": [vp, vp, vp, i32, vp, vp, vp, i32, vp, vp, vp, f32, f32, i32, i32, i32, i32, i32, i32, i32, i32, vp, i32, i32, vp, i64, vp],
     }
@@ -1040,9 +1040,10 @@ def decode_chain_supported(rows: int, hidden: int, num_heads: int, num_kv_heads:
     return bool(load_library().qe_decode_chain_supported(rows, hidden, num_heads, num_kv_heads, head_dim, intermediate, page_size))
 
 
-def decode_chain_preferred(rows: int, hidden: int, num_heads: int, num_kv_heads: int, head_dim: int, intermediate: int, page_size: int) -> bool:
-    """True if decode_chain takes such layers and is quicker than their kernels one after the other."""
-    return bool(load_library().qe_decode_chain_preferred(rows, hidden, num_heads, num_kv_heads, head_dim, intermediate, page_size))
+def decode_chain_preferred(rows: int, hidden: int, num_heads: int, num_kv_heads: int, head_dim: int, intermediate: int, page_size: int,
+                           max_position: int = 0) -> bool:
+    """True if decode_chain takes such layers and is quicker than their kernels one after the other, for rows up to max_position."""
+    return bool(load_library().qe_decode_chain_preferred(rows, hidden, num_heads, num_kv_heads, head_dim, intermediate, page_size, int(max_position)))
 
 
 def decode_chain(h: torch.Tensor, layers, positions: torch.Tensor, tok_seq: torch.Tensor, block_table: torch.Tensor,

@@ -57,7 +57,8 @@ def run_as_chain(blocks, schedule, h: torch.Tensor, ctx, bindings: List[CacheBin
     if ex["dec_tokens"] is None or ex["dec_tokens"].shape[0] != T or (ex["other_tokens"] is not None and ex["other_tokens"].shape[0]):
         return False
     kv = bindings[0][0].kv
-    if kv is None or g is None or not ops.decode_chain_preferred(T, h.shape[1], mix.hq, mix.hkv, mix.d, one.ffn.inter, kv.shape[3]):
+    if kv is None or g is None or not ops.decode_chain_preferred(T, h.shape[1], mix.hq, mix.hkv, mix.d, one.ffn.inter, kv.shape[3],
+                                                                 ex["max_dec_position"]):
         return False
     same = _of_all_layers(mix, one.ffn)
     table = mix.position.table() if mix.position is not None and same else None

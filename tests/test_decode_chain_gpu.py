@@ -278,3 +278,19 @@ def test_refuses_what_it_does_not_take(ops):
         ops.decode_chain(h0.to(DEV), [dict(dev[0], w_o=dev[0]["w_o"].float())], i32([5]), i32([0]), bt.to(DEV), None, 2, 0.1, 5)
     with pytest.raises(ops.KernelError):
         ops.decode_chain(h0.to(DEV), [dict(dev[0], k_norm=None)], i32([5]), i32([0]), bt.to(DEV), None, 2, 0.1, 5)
+
+
+@pytest.mark.parametrize("rows,H,Hq,Hkv,I,position,quicker", [
+    # rings of eight kilobytes: many rows, a wide middle, seven or eight queries to a key
+    (3, 2304, 16, 8, 9216, 200, True), (3, 2560, 32, 8, 9728, 200, False), (4, 3072, 24, 3, 8192, 200, False), (4, 2560, 32, 8, 9728, 32000, True),
+    (3, 3072, 24, 8, 12288, 32000, True), (6, 2048, 16, 8, 6144, 200, True),
+    (2, 3072, 28, 4, 12288, 200, True), (1, 3584, 28, 4, 18944, 200, False), (2, 4096, 32, 8, 16384, 200, True), (2, 5120, 40, 8, 14592, 200, False),
+    (1, 4224, 32, 4, 12288, 200, False), (2, 5120, 48, 6, 12288, 200, False), (2, 3584, 28, 7, 18944, 200, False),
+    # of twelve
+    (1, 3584, 28, 7, 18944, 200, True), (2, 5120, 40, 8, 13824, 200, True), (3, 3072, 24, 8, 8192, 200, True), (2, 4096, 32, 8, 12288, 40000, True),
+    # one request with one key/value head
+    (1, 1024, 8, 1, 3072, 45000, True), (1, 1024, 8, 1, 3072, 60000, False), (1, 1024, 4, 1, 3072, 60000, False), (2, 1024, 8, 1, 3072, 120000, True),
+    (1, 1024, 16, 2, 3072, 120000, True), (1, 2048, 8, 1, 6144, 60000, True), (1, 2048, 8, 1, 6144, 120000, False)])
+def test_where_it_is_the_quicker_way(ops, rows, H, Hq, Hkv, I, position, quicker):
+    """Both sides of every line of the rule, at sizes where both ways were measured."""
+    assert ops.decode_chain_preferred(rows, H, Hq, Hkv, 128, I, 16, position) == quicker
