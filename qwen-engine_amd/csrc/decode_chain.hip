@@ -1117,8 +1117,8 @@ extern "C" int qe_decode_chain_supported(int M, int H, int Hq, int Hkv, int head
 //     room for rings of eight, a compute unit has a third less on the way: up to width 2304 that costs less than the starts (2048 with 6144, six rows:
 //     56, 46 and 88, 83; 2304 with 9216, three: 66, 61 and 82, 79), with one or two rows up to 3072 (with 12288 and seven queries to a key, two:
 //     84, 80 and 89, 86), and up to 4096 where the width comes out even, four chunks of K a wave and four fours of outputs a unit (4096 with
-//     16384, two: 133, 116 and 144, 129).  Not beyond: three rows of 2560 with 9728 76, 74 and 92, 94, of 3072 with 12288 84, 84 and 101, 103, but
-//     where one of them has some 24000 keys or more (32000 keys each: 155, 143 and 164, 152; one of 32000, two of 4000: 123, 124); 3584 with 18944 and seven queries to a key, one 122, 122 and 122, 128, two 121, 128 and 126, 135; 4224 with
+//     16384, two: 133, 116 and 144, 129).  Not beyond: three rows of 2560 with 9728 76, 74 and 92, 94, of 3072 with 12288 84, 84 and 101, 103 (at
+//     32000 keys 155, 143 and 164, 152; but which way a row goes, and so its bits, is not to follow how far the rows beside it are); 3584 with 18944 and seven queries to a key, one 122, 122 and 122, 128, two 121, 128 and 126, 135; 4224 with
 //     12288 and eight, two 108, 113; 5120 with 14592, two 136, 144.
 //   * One request with one key/value head up to some 48 keys a number of the width: its keys are cut in 32 segments, which leave most of the chip
 //     idle (width 1024, 45000 keys 47, 46, 64000 53, 56, 120000 76, 85; width 2048, 60000 71, 66, 120000 95, 98).  Two key/value heads: 120000
@@ -1127,8 +1127,7 @@ extern "C" int qe_decode_chain_supported(int M, int H, int Hq, int Hkv, int head
 extern "C" int qe_decode_chain_preferred(int M, int H, int Hq, int Hkv, int head_dim, int I, int P, int max_position) {
     if (!qe_decode_chain_supported(M, H, Hq, Hkv, head_dim, I, P)) return 0;
     if (2.0 * H * ((Hq * 2.0 + 2.0 * Hkv) * head_dim + 3.0 * I) > 600e6 || (M > 2 && H > 3072)) return 0;
-    const int widest = M > 2 ? (max_position < 24576 ? 2304 : 3072) : H % 1024 ? 3072 : 4096;
-    if (chain_ring(M, H, Hq, Hkv, I) == 8 && H > widest) return 0;
+    if (chain_ring(M, H, Hq, Hkv, I) == 8 && H > (M > 2 ? 2304 : H % 1024 ? 3072 : 4096)) return 0;
     return M * Hkv > 1 || max_position / 48 < H;
 }
 

@@ -282,8 +282,8 @@ def test_refuses_what_it_does_not_take(ops):
 
 @pytest.mark.parametrize("rows,H,Hq,Hkv,I,position,quicker", [
     # rings of eight kilobytes: many rows, a wide middle, seven or eight queries to a key
-    (3, 2304, 16, 8, 9216, 200, True), (3, 2560, 32, 8, 9728, 200, False), (4, 3072, 24, 3, 8192, 200, False), (4, 2560, 32, 8, 9728, 32000, True),
-    (3, 3072, 24, 8, 12288, 32000, True), (6, 2048, 16, 8, 6144, 200, True),
+    (3, 2304, 16, 8, 9216, 200, True), (3, 2560, 32, 8, 9728, 200, False), (4, 3072, 24, 3, 8192, 200, False), (4, 2560, 32, 8, 9728, 32000, False),
+    (3, 3072, 24, 8, 12288, 32000, False), (6, 2048, 16, 8, 6144, 200, True),
     (2, 3072, 28, 4, 12288, 200, True), (1, 3584, 28, 4, 18944, 200, False), (2, 4096, 32, 8, 16384, 200, True), (2, 5120, 40, 8, 14592, 200, False),
     (1, 4224, 32, 4, 12288, 200, False), (2, 5120, 48, 6, 12288, 200, False), (2, 3584, 28, 7, 18944, 200, False),
     # of twelve
