@@ -35,7 +35,8 @@ TINY_D = dict(
     max_position_embeddings=1024, rms_norm_eps=1e-6, rope_theta=10000.0, tie_word_embeddings=False)
 
 # E: head size 128, the size of the family's models: in bfloat16 the q|k|v product of a portion norms,
-# rotates and writes the cache in its epilogue, and decode steps run the kernels the large models run.
+# rotates and writes the cache in its epilogue, and decode steps run, layer by layer, the kernels that the family's
+# models run for nine and more tokens (320 is no multiple of 128: never all layers in one launch).
 TINY_E = dict(
     architectures=["Qwen3ForCausalLM"], vocab_size=400, hidden_size=256, intermediate_size=320,
     num_hidden_layers=2, num_attention_heads=4, num_key_value_heads=2, head_dim=128,
