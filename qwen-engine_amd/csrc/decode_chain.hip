@@ -1154,6 +1154,16 @@ extern "C" int qe_decode_chain(void* h, const void* const* layers, const float* 
     for (int l = 0; l < n_layers; ++l) QE_REQUIRE(!layers[9 * l + 6] == !layers[9 * l + 7], "decode chain: a norm of q or of k alone");
     QE_REQUIRE(workspace_bytes >= qe_decode_chain_workspace_bytes(M, H, Hq, Hkv, I, n_layers, max_position),
                "decode chain: workspace of %ld bytes is too small", workspace_bytes);
+    // (three or four rows beyond width 3072 go two by two: a form that held them all spilled 37 registers, and the rule above never picks them)
+    if (M > 2 && H > 3072) {
+        for (int m = 0; m < M; m += 2) {
+            const int rc = qe_decode_chain((float*)h + (long)m * H, layers, eps, n_layers, positions + m, tok_seq + m, block_table, max_blocks, shared_keys,
+                                           slots ? slots + m : nullptr, rope, qk_eps, scale, min(2, M - m), H, Hq, Hkv, I, P, max_position, units, late,
+                                           limit_us, absent, workspace, workspace_bytes, stream);
+            if (rc) return rc;
+        }
+        return 0;
+    }
     ChainArgs a{};
     for (int l = 0; l < n_layers; ++l) {
         const void* const* p = layers + 9 * l;
@@ -1192,10 +1202,11 @@ extern "C" int qe_decode_chain(void* h, const void* const* layers, const float* 
     do {                                                                                      \
         if (H <= 1024) QE_CHAIN2(MV_, 1);                                                     \
         else if (H <= 2048) QE_CHAIN2(MV_, 2);                                                \
-        else if (H <= 3072) QE_CHAIN2(MV_, 3);                                                \
-        else QE_CHAIN2(MV_, 5);                                                               \
+        else QE_CHAIN2(MV_, 3);                                                               \
     } while (0)
-    if (M == 1) QE_CHAIN(1);
+    if (M == 1 && H > 3072) QE_CHAIN2(1, 5);
+    else if (M == 2 && H > 3072) QE_CHAIN2(2, 5);
+    else if (M == 1) QE_CHAIN(1);
     else if (M == 2) QE_CHAIN(2);
     else if (M <= 4) QE_CHAIN(4);
     else if (H <= 1024) QE_CHAIN2(8, 1);

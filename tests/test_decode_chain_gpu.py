@@ -116,7 +116,8 @@ def test_edges_of_tiles_segments_and_pages(ops, pos, Hq, Hkv, P):
 
 
 @pytest.mark.parametrize("H,Hq,Hkv,I,rows", [(128, 1, 1, 128, 1), (1024, 16, 8, 3072, 8), (1152, 9, 3, 2048, 3), (2048, 16, 8, 6144, 6), (2176, 8, 8, 640, 4),
-                                             (4096, 32, 8, 12288, 1), (2560, 32, 8, 9728, 2), (2560, 32, 8, 9728, 4), (5120, 40, 8, 17408, 1), (1024, 4, 4, 12800, 3)])
+                                             (4096, 32, 8, 12288, 1), (2560, 32, 8, 9728, 2), (2560, 32, 8, 9728, 4), (5120, 40, 8, 17408, 1), (1024, 4, 4, 12800, 3),
+                                             (4096, 32, 8, 12288, 3)])
 def test_widths(ops, H, Hq, Hkv, I, rows):
     """Products whose chunks of K do not come out even, shares that differ from block to block, both sizes of the rings."""
     assert ops.decode_chain_supported(rows, H, Hq, Hkv, D, I, 16)
