@@ -106,11 +106,12 @@ struct Exchange {
 };
 
 // A token's keys are cut in segments by its own position alone, so that its sums, and its bits, are the same alone and in company: of 128 keys, a
-// tile for each feeding wave, up to 16 of them; from 2048 keys on of 256, up to 32; then of as many 128s as make 32 at most.  More and
-// smaller segments suit one row, which has the chip to itself, fewer and larger ones eight, whose units are several a block (us a layer, width 1024
-// with 8 key/value heads, one row and eight rows of 2000 keys: segments of 128 20.8 and 42.1, of 256 22.6 and 40.2; of 4000: 128 23.2 and 57.7,
-// 256 24.2 and 54.0; of 16000: 512 31.1 and 117, 1024 39 and 116).
-__host__ __device__ constexpr int segment_keys(int p) { return 128 * (p < 2048 ? 1 : p < 8192 ? 2 : p / 4096 + 1); }
+// tile for each feeding wave, up to 20 of them; from 2560 keys on of 256, up to 32; then of as many 128s as make 32 at most.  More and
+// smaller segments suit one row, which has the chip to itself, fewer and larger ones eight, whose units are several a block (us a step of 28 layers,
+// width 1024 with 8 key/value heads, segments of 128 and of 256: at 2100 keys one row 648, 694, two 782, 770, four 978, 1005, eight 1327, 1332; at 2600
+// one 663, 701, two 793, 783, four 1000, 1015, eight 1417, 1353; at 3900 one 683, 708, eight 1659, 1572.  us a layer, at 16000: 512 and 1024 keys, one
+// row 31.1, 39, eight 117, 116).
+__host__ __device__ constexpr int segment_keys(int p) { return 128 * (p < 2560 ? 1 : p < 8192 ? 2 : p / 4096 + 1); }
 
 // A unit of the attention: the cached keys [lo, hi) of one segment for one row and key/value head; own: the token's own key belongs to it.
 struct Unit { int m, kvh, seg, lo, hi, tiles, own; };
@@ -1078,7 +1079,7 @@ __global__ __launch_bounds__(256) void decode_chain_clear_kernel(u4* work, unsig
 
 int chain_segments(int max_position) {
     const int small = max_position / 128 + 1, large = max_position / 256 + 1;      // (segment_keys() for all positions up to it)
-    return max(min(small, 16), min(large, MAX_SEGMENTS));
+    return max(min(small, 20), min(large, MAX_SEGMENTS));
 }
 
 // Shared memory for rings of `ring` kilobytes.

@@ -154,9 +154,9 @@ def test_traces(folder, plain, launches, tmp_path):
     assert {1, 2, 3, 4} <= set(launches) and max(launches) <= 8
 
 
-@pytest.mark.parametrize("start", [1010, 2038])
+@pytest.mark.parametrize("start", [1010, 2038, 2550])
 def test_across_the_positions_where_the_recorded_step_and_the_segments_change(model, plain, launches, start):
-    """Recorded steps are kept for positions up to multiples of 1024, and a token's keys are cut otherwise from 2048 on."""
+    """Recorded steps are kept for positions up to multiples of 1024, and a token's keys are cut otherwise from 2560 on."""
     from qwen_engine_amd.engine import StepEntry
     tokens = prompt_of(start + 24, seed=start)
     want = plain(tokens)[start:]
@@ -165,7 +165,7 @@ def test_across_the_positions_where_the_recorded_step_and_the_segments_change(mo
     runner.step([StepEntry("r", tokens[:start], [])])
     got = torch.cat([runner.step([StepEntry("r", tokens[i:i + 1], [0])]) for i in range(start, len(tokens))]).cpu()
     assert float((got - want).abs().max()) <= TOL * float(want.abs().max())
-    assert len(launches) >= 4 and set(launches) == {1}          # two recorded steps, each run once before
+    assert len(launches) >= (2 if start == 2550 else 4) and set(launches) == {1}          # one or two recorded steps, each run once before
 
 
 def test_requests_that_share_pages(model, launches):

@@ -183,7 +183,7 @@ def test_the_same_bits_again_recorded_and_on_two_streams(ops):
 def test_a_token_alone_and_in_company(ops, H, Hq, Hkv, I):
     """A row's bits, and those of the key and value it writes, follow neither the rows beside it nor the number of blocks: positions at
     both sides of where the segments' length changes, and rows whose units are dealt to one block and to many."""
-    pos = [2047, 0, 130, 8191, 700, 2048, 8192, 16500]
+    pos = [2559, 0, 130, 8191, 700, 2560, 8192, 16500]
     layers, table, bt, slots, perm, h0 = make(ops, 2, H, Hq, Hkv, I, 16, pos, seed=9)
     fresh = on_device(ops, layers)
     i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
