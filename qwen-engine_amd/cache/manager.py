@@ -97,10 +97,14 @@ class PagePool:
     def release(self, page: int, to_free_list: bool = True) -> bool:
         """Drop one reference; True if nobody holds the page any more (it then goes to the free
         list, unless the caller keeps it aside)."""
-        unheld = self.let_go((page,))[0] == 0
-        if unheld and to_free_list:
-            self.free.append(page)
-        return unheld
+        return bool(self.release_all((page,)) if to_free_list else self.let_go((page,))[0] == 0)
+
+    def release_all(self, pages: Sequence[int]) -> List[int]:
+        """let_go(), and those that nobody holds any more go to the free list, in their order; which."""
+        left = self.let_go(pages)
+        freed = list(compress(pages, map((0).__eq__, left))) if any(left) else list(pages)
+        self.free.extend(freed)
+        return freed
 
     def let_go(self, pages: Sequence[int]) -> List[int]:
         """One holder less for each of the pages, all of them different, none of which goes to the free list by that; how many each has left."""
@@ -265,26 +269,28 @@ class CacheManager:
 
     def free_request(self, req_id: Hashable) -> None:
         rc = self.get(req_id)
+        tables = rest = rc.tables
         if self.keep_freed:
             # registered pages go index by index, the pages of all groups together: an entry that
             # nobody holds any more is kept instead of freed
-            tables, shared = rc.tables, self._shared
+            shared = self._shared
             hashes = list(map(self._page_hash.get, tables[0]))     # (-1, no page, is never registered)
-            mine = [h in shared for h in hashes]
+            mine = list(map(shared.__contains__, hashes))
             if len(tables) > 1:
                 mine = [m and all(i < len(t) and t[i] == page for t, page in zip(tables, shared[hashes[i]].pages)) for i, m in enumerate(mine)]
             left = [pool.let_go(list(compress(t, mine))) for pool, t in zip(self.pools, tables)]
             if any(n != left[0] for n in left):
                 raise CacheError("the pages of a shared entry have different counts")
-            kept = [h for h, n in zip(compress(hashes, mine), left[0]) if n == 0]
-            for h in reversed(kept):               # the request's last page first: it is the first to go
-                self._kept[h] = shared[h]
-            for t in tables:
-                t[:len(mine)] = [-1 if m else page for m, page in zip(mine, t)]
-        for g, table in enumerate(rc.tables):
-            for page in [p for p in table if p >= 0]:
-                self._release(g, page)
-            table.clear()
+            kept = list(compress(hashes, mine))
+            if any(left[0]):
+                kept = [h for h, n in zip(kept, left[0]) if n == 0]
+            kept.reverse()                         # the request's last page first: it is the first to go
+            self._kept.update(zip(kept, map(shared.__getitem__, kept)))
+            others = [not m for m in mine]
+            rest = [list(compress(t, others)) + t[len(mine):] for t in tables]
+        for g, pages in enumerate(rest):
+            self._release(g, [page for page in pages if page >= 0])
+            tables[g].clear()
         self.slots.give_back(rc.state_slot)
         del self.requests[req_id]
 
@@ -397,19 +403,21 @@ class CacheManager:
                 continue
             live_from = min(self._first_live_page(g, new_len), len(table))
             kept = self.kept_first_pages(g)                # (the pages of the kept first positions never go back)
-            for i in range(max(rc.released[g], kept), live_from):   # pages below rc.released[g] went back earlier
-                if table[i] >= 0:
-                    self._release(g, table[i])
+            passed = [i for i in range(max(rc.released[g], kept), live_from) if table[i] >= 0]   # (below rc.released[g] they went back earlier)
+            if passed:
+                self._release(g, [table[i] for i in passed])
+                for i in passed:
                     table[i] = -1
-                    rc.dirty[g].append(i)
+                rc.dirty[g].extend(passed)
             rc.released[g] = max(rc.released[g], live_from)
 
-    def _release(self, g: int, page: int) -> None:
-        if self.pools[g].release(page):
-            self.stats["pages_freed"] += 1
-            if self.track_pages:
-                self._page_events.append((g, page))
-            if g == 0:
+    def _release(self, g: int, pages: List[int]) -> None:
+        freed = self.pools[g].release_all(pages)
+        self.stats["pages_freed"] += len(freed)
+        if self.track_pages:
+            self._page_events.extend((g, page) for page in freed)
+        if g == 0 and self._page_hash:
+            for page in freed:
                 h = self._page_hash.pop(page, None)
                 if h is not None:
                     self._unregister(h)

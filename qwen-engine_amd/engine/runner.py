@@ -158,8 +158,9 @@ class ModelRunner:
         self.shared_keys = torch.zeros(max_requests + 1, dtype=torch.int32, device=dev)
         self._shared_keys_host = [0] * (max_requests + 1)
         # what kernels write to whose blocks waited for each other in vain (StepContext.late)
-        self._late = torch.zeros(1, dtype=torch.int32).pin_memory()
-        self._late_np = self._late.numpy()
+        # (bfloat16 only, as those kernels: pinning it takes some 3 ms)
+        self._late = torch.zeros(1, dtype=torch.int32).pin_memory() if dt == torch.bfloat16 else None
+        self._late_np = np.zeros(1, dtype=np.int32) if self._late is None else self._late.numpy()
         # positions that a row standing on the spare row may have: inside every group's table row, and the model's
         self._spare_positions = min([w * page_size for w in self.table_width] + [model.spec.max_positions])
         # a part with per-request state is recorded into graphs only if it says that it can be
