@@ -275,7 +275,7 @@ class CacheManager:
             # nobody holds any more is kept instead of freed
             shared = self._shared
             hashes = list(map(self._page_hash.get, tables[0]))     # (-1, no page, is never registered)
-            mine = list(map(shared.__contains__, hashes))
+            mine = [h is not None for h in hashes]
             if len(tables) > 1:
                 mine = [m and all(i < len(t) and t[i] == page for t, page in zip(tables, shared[hashes[i]].pages)) for i, m in enumerate(mine)]
             left = [pool.let_go(list(compress(t, mine))) for pool, t in zip(self.pools, tables)]
