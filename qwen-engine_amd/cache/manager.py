@@ -238,7 +238,7 @@ class CacheManager:
             all(g.window is None for g in self.groups)
         self._shared: Dict[int, _SharedEntry] = {}
         # the same by what an admission goes along: the hash of the page before and the page's tokens, so that it makes no page's
-        # hash again (64 requests with 64 shared pages each: 11.4 ms on the host, now 5.8; their release 3.8 and 2.5)
+        # hash again (64 requests with 64 shared pages each: 11.4 ms on the host, now 5.8; their release 3.6 and 2.4)
         self._behind: Dict[Tuple[int, bytes], _SharedEntry] = {}
         self._page_hash: Dict[int, int] = {}   # page id of group 0 -> hash it is registered under
         self.keep_freed = bool(keep_freed_prefixes) and self.prefix_sharing

@@ -13,9 +13,11 @@
 //     publish the products' results.
 //
 // A step of 28 layers (16 heads of 128 on 8, width 1024), logits and all, with six kernels a layer and so, in us: one request at 64 keys
-// 914, 590; at 8192 1088, 785; four at 128 1010, 706; eight at 1024 1250, 1058; eight at 12288 3086, 2861.  Of six layers of width 4096 with
-// 12288 in the middle 853, 711 (one request at 512 keys).  What is left above the bytes is the waiting: of some 20 us a layer of one request
-// 14 are the same without any weights, and a look for numbers stands behind the kilobytes that its compute unit has asked for before.
+// 919, 600; at 2000 922, 643; at 8192 1129, 784; four at 128 1070, 757; eight at 1024 1324, 1128; at 4000 1746, 1586; at 12288 3310, 2967.  Of six
+// layers of width 4096 with 12288 in the middle, at 512 keys, one request 873, 715, two 878, 744.  What is left above the bytes is the waiting: with
+// the same kilobyte asked for again and again in the place of all weights and keys, a layer (of the first model) takes 14.5 us instead of 16.3 with one
+// request at 64 keys, 14.9 instead of 17.2 at 2040, and eight at 4000 take 35.5 instead of 50.7.  A look for numbers stands behind the
+// kilobytes that its compute unit has asked for before.
 //
 // A number that is not there yet is told by its bits: every place of the exchange holds ~0 (a NaN that no result has: a result of these
 // bits is published as another NaN) until its one writer fills it, and every reader asks until nothing is ~0.  So nothing beyond the
@@ -1119,8 +1121,9 @@ extern "C" int qe_decode_chain_supported(int M, int H, int Hq, int Hkv, int head
 //     56, 46 and 88, 83; 2304 with 9216, three: 66, 61 and 82, 79), with one or two rows up to 3072 (with 12288 and seven queries to a key, two:
 //     84, 80 and 89, 86), and up to 4096 where the width comes out even, four chunks of K a wave and four fours of outputs a unit (4096 with
 //     16384, two: 133, 116 and 144, 129).  Not beyond: three rows of 2560 with 9728 76, 74 and 92, 94, of 3072 with 12288 84, 84 and 101, 103 (at
-//     32000 keys 155, 143 and 164, 152; but which way a row goes, and so its bits, is not to follow how far the rows beside it are); 3584 with 18944 and seven queries to a key, one 122, 122 and 122, 128, two 121, 128 and 126, 135; 4224 with
-//     12288 and eight, two 108, 113; 5120 with 14592, two 136, 144.
+//     32000 keys 155, 143 and 164, 152; but which way a row goes, and so its bits, is not to follow how far the rows beside it are); 3584 with
+//     18944 and seven queries to a key, one 122, 122 and 122, 128, two 121, 128 and 126, 135; 4224 with 12288 and eight, two 108, 113; 5120
+//     with 14592, two 136, 144.
 //   * One request with one key/value head up to some 48 keys a number of the width: its keys are cut in 32 segments, which leave most of the chip
 //     idle (width 1024, 45000 keys 47, 46, 64000 53, 56, 120000 76, 85; width 2048, 60000 71, 66, 120000 95, 98).  Two key/value heads: 120000
 //     keys 89, 87.
