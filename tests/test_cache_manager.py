@@ -75,6 +75,19 @@ def test_pages_taken_over():
     assert [pool.refcount[p] for p in (held, kept, aside)] == [2, 1, 0]
 
 
+def test_pages_let_go_together():
+    """Those that nobody holds any more go to the free list, in their order; a list with a wrong page in it changes nothing."""
+    pool = PagePool(5)
+    a, b, c = (pool.allocate() for _ in range(3))
+    pool.retain(b)
+    for wrong in (3, 5, -1):                             # it is free, there is no such page
+        with pytest.raises(CacheError):
+            pool.release_all([a, b, wrong])
+    assert [pool.refcount[p] for p in (a, b, c)] == [1, 2, 1] and pool.num_free == 2
+    assert pool.release_all([c, b, a]) == [c, a] and pool.free[-2:] == [c, a] and pool.refcount[b] == 1
+    assert pool.release_all([]) == [] and pool.release(b) and pool.num_free == 5
+
+
 def test_state_slots():
     s = StateSlots(2)
     a, b = s.take("a"), s.take("b")
