@@ -332,6 +332,54 @@ struct NormRotate {
     }
 };
 
+// The token's own key: its score from q and the key as normed and turned.
+template <int D>
+__device__ __forceinline__ float own_score(const bf16x8 (&qreg)[D / 32], const bf16x8 (&kreg)[D / 32]) {
+    float dot = 0.f;
+#pragma unroll
+    for (int c = 0; c < D / 32; ++c)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dot += (float)qreg[c][e] * (float)kreg[c][e];
+    dot += __shfl_xor(dot, 16, 64);
+    dot += __shfl_xor(dot, 32, 64);
+    return dot;
+}
+// It joins a running maximum and sum: its weight, rounded, and the factor for what was summed before it
+// (the roundings are written out: one wave and four do the same).
+__device__ __forceinline__ float own_weight(float dot, float scale, int g, float& m, float& l, float& alpha) {
+    const float mn = fmaxf(m, dot * scale);
+    alpha = __expf(m - mn);                                // 0 when no cached key was seen
+    const float pn = __expf(__builtin_fmaf(dot, scale, -mn));
+    l = __builtin_fmaf(l, alpha, g == 0 ? pn : 0.f);       // (a lane's share of the sum: once per column)
+    m = mn;
+    return (float)(__bf16)pn;
+}
+__device__ __forceinline__ void add_own(floatx4& acc, float alpha, float weight, const short4_t& vv) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] = __builtin_fmaf(weight, bf16_bits_to_float((unsigned short)vv[j]), acc[j] * alpha);
+}
+// Key and value go to the cache.
+template <int D>
+__device__ __forceinline__ void store_own(bf16_t* cache, const bf16x8 (&kreg)[D / 32], const bf16_t* vsrc, int slot, long page_stride,
+                                          int kvh, int Hkv, int P, int g, int n) {
+    if (slot < 0) return;
+    const long page = slot / P;
+    const int off = slot % P;
+    if (n == 0) {
+#pragma unroll
+        for (int c = 0; c < D / 32; ++c)
+            *(bf16x8*)(cache + page * page_stride + ((long)kvh * P + off) * D + c * 32 + g * 8) = kreg[c];
+    }
+    if (n < D / 16) {                                      // the value tile is [D][P]: a column of single elements
+        bf16_t* vt = cache + page * page_stride + ((long)(Hkv + kvh) * P) * D + off;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int d = n * 16 + g * 4 + j;
+            vt[(long)d * P] = vsrc[d];
+        }
+    }
+}
+
 // AHEAD: how many tiles the loads of a whole split run ahead of the computation.  A wave with one
 // tile in flight gets 8 KB per trip to memory (about 0.7 us); that is enough when the chip holds
 // two waves or more per SIMD, whose loads together keep the memory busy, and far too little for one
@@ -374,51 +422,6 @@ __global__ __launch_bounds__(64 * (W > 1 ? W + 1 : 1)) void attention_decode_fus
 
     bf16x8 qreg[D / 32];
     bf16x8 kreg[D / 32];                                   // the token's own key, normed and turned
-    // its score
-    const auto own_score = [&]() {
-        float dot = 0.f;
-#pragma unroll
-        for (int c = 0; c < D / 32; ++c)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) dot += (float)qreg[c][e] * (float)kreg[c][e];
-        dot += __shfl_xor(dot, 16, 64);
-        dot += __shfl_xor(dot, 32, 64);
-        return dot;
-    };
-    // the key and the value to the cache
-    const auto store_own = [&]() {
-        const int slot = slots ? slots[t] : -1;
-        if (slot < 0) return;
-        const long page = slot / P;
-        const int off = slot % P;
-        if (n == 0) {
-#pragma unroll
-            for (int c = 0; c < D / 32; ++c)
-                *(bf16x8*)(cache + page * page_stride + ((long)kvh * P + off) * D + c * 32 + g * 8) = kreg[c];
-        }
-        if (n < D / 16) {                                  // the value tile is [D][P]: a column of single elements
-            bf16_t* vt = cache + page * page_stride + ((long)(Hkv + kvh) * P) * D + off;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int d = n * 16 + g * 4 + j;
-                vt[(long)d * P] = vsrc[d];
-            }
-        }
-    };
-    // the own key's score joins a running maximum and sum: its weight, rounded, and the factor for what was summed before it
-    // (the roundings are written out: one wave and four do the same)
-    const auto own_weight = [&](float dot, float& m, float& l, float& alpha) {
-        const float mn = fmaxf(m, dot * scale);
-        alpha = __expf(m - mn);                            // 0 when no cached key was seen
-        const float pn = __expf(__builtin_fmaf(dot, scale, -mn));
-        l = __builtin_fmaf(l, alpha, g == 0 ? pn : 0.f);   // (a lane's share of the sum: once per column)
-        m = mn;
-        return (float)(__bf16)pn;
-    };
-    const auto add_own = [&](floatx4& acc, float alpha, float weight, const short4_t& vv) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[j] = __builtin_fmaf(weight, bf16_bits_to_float((unsigned short)vv[j]), acc[j] * alpha);
-    };
     const int tile0 = (k_begin - split * SPLIT) / 16;
     const int tile1 = k_begin < k_end ? (k_end - split * SPLIT + 15) / 16 : tile0;
     int my_page = 0;
@@ -446,11 +449,11 @@ __global__ __launch_bounds__(64 * (W > 1 ? W + 1 : 1)) void attention_decode_fus
             }
             __syncthreads();
             if (owns) {
-                const float dot = own_score();
+                const float dot = own_score<D>(qreg, kreg);
                 if (g == 0) own_dot[n] = dot;
             }
             __syncthreads();
-            if (owns) store_own();
+            if (owns) store_own<D>(cache, kreg, vsrc, slots ? slots[t] : -1, page_stride, kvh, Hkv, P, g, n);
             return;
         }
         const auto first_key = [&](int i) { return split * SPLIT + (tile0 + i) * 16; };
@@ -483,7 +486,7 @@ __global__ __launch_bounds__(64 * (W > 1 ? W + 1 : 1)) void attention_decode_fus
             }
             if (owns) {
                 float alpha;
-                const float weight = own_weight(own_dot[n], m, l, alpha);
+                const float weight = own_weight(own_dot[n], scale, g, m, l, alpha);
 #pragma unroll
                 for (int b = 0; b < NV; ++b) add_own(acc[b], alpha, weight, vv[b]);
             }
@@ -546,12 +549,11 @@ __global__ __launch_bounds__(64 * (W > 1 ? W + 1 : 1)) void attention_decode_fus
         NormRotate<D> nk;
         nk.fetch(qkv + t * width + (long)(Hq + kvh) * D, true, k_w, cs, g);
         nk.finish(kreg, k_w != nullptr, eps, cs != nullptr);
-        const float dot = own_score();
         float alpha;
-        const float weight = own_weight(dot, st.m, st.l, alpha);
+        const float weight = own_weight(own_score<D>(qreg, kreg), scale, g, st.m, st.l, alpha);
 #pragma unroll
         for (int db = 0; db < D / 16; ++db) add_own(st.acc[db], alpha, weight, *(const short4_t*)(vsrc + db * 16 + g * 4));
-        store_own();
+        store_own<D>(cache, kreg, vsrc, slots ? slots[t] : -1, page_stride, kvh, Hkv, P, g, n);
     }
     float l = st.l;
     const float m = st.m;
@@ -562,6 +564,150 @@ __global__ __launch_bounds__(64 * (W > 1 ? W + 1 : 1)) void attention_decode_fus
         for (int db = 0; db < D / 16; ++db)
             *(floatx4*)(pacc + db * 16 + g * 4) = st.acc[db];
         if (g == 0) { pml[0] = m; pml[1] = l; }
+    }
+}
+
+// ---- a block a token and key/value head ---------------------------------------------------------
+// With tokens enough to give every compute unit a block, a token's keys are one block's: W waves take its tiles in turn, each with a
+// softmax of its own, and join them in shared memory, so that a walk's start (positions, table, pages, q: some 4 us before the first
+// key is there) is paid once and not for every 128 keys, nothing partial goes through memory and no second kernel waits for the
+// last block.  Where the tokens are too few for that, the keys go in segments (of whole tiles, cut at absolute positions), which the
+// merge kernel below joins.
+// FUSED: from the q|k|v rows, as the kernel above; the last wave takes the token's own key.
+template <int D, int W, bool FUSED>
+__global__ __launch_bounds__(64 * W, W == 4 ? (FUSED ? 2 : 3) : 1) void attention_decode_block_kernel(
+    const bf16_t* __restrict__ q, bf16_t* cache, const int* __restrict__ dec_tokens, const int* __restrict__ positions,
+    const int* __restrict__ tok_seq, const int* __restrict__ block_table, int max_blocks, const int* __restrict__ shared_keys,
+    const int* __restrict__ slots, const float* __restrict__ q_w, const float* __restrict__ k_w, float eps, const float* __restrict__ table,
+    bf16_t* __restrict__ out, float* __restrict__ part_acc, float* __restrict__ part_ml,
+    int Hq, int Hkv, int P, float scale, int window, int segments, int seg_keys, AttnTail tail) {
+    constexpr int ROW = D + 4;                             // floats of a wave's result for a head in shared memory
+    extern __shared__ __attribute__((aligned(16))) float joined[];
+    const int lane = threadIdx.x & 63, g = lane >> 4, n = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int seg = blockIdx.x, kvh = blockIdx.y, di = blockIdx.z;
+    const int G = Hq / Hkv;
+    const int t = dec_tokens ? dec_tokens[di] : di;       // (no list: every row, in order)
+    const int p = positions[t], row = tok_seq[t];
+    const int last = FUSED ? p : p + 1;                    // the cached keys end here
+    const int lo = first_seen_key(p, window);
+    const int k_begin = max(seg * seg_keys, lo);
+    const int k_end = min((seg + 1) * seg_keys, last);
+    const bool owns = FUSED && seg == p / seg_keys;        // this block takes the token's own key and value
+    const int head = kvh * G + n;
+    const bool head_ok = n < G;
+    if (k_begin >= k_end && !owns) {                       // nothing of this segment is seen by the token (never if it is the only one)
+        if (wave == 0 && head_ok && g == 0) {
+            float* pml = part_ml + (((long)di * Hq + head) * segments + seg) * 2;
+            pml[0] = -INFINITY;
+            pml[1] = 0.f;
+        }
+        return;
+    }
+    const long page_stride = 2L * Hkv * P * D;
+    const int* bt = block_table + (long)row * max_blocks;
+    const int shared = shared_keys ? shared_keys[row] : 0;
+    // the wave's i-th tile is the segment's (wave + W i)-th; lane l holds the page and the place of the (i0 + l)-th
+    const int first = k_begin / 16 + wave, tiles = k_begin < k_end ? max(0, ((k_end + 15) / 16 - first + W - 1) / W) : 0;
+    int my_page = 0, my_place = 0;
+    const auto look_up = [&](int i0) {
+        const int key = (first + (i0 + lane) * W) * 16;
+        if (i0 + lane < tiles) my_page = bt[key / P];
+        my_place = key % P;
+    };
+    look_up(0);
+    bf16x8 qreg[D / 32];
+    const long width = FUSED ? (long)(Hq + 2 * Hkv) * D : (long)Hq * D;
+    const float* cs = FUSED && table ? table + (long)p * D : nullptr;
+    [[maybe_unused]] NormRotate<D> nq;
+    if constexpr (FUSED) {
+        nq.fetch(q + t * width + (long)head * D, head_ok, q_w, cs, g);
+    } else {
+        const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int c = 0; c < D / 32; ++c) qreg[c] = head_ok ? *(const bf16x8*)(q + t * width + (long)head * D + c * 32 + g * 8) : zero8;
+    }
+    AttnState<D> st;
+    st.init();
+    KVTile<D> ta, tb;
+#define LOAD(buf_, i_) load_tile<D>(buf_, cache, __builtin_amdgcn_readlane(my_page, (i_) & 63), page_stride, kvh, Hkv, P, \
+                                    __builtin_amdgcn_readlane(my_place, (i_) & 63), g, n, (first + (i_) * W) * 16 >= shared)
+#define STEP(buf_, i_) attn_tile_step<D>(st, buf_, qreg, scale, (first + (i_) * W) * 16, g, k_begin, k_end, k_begin, k_end)
+    if (tiles > 0) LOAD(ta, 0);
+    if (tiles > 1) LOAD(tb, 1);
+    if constexpr (FUSED) nq.finish(qreg, q_w != nullptr, eps, cs != nullptr);
+    for (int i = 0; i < tiles;) {
+        STEP(ta, i);
+        if (i + 2 < tiles) {
+            if ((i + 2) % 64 == 0) look_up(i + 2);         // (the tile after the next begins 64 others; the next one's loads are on their way)
+            LOAD(ta, i + 2);
+        }
+        if (++i >= tiles) break;
+        STEP(tb, i);
+        if (i + 2 < tiles) LOAD(tb, i + 2);
+        ++i;
+    }
+#undef LOAD
+#undef STEP
+    if constexpr (FUSED) {
+        if (owns && wave == W - 1) {
+            const bf16_t* vsrc = q + t * width + (long)(Hq + Hkv + kvh) * D;
+            bf16x8 kreg[D / 32];
+            NormRotate<D> nk;
+            nk.fetch(q + t * width + (long)(Hq + kvh) * D, true, k_w, cs, g);
+            short4_t vv[D / 16];
+#pragma unroll
+            for (int db = 0; db < D / 16; ++db) vv[db] = *(const short4_t*)(vsrc + db * 16 + g * 4);
+            nk.finish(kreg, k_w != nullptr, eps, cs != nullptr);
+            float alpha;
+            const float weight = own_weight(own_score<D>(qreg, kreg), scale, g, st.m, st.l, alpha);
+#pragma unroll
+            for (int db = 0; db < D / 16; ++db) add_own(st.acc[db], alpha, weight, vv[db]);
+            store_own<D>(cache, kreg, vsrc, slots ? slots[t] : -1, page_stride, kvh, Hkv, P, g, n);
+        }
+    }
+    float l = st.l;
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    float* const ml = joined + W * G * ROW;
+    if (head_ok) {
+        float* acc = joined + (wave * G + n) * ROW;
+#pragma unroll
+        for (int db = 0; db < D / 16; ++db) *(floatx4*)(acc + db * 16 + g * 4) = st.acc[db];
+        if (g == 0) {
+            ml[(wave * G + n) * 2] = st.m;
+            ml[(wave * G + n) * 2 + 1] = l;
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < G * D; i += 64 * W) {
+        const int j = i / D, d = i % D;
+        float m[W], s[W], o[W], top = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            m[w] = ml[(w * G + j) * 2];
+            s[w] = ml[(w * G + j) * 2 + 1];
+            o[w] = joined[(w * G + j) * ROW + d];
+        }
+#pragma unroll
+        for (int w = 0; w < W; ++w) top = fmaxf(top, m[w]);
+        float sum = 0.f, x = 0.f;
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            const float e = __expf(m[w] - top);            // (0 of a wave that had no tile)
+            sum += e * s[w];
+            x += e * o[w];
+        }
+        if (segments == 1) {
+            tail.store(out, t, kvh * G + j, d, x * (1.f / sum));   // (as the merge of one segment has it)
+        } else {
+            const long at = ((long)di * Hq + kvh * G + j) * segments + seg;
+            part_acc[at * D + d] = x;
+            if (d == 0) {
+                part_ml[at * 2] = top;
+                part_ml[at * 2 + 1] = sum;
+            }
+        }
     }
 }
 
@@ -648,20 +794,57 @@ size_t qe_attention_decode_workspace(int n_dec, int Hq, int D, int num_splits) {
     return (size_t)n_dec * Hq * num_splits * (D + 2) * sizeof(float);
 }
 
+// The segments of a block's form: 0 (the splits are the better way), else how many, of seg_keys keys each.  (us, 16 heads of 128 on 8, rows of half to
+// one and a half times the keys; splits of 128 and their merge, then blocks of four waves.  In one segment: 16 rows of 200 keys 18.2, 12.4, of 400
+// 18.3, 16.0; 24 of 400 20.7, 15.2; 64 of 200 37.4, 14.9, of 400 42.4, 26.2, of 1030 75.1, 57.4, of 2000 115, 107; of 1030 with 64 heads
+// 83.7, 60.1.  Cut: 9 rows of 1900 22.8, 22.8 (7 segments), of 3800 40.6, 38.6; 16 of 1040 25.2, 21.5 (4; in one 27.5), of 4000 63.6, 57.7; 24 of
+// 4000 87.2, 79.7 (5; in one 93.7); 32 of 4000 113, 106 (2; in one 112).  Four rows of 400 13.0, 13.4, of 1000 14.3, 16.0, of 2000 16.2, 16.4: up to eight
+// tokens are the splits'.)  Up to 16 tokens, which every other kernel of their step takes in one order, a token's segments follow its own position
+// alone: its bits are the same beside any others.
+static int block_segments(int n_dec, int Hkv, int max_position, int window, int sink, float softcap, int& seg_keys) {
+    if (n_dec <= 8 || window != 0 || sink || softcap > 0.f) return 0;
+    int segments = max_position / 512 + 1;
+    seg_keys = 512;
+    if (n_dec > 16) {
+        const long blocks = (long)Hkv * n_dec;
+        const int want = max_position < 1536 ? 1 : (int)min(768 / blocks, (long)segments);
+        seg_keys = qe_cdiv(qe_cdiv(max_position + 1, max(1, want)), 16) * 16;
+        segments = max_position / seg_keys + 1;
+    }
+    return segments;
+}
+
+template <int D, bool FUSED>
+static void launch_block(const bf16_t* q, bf16_t* cache, const int* dec_tokens, int n_dec, const int* positions, const int* tok_seq,
+                         const int* block_table, int max_blocks, const int* shared_keys, const int* slots, const float* q_w, const float* k_w,
+                         float eps, const float* table, bf16_t* out, float* part, int Hq, int Hkv, int P, float scale, int window, int segments,
+                         int seg_keys, hipStream_t stream, const AttnTail& tail) {
+    constexpr int W = 4;
+    float* part_ml = part + (size_t)n_dec * Hq * segments * D;
+    attention_decode_block_kernel<D, W, FUSED><<<dim3(segments, Hkv, n_dec), 64 * W, (size_t)W * (Hq / Hkv) * (D + 6) * sizeof(float), stream>>>(
+        q, cache, dec_tokens, positions, tok_seq, block_table, max_blocks, shared_keys, slots, q_w, k_w, eps, table, out, part, part_ml,
+        Hq, Hkv, P, scale, window, segments, seg_keys, tail);
+    if (segments > 1)
+        attention_decode_merge_kernel<D><<<dim3(n_dec, Hq), 256, 0, stream>>>(part, part_ml, dec_tokens, out, Hq, segments, 0, tail);
+}
+
 // dec_tokens: the rows of q that are single new tokens of their requests (null: the rows
 // 0 .. n_dec - 1, which saves every wave a dependent load).  max_position: the
 // largest of their positions (fixes the number of splits).  workspace: at least
 // qe_attention_decode_workspace(...) bytes.  shared_keys: null, or for every row of the block table
 // the number of the request's first keys that other requests of the step may read as well (pages they
-// hold together): a hint for the caches, results do not depend on it.
+// hold together): a hint for the caches, results do not depend on it.  split_keys: 128 or 256; or 0, splits of 128 or, where that
+// is quicker, a block a token and key/value head, whose sums have another order (the workspace is that of splits of 128).
 int qe_attention_decode(const void* q, void* out, const void* cache, const int* dec_tokens, int n_dec,
                         const int* positions, const int* tok_seq, const int* block_table, int max_blocks,
                         const int* shared_keys, int Hq, int Hkv, int D, int P, float scale, int window, int keep_first,
                         int sink, float softcap, int max_position, int split_keys, void* workspace, size_t workspace_bytes,
                         hipStream_t stream, const AttnTail& tail) {
     QE_REQUIRE(qe_attention_decode_ok(Hq, Hkv, D, P, QE_BF16), "decode attention: sizes not taken");
-    QE_REQUIRE(split_keys == 128 || split_keys == 256, "decode attention: splits of 128 or 256 keys, not %d", split_keys);
+    QE_REQUIRE(split_keys == 0 || split_keys == 128 || split_keys == 256, "decode attention: splits of 128 or 256 keys, not %d", split_keys);
     if (n_dec == 0) return 0;
+    const bool blocks = split_keys == 0;
+    if (blocks) split_keys = 128;
     const int num_splits = max_position / split_keys + 1;
     QE_REQUIRE(num_splits <= 65535 && n_dec <= 65535, "decode attention: too many splits or tokens");
     QE_REQUIRE(workspace_bytes >= qe_attention_decode_workspace(n_dec, Hq, D, num_splits),
@@ -671,6 +854,18 @@ int qe_attention_decode(const void* q, void* out, const void* cache, const int* 
     (void)qe_cdiv;
     dim3 grid(num_splits, Hkv, n_dec);
     dim3 mgrid(n_dec, Hq);
+    int seg_keys = 0;
+    if (const int segments = blocks ? block_segments(n_dec, Hkv, max_position, window, sink, softcap, seg_keys) : 0) {
+#define QE_DECODE_BLOCK(D_)                                                                             \
+        launch_block<D_, false>((const bf16_t*)q, (bf16_t*)cache, dec_tokens, n_dec, positions, tok_seq, block_table, max_blocks, shared_keys, \
+                                nullptr, nullptr, nullptr, 0.f, nullptr, (bf16_t*)out, part_acc, Hq, Hkv, P, scale, window, segments, \
+                                seg_keys, stream, tail)
+        if (D == 128) QE_DECODE_BLOCK(128);
+        else QE_DECODE_BLOCK(64);
+#undef QE_DECODE_BLOCK
+        QE_LAUNCH_CHECK();
+        return 0;
+    }
     // (512 splits of 8 tokens over 1000 keys: 14.0 us with one wave a split, 12.6 with four; from 576 on the two are within 3 %
     // of each other: 14.2 and 14.4, 1024 17.6 and 17.4)
     const bool four = (long)num_splits * Hkv * n_dec <= 512 && max_position >= 16 * ALONE;
@@ -712,8 +907,10 @@ int qe_attention_decode_fused(const void* qkv, void* out, void* cache, const int
                               int Hq, int Hkv, int D, int P, float scale, int window, int max_position,
                               int split_keys, void* workspace, size_t workspace_bytes, hipStream_t stream) {
     QE_REQUIRE(qe_attention_decode_ok(Hq, Hkv, D, P, QE_BF16), "decode attention: sizes not taken");
-    QE_REQUIRE(split_keys == 128 || split_keys == 256, "decode attention: splits of 128 or 256 keys, not %d", split_keys);
+    QE_REQUIRE(split_keys == 0 || split_keys == 128 || split_keys == 256, "decode attention: splits of 128 or 256 keys, not %d", split_keys);
     if (n_dec == 0) return 0;
+    const bool blocks = split_keys == 0;
+    if (blocks) split_keys = 128;
     const int num_splits = max_position / split_keys + 1;
     QE_REQUIRE(num_splits <= 65535 && n_dec <= 65535, "decode attention: too many splits or tokens");
     QE_REQUIRE(workspace_bytes >= qe_attention_decode_workspace(n_dec, Hq, D, num_splits),
@@ -725,6 +922,17 @@ int qe_attention_decode_fused(const void* qkv, void* out, void* cache, const int
     AttnTail tail{};
     tail.out_stride = (long)Hq * D;
     tail.dv = D;
+    int seg_keys = 0;
+    if (const int segments = blocks ? block_segments(n_dec, Hkv, max_position, window, 0, 0.f, seg_keys) : 0) {
+#define QE_DECODE_BLOCK(D_)                                                                             \
+        launch_block<D_, true>((const bf16_t*)qkv, (bf16_t*)cache, dec_tokens, n_dec, positions, tok_seq, block_table, max_blocks, shared_keys, \
+                               slots, q_w, k_w, eps, table, (bf16_t*)out, part_acc, Hq, Hkv, P, scale, window, segments, seg_keys, stream, tail)
+        if (D == 128) QE_DECODE_BLOCK(128);
+        else QE_DECODE_BLOCK(64);
+#undef QE_DECODE_BLOCK
+        QE_LAUNCH_CHECK();
+        return 0;
+    }
     const long waves = (long)num_splits * Hkv * n_dec;
     const bool few = waves <= 1024;                            // at most a wave per SIMD: loads further ahead
     // (every wave prepares q: 256 splits of one request each take 11.4 us with four, 12.6 with one; 384 13.2 with one, 17.1 with four)

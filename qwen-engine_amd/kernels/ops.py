@@ -825,7 +825,7 @@ def attention(q: torch.Tensor, cache: torch.Tensor, positions: torch.Tensor, tok
               max_other_keys: int = 0, prefill_segment_keys: int = -1,
               other_keys_row: Optional[int] = None, shared_keys: Optional[torch.Tensor] = None,
               keep_first: int = 0, sink=False, chunk: int = 0, softcap: float = 0.0, v_dim: int = 0,
-              gate: Optional[torch.Tensor] = None) -> torch.Tensor:
+              gate: Optional[torch.Tensor] = None, dec_blocks: bool = False) -> torch.Tensor:
     """q [T, Hq, D]; cache [pages, 2, Hkv, P, D] (key tiles [P][D], value tiles transposed [D][P]);
     positions, tok_seq int32 [T]; block_table int32 [B, max_blocks].  Token t sees the keys at
     positions max(0, p - window + 1) .. p of request tok_seq[t] (window 0: all).  The caller
@@ -855,7 +855,10 @@ def attention(q: torch.Tensor, cache: torch.Tensor, positions: torch.Tensor, tok
     softcap * tanh(. / softcap) before the softmax.
 
     shared_keys (int32, an entry per row of block_table, or None): how many of a request's first keys
-    other requests read too.  A hint for the decode kernel's loads; results do not depend on it."""
+    other requests read too.  A hint for the decode kernel's loads; results do not depend on it.
+
+    dec_blocks: more than eight dec_tokens may have a block each that walks a token's keys (quicker; a row's sums then have another
+    order than alone, where every 128 keys are summed by themselves)."""
     lib = load_library()
     _need(q, "q", _ACT, (None, None, None))
     T, Hq, D = q.shape
@@ -928,7 +931,7 @@ def attention(q: torch.Tensor, cache: torch.Tensor, positions: torch.Tensor, tok
                                                tok_seq.data_ptr(), block_table.data_ptr(), max_blocks,
                                                _ptr(shared_keys), Hq, Hkv,
                                                D, P, float(scale), int(window), keep_first, sink, softcap, int(max_dec_position),
-                                               DECODE_SPLIT_KEYS, ws.data_ptr(), nbytes, *tail, _stream()),
+                                               0 if dec_blocks else DECODE_SPLIT_KEYS, ws.data_ptr(), nbytes, *tail, _stream()),
                    "attention (decode)")
         else:
             generic(dec_tokens)
@@ -985,13 +988,13 @@ def attention_decode_fused(qkv: torch.Tensor, num_heads: int, cache: torch.Tenso
                            q_weight: Optional[torch.Tensor], k_weight: Optional[torch.Tensor], eps: float,
                            table: Optional[torch.Tensor], slots: Optional[torch.Tensor],
                            out: Optional[torch.Tensor] = None,
-                           shared_keys: Optional[torch.Tensor] = None) -> torch.Tensor:
+                           shared_keys: Optional[torch.Tensor] = None, dec_blocks: bool = False) -> torch.Tensor:
     """Attention of single new tokens with the step before it inside: per-head q/k RMSNorm
     (weights or None), half-split rotation from ``table`` (rows [cos | sin] of the head size, or
     None) and the write of each token's key and value to cache slot ``slots[t]`` (negative or no
     slots: not written).  qkv [T, (Hq + 2 Hkv) D] bfloat16; the rows ``dec_tokens`` (None: all
     rows) are computed into out [T, Hq, D]; the cache holds each request's keys before the
-    token's own position.  shared_keys: as for attention()."""
+    token's own position.  shared_keys, dec_blocks: as for attention()."""
     lib = load_library()
     _need(qkv, "qkv", torch.bfloat16, (None, None))
     T, dev = qkv.shape[0], qkv.device
@@ -1030,7 +1033,7 @@ def attention_decode_fused(qkv: torch.Tensor, num_heads: int, cache: torch.Tenso
                                              block_table.shape[1], _ptr(shared_keys), _ptr(slots), _ptr(q_weight),
                                              _ptr(k_weight),
                                              float(eps), _ptr(table), Hq, Hkv, D, P, float(scale), int(window),
-                                             int(max_dec_position), DECODE_SPLIT_KEYS, ws.data_ptr(), nbytes,
+                                             int(max_dec_position), 0 if dec_blocks else DECODE_SPLIT_KEYS, ws.data_ptr(), nbytes,
                                              _stream()), "attention (decode, fused)")
     return out
 

@@ -21,8 +21,12 @@ from .registry import build_part, register_part
 
 # Up to this many single new tokens in a step, the decode attention kernel norms, rotates and
 # writes the cache itself; above, the separate kernel is quicker (every wave of the attention
-# kernel repeats the preparation of q, which then outweighs the kernel saved).
+# kernel repeats the preparation of q, which then outweighs the kernel saved).  With a window a token's
+# keys go in splits of a wave each, else four waves walk them (16 heads, the two kernels and the one: 32 tokens of 400 keys
+# 19.9 us and 17.7, of 4000 122 and 118; 64 of 400 32.7 and 29.9, of 2000 115 and 111; slower from 24 of 1000 keys, 38.1 and 39.1, to 48 of 2000,
+# 94.6 and 100.4).
 FUSED_DECODE_MAX_TOKENS = 16
+FUSED_DECODE_MAX_TOKENS_UNWINDOWED = 64
 
 
 def prefill_tiles(portions, rows_per_tile: int) -> List[int]:
@@ -60,9 +64,12 @@ class PagedAttention:
     @classmethod
     def graph_key(cls, max_position: int) -> int:
         """The decode kernel's grid and workspace follow the number of key splits: recorded steps are
-        kept per bucket of splits."""
+        kept per bucket of splits (half a bucket for short contexts, whose keys more than eight tokens have in one segment: with the second,
+        empty one and its merge 16 tokens of 400 keys take 3 us a layer more)."""
         splits = int(max_position) // ops.DECODE_SPLIT_KEYS + 1
         b = cls.GRAPH_SPLIT_BUCKET
+        if splits <= b // 2:
+            return b // 2
         return (splits + b - 1) // b * b
 
     @staticmethod
@@ -239,14 +246,14 @@ class PagedAttention:
             ex = self._extras(ctx)
             only_new_tokens = (ex["dec_tokens"] is not None and ex["dec_tokens"].shape[0] == T and
                                (ex["other_tokens"] is None or ex["other_tokens"].shape[0] == 0))
-            if (only_new_tokens and T <= FUSED_DECODE_MAX_TOKENS and binding.write and
+            if (only_new_tokens and T <= (FUSED_DECODE_MAX_TOKENS if self.window else FUSED_DECODE_MAX_TOKENS_UNWINDOWED) and binding.write and
                     ops.attention_decode_fused_supported(qkv, cache, self.hq, table)):
                 # every row is the one new token of its request: norm, rotation and cache write
                 # happen inside the attention kernel
                 o = ops.attention_decode_fused(qkv, self.hq, cache, ctx.positions, ctx.tok_seq, ctx.block_tables[g],
                                                self.scale, self.window, None, ex["max_dec_position"],
                                                self.q_norm, self.k_norm, eps, table, slots,
-                                               shared_keys=ctx.shared_keys)
+                                               shared_keys=ctx.shared_keys, dec_blocks=True)
                 return self._project_out(o.view(T, self.hq * self.d))
             q = ops.qk_rope_store(qkv, self.hq, self.hkv, self.d, ctx.positions, self.q_norm, self.k_norm,
                                   eps, table, slots, cache, ctx.page_size)
@@ -267,7 +274,7 @@ class PagedAttention:
                           other_tokens=ex["other_tokens"],
                           other_tiles=self._other_tiles(ctx) if ex["other_tokens"] is not None else None,
                           max_other_keys=ex.get("max_other_keys", 0), other_keys_row=ex.get("other_keys_row"),
-                          shared_keys=ctx.shared_keys)
+                          shared_keys=ctx.shared_keys, dec_blocks=True)
         return self._project_out(o.view(T, self.hq * self.d))
 
     def _project_out(self, o: torch.Tensor) -> torch.Tensor:

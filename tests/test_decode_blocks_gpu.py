@@ -1,0 +1,99 @@
+"""Single new tokens whose keys one block walks (four waves, each with every fourth tile and a softmax of its own), in one segment and in several."""
+import pytest
+import torch
+
+import qwen_engine_amd  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from qwen_engine_amd.kernels import ops as o
+    return o
+
+
+def rand(*shape, seed=0):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed))
+
+
+def _requests(pos, hkv, D, P):
+    """(cache, block table, keys and values of every request): shuffled pages, NaN wherever nothing was written."""
+    pages = [p // P + 1 for p in pos]
+    order = torch.randperm(sum(pages), generator=torch.Generator().manual_seed(7)).int()
+    table, at = torch.full((len(pos), max(pages)), -1, dtype=torch.int32), 0
+    cache = torch.full((sum(pages), 2, hkv, P * D), float("nan"), dtype=torch.bfloat16)     # (a key tile [P][D], a value tile [D][P])
+    ks, vs = [], []
+    for i, p in enumerate(pos):
+        k, v = rand(p + 1, hkv, D, seed=20 + i).bfloat16(), rand(p + 1, hkv, D, seed=160 + i).bfloat16()
+        ids = order[at:at + pages[i]]
+        at += pages[i]
+        table[i, :pages[i]] = ids
+        for j in range(pages[i]):
+            part = slice(j * P, min(p + 1, (j + 1) * P))
+            n = part.stop - part.start
+            cache[ids[j], 0].view(hkv, P, D)[:, :n] = k[part].transpose(0, 1)
+            cache[ids[j], 1].view(hkv, D, P)[:, :, :n] = v[part].permute(1, 2, 0)
+        ks.append(k)
+        vs.append(v)
+    return cache.view(-1, 2, hkv, P, D).to(DEV), table.to(DEV), ks, vs
+
+
+EDGES = [0, 1, 15, 16, 17, 47, 48, 63, 64, 511, 512, 513, 800, 1023]
+# nine tokens and sixteen (segments of 512 keys), one segment for seventeen, segments by the launch beyond 1536 keys, a walk of more
+# tiles than a wave holds pages of
+MANY = {"nine": EDGES[5:], "sixteen": EDGES + [1024, 1100], "seventeen": EDGES + [1024, 1100, 1535], "cut": EDGES + [1536, 2100, 2101, 300, 301, 302],
+        "long": EDGES + [4300] + [33] * 185}
+
+
+@pytest.mark.parametrize("hq,hkv,D,P", [(8, 4, 128, 16), (16, 1, 128, 48), (6, 2, 64, 16), (4, 4, 64, 32)])
+@pytest.mark.parametrize("which", list(MANY))
+def test_a_block_walks_a_tokens_keys(ops, hq, hkv, D, P, which):
+    pos = MANY[which]
+    n = len(pos)
+    cache, table, ks, vs = _requests(pos, hkv, D, P)
+    q = rand(n, hq, D, seed=hq).bfloat16()
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    scale = 1.5 / D ** 0.5
+    seen = dict(dec_tokens=i32(range(n)), max_dec_position=max(pos), dec_blocks=True)
+    out = ops.attention(q.to(DEV), cache, i32(pos), i32(range(n)), table, scale, **seen).cpu()
+    qkv = torch.stack([torch.cat([q[i].flatten(), ks[i][-1].flatten(), vs[i][-1].flatten()]) for i in range(n)])
+    # (the new key and value are written where they already lie: unwritten for it)
+    slots = [int(table[i, p // P]) * P + p % P for i, p in enumerate(pos)]
+    fresh = cache.clone()
+    for s in slots:
+        fresh[s // P, 0, :, s % P] = float("nan")
+        fresh[s // P, 1].view(hkv, D, P)[:, :, s % P] = float("nan")
+    fused = ops.attention_decode_fused(qkv.to(DEV), hq, fresh, i32(pos), i32(range(n)), table, scale, 0, None, max(pos), None, None, 1e-6,
+                                       None, i32(slots), dec_blocks=True).cpu()
+    assert torch.equal(torch.nan_to_num(fresh.float()), torch.nan_to_num(cache.float()))
+    for i, p in enumerate(pos):
+        k, v = ks[i].double(), vs[i].double()
+        w = torch.softmax(torch.stack([k[:, h * hkv // hq] @ q[i, h].double() for h in range(hq)]) * scale, -1)
+        want = torch.stack([w[h] @ v[:, h * hkv // hq] for h in range(hq)])
+        # (the weights and the result are rounded to bfloat16: 2^-9 of each weight times its value, and of the result)
+        bound = 2.0 ** -8 * (torch.stack([w[h] @ v[:, h * hkv // hq].abs() for h in range(hq)]) + want.abs())
+        for got in (out, fused):
+            assert ((got.view(n, hq, D)[i].double() - want).abs() <= bound).all(), p
+
+
+def test_bits_of_nine_to_sixteen_tokens(ops):
+    """A token's bits are the same beside eight others and beside fifteen, with keys in one segment (written as they are joined) and in several
+    (through the merge), and with its rows in another order."""
+    hq, hkv, D, P = 8, 4, 128, 16
+    pos = [5, 100, 300, 400, 500, 511, 64, 17, 250, 700, 1500, 512, 900, 30, 31, 2]
+    cache, table, _, _ = _requests(pos, hkv, D, P)
+    qkv = rand(len(pos), (hq + 2 * hkv) * D, seed=3).bfloat16().to(DEV)
+    qw, kw, turn = 1 + rand(D, seed=1).to(DEV) / 4, 1 + rand(D, seed=2).to(DEV) / 4, rand(2048, D, seed=4).to(DEV)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+
+    def run(which, most):
+        got = ops.attention_decode_fused(qkv, hq, cache.clone(), i32(pos), i32(range(len(pos))), table, 0.1, 0, i32(which), most, qw, kw, 1e-6,
+                                         turn, None, dec_blocks=True)
+        return got[which]
+    every = run(list(range(16)), 1500)
+    assert torch.equal(run(list(range(9)), 511), every[:9])
+    assert torch.equal(run(list(range(9)), 4000), every[:9])
+    back = list(range(15, 3, -1))
+    assert torch.equal(run(back, 1535), every[back])
