@@ -48,14 +48,25 @@ size_t qe_attention_prefill_workspace(int num_tiles, int Hq, int Hkv, int D, int
 
 int qe_attention_prefill_tile_rows(int Hq, int Hkv);
 int qe_attention_prefill_tiles(const int* portions, int n_portions, int rows_per_tile, int* tiles, int max_groups,
-                               hipStream_t stream);
+                               int singles, hipStream_t stream);
 
 // The tile list for qe_attention_prefill_run from portions [n_portions][2] = (first row, rows) that lie
-// on the device: tiles [4 max_groups][2], whatever is beyond the portions' groups being groups of no
-// rows.  The caller guarantees that the portions have at most max_groups groups of 4 tiles.
+// on the device: tiles [4 (singles + max_groups)][2], a group for each of the rows 0 .. singles - 1, then the portions', whatever is
+// beyond those being groups of no rows.  The caller guarantees that the portions have at most max_groups groups of 4 tiles.
 extern "C" int qe_attention_prefill_tiles_run(const int* portions, int n_portions, int rows_per_tile, int* tiles,
-                                              int max_groups, hipStream_t stream) {
-    return qe_attention_prefill_tiles(portions, n_portions, rows_per_tile, tiles, max_groups, stream);
+                                              int max_groups, int singles, hipStream_t stream) {
+    return qe_attention_prefill_tiles(portions, n_portions, rows_per_tile, tiles, max_groups, singles, stream);
+}
+
+// Whether n_dec single new tokens at positions up to max_position are best taken along by the prefill kernel, as groups of one row beside
+// the rows of portions (whose rows see at most max_keys keys), instead of by the decode kernel and then the portions by themselves: a launch or two are
+// saved, and the tokens' walks pass beside the portions'.  (us, 16 heads of 128 on 8, a portion of 400 rows from the start; apart, tokens a block each from nine on,
+// and in one: one token of 400 keys 25.2, 16.7, of 1000 25.9, 22.4, of 2000 26.0, 35.8; 15 of 400 28, 17.6, of 1000 35, 25.4, of 2000 48, 39.5; 64 of 400
+// 40, 34.8, of 1000 71, 61.9.  A portion of 64 rows: one of 1000 20.0, 22.1, eight 24.1, 23.1.)  Not where the walks are cut into segments: more
+// blocks would leave fewer of those.
+extern "C" int qe_attention_prefill_takes_single(int n_dec, int max_position, int rows, int max_keys) {
+    if (n_dec <= 0 || rows <= 0 || max_keys > qe_attention_prefill_uncut_keys()) return 0;
+    return max_position < 512 || (max_position < 1024 && (rows >= 256 || n_dec >= 8));
 }
 
 // rows of a tile for these head counts

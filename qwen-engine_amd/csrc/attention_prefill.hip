@@ -615,11 +615,22 @@ __global__ __launch_bounds__(256) void attention_prefill_merge_kernel(
 // The tile list of qe_attention_prefill from the step's portions, made on the device (a recorded step
 // does not know its portions' lengths on the host): portions [n_portions][2] = (first row, rows), each
 // cut into tiles of at most `rows_per_tile` rows in groups of four, a group filled up with tiles of no
-// rows; the list is filled up to max_groups groups with groups of no rows.  One thread per group.
+// rows; the list is filled up to max_groups groups with groups of no rows.  The step's first `singles` rows, each of a
+// request of its own, are a group each before those.  One thread per group.
 __global__ void prefill_tiles_kernel(const int* __restrict__ portions, int n_portions, int rows_per_tile,
-                                     int* __restrict__ tiles, int max_groups) {
-    const int grp = blockIdx.x * blockDim.x + threadIdx.x;
-    if (grp >= max_groups) return;
+                                     int* __restrict__ tiles, int max_groups, int singles) {
+    int grp = blockIdx.x * blockDim.x + threadIdx.x;
+    if (grp >= singles + max_groups) return;
+    if (grp < singles) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            tiles[8 * grp + 2 * j] = grp;
+            tiles[8 * grp + 2 * j + 1] = j == 0;
+        }
+        return;
+    }
+    grp -= singles;
+    tiles += 8 * singles;
     int first = 0, start = 0, rows = 0, in_portion = -1;   // which portion the group lies in, and the group's place in it
     for (int i = 0; i < n_portions; ++i) {
         const int n = portions[2 * i + 1];
@@ -642,10 +653,10 @@ __global__ void prefill_tiles_kernel(const int* __restrict__ portions, int n_por
 }
 
 int qe_attention_prefill_tiles(const int* portions, int n_portions, int rows_per_tile, int* tiles, int max_groups,
-                               hipStream_t stream) {
-    QE_REQUIRE(portions && tiles && n_portions >= 1 && n_portions <= 64 && rows_per_tile >= 1 && max_groups >= 1,
-               "prefill tiles: %d portions, tiles of %d rows, %d groups", n_portions, rows_per_tile, max_groups);
-    prefill_tiles_kernel<<<qe_cdiv(max_groups, 64), 64, 0, stream>>>(portions, n_portions, rows_per_tile, tiles, max_groups);
+                               int singles, hipStream_t stream) {
+    QE_REQUIRE(portions && tiles && n_portions >= 1 && n_portions <= 64 && rows_per_tile >= 1 && max_groups >= 1 && singles >= 0,
+               "prefill tiles: %d portions, tiles of %d rows, %d groups, %d single rows", n_portions, rows_per_tile, max_groups, singles);
+    prefill_tiles_kernel<<<qe_cdiv(singles + max_groups, 64), 64, 0, stream>>>(portions, n_portions, rows_per_tile, tiles, max_groups, singles);
     QE_LAUNCH_CHECK();
     return 0;
 }

@@ -64,7 +64,8 @@ def load_library():
         "qe_attention_prefill_run": [vp, vp, vp, vp, i32, vp, vp, vp, i32, i32, i32, i32, i32, f32, i32, i32, i32, f32, i32, i32, i32,
                                      i32, vp, i64, i64, i32, vp, vp, i64, i32, vp],
         "qe_attention_prefill_plan_segments": [i32, i32, i32],
-        "qe_attention_prefill_tiles_run": [vp, i32, i32, vp, i32, vp],
+        "qe_attention_prefill_tiles_run": [vp, i32, i32, vp, i32, i32, vp],
+        "qe_attention_prefill_takes_single": [i32, i32, i32, i32],
         "qe_attention_prefill_workspace_bytes_for": [i32, i32, i32, i32, i32],
         "qe_attention_prefill_plan": [i32, i32, i32, i32],
         "qe_attention_prefill_plan_uncut_keys": [],
@@ -791,16 +792,23 @@ def prefill_tile_rows(num_heads: int, num_kv_heads: int) -> int:
     return load_library().qe_attention_prefill_rows(num_heads, num_kv_heads)
 
 
-def prefill_tiles_on_device(portions: torch.Tensor, rows_per_tile: int, max_groups: int) -> torch.Tensor:
+def prefill_takes_single(n_dec: int, max_position: int, rows: int, max_keys: int) -> bool:
+    """True if ``n_dec`` single new tokens at positions up to ``max_position`` are best computed by the prefill attention kernel, together
+    with ``rows`` rows of portions that see at most ``max_keys`` keys."""
+    return bool(load_library().qe_attention_prefill_takes_single(int(n_dec), int(max_position), int(rows), int(max_keys)))
+
+
+def prefill_tiles_on_device(portions: torch.Tensor, rows_per_tile: int, max_groups: int, singles: int = 0) -> torch.Tensor:
     """The ``other_tiles`` of attention() for portions int32 [n, 2] = (first row, rows) that lie on the
     device (a recorded step does not know them on the host): int32 [4 * max_groups, 2], groups of no rows
     beyond what the portions need.  The caller guarantees that the portions need at most max_groups
-    groups of four tiles (every portion: ceil(rows / (4 * rows_per_tile)))."""
+    groups of four tiles (every portion: ceil(rows / (4 * rows_per_tile))).  singles: so many groups more, in front, of the rows
+    0 .. singles - 1, each by itself."""
     lib = load_library()
     _need(portions, "portions", torch.int32, (None, 2))
-    tiles = torch.empty((4 * int(max_groups), 2), dtype=torch.int32, device=portions.device)
+    tiles = torch.empty((4 * (int(singles) + int(max_groups)), 2), dtype=torch.int32, device=portions.device)
     _check(lib.qe_attention_prefill_tiles_run(portions.data_ptr(), portions.shape[0], int(rows_per_tile),
-                                              tiles.data_ptr(), int(max_groups), _stream()), "prefill tiles")
+                                              tiles.data_ptr(), int(max_groups), int(singles), _stream()), "prefill tiles")
     return tiles
 
 

@@ -113,6 +113,7 @@ class PagedAttention:
                 "other_tokens": torch.arange(rows, rows + tokens, dtype=torch.int32, device=device),
                 "max_dec_position": splits * ops.DECODE_SPLIT_KEYS - 1, "max_other_keys": 0,
                 "other_keys_row": rows + tokens - 1 if cut else None,
+                "all_tokens": torch.arange(rows + tokens, dtype=torch.int32, device=device),
                 "portions": dynamic.view(2, 2), "portion_rows": int(tokens)}
 
     def _extras(self, ctx) -> dict:
@@ -122,6 +123,28 @@ class PagedAttention:
             if cls in ctx.extras:
                 return ctx.extras[cls]
         return {"dec_tokens": None, "other_tokens": None, "max_dec_position": 0, "max_other_keys": 0}
+
+    def _all_tiles(self, ctx, ex, q: torch.Tensor, cache: torch.Tensor):
+        """For a step of single new tokens and portions whose attention is quickest in one launch of the prefill kernel: (all rows, all
+        rows cut into tiles, a group for every single token), once per step and tile size; else None."""
+        dec, other = ex["dec_tokens"], ex["other_tokens"]
+        if dec is None or other is None or not dec.shape[0] or not other.shape[0] or not ops.attention_prefill_supported(q, cache):
+            return None
+        max_keys = ops.prefill_uncut_keys() + 1 if ex.get("other_keys_row") is not None else ex.get("max_other_keys", 0)
+        if not ops.prefill_takes_single(dec.shape[0], ex["max_dec_position"], other.shape[0], max_keys):
+            return None
+        rows_per_tile = ops.prefill_tile_rows(self.hq, self.hkv)
+        key = ("paged_attention.all_tiles", rows_per_tile)
+        if key not in ctx.memo:
+            if ex.get("portions") is not None:             # (a recorded step: the single tokens come first, see _other_tiles)
+                portions = ex["portions"]
+                groups = -(-ex["portion_rows"] // (4 * rows_per_tile)) + portions.shape[0]
+                ctx.memo[key] = ex["all_tokens"], ops.prefill_tiles_on_device(portions, rows_per_tile, groups, dec.shape[0])
+            else:
+                flat = prefill_tiles([(s.q_start, s.q_len) for s in sorted(ctx.seqs, key=lambda s: s.q_len)], rows_per_tile)
+                ctx.memo[key] = (torch.arange(ctx.num_tokens, dtype=torch.int32, device=q.device),
+                                 torch.tensor(flat, dtype=torch.int32).view(-1, 2).to(q.device))
+        return ctx.memo[key]
 
     def _other_tiles(self, ctx) -> Optional[torch.Tensor]:
         """The rows of requests that bring several tokens, cut into tiles for the prefill kernel: built
@@ -269,12 +292,17 @@ class PagedAttention:
 
     def _attend(self, q: torch.Tensor, ctx, cache: torch.Tensor, g: int, T: int) -> torch.Tensor:
         ex = self._extras(ctx)
-        o = ops.attention(q, cache, ctx.positions, ctx.tok_seq, ctx.block_tables[g], self.scale, self.window,
-                          dec_tokens=ex["dec_tokens"], max_dec_position=ex["max_dec_position"],
-                          other_tokens=ex["other_tokens"],
-                          other_tiles=self._other_tiles(ctx) if ex["other_tokens"] is not None else None,
-                          max_other_keys=ex.get("max_other_keys", 0), other_keys_row=ex.get("other_keys_row"),
-                          shared_keys=ctx.shared_keys, dec_blocks=True)
+        together = self._all_tiles(ctx, ex, q, cache)
+        if together is not None:
+            o = ops.attention(q, cache, ctx.positions, ctx.tok_seq, ctx.block_tables[g], self.scale, self.window,
+                              other_tokens=together[0], other_tiles=together[1])
+        else:
+            o = ops.attention(q, cache, ctx.positions, ctx.tok_seq, ctx.block_tables[g], self.scale, self.window,
+                              dec_tokens=ex["dec_tokens"], max_dec_position=ex["max_dec_position"],
+                              other_tokens=ex["other_tokens"],
+                              other_tiles=self._other_tiles(ctx) if ex["other_tokens"] is not None else None,
+                              max_other_keys=ex.get("max_other_keys", 0), other_keys_row=ex.get("other_keys_row"),
+                              shared_keys=ctx.shared_keys, dec_blocks=True)
         return self._project_out(o.view(T, self.hq * self.d))
 
     def _project_out(self, o: torch.Tensor) -> torch.Tensor:

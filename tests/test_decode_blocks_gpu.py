@@ -97,3 +97,32 @@ def test_bits_of_nine_to_sixteen_tokens(ops):
     assert torch.equal(run(list(range(9)), 4000), every[:9])
     back = list(range(15, 3, -1))
     assert torch.equal(run(back, 1535), every[back])
+
+
+@pytest.mark.parametrize("hq,hkv,rows", [(8, 4, 1), (8, 4, 70), (8, 1, 200), (6, 2, 33)])
+@pytest.mark.parametrize("singles", [1, 15, 40])
+def test_single_tokens_beside_a_portion_in_one_launch(ops, hq, hkv, rows, singles):
+    """Single tokens as groups of one row of the prefill kernel, beside a portion's rows: what the decode and the prefill kernel compute apart,
+    with the tiles from the host and made on the device."""
+    from qwen_engine_amd.parts.attention import prefill_tiles
+    D, P, behind = 128, 16, 45
+    pos = [(i * 37) % 600 for i in range(singles)]
+    cache, table, _, _ = _requests(pos + [behind + rows - 1], hkv, D, P)
+    T, R = singles + rows, ops.prefill_tile_rows(hq, hkv)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    positions, seq = i32(pos + list(range(behind, behind + rows))), i32(list(range(singles)) + [singles] * rows)
+    q = rand(T, hq, D, seed=5).bfloat16().to(DEV)
+    scale = 1.5 / D ** 0.5
+    apart = ops.attention(q, cache, positions, seq, table, scale, dec_tokens=i32(range(singles)), max_dec_position=max(pos),
+                          other_tokens=i32(range(singles, T)), other_tiles=i32(prefill_tiles([(singles, rows)], R)).view(-1, 2))
+    flat = prefill_tiles([(i, 1) for i in range(singles)] + [(singles, rows)], R)
+    tiles = ops.prefill_tiles_on_device(i32([[singles, 0], [singles, rows]]), R, -(-rows // (4 * R)) + 1, singles)
+    assert tiles.cpu().flatten().tolist()[:len(flat)] == flat and tiles[len(flat) // 2:, 1].cpu().tolist() == [0] * 4
+    together = [ops.attention(q, cache, positions, seq, table, scale, other_tokens=i32(range(T)), other_tiles=t)
+                for t in (tiles, i32(flat).view(-1, 2))]
+    assert torch.equal(together[0], together[1])
+    # (weights and results are rounded to bfloat16 on both sides, at other references: 2^-8 of values of order one, weighed)
+    assert (together[0].float() - apart.float()).abs().max() <= 2.0 ** -7 * 4
+    assert float((together[0].float() - apart.float()).norm() / apart.float().norm()) < 2.0 ** -8
+    if rows > 1 and hq // hkv in (1, 2, 4, 8):
+        assert torch.equal(together[0][singles:], apart[singles:])
