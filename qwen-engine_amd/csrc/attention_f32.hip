@@ -35,28 +35,36 @@ __device__ __forceinline__ float max_over_rows_of_lanes(float v) {
 #define F32_WALKS 8
 #define F32_SLOTS 4           // results in shared memory: one for the walks w and w + 4 together
 
-// NW waves.  AHEAD: a tile's values are asked for before its scores, the next tile's keys before this tile's softmax.  Few
-// tokens are bound by their walks' trips to memory (2 tokens of 16 heads on 8 over 744 keys: 32 us, 55 with four waves, each
-// with 12 tiles one after the other and every load where it is used); with many tokens other waves fill the time, and the
+// NW waves.  AHEAD: 1: a tile's values are asked for before its scores, the next tile's keys before this tile's softmax; 2 (pages of whole
+// tiles): the next tile whole before this one's scores.  Few tokens are bound by their walks' trips to memory (2 tokens of 16 heads on 8
+// over 744 keys: 55 us with four waves, each with 12 tiles one after the other and every load where it is used, 32 with eight and AHEAD 1; over 512 keys
+// 27.8, with 2 22.7, over 2048 93 and 63; what is left is what a compute unit alone gets, some 35 GB/s); with many tokens other waves fill the time, and the
 // registers that this takes cost more.
-template <int DB, int NW, bool AHEAD>     // DB: head size / 16
-__global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? 3 : 1) void attention_f32_kernel(
+//
+// ROWS (no window, at most eight heads a key/value head): the 16 columns are 16 / G tokens' heads, which see the keys of one
+// request up to their own positions, so that many tokens read and multiply a tile once instead of each by itself; neighbours in the list that belong to
+// different requests are walked one request after the other.  A column's sums are those it has alone: a tile it sees nothing of leaves
+// them as they are.  (Portions of 328 and 416 rows of 16 heads of 128 on 8: 200 us, a block a token, and 42; 2048 rows 1980, 300; 400 of 64
+// heads 120, 78; 40 rows 11.7, 11.2; two of 50 and 30, where a block holds tokens of both, 12.8, 16.6.)
+template <int DB, int NW, int AHEAD, bool ROWS>      // DB: head size / 16
+__global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? (ROWS || AHEAD ? 2 : 3) : 1) void attention_f32_kernel(
     const float* __restrict__ q, float* __restrict__ out, const float* __restrict__ cache,
     const int* __restrict__ positions, const int* __restrict__ tok_seq,
-    const int* __restrict__ block_table, int max_blocks, const int* __restrict__ tokens,
+    const int* __restrict__ block_table, int max_blocks, const int* __restrict__ tokens, int T,
     int Hq, int Hkv, int P, float scale, int window, int keep_first, int sink, float softcap, AttnTail tail) {
     constexpr int D = DB * 16;
     extern __shared__ float merge_lds[];                  // [F32_SLOTS][DB * 4 + 2][64]
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, n = lane & 15;
-    const long t = tokens ? tokens[blockIdx.x] : blockIdx.x;
-    const int G = Hq / Hkv;
-    const int groups16 = (G + 15) / 16;
-    const int kvh = blockIdx.y / groups16, hg = blockIdx.y % groups16;
-    const int head = kvh * G + hg * 16 + n;
-    const bool head_ok = hg * 16 + n < G;
-    const int p = positions[t];
-    const int lo = first_seen_key(p, window);
-    const int* bt = block_table + (long)tok_seq[t] * max_blocks;
+    const int G = Hq / Hkv, R = ROWS ? 16 / G : 1;         // (R: tokens a block)
+    const int groups16 = ROWS ? 1 : (G + 15) / 16;
+    // (ROWS: a compute die has the blocks of every eighth key/value head, whose keys its L2 holds; later tokens, which see more keys, start first)
+    const int kvh = ROWS ? blockIdx.x : blockIdx.y / groups16, hg = ROWS ? 0 : blockIdx.y % groups16;
+    const int mine = ROWS ? n / G : 0, first = ROWS ? (int)(gridDim.y - 1 - blockIdx.y) * R : blockIdx.x;      // the column's token of the block's
+    const int at = min(first + min(mine, R - 1), T - 1);
+    const long t = tokens ? tokens[at] : at;
+    const int head = kvh * G + (ROWS ? n - mine * G : hg * 16 + n);
+    const bool head_ok = ROWS ? mine < R && first + mine < T : hg * 16 + n < G;
+    const int p = positions[t], seq = tok_seq[t];
     const long page_stride = 2L * Hkv * P * D;
     const bool vec_v = (P & 3) == 0;                      // four consecutive keys of a value row lie in one page, aligned
 
@@ -66,13 +74,38 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? 3 : 1) void a
         qv[c] = floatx4{0.f, 0.f, 0.f, 0.f};
         if (head_ok) qv[c] = *(const floatx4*)(q + (t * Hq + head) * D + c * 16 + g * 4);
     }
+    // (one round, but for a block whose tokens belong to several requests, and for one with a value that is infinite or NaN: where a column does
+    // not see it, it has met a weight of 0, so each token then has a round of its own)
+    unsigned long todo = ROWS ? __ballot(head_ok) : 1ul;
+    bool one_by_one = false;
+    do {
+    const int next = ROWS ? __builtin_ctzl(todo) : 0;
+    const int first_seq = ROWS ? __builtin_amdgcn_readlane(seq, next) : seq;
+    // the column's token is of this round's request
+    const bool on = head_ok && seq == first_seq && (!one_by_one || mine == __builtin_amdgcn_readlane(mine, next));
+    if (ROWS) todo &= ~__ballot(on);
+    bool odd = false;
+    int top = p, first_p = p;                              // no column of the round sees a key beyond top, all see those up to first_p
+    if (ROWS) {
+        top = on ? p : -1;
+        first_p = on ? p : 0x7fffffff;
+#pragma unroll
+        for (int k = 1; k < 16; k <<= 1) {
+            top = max(top, __shfl_xor(top, k, 64));
+            first_p = min(first_p, __shfl_xor(first_p, k, 64));
+        }
+        top = __builtin_amdgcn_readfirstlane(top);
+        first_p = __builtin_amdgcn_readfirstlane(first_p);
+    }
+    const int lo = ROWS ? 0 : first_seen_key(p, window);
+    const int* bt = block_table + (long)first_seq * max_blocks;
     // The tiles of the walks: those of the kept first keys 0 .. kf - 1 that lie wholly before the window's
     // first tile, then the tiles from the window's first on (which holds the rest of the kept keys, if
     // any); tile number i of this list is walk i % F32_WALKS's.
     const int kf = keep_first < lo ? keep_first : lo;
     const int tile_lo = lo / 16;
     const int n_first = (kf + 15) / 16 < tile_lo ? (kf + 15) / 16 : tile_lo;
-    const int n_tiles = n_first + p / 16 - tile_lo + 1;
+    const int n_tiles = n_first + top / 16 - tile_lo + 1;
     const auto tile_key = [&](int ti) { return 16 * (ti < n_first ? ti : tile_lo + ti - n_first); };
     // Pages of whole tiles: lane i holds the page of the walk's i-th tile of 64 (one load for all of them, where each tile's lookups
     // were two trips to memory of their own); a tile's page is then the same for the wave, and so is its place in it.  Other page sizes:
@@ -90,7 +123,7 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? 3 : 1) void a
     };
     const auto load_keys = [&](int kk, int page, floatx4 (&kr)[DB]) {      // S^T: this lane brings the key row kk + n
         const int key_r = kk + n;
-        const bool row_ok = (key_r >= lo || key_r < kf) && key_r <= p;
+        const bool row_ok = (key_r >= lo || key_r < kf) && key_r <= top;
         const float* krow = cache + (long)page * page_stride + ((long)kvh * P + kk % P + n) * D + g * 4;
         if (!whole && row_ok) krow = cache + (long)bt[key_r / P] * page_stride + ((long)kvh * P + key_r % P) * D + g * 4;
 #pragma unroll
@@ -105,7 +138,7 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? 3 : 1) void a
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int kc = ok[i] ? kk + 4 * g + i : p;     // (an address that is valid; the value is not used)
+            const int kc = ok[i] ? kk + 4 * g + i : top;   // (an address that is valid; the value is not used)
             voff[i] = (long)bt[kc / P] * page_stride + ((long)(Hkv + kvh) * P) * D + kc % P;
         }
     };
@@ -155,75 +188,144 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? 3 : 1) void a
         l = 0.f;                                           // this lane's share of the column's sum
 #pragma unroll
         for (int db = 0; db < DB; ++db) acc[db] = floatx4{0.f, 0.f, 0.f, 0.f};
-        floatx4 kr[DB], vr[AHEAD ? DB : 1];
-        int page = 0;
-        if (AHEAD && walk < n_tiles) {
-            page = page_of(walk, walk);
-            load_keys(tile_key(walk), page, kr);
-        }
-        for (int ti = walk; ti < n_tiles; ti += F32_WALKS) {
-            const int kk = tile_key(ti);
-            bool ok[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int key = kk + 4 * g + i;
-                ok[i] = (key >= lo || key < kf) && key <= p;
-            }
-            if (!AHEAD) {
-                page = page_of(ti, walk);
-                load_keys(kk, page, kr);
-            }
-            long voff[4];
-            if (AHEAD) {
-                value_places(kk, page, ok, voff);
-#pragma unroll
-                for (int db = 0; db < DB; ++db) vr[AHEAD ? db : 0] = load_value(db, ok, voff);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            floatx4 s = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int c = 0; c < DB; ++c)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[c][j], qv[c][j], s, 0, 0, 0);
-            if (AHEAD && ti + F32_WALKS < n_tiles) {
-                page = page_of(ti + F32_WALKS, walk);
-                load_keys(tile_key(ti + F32_WALKS), page, kr);
-            }
-            // the lane now holds the scores of keys kk + 4 g + i of column n
+        // From a tile's scores its weights (s holds those of keys kk + 4 g + i of column n), with the running maximum and sum; returns the factor for
+        // what was summed before.  sees: the keys that the column sees.
+        const auto weigh = [&](floatx4& s, const bool (&sees)[4]) {
             float tmax = -INFINITY;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 s[i] *= scale;
                 if (softcap > 0.f) s[i] = softcap * tanhf(s[i] / softcap);
-                if (!ok[i]) s[i] = -INFINITY;
+                if (!sees[i]) s[i] = -INFINITY;
                 tmax = fmaxf(tmax, s[i]);
             }
             tmax = max_over_rows_of_lanes(tmax);
-            const float mn = fmaxf(m, tmax);               // finite: every tile of the walk holds a key that is seen
-            const float alpha = expf(m - mn);              // 0 on the first tile
-            floatx4 pr;
+            const float mn = fmaxf(m, tmax);               // finite, as every tile of the walk holds a key that is seen (ROWS: by some column)
+            const float ref = ROWS && mn == -INFINITY ? 0.f : mn;
+            const float alpha = expf(m - ref);             // 0 on the first tile
             float psum = 0.f;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                pr[i] = ok[i] ? expf(s[i] - mn) : 0.f;
-                psum += pr[i];
+                s[i] = sees[i] ? expf(s[i] - ref) : 0.f;
+                psum += s[i];
             }
             l = l * alpha + psum;
             m = mn;
-            // O^T: this lane brings, of the value rows d = 16 db + n, the keys kk + 4 g .. + 3
-            if (!AHEAD) value_places(kk, page, ok, voff);
+            return alpha;
+        };
+        const auto score = [&](const floatx4 (&kr)[DB]) {
+            floatx4 s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int db = 0; db < DB; ++db) {
-                const floatx4 vf = AHEAD ? vr[AHEAD ? db : 0] : load_value(db, ok, voff);
-                acc[db] *= alpha;
+            for (int c = 0; c < DB; ++c)
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    acc[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[j], pr[j], acc[db], 0, 0, 0);
+                for (int j = 0; j < 4; ++j) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[c][j], qv[c][j], s, 0, 0, 0);
+            return s;
+        };
+        // O^T: the lane brings, of the value rows d = 16 db + n, the keys kk + 4 g .. + 3
+        const auto add_values = [&](int db, const floatx4& vf, const floatx4& pr, float alpha) {
+            acc[db] *= alpha;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[j], pr[j], acc[db], 0, 0, 0);
+        };
+        // the keys of the lane's four that are there, and those of them that the column sees
+        const auto look = [&](int kk, bool (&ok)[4], bool (&sees)[4]) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int key = kk + 4 * g + i;
+                ok[i] = (key >= lo || key < kf) && key <= top;
+                sees[i] = ROWS ? key <= p && on : ok[i];
+            }
+        };
+        if constexpr (AHEAD == 2) {
+            // (pages of whole tiles.  What of a tile is not there lies in its page all the same: it is read, and zeros take its place)
+            floatx4 ka[DB], va[DB], kb[DB], vb[DB];
+            const auto ask = [&](int ti, floatx4 (&kr)[DB], floatx4 (&vr)[DB]) {
+                const int in = tile_key(ti) % P;
+                const float* const page = cache + (long)page_of(ti, walk) * page_stride;
+                const float* const krow = page + ((long)kvh * P + in + n) * D + g * 4;
+                const float* const vrow = page + ((long)(Hkv + kvh) * D + n) * P + in + 4 * g;
+#pragma unroll
+                for (int c = 0; c < DB; ++c) kr[c] = *(const floatx4*)(krow + c * 16);
+#pragma unroll
+                for (int db = 0; db < DB; ++db) vr[db] = *(const floatx4*)(vrow + (long)db * 16 * P);
+            };
+            const auto step = [&](int ti, floatx4 (&kr)[DB], floatx4 (&vr)[DB]) {
+                const int kk = tile_key(ti);
+                bool ok[4], sees[4];
+                look(kk, ok, sees);
+                if (kk < lo || kk + 15 > top) {
+                    const bool row_ok = (kk + n >= lo || kk + n < kf) && kk + n <= top;
+#pragma unroll
+                    for (int c = 0; c < DB; ++c)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            kr[c][i] = row_ok ? kr[c][i] : 0.f;
+                            vr[c][i] = ok[i] ? vr[c][i] : 0.f;
+                        }
+                }
+                floatx4 pr = score(kr);
+                const float alpha = weigh(pr, sees);
+#pragma unroll
+                for (int db = 0; db < DB; ++db) add_values(db, vr[db], pr, alpha);
+            };
+            int ti = walk;
+            if (ti < n_tiles) ask(ti, ka, va);
+            while (ti < n_tiles) {
+                if (ti + F32_WALKS < n_tiles) ask(ti + F32_WALKS, kb, vb);
+                step(ti, ka, va);
+                ti += F32_WALKS;
+                if (ti >= n_tiles) break;
+                if (ti + F32_WALKS < n_tiles) ask(ti + F32_WALKS, ka, va);
+                step(ti, kb, vb);
+                ti += F32_WALKS;
+            }
+        } else {
+            floatx4 kr[DB], vr[AHEAD ? DB : 1];
+            int page = 0;
+            if (AHEAD && walk < n_tiles) {
+                page = page_of(walk, walk);
+                load_keys(tile_key(walk), page, kr);
+            }
+            for (int ti = walk; ti < n_tiles; ti += F32_WALKS) {
+                const int kk = tile_key(ti);
+                bool ok[4], sees[4];
+                look(kk, ok, sees);
+                if (!AHEAD) {
+                    page = page_of(ti, walk);
+                    load_keys(kk, page, kr);
+                }
+                long voff[4];
+                if (AHEAD) {
+                    value_places(kk, page, ok, voff);
+#pragma unroll
+                    for (int db = 0; db < DB; ++db) vr[AHEAD ? db : 0] = load_value(db, ok, voff);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                floatx4 pr = score(kr);
+                if (AHEAD && ti + F32_WALKS < n_tiles) {
+                    page = page_of(ti + F32_WALKS, walk);
+                    load_keys(tile_key(ti + F32_WALKS), page, kr);
+                }
+                const float alpha = weigh(pr, sees);
+                if (!AHEAD) value_places(kk, page, ok, voff);
+#pragma unroll
+                for (int db = 0; db < DB; ++db) add_values(db, AHEAD ? vr[AHEAD ? db : 0] : load_value(db, ok, voff), pr, alpha);
             }
         }
         l += __shfl_xor(l, 16, 64);
         l += __shfl_xor(l, 32, 64);
+        if (ROWS) {
+#pragma unroll
+            for (int db = 0; db < DB; ++db)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) odd = odd || !(fabsf(acc[db][i]) < INFINITY);
+        }
         if (NW == F32_SLOTS && walk < F32_SLOTS) leave();  // (read again by the same lane)
+    }
+    if (ROWS && __syncthreads_or(odd && on) && !one_by_one && first_p < top) {
+        todo |= __ballot(on);
+        one_by_one = true;
+        continue;
     }
     // walks w and w + 4
     if (NW == F32_SLOTS) {
@@ -242,7 +344,7 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? 3 : 1) void a
         }
     }
     __syncthreads();
-    if (wave != 0) return;
+    if (wave == 0) {
     // the four results, merged by the first wave in their order (one without a tile has m = -inf and weighs nothing)
     const float sk = sink && head_ok ? tail.sink_of(head) : 0.f;
     float M = sink ? sk : -INFINITY;                      // (the sink: one more entry without a value)
@@ -255,7 +357,7 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? 3 : 1) void a
         wgt[w] = (mw == -INFINITY) ? 0.f : expf(mw - M);
         lsum += wgt[w] * merge_lds[((long)w * (DB * 4 + 2) + DB * 4 + 1) * 64 + lane];
     }
-    if (head_ok) {
+    if (ROWS ? on : head_ok) {
         const float inv = 1.f / lsum;
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
@@ -273,6 +375,9 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? 3 : 1) void a
                 for (int i = 0; i < 4; ++i) tail.store(out, t, head, db * 16 + g * 4 + i, o[i]);
         }
     }
+    }
+    if (ROWS && todo) __syncthreads();                     // (the results' places are written again)
+    } while (ROWS && todo);
 }
 
 bool qe_attention_f32_ok(int Hq, int Hkv, int D, int P) {
@@ -288,17 +393,24 @@ int qe_attention_f32(const float* q, float* out, const float* cache, const int* 
     dim3 grid(T, Hkv * groups16);
     // eight waves while the blocks leave compute units idle
     const bool few = (long)T * Hkv * groups16 <= 256;
-#define QE_ATTN_F32_RUN(DB_, NW_, AHEAD_)                                                             \
+    const int G = Hq / Hkv;
+    const bool rows = !few && window == 0 && keep_first == 0 && G <= 8 && T / (16 / G) < 65535;
+    if (rows) grid = dim3(Hkv, qe_cdiv(T, 16 / G));
+#define QE_ATTN_F32_FORM(DB_, NW_, AHEAD_, ROWS_)                                                     \
     do {                                                                                              \
         const size_t lds = (size_t)F32_SLOTS * (DB_ * 4 + 2) * 64 * sizeof(float);                    \
-        if (lds > 48 * 1024) QE_RAISE_SHARED((attention_f32_kernel<DB_, NW_, AHEAD_>), lds);          \
-        attention_f32_kernel<DB_, NW_, AHEAD_><<<grid, 64 * NW_, lds, stream>>>(q, out, cache, positions, tok_seq, \
-                                                    block_table, max_blocks, tokens, Hq, Hkv, P, scale, window, keep_first, sink, softcap, tail); \
+        if (lds > 48 * 1024) QE_RAISE_SHARED((attention_f32_kernel<DB_, NW_, AHEAD_, ROWS_>), lds);   \
+        attention_f32_kernel<DB_, NW_, AHEAD_, ROWS_><<<grid, 64 * NW_, lds, stream>>>(q, out, cache, positions, tok_seq, \
+                                                    block_table, max_blocks, tokens, T, Hq, Hkv, P, scale, window, keep_first, sink, softcap, tail); \
     } while (0)
+#define QE_ATTN_F32_RUN(DB_, NW_, AHEAD_) QE_ATTN_F32_FORM(DB_, NW_, AHEAD_, false)
     // (beyond heads of 128 a tile ahead does not fit the registers)
+    const bool whole = P % 16 == 0;
 #define QE_ATTN_F32(DB_)                                                                              \
     case DB_:                                                                                         \
-        if (few) QE_ATTN_F32_RUN(DB_, 8, (DB_ <= 8)); else QE_ATTN_F32_RUN(DB_, 4, false);            \
+        if (few) { if (DB_ <= 8 && whole) QE_ATTN_F32_RUN(DB_, 8, (DB_ <= 8 ? 2 : 0)); else QE_ATTN_F32_RUN(DB_, 8, (DB_ <= 8)); } \
+        else if (rows) QE_ATTN_F32_FORM(DB_, 4, (DB_ <= 8), true);                                    \
+        else QE_ATTN_F32_RUN(DB_, 4, 0);                                                              \
         break;
     switch (D / 16) {
         QE_ATTN_F32(1) QE_ATTN_F32(2) QE_ATTN_F32(3) QE_ATTN_F32(4) QE_ATTN_F32(5) QE_ATTN_F32(6)
@@ -307,6 +419,7 @@ int qe_attention_f32(const float* q, float* out, const float* cache, const int* 
     }
 #undef QE_ATTN_F32
 #undef QE_ATTN_F32_RUN
+#undef QE_ATTN_F32_FORM
     QE_LAUNCH_CHECK();
     return 0;
 }
