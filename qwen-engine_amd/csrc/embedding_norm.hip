@@ -2,25 +2,41 @@
 // fused residual add and an optional row gather.
 #include "common.h"
 
-// out[t, :] = float(table[ids[t], :]).  One block per token.
+// out[t, :] = float(table[ids[t], :]).  One block per token.  And, in the blocks behind those, blocks[idx[i]] = val[i] for idx[i] >= 0, i < n: the
+// device's copy of a block table (a launch of its own is some 4 us of a decode step).
 template <typename TW>
 __global__ void embedding_kernel(const int* __restrict__ ids, const TW* __restrict__ table,
-                                 float* __restrict__ out, int H) {
+                                 float* __restrict__ out, int T, int H, int* __restrict__ blocks, const int* __restrict__ idx,
+                                 const int* __restrict__ val, int n) {
     const long t = blockIdx.x;
+    if (t >= T) {
+        const int i = (blockIdx.x - T) * blockDim.x + threadIdx.x;
+        if (i < n && idx[i] >= 0) blocks[idx[i]] = val[i];
+        return;
+    }
     const TW* row = table + (long)ids[t] * H;
     float* o = out + t * H;
+    if (H % 4 == 0 && ((unsigned long)table % (4 * sizeof(TW)) | (unsigned long)out % 16) == 0) {
+        for (int c = threadIdx.x * 4; c < H; c += blockDim.x * 4) {
+            float x[4];
+            Vec4<TW>::load(row + c, x);
+            Vec4<float>::store(o + c, x);
+        }
+        return;
+    }
     for (int c = threadIdx.x; c < H; c += blockDim.x) o[c] = Elem<TW>::load(row + c);
 }
 
 extern "C" int qe_embedding(const int* ids, const void* table, float* out, int T, int V, int H,
-                            int dt_w, hipStream_t stream) {
-    QE_REQUIRE(T >= 0 && V > 0 && H > 0, "embedding: bad sizes T=%d V=%d H=%d", T, V, H);
-    if (T == 0) return 0;
+                            int dt_w, int* blocks, const int* idx, const int* val, int n, hipStream_t stream) {
+    QE_REQUIRE(T >= 0 && V > 0 && H > 0 && n >= 0, "embedding: bad sizes T=%d V=%d H=%d, %d updates", T, V, H, n);
+    if (T == 0 && n == 0) return 0;
     const int threads = H >= 1024 ? 256 : (H >= 256 ? 128 : 64);
+    const int grid = T + qe_cdiv(n, threads);
     if (dt_w == QE_F32)
-        embedding_kernel<float><<<T, threads, 0, stream>>>(ids, (const float*)table, out, H);
+        embedding_kernel<float><<<grid, threads, 0, stream>>>(ids, (const float*)table, out, T, H, blocks, idx, val, n);
     else if (dt_w == QE_BF16)
-        embedding_kernel<bf16_t><<<T, threads, 0, stream>>>(ids, (const bf16_t*)table, out, H);
+        embedding_kernel<bf16_t><<<grid, threads, 0, stream>>>(ids, (const bf16_t*)table, out, T, H, blocks, idx, val, n);
     else
         QE_REQUIRE(false, "embedding: unknown table dtype %d", dt_w);
     QE_LAUNCH_CHECK();

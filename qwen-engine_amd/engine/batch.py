@@ -3,7 +3,7 @@ tokens.  The same description serves every mixer; each consumes what it needs.""
 from __future__ import annotations
 
 from dataclasses import dataclass, field
-from typing import Dict, Hashable, List, Optional
+from typing import Dict, Hashable, List, Optional, Sequence
 
 import torch
 
@@ -42,6 +42,9 @@ class StepContext:
     # int32 [1] in pinned host memory, or None: kernels whose blocks wait for each other write 1 to it when they have given
     # a wait up, and the step's rows are then NaN (ModelRunner.check looks at it).
     late: Optional[torch.Tensor] = None
+    # Per cache group (indices into its block table, what to write there, at -1 nothing): the model brings the tables up to date before the
+    # first layer reads them (a recorded step; else that has been done).
+    table_updates: Sequence[tuple] = ()
     # What single parts asked to have prepared for this step, by part class (see
     # ``parts.base``: step_extras / graph_extras), and a place where a part may keep what it
     # builds once per step and shares between its layers.

@@ -540,7 +540,7 @@ class ModelRunner:
 
     # ---- decoding through a recorded graph ------------------------------------------------
     def _recorded_argmax(self, logits: torch.Tensor) -> Optional[torch.Tensor]:
-        """Inside a recording: the largest logit's index of every row, into a buffer that stays (through the
+        """Inside the recording of a greedy step: the largest logit's index of every row, into a buffer that stays (through the
         entry point that allocates nothing, where the rows fit its buffer)."""
         if logits.shape[0] == 0:
             return None
@@ -579,7 +579,7 @@ class ModelRunner:
                     ops.scatter_int(self.tables[g], torch.from_numpy(upd_idx[g]).to(self.rt.device),
                                     torch.from_numpy(upd_val[g]).to(self.rt.device))
                 upd_idx[g] = upd_val[g] = np.zeros(0, dtype=i32)
-        rec = self._graph_for((B, part_keys), "decode", lambda: self._record_decode_graph(B, part_keys, cap))
+        rec = self._graph_for((B, part_keys, greedy), "decode", lambda: self._record_decode_graph(B, part_keys, cap, greedy))
         iota, none, zero = rec["iota"], rec["none"], rec["zero"]       # 0 .. B - 1; cap times -1; cap zeros
         # (a row's table row is its request's state slot: tok_seq serves as both)
         parts = [token_ids, positions, tok_seq, iota, tok_seq]
@@ -628,7 +628,7 @@ class ModelRunner:
         max_dec_position = max([self.cache.get(e.req_id).num_tokens for e in ordered[:-1]], default=0)
         portion_keys = self.cache.get(ordered[-1].req_id).num_tokens + T1
         part_keys = tuple(cls.mixed_graph_key(max_dec_position, portion_keys) for cls in self._step_classes)
-        rec = self._graph_for(("mixed", B, T, part_keys), "mixed", lambda: self._record_mixed_graph(B, T, part_keys, cap))
+        rec = self._graph_for(("mixed", B, T, part_keys, greedy), "mixed", lambda: self._record_mixed_graph(B, T, part_keys, cap, greedy))
         if rec is None:
             return None
         tokens = self._check_and_reserve(ordered)
@@ -685,7 +685,7 @@ class ModelRunner:
             return logits[:n_dec].clone()
         return logits[torch.tensor(picked, dtype=torch.long).to(self.rt.device)]
 
-    def _record_mixed_graph(self, B: int, T: int, part_keys: tuple, cap: int):
+    def _record_mixed_graph(self, B: int, T: int, part_keys: tuple, cap: int, greedy: bool = False):
         """Static buffers for a step of B single new tokens beside one prompt portion filled up to T
         tokens, one run outside the graph, then the recording.  The stand-in batch: every single token
         at position 0 of the tables' spare row, the portion at its positions 0 .. T - 1, writing nowhere."""
@@ -721,15 +721,13 @@ class ModelRunner:
         ctx = StepContext(rt=self.rt, page_size=self.page_size, num_tokens=B + T, seqs=seqs, token_ids=d_tok,
                           positions=d_pos, tok_seq=d_seq, block_tables=self.tables,
                           shared_keys=self.shared_keys, late=self._late, slots=d_slots,
-                          logit_rows=d_rows, state_slots=d_state, max_position=0,
+                          logit_rows=d_rows, state_slots=d_state, max_position=0, table_updates=d_upd,
                           extras={cls: dict(cls.mixed_graph_extras(B, T, k, dev, dyn))
                                   for cls, k, dyn in zip(self._step_classes, part_keys, d_dyn)})
 
         def run():
-            for g in range(n_groups):
-                ops.scatter_int(self.tables[g], d_upd[g][0], d_upd[g][1])
             logits = self.model.forward(ctx, self.bindings)
-            return logits, self._recorded_argmax(logits)
+            return logits, self._recorded_argmax(logits) if greedy else None
 
         torch.cuda.synchronize()
         stream = torch.cuda.Stream()
@@ -752,8 +750,8 @@ class ModelRunner:
         keys = self.cache.get(entry.req_id).num_tokens + T
         part_keys = tuple(cls.portion_graph_key(T, keys) if hasattr(cls, "portion_graph_key") else None
                           for cls in self._step_classes)
-        rec = self._graph_for(("portion", T, n_want, part_keys), "portion",
-                              lambda: self._record_portion_graph(T, n_want, cap, part_keys))
+        rec = self._graph_for(("portion", T, n_want, part_keys, greedy), "portion",
+                              lambda: self._record_portion_graph(T, n_want, cap, part_keys, greedy))
         if rec is None:
             return None
         tokens = self._check_and_reserve([entry])
@@ -783,7 +781,7 @@ class ModelRunner:
             return rec["tokens"].tolist() if rec["tokens"] is not None else []
         return rec["logits"].clone()
 
-    def _record_portion_graph(self, T: int, n_want: int, cap: int, part_keys: tuple):
+    def _record_portion_graph(self, T: int, n_want: int, cap: int, part_keys: tuple, greedy: bool = False):
         """Static buffers for a step that is one prompt portion of T tokens with n_want (0 or 1) rows
         of logits, at a place that gives the parts' ``part_keys``, one run outside the graph, then the
         recording.  The stand-in batch stands at
@@ -813,16 +811,14 @@ class ModelRunner:
         ctx = StepContext(rt=self.rt, page_size=self.page_size, num_tokens=T, seqs=seqs, token_ids=d_tok,
                           positions=d_pos, tok_seq=d_seq, block_tables=self.tables,
                           shared_keys=self.shared_keys, late=self._late, slots=d_slots,
-                          logit_rows=d_rows, state_slots=d_state, max_position=0,
+                          logit_rows=d_rows, state_slots=d_state, max_position=0, table_updates=d_upd,
                           extras={cls: dict(cls.portion_graph_extras(T, dev) if k is None
                                             else cls.portion_graph_extras(T, dev, k))
                                   for cls, k in zip(self._step_classes, part_keys)})
 
         def run():
-            for g in range(n_groups):
-                ops.scatter_int(self.tables[g], d_upd[g][0], d_upd[g][1])
             logits = self.model.forward(ctx, self.bindings)
-            return logits, self._recorded_argmax(logits)
+            return logits, self._recorded_argmax(logits) if greedy else None
 
         torch.cuda.synchronize()
         stream = torch.cuda.Stream()
@@ -836,7 +832,7 @@ class ModelRunner:
         return {"graph": graph, "held": held, "ctx": ctx, "host": host, "host_np": host.numpy(), "meta": meta, "logits": logits, "tokens": tokens,
                 "event": event, "none": np.full(cap, -1, dtype=np.int32), "zero": np.zeros(cap, dtype=np.int32)}
 
-    def _record_decode_graph(self, B: int, part_keys: tuple, cap: int):
+    def _record_decode_graph(self, B: int, part_keys: tuple, cap: int, greedy: bool = False):
         """Static buffers for a decode step of B requests whose positions give the parts'
         ``part_keys``, one run outside the graph (so that nothing is set up for the first time
         while recording), then the recording."""
@@ -867,15 +863,13 @@ class ModelRunner:
         ctx = StepContext(rt=self.rt, page_size=self.page_size, num_tokens=B, seqs=seqs, token_ids=d_tok,
                           positions=d_pos, tok_seq=d_seq, block_tables=self.tables,
                           shared_keys=self.shared_keys, late=self._late, slots=d_slots,
-                          logit_rows=d_rows, state_slots=d_state, max_position=0,
+                          logit_rows=d_rows, state_slots=d_state, max_position=0, table_updates=d_upd,
                           extras={cls: dict(cls.graph_extras(B, k, dev)) if hasattr(cls, "graph_extras") else {}
                                   for cls, k in zip(self._step_classes, part_keys)})
 
         def run():
-            for g in range(n_groups):
-                ops.scatter_int(self.tables[g], d_upd[g][0], d_upd[g][1])
             logits = self.model.forward(ctx, self.bindings)
-            return logits, self._recorded_argmax(logits)
+            return logits, self._recorded_argmax(logits) if greedy else None
 
         torch.cuda.synchronize()
         stream = torch.cuda.Stream()

@@ -42,7 +42,7 @@ def load_library():
     lib.qe_last_error.restype = ctypes.c_char_p
     vp, i32, f32, i64 = ctypes.c_void_p, ctypes.c_int, ctypes.c_float, ctypes.c_long
     sigs = {
-        "qe_embedding": [vp, vp, vp, i32, i32, i32, i32, vp],
+        "qe_embedding": [vp, vp, vp, i32, i32, i32, i32, vp, vp, vp, i32, vp],
         "qe_rmsnorm": [vp, vp, i32, i32, i64, vp, vp, vp, i32, i32, f32, i32, i32, vp],
         "qe_stream_norm": [vp, vp, i32, i32, vp, vp, i32, vp, vp, i32, vp, vp, vp, i32, i32, f32, i32, i32, vp, vp, vp, i32, vp],
         "qe_norm_conv": [vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, vp],
@@ -242,17 +242,24 @@ def _need(t: torch.Tensor, name: str, dtype=None, shape=None, device=None) -> No
 _ACT = (torch.float32, torch.bfloat16)
 
 
-def embedding(ids: torch.Tensor, table: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """out[t] = float32(table[ids[t]]).  ids int32 [T] with 0 <= id < V (the caller checks the range)."""
+def embedding(ids: torch.Tensor, table: torch.Tensor, out: Optional[torch.Tensor] = None, update: Optional[tuple] = None) -> torch.Tensor:
+    """out[t] = float32(table[ids[t]]).  ids int32 [T] with 0 <= id < V (the caller checks the range).
+    ``update``: (a block table, idx, val) of scatter_int, done in the same launch."""
     lib = load_library()
     _need(ids, "ids", torch.int32, (None,))
+    if update is not None:
+        blocks, idx, val = update
+        _need(blocks, "block table", torch.int32, None, ids.device)
+        _need(idx, "idx", torch.int32, (None,), ids.device)
+        _need(val, "val", torch.int32, (idx.shape[0],), ids.device)
     _need(table, "table", _ACT, (None, None), ids.device)
     T, (V, H) = ids.shape[0], table.shape
     if out is None:
         out = torch.empty((T, H), dtype=torch.float32, device=ids.device)
     _need(out, "out", torch.float32, (T, H), ids.device)
+    up = (blocks.data_ptr(), idx.data_ptr(), val.data_ptr(), idx.shape[0]) if update is not None else (None, None, None, 0)
     _check(lib.qe_embedding(ids.data_ptr(), table.data_ptr(), out.data_ptr(), T, V, H,
-                            _DT[table.dtype], _stream()), "embedding")
+                            _DT[table.dtype], *up, _stream()), "embedding")
     return out
 
 

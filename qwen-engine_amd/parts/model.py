@@ -140,10 +140,15 @@ class DecoderModel:
     def forward(self, ctx, bindings: List[CacheBinding]) -> torch.Tensor:
         """Runs the tokens of ctx through the schedule; returns float32 logits [R, V]."""
         with ops.one_stream():           # (the whole step runs on the stream that is current now)
+            updates = [(t, *u) for t, u in zip(ctx.block_tables, ctx.table_updates)]
+            if len(updates) != 1 or hasattr(self.prologue, "embed"):
+                for table, idx, val in updates:
+                    ops.scatter_int(table, idx, val)
+                updates = []
             if hasattr(self.prologue, "embed"):
                 h = self.prologue.embed(self.embed, ctx, bindings[len(self.spec.schedule)][0])
             else:
-                h = ops.embedding(ctx.token_ids, self.embed)
+                h = ops.embedding(ctx.token_ids, self.embed, update=updates[0] if updates else None)
                 if self.prologue is not None:
                     self.prologue.forward(h, ctx)
             pending = None

@@ -126,3 +126,20 @@ def test_single_tokens_beside_a_portion_in_one_launch(ops, hq, hkv, rows, single
     assert float((together[0].float() - apart.float()).norm() / apart.float().norm()) < 2.0 ** -8
     if rows > 1 and hq // hkv in (1, 2, 4, 8):
         assert torch.equal(together[0][singles:], apart[singles:])
+
+
+@pytest.mark.parametrize("T,H,n", [(1, 8, 2), (3, 100, 300), (9, 1024, 1), (2, 1030, 700)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_embedding_with_a_block_tables_updates(ops, T, H, n, dtype):
+    """The rows, and the table's entries as scatter_int writes them, in one launch; rows at odd addresses."""
+    emb = rand(50, H + 1, seed=1).to(dtype).to(DEV)[:, 1:].contiguous()
+    odd = torch.empty(50 * H + 1, dtype=dtype, device=DEV)[1:].view(50, H).copy_(emb)
+    ids = torch.randint(0, 50, (T,), generator=torch.Generator().manual_seed(2)).int().to(DEV)
+    idx = torch.randperm(4 * n, generator=torch.Generator().manual_seed(3))[:n].int().to(DEV)
+    idx[::3] = -1
+    val = torch.arange(n, dtype=torch.int32, device=DEV)
+    want, got = torch.full((4, n), 7, dtype=torch.int32, device=DEV), torch.full((4, n), 7, dtype=torch.int32, device=DEV)
+    ops.scatter_int(want, idx, val)
+    for table in (emb, odd):
+        assert torch.equal(ops.embedding(ids, table, update=(got, idx, val)), emb[ids.long()].float())
+    assert torch.equal(got, want) and torch.equal(ops.embedding(ids, emb), emb[ids.long()].float())
