@@ -355,3 +355,23 @@ extern "C" int qe_scatter_int(int* table, const int* idx, const int* val, int n,
     QE_LAUNCH_CHECK();
     return 0;
 }
+
+// table[idx[i]] = val[i], i < n <= 64, from the arguments: what the host knows gets there without a copy that would wait for the stream.
+struct FewInts { int idx[64], val[64]; };
+__global__ void set_ints_kernel(int* __restrict__ table, FewInts few, int n) {
+    if ((int)threadIdx.x < n) table[few.idx[threadIdx.x]] = few.val[threadIdx.x];
+}
+
+extern "C" int qe_set_ints(int* table, const int* idx, const int* val, int n, long table_size, hipStream_t stream) {
+    QE_REQUIRE(n >= 0 && n <= 64, "set ints: %d of them", n);
+    if (n == 0) return 0;
+    FewInts few{};
+    for (int i = 0; i < n; ++i) {
+        QE_REQUIRE(idx[i] >= 0 && idx[i] < table_size, "set ints: place %d of %ld", idx[i], table_size);
+        few.idx[i] = idx[i];
+        few.val[i] = val[i];
+    }
+    set_ints_kernel<<<1, 64, 0, stream>>>(table, few, n);
+    QE_LAUNCH_CHECK();
+    return 0;
+}

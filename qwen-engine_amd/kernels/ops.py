@@ -8,7 +8,7 @@ present, importing the kernels fails with the reason.
 from __future__ import annotations
 
 import ctypes
-from typing import Optional
+from typing import Optional, Sequence
 
 import torch
 
@@ -42,6 +42,7 @@ def load_library():
     lib.qe_last_error.restype = ctypes.c_char_p
     vp, i32, f32, i64 = ctypes.c_void_p, ctypes.c_int, ctypes.c_float, ctypes.c_long
     sigs = {
+        "qe_set_ints": [vp, vp, vp, i32, i64, vp],
         "qe_embedding": [vp, vp, vp, i32, i32, i32, i32, vp, vp, vp, i32, vp],
         "qe_rmsnorm": [vp, vp, i32, i32, i64, vp, vp, vp, i32, i32, f32, i32, i32, vp],
         "qe_stream_norm": [vp, vp, i32, i32, vp, vp, i32, vp, vp, i32, vp, vp, vp, i32, i32, f32, i32, i32, vp, vp, vp, i32, vp],
@@ -439,6 +440,16 @@ def scatter_int(table: torch.Tensor, idx: torch.Tensor, val: torch.Tensor) -> No
     _need(val, "val", torch.int32, (idx.shape[0],), table.device)
     _check(lib.qe_scatter_int(table.data_ptr(), idx.data_ptr(), val.data_ptr(), idx.shape[0], table.numel(),
                               _stream()), "scatter_int")
+
+
+def set_ints(table: torch.Tensor, places: Sequence[int], values: Sequence[int]) -> None:
+    """table.flatten()[places[i]] = values[i] (int32, no place twice), a launch for every 64: the numbers travel with the launch."""
+    lib = load_library()
+    _need(table, "table", torch.int32)
+    for at in range(0, len(places), 64):
+        n = min(64, len(places) - at)
+        idx, val = (ctypes.c_int * n)(*places[at:at + n]), (ctypes.c_int * n)(*values[at:at + n])
+        _check(lib.qe_set_ints(table.data_ptr(), idx, val, n, table.numel(), _stream()), "set_ints")
 
 
 def interleave_gate_up(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
