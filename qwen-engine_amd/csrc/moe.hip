@@ -36,20 +36,67 @@ __device__ __forceinline__ void wave_argmax(float& v, int& i) {
     }
 }
 
+// One token's routing by one wave, up to 64 experts, a lane each: an expert's place among the chosen is how many come before it, counted by going
+// through the lanes, and so is a group's.  (A token of 32 experts in four groups: with an argmax by shuffles for each of the two groups and four experts
+// 7.9 us, the sort behind it 6.4 in a launch of its own.)  The same scores, choices and weights as the kernel below.  zs: between two logits.
+__device__ __forceinline__ void route_grouped_lanes(const float* __restrict__ z, long zs, int* ids, float* weights, int E, int G, int keep,
+                                                    int top, int lane) {
+    const float zv = z[min(lane, E - 1) * zs];
+    const bool there = lane < E;
+    const float mx = wave_max(there ? zv : -INFINITY);
+    const float ex = there ? expf(zv - mx) : 0.f;
+    float v = ex / wave_sum(ex);
+    if (!(v == v)) v = 0.f;                // (a row of garbage still gets experts inside the table)
+    if (!there) v = -2.f;
+    const auto at = [&](float x, int l) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), l)); };
+    if (keep < G) {
+        const int per = E / G, mine = lane / per;
+        float best = -2.f;
+        int own = 0;                       // the lane's group's largest score; how many groups come before the lane's
+        for (int g = 0; g < G; ++g) {
+            float m = -1.f;
+            for (int e = g * per; e < (g + 1) * per; ++e) m = fmaxf(m, at(v, e));
+            best = g == mine ? m : best;
+        }
+        for (int g = 0; g < G; ++g) {
+            const float m = at(best, g * per);
+            own += m > best || (m == best && g < mine);
+        }
+        if (own >= keep) v = -2.f;
+    }
+    int before = 0;
+    for (int e = 0; e < E; ++e) {
+        const float o = at(v, e);
+        before += o > v || (o == v && e < lane);
+    }
+    if (there && v > -1.f && before < top) {
+        ids[before] = lane;
+        weights[before] = v;
+    }
+}
+
+__global__ __launch_bounds__(256) void moe_route_lanes_kernel(const float* __restrict__ logits, int* __restrict__ ids, float* __restrict__ weights,
+                                                              int T, int E, int G, int keep, int top, int transposed) {
+    const long t = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (t >= T) return;
+    route_grouped_lanes(transposed ? logits + t : logits + t * E, transposed ? T : 1, ids + t * top, weights + t * top, E, G, keep, top,
+                        threadIdx.x & 63);
+}
+
 // One wave per token.  Marks in the score table: -2 not (or no longer) a candidate.
 __global__ __launch_bounds__(64) void moe_route_kernel(const float* __restrict__ logits, int* __restrict__ ids,
-                                                       float* __restrict__ weights, int E, int G, int keep, int top) {
+                                                       float* __restrict__ weights, int E, int G, int keep, int top, int transposed) {
     extern __shared__ float sc[];          // E scores, G group scores
     float* gs = sc + E;
-    const long t = blockIdx.x;
+    const long t = blockIdx.x, zs = transposed ? gridDim.x : 1;
     const int lane = threadIdx.x;
-    const float* z = logits + t * E;
+    const float* z = transposed ? logits + t : logits + t * E;
     float mx = -INFINITY;
-    for (int e = lane; e < E; e += 64) mx = fmaxf(mx, z[e]);
+    for (int e = lane; e < E; e += 64) mx = fmaxf(mx, z[e * zs]);
     mx = wave_max(mx);
     float sum = 0.f;
     for (int e = lane; e < E; e += 64) {
-        const float ex = expf(z[e] - mx);
+        const float ex = expf(z[e * zs] - mx);
         sc[e] = ex;
         sum += ex;
     }
@@ -96,13 +143,15 @@ __global__ __launch_bounds__(64) void moe_route_kernel(const float* __restrict__
     }
 }
 
+// transposed: logits [E, T]
 extern "C" int qe_moe_route(const float* logits, int* ids, float* weights, int T, int E, int G, int keep, int top,
-                            hipStream_t stream) {
+                            int transposed, hipStream_t stream) {
     QE_REQUIRE(T >= 0 && E > 0 && G > 0 && E % G == 0, "moe_route: %d experts in %d groups", E, G);
     QE_REQUIRE(keep >= 1 && keep <= G && top >= 1 && top <= keep * (E / G), "moe_route: top %d of %d groups of %d", top, keep, E / G);
     QE_REQUIRE((E + G) * sizeof(float) <= 60000, "moe_route: too many experts");
     if (T == 0) return 0;
-    moe_route_kernel<<<T, 64, (E + G) * sizeof(float), stream>>>(logits, ids, weights, E, G, keep, top);
+    if (E <= 64) moe_route_lanes_kernel<<<qe_cdiv(T, 4), 256, 0, stream>>>(logits, ids, weights, T, E, G, keep, top, transposed);
+    else moe_route_kernel<<<T, 64, (E + G) * sizeof(float), stream>>>(logits, ids, weights, E, G, keep, top, transposed);
     QE_LAUNCH_CHECK();
     return 0;
 }
@@ -238,15 +287,31 @@ __device__ __forceinline__ void sort_pairs(const int* ids, int n, int E, int til
     __syncthreads();
     for (int i = tid; i < n; i += blockDim.x) atomicAdd(&counts[ids[i]], 1);
     __syncthreads();
-    for (int e = tid; e < E; e += blockDim.x) {
-        int off = 0, tb = 0;
-        for (int j = 0; j < e; ++j) {
-            off += counts[j];
-            if (j < tile_experts) tb += (counts[j] + tile_rows - 1) / tile_rows;
+    for (int e = tid; e < (E <= 64 ? min(64, (int)blockDim.x) : E); e += blockDim.x) {
+        int off = 0, tb = 0, c = 0, mine = 0;
+        if (E <= 64) {                     // (the first wave's lanes add up what lies before them)
+            c = e < E ? counts[e] : 0;
+            mine = e < tile_experts ? (c + tile_rows - 1) / tile_rows : 0;
+            off = c;
+            tb = mine;
+#pragma unroll
+            for (int k = 1; k < 64; k <<= 1) {
+                const int o = __shfl_up(off, k, 64), b = __shfl_up(tb, k, 64);
+                off += e >= k ? o : 0;
+                tb += e >= k ? b : 0;
+            }
+            off -= c;
+            tb -= mine;
+            if (e >= E) break;
+        } else {
+            for (int j = 0; j < e; ++j) {
+                off += counts[j];
+                if (j < tile_experts) tb += (counts[j] + tile_rows - 1) / tile_rows;
+            }
+            c = counts[e];
+            mine = e < tile_experts ? (c + tile_rows - 1) / tile_rows : 0;
         }
         cursor[e] = off;
-        const int c = counts[e];
-        const int mine = e < tile_experts ? (c + tile_rows - 1) / tile_rows : 0;
         for (int k = 0; k < mine; ++k) {
             tiles[3 * (tb + k)] = e;
             tiles[3 * (tb + k) + 1] = off + k * tile_rows;
@@ -307,6 +372,42 @@ __global__ __launch_bounds__(1024) void moe_front_small_kernel(
             for (int c = threadIdx.x; c < H; c += blockDim.x) dst[c] = wgt * Elem<TA>::load(src + c);
         }
     }
+}
+
+// The same for grouped routing (up to 64 experts, no identity experts).
+__global__ __launch_bounds__(1024) void moe_front_grouped_kernel(
+    const float* __restrict__ logits, int* __restrict__ ids, float* __restrict__ weights, int* __restrict__ perm, int* __restrict__ inv,
+    int* __restrict__ tiles, int* __restrict__ n_tiles, int T, int E, int G, int keep, int top, int tile_rows) {
+    extern __shared__ int sm[];
+    const int n = T * top;
+    int* ids_s = sm;                                     // n
+    float* w_s = (float*)(sm + n);                       // n
+    int* counts = sm + 2 * n;                            // E, then E cursors
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    for (int t = wave; t < T; t += waves)
+        route_grouped_lanes(logits + (long)t * E, 1, ids_s + t * top, w_s + t * top, E, G, keep, top, lane);
+    __syncthreads();
+    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+        ids[i] = ids_s[i];
+        weights[i] = w_s[i];
+    }
+    sort_pairs(ids_s, n, E, E, tile_rows, perm, inv, tiles, n_tiles, counts, counts + E);
+}
+
+extern "C" int qe_moe_front_grouped_supported(int T, int E, int top) { return T > 0 && E <= 64 && (long)T * top <= 1024; }
+
+// logits float [T, E]; otherwise as qe_moe_route and qe_moe_sort.
+extern "C" int qe_moe_front_grouped(const float* logits, int* ids, float* weights, int* perm, int* inv, int* tiles, int* n_tiles, int max_tiles,
+                                    int T, int E, int G, int keep, int top, int tile_rows, hipStream_t stream) {
+    QE_REQUIRE(qe_moe_front_grouped_supported(T, E, top), "moe_front_grouped: %d tokens, %d experts, top %d", T, E, top);
+    QE_REQUIRE(G > 0 && E % G == 0 && keep >= 1 && keep <= G && top >= 1 && top <= keep * (E / G) && tile_rows > 0, "moe_front_grouped: top %d of %d groups of %d of %d",
+               top, keep, G, E);
+    const int n = T * top;
+    QE_REQUIRE(max_tiles >= (n + tile_rows - 1) / tile_rows + (E < n ? E : n), "moe_front_grouped: %d tiles may not be enough", max_tiles);
+    moe_front_grouped_kernel<<<1, 64 * (T < 16 ? T : 16), (2 * n + 2 * E) * sizeof(int), stream>>>(logits, ids, weights, perm, inv, tiles, n_tiles, T, E, G,
+                                                                                                 keep, top, tile_rows);
+    QE_LAUNCH_CHECK();
+    return 0;
 }
 
 extern "C" int qe_moe_front_small_supported(int T, int E, int top) {

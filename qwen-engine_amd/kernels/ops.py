@@ -130,7 +130,9 @@ def load_library():
         "qe_gemm_heads": [vp, i64, i64, vp, vp, i64, i64, vp, i64, i64, i64, i32, i32, i32, i32, i32, i32, vp],
         "qe_gemm_heads_mfma_supported": [i32, i64, i64],
         "qe_gemm_heads_mfma": [vp, i64, i64, vp, vp, i64, i64, vp, i64, i64, i64, i32, i32, i32, i32, vp],
-        "qe_moe_route": [vp, vp, vp, i32, i32, i32, i32, i32, vp],
+        "qe_moe_route": [vp, vp, vp, i32, i32, i32, i32, i32, i32, vp],
+        "qe_moe_front_grouped_supported": [i32, i32, i32],
+        "qe_moe_front_grouped": [vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, i32, vp],
         "qe_moe_sort": [vp, i32, i32, i32, i32, vp, vp, vp, vp, i32, vp],
         "qe_moe_gemm": [vp, vp, i32, vp, vp, vp, vp, vp, i32, i32, i32, i32, f32, f32, i32, i32, i32, i32, vp],
         "qe_moe_gather": [vp, vp, i32, vp, i32, i32, i32, vp],
@@ -1462,17 +1464,17 @@ def gemm_heads(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gate: Option
 
 
 # ---- mixture of experts -----------------------------------------------------------------------------------
-def moe_route(logits: torch.Tensor, groups: int, keep: int, top: int):
-    """logits float32 [T, E] -> (ids int32 [T, top], weights float32 [T, top]): softmax over all experts,
+def moe_route(logits: torch.Tensor, groups: int, keep: int, top: int, transposed: bool = False):
+    """logits float32 [T, E] (``transposed``: [E, T]) -> (ids int32 [T, top], weights float32 [T, top]): softmax over all experts,
     the ``keep`` best of ``groups`` equal groups of neighbours (a group's score is its largest), the ``top``
     largest scores among them, as they are."""
     lib = load_library()
     _need(logits, "logits", torch.float32, (None, None))
-    T, E = logits.shape
+    T, E = reversed(logits.shape) if transposed else logits.shape
     ids = torch.empty((T, top), dtype=torch.int32, device=logits.device)
     weights = torch.empty((T, top), dtype=torch.float32, device=logits.device)
     _check(lib.qe_moe_route(logits.data_ptr(), ids.data_ptr(), weights.data_ptr(), T, E, int(groups), int(keep),
-                            int(top), _stream()), "moe_route")
+                            int(top), int(transposed), _stream()), "moe_route")
     return ids, weights
 
 
@@ -1561,7 +1563,7 @@ def moe_experts(x: torch.Tensor, ids: Optional[torch.Tensor], weights: Optional[
                 algo: int = ALGO_AUTO, act: str = "gated", identity: int = 0,
                 rows_dtype: torch.dtype = torch.float32, biased_route=None,
                 parts_out: Optional[torch.Tensor] = None, sigmoid_route: bool = False,
-                weigh_input: bool = False) -> torch.Tensor:
+                weigh_input: bool = False, grouped_route=None) -> torch.Tensor:
     """The chosen experts' outputs, weighted: float32 [S, T, H] whose sum over S, in order, is the mixture's
     output (S = top: a token's choices in their order; or S = 1: already added up in that order).
     x [T, K]; w_gate_up [E, 2 F, K] (gate rows, then up rows; or, ``interleaved``, in alternating blocks of
@@ -1578,7 +1580,8 @@ def moe_experts(x: torch.Tensor, ids: Optional[torch.Tensor], weights: Optional[
     where they are the first of more): a step of few tokens then
     routes, sorts and writes the identity experts' rows in one launch.  ``limit`` 0: the plain silu(g) u.  ``parts_out``: float32 [top, T, H] to take the
     parts (the paths of fewer than 1024 pairs only).  ``sigmoid_route``: the routing's scores are sigmoids, see
-    moe_route_biased.  ``weigh_input``: a pair's weight multiplies what its expert reads instead of what it gives.
+    moe_route_biased.  ``grouped_route``: instead of ids and weights, (logits, groups, keep, top, transposed) for the routing of moe_route: a step
+    of few tokens then routes and sorts in one launch.  ``weigh_input``: a pair's weight multiplies what its expert reads instead of what it gives.
 
     The (token, choice) pairs are grouped by expert on the device.  bfloat16 with many pairs: their rows are
     gathered side by side and both products run on the tiled kernel of the dense products, a tile of 128
@@ -1606,6 +1609,12 @@ def moe_experts(x: torch.Tensor, ids: Optional[torch.Tensor], weights: Optional[
             _need(r_corr, "correction", torch.float32, (r_outputs,), dev)
         if r_bias is not None:
             _need(r_bias, "logit_bias", torch.float32, (r_outputs,), dev)
+    elif grouped_route is not None:
+        if ids is not None or weights is not None or identity:
+            raise KernelError("moe_experts: ids and weights, or a route to compute them, not both; no identity experts with groups")
+        g_logits, g_groups, g_keep, top, g_transposed = grouped_route
+        top = int(top)
+        _need(g_logits, "logits", torch.float32, (w_gate_up.shape[0], T) if g_transposed else (T, w_gate_up.shape[0]), dev)
     else:
         _need(ids, "ids", torch.int32, (T, None), dev)
         top = ids.shape[1]
@@ -1665,6 +1674,16 @@ def moe_experts(x: torch.Tensor, ids: Optional[torch.Tensor], weights: Optional[
         else:
             ids, weights = moe_route_biased(r_logits, r_corr, top, r_scale, transposed=r_transposed, logit_bias=r_bias,
                                             experts=r_outputs, sigmoid=sigmoid_route)
+    if grouped_route is not None:
+        if not g_transposed and lib.qe_moe_front_grouped_supported(T, E, top):
+            ids = torch.empty((T, top), dtype=torch.int32, device=dev)
+            weights = torch.empty((T, top), dtype=torch.float32, device=dev)
+            _check(lib.qe_moe_front_grouped(g_logits.data_ptr(), ids.data_ptr(), weights.data_ptr(), perm.data_ptr(), inv.data_ptr(),
+                                            tiles.data_ptr(), n_tiles.data_ptr(), max_tiles, T, E, int(g_groups), int(g_keep), top,
+                                            tile_rows, _stream()), "moe_front_grouped")
+            fused_front = True
+        else:
+            ids, weights = moe_route(g_logits, g_groups, g_keep, top, bool(g_transposed))
     # (identity experts are buckets of the sort like the others, behind them, and get no tiles)
     if not fused_front:
         _check(lib.qe_moe_sort(ids.data_ptr(), n, E + identity, E, tile_rows, perm.data_ptr(), inv.data_ptr(), tiles.data_ptr(),

@@ -91,9 +91,12 @@ class GroupedMoE:
 
     def forward(self, x: torch.Tensor, ctx, parts_out: Optional[torch.Tensor] = None) -> torch.Tensor:
         s = self.spec
-        logits = ops.gemm(x, self.w_router, out_dtype=torch.float32)
-        ids, weights = ops.moe_route(logits, s.num_groups, s.keep_groups, s.top)
-        return ops.moe_experts(x, ids, weights, self.w_gate_up, self.w_down, s.limit, s.slope, interleaved=self.interleaved)
+        # (many rows against the router's few: the product the other way round fills the chip, see BiasedMoE)
+        transposed = x.shape[0] > 64 and self.w_router.shape[0] <= 64
+        logits = ops.gemm(self.w_router, x, out_dtype=torch.float32) if transposed else \
+            ops.gemm(x, self.w_router, out_dtype=torch.float32)
+        return ops.moe_experts(x, None, None, self.w_gate_up, self.w_down, s.limit, s.slope, interleaved=self.interleaved,
+                               grouped_route=(logits, s.num_groups, s.keep_groups, s.top, transposed))
 
 
 class BiasedMoE:
