@@ -201,6 +201,14 @@ __device__ __forceinline__ float block_max(float v, float* scratch) {
     return r;
 }
 
+// A thread's share of a row's sum of squares, four numbers more: rounding by rounding the same wherever a row is normed.
+__device__ __forceinline__ float add_squares(float ss, const float (&v)[4], bool first) {
+    ss = __builtin_fmaf(v[0], v[0], first ? v[1] * v[1] : ss);
+    if (!first) ss = __builtin_fmaf(v[1], v[1], ss);
+    ss = __builtin_fmaf(v[2], v[2], ss);
+    return __builtin_fmaf(v[3], v[3], ss);
+}
+
 // ---- host side ---------------------------------------------------------------
 // Entry points return 0 on success, a positive hipError_t, or -1 for an argument
 // the kernels do not take; qe_last_error() then holds the reason.

@@ -223,8 +223,8 @@ __global__ __launch_bounds__(256) void rmsnorm_regs_kernel(float* __restrict__ h
 #pragma unroll
     for (int i = 0; i < NV; ++i)
         if (ok[i]) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) ss += (v[i][e] - mean) * (v[i][e] - mean);
+            const float off[4] = {v[i][0] - mean, v[i][1] - mean, v[i][2] - mean, v[i][3] - mean};
+            ss = add_squares(ss, off, i == 0);
         }
     ss = block_sum(ss, red);
     const float rstd = rsqrtf(ss / (float)H + eps);

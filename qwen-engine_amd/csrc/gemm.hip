@@ -9,6 +9,10 @@ int qe_gemm_skinny(const void* x, const void* w, const float* bias, void* out, i
                    const float* delta, int n_delta, float* h_out, hipStream_t stream);
 bool qe_gemm_skinny_norm_ok(int M, int N, int K);
 int qe_gemm_skinny_splits(int N, int K);
+bool qe_gemm_f32_silu_ok(int M, int N, int K);
+bool qe_gemm_f32_norm_ok(int M, int N, int K);
+int qe_gemm_f32_few(const float* x, const float* w, const float* bias, float* out, int M, int N, int K, bool silu, const float* norm_w,
+                    float norm_eps, const float* delta, int n_delta, float* h_out, hipStream_t stream);
 bool qe_gemm_mfma_ok(int M, int N, int K, int dt_a, int dt_w);
 float qe_gemm_mfma_shape(int M, int N, int K, int splits, int* tile, bool largest = true);
 float qe_gemm_mfma_uncut(int M, int N, int K);
@@ -28,8 +32,9 @@ extern "C" int qe_gemm_fused_supported(int M, int N, int K, int dt_a, int dt_w) 
 }
 
 // 1 if the product can take the RMSNorm before it as its prologue (qe_gemm's norm_w): x is then the
-// 32-bit stream; few rows, bfloat16 weights (N counts the weight rows)
+// 32-bit stream; few rows, bfloat16 or 32-bit weights (N counts the weight rows)
 extern "C" int qe_gemm_norm_supported(int M, int N, int K, int dt_w) {
+    if (dt_w == QE_F32) return qe_gemm_f32_norm_ok(M, N, K) ? 1 : 0;
     return (dt_w == QE_BF16 && qe_gemm_skinny_ok(M, N, K, QE_BF16, dt_w) && qe_gemm_skinny_norm_ok(M, N, K) &&
             !((long)N * K >= (16L << 20) && M > 16)) ? 1 : 0;
 }
@@ -44,13 +49,14 @@ extern "C" int qe_gemm_norm_max_rows() { return 16; }
 // 7 % longer with the prologue), and at most 192 KB of rows and partial products (every block reads all of
 // them for all rows; beyond that the norm's kernel, which reads them once, is quicker).
 extern "C" int qe_gemm_norm_preferred(int M, int N, int K, int dt_w, int n_delta) {
-    return (qe_gemm_norm_supported(M, N, K, dt_w) && (long)N * K <= (8L << 20) &&
+    return (qe_gemm_norm_supported(M, N, K, dt_w) && (long)N * K <= (8L << 20) && (dt_w == QE_BF16 || n_delta <= 1) &&
             (long)M * K * 4 * (1 + n_delta) <= 192L * 1024) ? 1 : 0;
 }
 
 // 1 if epilogue 4 (silu-mul over interleaved gate|up rows) can be used: N counts the outputs
 extern "C" int qe_gemm_silu_supported(int M, int N, int K, int dt_a, int dt_w) {
-    return (N % 32 == 0 && (qe_gemm_skinny_ok(M, N, K, dt_a, dt_w) || qe_gemm_mfma_ok(M, 2 * N, K, dt_a, dt_w))) ? 1 : 0;
+    return (N % 32 == 0 && (qe_gemm_skinny_ok(M, N, K, dt_a, dt_w) || qe_gemm_mfma_ok(M, 2 * N, K, dt_a, dt_w) ||
+                            (dt_a == QE_F32 && dt_w == QE_F32 && qe_gemm_f32_silu_ok(M, 2 * N, K)))) ? 1 : 0;
 }
 
 // 1 if epilogue 5 (the exact gelu) can be used
@@ -151,10 +157,18 @@ extern "C" int qe_gemm(const void* x, const void* w, const float* bias, void* ou
                    "gemm: M=%d N=%d K=%d is not taken with the norm as prologue", M, N, K);
         QE_REQUIRE(epilogue == EPI_STORE || epilogue == EPI_SILU_MUL || epilogue == EPI_SILU_MUL_IL,
                    "gemm: the norm prologue goes with the store and silu-mul epilogues");
+        if (dt_w == QE_F32) {
+            QE_REQUIRE(dt_o == QE_F32 && epilogue != EPI_SILU_MUL, "gemm: the norm prologue of 32-bit weights gives 32-bit numbers, with silu-mul "
+                       "over interleaved rows");
+            return qe_gemm_f32_few((const float*)x, (const float*)w, bias, (float*)out, M, N, K, epilogue == EPI_SILU_MUL_IL, norm_w, norm_eps,
+                                   delta, n_delta, h_out, stream);
+        }
         return qe_gemm_skinny(x, w, bias, out, M, N, K, dt_o, epilogue, 1, norm_w, norm_eps, delta, n_delta, h_out, stream);
     }
     const bool skinny = qe_gemm_skinny_ok(M, N, K, dt_a, dt_w);
     const bool tiled = qe_gemm_mfma_ok(M, N, K, dt_a, dt_w);
+    if (epilogue == EPI_SILU_MUL_IL && dt_a == QE_F32 && dt_w == QE_F32 && dt_o == QE_F32)
+        return qe_gemm_f32_few((const float*)x, (const float*)w, bias, (float*)out, M, N, K, true, nullptr, 0.f, nullptr, 0, nullptr, stream);
     if (epilogue == EPI_SILU_MUL_IL && (!skinny || tiled_for_few_rows(M, 2 * N, K, dt_a, dt_w))) {
         QE_REQUIRE(N % 32 == 0 && qe_gemm_mfma_ok(M, 2 * N, K, dt_a, dt_w),
                    "gemm: M=%d N=%d K=%d is not taken by a silu-mul kernel", M, N, K);

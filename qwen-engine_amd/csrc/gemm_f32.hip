@@ -79,22 +79,99 @@ __device__ __forceinline__ floatx4 four_of_row(const float* __restrict__ row, in
     return v;
 }
 
+// The residual sum and the RMSNorm in front of a product of few rows: delta (or null): n_delta tensors [M, K] one after the other; the sums go to
+// h_out [M, K].
+struct RowsNorm {
+    const float* weight;
+    float eps;
+    const float* delta;
+    int n_delta;
+    float* h_out;
+};
+constexpr int NORM_ROOM = 8192, NORM_PAD = 16;       // numbers of the normed rows; behind each (rows' reads in other banks)
+
+// A row is normed by the number of threads that the norm's own kernel has for it (a thread a piece of four, at most 256), pieces and sums
+// in its order, as many rows at once as the block has such groups.
+__device__ __forceinline__ void norm_rows(const float* __restrict__ h, const RowsNorm& norm, float* normed, int M, int K, bool store) {
+    __shared__ float red[CHUNKS];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), waves = blockDim.x >> 6;
+    const int wide = min(4, (K + 255) / 256), threads = wide * 64, at_once = waves / wide, mine = wave / wide;
+    const int tid = threadIdx.x - mine * threads;
+    constexpr int NV = 4;                                   // (K <= 4096)
+    for (int m0 = 0; m0 < M; m0 += at_once) {
+        const int m = m0 + mine;
+        const bool on = mine < at_once && m < M;
+        const long row = (long)min(m, M - 1) * K;
+        float v[NV][4], wv[NV][4];
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+            if (i * threads * 4 < K) {
+                const int c = (tid + i * threads) * 4, at = c < K ? c : 0;
+                Vec4<float>::load(h + row + at, v[i]);
+                Vec4<float>::load(norm.weight + at, wv[i]);
+            }
+        for (int s = 0; s < norm.n_delta; ++s) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i)
+                if (i * threads * 4 < K) {
+                    const int c = (tid + i * threads) * 4, at = c < K ? c : 0;
+                    float d[4];
+                    Vec4<float>::load(norm.delta + (long)s * M * K + row + at, d);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[i][e] += d[e];
+                }
+        }
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+            if ((tid + i * threads) * 4 < K) ss = add_squares(ss, v[i], i == 0);
+        ss = wave_sum(ss);
+        if (m0) __syncthreads();                            // (the rows before have been read out)
+        if ((threadIdx.x & 63) == 0) red[wave] = ss;
+        __syncthreads();
+        float sum = 0.f;
+        for (int i = 0; i < wide; ++i) sum += red[min(mine * wide + i, waves - 1)];
+        const float rstd = rsqrtf(sum / (float)K + norm.eps);
+        if (on) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i) {
+                const int c = (tid + i * threads) * 4;
+                if (c < K) {
+                    if (store && norm.delta) Vec4<float>::store(norm.h_out + row + c, v[i]);
+                    float o[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) o[e] = v[i][e] * rstd * wv[i][e];
+                    Vec4<float>::store(normed + m * (K + NORM_PAD) + c, o);
+                }
+            }
+        }
+    }
+    __syncthreads();
+}
+
 // 16 MT rows a block (blockIdx.y: which).  Lane (g, r), g = lane / 16, r = lane % 16, brings W[n0 + r][k + 4 g .. + 4] and the same of x's row r.
 // BATCH steps are asked for at once, the next batch before the current one is multiplied.
-template <int MT, int NT, int BATCH, int ROWS>
+// SILU (NT = 2): w has the gate and up rows in alternating blocks of 32; a block has 16 outputs, their gate rows and their up rows, and stores
+// silu(gate) * up.
+// NORM (rows of at most NORM_ROOM numbers in all): x is the stream; what is to be added to it and the RMSNorm come first, with the sums and
+// roundings of the norm's own kernel, while the first weights are on their way; the normed rows stay in shared memory.
+template <int MT, int NT, int BATCH, int ROWS, bool SILU = false, bool NORM = false>
 __global__ __launch_bounds__(64 * CHUNKS) void gemm_f32_rows_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                     const float* __restrict__ bias, float* __restrict__ out,
-                                                                    int M, int N, int K, int chunk) {
-    __shared__ float part[CHUNKS][MT * NT][4][64];
+                                                                    int M, int N, int K, int chunk, RowsNorm norm) {
+    __shared__ float sums[NORM ? 1 : CHUNKS * MT * NT * 256];
+    extern __shared__ __attribute__((aligned(16))) float normed[];     // NORM: [M][K + NORM_PAD], then the chunks' sums in their place
+    float* const part = NORM ? normed : sums;                          // [chunk][MT * NT][4][64]
+    constexpr int TILE = 256, PART = MT * NT * TILE;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, r = lane & 15;
-    const int n0 = blockIdx.x * (16 * NT), m0 = blockIdx.y * (16 * MT);
+    const int n0 = blockIdx.x * (SILU ? 16 : 16 * NT), m0 = blockIdx.y * (16 * MT);
     const int k_lo = wave * chunk, k_hi = k_lo + chunk < K ? k_lo + chunk : K;   // (a block has a wave per chunk that holds some of K)
     const float* wrow[NT];
     const float* xrow[MT];
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
-        const int n = n0 + 16 * j + r;
-        wrow[j] = w + (long)(n < N ? n : N - 1) * K + 4 * g;
+        const int n = SILU ? (n0 & ~31) * 2 + 32 * j + (n0 & 31) + r : n0 + 16 * j + r;
+        wrow[j] = w + (long)(SILU || n < N ? n : N - 1) * K + 4 * g;
     }
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
@@ -115,13 +192,15 @@ __global__ __launch_bounds__(64 * CHUNKS) void gemm_f32_rows_kernel(const float*
 #pragma unroll
             for (int j = 0; j < NT; ++j) wv[buf][b][j] = four_of_row<ROWS>(wrow[j], k, K - 4 * g);
 #pragma unroll
-            for (int i = 0; i < MT; ++i) xv[buf][b][i] = four_of_row<ROWS>(xrow[i], k, K - 4 * g);
+            for (int i = 0; i < MT; ++i)
+                if (!NORM) xv[buf][b][i] = four_of_row<ROWS>(xrow[i], k, K - 4 * g);
         }
     };
     auto multiply = [&](int buf, int k0) {
 #pragma unroll
         for (int b = 0; b < BATCH; ++b) {
             if (k0 + b * FK > last) break;
+            if (NORM) xv[buf][b][0] = *(const floatx4*)(normed + min(r, M - 1) * (K + NORM_PAD) + 4 * g + k0 + b * FK);
 #pragma unroll
             for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -132,28 +211,47 @@ __global__ __launch_bounds__(64 * CHUNKS) void gemm_f32_rows_kernel(const float*
         }
     };
     ask(0, k_lo);
+    if constexpr (NORM) norm_rows(x, norm, normed, M, K, blockIdx.x == 0);
     for (int k0 = k_lo; k0 <= last; k0 += 2 * BATCH * FK) {
         ask(1, k0 + BATCH * FK);
         multiply(0, k0);
         ask(0, k0 + 2 * BATCH * FK);
         multiply(1, k0 + BATCH * FK);
     }
+    if (NORM) __syncthreads();
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) part[wave][i * NT + j][e][lane] = acc[i][j][e];
+            for (int e = 0; e < 4; ++e) part[wave * PART + (i * NT + j) * TILE + e * 64 + lane] = acc[i][j][e];
     __syncthreads();
     const int waves = blockDim.x >> 6;
-    for (int at = threadIdx.x; at < MT * NT * 256; at += blockDim.x) {
-        const int l = at & 63, e = (at >> 6) & 3, tile = at >> 8;
+    const auto sum_of = [&](int tile, int e, int l) {
+        const float* const of = part + tile * TILE + e * 64 + l;
         float total = 0.f;
         for (int q = 0; 4 * q < waves; ++q) {
-            float quarter = part[4 * q][tile][e][l];
-            for (int c = 4 * q + 1; c < 4 * q + 4 && c < waves; ++c) quarter += part[c][tile][e][l];
+            float quarter = of[4 * q * PART];
+            for (int c = 4 * q + 1; c < 4 * q + 4 && c < waves; ++c) quarter += of[c * PART];
             total = q ? total + quarter : quarter;
         }
+        return total;
+    };
+    if constexpr (SILU) {
+        for (int at = threadIdx.x; at < 256; at += blockDim.x) {
+            const int l = at & 63, e = at >> 6, m = m0 + 4 * (l >> 4) + e, n = n0 + (l & 15), row = (n & ~31) * 2 + (n & 31);
+            float gate = sum_of(0, e, l), up = sum_of(1, e, l);
+            if (bias) {
+                gate += bias[row];
+                up += bias[row + 32];
+            }
+            if (m < M) out[(long)m * N + n] = gate / (1.f + expf(-gate)) * up;
+        }
+        return;
+    }
+    for (int at = threadIdx.x; at < MT * NT * 256; at += blockDim.x) {
+        const int l = at & 63, e = (at >> 6) & 3, tile = at >> 8;
+        const float total = sum_of(tile, e, l);
         const int m = m0 + (tile / NT) * 16 + 4 * (l >> 4) + e, n = n0 + (tile % NT) * 16 + (l & 15);
         if (m < M && n < N) out[(long)m * N + n] = bias ? total + bias[n] : total;
     }
@@ -338,12 +436,47 @@ static void launch_rows(const float* x, const float* w, const float* bias, float
                         hipStream_t stream) {
     const int chunk = chunk_len(K), waves = qe_cdiv(K, chunk);
     const dim3 grid(qe_cdiv(N, 16 * NT), qe_cdiv(M, 16 * MT));
-#define QE_F32_ROWS(R_) gemm_f32_rows_kernel<MT, NT, BATCH, R_><<<grid, 64 * waves, 0, stream>>>(x, w, bias, out, M, N, K, chunk)
+#define QE_F32_ROWS(R_) gemm_f32_rows_kernel<MT, NT, BATCH, R_><<<grid, 64 * waves, 0, stream>>>(x, w, bias, out, M, N, K, chunk, RowsNorm{})
     if (rows == ROWS_STEPS) QE_F32_ROWS(ROWS_STEPS);
     else if (rows == ROWS_FOURS) QE_F32_ROWS(ROWS_FOURS);
     else if (rows == ROWS_ANY) QE_F32_ROWS(ROWS_ANY);
     else QE_F32_ROWS(ROWS_SHORT);
 #undef QE_F32_ROWS
+}
+
+// Whether up to 16 rows against a matrix [N, K] go by whole lines (see qe_gemm_f32).
+static bool by_lines(int M, int N, int K) {
+    return N >= 16384 && (K >= 608 || (K > 512 && (M > 2 || N >= 30000))) && K <= 4 * FK * CHUNKS && K % 32 == 0;
+}
+
+// The products of few rows with the steps beside them inside (N: the rows of w): silu(gate) * up over rows interleaved in blocks of 32, and
+// the residual sum and the norm in front.  K in whole steps of 16.
+bool qe_gemm_f32_silu_ok(int M, int N, int K) { return M <= 16 && N % 64 == 0 && K % FK == 0 && !by_lines(M, N, K); }
+bool qe_gemm_f32_norm_ok(int M, int N, int K) {
+    return M <= 16 && K % FK == 0 && K >= 256 && K <= 4096 && (long)M * K <= NORM_ROOM && !by_lines(M, N, K);
+}
+
+// N: outputs.  norm_w null: no norm.
+int qe_gemm_f32_few(const float* x, const float* w, const float* bias, float* out, int M, int N, int K, bool silu, const float* norm_w,
+                    float norm_eps, const float* delta, int n_delta, float* h_out, hipStream_t stream) {
+    const int rows = silu ? 2 * N : N;
+    QE_REQUIRE((silu || norm_w) && (!silu || qe_gemm_f32_silu_ok(M, rows, K)) && (!norm_w || qe_gemm_f32_norm_ok(M, rows, K)),
+               "gemm (32-bit): %d rows against [%d, %d] are not taken with the steps beside them", M, rows, K);
+    QE_REQUIRE(!delta || (n_delta >= 1 && h_out && h_out != x), "gemm (32-bit): the sums of %d tensors want a place of their own", n_delta);
+    const int chunk = chunk_len(K), waves = qe_cdiv(K, chunk);
+    const RowsNorm norm = {norm_w, norm_eps, delta, delta ? n_delta : 0, h_out};
+    const long rows_room = (long)M * (K + NORM_PAD);
+#define QE_F32_FEW(NT_, B_, S_, N_)                                                                                  \
+    const size_t room = (N_) ? (rows_room > (NT_) * waves * 256L ? rows_room : (NT_) * waves * 256L) * sizeof(float) : 0; \
+    gemm_f32_rows_kernel<1, NT_, B_, ROWS_STEPS, S_, N_><<<qe_cdiv(N, (S_) ? 16 : 16 * (NT_)), 64 * waves, room, stream>>>( \
+        x, w, bias, out, M, N, K, chunk, norm)
+    if (silu && norm_w) { QE_F32_FEW(2, 1, true, true); }
+    else if (silu) { QE_F32_FEW(2, 1, true, false); }
+    else if (M > 4 && N >= 6144) { QE_F32_FEW(2, 1, false, true); }
+    else { QE_F32_FEW(1, 2, false, true); }
+#undef QE_F32_FEW
+    QE_LAUNCH_CHECK();
+    return 0;
 }
 
 int qe_gemm_f32(const float* x, const float* w, const float* bias, float* out, int M, int N, int K,
@@ -361,7 +494,7 @@ int qe_gemm_f32(const float* x, const float* w, const float* bias, float* out, i
         // and nine chunks, a matrix of fewer than 30000 rows goes by a wave a chunk (one row, by rows and by lines: 18000 x 544 12.7 us and
         // 14.5, 20001 x 576 13.5 and 15.6, 18000 x 608 13.9 and 14.8, 20001 x 608 15.5 and 15.7, 32768 x 544 20.6 and 19.1; eight rows: 20001 x 576 16.8 and
         // 15.9, 32768 x 608 26.6 and 21.0; with eight chunks or fewer a wave's walk is not worth a block: 20000 x 96 4.7 and 6.9)
-        if (M <= 16 && N >= 16384 && (K >= 608 || (K > 512 && (M > 2 || N >= 30000))) && K <= 4 * FK * CHUNKS && K % 32 == 0 && (((unsigned long)w) & 15) == 0)
+        if (M <= 16 && by_lines(M, N, K) && (((unsigned long)w) & 15) == 0)
             gemm_f32_lines_kernel<<<qe_cdiv(N, 16), 64 * qe_cdiv(K, 16 * FK), 0, stream>>>(x, w, bias, out, M, N, K);
         else if (M > 4 && M <= 16 && N >= 6144) launch_rows<1, 2, 1>(x, w, bias, out, M, N, K, rows, stream);
         else if (M <= 16) launch_rows<1, 1, 2>(x, w, bias, out, M, N, K, rows, stream);

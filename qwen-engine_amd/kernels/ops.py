@@ -492,7 +492,7 @@ def gemm_silu_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 def gemm_norm_supported(M: int, w: torch.Tensor) -> bool:
     """True if gemm can take the RMSNorm that stands before the product as its prologue (``norm_weight``)
-    for M rows of the stream against w: up to 16 rows, bfloat16 weights."""
+    for M rows of the stream against w: up to 16 rows (float32 weights: of at most 8192 numbers in all)."""
     lib = load_library()
     return w.dtype in _DT and bool(lib.qe_gemm_norm_supported(int(M), w.shape[0], w.shape[1], _DT[w.dtype]))
 
@@ -527,7 +527,7 @@ def gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
     epilogue EPI_GELU: the exact gelu of the 32-bit sums, in bfloat16, without a bias; needs gemm_gelu_supported(x, w).
 
     norm_weight (float32 [K]) with norm_eps: x is the 32-bit stream and the RMSNorm of its rows, rounded
-    to bfloat16 as the norm kernel rounds it, is what is multiplied (out_dtype defaults to bfloat16);
+    to w's type as the norm kernel rounds it, is what is multiplied (out_dtype defaults to w's type);
     needs gemm_norm_supported(M, w); with the store and silu-mul epilogues.  With it, ``delta`` (float32
     [S, M, K], the partial products of the branch before) is added to the stream's rows, in the order
     of S, before the norm, and the sums are written to ``stream_out`` [M, K], another tensor than x (every
@@ -546,7 +546,7 @@ def gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
         _need(norm_weight, "norm_weight", torch.float32, (K,), x.device)
         if not gemm_norm_supported(M, w):
             raise KernelError(f"gemm: {M} rows against {tuple(w.shape)} are not taken with the norm as prologue")
-        out_dtype = out_dtype or torch.bfloat16
+        out_dtype = out_dtype or w.dtype
         if delta is not None:
             _need(delta, "delta", torch.float32, (None, M, K), x.device)
             if stream_out is None:

@@ -198,23 +198,24 @@ class StreamInput:
 
     def fusable(self) -> bool:
         """True if a product can take the residual sum and the norm as its prologue at all: nothing to
-        add, or float32 partial products and a second buffer for the sums."""
+        add, or float32 partial products (in the float32 mode also a whole one) and a second buffer for the sums."""
         d = self.delta
         if isinstance(d, (BranchSum, NormedBranch)):
             return False
-        return d is None or (d.dim() == 3 and d.dtype == torch.float32 and self.stream.spare is not None)
+        return d is None or ((d.dim() == 3 or self.rt.dtype == torch.float32) and d.dtype == torch.float32 and self.stream.spare is not None)
 
     def prefers_prologue(self, ops, w: torch.Tensor) -> bool:
         """True if the product against w should do the sum and the norm itself (the kernel library knows up
         to which sizes that is quicker than the norm's own kernel); else the part calls materialize()."""
-        parts = 0 if self.delta is None else self.delta.shape[0]
-        return self.rt.dtype == torch.bfloat16 and ops.gemm_norm_preferred(self.rows, w, parts)
+        parts = 0 if self.delta is None else self.delta.shape[0] if self.delta.dim() == 3 else 1
+        return w.dtype == self.rt.dtype and ops.gemm_norm_preferred(self.rows, w, parts)
 
     def gemm(self, ops, w: torch.Tensor, bias=None, **kw) -> torch.Tensor:
         """The product of the normed rows with w, the residual sum and the norm inside it."""
         if self.delta is None:
             return ops.gemm(self.stream.h, w, bias, norm_weight=self.weight, norm_eps=self.eps, **kw)
-        y = ops.gemm(self.stream.h, w, bias, norm_weight=self.weight, norm_eps=self.eps, delta=self.delta,
+        delta = self.delta if self.delta.dim() == 3 else self.delta.unsqueeze(0)
+        y = ops.gemm(self.stream.h, w, bias, norm_weight=self.weight, norm_eps=self.eps, delta=delta,
                      stream_out=self.stream.spare, **kw)
         self.stream.swap()
         return y

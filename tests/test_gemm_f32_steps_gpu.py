@@ -1,0 +1,62 @@
+"""32-bit products of few rows with the residual sum and the norm in front, or silu(gate) * up behind: the numbers that the kernels one by
+one give, bit for bit, and those of 64 bits."""
+import pytest
+import torch
+
+import qwen_engine_amd  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from qwen_engine_amd.kernels import ops
+    return ops
+
+
+# (rows of two passes of the norm, groups of one to four waves, chunks that are not whole, the most that is taken; columns that are no
+# multiple of a block's)
+@pytest.mark.parametrize("M,N,K", [(1, 4096, 1024), (2, 6144, 1024), (8, 6144, 1024), (5, 6272, 1024), (3, 1000, 272), (16, 256, 496), (16, 320, 256),
+                                   (7, 512, 1040), (4, 1024, 2048), (2, 192, 4096), (1, 64, 3104)])
+def test_norm_in_front(ops, M, N, K):
+    g = torch.Generator().manual_seed(M * K + N)
+    h, parts = torch.randn(M, K, generator=g).cuda(), torch.randn(2, M, K, generator=g).cuda()
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).cuda()
+    weight, bias = (1 + 0.1 * torch.randn(K, generator=g)).cuda(), torch.randn(N, generator=g).cuda()
+    assert ops.gemm_norm_supported(M, w)
+    for delta, b in ((None, None), (parts[:1], bias), (parts, None)):
+        stream = h.clone()
+        x = ops.rmsnorm(stream, weight, 1e-6, torch.float32, delta=delta)
+        want = ops.gemm(x, w, b)
+        summed = torch.full_like(h, float("nan")) if delta is not None else None
+        got = ops.gemm(h, w, b, norm_weight=weight, norm_eps=1e-6, delta=delta, stream_out=summed)
+        assert got.dtype == torch.float32 and torch.equal(got, want)
+        if delta is not None:
+            assert torch.equal(summed, stream)
+        s = (h if delta is None else h + delta.sum(0)).double()
+        ref = (s / (s.pow(2).mean(1, keepdim=True) + 1e-6).sqrt() * weight.double()) @ w.double().t() + (0 if b is None else b.double())
+        # (K products of a row of order one, each rounded to 2^-24, and the sums' own roundings)
+        assert float((got - ref).abs().max()) <= K ** 0.5 * 2.0 ** -22
+        if N % 64 == 0 and ops.gemm_silu_supported(h, w):
+            want = ops.silu_mul(ops.gemm(x, w, b), interleaved=True)
+            got = ops.gemm(h, w, b, norm_weight=weight, norm_eps=1e-6, delta=delta, stream_out=summed, epilogue=ops.EPI_SILU_MUL_IL)
+            assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 64, 16), (16, 128, 80), (13, 6144, 1024), (2, 24576, 4096), (16, 16384, 1040)])
+def test_silu_behind(ops, M, N, K):
+    g = torch.Generator().manual_seed(M + K + N)
+    x, w, bias = torch.randn(M, K, generator=g).cuda(), (torch.randn(N, K, generator=g) * K ** -0.5).cuda(), torch.randn(N, generator=g).cuda()
+    assert ops.gemm_silu_supported(x, w)
+    for b in (None, bias):
+        assert torch.equal(ops.gemm(x, w, b, epilogue=ops.EPI_SILU_MUL_IL), ops.silu_mul(ops.gemm(x, w, b), interleaved=True))
+
+
+def test_what_is_not_taken(ops):
+    """More numbers than the norm has room for, rows of no whole steps, logits by whole lines: refused, and by the model's parts never asked for."""
+    w = torch.zeros(64, 1024, device="cuda")
+    assert not ops.gemm_norm_supported(9, w) and not ops.gemm_norm_supported(17, w)
+    assert not ops.gemm_norm_supported(1, torch.zeros(64, 1032, device="cuda")) and not ops.gemm_norm_supported(1, torch.zeros(64, 240, device="cuda"))
+    assert not ops.gemm_silu_supported(torch.zeros(17, 1024, device="cuda"), w)
+    with pytest.raises(ops.KernelError):
+        ops.gemm(torch.zeros(9, 1024, device="cuda"), w, norm_weight=torch.ones(1024, device="cuda"), norm_eps=1e-6)
