@@ -75,7 +75,7 @@ class ModelRunner:
     PORTION_GRAPH_STEP = 128
     # A step of single new tokens beside exactly one prompt portion (what a server runs while requests
     # keep arriving) is recorded too: the single tokens' rows are filled up as in a decode graph, the
-    # portion to 16, 32, 64 or a multiple of MIXED_GRAPH_STEP tokens with rows of the tables' spare row that write
+    # portion to a multiple of MIXED_GRAPH_STEP tokens with rows of the tables' spare row that write
     # nowhere.  Run as it comes, such a step costs the host some 370 launches (3.7 ms at the small
     # model's sizes, more than its kernels take).
     MIXED_GRAPH_STEP = 128
@@ -211,14 +211,6 @@ class ModelRunner:
             return n
         step = 8 if n <= 64 else 32
         return -(-n // step) * step
-
-    @classmethod
-    def mixed_rows(cls, n: int) -> int:
-        """The rows that a portion of n tokens has in a recorded step: short ones have powers of two from 16 on (up to 16 rows the products
-        stream their matrices with the norms inside; a portion of 9 tokens behind 2032 keys takes 2.0 ms at the 0.6B sizes filled up to 128
-        rows, 1.5 with 16)."""
-        step = cls.MIXED_GRAPH_STEP
-        return max(16, 1 << (n - 1).bit_length()) if n <= step // 2 else -(-n // step) * step
 
     def _graph_for(self, key, kind: str, record):
         """The recorded step for ``key`` (most recently used last), recorded now by ``record()`` if its
@@ -618,7 +610,7 @@ class ModelRunner:
                 if list(e.want) != [0]:
                     return False
             elif portion is not None or n < 2 or n > self.MIXED_GRAPH_MAX_TOKENS or list(e.want) not in ([], [n - 1]) \
-                    or self.mixed_rows(n) > self._spare_positions:
+                    or -(-n // self.MIXED_GRAPH_STEP) * self.MIXED_GRAPH_STEP > self._spare_positions:
                 return False                              # (the rows that fill up, and the stand-in batch, stand at the
             else:                                         # positions 0 .. T - 1 of the spare table row)
                 portion = e
@@ -631,7 +623,7 @@ class ModelRunner:
         n_dec, n_groups, i32 = len(ordered) - 1, len(self.cache.groups), np.int32
         T1 = len(ordered[-1].tokens)
         B = self.graph_rows(n_dec)
-        T = self.mixed_rows(T1)
+        T = -(-T1 // self.MIXED_GRAPH_STEP) * self.MIXED_GRAPH_STEP
         cap = 2 * B + 2 * (T // self.page_size + 2)
         # which recorded step this is, from the requests' lengths alone (nothing is reserved yet: a shape
         # that is not recorded runs as it comes)
