@@ -200,6 +200,26 @@ extern "C" int qe_attention_decode_fused_run(const void* qkv, void* out, void* c
                                      max_position, split_keys, workspace, (size_t)workspace_bytes, stream);
 }
 
+bool qe_attention_f32_fused_ok(int T, int Hq, int Hkv, int D, int P);
+int qe_attention_f32_fused(const float* qkv, float* out, float* cache, const int* positions, const int* tok_seq, const int* block_table,
+                           int max_blocks, const int* slots, const float* q_w, const float* k_w, float eps, const float* table,
+                           const int* tokens, int T, int rows, int Hq, int Hkv, int D, int P, float scale, int window, hipStream_t stream);
+
+// 1 if qe_attention_f32_fused_run takes T rows of these sizes
+extern "C" int qe_attention_f32_fused_supported(int T, int Hq, int Hkv, int D, int P) {
+    return Hq > 0 && Hkv > 0 && P > 0 && qe_attention_f32_fused_ok(T, Hq, Hkv, D, P) ? 1 : 0;
+}
+
+// As qe_attention_decode_fused_run, 32-bit: n_dec of the rows (tokens; null: all, in order).
+extern "C" int qe_attention_f32_fused_run(const float* qkv, float* out, float* cache, const int* tokens, int n_dec, int rows, const int* positions,
+                                          const int* tok_seq, const int* block_table, int max_blocks, const int* slots, const float* q_w,
+                                          const float* k_w, float eps, const float* table, int Hq, int Hkv, int D, int P, float scale, int window,
+                                          hipStream_t stream) {
+    QE_REQUIRE(Hq > 0 && Hkv > 0 && P > 0 && max_blocks > 0, "decode attention: bad sizes");
+    return qe_attention_f32_fused(qkv, out, cache, positions, tok_seq, block_table, max_blocks, slots, q_w, k_w, eps, table, tokens, n_dec, rows,
+                                  Hq, Hkv, D, P, scale, window, stream);
+}
+
 extern "C" int qe_attention_decode_run(const void* q, void* out, const void* cache, const int* dec_tokens,
                                        int n_dec, const int* positions, const int* tok_seq,
                                        const int* block_table, int max_blocks, const int* shared_keys,

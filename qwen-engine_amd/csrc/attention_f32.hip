@@ -46,14 +46,27 @@ __device__ __forceinline__ float max_over_rows_of_lanes(float v) {
 // different requests are walked one request after the other.  A column's sums are those it has alone: a tile it sees nothing of leaves
 // them as they are.  (Portions of 328 and 416 rows of 16 heads of 128 on 8: 200 us, a block a token, and 42; 2048 rows 1980, 300; 400 of 64
 // heads 120, 78; 40 rows 11.7, 11.2; two of 50 and 30, where a block holds tokens of both, 12.8, 16.6.)
-template <int DB, int NW, int AHEAD, bool ROWS>      // DB: head size / 16
+//
+// FUSED (eight waves, AHEAD 2, at most 16 heads a key/value head): q is the q|k|v rows; the waves first norm and turn the token's heads and write its key
+// and value to the cache, with the sums and roundings of the kernel that does this for few tokens, while the walks' first tiles are on their
+// way; the tile with the token's own key is asked for behind that.  (The two kernels 22.6 and 3.9 us, with 2 tokens of 16 heads on 8 over 512 keys, and one launch
+// more for the host, some 12 us of a step that is not recorded.)
+struct OwnToken {
+    const float* q_w;
+    const float* k_w;
+    float eps;
+    const float* table;
+    const int* slots;
+};
+template <int DB, int NW, int AHEAD, bool ROWS, bool FUSED = false>      // DB: head size / 16
 __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? (ROWS || AHEAD ? 2 : 3) : 1) void attention_f32_kernel(
     const float* __restrict__ q, float* __restrict__ out, const float* __restrict__ cache,
     const int* __restrict__ positions, const int* __restrict__ tok_seq,
     const int* __restrict__ block_table, int max_blocks, const int* __restrict__ tokens, int T,
-    int Hq, int Hkv, int P, float scale, int window, int keep_first, int sink, float softcap, AttnTail tail) {
+    int Hq, int Hkv, int P, float scale, int window, int keep_first, int sink, float softcap, AttnTail tail, OwnToken own) {
+    static_assert(!FUSED || (NW == F32_WALKS && AHEAD == 2 && !ROWS), "");
     constexpr int D = DB * 16;
-    extern __shared__ float merge_lds[];                  // [F32_SLOTS][DB * 4 + 2][64]
+    extern __shared__ float merge_lds[];                  // [F32_SLOTS][DB * 4 + 2][64]; FUSED: the token's heads before that, [G + 1][D]
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, n = lane & 15;
     const int G = Hq / Hkv, R = ROWS ? 16 / G : 1;         // (R: tokens a block)
     const int groups16 = ROWS ? 1 : (G + 15) / 16;
@@ -72,7 +85,7 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? (ROWS || AHEA
 #pragma unroll
     for (int c = 0; c < DB; ++c) {
         qv[c] = floatx4{0.f, 0.f, 0.f, 0.f};
-        if (head_ok) qv[c] = *(const floatx4*)(q + (t * Hq + head) * D + c * 16 + g * 4);
+        if (!FUSED && head_ok) qv[c] = *(const floatx4*)(q + (t * Hq + head) * D + c * 16 + g * 4);
     }
     // (one round, but for a block whose tokens belong to several requests, and for one with a value that is infinite or NaN: where a column does
     // not see it, it has met a weight of 0, so each token then has a round of its own)
@@ -180,6 +193,49 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? (ROWS || AHEA
                 acc[db][i] = own_first ? fmaf(o, b, acc[db][i] * a) : fmaf(acc[db][i], a, o * b);
             }
     };
+    // the token's query heads to shared memory, normed and turned, its key and value to the cache; a wave a head
+    [[maybe_unused]] const auto prepare = [&]() {
+        const int slot = own.slots ? own.slots[t] : -1;
+        float* const kv = const_cast<float*>(cache) + (slot < 0 ? 0 : (long)(slot / P) * page_stride);
+        const float* const cs = own.table ? own.table + (long)p * D : nullptr;
+        for (int j = wave; j < G + 2; j += NW) {
+            const float* src = q + (t * (Hq + 2 * Hkv) + (j < G ? kvh * G + j : j == G ? Hq + kvh : Hq + Hkv + kvh)) * D;
+            if (j > G) {                                   // the value tile is [D][P]
+                if (slot >= 0)
+                    for (int d = lane; d < D; d += 64) kv[((long)(Hkv + kvh) * D + d) * P + slot % P] = src[d];
+                continue;
+            }
+            const float* w = j < G ? own.q_w : own.k_w;
+            float* const row = merge_lds + j * D;
+            float ss = 0.f;
+            for (int d = lane; d < D; d += 64) {
+                const float v = src[d];
+                row[d] = v;
+                ss = __builtin_fmaf(v, v, ss);
+            }
+            if (w) {
+                ss = wave_sum(ss);
+                const float rstd = rsqrtf(ss / (float)D + own.eps);
+                for (int d = lane; d < D; d += 64) row[d] = row[d] * rstd * w[d];
+            }
+            __builtin_amdgcn_wave_barrier();               // (a wave's accesses to shared memory are done in their order)
+            if (cs)
+                for (int i = lane; i < D / 2; i += 64) {
+                    float x1 = row[i], x2 = row[D / 2 + i];
+                    rotate_pair(cs[i], cs[D / 2 + i], x1, x2);
+                    row[i] = x1;
+                    row[D / 2 + i] = x2;
+                }
+            __builtin_amdgcn_wave_barrier();
+            if (j == G && slot >= 0)
+                for (int d = lane; d < D; d += 64) kv[((long)kvh * P + slot % P) * D + d] = row[d];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < DB; ++c)
+            if (head_ok) qv[c] = *(const floatx4*)(merge_lds + n * D + c * 16 + g * 4);
+        __syncthreads();                                   // (the walks' results take their place)
+    };
     // (a walk without a tile changes nothing where it is joined: where a wave's second walk, or every walk from the fifth on, has none,
     // there is nothing to join)
     const bool second = wave + F32_SLOTS < n_tiles, joins = F32_SLOTS < n_tiles;
@@ -269,7 +325,12 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? (ROWS || AHEA
                 for (int db = 0; db < DB; ++db) add_values(db, vr[db], pr, alpha);
             };
             int ti = walk;
-            if (ti < n_tiles) ask(ti, ka, va);
+            const bool last_first = FUSED && ti == n_tiles - 1;        // (the walk begins with the token's own tile)
+            if (ti < n_tiles && !last_first) ask(ti, ka, va);
+            if constexpr (FUSED) {
+                prepare();
+                if (last_first) ask(ti, ka, va);
+            }
             while (ti < n_tiles) {
                 if (ti + F32_WALKS < n_tiles) ask(ti + F32_WALKS, kb, vb);
                 step(ti, ka, va);
@@ -401,7 +462,7 @@ int qe_attention_f32(const float* q, float* out, const float* cache, const int* 
         const size_t lds = (size_t)F32_SLOTS * (DB_ * 4 + 2) * 64 * sizeof(float);                    \
         if (lds > 48 * 1024) QE_RAISE_SHARED((attention_f32_kernel<DB_, NW_, AHEAD_, ROWS_>), lds);   \
         attention_f32_kernel<DB_, NW_, AHEAD_, ROWS_><<<grid, 64 * NW_, lds, stream>>>(q, out, cache, positions, tok_seq, \
-                                                    block_table, max_blocks, tokens, T, Hq, Hkv, P, scale, window, keep_first, sink, softcap, tail); \
+                                                    block_table, max_blocks, tokens, T, Hq, Hkv, P, scale, window, keep_first, sink, softcap, tail, OwnToken{}); \
     } while (0)
 #define QE_ATTN_F32_RUN(DB_, NW_, AHEAD_) QE_ATTN_F32_FORM(DB_, NW_, AHEAD_, false)
     // (beyond heads of 128 a tile ahead does not fit the registers)
@@ -420,6 +481,39 @@ int qe_attention_f32(const float* q, float* out, const float* cache, const int* 
 #undef QE_ATTN_F32
 #undef QE_ATTN_F32_RUN
 #undef QE_ATTN_F32_FORM
+    QE_LAUNCH_CHECK();
+    return 0;
+}
+
+// The same for single new tokens from the q|k|v rows, with the norm, the rotation (over the whole head) and the cache write inside: for as many tokens
+// as leave compute units idle and as have a wave for each head where these steps have a kernel of their own (whose order of sums this is).
+bool qe_attention_f32_fused_ok(int T, int Hq, int Hkv, int D, int P) {
+    return D % 16 == 0 && D >= 16 && D <= 128 && Hq % Hkv == 0 && Hq / Hkv <= 16 && P % 16 == 0 && (long)T * Hkv <= 256 &&
+           (long)T * (Hq + 2 * Hkv) <= 2048;
+}
+
+int qe_attention_f32_fused(const float* qkv, float* out, float* cache, const int* positions, const int* tok_seq, const int* block_table,
+                           int max_blocks, const int* slots, const float* q_w, const float* k_w, float eps, const float* table,
+                           const int* tokens, int T, int rows, int Hq, int Hkv, int D, int P, float scale, int window, hipStream_t stream) {
+    QE_REQUIRE(qe_attention_f32_fused_ok(rows, Hq, Hkv, D, P) && T <= rows, "attention (32-bit, fused): sizes not taken");
+    if (T == 0) return 0;
+    AttnTail tail{};
+    tail.out_stride = (long)Hq * D;
+    tail.dv = D;
+    tail.plain = true;
+    const OwnToken own = {q_w, k_w, eps, table, slots};
+#define QE_ATTN_F32_FUSED(DB_)                                                                        \
+    case DB_: {                                                                                       \
+        const size_t walks = (size_t)F32_SLOTS * (DB_ * 4 + 2) * 64 * sizeof(float), heads = (size_t)(Hq / Hkv + 1) * D * sizeof(float); \
+        attention_f32_kernel<DB_, F32_WALKS, 2, false, true><<<dim3(T, Hkv), 64 * F32_WALKS, walks > heads ? walks : heads, stream>>>( \
+            qkv, out, cache, positions, tok_seq, block_table, max_blocks, tokens, T, Hq, Hkv, P, scale, window, 0, 0, 0.f, tail, own); \
+        break;                                                                                        \
+    }
+    switch (D / 16) {
+        QE_ATTN_F32_FUSED(1) QE_ATTN_F32_FUSED(2) QE_ATTN_F32_FUSED(3) QE_ATTN_F32_FUSED(4)
+        QE_ATTN_F32_FUSED(5) QE_ATTN_F32_FUSED(6) QE_ATTN_F32_FUSED(7) QE_ATTN_F32_FUSED(8)
+    }
+#undef QE_ATTN_F32_FUSED
     QE_LAUNCH_CHECK();
     return 0;
 }

@@ -59,7 +59,7 @@ __global__ __launch_bounds__(64) void qk_rope_store_kernel(
     for (int d = lane; d < D; d += 64) {
         const float v = Elem<TA>::load(src + d);
         row[d] = v;
-        ss += v * v;
+        ss = __builtin_fmaf(v, v, ss);
     }
     if (w) {
         ss = wave_sum(ss);

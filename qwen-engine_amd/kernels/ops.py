@@ -64,6 +64,8 @@ def load_library():
         "qe_attention_prefill_rows": [i32, i32],
         "qe_attention_prefill_run": [vp, vp, vp, vp, i32, vp, vp, vp, i32, i32, i32, i32, i32, f32, i32, i32, i32, f32, i32, i32, i32,
                                      i32, vp, i64, i64, i32, vp, vp, i64, i32, vp],
+        "qe_attention_f32_fused_supported": [i32, i32, i32, i32, i32],
+        "qe_attention_f32_fused_run": [vp, vp, vp, vp, i32, i32, vp, vp, vp, i32, vp, vp, vp, f32, vp, i32, i32, i32, i32, f32, i32, vp],
         "qe_attention_prefill_plan_segments": [i32, i32, i32],
         "qe_attention_prefill_tiles_run": [vp, i32, i32, vp, i32, i32, vp],
         "qe_attention_prefill_takes_single": [i32, i32, i32, i32],
@@ -1006,7 +1008,11 @@ def attention_decode_fused_supported(qkv: torch.Tensor, cache: torch.Tensor, num
     rotation (if any) over the whole head."""
     lib = load_library()
     D = cache.shape[4]
-    return (qkv.dtype == torch.bfloat16 and (table is None or table.shape[1] == D) and
+    if table is not None and table.shape[1] != D:
+        return False
+    if qkv.dtype == torch.float32 and cache.dtype == torch.float32:
+        return bool(lib.qe_attention_f32_fused_supported(qkv.shape[0], num_heads, cache.shape[2], D, cache.shape[3]))
+    return (qkv.dtype == torch.bfloat16 and
             bool(lib.qe_attention_decode_supported(num_heads, cache.shape[2], D, cache.shape[3], _DT[qkv.dtype])))
 
 
@@ -1020,13 +1026,13 @@ def attention_decode_fused(qkv: torch.Tensor, num_heads: int, cache: torch.Tenso
     """Attention of single new tokens with the step before it inside: per-head q/k RMSNorm
     (weights or None), half-split rotation from ``table`` (rows [cos | sin] of the head size, or
     None) and the write of each token's key and value to cache slot ``slots[t]`` (negative or no
-    slots: not written).  qkv [T, (Hq + 2 Hkv) D] bfloat16; the rows ``dec_tokens`` (None: all
+    slots: not written).  qkv [T, (Hq + 2 Hkv) D], cache and result bfloat16 or float32; the rows ``dec_tokens`` (None: all
     rows) are computed into out [T, Hq, D]; the cache holds each request's keys before the
     token's own position.  shared_keys, dec_blocks: as for attention()."""
     lib = load_library()
-    _need(qkv, "qkv", torch.bfloat16, (None, None))
-    T, dev = qkv.shape[0], qkv.device
-    _need(cache, "cache", torch.bfloat16, (None, 2, None, None, None), dev)
+    _need(qkv, "qkv", _ACT, (None, None))
+    T, dev, dtype = qkv.shape[0], qkv.device, qkv.dtype
+    _need(cache, "cache", dtype, (None, 2, None, None, None), dev)
     Hkv, P, D = cache.shape[2], cache.shape[3], cache.shape[4]
     Hq = int(num_heads)
     if qkv.shape[1] != (Hq + 2 * Hkv) * D:
@@ -1049,10 +1055,16 @@ def attention_decode_fused(qkv: torch.Tensor, num_heads: int, cache: torch.Tenso
     if shared_keys is not None:
         _need(shared_keys, "shared_keys", torch.int32, (block_table.shape[0],), dev)
     if out is None:
-        out = torch.empty((T, Hq, D), dtype=torch.bfloat16, device=dev)
-    _need(out, "out", torch.bfloat16, (T, Hq, D), dev)
+        out = torch.empty((T, Hq, D), dtype=dtype, device=dev)
+    _need(out, "out", dtype, (T, Hq, D), dev)
     n_dec = dec_tokens.shape[0] if dec_tokens is not None else T
     if n_dec == 0:
+        return out
+    if dtype == torch.float32:
+        _check(lib.qe_attention_f32_fused_run(qkv.data_ptr(), out.data_ptr(), cache.data_ptr(), _ptr(dec_tokens), n_dec, T, positions.data_ptr(),
+                                              tok_seq.data_ptr(), block_table.data_ptr(), block_table.shape[1], _ptr(slots), _ptr(q_weight),
+                                              _ptr(k_weight), float(eps), _ptr(table), Hq, Hkv, D, P, float(scale), int(window), _stream()),
+               "attention (32-bit, fused)")
         return out
     nbytes = lib.qe_attention_decode_workspace_bytes(n_dec, Hq, D, int(max_dec_position), DECODE_SPLIT_KEYS)
     ws = torch.empty((nbytes,), dtype=torch.uint8, device=dev)
