@@ -11,7 +11,7 @@
 // k by one load and use them in four instructions).  The chunks of a quarter are added in order, then
 // the quarters in order.
 //
-// Three kernels share that order (the third, for the logits, beside itself):
+// Four kernels share that order (those for the logits and for few rows and whole chunks stand by themselves):
 //   few rows: a block owns 16 outputs (or 32) and has a wave per chunk (16 from K = 1024 on), so that the weights are asked for
 //     by all its waves at once and the sums meet in shared memory.  Bound by the stream of the weights and
 //     a kernel's fixed cost.  Two rows (as 64 x 64 tiles before): 4096 x 1024 7.1 us (42), 6144 x 1024 10.6 (42),
@@ -324,6 +324,61 @@ __global__ __launch_bounds__(256, 5) void gemm_f32_lines_kernel(const float* __r
     }
 }
 
+// The same for up to 16 rows where K is whole chunks of whole lines: a block has COLS rows of w (4, 8 or 16; the matrix instruction's other columns
+// repeat them) and a wave a chunk of 16 STEPS numbers, which come in one trip, as whole lines, straight to shared memory (a row's piece p at
+// place p ^ 4 (row % 4), so that the reads in the operands' layout fall into distinct banks); by pieces of half a line, two steps at a time, a chunk took a
+// trip after the other.  Few columns a block where the matrix has few rows: 64 blocks of 16 would leave three units of four idle.  Bound by the
+// trip and the launch.  (Two rows, by rows and so: 1024 x 1024 6.1 and 4.2 us, 1024 x 3072 11.7 and 7.0, 2048 x 1024 6.6 and 4.5, 4096 x 1024 7.1 and 6.1,
+// 6144 x 1024 10.9 and 8.1, 12288 x 2048 23.6 and 23.1; sixteen: 1024 x 2048 12.4 and 6.8, 6144 x 1024 12.0 and 9.2.)
+// (With the norm in front and silu behind, 384 blocks that norm the rows themselves took 13.7 us for 6144 x 1024 where 192 by rows take 12.5.)
+template <int COLS, int STEPS>
+__global__ __launch_bounds__(64 * CHUNKS) void gemm_f32_chunks_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                                      const float* __restrict__ bias, float* __restrict__ out,
+                                                                      int M, int N, int K) {
+    typedef __attribute__((ext_vector_type(4))) unsigned int uint4_t;
+    constexpr int C = STEPS * FK, PIECES = C / 4, LOADS = COLS * PIECES / 64;
+    extern __shared__ __attribute__((aligned(16))) float chunks[];          // [wave][COLS][C], then a wave's sums [4][64] in its place
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, r = lane & 15;
+    const int waves = blockDim.x >> 6, n0 = blockIdx.x * COLS, k_lo = wave * C;
+    float* const mine = chunks + wave * (COLS * C);
+    const float* xrow = x + (long)min(r, M - 1) * K + 4 * g + k_lo;
+    floatx4 xv[STEPS];
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) xv[s] = *(const floatx4_any*)(xrow + s * FK);
+    __builtin_amdgcn_sched_barrier(0);
+    // (rows beyond the matrix are out of the descriptor's range and arrive as zeros)
+    const unsigned long base = (unsigned long)(w + (long)n0 * K);
+    const uint4_t rsrc = {(unsigned)base, (unsigned)(base >> 32) & 0xffffu, (unsigned)(min(COLS, N - n0) * K) * 4u, 0x00020000u};
+    const unsigned to = (unsigned)(unsigned long)(__attribute__((address_space(3))) float*)chunks + wave * (COLS * C * 4);
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+        const int at = i * 64 + lane, col = at / PIECES, piece = (at % PIECES) ^ ((col & 3) * 4);
+        QE_LOAD_TO_SHARED(to + i * 1024, (col * K + piece * 4) * 4, rsrc, k_lo * 4, "0", " nt");
+    }
+    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");                     // (the wave's own lines: no barrier)
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) {
+        const floatx4 wv = *(const floatx4*)(mine + (r % COLS) * C + ((s * 4 + g) ^ ((r & 3) * 4)) * 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[s][e], wv[e], acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) mine[e * 64 + lane] = acc[e];
+    __syncthreads();
+    for (int at = threadIdx.x; at < 256; at += blockDim.x) {
+        const int l = at & 63, m = 4 * (l >> 4) + (at >> 6), n = n0 + (l & 15);
+        if ((l & 15) >= COLS || m >= M || n >= N) continue;
+        float total = 0.f;
+        for (int q = 0; 4 * q < waves; ++q) {
+            float quarter = chunks[4 * q * (COLS * C) + at];
+            for (int c = 4 * q + 1; c < 4 * q + 4 && c < waves; ++c) quarter += chunks[c * (COLS * C) + at];
+            total = q ? total + quarter : quarter;
+        }
+        out[(long)m * N + n] = bias ? total + bias[n] : total;
+    }
+}
+
 // Tiles of 64 x 64, GROUPS (1 or 4) groups of four waves.  For a step, lane (h, r), h = lane / 32, r = lane % 32, reads
 // x[row r][4 h .. + 4] and [8 + 4 h .. + 4], and the same of W: with the instructions taking element j of the first and of
 // the second piece in turn, the order is the one above.
@@ -444,6 +499,33 @@ static void launch_rows(const float* x, const float* w, const float* bias, float
 #undef QE_F32_ROWS
 }
 
+// gemm_f32_chunks_kernel takes up to 16 rows of these sizes.
+static bool by_chunks(const float* w, int K) {
+    const int chunk = chunk_len(K);
+    return K % chunk == 0 && chunk % 64 == 0 && chunk <= 256 && (((unsigned long)w) & 15) == 0;
+}
+
+template <int COLS>
+static int launch_chunks(const float* x, const float* w, const float* bias, float* out, int M, int N, int K, hipStream_t stream) {
+    const int chunk = chunk_len(K), waves = K / chunk;
+#define QE_F32_CHUNKS(S_)                                                                             \
+    case S_: {                                                                                        \
+        constexpr size_t most = CHUNKS * COLS * (S_) * FK * sizeof(float);                            \
+        if constexpr (most <= 128 * 1024) {                                                           \
+            QE_RAISE_SHARED((gemm_f32_chunks_kernel<COLS, S_>), most);                                 \
+            gemm_f32_chunks_kernel<COLS, S_><<<qe_cdiv(N, COLS), 64 * waves, (size_t)K * COLS * sizeof(float), stream>>>(x, w, bias, out, M, N, K); \
+            QE_LAUNCH_CHECK();                                                                        \
+            return 0;                                                                                 \
+        }                                                                                             \
+        break;                                                                                        \
+    }
+    switch (chunk / FK) {
+        QE_F32_CHUNKS(4) QE_F32_CHUNKS(8) QE_F32_CHUNKS(12) QE_F32_CHUNKS(16)
+    }
+#undef QE_F32_CHUNKS
+    QE_REQUIRE(false, "gemm (32-bit): no kernel for chunks of %d numbers of %d rows a block", chunk, COLS);
+}
+
 // Whether up to 16 rows against a matrix [N, K] go by whole lines (see qe_gemm_f32).
 static bool by_lines(int M, int N, int K) {
     return N >= 16384 && (K >= 608 || (K > 512 && (M > 2 || N >= 30000))) && K <= 4 * FK * CHUNKS && K % 32 == 0;
@@ -496,6 +578,11 @@ int qe_gemm_f32(const float* x, const float* w, const float* bias, float* out, i
         // 15.9, 32768 x 608 26.6 and 21.0; with eight chunks or fewer a wave's walk is not worth a block: 20000 x 96 4.7 and 6.9)
         if (M <= 16 && by_lines(M, N, K) && (((unsigned long)w) & 15) == 0)
             gemm_f32_lines_kernel<<<qe_cdiv(N, 16), 64 * qe_cdiv(K, 16 * FK), 0, stream>>>(x, w, bias, out, M, N, K);
+        // (two rows, us with 4, 8 and 16 columns a block: 1024 x 2048 5.5, 5.8, 6.5; 2048 x 1024 5.5, 4.5, 4.9; 4096 x 1024 9.6, 6.2, 6.1; 12288 x 1024
+        // 24.9, 15.1, 12.1; 8192 x 3072, 8 columns, 29.5, and 25.2 by rows)
+        else if (M <= 16 && N <= 1024 && by_chunks(w, K)) return launch_chunks<4>(x, w, bias, out, M, N, K, stream);
+        else if (M <= 16 && N <= 2048 && by_chunks(w, K)) return launch_chunks<8>(x, w, bias, out, M, N, K, stream);
+        else if (M <= 16 && by_chunks(w, K) && chunk_len(K) <= 128) return launch_chunks<16>(x, w, bias, out, M, N, K, stream);
         else if (M > 4 && M <= 16 && N >= 6144) launch_rows<1, 2, 1>(x, w, bias, out, M, N, K, rows, stream);
         else if (M <= 16) launch_rows<1, 1, 2>(x, w, bias, out, M, N, K, rows, stream);
         else if (M <= 32) launch_rows<2, 1, 2>(x, w, bias, out, M, N, K, rows, stream);

@@ -52,6 +52,20 @@ def test_silu_behind(ops, M, N, K):
         assert torch.equal(ops.gemm(x, w, b, epilogue=ops.EPI_SILU_MUL_IL), ops.silu_mul(ops.gemm(x, w, b), interleaved=True))
 
 
+@pytest.mark.parametrize("N", [1, 5, 1000, 1024, 1030, 2048, 2052, 4100])
+@pytest.mark.parametrize("K", [64, 192, 512, 1024, 1920, 2048, 3072, 4096, 4160])
+def test_few_rows_and_many(ops, N, K):
+    """A row's sums beside up to sixteen others, by whole chunks where K is some, and beside forty: one order.  Behind w's end is NaN."""
+    g = torch.Generator().manual_seed(N + K)
+    x, bias = torch.randn(40, K, generator=g).cuda(), torch.randn(N, generator=g).cuda()
+    room = torch.full((N * K + 64 * K,), float("nan"), device="cuda")
+    room[:N * K] = torch.randn(N * K, generator=g).cuda()
+    w = room[:N * K].view(N, K)
+    want = ops.gemm(x, w, bias)
+    for m in (1, 3, 16):
+        assert torch.equal(ops.gemm(x[:m], w, bias), want[:m]), m
+
+
 def test_what_is_not_taken(ops):
     """More numbers than the norm has room for, rows of no whole steps, logits by whole lines: refused, and by the model's parts never asked for."""
     w = torch.zeros(64, 1024, device="cuda")
