@@ -206,7 +206,10 @@ class StreamInput:
 
     def prefers_prologue(self, ops, w: torch.Tensor) -> bool:
         """True if the product against w should do the sum and the norm itself (the kernel library knows up
-        to which sizes that is quicker than the norm's own kernel); else the part calls materialize()."""
+        to which sizes that is quicker than the norm's own kernel); else the part calls materialize().  In the float32 mode, in which
+        programs look into a model's parts, a norm whose ``forward`` has been replaced is called."""
+        if self.rt.dtype == torch.float32 and getattr(self.norm, "replaced", bool)():
+            return False
         parts = 0 if self.delta is None else self.delta.shape[0] if self.delta.dim() == 3 else 1
         return w.dtype == self.rt.dtype and ops.gemm_norm_preferred(self.rows, w, parts)
 

@@ -42,6 +42,10 @@ class RMSNorm:
         """(weight, eps): this is a plain RMSNorm, which a product can take as its prologue."""
         return self.weight, self.eps
 
+    def replaced(self) -> bool:
+        """True if a program has put something else in the place of ``forward`` (a trace, a change of its own)."""
+        return "forward" in vars(self) or type(self).forward is not _FORWARD
+
     def forward(self, h: torch.Tensor, rt: Runtime, delta: Optional[torch.Tensor] = None,
                 rows: Optional[torch.Tensor] = None) -> torch.Tensor:
         return _norm(h, self.weight, self.eps, rt, delta, rows, self.center)
@@ -50,6 +54,9 @@ class RMSNorm:
         """The norm of a post-norm block: x <- w * z / rms(z) with z = alpha * x + delta, on the 32-bit stream in
         place; returns the new x in the activation type where that is not 32-bit."""
         return ops.postnorm(x, delta, alpha, self.weight, self.eps, rt.dtype)
+
+
+_FORWARD = RMSNorm.forward
 
 
 class ScalarRMSNorm:

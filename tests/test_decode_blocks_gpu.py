@@ -143,3 +143,17 @@ def test_embedding_with_a_block_tables_updates(ops, T, H, n, dtype):
     for table in (emb, odd):
         assert torch.equal(ops.embedding(ids, table, update=(got, idx, val)), emb[ids.long()].float())
     assert torch.equal(got, want) and torch.equal(ops.embedding(ids, emb), emb[ids.long()].float())
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 130])
+def test_numbers_that_travel_with_the_launch(ops, n):
+    g = torch.Generator().manual_seed(n)
+    places, values = torch.randperm(200, generator=g)[:n], torch.randint(-5, 1 << 30, (n,), generator=g)
+    table = torch.full((200,), 7, dtype=torch.int32, device=DEV)
+    want = table.cpu()
+    want[places] = values.int()
+    ops.set_ints(table, places.tolist(), values.tolist())
+    assert torch.equal(table.cpu(), want)
+    with pytest.raises(ops.KernelError):
+        ops.set_ints(table, [200], [0])
+    assert torch.equal(table.cpu(), want)
