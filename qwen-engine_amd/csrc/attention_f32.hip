@@ -49,8 +49,8 @@ __device__ __forceinline__ float max_over_rows_of_lanes(float v) {
 //
 // FUSED (eight waves, AHEAD 2, at most 16 heads a key/value head): q is the q|k|v rows; the waves first norm and turn the token's heads and write its key
 // and value to the cache, with the sums and roundings of the kernel that does this for few tokens, while the walks' first tiles are on their
-// way; the tile with the token's own key is asked for behind that.  (The two kernels 22.6 and 3.9 us, with 2 tokens of 16 heads on 8 over 512 keys, and one launch
-// more for the host, some 12 us of a step that is not recorded.)
+// way; the tile with the token's own key is asked for behind that.  (2 tokens of 16 heads on 8 over 512 keys: the two kernels 22.6 and 3.9 us, in one 21.6, and a launch
+// less for the host, some 12 us of a step that is not recorded.)
 struct OwnToken {
     const float* q_w;
     const float* k_w;

@@ -155,6 +155,8 @@ __device__ __forceinline__ void norm_rows(const float* __restrict__ h, const Row
 // silu(gate) * up.
 // NORM (rows of at most NORM_ROOM numbers in all): x is the stream; what is to be added to it and the RMSNorm come first, with the sums and
 // roundings of the norm's own kernel, while the first weights are on their way; the normed rows stay in shared memory.
+// (Two rows against 4096 x 1024 8.6 us, with the norm before 7.4 + 3.4; 6144 x 1024 with norm and silu 12.5, as three kernels 11.0 + 3.4 + 2.5; and for the
+// host two launches of some 12 us each less.)
 template <int MT, int NT, int BATCH, int ROWS, bool SILU = false, bool NORM = false>
 __global__ __launch_bounds__(64 * CHUNKS) void gemm_f32_rows_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                     const float* __restrict__ bias, float* __restrict__ out,
