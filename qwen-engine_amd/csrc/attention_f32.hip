@@ -487,8 +487,9 @@ int qe_attention_f32(const float* q, float* out, const float* cache, const int* 
 
 // The same for single new tokens from the q|k|v rows, with the norm, the rotation (over the whole head) and the cache write inside: for as many tokens
 // as leave compute units idle and as have a wave for each head where these steps have a kernel of their own (whose order of sums this is).
+extern int g_qe_matrix_f32;      // (switched off: the vector units' kernel and the one before it)
 bool qe_attention_f32_fused_ok(int T, int Hq, int Hkv, int D, int P) {
-    return D % 16 == 0 && D >= 16 && D <= 128 && Hq % Hkv == 0 && Hq / Hkv <= 16 && P % 16 == 0 && (long)T * Hkv <= 256 &&
+    return g_qe_matrix_f32 && D % 16 == 0 && D >= 16 && D <= 128 && Hq % Hkv == 0 && Hq / Hkv <= 16 && P % 16 == 0 && (long)T * Hkv <= 256 &&
            (long)T * (Hq + 2 * Hkv) <= 2048;
 }
 

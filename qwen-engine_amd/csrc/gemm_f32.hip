@@ -535,9 +535,10 @@ static bool by_lines(int M, int N, int K) {
 
 // The products of few rows with the steps beside them inside (N: the rows of w): silu(gate) * up over rows interleaved in blocks of 32, and
 // the residual sum and the norm in front.  K in whole steps of 16.
-bool qe_gemm_f32_silu_ok(int M, int N, int K) { return M <= 16 && N % 64 == 0 && K % FK == 0 && !by_lines(M, N, K); }
+extern int g_qe_matrix_f32;      // (switched off: the vector units' kernels do it all, one by one)
+bool qe_gemm_f32_silu_ok(int M, int N, int K) { return g_qe_matrix_f32 && M <= 16 && N % 64 == 0 && K % FK == 0 && !by_lines(M, N, K); }
 bool qe_gemm_f32_norm_ok(int M, int N, int K) {
-    return M <= 16 && K % FK == 0 && K >= 256 && K <= 4096 && (long)M * K <= NORM_ROOM && !by_lines(M, N, K);
+    return g_qe_matrix_f32 && M <= 16 && K % FK == 0 && K >= 256 && K <= 4096 && (long)M * K <= NORM_ROOM && !by_lines(M, N, K);
 }
 
 // N: outputs.  norm_w null: no norm.

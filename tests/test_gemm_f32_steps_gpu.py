@@ -74,3 +74,18 @@ def test_what_is_not_taken(ops):
     assert not ops.gemm_silu_supported(torch.zeros(17, 1024, device="cuda"), w)
     with pytest.raises(ops.KernelError):
         ops.gemm(torch.zeros(9, 1024, device="cuda"), w, norm_weight=torch.ones(1024, device="cuda"), norm_eps=1e-6)
+
+
+def test_matrix_units_switched_off(ops):
+    """What goes together on the matrix units is taken apart with them switched off."""
+    x, w = torch.zeros(2, 1024, device="cuda"), torch.zeros(4096, 1024, device="cuda")
+    qkv, cache = torch.zeros(2, 4096, device="cuda"), torch.zeros(4, 2, 8, 16, 128, device="cuda")
+    taken = lambda: (ops.gemm_norm_supported(2, w), ops.gemm_norm_preferred(2, w, 1), ops.gemm_silu_supported(x, w),
+                     ops.attention_decode_fused_supported(qkv, cache, 16, None))
+    assert taken() == (True,) * 4
+    try:
+        ops.use_matrix_f32(False)
+        assert taken() == (False,) * 4
+    finally:
+        ops.use_matrix_f32(True)
+    assert taken() == (True,) * 4
