@@ -558,6 +558,10 @@ def gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
                 raise KernelError("gemm: the summed stream cannot be written over the stream that is read")
         elif stream_out is not None:
             raise KernelError("gemm: stream_out goes with delta")
+        if epilogue == EPI_SILU_MUL and w.dtype == torch.float32:      # (its kernel has the activation over interleaved rows only)
+            if out_dtype != torch.float32:
+                raise KernelError("gemm: the norm prologue of 32-bit weights gives 32-bit numbers")
+            return silu_mul(gemm(x, w, bias, algo=algo, norm_weight=norm_weight, norm_eps=norm_eps, delta=delta, stream_out=stream_out), out)
     elif delta is not None or stream_out is not None:
         raise KernelError("gemm: delta and stream_out go with norm_weight")
     elif x.dtype == torch.float32 and w.dtype != torch.float32:

@@ -66,8 +66,43 @@ def test_few_rows_and_many(ops, N, K):
         assert torch.equal(ops.gemm(x[:m], w, bias), want[:m]), m
 
 
+@pytest.mark.parametrize("width", [688, 704, 1000, 2736])
+@pytest.mark.parametrize("hidden,rows", [(256, 1), (256, 16), (1024, 2), (1024, 8), (240, 3), (1024, 9)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_a_feed_forward_of_any_width(ops, width, hidden, rows, bias):
+    """From the stream, with what is to be added to it, and from rows that the norm's own kernel made: the same bits, also where gate and up
+    rows are not interleaved (a width that is no multiple of 32) and where the norm has no room inside the product."""
+    from qwen_engine_amd.config import RMSNormSpec, SwiGLUSpec
+    from qwen_engine_amd.parts import Runtime, build_part
+    from qwen_engine_amd.parts.base import Stream, StreamInput
+    g = torch.Generator().manual_seed(width + rows)
+    rt = Runtime(torch.device("cuda:0"), torch.float32)
+    spec = SwiGLUSpec(intermediate_size=width, bias=True) if bias else SwiGLUSpec(intermediate_size=width)
+    ffn, norm = build_part(spec, hidden), build_part(RMSNormSpec(eps=1e-6), hidden)
+    ffn.load({n: torch.randn(tuple(t.shape), generator=g) * hidden ** -0.5 for n, t in type(ffn).expected_tensors(spec, hidden).items()}, rt)
+    norm.load({"weight": 1 + 0.1 * torch.randn(hidden, generator=g)}, rt)
+    assert ffn.interleaved == (width % 32 == 0)
+    h, parts = torch.randn(rows, hidden, generator=g).cuda(), torch.randn(2, rows, hidden, generator=g).cuda()
+    for delta in (None, parts[0], parts[:1], parts):
+        stream = Stream(h.clone(), torch.full_like(h, float("nan")))
+        want = ffn.forward(norm.forward(want_h := h.clone(), rt, delta=delta), None)
+        x = StreamInput(stream, delta, norm, *norm.fusable_weight(), rt)
+        assert x.fusable() and torch.equal(ffn.forward(x, None), want) and torch.equal(stream.h, want_h)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 2000, 1024), (16, 1376, 256), (3, 34, 496)])
+def test_norm_in_front_of_gate_and_up_rows(ops, M, N, K):
+    g = torch.Generator().manual_seed(M * K + N)
+    h, w, weight = torch.randn(M, K, generator=g).cuda(), torch.randn(N, K, generator=g).cuda(), torch.randn(K, generator=g).cuda()
+    out = torch.empty(M, N // 2, device="cuda")
+    got = ops.gemm(h, w, out=out, epilogue=ops.EPI_SILU_MUL, norm_weight=weight, norm_eps=1e-6)
+    assert got is out and torch.equal(got, ops.silu_mul(ops.gemm(ops.rmsnorm(h, weight, 1e-6, torch.float32), w)))
+    with pytest.raises(ops.KernelError):
+        ops.gemm(h, w, out_dtype=torch.bfloat16, epilogue=ops.EPI_SILU_MUL, norm_weight=weight, norm_eps=1e-6)
+
+
 def test_what_is_not_taken(ops):
-    """More numbers than the norm has room for, rows of no whole steps, logits by whole lines: refused, and by the model's parts never asked for."""
+    """More numbers than the norm has room for, rows of no whole steps: refused."""
     w = torch.zeros(64, 1024, device="cuda")
     assert not ops.gemm_norm_supported(9, w) and not ops.gemm_norm_supported(17, w)
     assert not ops.gemm_norm_supported(1, torch.zeros(64, 1032, device="cuda")) and not ops.gemm_norm_supported(1, torch.zeros(64, 240, device="cuda"))
