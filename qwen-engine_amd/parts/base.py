@@ -116,6 +116,12 @@ class Runtime:
         return t.to(torch.float32).contiguous().to(self.device)
 
 
+def is_replaced(part, written) -> bool:
+    """True if a program, or a class derived from the part's, has put something else in the place of the method ``written`` (a trace, a
+    change of its own): what would pass it by calls it then."""
+    return written.__name__ in vars(part) or getattr(type(part), written.__name__) is not written
+
+
 class Stream:
     """The 32-bit residual stream of a step, [T, H], with a second buffer of the same size: a
     product that adds a branch's partial products to the stream in its prologue writes the sums

@@ -9,7 +9,7 @@ from typing import Dict, Optional
 import torch
 
 from ..kernels import ops
-from .base import Runtime, StreamInput, TensorInfo
+from .base import Runtime, StreamInput, TensorInfo, is_replaced
 from .registry import register_part
 
 
@@ -65,10 +65,10 @@ class SwiGLU:
 
     def forward(self, x, ctx) -> torch.Tensor:
         """Returns the feed-forward output [T, H], or float32 partial products [S, T, H] of it.
-        x: the normed rows, or a StreamInput."""
+        x: the normed rows, or a StreamInput (an ``activation`` that has been replaced gets the normed rows)."""
         a = None
         if isinstance(x, StreamInput):
-            if x.prefers_prologue(ops, self.w_gu):
+            if x.prefers_prologue(ops, self.w_gu) and not is_replaced(self, _ACTIVATION):
                 a = x.gemm(ops, self.w_gu, self.b_gu, epilogue=ops.EPI_SILU_MUL_IL if self.interleaved else ops.EPI_SILU_MUL)
             else:
                 x = x.materialize()
@@ -78,6 +78,9 @@ class SwiGLU:
         if splits:   # partial products along K, added by the norm that follows
             return ops.gemm(a, self.w_down, self.b_down, epilogue=ops.EPI_PARTIAL, splits=splits)
         return ops.gemm(a, self.w_down, self.b_down)
+
+
+_ACTIVATION = SwiGLU.activation
 
 
 class GeluMLP:

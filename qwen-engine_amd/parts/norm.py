@@ -7,7 +7,7 @@ from typing import Dict, Optional
 import torch
 
 from ..kernels import ops
-from .base import BranchSum, NormedBranch, Runtime, TensorInfo, add_pending
+from .base import BranchSum, NormedBranch, Runtime, TensorInfo, add_pending, is_replaced
 from .registry import register_part
 
 
@@ -43,8 +43,8 @@ class RMSNorm:
         return self.weight, self.eps
 
     def replaced(self) -> bool:
-        """True if a program has put something else in the place of ``forward`` (a trace, a change of its own)."""
-        return "forward" in vars(self) or type(self).forward is not _FORWARD
+        """True if a program has put something else in the place of ``forward``."""
+        return is_replaced(self, _FORWARD)
 
     def forward(self, h: torch.Tensor, rt: Runtime, delta: Optional[torch.Tensor] = None,
                 rows: Optional[torch.Tensor] = None) -> torch.Tensor:
