@@ -15,7 +15,7 @@ import torch
 
 from ..cache.plan import KVNeed
 from ..kernels import ops
-from .base import CacheBinding, Runtime, StreamInput, TensorInfo
+from .base import CacheBinding, Runtime, StreamInput, TensorInfo, is_replaced
 from .registry import build_part, register_part
 
 
@@ -270,9 +270,9 @@ class PagedAttention:
             only_new_tokens = (ex["dec_tokens"] is not None and ex["dec_tokens"].shape[0] == T and
                                (ex["other_tokens"] is None or ex["other_tokens"].shape[0] == 0))
             if (only_new_tokens and T <= (FUSED_DECODE_MAX_TOKENS if self.window else FUSED_DECODE_MAX_TOKENS_UNWINDOWED) and binding.write and
-                    ops.attention_decode_fused_supported(qkv, cache, self.hq, table)):
+                    not is_replaced(self, _ATTEND) and ops.attention_decode_fused_supported(qkv, cache, self.hq, table)):
                 # every row is the one new token of its request: norm, rotation and cache write
-                # happen inside the attention kernel
+                # happen inside the attention kernel (an _attend that has been replaced gets q)
                 o = ops.attention_decode_fused(qkv, self.hq, cache, ctx.positions, ctx.tok_seq, ctx.block_tables[g],
                                                self.scale, self.window, None, ex["max_dec_position"],
                                                self.q_norm, self.k_norm, eps, table, slots,
@@ -312,6 +312,9 @@ class PagedAttention:
             # compute unit blocks to overlap); the norm that follows adds the parts
             return ops.gemm(o, self.w_o, self.b_o, epilogue=ops.EPI_PARTIAL, splits=splits)
         return ops.gemm(o, self.w_o, self.b_o)
+
+
+_ATTEND = PagedAttention._attend
 
 
 def common_head_dim(k_dim: int, v_dim: int) -> int:

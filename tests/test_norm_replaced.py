@@ -1,5 +1,5 @@
 """What a program has replaced is called: a norm, in the float32 mode, instead of norming inside the product behind it; a feed-forward's
-activation."""
+activation, and what an attention part does with q."""
 from types import SimpleNamespace
 
 import pytest
@@ -7,7 +7,8 @@ import torch
 
 import qwen_engine_amd  # noqa: F401
 from qwen_engine_amd.parts.base import Stream, StreamInput
-from qwen_engine_amd.parts import mlp
+from qwen_engine_amd.parts import attention, mlp
+from qwen_engine_amd.parts.attention import PagedAttention
 from qwen_engine_amd.parts.mlp import SwiGLU
 from qwen_engine_amd.parts.norm import RMSNorm
 
@@ -53,3 +54,28 @@ def test_a_replaced_activation_is_called(monkeypatch, dtype, how):
         ffn.__class__ = type("Derived", (SwiGLU,), {"activation": lambda self, x: mine(x)})
     ffn.forward(x, None)
     assert seen == [rows]
+
+
+@pytest.mark.parametrize("how", ["class", "part", "derived"])
+def test_a_replaced_attend_is_called(monkeypatch, how):
+    """Steps of single tokens whose norm, rotation and cache write are inside the attention kernel have no q to hand on: they go one by one."""
+    one, q = [], torch.ones(2, 4, 16)
+    fake = SimpleNamespace(gemm=lambda x, w, b=None, **kw: x, gemm_qkv_supported=lambda *a: False, gemm_partial_preferred=lambda *a: False,
+                           gemm_branch_splits=lambda *a: 0, attention_decode_fused_supported=lambda *a: True, qk_rope_store=lambda *a: q,
+                           attention_decode_fused=lambda *a, **kw: one.append(a) or q)
+    monkeypatch.setattr(attention, "ops", fake)
+    part = PagedAttention(SimpleNamespace(num_heads=4, num_kv_heads=2, head_dim=16, scale=0.25, window=None, qk_norm_eps=None, position=None), 64)
+    ctx = SimpleNamespace(positions=None, tok_seq=None, block_tables=[None], slots=[None], shared_keys=None, max_position=9, page_size=16, memo={},
+                          extras={PagedAttention: {"dec_tokens": torch.zeros(2, dtype=torch.int32), "other_tokens": None, "max_dec_position": 9}})
+    binding = SimpleNamespace(kv=torch.zeros(1, 2, 2, 16, 16), group=0, write=True)
+    part.forward(torch.zeros(2, 64), ctx, binding)
+    assert len(one) == 1
+    seen, mine = [], lambda q, ctx, cache, g, T: seen.append(q) or q
+    if how == "class":
+        monkeypatch.setattr(PagedAttention, "_attend", lambda self, *a: mine(*a))
+    elif how == "part":
+        part._attend = mine
+    else:
+        part.__class__ = type("Derived", (PagedAttention,), {"_attend": lambda self, *a: mine(*a)})
+    part.forward(torch.zeros(2, 64), ctx, binding)
+    assert len(one) == 1 and len(seen) == 1 and seen[0] is q
