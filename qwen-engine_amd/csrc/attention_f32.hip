@@ -49,7 +49,8 @@ __device__ __forceinline__ float max_over_rows_of_lanes(float v) {
 //
 // FUSED (eight waves, AHEAD 2, at most 16 heads a key/value head): q is the q|k|v rows; the waves first norm and turn the token's heads and write its key
 // and value to the cache, with the sums and roundings of the kernel that does this for few tokens, while the walks' first tiles are on their
-// way; the tile with the token's own key is asked for behind that.  (2 tokens of 16 heads on 8 over 512 keys: the two kernels 22.6 and 3.9 us, in one 21.6, and a launch
+// way.  The walk with the token's own key takes it, and its value, from shared memory: they may be written nowhere, and their page may not be
+// there.  (2 tokens of 16 heads on 8 over 512 keys: the two kernels 22.6 and 3.9 us, in one 21.6, and a launch
 // less for the host, some 12 us of a step that is not recorded.)
 struct OwnToken {
     const float* q_w;
@@ -66,7 +67,9 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? (ROWS || AHEA
     int Hq, int Hkv, int P, float scale, int window, int keep_first, int sink, float softcap, AttnTail tail, OwnToken own) {
     static_assert(!FUSED || (NW == F32_WALKS && AHEAD == 2 && !ROWS), "");
     constexpr int D = DB * 16;
-    extern __shared__ float merge_lds[];                  // [F32_SLOTS][DB * 4 + 2][64]; FUSED: the token's heads before that, [G + 1][D]
+    // [F32_SLOTS][DB * 4 + 2][64]; FUSED: the token's query heads before that, [G][D], and behind it its key and its value
+    extern __shared__ float merge_lds[];
+    [[maybe_unused]] float* const own_kv = merge_lds + (long)F32_SLOTS * (DB * 4 + 2) * 64;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, n = lane & 15;
     const int G = Hq / Hkv, R = ROWS ? 16 / G : 1;         // (R: tokens a block)
     const int groups16 = ROWS ? 1 : (G + 15) / 16;
@@ -124,13 +127,15 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? (ROWS || AHEA
     // were two trips to memory of their own); a tile's page is then the same for the wave, and so is its place in it.  Other page sizes:
     // every lane looks its own keys' pages up.
     const bool whole = P % 16 == 0;
+    // (FUSED: the last tile may hold no key but the token's own; its page is then not looked up)
+    const bool own_alone = FUSED && max(p / 16 * 16, lo) >= p;
     int my_page = 0;
     const auto page_of = [&](int ti, int walk) {               // asked for tile by tile, in order
         const int j = (ti - walk) / F32_WALKS;
         if (!whole) return 0;
         if ((j & 63) == 0) {
             const int tl = ti + lane * F32_WALKS;
-            if (tl < n_tiles) my_page = bt[tile_key(tl) / P];
+            if (tl < n_tiles - own_alone) my_page = bt[tile_key(tl) / P];
         }
         return __builtin_amdgcn_readlane(my_page, j & 63);
     };
@@ -193,7 +198,7 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? (ROWS || AHEA
                 acc[db][i] = own_first ? fmaf(o, b, acc[db][i] * a) : fmaf(acc[db][i], a, o * b);
             }
     };
-    // the token's query heads to shared memory, normed and turned, its key and value to the cache; a wave a head
+    // the token's heads to shared memory, normed and turned, its key and value to the cache too; a wave a head
     [[maybe_unused]] const auto prepare = [&]() {
         const int slot = own.slots ? own.slots[t] : -1;
         float* const kv = const_cast<float*>(cache) + (slot < 0 ? 0 : (long)(slot / P) * page_stride);
@@ -201,12 +206,15 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? (ROWS || AHEA
         for (int j = wave; j < G + 2; j += NW) {
             const float* src = q + (t * (Hq + 2 * Hkv) + (j < G ? kvh * G + j : j == G ? Hq + kvh : Hq + Hkv + kvh)) * D;
             if (j > G) {                                   // the value tile is [D][P]
-                if (slot >= 0)
-                    for (int d = lane; d < D; d += 64) kv[((long)(Hkv + kvh) * D + d) * P + slot % P] = src[d];
+                for (int d = lane; d < D; d += 64) {
+                    const float v = src[d];
+                    own_kv[D + d] = v;
+                    if (slot >= 0) kv[((long)(Hkv + kvh) * D + d) * P + slot % P] = v;
+                }
                 continue;
             }
             const float* w = j < G ? own.q_w : own.k_w;
-            float* const row = merge_lds + j * D;
+            float* const row = j < G ? merge_lds + j * D : own_kv;
             float ss = 0.f;
             for (int d = lane; d < D; d += 64) {
                 const float v = src[d];
@@ -234,7 +242,7 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? (ROWS || AHEA
 #pragma unroll
         for (int c = 0; c < DB; ++c)
             if (head_ok) qv[c] = *(const floatx4*)(merge_lds + n * D + c * 16 + g * 4);
-        __syncthreads();                                   // (the walks' results take their place)
+        __syncthreads();                                   // (the walks' results take the query heads' place)
     };
     // (a walk without a tile changes nothing where it is joined: where a wave's second walk, or every walk from the fifth on, has none,
     // there is nothing to join)
@@ -296,6 +304,7 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? (ROWS || AHEA
             // (pages of whole tiles.  What of a tile is not there lies in its page all the same: it is read, and zeros take its place)
             floatx4 ka[DB], va[DB], kb[DB], vb[DB];
             const auto ask = [&](int ti, floatx4 (&kr)[DB], floatx4 (&vr)[DB]) {
+                if (FUSED && own_alone && ti == n_tiles - 1) return;
                 const int in = tile_key(ti) % P;
                 const float* const page = cache + (long)page_of(ti, walk) * page_stride;
                 const float* const krow = page + ((long)kvh * P + in + n) * D + g * 4;
@@ -319,18 +328,32 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? (ROWS || AHEA
                             vr[c][i] = ok[i] ? vr[c][i] : 0.f;
                         }
                 }
+                if (FUSED && ti == n_tiles - 1) {          // (what was read in the own key's place, written by now or not, is not used)
+                    const int in = p % 16;
+                    int here = lane;                       // (so that nothing of this is kept in registers through the walk)
+                    asm volatile("" : "+v"(here));
+                    const int g = here >> 4, n = here & 15;
+                    if (n == in) {
+#pragma unroll
+                        for (int c = 0; c < DB; ++c) kr[c] = *(const floatx4*)(own_kv + c * 16 + g * 4);
+                    }
+                    if (g == in / 4) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            if (in % 4 == i) {
+#pragma unroll
+                                for (int c = 0; c < DB; ++c) vr[c][i] = own_kv[D + c * 16 + n];
+                            }
+                    }
+                }
                 floatx4 pr = score(kr);
                 const float alpha = weigh(pr, sees);
 #pragma unroll
                 for (int db = 0; db < DB; ++db) add_values(db, vr[db], pr, alpha);
             };
             int ti = walk;
-            const bool last_first = FUSED && ti == n_tiles - 1;        // (the walk begins with the token's own tile)
-            if (ti < n_tiles && !last_first) ask(ti, ka, va);
-            if constexpr (FUSED) {
-                prepare();
-                if (last_first) ask(ti, ka, va);
-            }
+            if (ti < n_tiles) ask(ti, ka, va);
+            if constexpr (FUSED) prepare();
             while (ti < n_tiles) {
                 if (ti + F32_WALKS < n_tiles) ask(ti + F32_WALKS, kb, vb);
                 step(ti, ka, va);
@@ -505,8 +528,9 @@ int qe_attention_f32_fused(const float* qkv, float* out, float* cache, const int
     const OwnToken own = {q_w, k_w, eps, table, slots};
 #define QE_ATTN_F32_FUSED(DB_)                                                                        \
     case DB_: {                                                                                       \
-        const size_t walks = (size_t)F32_SLOTS * (DB_ * 4 + 2) * 64 * sizeof(float), heads = (size_t)(Hq / Hkv + 1) * D * sizeof(float); \
-        attention_f32_kernel<DB_, F32_WALKS, 2, false, true><<<dim3(T, Hkv), 64 * F32_WALKS, walks > heads ? walks : heads, stream>>>( \
+        constexpr size_t walks = (size_t)F32_SLOTS * (DB_ * 4 + 2) * 64, heads = 16 * 16 * DB_;   \
+        static_assert(heads <= walks, "");                                                            \
+        attention_f32_kernel<DB_, F32_WALKS, 2, false, true><<<dim3(T, Hkv), 64 * F32_WALKS, (walks + 2 * 16 * DB_) * sizeof(float), stream>>>( \
             qkv, out, cache, positions, tok_seq, block_table, max_blocks, tokens, T, Hq, Hkv, P, scale, window, 0, 0, 0.f, tail, own); \
         break;                                                                                        \
     }

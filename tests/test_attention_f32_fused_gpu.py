@@ -1,4 +1,5 @@
-"""Float32 attention of single new tokens with norm, rotation and cache write inside: the bits, and the cache, of the kernels one by one."""
+"""Float32 attention of single new tokens with norm, rotation and cache write inside: the bits, and the cache, of the kernels one by one.  What is
+written nowhere counts for its own token all the same, which needs no page for it."""
 import pytest
 import torch
 
@@ -19,7 +20,7 @@ POS = [0, 1, 15, 16, 17, 47, 112, 127, 128, 143, 500, 1100]
 
 
 @pytest.mark.parametrize("hq,hkv,D,P,window", [(16, 8, 128, 16, 0), (8, 4, 64, 48, 0), (32, 2, 128, 16, 0), (6, 6, 80, 32, 0), (4, 2, 16, 16, 40)])
-@pytest.mark.parametrize("steps", ["all", "no norm", "no rotation", "not written", "some rows"])
+@pytest.mark.parametrize("steps", ["all", "no norm", "no rotation", "not written", "some not written", "some rows"])
 def test_one_launch_and_two(ops, hq, hkv, D, P, window, steps):
     g = torch.Generator().manual_seed(hq * D + P)
     n = len(POS)
@@ -33,9 +34,8 @@ def test_one_launch_and_two(ops, hq, hkv, D, P, window, steps):
         at += pages[i]
         table[i, :pages[i]] = ids
         slots.append(int(ids[p // P]) * P + p % P)
-        there = p + (steps == "not written")
         for j in range(pages[i]):
-            m = max(0, min(there - j * P, P))
+            m = max(0, min(p - j * P, P))
             cache[ids[j], 0].view(hkv, P, D)[:, :m] = torch.randn(hkv, m, D, generator=g)
             cache[ids[j], 1].view(hkv, D, P)[:, :, :m] = torch.randn(hkv, D, m, generator=g)
     cache = cache.view(-1, 2, hkv, P, D).to(DEV)
@@ -47,7 +47,7 @@ def test_one_launch_and_two(ops, hq, hkv, D, P, window, steps):
         qw = kw = None
     if steps == "no rotation":
         rot = None
-    slots = None if steps == "not written" else i32(slots)
+    slots = i32(slots)
     pos, seq, table = i32(POS), i32(range(n)), table.to(DEV)
     assert ops.attention_decode_fused_supported(qkv, cache, hq, rot)
     two = cache.clone()
@@ -57,6 +57,14 @@ def test_one_launch_and_two(ops, hq, hkv, D, P, window, steps):
         rows = i32([3, 0, 11])
     want = ops.attention(q, two, pos, seq, table, D ** -0.5, window, dec_tokens=rows, max_dec_position=max(POS))
     one = cache.clone()
+    if "not written" in steps:
+        left = torch.arange(n, device=DEV) % 2 == 1 if steps == "some not written" else torch.ones(n, dtype=torch.bool, device=DEV)
+        two = cache.clone()
+        ops.qk_rope_store(qkv, hq, hkv, D, pos, qw, kw, 1e-6, rot, torch.where(left, -1, slots), two, P)
+        for i, p in enumerate(POS):                          # (where a page would begin with the token, there is none)
+            if left[i] and p % P == 0:
+                table[i, p // P] = -1
+        slots = None if bool(left.all()) else torch.where(left, -1, slots)
     got = ops.attention_decode_fused(qkv, hq, one, pos, seq, table, D ** -0.5, window, rows if steps == "some rows" else None, max(POS), qw, kw, 1e-6,
                                      rot, slots)
     assert bool(torch.isfinite(want[rows.long()]).all())
