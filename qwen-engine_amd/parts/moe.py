@@ -11,6 +11,17 @@ from .base import Runtime, TensorInfo
 from .registry import register_part
 
 
+def router_logits(x: torch.Tensor, w: torch.Tensor):
+    """The logits of x's rows in 32-bit, float32 [T, outputs], or (True beside them) transposed, float32 [outputs, T].
+
+    Many rows against the router's few: the product the other way round, logits^T = W x^T, is a product of few rows against a
+    large matrix, which fills the chip where the router's few outputs give a handful of tiles; the logits are 32-bit sums of the same
+    products either way.  A router that is held in 32-bit takes bfloat16 rows on its own side only."""
+    if x.shape[0] > 64 and w.shape[0] <= 64 and w.dtype == x.dtype:
+        return ops.gemm(w, x, out_dtype=torch.float32), True
+    return ops.gemm(x, w, out_dtype=torch.float32), False
+
+
 class PolyNormMLP:
     """down(a N(z) + b N(z^2) + c N(z^3) + e), z = up x, N(v) = v / sqrt(mean(v^2) + eps) per token.  The
     up product leaves z in 32-bit; the activation is formed in 32-bit and rounded once."""
@@ -91,10 +102,7 @@ class GroupedMoE:
 
     def forward(self, x: torch.Tensor, ctx, parts_out: Optional[torch.Tensor] = None) -> torch.Tensor:
         s = self.spec
-        # (many rows against the router's few: the product the other way round fills the chip, see BiasedMoE)
-        transposed = x.shape[0] > 64 and self.w_router.shape[0] <= 64
-        logits = ops.gemm(self.w_router, x, out_dtype=torch.float32) if transposed else \
-            ops.gemm(x, self.w_router, out_dtype=torch.float32)
+        logits, transposed = router_logits(x, self.w_router)
         return ops.moe_experts(x, None, None, self.w_gate_up, self.w_down, s.limit, s.slope, interleaved=self.interleaved,
                                grouped_route=(logits, s.num_groups, s.keep_groups, s.top, transposed))
 
@@ -148,12 +156,7 @@ class BiasedMoE:
 
     def forward(self, x: torch.Tensor, ctx, parts_out: Optional[torch.Tensor] = None) -> torch.Tensor:
         s = self.spec
-        # Many rows against the router's few: the product the other way round, logits^T = W_router x^T, is a product of
-        # few rows against a large matrix, which fills the chip where the router's few outputs give a handful of tiles;
-        # the logits are 32-bit sums of the same products either way.
-        transposed = x.shape[0] > 64 and self.w_router.shape[0] <= 64
-        logits = ops.gemm(self.w_router, x, out_dtype=torch.float32) if transposed else \
-            ops.gemm(x, self.w_router, out_dtype=torch.float32)
+        logits, transposed = router_logits(x, self.w_router)
         # (rows_in_activation_type: the experts' output rows of a long portion in bfloat16 instead of 32-bit before
         # they are weighed and added in 32-bit: 7 % less time for the down product and 18 % for the sum at 8192
         # pairs of width 2048, for one more rounding of every expert's output; off)
@@ -241,11 +244,7 @@ class TopSoftmaxMoE:
 
     def forward(self, x: torch.Tensor, ctx) -> torch.Tensor:
         T = x.shape[0]
-        outputs = self.w_router.shape[0]
-        # (many rows against the router's few: the product the other way round fills the chip, see BiasedMoE)
-        transposed = T > 64 and outputs <= 64
-        logits = ops.gemm(self.w_router, x, out_dtype=torch.float32) if transposed else \
-            ops.gemm(x, self.w_router, out_dtype=torch.float32)
+        logits, transposed = router_logits(x, self.w_router)
         route = (logits, None, self.top, 1.0, transposed, self.router_bias, self.e)
         how = self._routing()
         if self.shared is None:

@@ -60,3 +60,29 @@ def test_experts_with_the_routing_inside(ops, T, E, G, keep, top, dtype):
     for z, transposed in ((logits, False), (logits.t().contiguous(), True)):
         got = ops.moe_experts(x, None, None, wgu, wd, 0.8, 1.702, interleaved=True, grouped_route=(z, G, keep, top, transposed))
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("kind", ["grouped", "biased", "top_softmax", "sigmoid"])
+@pytest.mark.parametrize("T", [64, 65, 300])
+def test_a_router_held_in_32_bit(ops, kind, T):
+    """Beside bfloat16 rows and experts, with rows enough for the router's product to be turned: what the rows give in portions of 50."""
+    from qwen_engine_amd.config import spec as S
+    from qwen_engine_amd.parts import Runtime, build_part
+    E, H, F = 16, 128, 64
+    spec = {"grouped": lambda: S.GroupedMoESpec(num_experts=E, top=4, num_groups=4, keep_groups=2, intermediate_size=F, limit=7.0),
+            "biased": lambda: S.BiasedMoESpec(num_experts=E, num_identity=2, top=3, intermediate_size=F, route_scale=1.5),
+            "top_softmax": lambda: S.TopSoftmaxMoESpec(num_experts=E, top=4, intermediate_size=F, shared_intermediate_size=96, shared_gate=True),
+            "sigmoid": lambda: S.SigmoidMoESpec(num_experts=E, top=2, intermediate_size=F)}[kind]()
+    part, rt = build_part(spec, H), Runtime(torch.device(DEV), torch.bfloat16)
+    g = torch.Generator().manual_seed(T)
+    tensors = {n: torch.randn(tuple(t.shape), generator=g) * H ** -0.5 for n, t in type(part).expected_tensors(spec, H).items()}
+    tensors = {n: t if n in ("router", "correction") else t.bfloat16() for n, t in tensors.items()}
+    part.load(tensors, rt)
+    assert part.w_router.dtype == torch.float32
+    from types import SimpleNamespace
+    ctx = SimpleNamespace(rt=rt)
+    x = torch.randn(T, H, generator=g).bfloat16().to(DEV)
+    got = part.forward(x, ctx).sum(0)
+    want = torch.cat([part.forward(part_x, ctx).sum(0) for part_x in x.split(50)])
+    # (the same logits and choices; the experts' products in other forms, whose sums are rounded to bfloat16 once on the way)
+    assert float((got - want).norm() / want.norm()) < 2.0 ** -7
