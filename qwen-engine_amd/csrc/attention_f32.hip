@@ -51,7 +51,7 @@ __device__ __forceinline__ float max_over_rows_of_lanes(float v) {
 // and value to the cache, with the sums and roundings of the kernel that does this for few tokens, while the walks' first tiles are on their
 // way.  The walk with the token's own key takes it, and its value, from shared memory: they may be written nowhere, and their page may not be
 // there.  (2 tokens of 16 heads on 8 over 512 keys: the two kernels 22.6 and 3.9 us, in one 21.6, and a launch
-// less for the host, some 12 us of a step that is not recorded.)
+// less for the host, some 12 us of a step that is not recorded; of 414 and 731 keys 27.3, 26.5 with the own key read back from the cache.)
 struct OwnToken {
     const float* q_w;
     const float* k_w;
@@ -127,7 +127,7 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? (ROWS || AHEA
     // were two trips to memory of their own); a tile's page is then the same for the wave, and so is its place in it.  Other page sizes:
     // every lane looks its own keys' pages up.
     const bool whole = P % 16 == 0;
-    // (FUSED: the last tile may hold no key but the token's own; its page is then not looked up)
+    // (FUSED: the last tile may hold no key but the token's own; its page is then not looked up, and what is read is some page of the cache)
     const bool own_alone = FUSED && max(p / 16 * 16, lo) >= p;
     int my_page = 0;
     const auto page_of = [&](int ti, int walk) {               // asked for tile by tile, in order
@@ -206,11 +206,9 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? (ROWS || AHEA
         for (int j = wave; j < G + 2; j += NW) {
             const float* src = q + (t * (Hq + 2 * Hkv) + (j < G ? kvh * G + j : j == G ? Hq + kvh : Hq + Hkv + kvh)) * D;
             if (j > G) {                                   // the value tile is [D][P]
-                for (int d = lane; d < D; d += 64) {
-                    const float v = src[d];
-                    own_kv[D + d] = v;
-                    if (slot >= 0) kv[((long)(Hkv + kvh) * D + d) * P + slot % P] = v;
-                }
+                for (int d = lane; d < D; d += 64) own_kv[D + d] = src[d];
+                if (slot >= 0)
+                    for (int d = lane; d < D; d += 64) kv[((long)(Hkv + kvh) * D + d) * P + slot % P] = own_kv[D + d];
                 continue;
             }
             const float* w = j < G ? own.q_w : own.k_w;
@@ -304,7 +302,6 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? (ROWS || AHEA
             // (pages of whole tiles.  What of a tile is not there lies in its page all the same: it is read, and zeros take its place)
             floatx4 ka[DB], va[DB], kb[DB], vb[DB];
             const auto ask = [&](int ti, floatx4 (&kr)[DB], floatx4 (&vr)[DB]) {
-                if (FUSED && own_alone && ti == n_tiles - 1) return;
                 const int in = tile_key(ti) % P;
                 const float* const page = cache + (long)page_of(ti, walk) * page_stride;
                 const float* const krow = page + ((long)kvh * P + in + n) * D + g * 4;

@@ -1015,7 +1015,7 @@ def attention_decode_fused_supported(qkv: torch.Tensor, cache: torch.Tensor, num
     if table is not None and table.shape[1] != D:
         return False
     if qkv.dtype == torch.float32 and cache.dtype == torch.float32:
-        return bool(lib.qe_attention_f32_fused_supported(qkv.shape[0], num_heads, cache.shape[2], D, cache.shape[3]))
+        return cache.shape[0] > 0 and bool(lib.qe_attention_f32_fused_supported(qkv.shape[0], num_heads, cache.shape[2], D, cache.shape[3]))
     return (qkv.dtype == torch.bfloat16 and
             bool(lib.qe_attention_decode_supported(num_heads, cache.shape[2], D, cache.shape[3], _DT[qkv.dtype])))
 

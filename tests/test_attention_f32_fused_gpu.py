@@ -82,4 +82,5 @@ def test_what_is_not_taken(ops):
     assert not ops.attention_decode_fused_supported(qkv(1, 34, 2, 16), cache(2, 16, 16), 34, None)
     assert not ops.attention_decode_fused_supported(qkv(1, 4, 2, 144), cache(2, 16, 144), 4, None)
     assert not ops.attention_decode_fused_supported(qkv(1, 4, 2, 16), cache(2, 5, 16), 4, None)
+    assert not ops.attention_decode_fused_supported(qkv(1, 4, 2, 16), cache(2, 16, 16)[:0], 4, None)
     assert not ops.attention_decode_fused_supported(qkv(1, 4, 2, 16), cache(2, 16, 16).bfloat16(), 4, None)
