@@ -10,7 +10,7 @@
 int qe_attention_generic(const void* q, void* out, const void* cache, const int* positions,
                          const int* tok_seq, const int* block_table, int max_blocks, const int* tokens,
                          int T, int Hq, int Hkv, int D, int P, float scale, int window, int keep_first, int sink,
-                         float softcap, int dt_a, hipStream_t stream, const AttnTail& tail);
+                         float softcap, int dt_a, int requests, hipStream_t stream, const AttnTail& tail);
 bool qe_attention_decode_ok(int Hq, int Hkv, int D, int P, int dt_a);
 size_t qe_attention_decode_workspace(int n_dec, int Hq, int D, int num_splits);
 int qe_attention_decode(const void* q, void* out, const void* cache, const int* dec_tokens, int n_dec,
@@ -138,19 +138,20 @@ extern "C" int qe_attention_prefill_run(const void* q, void* out, const void* ca
 
 // out_stride, dv, sink_heads, gate, gate_stride, dt_g, here and below: see AttnTail (0, 0, null, null: plain rows of Hq * D
 // numbers, a sink of score 0).  tokens: null for all T rows of q, else n_tokens row indices.  keep_first: the first keys of a request
-// that every later query sees wherever its window stands; sink: a 1 is added to the softmax's denominator.
+// that every later query sees wherever its window stands; sink: a 1 is added to the softmax's denominator.  requests: to how many
+// requests the tokens belong, or 0: it only chooses between forms that give the same numbers.
 extern "C" int qe_attention_tail(const void* q, void* out, const void* cache, const int* positions,
                             const int* tok_seq, const int* block_table, int max_blocks, const int* tokens,
                             int n_tokens, int Hq, int Hkv, int D, int P, float scale, int window, int keep_first,
                             int sink, float softcap, int dt_a, long out_stride, int dv, const float* sink_heads,
-                            const void* gate, long gate_stride, int dt_g, hipStream_t stream) {
+                            const void* gate, long gate_stride, int dt_g, int requests, hipStream_t stream) {
     QE_TAIL_CHECK();
     QE_REQUIRE(n_tokens >= 0 && Hq > 0 && Hkv > 0 && D > 0 && P > 0 && max_blocks > 0, "attention: bad sizes");
     QE_REQUIRE(Hq % Hkv == 0, "attention: %d query heads are no multiple of %d key/value heads", Hq, Hkv);
     QE_REQUIRE(keep_first >= 0 && (window >= 0 || keep_first == 0), "attention: kept first keys go with a window of the last keys");
     if (n_tokens == 0) return 0;
     return qe_attention_generic(q, out, cache, positions, tok_seq, block_table, max_blocks, tokens, n_tokens,
-                                Hq, Hkv, D, P, scale, window, keep_first, sink, softcap, dt_a, stream,
+                                Hq, Hkv, D, P, scale, window, keep_first, sink, softcap, dt_a, requests, stream,
                                 make_tail(Hq, D, out, out_stride, dv, sink_heads, gate, gate_stride, dt_g));
 }
 
@@ -159,7 +160,7 @@ extern "C" int qe_attention(const void* q, void* out, const void* cache, const i
                             const int* block_table, int max_blocks, const int* tokens, int n_tokens, int Hq, int Hkv, int D,
                             int P, float scale, int window, int keep_first, int sink, float softcap, int dt_a, hipStream_t stream) {
     return qe_attention_tail(q, out, cache, positions, tok_seq, block_table, max_blocks, tokens, n_tokens, Hq, Hkv, D, P, scale,
-                             window, keep_first, sink, softcap, dt_a, 0, 0, nullptr, nullptr, 0, QE_F32, stream);
+                             window, keep_first, sink, softcap, dt_a, 0, 0, nullptr, nullptr, 0, QE_F32, 0, stream);
 }
 
 extern "C" int qe_attention_decode_supported(int Hq, int Hkv, int D, int P, int dt_a) {

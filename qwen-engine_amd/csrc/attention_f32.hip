@@ -43,9 +43,9 @@ __device__ __forceinline__ float max_over_rows_of_lanes(float v) {
 //
 // ROWS (no window, at most eight heads a key/value head): the 16 columns are 16 / G tokens' heads, which see the keys of one
 // request up to their own positions, so that many tokens read and multiply a tile once instead of each by itself; neighbours in the list that belong to
-// different requests are walked one request after the other.  A column's sums are those it has alone: a tile it sees nothing of leaves
+// different requests are walked by blocks of their own, block z the z-th request's, the last block what is left, one after the other.  A column's sums are those it has alone: a tile it sees nothing of leaves
 // them as they are.  (Portions of 328 and 416 rows of 16 heads of 128 on 8: 200 us, a block a token, and 42; 2048 rows 1980, 300; 400 of 64
-// heads 120, 78; 40 rows 11.7, 11.2; two of 50 and 30, where a block holds tokens of both, 12.8, 16.6.)
+// heads 120, 78; 40 rows 11.7, 11.2.)
 //
 // FUSED (eight waves, AHEAD 2, at most 16 heads a key/value head): q is the q|k|v rows; the waves first norm and turn the token's heads and write its key
 // and value to the cache, with the sums and roundings of the kernel that does this for few tokens, while the walks' first tiles are on their
@@ -93,6 +93,14 @@ __global__ __launch_bounds__(64 * NW, NW == F32_SLOTS && DB <= 8 ? (ROWS || AHEA
     // (one round, but for a block whose tokens belong to several requests, and for one with a value that is infinite or NaN: where a column does
     // not see it, it has met a weight of 0, so each token then has a round of its own)
     unsigned long todo = ROWS ? __ballot(head_ok) : 1ul;
+    if (ROWS) {
+        const auto of_first = [&]() { return __ballot(head_ok && seq == __builtin_amdgcn_readlane(seq, __builtin_ctzl(todo))); };
+        for (int z = blockIdx.z; z > 0; --z) {
+            todo &= ~of_first();
+            if (!todo) return;                             // (the whole block: no barrier has been met yet)
+        }
+        if (blockIdx.z + 1 < gridDim.z) todo &= of_first();
+    }
     bool one_by_one = false;
     do {
     const int next = ROWS ? __builtin_ctzl(todo) : 0;
@@ -465,9 +473,15 @@ bool qe_attention_f32_ok(int Hq, int Hkv, int D, int P) {
     return D % 16 == 0 && D >= 16 && D <= 256 && Hq % Hkv == 0 && P >= 1;
 }
 
+// requests: to how many requests the tokens belong (0: not known).  Tokens each of a request of its own share nothing, and a few short portions
+// little that a block a token, with a third more waves on a unit, does not make up for.  (us, 16 heads of 128 on 8, tokens several to a block with the blocks' requests one after
+// the other, each by a block, and a token a block: 33 single tokens of 400 keys 271, 56.9, 56.2; 64 of 400 346, 78.6, 82.0, of 1000 762, 168, 184; 256 of 100 143,
+// 104, 78.3, of 400 366, 258, 220.  16 portions of 4 from the start 15.9, 11.5, 9.8; 64 of 4 16.2, 14.7, 25.7; 64 of 2 behind 500 keys 202, 73.3, 129; 8 of 9 behind 1000
+// 144, 74.7, 113; 50 and 30 rows 16.3, 11.5, 12.1; one of 40 10.5, 11.1, 10.9.)  Where there are more blocks than units the requests of a block
+// take turns: others fill the time (32 portions of 20 behind 100 keys 46.7 and 41.9, 117 a token a block; 328 and 416 rows 39.6 and 43.3).
 int qe_attention_f32(const float* q, float* out, const float* cache, const int* positions, const int* tok_seq,
                      const int* block_table, int max_blocks, const int* tokens, int T, int Hq, int Hkv, int D,
-                     int P, float scale, int window, int keep_first, int sink, float softcap, hipStream_t stream, const AttnTail& tail) {
+                     int P, float scale, int window, int keep_first, int sink, float softcap, int requests, hipStream_t stream, const AttnTail& tail) {
     QE_REQUIRE(qe_attention_f32_ok(Hq, Hkv, D, P), "attention (32-bit): sizes not taken");
     const int groups16 = (Hq / Hkv + 15) / 16;
     QE_REQUIRE((long)Hkv * groups16 <= 65535, "attention (32-bit): too many heads");
@@ -475,8 +489,12 @@ int qe_attention_f32(const float* q, float* out, const float* cache, const int* 
     // eight waves while the blocks leave compute units idle
     const bool few = (long)T * Hkv * groups16 <= 256;
     const int G = Hq / Hkv;
-    const bool rows = !few && window == 0 && keep_first == 0 && G <= 8 && T / (16 / G) < 65535;
-    if (rows) grid = dim3(Hkv, qe_cdiv(T, 16 / G));
+    const bool apart = requests > 0 && (requests >= T || (T < 8L * requests && (long)T * Hkv <= 512));
+    const bool rows = !few && !apart && window == 0 && keep_first == 0 && G <= 8 && T / (16 / G) < 65535;
+    if (rows) {
+        grid = dim3(Hkv, qe_cdiv(T, 16 / G));
+        if (requests != 1 && (long)grid.x * grid.y <= 256) grid.z = min(4, 16 / G);
+    }
 #define QE_ATTN_F32_FORM(DB_, NW_, AHEAD_, ROWS_)                                                     \
     do {                                                                                              \
         const size_t lds = (size_t)F32_SLOTS * (DB_ * 4 + 2) * 64 * sizeof(float);                    \

@@ -97,7 +97,7 @@ __global__ __launch_bounds__(64) void attention_generic_kernel(
 bool qe_attention_f32_ok(int Hq, int Hkv, int D, int P);
 int qe_attention_f32(const float* q, float* out, const float* cache, const int* positions, const int* tok_seq,
                      const int* block_table, int max_blocks, const int* tokens, int T, int Hq, int Hkv, int D,
-                     int P, float scale, int window, int keep_first, int sink, float softcap, hipStream_t stream, const AttnTail& tail);
+                     int P, float scale, int window, int keep_first, int sink, float softcap, int requests, hipStream_t stream, const AttnTail& tail);
 
 // 32-bit attention goes to the kernel on the matrix units (attention_f32.hip) where it takes the
 // sizes, unless qe_use_matrix_f32(0) has switched that off.
@@ -106,10 +106,10 @@ extern int g_qe_matrix_f32;
 int qe_attention_generic(const void* q, void* out, const void* cache, const int* positions,
                          const int* tok_seq, const int* block_table, int max_blocks, const int* tokens,
                          int T, int Hq, int Hkv, int D, int P, float scale, int window, int keep_first, int sink,
-                         float softcap, int dt_a, hipStream_t stream, const AttnTail& tail) {
+                         float softcap, int dt_a, int requests, hipStream_t stream, const AttnTail& tail) {
     if (dt_a == QE_F32 && g_qe_matrix_f32 && qe_attention_f32_ok(Hq, Hkv, D, P))
         return qe_attention_f32((const float*)q, (float*)out, (const float*)cache, positions, tok_seq, block_table,
-                                max_blocks, tokens, T, Hq, Hkv, D, P, scale, window, keep_first, sink, softcap, stream, tail);
+                                max_blocks, tokens, T, Hq, Hkv, D, P, scale, window, keep_first, sink, softcap, requests, stream, tail);
     QE_REQUIRE(D <= ATTN_MAX_D, "attention: head_dim=%d exceeds %d", D, ATTN_MAX_D);
     QE_REQUIRE(Hq <= 65535, "attention: too many heads");
     dim3 grid(T, Hq);

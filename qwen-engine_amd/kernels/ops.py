@@ -87,7 +87,7 @@ def load_library():
         "qe_gemm_first_columns": [i32, i32, i32, i32],
         "qe_attention": [vp, vp, vp, vp, vp, vp, i32, vp, i32, i32, i32, i32, i32, f32, i32, i32, i32, f32, i32, vp],
         "qe_attention_tail": [vp, vp, vp, vp, vp, vp, i32, vp, i32, i32, i32, i32, i32, f32, i32, i32, i32, f32, i32,
-                              i64, i32, vp, vp, i64, i32, vp],
+                              i64, i32, vp, vp, i64, i32, i32, vp],
         "qe_qkv_conv_rope_store": [vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, i32, i32, i32, i32, i32, vp],
         "qe_scale_f32": [vp, i64, f32, vp],
         "qe_moe_route_biased": [vp, vp, vp, vp, i32, i32, i32, f32, i32, vp, i32, i32, vp],
@@ -859,7 +859,7 @@ def attention(q: torch.Tensor, cache: torch.Tensor, positions: torch.Tensor, tok
               max_other_keys: int = 0, prefill_segment_keys: int = -1,
               other_keys_row: Optional[int] = None, shared_keys: Optional[torch.Tensor] = None,
               keep_first: int = 0, sink=False, chunk: int = 0, softcap: float = 0.0, v_dim: int = 0,
-              gate: Optional[torch.Tensor] = None, dec_blocks: bool = False) -> torch.Tensor:
+              gate: Optional[torch.Tensor] = None, dec_blocks: bool = False, other_requests: int = 0) -> torch.Tensor:
     """q [T, Hq, D]; cache [pages, 2, Hkv, P, D] (key tiles [P][D], value tiles transposed [D][P]);
     positions, tok_seq int32 [T]; block_table int32 [B, max_blocks].  Token t sees the keys at
     positions max(0, p - window + 1) .. p of request tok_seq[t] (window 0: all).  The caller
@@ -892,7 +892,9 @@ def attention(q: torch.Tensor, cache: torch.Tensor, positions: torch.Tensor, tok
     other requests read too.  A hint for the decode kernel's loads; results do not depend on it.
 
     dec_blocks: more than eight dec_tokens may have a block each that walks a token's keys (quicker; a row's sums then have another
-    order than alone, where every 128 keys are summed by themselves)."""
+    order than alone, where every 128 keys are summed by themselves).
+
+    other_requests: to how many requests other_tokens belong, or 0.  A hint for the float32 kernel; results do not depend on it."""
     lib = load_library()
     _need(q, "q", _ACT, (None, None, None))
     T, Hq, D = q.shape
@@ -944,11 +946,11 @@ def attention(q: torch.Tensor, cache: torch.Tensor, positions: torch.Tensor, tok
     if keep_first or sink or chunk:
         prefill_segment_keys = 0    # (no segments of keys: such walks are short)
 
-    def generic(tokens):
+    def generic(tokens, requests=0):
         n = T if tokens is None else tokens.shape[0]
         _check(lib.qe_attention_tail(q.data_ptr(), out.data_ptr(), cache.data_ptr(), positions.data_ptr(),
                                 tok_seq.data_ptr(), block_table.data_ptr(), max_blocks, _ptr(tokens), n,
-                                Hq, Hkv, D, P, float(scale), int(window), keep_first, sink, softcap, _DT[q.dtype], *tail, _stream()),
+                                Hq, Hkv, D, P, float(scale), int(window), keep_first, sink, softcap, _DT[q.dtype], *tail, int(requests), _stream()),
                "attention")
 
     if dec_tokens is None and other_tokens is None:
@@ -968,7 +970,7 @@ def attention(q: torch.Tensor, cache: torch.Tensor, positions: torch.Tensor, tok
                                                0 if dec_blocks else DECODE_SPLIT_KEYS, ws.data_ptr(), nbytes, *tail, _stream()),
                    "attention (decode)")
         else:
-            generic(dec_tokens)
+            generic(dec_tokens, n_dec)
     if other_tokens is not None and other_tokens.shape[0]:
         _need(other_tokens, "other_tokens", torch.int32, (None,), dev)
         if other_tiles is not None and algo != ALGO_GENERIC and attention_prefill_supported(q, cache):
@@ -1002,7 +1004,7 @@ def attention(q: torch.Tensor, cache: torch.Tensor, positions: torch.Tensor, tok
                                                 *tail, _stream()),
                    "attention (prefill)")
         else:
-            generic(other_tokens)
+            generic(other_tokens, other_requests)
     return out
 
 

@@ -57,7 +57,8 @@ class PagedAttention:
         return {"dec_tokens": np.asarray(dec, dtype=np.int32),
                 "other_tokens": np.concatenate(other) if other else np.zeros(0, dtype=np.int32),
                 "max_dec_position": max([s.kv_before for s in seqs if s.q_len == 1], default=0),
-                "max_other_keys": max([s.kv_before + s.q_len for s in seqs if s.q_len > 1], default=0)}
+                "max_other_keys": max([s.kv_before + s.q_len for s in seqs if s.q_len > 1], default=0),
+                "other_requests": len(other)}
 
     GRAPH_SPLIT_BUCKET = 8      # a recorded decode step serves positions up to the next multiple of this many key splits
 
@@ -302,6 +303,7 @@ class PagedAttention:
                               other_tokens=ex["other_tokens"],
                               other_tiles=self._other_tiles(ctx) if ex["other_tokens"] is not None else None,
                               max_other_keys=ex.get("max_other_keys", 0), other_keys_row=ex.get("other_keys_row"),
+                              other_requests=ex.get("other_requests", 0),
                               shared_keys=ctx.shared_keys, dec_blocks=True)
         return self._project_out(o.view(T, self.hq * self.d))
 
@@ -442,6 +444,7 @@ class ConvAttention(PagedAttention):
                           other_tokens=ex["other_tokens"],
                           other_tiles=self._other_tiles(ctx) if ex["other_tokens"] is not None else None,
                           max_other_keys=ex.get("max_other_keys", 0), other_keys_row=ex.get("other_keys_row"),
+                          other_requests=ex.get("other_requests", 0),
                           shared_keys=ctx.shared_keys, keep_first=self.keep_first, sink=self.sink, softcap=self.softcap)
         o = o.view(T, self.hq * self.d)
         if parts_out is not None:
@@ -657,6 +660,7 @@ class ChunkAttention(PagedAttention):
                       other_tokens=ex["other_tokens"],
                       other_tiles=self._other_tiles(ctx) if ex["other_tokens"] is not None else None,
                       max_other_keys=ex.get("max_other_keys", 0), other_keys_row=ex.get("other_keys_row"),
+                      other_requests=ex.get("other_requests", 0),
                       shared_keys=ctx.shared_keys, chunk=self.chunk, sink=False if self.sink is None else self.sink,
                       v_dim=self.dv, gate=y[:, y.shape[1] - n:] if self.spec.output_gate else None, out=out)
 

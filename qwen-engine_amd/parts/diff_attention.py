@@ -112,6 +112,7 @@ class DiffAttention(PagedAttention):
                           other_tokens=ex["other_tokens"],
                           other_tiles=self._other_tiles(ctx) if ex["other_tokens"] is not None else None,
                           max_other_keys=ex.get("max_other_keys", 0), other_keys_row=ex.get("other_keys_row"),
+                          other_requests=ex.get("other_requests", 0),
                           shared_keys=ctx.shared_keys)
         gate = rows[:, rows.shape[1] - self.h:] if self.gated else None
         o = ops.diff_heads(a, self.h, self.g, self.dv, self.lam, self.eps, 1.0 - self.diff, gate=gate)

@@ -50,6 +50,10 @@ def test_tokens_of_a_block_and_alone(ops, hq, hkv, D, P, softcap, portions, odd)
     run = lambda which: ops.attention(q.to(DEV), cache, i32(pos), i32(seq), table, D ** -0.5, dec_tokens=i32([]), other_tokens=i32(which),
                                       softcap=softcap).cpu()
     every = run(range(T))
+    for requests in (1, len(portions), T):       # (a hint: other forms, the same bits; NaN compares as NaN)
+        hinted = ops.attention(q.to(DEV), cache, i32(pos), i32(seq), table, D ** -0.5, dec_tokens=i32([]), other_tokens=i32(range(T)), softcap=softcap,
+                               other_requests=requests).cpu()
+        assert torch.equal(hinted.nan_to_num(), every.nan_to_num()) and torch.equal(hinted.isnan(), every.isnan()), requests
     for t in sorted({0, 1, T // 2, T - 21, T - 20, T - 8, T - 1, *range(60, 80)}):
         alone = run([t])[t]
         assert torch.equal(torch.nan_to_num(every[t]), torch.nan_to_num(alone)) and torch.equal(every[t].isnan(), alone.isnan()), t
@@ -61,3 +65,57 @@ def test_tokens_of_a_block_and_alone(ops, hq, hkv, D, P, softcap, portions, odd)
             assert float((every[t].double() - want).norm() / want.norm()) < 1e-5, t
         else:
             assert not every[t, 0, 5].isfinite()
+
+
+@pytest.mark.parametrize("hq,hkv", [(8, 4), (8, 8), (20, 4)])
+@pytest.mark.parametrize("counts", [[1] * 67, [2, 3] * 14, [4] * 40, [1, 9, 1, 5, 30, 1, 1, 2] * 4])
+def test_many_requests_of_few_tokens(ops, hq, hkv, counts):
+    """Blocks whose tokens belong to two to sixteen requests, some of which other blocks take: a token's bits are those it has alone."""
+    D, P = 64, 16
+    g = torch.Generator().manual_seed(len(counts))
+    before = [(37 * i) % 90 for i in range(len(counts))]
+    pages = [-(-(b + c) // P) for b, c in zip(before, counts)]
+    table, at = torch.full((len(counts), max(pages)), -1, dtype=torch.int32), 0
+    for i, n in enumerate(pages):
+        table[i, :n] = torch.arange(at, at + n, dtype=torch.int32)
+        at += n
+    cache = torch.randn(at, 2, hkv, P, D, generator=g).to(DEV)
+    pos = [b + j for b, c in zip(before, counts) for j in range(c)]
+    seq = [i for i, c in enumerate(counts) for _ in range(c)]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    q, T = torch.randn(len(pos), hq, D, generator=g).to(DEV), len(pos)
+    assert T * hkv > 256                     # (fewer have a block each)
+    run = lambda which, **kw: ops.attention(q, cache, i32(pos), i32(seq), table.to(DEV), 0.1, dec_tokens=i32([]), other_tokens=i32(which), **kw)
+    alone = torch.stack([run([t])[t] for t in range(T)])
+    for requests in (0, 1, len(counts)):
+        assert torch.equal(run(range(T), other_requests=requests), alone), requests
+    assert torch.equal(ops.attention(q, cache, i32(pos), i32(seq), table.to(DEV), 0.1), alone)
+    if max(counts) == 1:
+        got = ops.attention(q, cache, i32(pos), i32(seq), table.to(DEV), 0.1, dec_tokens=i32(range(T)), max_dec_position=max(pos))
+        assert torch.equal(got, alone)
+
+
+def test_many_single_tokens_take_no_turns(ops):
+    """Twice the tokens, each of a request of its own, take less than three times as long (with a block's requests one after another, six times)."""
+    hq, hkv, D, P, keys = 16, 8, 128, 16, 400
+    cache = torch.randn(64 * keys // P, 2, hkv, P, D, device=DEV)
+    table = torch.arange(64 * keys // P, dtype=torch.int32, device=DEV).view(64, -1)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    q = torch.randn(64, hq, D, device=DEV)
+
+    def took(n):
+        rows, pos = i32(range(n)), i32([keys - 1] * 64)
+        run = lambda: ops.attention(q, cache, pos, i32(range(64)), table, 0.1, dec_tokens=rows, max_dec_position=keys - 1)
+        run()
+        times = []
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            torch.cuda.synchronize()
+            a.record()
+            for _ in range(20):
+                run()
+            b.record()
+            b.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+    assert took(64) < 3 * took(32)
