@@ -19,8 +19,8 @@ from ..cache.manager import CacheManager, OutOfPages
 from ..cache.plan import CachePlan
 from ..config.registry import config_from_folder
 from ..kernels import ops
-from ..parts.base import CacheBinding, Runtime
-from ..parts.model import DecoderModel, cache_plan, expected_tensors
+from ..parts.base import CacheBinding, Runtime, is_replaced
+from ..parts.model import MODEL_FORWARD, DecoderModel, cache_plan, expected_tensors
 from ..weights.loader import read_checked
 from .batch import SeqInfo, StepContext
 
@@ -551,6 +551,16 @@ class ModelRunner:
             return ops.argmax_static(logits, tokens)
         return ops.argmax(logits, out=tokens)
 
+    def _recorded_forward(self, ctx: StepContext, updates) -> torch.Tensor:
+        """Inside a recording: the model's logits, the block tables brought up to date before.  The model does that beside its embedding; a
+        forward that a program has put in the place of its own need not know of it."""
+        if is_replaced(self.model, MODEL_FORWARD):
+            for table, (idx, val) in zip(self.tables, updates):
+                ops.scatter_int(table, idx, val)
+        else:
+            ctx.table_updates = updates
+        return self.model.forward(ctx, self.bindings)
+
     def _decode_step_with_graph(self, entries: Sequence[StepEntry], greedy: bool = False):
         seqs, token_ids, positions, tok_seq, rows, slots, upd_idx, upd_val = self._single_token_layout(entries)
         self._check_bounds(seqs, slots, upd_idx, upd_val)
@@ -723,12 +733,12 @@ class ModelRunner:
         ctx = StepContext(rt=self.rt, page_size=self.page_size, num_tokens=B + T, seqs=seqs, token_ids=d_tok,
                           positions=d_pos, tok_seq=d_seq, block_tables=self.tables,
                           shared_keys=self.shared_keys, late=self._late, slots=d_slots,
-                          logit_rows=d_rows, state_slots=d_state, max_position=0, table_updates=d_upd,
+                          logit_rows=d_rows, state_slots=d_state, max_position=0,
                           extras={cls: dict(cls.mixed_graph_extras(B, T, k, dev, dyn))
                                   for cls, k, dyn in zip(self._step_classes, part_keys, d_dyn)})
 
         def run():
-            logits = self.model.forward(ctx, self.bindings)
+            logits = self._recorded_forward(ctx, d_upd)
             return logits, self._recorded_argmax(logits) if greedy else None
 
         torch.cuda.synchronize()
@@ -813,13 +823,13 @@ class ModelRunner:
         ctx = StepContext(rt=self.rt, page_size=self.page_size, num_tokens=T, seqs=seqs, token_ids=d_tok,
                           positions=d_pos, tok_seq=d_seq, block_tables=self.tables,
                           shared_keys=self.shared_keys, late=self._late, slots=d_slots,
-                          logit_rows=d_rows, state_slots=d_state, max_position=0, table_updates=d_upd,
+                          logit_rows=d_rows, state_slots=d_state, max_position=0,
                           extras={cls: dict(cls.portion_graph_extras(T, dev) if k is None
                                             else cls.portion_graph_extras(T, dev, k))
                                   for cls, k in zip(self._step_classes, part_keys)})
 
         def run():
-            logits = self.model.forward(ctx, self.bindings)
+            logits = self._recorded_forward(ctx, d_upd)
             return logits, self._recorded_argmax(logits) if greedy else None
 
         torch.cuda.synchronize()
@@ -865,12 +875,12 @@ class ModelRunner:
         ctx = StepContext(rt=self.rt, page_size=self.page_size, num_tokens=B, seqs=seqs, token_ids=d_tok,
                           positions=d_pos, tok_seq=d_seq, block_tables=self.tables,
                           shared_keys=self.shared_keys, late=self._late, slots=d_slots,
-                          logit_rows=d_rows, state_slots=d_state, max_position=0, table_updates=d_upd,
+                          logit_rows=d_rows, state_slots=d_state, max_position=0,
                           extras={cls: dict(cls.graph_extras(B, k, dev)) if hasattr(cls, "graph_extras") else {}
                                   for cls, k in zip(self._step_classes, part_keys)})
 
         def run():
-            logits = self.model.forward(ctx, self.bindings)
+            logits = self._recorded_forward(ctx, d_upd)
             return logits, self._recorded_argmax(logits) if greedy else None
 
         torch.cuda.synchronize()
