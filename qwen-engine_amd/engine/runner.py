@@ -83,7 +83,7 @@ class ModelRunner:
     # Recorded graphs kept; the least recently used goes first.  Each holds its own activations and
     # workspaces (tens of MB at the small model's sizes, a GB for a long portion at the large models'),
     # so they are bounded by their bytes too (graph_memory_bytes).  A server whose batch
-    # and contexts wander passes through 15 row counts up to 64 rows times a bucket per 1024 keys, and
+    # and contexts wander passes through 15 row counts up to 64 rows times a bucket per 1024 keys (the first two, of 512), and
     # recording a step again costs several replays of it.
     MAX_GRAPHS = 96
 
@@ -212,12 +212,17 @@ class ModelRunner:
         step = 8 if n <= 64 else 32
         return -(-n // step) * step
 
-    def _graph_for(self, key, kind: str, record):
+    def _graph_for(self, key, kind: str, greedy: bool, record):
         """The recorded step for ``key`` (most recently used last), recorded now by ``record()`` if its
-        shape has been met often enough, or None: the step then runs as it comes."""
+        shape has been met often enough, or None: the step then runs as it comes.  One recording a shape: with the picks of every row's
+        largest logit if they have ever been asked for (the logits are there either way)."""
         rec = self._graphs.pop(key, None)
+        no_picks = rec is not None and greedy and rec["tokens"] is None and rec["logits"].shape[0] > 0
+        if no_picks:                                           # (recorded anew with them, when what still runs of it is done)
+            torch.cuda.synchronize()
+            rec = None
         if rec is None:
-            if kind != "decode":
+            if kind != "decode" and not no_picks:
                 seen = self._graph_seen.get(key, 0) + 1
                 if seen < self.graph_record_after:
                     if len(self._graph_seen) >= 4096:          # (shapes that never came back)
@@ -591,7 +596,7 @@ class ModelRunner:
                     ops.scatter_int(self.tables[g], torch.from_numpy(upd_idx[g]).to(self.rt.device),
                                     torch.from_numpy(upd_val[g]).to(self.rt.device))
                 upd_idx[g] = upd_val[g] = np.zeros(0, dtype=i32)
-        rec = self._graph_for((B, part_keys, greedy), "decode", lambda: self._record_decode_graph(B, part_keys, cap, greedy))
+        rec = self._graph_for((B, part_keys), "decode", greedy, lambda: self._record_decode_graph(B, part_keys, cap, greedy))
         iota, none, zero = rec["iota"], rec["none"], rec["zero"]       # 0 .. B - 1; cap times -1; cap zeros
         # (a row's table row is its request's state slot: tok_seq serves as both)
         parts = [token_ids, positions, tok_seq, iota, tok_seq]
@@ -640,7 +645,7 @@ class ModelRunner:
         max_dec_position = max([self.cache.get(e.req_id).num_tokens for e in ordered[:-1]], default=0)
         portion_keys = self.cache.get(ordered[-1].req_id).num_tokens + T1
         part_keys = tuple(cls.mixed_graph_key(max_dec_position, portion_keys) for cls in self._step_classes)
-        rec = self._graph_for(("mixed", B, T, part_keys, greedy), "mixed", lambda: self._record_mixed_graph(B, T, part_keys, cap, greedy))
+        rec = self._graph_for(("mixed", B, T, part_keys), "mixed", greedy, lambda: self._record_mixed_graph(B, T, part_keys, cap, greedy))
         if rec is None:
             return None
         tokens = self._check_and_reserve(ordered)
@@ -762,7 +767,7 @@ class ModelRunner:
         keys = self.cache.get(entry.req_id).num_tokens + T
         part_keys = tuple(cls.portion_graph_key(T, keys) if hasattr(cls, "portion_graph_key") else None
                           for cls in self._step_classes)
-        rec = self._graph_for(("portion", T, n_want, part_keys, greedy), "portion",
+        rec = self._graph_for(("portion", T, n_want, part_keys), "portion", greedy,
                               lambda: self._record_portion_graph(T, n_want, cap, part_keys, greedy))
         if rec is None:
             return None
