@@ -800,15 +800,17 @@ size_t qe_attention_decode_workspace(int n_dec, int Hq, int D, int num_splits) {
 // 83.7, 60.1.  Cut: 9 rows of 1900 22.8, 22.8 (7 segments), of 3800 40.6, 38.6; 16 of 1040 25.2, 21.5 (4; in one 27.5), of 4000 63.6, 57.7; 24 of
 // 4000 87.2, 79.7 (5; in one 93.7); 32 of 4000 113, 106 (2; in one 112).  Four rows of 400 13.0, 13.4, of 1000 14.3, 16.0, of 2000 16.2, 16.4: up to eight
 // tokens are the splits'.)  Up to 16 tokens, which every other kernel of their step takes in one order, a token's segments follow its own position
-// alone: its bits are the same beside any others.
+// alone: its bits are the same beside any others.  With more they follow how many those are, and the last position as recorded steps know it, the end
+// of a stretch of 1024 (the first two, of 512): a step has the same ones whether it is recorded or runs as it comes.
 static int block_segments(int n_dec, int Hkv, int max_position, int window, int sink, float softcap, int& seg_keys) {
     if (n_dec <= 8 || window != 0 || sink || softcap > 0.f) return 0;
     int segments = max_position / 512 + 1;
     seg_keys = 512;
     if (n_dec > 16) {
         const long blocks = (long)Hkv * n_dec;
-        const int want = max_position < 1536 ? 1 : (int)min(768 / blocks, (long)segments);
-        seg_keys = qe_cdiv(qe_cdiv(max_position + 1, max(1, want)), 16) * 16;
+        const int last = max_position < 512 ? 511 : max_position | 1023;
+        const int want = last < 1536 ? 1 : (int)min(768 / blocks, last / 512 + 1L);
+        seg_keys = qe_cdiv(qe_cdiv(last + 1, max(1, want)), 16) * 16;
         segments = max_position / seg_keys + 1;
     }
     return segments;

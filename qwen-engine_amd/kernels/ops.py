@@ -892,7 +892,8 @@ def attention(q: torch.Tensor, cache: torch.Tensor, positions: torch.Tensor, tok
     other requests read too.  A hint for the decode kernel's loads; results do not depend on it.
 
     dec_blocks: more than eight dec_tokens may have a block each that walks a token's keys (quicker; a row's sums then have another
-    order than alone, where every 128 keys are summed by themselves).
+    order than alone, where every 128 keys are summed by themselves; with more than sixteen it follows their number and the stretch of
+    1024 positions that max_dec_position lies in, the first two stretches being of 512).
 
     other_requests: to how many requests other_tokens belong, or 0.  A hint for the float32 kernel; results do not depend on it."""
     lib = load_library()

@@ -99,6 +99,19 @@ def test_bits_of_nine_to_sixteen_tokens(ops):
     assert torch.equal(run(back, 1535), every[back])
 
 
+@pytest.mark.parametrize("n,longest,ends", [(24, 300, (511,)), (24, 700, (1023,)), (40, 1100, (1535, 2047)), (17, 1700, (2047,)), (33, 2100, (2200, 3071))])
+def test_bits_of_a_step_as_it_comes_and_recorded(ops, n, longest, ends):
+    """More than sixteen tokens: a recorded step knows the end of the stretch that the last position lies in, another the position."""
+    hq, hkv, D, P = 16, 8, 128, 16
+    pos = [longest] + [(97 * i) % longest for i in range(1, n)]
+    cache, table, _, _ = _requests(pos, hkv, D, P)
+    q, i32 = rand(n, hq, D, seed=1).bfloat16().to(DEV), lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    run = lambda most: ops.attention(q, cache, i32(pos), i32(range(n)), table, 0.1, dec_tokens=i32(range(n)), max_dec_position=most, dec_blocks=True)
+    want = run(longest)
+    for end in ends:
+        assert torch.equal(run(end), want), end
+
+
 @pytest.mark.parametrize("hq,hkv,rows", [(8, 4, 1), (8, 4, 70), (8, 1, 200), (6, 2, 33)])
 @pytest.mark.parametrize("singles", [1, 15, 40])
 def test_single_tokens_beside_a_portion_in_one_launch(ops, hq, hkv, rows, singles):
