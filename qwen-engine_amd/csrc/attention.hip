@@ -62,11 +62,13 @@ extern "C" int qe_attention_prefill_tiles_run(const int* portions, int n_portion
 // the rows of portions (whose rows see at most max_keys keys), instead of by the decode kernel and then the portions by themselves: a launch or two are
 // saved, and the tokens' walks pass beside the portions'.  (us, 16 heads of 128 on 8, a portion of 400 rows from the start; apart, tokens a block each from nine on,
 // and in one: one token of 400 keys 25.2, 16.7, of 1000 25.9, 22.4, of 2000 26.0, 35.8; 15 of 400 28, 17.6, of 1000 35, 25.4, of 2000 48, 39.5; 64 of 400
-// 40, 34.8, of 1000 71, 61.9.  A portion of 64 rows: one of 1000 20.0, 22.1, eight 24.1, 23.1.)  Not where the walks are cut into segments: more
-// blocks would leave fewer of those.
+// 40, 34.8, of 1000 71, 61.9.  A portion of 64 rows: one of 1000 20.0, 22.1, eight 24.1, 23.1.  200 rows: one of 870 20.8, 14.6; tokens of 160 to 480 or 330 to
+// 990 keys: 96 42.7, 36.5 and 66.7, 59.9, 128 52.9, 42.7 and 87.5, 73.0, 256 81.9, 73.5 and 144, 129.)  Not where the walks are cut into segments: more
+// blocks would leave fewer of those.  The lines are where a recorded step, which has its portion filled up to 128 rows and the positions to 512 or 1024,
+// falls on the same side as the step as it comes.
 extern "C" int qe_attention_prefill_takes_single(int n_dec, int max_position, int rows, int max_keys) {
     if (n_dec <= 0 || rows <= 0 || max_keys > qe_attention_prefill_uncut_keys()) return 0;
-    return max_position < 512 || (max_position < 1024 && (rows >= 256 || n_dec >= 8));
+    return max_position < 512 || (max_position < 1024 && (rows > 128 || n_dec >= 8));
 }
 
 // rows of a tile for these head counts

@@ -141,6 +141,20 @@ def test_single_tokens_beside_a_portion_in_one_launch(ops, hq, hkv, rows, single
         assert torch.equal(together[0][singles:], apart[singles:])
 
 
+def test_recorded_steps_choose_as_steps_that_run_as_they_come(ops):
+    """Single tokens beside a portion: in one launch or two does not hang on what a recorded step fills up."""
+    from qwen_engine_amd.engine import ModelRunner
+    from qwen_engine_amd.parts.attention import PagedAttention
+    step = ModelRunner.MIXED_GRAPH_STEP
+    for n in (1, 2, 7, 8, 9, 15, 33, 70):
+        for last in (0, 300, 511, 512, 700, 1023, 1024, 1500):
+            end = PagedAttention.graph_key(last) * ops.DECODE_SPLIT_KEYS - 1
+            for rows in (2, 100, 127, 128, 129, 200, 255, 256, 257, 500):
+                for keys in (rows, 1024, 1025, 3000):
+                    comes = ops.prefill_takes_single(n, last, rows, keys)
+                    assert comes == ops.prefill_takes_single(ModelRunner.graph_rows(n), end, -(-rows // step) * step, keys), (n, last, rows, keys)
+
+
 @pytest.mark.parametrize("T,H,n", [(1, 8, 2), (3, 100, 300), (9, 1024, 1), (2, 1030, 700)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_embedding_with_a_block_tables_updates(ops, T, H, n, dtype):
