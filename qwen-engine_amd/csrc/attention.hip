@@ -23,7 +23,7 @@ int qe_attention_prefill(const void* q, void* out, const void* cache, const int*
                          const int* positions, const int* tok_seq, const int* block_table, int max_blocks,
                          int Hq, int Hkv, int D, int P, float scale, int window, int groups,
                          int seg_keys, int max_keys, int keys_row, void* workspace, size_t workspace_bytes,
-                         hipStream_t stream, int keep_first, int sink, float softcap, const AttnTail& tail);
+                         hipStream_t stream, int keep_first, int sink, float softcap, int singles, const AttnTail& tail);
 static AttnTail make_tail(int Hq, int D, const void* out, long out_stride, int dv, const float* sink_heads, const void* gate,
                           long gate_stride, int dt_g) {
     AttnTail t{};
@@ -121,12 +121,13 @@ extern "C" long qe_attention_prefill_workspace_bytes_for(int num_tiles, int Hq, 
 // sees more than max_keys keys and the workspace has qe_attention_prefill_workspace_bytes bytes.  Or
 // minus a number of segments (2 to 8): the kernels take the keys that row keys_row of q sees (no row
 // sees more) from its position and cut them into that many segments, or fewer, themselves; the
-// workspace then has qe_attention_prefill_workspace_bytes_for that number.
+// workspace then has qe_attention_prefill_workspace_bytes_for that number.  singles: the first so many groups of four tiles
+// are single new tokens, whose weights are taken against the exact largest score (not with a soft cap).
 extern "C" int qe_attention_prefill_run(const void* q, void* out, const void* cache, const int* tiles,
                                         int num_tiles, const int* positions, const int* tok_seq,
                                         const int* block_table, int max_blocks, int Hq, int Hkv, int D, int P,
                                         float scale, int window, int keep_first, int sink, float softcap, int groups, int seg_keys,
-                                        int max_keys, int keys_row, void* workspace, long workspace_bytes,
+                                        int max_keys, int keys_row, int singles, void* workspace, long workspace_bytes,
                                         long out_stride, int dv, const float* sink_heads, const void* gate,
                                         long gate_stride, int dt_g, hipStream_t stream) {
     QE_TAIL_CHECK();
@@ -134,7 +135,7 @@ extern "C" int qe_attention_prefill_run(const void* q, void* out, const void* ca
                workspace_bytes >= 0, "prefill attention: bad sizes");
     return qe_attention_prefill(q, out, cache, tiles, num_tiles, positions, tok_seq, block_table, max_blocks,
                                 Hq, Hkv, D, P, scale, window, groups, seg_keys, max_keys, keys_row, workspace,
-                                (size_t)workspace_bytes, stream, keep_first, sink, softcap,
+                                (size_t)workspace_bytes, stream, keep_first, sink, softcap, singles,
                                 make_tail(Hq, D, out, out_stride, dv, sink_heads, gate, gate_stride, dt_g));
 }
 

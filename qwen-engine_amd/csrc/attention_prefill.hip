@@ -137,13 +137,14 @@ __device__ __forceinline__ void store_columns(bf16_t* __restrict__ out, const fl
 // DIRECT: the cache begins at a whole 16-byte piece, which loads that write to shared memory themselves want.  Tiles of a cache that lies
 // elsewhere come through registers, asked for a round before they are stored to their place; the same bits (8192 tokens of 32 heads of 128 on 8
 // 546 us and 609, 2048 of 16 heads 45 and 58, 512 rows behind 7680 keys 50 and 61).
-template <int D, int NG, bool CAP, bool DIRECT>
+// SINGLES: the first groups are single new tokens (its own form: the comparison with a number of the group's own instead of 8 cost prompts 0.6 %).
+template <int D, int NG, bool CAP, bool DIRECT, bool SINGLES>
 __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_kernel(
     const bf16_t* __restrict__ q, bf16_t* __restrict__ out, const bf16_t* __restrict__ cache,
     const int* __restrict__ tiles, const int* __restrict__ positions, const int* __restrict__ tok_seq,
     const int* __restrict__ block_table, int max_blocks,
     int Hq, int Hkv, int P, int log2P, float scale_log2, int window, int R, int seg_param, int keys_row,
-    float* __restrict__ part, int keep_first, int sink, float cap_in, float cap_out, AttnTail tail) {
+    float* __restrict__ part, int keep_first, int sink, float cap_in, float cap_out, int singles, AttnTail tail) {
     constexpr int KROW = D * 2, KBYTES = 32 * KROW, BUF = 2 * KBYTES;    // bytes of a key row, of a tile's keys, of a tile
     constexpr int LP = D / 64;                       // loads of a wave for a tile's keys, and for its values
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_all[];      // NG rings of RING tiles
@@ -167,6 +168,7 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
     const int* bt4 = tiles + 8 * (gridDim.z - 1 - bgroup);   // later rows see more keys: they start first
     if (bt4[1] <= 0) return;                               // a group without rows (a list filled up to a fixed length)
     const int row_first = bt4[0];
+    const float slack = SINGLES && (int)(gridDim.z - 1 - bgroup) < singles ? 0.f : 8.f;
     int last = 0;
 #pragma unroll
     for (int j = 1; j < 4; ++j) if (bt4[2 * j + 1] > 0) last = j;
@@ -407,8 +409,9 @@ __global__ __launch_bounds__(256 * NG, NG == 1 ? 2 : 1) void attention_prefill_k
             // m is the reference the weights are taken against, not the exact maximum: a column moves
             // it only when a score exceeds it by more than 8 (a weight above 2^8), which after the
             // first tiles is rare, so that the accumulators are seldom rescaled.  The decision is the
-            // column's own: its sums do not depend on the other columns of the wave.
-            const bool moves = tmax > m + 8.f;                 // (never for a tile without a visible key)
+            // column's own: its sums do not depend on the other columns of the wave.  (A single new token's is the exact maximum,
+            // as in the decode kernel: its largest weight is then 1 and not rounded, without which it errs by a tenth to a third more.)
+            const bool moves = tmax > m + slack;               // (never for a tile without a visible key)
             if (__any(moves)) {
                 const float alpha = moves ? __builtin_amdgcn_exp2f(m - tmax) : 1.f;   // 0 from a column's first keys
                 m = moves ? tmax : m;
@@ -712,14 +715,15 @@ size_t qe_attention_prefill_workspace(int num_tiles, int Hq, int Hkv, int D, int
 // seg_keys: 0; or the keys of a segment (a multiple of 64) with max_keys, the most keys a row sees; or,
 // for a caller that does not know the positions, minus the number of segments (at most 8) into which
 // the keys of row keys_row, which sees the most, are to be cut.  The workspace has
-// qe_attention_prefill_workspace(..., segments) bytes.
+// qe_attention_prefill_workspace(..., segments) bytes.  singles: the first so many groups are single new tokens.
 int qe_attention_prefill(const void* q, void* out, const void* cache, const int* tiles, int num_tiles,
                          const int* positions, const int* tok_seq, const int* block_table, int max_blocks,
                          int Hq, int Hkv, int D, int P, float scale, int window, int groups,
                          int seg_keys, int max_keys, int keys_row, void* workspace, size_t workspace_bytes,
-                         hipStream_t stream, int keep_first, int sink, float softcap, const AttnTail& tail) {
+                         hipStream_t stream, int keep_first, int sink, float softcap, int singles, const AttnTail& tail) {
     QE_REQUIRE(seg_keys == 0 || (keep_first == 0 && !sink),
                "prefill attention: kept first keys and a sink go with uncut walks only");
+    QE_REQUIRE(singles >= 0 && (singles == 0 || softcap == 0.f), "prefill attention: %d single tokens, which go without a soft cap", singles);
     QE_REQUIRE((D == 64 || D == 128) && P >= 16 && (P & (P - 1)) == 0 && Hq % Hkv == 0,
                "prefill attention: sizes not taken");
     int log2P = 0;
@@ -752,17 +756,17 @@ int qe_attention_prefill(const void* q, void* out, const void* cache, const int*
     QE_REQUIRE(groups == 1 || groups == 2, "prefill attention: %d groups a block", groups);
     // (a cache may begin at any element of a larger buffer)
     const bool direct = ((unsigned long)cache & 15) == 0;
-#define QE_PREFILL_FORM(D_, NG_, CAP_, DIRECT_)                                                               \
+#define QE_PREFILL_FORM(D_, NG_, CAP_, DIRECT_, SINGLES_)                                                     \
     {                                                                                               \
         constexpr int shmem_ = NG_ * RING * 2 * 32 * D_ * 2;                                       \
-        QE_RAISE_SHARED((attention_prefill_kernel<D_, NG_, CAP_, DIRECT_>), shmem_);                \
-        attention_prefill_kernel<D_, NG_, CAP_, DIRECT_><<<grid, 256 * NG_, shmem_, stream>>>(               \
+        QE_RAISE_SHARED((attention_prefill_kernel<D_, NG_, CAP_, DIRECT_, SINGLES_>), shmem_);      \
+        attention_prefill_kernel<D_, NG_, CAP_, DIRECT_, SINGLES_><<<grid, 256 * NG_, shmem_, stream>>>(      \
         (const bf16_t*)q, (bf16_t*)out, (const bf16_t*)cache, tiles, positions, tok_seq, block_table, \
         max_blocks, Hq, Hkv, P, log2P, scale_log2, window, R, seg_keys, keys_row, (float*)workspace, keep_first, sink, \
-        cap_in, cap_out, tail);                                                                     \
+        cap_in, cap_out, singles, tail);                                                            \
     }
-#define QE_PREFILL_CAP(D_, NG_, CAP_) { if (direct) QE_PREFILL_FORM(D_, NG_, CAP_, true) else QE_PREFILL_FORM(D_, NG_, CAP_, false) }
-#define QE_PREFILL(D_, NG_) do { if (softcap > 0.f) QE_PREFILL_CAP(D_, NG_, true) else QE_PREFILL_CAP(D_, NG_, false) } while (0)
+#define QE_PREFILL_CAP(D_, NG_, CAP_, S_) { if (direct) QE_PREFILL_FORM(D_, NG_, CAP_, true, S_) else QE_PREFILL_FORM(D_, NG_, CAP_, false, S_) }
+#define QE_PREFILL(D_, NG_) do { if (softcap > 0.f) QE_PREFILL_CAP(D_, NG_, true, false) else if (singles) QE_PREFILL_CAP(D_, NG_, false, true) else QE_PREFILL_CAP(D_, NG_, false, false) } while (0)
     if (D == 128) { if (groups == 2) QE_PREFILL(128, 2); else QE_PREFILL(128, 1); }
     else          { if (groups == 2) QE_PREFILL(64, 2); else QE_PREFILL(64, 1); }
 #undef QE_PREFILL

@@ -63,7 +63,7 @@ def load_library():
         "qe_attention_prefill_supported": [i32, i32, i32, i32, i32],
         "qe_attention_prefill_rows": [i32, i32],
         "qe_attention_prefill_run": [vp, vp, vp, vp, i32, vp, vp, vp, i32, i32, i32, i32, i32, f32, i32, i32, i32, f32, i32, i32, i32,
-                                     i32, vp, i64, i64, i32, vp, vp, i64, i32, vp],
+                                     i32, i32, vp, i64, i64, i32, vp, vp, i64, i32, vp],
         "qe_attention_f32_fused_supported": [i32, i32, i32, i32, i32],
         "qe_attention_f32_fused_run": [vp, vp, vp, vp, i32, i32, vp, vp, vp, i32, vp, vp, vp, f32, vp, i32, i32, i32, i32, f32, i32, vp],
         "qe_attention_prefill_plan_segments": [i32, i32, i32],
@@ -859,7 +859,8 @@ def attention(q: torch.Tensor, cache: torch.Tensor, positions: torch.Tensor, tok
               max_other_keys: int = 0, prefill_segment_keys: int = -1,
               other_keys_row: Optional[int] = None, shared_keys: Optional[torch.Tensor] = None,
               keep_first: int = 0, sink=False, chunk: int = 0, softcap: float = 0.0, v_dim: int = 0,
-              gate: Optional[torch.Tensor] = None, dec_blocks: bool = False, other_requests: int = 0) -> torch.Tensor:
+              gate: Optional[torch.Tensor] = None, dec_blocks: bool = False, other_requests: int = 0,
+              prefill_singles: int = 0) -> torch.Tensor:
     """q [T, Hq, D]; cache [pages, 2, Hkv, P, D] (key tiles [P][D], value tiles transposed [D][P]);
     positions, tok_seq int32 [T]; block_table int32 [B, max_blocks].  Token t sees the keys at
     positions max(0, p - window + 1) .. p of request tok_seq[t] (window 0: all).  The caller
@@ -895,7 +896,11 @@ def attention(q: torch.Tensor, cache: torch.Tensor, positions: torch.Tensor, tok
     order than alone, where every 128 keys are summed by themselves; with more than sixteen it follows their number and the stretch of
     1024 positions that max_dec_position lies in, the first two stretches being of 512).
 
-    other_requests: to how many requests other_tokens belong, or 0.  A hint for the float32 kernel; results do not depend on it."""
+    other_requests: to how many requests other_tokens belong, or 0.  A hint for the float32 kernel; results do not depend on it.
+
+    prefill_singles: the first so many groups of other_tiles are single new tokens; their weights are taken against the exact largest
+    score, as the decode kernel takes them (a portion's rows against one that may lag by 2^8: their largest weight is rounded too); not with
+    a soft cap."""
     lib = load_library()
     _need(q, "q", _ACT, (None, None, None))
     T, Hq, D = q.shape
@@ -1001,7 +1006,7 @@ def attention(q: torch.Tensor, cache: torch.Tensor, positions: torch.Tensor, tok
                                                 other_tiles.data_ptr(), n_tiles,
                                                 positions.data_ptr(), tok_seq.data_ptr(), block_table.data_ptr(),
                                                 max_blocks, Hq, Hkv, D, P, float(scale), int(window), keep_first, sink, softcap,
-                                                int(prefill_groups), seg, max_keys, keys_row, _ptr(ws), nbytes,
+                                                int(prefill_groups), seg, max_keys, keys_row, int(prefill_singles), _ptr(ws), nbytes,
                                                 *tail, _stream()),
                    "attention (prefill)")
         else:

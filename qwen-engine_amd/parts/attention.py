@@ -296,7 +296,7 @@ class PagedAttention:
         together = self._all_tiles(ctx, ex, q, cache)
         if together is not None:
             o = ops.attention(q, cache, ctx.positions, ctx.tok_seq, ctx.block_tables[g], self.scale, self.window,
-                              other_tokens=together[0], other_tiles=together[1])
+                              other_tokens=together[0], other_tiles=together[1], prefill_singles=ex["dec_tokens"].shape[0])
         else:
             o = ops.attention(q, cache, ctx.positions, ctx.tok_seq, ctx.block_tables[g], self.scale, self.window,
                               dec_tokens=ex["dec_tokens"], max_dec_position=ex["max_dec_position"],

@@ -141,6 +141,35 @@ def test_single_tokens_beside_a_portion_in_one_launch(ops, hq, hkv, rows, single
         assert torch.equal(together[0][singles:], apart[singles:])
 
 
+@pytest.mark.parametrize("wide", [1.0, 4.0])
+@pytest.mark.parametrize("singles,keys", [(15, 300), (40, 600)])
+def test_single_tokens_beside_a_portion_err_as_by_themselves(ops, singles, keys, wide):
+    """Against 64 bits, in the mean of six inputs, hardly more than what the decode kernel gives.  An error is the weights' rounding, but for each walk's
+    largest, which is 1: the decode kernel has a walk for every 128 keys.  Of 128 keys with scores of spread 1 the largest weight's square, about e^(2 * 2.5),
+    is a sixth of the squares' sum, 128 e^2: one exact weight in 600 keys instead of five errs by a twelfth at the most more."""
+    from qwen_engine_amd.parts.attention import prefill_tiles
+    hq, hkv, D, P, rows = 16, 8, 128, 16, 20
+    R, i32 = ops.prefill_tile_rows(hq, hkv), lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    apart = together = 0.0
+    for seed in range(6):
+        pos = [(keys // 2 + (i + seed) * 37) % keys for i in range(singles)]
+        cache, table, ks, vs = _requests(pos + [rows - 1], hkv, D, P)
+        T, scale = singles + rows, wide * D ** -0.5
+        q = rand(T, hq, D, seed=seed).bfloat16()
+        positions, seq = i32(pos + list(range(rows))), i32(list(range(singles)) + [singles] * rows)
+        flat = prefill_tiles([(i, 1) for i in range(singles)] + [(singles, rows)], R)
+        one = ops.attention(q.to(DEV), cache, positions, seq, table, scale, other_tokens=i32(range(T)), other_tiles=i32(flat).view(-1, 2),
+                            prefill_singles=singles)
+        two = ops.attention(q.to(DEV), cache, positions, seq, table, scale, dec_tokens=i32(range(singles)), max_dec_position=max(pos))
+        for i in range(singles):
+            k, v = ks[i].double(), vs[i].double()
+            w = torch.softmax(torch.stack([k[:, h * hkv // hq] @ q[i, h].double() for h in range(hq)]) * scale, -1)
+            want = torch.stack([w[h] @ v[:, h * hkv // hq] for h in range(hq)])
+            together += float((one[i].cpu().double() - want).norm() / want.norm())
+            apart += float((two[i].cpu().double() - want).norm() / want.norm())
+    assert together <= 13 / 12 * apart
+
+
 def test_recorded_steps_choose_as_steps_that_run_as_they_come(ops):
     """Single tokens beside a portion: in one launch or two does not hang on what a recorded step fills up."""
     from qwen_engine_amd.engine import ModelRunner
