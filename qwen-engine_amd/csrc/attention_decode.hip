@@ -802,18 +802,31 @@ size_t qe_attention_decode_workspace(int n_dec, int Hq, int D, int num_splits) {
 // tokens are the splits'.)  Up to 16 tokens, which every other kernel of their step takes in one order, a token's segments follow its own position
 // alone: its bits are the same beside any others.  With more they follow how many those are, and the last position as recorded steps know it, the end
 // of a stretch of 1024 (the first two, of 512): a step has the same ones whether it is recorded or runs as it comes.
+static int last_of_stretch(int position) { return position < 512 ? 511 : position | 1023; }
 static int block_segments(int n_dec, int Hkv, int max_position, int window, int sink, float softcap, int& seg_keys) {
     if (n_dec <= 8 || window != 0 || sink || softcap > 0.f) return 0;
     int segments = max_position / 512 + 1;
     seg_keys = 512;
     if (n_dec > 16) {
         const long blocks = (long)Hkv * n_dec;
-        const int last = max_position < 512 ? 511 : max_position | 1023;
+        const int last = last_of_stretch(max_position);
         const int want = last < 1536 ? 1 : (int)min(768 / blocks, last / 512 + 1L);
         seg_keys = qe_cdiv(qe_cdiv(last + 1, max(1, want)), 16) * 16;
         segments = max_position / seg_keys + 1;
     }
     return segments;
+}
+
+// 1 if n single tokens without a window are best given norm, rotation and cache write inside the attention kernel: up to 16, and up to 64 but where their segments
+// are about three blocks a unit, which is how many of the other form's share one; of the fused form's two do, and the third is a turn by itself.  (The two kernels' time and the
+// one's, 16 heads of 128 on 8: 24 tokens of 600 keys 24.4, 19.8 us, 32 27.1, 23.1, 64 41.2, 38.8; of 1000 to 4000 keys, in the mean of one to three times the keys: 17 and 28 tokens
+// 0.86 to 0.95, 32 0.92 to 1.00, 36 0.85 to 0.93, 40 0.95 to 1.01, 52 to 64 0.95 to 0.97; in four segments 20 tokens 0.95 to 1.05, 24 1.01 to 1.04; in two 44 1.01 to 1.04, 48 1.02 to 1.06.)
+extern "C" int qe_attention_decode_fused_preferred(int n, int Hkv, int max_position) {
+    if (n <= 16 || n > 64) return n <= 16;
+    int seg_keys;
+    const int segments = block_segments(n, Hkv, last_of_stretch(max_position), 0, 0, 0.f, seg_keys);
+    const long blocks = (long)segments * Hkv * n;
+    return !((segments == 4 && blocks >= 640) || (segments == 2 && blocks > 640));
 }
 
 template <int D, bool FUSED>

@@ -76,6 +76,7 @@ def load_library():
         "qe_attention_prefill_workspace_bytes": [i32, i32, i32, i32, i32, i32],
         "qe_attention_decode_run": [vp, vp, vp, vp, i32, vp, vp, vp, i32, vp, i32, i32, i32, i32, f32, i32, i32, i32, f32, i32, i32, vp, i64,
                                     i64, i32, vp, vp, i64, i32, vp],
+        "qe_attention_decode_fused_preferred": [i32, i32, i32],
         "qe_attention_decode_fused_run": [vp, vp, vp, vp, i32, vp, vp, vp, i32, vp, vp, vp, vp, f32, vp,
                                           i32, i32, i32, i32, f32, i32, i32, i32, vp, i64, vp],
         "qe_qk_rope_store": [vp, vp, vp, vp, f32, vp, i32, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, vp],
@@ -1026,6 +1027,14 @@ def attention_decode_fused_supported(qkv: torch.Tensor, cache: torch.Tensor, num
         return cache.shape[0] > 0 and bool(lib.qe_attention_f32_fused_supported(qkv.shape[0], num_heads, cache.shape[2], D, cache.shape[3]))
     return (qkv.dtype == torch.bfloat16 and
             bool(lib.qe_attention_decode_supported(num_heads, cache.shape[2], D, cache.shape[3], _DT[qkv.dtype])))
+
+
+def attention_decode_fused_preferred(qkv: torch.Tensor, num_kv_heads: int, max_dec_position: int) -> bool:
+    """True if the rows of qkv, all single new tokens without a window, are best given to attention_decode_fused (with dec_blocks) where it takes
+    them, rather than to qk_rope_store and attention."""
+    if qkv.dtype == torch.float32:
+        return qkv.shape[0] <= 64
+    return bool(load_library().qe_attention_decode_fused_preferred(qkv.shape[0], int(num_kv_heads), int(max_dec_position)))
 
 
 def attention_decode_fused(qkv: torch.Tensor, num_heads: int, cache: torch.Tensor, positions: torch.Tensor,

@@ -21,12 +21,9 @@ from .registry import build_part, register_part
 
 # Up to this many single new tokens in a step, the decode attention kernel norms, rotates and
 # writes the cache itself; above, the separate kernel is quicker (every wave of the attention
-# kernel repeats the preparation of q, which then outweighs the kernel saved).  With a window a token's
-# keys go in splits of a wave each, else four waves walk them (16 heads, the two kernels and the one: 32 tokens of 400 keys
-# 19.9 us and 17.7, of 4000 122 and 118; 64 of 400 32.7 and 29.9, of 2000 115 and 111; slower from 24 of 1000 keys, 38.1 and 39.1, to 48 of 2000,
-# 94.6 and 100.4).
+# kernel repeats the preparation of q, which then outweighs the kernel saved).  So with a window, where a token's
+# keys go in splits of a wave each; else four waves walk them, and the kernel library knows up to where one kernel is quicker.
 FUSED_DECODE_MAX_TOKENS = 16
-FUSED_DECODE_MAX_TOKENS_UNWINDOWED = 64
 
 
 def prefill_tiles(portions, rows_per_tile: int) -> List[int]:
@@ -270,7 +267,9 @@ class PagedAttention:
             ex = self._extras(ctx)
             only_new_tokens = (ex["dec_tokens"] is not None and ex["dec_tokens"].shape[0] == T and
                                (ex["other_tokens"] is None or ex["other_tokens"].shape[0] == 0))
-            if (only_new_tokens and T <= (FUSED_DECODE_MAX_TOKENS if self.window else FUSED_DECODE_MAX_TOKENS_UNWINDOWED) and binding.write and
+            if (only_new_tokens and binding.write and
+                    (T <= FUSED_DECODE_MAX_TOKENS if self.window else
+                     ops.attention_decode_fused_preferred(qkv, self.hkv, ex["max_dec_position"])) and
                     not is_replaced(self, _ATTEND) and ops.attention_decode_fused_supported(qkv, cache, self.hq, table)):
                 # every row is the one new token of its request: norm, rotation and cache write
                 # happen inside the attention kernel (an _attend that has been replaced gets q)

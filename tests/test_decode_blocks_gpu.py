@@ -184,6 +184,22 @@ def test_recorded_steps_choose_as_steps_that_run_as_they_come(ops):
                     assert comes == ops.prefill_takes_single(ModelRunner.graph_rows(n), end, -(-rows // step) * step, keys), (n, last, rows, keys)
 
 
+def test_where_the_step_before_goes_inside(ops):
+    """Up to 16 tokens always, up to 64 but where that was slower, the same for every position of a stretch that recorded steps have in one; up to 64
+    rows of 32 bits."""
+    asked = lambda n, last, dtype=torch.bfloat16: ops.attention_decode_fused_preferred(torch.empty(n, 8, dtype=dtype, device=DEV), 8, last)
+    for last in (0, 511, 512, 1023, 1024, 2500, 9000):
+        assert asked(1, last) and asked(16, last) and not asked(65, last)
+        assert asked(24, last, torch.float32) and not asked(65, last, torch.float32)
+        for n in (17, 28, 32, 36, 40, 56, 64):
+            assert asked(n, last), (n, last)
+        for n in (20, 24, 44, 48):
+            assert asked(n, last) == (last < 1024), (n, last)
+    for n in range(17, 65):
+        for last in (512, 600, 1024, 1500, 1600, 2047, 2048, 2600):
+            assert asked(n, last) == asked(n, last | 1023), (n, last)
+
+
 @pytest.mark.parametrize("T,H,n", [(1, 8, 2), (3, 100, 300), (9, 1024, 1), (2, 1030, 700)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_embedding_with_a_block_tables_updates(ops, T, H, n, dtype):

@@ -61,7 +61,8 @@ def test_a_replaced_attend_is_called(monkeypatch, how):
     """Steps of single tokens whose norm, rotation and cache write are inside the attention kernel have no q to hand on: they go one by one."""
     one, q = [], torch.ones(2, 4, 16)
     fake = SimpleNamespace(gemm=lambda x, w, b=None, **kw: x, gemm_qkv_supported=lambda *a: False, gemm_partial_preferred=lambda *a: False,
-                           gemm_branch_splits=lambda *a: 0, attention_decode_fused_supported=lambda *a: True, qk_rope_store=lambda *a: q,
+                           gemm_branch_splits=lambda *a: 0, attention_decode_fused_supported=lambda *a: True,
+                           attention_decode_fused_preferred=lambda *a: True, qk_rope_store=lambda *a: q,
                            attention_decode_fused=lambda *a, **kw: one.append(a) or q)
     monkeypatch.setattr(attention, "ops", fake)
     part = PagedAttention(SimpleNamespace(num_heads=4, num_kv_heads=2, head_dim=16, scale=0.25, window=None, qk_norm_eps=None, position=None), 64)
