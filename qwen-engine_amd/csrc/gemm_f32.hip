@@ -582,10 +582,12 @@ int qe_gemm_f32(const float* x, const float* w, const float* bias, float* out, i
         if (M <= 16 && by_lines(M, N, K) && (((unsigned long)w) & 15) == 0)
             gemm_f32_lines_kernel<<<qe_cdiv(N, 16), 64 * qe_cdiv(K, 16 * FK), 0, stream>>>(x, w, bias, out, M, N, K);
         // (two rows, us with 4, 8 and 16 columns a block: 1024 x 2048 5.5, 5.8, 6.5; 2048 x 1024 5.5, 4.5, 4.9; 4096 x 1024 9.6, 6.2, 6.1; 12288 x 1024
-        // 24.9, 15.1, 12.1; 8192 x 3072, 8 columns, 29.5, and 25.2 by rows)
+        // 24.9, 15.1, 12.1; 8192 x 3072, 8 columns, 29.5, and 25.2 by rows.  By rows and with 16 columns, beyond 12288 rows: 24576 x 512 14.7, 10.6, 151936 x 512
+        // 71.0, 46.7, 16383 x 1024 18.5, 14.8, 24576 x 2048 41.6, 40.9, 151936 x 2048 238, 235, eight rows 326, 261; but one row 24576 x 2048 39.9, 40.6, 151936 x 2048
+        // 225, 230: one block of 128 KB a unit, nothing beside it)
         else if (M <= 16 && N <= 1024 && by_chunks(w, K)) return launch_chunks<4>(x, w, bias, out, M, N, K, stream);
         else if (M <= 16 && N <= 2048 && by_chunks(w, K)) return launch_chunks<8>(x, w, bias, out, M, N, K, stream);
-        else if (M <= 16 && by_chunks(w, K) && chunk_len(K) <= 128) return launch_chunks<16>(x, w, bias, out, M, N, K, stream);
+        else if (M <= 16 && by_chunks(w, K) && chunk_len(K) <= 128 && (M > 1 || chunk_len(K) == 64 || N <= 16384)) return launch_chunks<16>(x, w, bias, out, M, N, K, stream);
         else if (M > 4 && M <= 16 && N >= 6144) launch_rows<1, 2, 1>(x, w, bias, out, M, N, K, rows, stream);
         else if (M <= 16) launch_rows<1, 1, 2>(x, w, bias, out, M, N, K, rows, stream);
         else if (M <= 32) launch_rows<2, 1, 2>(x, w, bias, out, M, N, K, rows, stream);

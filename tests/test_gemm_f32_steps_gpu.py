@@ -101,6 +101,16 @@ def test_norm_in_front_of_gate_and_up_rows(ops, M, N, K):
         ops.gemm(h, w, out_dtype=torch.bfloat16, epilogue=ops.EPI_SILU_MUL, norm_weight=weight, norm_eps=1e-6)
 
 
+@pytest.mark.parametrize("N,K", [(16384, 2048), (16385, 2048), (20000, 1152), (20000, 512)])
+def test_few_rows_against_many(ops, N, K):
+    """One row goes by rows where two go by chunks: one order."""
+    g = torch.Generator().manual_seed(N + K)
+    x, w = torch.randn(17, K, generator=g).cuda(), torch.randn(N, K, generator=g).cuda()
+    want = ops.gemm(x, w)
+    for m in (1, 2, 16):
+        assert torch.equal(ops.gemm(x[:m], w), want[:m]), m
+
+
 def test_what_is_not_taken(ops):
     """More numbers than the norm has room for, rows of no whole steps: refused."""
     w = torch.zeros(64, 1024, device="cuda")
