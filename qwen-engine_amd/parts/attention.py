@@ -290,6 +290,8 @@ class PagedAttention:
                                   None, slots, cache, ctx.page_size)
         return self._attend(q, ctx, cache, g, T)
 
+    stream_forward = forward      # (as it is written)
+
     def _attend(self, q: torch.Tensor, ctx, cache: torch.Tensor, g: int, T: int) -> torch.Tensor:
         ex = self._extras(ctx)
         together = self._all_tiles(ctx, ex, q, cache)

@@ -8,7 +8,7 @@ from typing import Dict, Optional
 
 import torch
 
-from .base import (BranchSum, CacheBinding, DepthAverage, NormedBranch, Runtime, Stream, StreamInput, TensorInfo, add_pending, join_name,
+from .base import (BranchSum, CacheBinding, DepthAverage, NormedBranch, Runtime, Stream, StreamInput, TensorInfo, add_pending, is_replaced, join_name,
                    named_tensors, sub_tensors)
 from ..kernels import ops
 from .registry import build_part, part_class, register_part
@@ -92,9 +92,11 @@ class PreNormBlock:
     def _input(norm, part, stream: Stream, delta, ctx):
         """The part's input: the normed rows, or, with few rows (the model then gave the stream a second
         buffer) and where both the norm and the part can do it, the stream, what is to be added, and
-        the norm, for the part's first product."""
+        the norm, for the part's first product.  In the float32 mode, in which programs look into a model's parts, a
+        ``forward`` that has been replaced gets the normed rows."""
         if (getattr(part, "takes_stream", False) and hasattr(norm, "fusable_weight") and
-                stream.spare is not None):
+                stream.spare is not None and
+                not (ctx.rt.dtype == torch.float32 and hasattr(part, "stream_forward") and is_replaced(part, type(part).stream_forward))):
             fw = norm.fusable_weight()
             si = StreamInput(stream, delta, norm, fw[0], fw[1], ctx.rt) if fw is not None else None
             if si is not None and si.fusable():

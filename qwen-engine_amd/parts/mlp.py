@@ -79,6 +79,8 @@ class SwiGLU:
             return ops.gemm(a, self.w_down, self.b_down, epilogue=ops.EPI_PARTIAL, splits=splits)
         return ops.gemm(a, self.w_down, self.b_down)
 
+    stream_forward = forward      # (as it is written)
+
 
 _ACTIVATION = SwiGLU.activation
 

@@ -1,5 +1,6 @@
 """What a program has replaced is called: a norm, in the float32 mode, instead of norming inside the product behind it; a feed-forward's
-activation, and what an attention part does with q."""
+activation, what an attention part does with q.  A part's forward, in the float32 mode,
+gets the normed rows."""
 from types import SimpleNamespace
 
 import pytest
@@ -9,6 +10,7 @@ import qwen_engine_amd  # noqa: F401
 from qwen_engine_amd.parts.base import Stream, StreamInput
 from qwen_engine_amd.parts import attention, mlp
 from qwen_engine_amd.parts.attention import PagedAttention
+from qwen_engine_amd.parts.block import PreNormBlock
 from qwen_engine_amd.parts.mlp import SwiGLU
 from qwen_engine_amd.parts.norm import RMSNorm
 
@@ -80,3 +82,23 @@ def test_a_replaced_attend_is_called(monkeypatch, how):
         part.__class__ = type("Derived", (PagedAttention,), {"_attend": lambda self, *a: mine(*a)})
     part.forward(torch.zeros(2, 64), ctx, binding)
     assert len(one) == 1 and len(seen) == 1 and seen[0] is q
+
+
+@pytest.mark.parametrize("part", [SwiGLU, PagedAttention])
+@pytest.mark.parametrize("how", ["class", "part", "derived"])
+@pytest.mark.parametrize("delta", [None, torch.zeros(2, 8), torch.zeros(1, 2, 8)])
+def test_a_replaced_forward_gets_the_normed_rows(monkeypatch, part, how, delta):
+    rows, norm = torch.ones(2, 8), RMSNorm(SimpleNamespace(eps=1e-6), 8)
+    norm.forward = lambda h, rt, delta=None: rows
+    ctx, one = SimpleNamespace(rt=SimpleNamespace(dtype=torch.float32)), object.__new__(part)
+    given = lambda: PreNormBlock._input(norm, one, Stream(torch.zeros(2, 8), torch.zeros(2, 8)), delta, ctx)
+    assert isinstance(given(), StreamInput)
+    if how == "class":
+        monkeypatch.setattr(part, "forward", lambda self, *a: None)
+    elif how == "part":
+        one.forward = lambda *a: None
+    else:
+        one = object.__new__(type("Derived", (part,), {"forward": lambda self, *a: None}))
+    assert given() is rows
+    ctx.rt.dtype = torch.bfloat16                  # (there a part that says it takes the stream gets it, as it always did)
+    assert isinstance(given(), StreamInput) == (delta is None or delta.dim() == 3)
