@@ -137,11 +137,12 @@ class PagedAttention:
             if ex.get("portions") is not None:             # (a recorded step: the single tokens come first, see _other_tiles)
                 portions = ex["portions"]
                 groups = -(-ex["portion_rows"] // (4 * rows_per_tile)) + portions.shape[0]
-                ctx.memo[key] = ex["all_tokens"], ops.prefill_tiles_on_device(portions, rows_per_tile, groups, dec.shape[0])
+                tiles = ops.prefill_tiles_on_device(portions, rows_per_tile, groups, dec.shape[0])
             else:
                 flat = prefill_tiles([(s.q_start, s.q_len) for s in sorted(ctx.seqs, key=lambda s: s.q_len)], rows_per_tile)
-                ctx.memo[key] = (torch.arange(ctx.num_tokens, dtype=torch.int32, device=q.device),
-                                 torch.tensor(flat, dtype=torch.int32).view(-1, 2).to(q.device))
+                tiles = torch.tensor(flat, dtype=torch.int32).view(-1, 2).to(q.device)
+            rows = ex.get("all_tokens")                    # (a derived class's recorded steps need not bring them)
+            ctx.memo[key] = torch.arange(ctx.num_tokens, dtype=torch.int32, device=q.device) if rows is None else rows, tiles
         return ctx.memo[key]
 
     def _other_tiles(self, ctx) -> Optional[torch.Tensor]:

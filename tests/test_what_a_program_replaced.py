@@ -102,3 +102,17 @@ def test_a_replaced_forward_gets_the_normed_rows(monkeypatch, part, how, delta):
     assert given() is rows
     ctx.rt.dtype = torch.bfloat16                  # (there a part that says it takes the stream gets it, as it always did)
     assert isinstance(given(), StreamInput) == (delta is None or delta.dim() == 3)
+
+
+def test_recorded_steps_of_a_derived_class(monkeypatch):
+    """What a class prepares for its recorded mixed steps need not hold every row: single tokens beside a portion in one launch make the list then."""
+    fake = SimpleNamespace(attention_prefill_supported=lambda *a: True, prefill_uncut_keys=lambda: 1024, prefill_takes_single=lambda *a: True,
+                           prefill_tile_rows=lambda *a: 16, prefill_tiles_on_device=lambda *a: "tiles")
+    monkeypatch.setattr(attention, "ops", fake)
+    part, i32 = object.__new__(PagedAttention), lambda n: torch.arange(n, dtype=torch.int32)
+    part.hq = part.hkv = 4
+    ex = {"dec_tokens": i32(3), "other_tokens": i32(8) + 3, "max_dec_position": 511, "other_keys_row": None, "portions": torch.zeros(2, 2), "portion_rows": 8}
+    rows, tiles = part._all_tiles(SimpleNamespace(memo={}, num_tokens=11, seqs=[]), ex, torch.zeros(11, 4, 16), None)
+    assert tiles == "tiles" and torch.equal(rows, i32(11))
+    ex["all_tokens"] = i32(11)
+    assert part._all_tiles(SimpleNamespace(memo={}, num_tokens=11, seqs=[]), ex, torch.zeros(11, 4, 16), None)[0] is ex["all_tokens"]
