@@ -137,7 +137,7 @@ extern "C" int qe_gemm_branch_splits(int M, int N, int K, int dt_a, int dt_w) {
 //    taken by the kernel for few rows and by the tiled one.
 // 5: out = gelu(product) in bfloat16, no bias; where qe_gemm_gelu_supported.
 // norm_w (or null): the weight of an RMSNorm (eps norm_eps) that stands before the product: x is then the
-// 32-bit stream [M, K]; needs qe_gemm_norm_supported and epilogue 0, 2 or 4.  With it, delta (or null):
+// 32-bit stream [M, K]; needs qe_gemm_norm_supported and epilogue 0, 2 or 4 (32-bit weights: 0 or 4).  With it, delta (or null):
 // n_delta float tensors [M, K] one after the other that are added to the stream's rows, in order, before
 // the norm (the partial products of the branch before); the sums are written to h_out [M, K] (not x).
 // algo: 0 = choose, 1 = the generic 32-bit kernel, 2 = an MFMA kernel (the one for few rows up to
