@@ -90,6 +90,40 @@ def test_a_feed_forward_of_any_width(ops, width, hidden, rows, bias):
         assert x.fusable() and torch.equal(ffn.forward(x, None), want) and torch.equal(stream.h, want_h)
 
 
+@pytest.mark.parametrize("hidden,rows,heads,kv_heads", [(256, 1, 4, 2), (256, 16, 4, 4), (1024, 2, 16, 8), (1024, 8, 16, 2), (240, 3, 4, 2), (1024, 9, 16, 8)])
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("window", [None, 20])
+def test_an_attention_part_of_few_rows(ops, hidden, rows, heads, kv_heads, bias, window):
+    """Single tokens, an attention part from the stream with what is to be added to it, and from rows that the norm's own kernel made: the same output, cache
+    and stream, also where the norm has no room inside the product."""
+    from types import SimpleNamespace
+    from qwen_engine_amd.config import AttentionSpec, RMSNormSpec, RopeSpec
+    from qwen_engine_amd.parts import Runtime, build_part
+    from qwen_engine_amd.parts.base import Stream, StreamInput
+    D, P = 64, 16
+    g = torch.Generator().manual_seed(hidden + rows + heads)
+    rt = Runtime(torch.device("cuda:0"), torch.float32)
+    spec = AttentionSpec(heads, kv_heads, D, D ** -0.5, qkv_bias=bias, qk_norm_eps=1e-6, window=window, position=RopeSpec(10000.0, D, 128))
+    part, norm = build_part(spec, hidden), build_part(RMSNormSpec(eps=1e-6), hidden)
+    part.load({n: torch.randn(tuple(t.shape), generator=g) * hidden ** -0.5 for n, t in type(part).expected_tensors(spec, hidden).items()}, rt)
+    norm.load({"weight": 1 + 0.1 * torch.randn(hidden, generator=g)}, rt)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device="cuda")
+    pos = [(11 * i + 5) % 64 for i in range(rows)]
+    cache = torch.randn(4 * rows, 2, kv_heads, P, D, generator=g).cuda()
+    table = torch.arange(4 * rows, dtype=torch.int32, device="cuda").view(rows, 4)
+    ctx = SimpleNamespace(rt=rt, positions=i32(pos), tok_seq=i32(range(rows)), block_tables=[table], shared_keys=None, max_position=max(pos), page_size=P,
+                          slots=[i32([(4 * i + p // P) * P + p % P for i, p in enumerate(pos)])], memo={}, num_tokens=rows,
+                          extras={type(part): {"dec_tokens": i32(range(rows)), "other_tokens": None, "max_dec_position": max(pos)}})
+    bind = lambda kv: SimpleNamespace(kv=kv, group=0, write=True)
+    h, parts = torch.randn(rows, hidden, generator=g).cuda(), torch.randn(2, rows, hidden, generator=g).cuda()
+    for delta in (None, parts[0], parts[:1], parts):
+        stream, one, two = Stream(h.clone(), torch.full_like(h, float("nan"))), cache.clone(), cache.clone()
+        want = part.forward(norm.forward(want_h := h.clone(), rt, delta=delta), ctx, bind(two))
+        x = StreamInput(stream, delta, norm, *norm.fusable_weight(), rt)
+        assert x.fusable() and torch.equal(part.forward(x, ctx, bind(one)), want)
+        assert torch.equal(stream.h, want_h) and torch.equal(one, two)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 2000, 1024), (16, 1376, 256), (3, 34, 496)])
 def test_norm_in_front_of_gate_and_up_rows(ops, M, N, K):
     g = torch.Generator().manual_seed(M * K + N)
