@@ -51,6 +51,7 @@ def load_library():
         "qe_scatter_int": [vp, vp, vp, i32, i64, vp],
         "qe_silu_mul": [vp, vp, i32, i32, i32, i32, vp],
         "qe_gemm_silu_supported": [i32, i32, i32, i32, i32],
+        "qe_gemm_f32_silu_inside": [i32, i32, i32],
         "qe_gemm": [vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, i32, i32, i32, vp, f32, vp, i32, vp, vp],
         "qe_gemm_norm_supported": [i32, i32, i32, i32],
         "qe_gemm_norm_preferred": [i32, i32, i32, i32, i32],
@@ -569,6 +570,9 @@ def gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
         raise KernelError("gemm: 32-bit activations need 32-bit weights")
     if bias is not None:
         _need(bias, "bias", torch.float32, (w.shape[0],), x.device)
+    if (epilogue == EPI_SILU_MUL_IL and x.dtype == w.dtype == (out_dtype or x.dtype) == torch.float32 and gemm_silu_supported(x, w) and
+            not lib.qe_gemm_f32_silu_inside(M, w.shape[0], K)):        # (quicker by itself; the same bits)
+        return silu_mul(gemm(x, w, bias, algo=algo, norm_weight=norm_weight, norm_eps=norm_eps, delta=delta, stream_out=stream_out), out, interleaved=True)
     if epilogue == EPI_RESIDUAL:
         if out is None:
             raise KernelError("gemm: the residual epilogue needs the stream to add into")

@@ -43,7 +43,7 @@ def test_norm_in_front(ops, M, N, K):
             assert torch.equal(got, want)
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 64, 16), (16, 128, 80), (13, 6144, 1024), (2, 24576, 4096), (16, 16384, 1040)])
+@pytest.mark.parametrize("M,N,K", [(1, 64, 16), (16, 128, 80), (13, 6144, 1024), (2, 24576, 4096), (16, 16384, 1040), (8, 12288, 2560), (3, 2048, 4096), (2, 8256, 512)])
 def test_silu_behind(ops, M, N, K):
     g = torch.Generator().manual_seed(M + K + N)
     x, w, bias = torch.randn(M, K, generator=g).cuda(), (torch.randn(N, K, generator=g) * K ** -0.5).cuda(), torch.randn(N, generator=g).cuda()
@@ -122,6 +122,15 @@ def test_an_attention_part_of_few_rows(ops, hidden, rows, heads, kv_heads, bias,
         x = StreamInput(stream, delta, norm, *norm.fusable_weight(), rt)
         assert x.fusable() and torch.equal(part.forward(x, ctx, bind(one)), want)
         assert torch.equal(stream.h, want_h) and torch.equal(one, two)
+
+
+def test_silu_in_the_products_launch(ops):
+    """Only where that is not slower: two rows against 24576 x 4096 took 127 us in it, 78 apart."""
+    inside = ops.load_library().qe_gemm_f32_silu_inside
+    for taken in ((2, 6144, 1024), (16, 1024, 512), (2, 24576, 256), (2, 24576, 1536), (8, 24576, 4096), (8, 8192, 4096)):
+        assert inside(*taken), taken
+    for apart in ((2, 24576, 4096), (2, 2048, 4096), (16, 512, 2048), (8, 24576, 2048), (1, 12288, 1024), (2, 24576, 1024), (2, 6144, 4096), (17, 6144, 1024)):
+        assert not inside(*apart), apart
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 2000, 1024), (16, 1376, 256), (3, 34, 496)])
