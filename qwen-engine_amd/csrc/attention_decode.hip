@@ -607,15 +607,10 @@ __global__ __launch_bounds__(64 * W, W == 4 ? (FUSED ? 2 : 3) : 1) void attentio
     const long page_stride = 2L * Hkv * P * D;
     const int* bt = block_table + (long)row * max_blocks;
     const int shared = shared_keys ? shared_keys[row] : 0;
-    // the wave's i-th tile is the segment's (wave + W i)-th; lane l holds the page and the place of the (i0 + l)-th
+    // the wave's i-th tile is the segment's (wave + W i)-th; lane l holds the page and the place of the l-th (a segment has at most 2048 keys)
     const int first = k_begin / 16 + wave, tiles = k_begin < k_end ? max(0, ((k_end + 15) / 16 - first + W - 1) / W) : 0;
-    int my_page = 0, my_place = 0;
-    const auto look_up = [&](int i0) {
-        const int key = (first + (i0 + lane) * W) * 16;
-        if (i0 + lane < tiles) my_page = bt[key / P];
-        my_place = key % P;
-    };
-    look_up(0);
+    const int my_key = (first + lane * W) * 16, my_place = my_key % P;
+    const int my_page = lane < tiles ? bt[my_key / P] : 0;
     bf16x8 qreg[D / 32];
     const long width = FUSED ? (long)(Hq + 2 * Hkv) * D : (long)Hq * D;
     const float* cs = FUSED && table ? table + (long)p * D : nullptr;
@@ -630,18 +625,15 @@ __global__ __launch_bounds__(64 * W, W == 4 ? (FUSED ? 2 : 3) : 1) void attentio
     AttnState<D> st;
     st.init();
     KVTile<D> ta, tb;
-#define LOAD(buf_, i_) load_tile<D>(buf_, cache, __builtin_amdgcn_readlane(my_page, (i_) & 63), page_stride, kvh, Hkv, P, \
-                                    __builtin_amdgcn_readlane(my_place, (i_) & 63), g, n, (first + (i_) * W) * 16 >= shared)
+#define LOAD(buf_, i_) load_tile<D>(buf_, cache, __builtin_amdgcn_readlane(my_page, i_), page_stride, kvh, Hkv, P, \
+                                    __builtin_amdgcn_readlane(my_place, i_), g, n, (first + (i_) * W) * 16 >= shared)
 #define STEP(buf_, i_) attn_tile_step<D>(st, buf_, qreg, scale, (first + (i_) * W) * 16, g, k_begin, k_end, k_begin, k_end)
     if (tiles > 0) LOAD(ta, 0);
     if (tiles > 1) LOAD(tb, 1);
     if constexpr (FUSED) nq.finish(qreg, q_w != nullptr, eps, cs != nullptr);
     for (int i = 0; i < tiles;) {
         STEP(ta, i);
-        if (i + 2 < tiles) {
-            if ((i + 2) % 64 == 0) look_up(i + 2);         // (the tile after the next begins 64 others; the next one's loads are on their way)
-            LOAD(ta, i + 2);
-        }
+        if (i + 2 < tiles) LOAD(ta, i + 2);
         if (++i >= tiles) break;
         STEP(tb, i);
         if (i + 2 < tiles) LOAD(tb, i + 2);
@@ -794,39 +786,31 @@ size_t qe_attention_decode_workspace(int n_dec, int Hq, int D, int num_splits) {
     return (size_t)n_dec * Hq * num_splits * (D + 2) * sizeof(float);
 }
 
-// The segments of a block's form: 0 (the splits are the better way), else how many, of seg_keys keys each.  (us, 16 heads of 128 on 8, rows of half to
-// one and a half times the keys; splits of 128 and their merge, then blocks of four waves.  In one segment: 16 rows of 200 keys 18.2, 12.4, of 400
-// 18.3, 16.0; 24 of 400 20.7, 15.2; 64 of 200 37.4, 14.9, of 400 42.4, 26.2, of 1030 75.1, 57.4, of 2000 115, 107; of 1030 with 64 heads
-// 83.7, 60.1.  Cut: 9 rows of 1900 22.8, 22.8 (7 segments), of 3800 40.6, 38.6; 16 of 1040 25.2, 21.5 (4; in one 27.5), of 4000 63.6, 57.7; 24 of
-// 4000 87.2, 79.7 (5; in one 93.7); 32 of 4000 113, 106 (2; in one 112).  Four rows of 400 13.0, 13.4, of 1000 14.3, 16.0, of 2000 16.2, 16.4: up to eight
-// tokens are the splits'.)  Up to 16 tokens, which every other kernel of their step takes in one order, a token's segments follow its own position
-// alone: its bits are the same beside any others.  With more they follow how many those are, and the last position as recorded steps know it, the end
-// of a stretch of 1024 (the first two, of 512): a step has the same ones whether it is recorded or runs as it comes.
+// The segments of a block's form: 0 (the splits are the better way), else how many, of seg_keys keys each.  (us, norm, rotation and cache write inside, 16 heads of 128
+// on 8 if nothing else is said, rows of half to one and a half times the keys; splits of 128 and their merge, then blocks of four waves.)
+// Up to eight tokens are the splits': four of 400 keys 13.0, 13.4, of 1000 14.3, 16.0, of 2000 16.2, 16.4.
+// Up to 16 tokens, which every other kernel of their step takes in one order, the way is the model's and a token's segments follow its own position
+// alone: its bits are the same beside any others.  With four key/value heads or fewer the blocks are too few: 9 tokens of one of 100 keys 10.4, 8.4, of 300 10.2, 11.4, of
+// 640 10.6, 14.6, of 3000 13.5, 14.5; 12 of four of 200 10.8, 10.2, of 640 13.4, 14.8, of 1900 18.8, 21.2, of 6000 36.4, 36.2.  With more: 9 of 60 12.3, 6.7, of 300 13.5, 10.9, of 680 13.4, 15.3, of
+// 1000 17.6, 20.4, of 3000 26.8, 25.7; 16 of 60 14.1, 6.8, of 300 15.7, 11.1, of 680 15.8, 16.0, of 1000 21.4, 21.5, of 3000 38.8, 37.5, of 6000 85.5, 82.0 (tokens at 512 to 1535 in segments of 384:
+// 9 of 1000 19.2, but 16 of 680 18.6).
+// More tokens: one segment up to 1024 positions, and up to 2048 for more than 128 blocks, but where the splits are few enough to run four waves each; else segments of 512.  The
+// last position counts as recorded steps know it, as the end of a stretch of 1024 (the first two, of 512): a step has the same segments whether it is recorded or runs as it comes.
+// (Splits, 512 keys and one segment: 20 tokens of one key/value head of 640 keys 10.6, 14.5, 16.8, 64 of 1000 16.1, 17.8, 23.6; 64 of two of 1000 22.9, 22.6, 24.5; 20 of eight of 1000 27.3, 28.5,
+// 23.8, of 3000 47.9, 49.7, 55.3; 32 of 3000 86.7, 81.8, 84.3; 64 of 1000 64.0, 67.1, 46.7, of 1900 109.7, 103.9, 99.3; 48 of four of 3000 69.5, 61.2, 68.2.  Cut into as many as fill the units three
+// times: 20 of 3000 63.4, 32 96.5.)
 static int last_of_stretch(int position) { return position < 512 ? 511 : position | 1023; }
 static int block_segments(int n_dec, int Hkv, int max_position, int window, int sink, float softcap, int& seg_keys) {
     if (n_dec <= 8 || window != 0 || sink || softcap > 0.f) return 0;
-    int segments = max_position / 512 + 1;
-    seg_keys = 512;
-    if (n_dec > 16) {
-        const long blocks = (long)Hkv * n_dec;
-        const int last = last_of_stretch(max_position);
-        const int want = last < 1536 ? 1 : (int)min(768 / blocks, last / 512 + 1L);
-        seg_keys = qe_cdiv(qe_cdiv(last + 1, max(1, want)), 16) * 16;
-        segments = max_position / seg_keys + 1;
+    if (n_dec <= 16) {
+        seg_keys = 512;
+        return Hkv <= 4 ? 0 : max_position / seg_keys + 1;
     }
-    return segments;
-}
-
-// 1 if n single tokens without a window are best given norm, rotation and cache write inside the attention kernel: up to 16, and up to 64 but where their segments
-// are about three blocks a unit, which is how many of the other form's share one; of the fused form's two do, and the third is a turn by itself.  (The two kernels' time and the
-// one's, 16 heads of 128 on 8: 24 tokens of 600 keys 24.4, 19.8 us, 32 27.1, 23.1, 64 41.2, 38.8; of 1000 to 4000 keys, in the mean of one to three times the keys: 17 and 28 tokens
-// 0.86 to 0.95, 32 0.92 to 1.00, 36 0.85 to 0.93, 40 0.95 to 1.01, 52 to 64 0.95 to 0.97; in four segments 20 tokens 0.95 to 1.05, 24 1.01 to 1.04; in two 44 1.01 to 1.04, 48 1.02 to 1.06.)
-extern "C" int qe_attention_decode_fused_preferred(int n, int Hkv, int max_position) {
-    if (n <= 16 || n > 64) return n <= 16;
-    int seg_keys;
-    const int segments = block_segments(n, Hkv, last_of_stretch(max_position), 0, 0, 0.f, seg_keys);
-    const long blocks = (long)segments * Hkv * n;
-    return !((segments == 4 && blocks >= 640) || (segments == 2 && blocks > 640));
+    const long blocks = (long)Hkv * n_dec;
+    const int last = last_of_stretch(max_position);
+    if (last >= 512 && (last / 128 + 1) * blocks <= 544) return 0;
+    seg_keys = last < 1024 || (last < 2048 && blocks > 128) ? last + 1 : 512;
+    return max_position / seg_keys + 1;
 }
 
 template <int D, bool FUSED>
@@ -834,7 +818,7 @@ static void launch_block(const bf16_t* q, bf16_t* cache, const int* dec_tokens, 
                          const int* block_table, int max_blocks, const int* shared_keys, const int* slots, const float* q_w, const float* k_w,
                          float eps, const float* table, bf16_t* out, float* part, int Hq, int Hkv, int P, float scale, int window, int segments,
                          int seg_keys, hipStream_t stream, const AttnTail& tail) {
-    constexpr int W = 4;
+    constexpr int W = 4;                                   // (2048 keys a segment at the most: a wave's 32 tiles)
     float* part_ml = part + (size_t)n_dec * Hq * segments * D;
     attention_decode_block_kernel<D, W, FUSED><<<dim3(segments, Hkv, n_dec), 64 * W, (size_t)W * (Hq / Hkv) * (D + 6) * sizeof(float), stream>>>(
         q, cache, dec_tokens, positions, tok_seq, block_table, max_blocks, shared_keys, slots, q_w, k_w, eps, table, out, part, part_ml,

@@ -77,7 +77,6 @@ def load_library():
         "qe_attention_prefill_workspace_bytes": [i32, i32, i32, i32, i32, i32],
         "qe_attention_decode_run": [vp, vp, vp, vp, i32, vp, vp, vp, i32, vp, i32, i32, i32, i32, f32, i32, i32, i32, f32, i32, i32, vp, i64,
                                     i64, i32, vp, vp, i64, i32, vp],
-        "qe_attention_decode_fused_preferred": [i32, i32, i32],
         "qe_attention_decode_fused_run": [vp, vp, vp, vp, i32, vp, vp, vp, i32, vp, vp, vp, vp, f32, vp,
                                           i32, i32, i32, i32, f32, i32, i32, i32, vp, i64, vp],
         "qe_qk_rope_store": [vp, vp, vp, vp, f32, vp, i32, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, vp],
@@ -1033,12 +1032,12 @@ def attention_decode_fused_supported(qkv: torch.Tensor, cache: torch.Tensor, num
             bool(lib.qe_attention_decode_supported(num_heads, cache.shape[2], D, cache.shape[3], _DT[qkv.dtype])))
 
 
-def attention_decode_fused_preferred(qkv: torch.Tensor, num_kv_heads: int, max_dec_position: int) -> bool:
+def attention_decode_fused_preferred(qkv: torch.Tensor) -> bool:
     """True if the rows of qkv, all single new tokens without a window, are best given to attention_decode_fused (with dec_blocks) where it takes
     them, rather than to qk_rope_store and attention."""
-    if qkv.dtype == torch.float32:
-        return qkv.shape[0] <= 64
-    return bool(load_library().qe_attention_decode_fused_preferred(qkv.shape[0], int(num_kv_heads), int(max_dec_position)))
+    # (us, bfloat16, 16 heads of 128 on 8, the two kernels and the one: 20 tokens of 640 keys 25.3, 21.8, of 1000 27.5, 23.8, of 1900 35.0, 36.8, of 6000 99.8, 95.1; 32 of
+    # 1000 30.7, 28.3, of 1900 49.5, 51.9; 64 of 1000 50.1, 46.7, of 1900 102.6, 103.9; four tokens of 2 key/value heads more, 24 of 3000, 24.4, 22.5)
+    return qkv.shape[0] <= 64
 
 
 def attention_decode_fused(qkv: torch.Tensor, num_heads: int, cache: torch.Tensor, positions: torch.Tensor,

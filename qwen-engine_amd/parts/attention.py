@@ -270,7 +270,7 @@ class PagedAttention:
                                (ex["other_tokens"] is None or ex["other_tokens"].shape[0] == 0))
             if (only_new_tokens and binding.write and
                     (T <= FUSED_DECODE_MAX_TOKENS if self.window else
-                     ops.attention_decode_fused_preferred(qkv, self.hkv, ex["max_dec_position"])) and
+                     ops.attention_decode_fused_preferred(qkv)) and
                     not is_replaced(self, _ATTEND) and ops.attention_decode_fused_supported(qkv, cache, self.hq, table)):
                 # every row is the one new token of its request: norm, rotation and cache write
                 # happen inside the attention kernel (an _attend that has been replaced gets q)
