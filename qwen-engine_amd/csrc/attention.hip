@@ -64,11 +64,14 @@ extern "C" int qe_attention_prefill_tiles_run(const int* portions, int n_portion
 // and in one: one token of 400 keys 25.2, 16.7, of 1000 25.9, 22.4, of 2000 26.0, 35.8; 15 of 400 28, 17.6, of 1000 35, 25.4, of 2000 48, 39.5; 64 of 400
 // 40, 34.8, of 1000 71, 61.9.  A portion of 64 rows: one of 1000 20.0, 22.1, eight 24.1, 23.1.  200 rows: one of 870 20.8, 14.6; tokens of 160 to 480 or 330 to
 // 990 keys: 96 42.7, 36.5 and 66.7, 59.9, 128 52.9, 42.7 and 87.5, 73.0, 256 81.9, 73.5 and 144, 129.)  Not where the walks are cut into segments: more
-// blocks would leave fewer of those.  The lines are where a recorded step, which has its portion filled up to 128 rows and the positions to 512 or 1024,
+// blocks would leave fewer of those.  Between 512 and 1024 positions and beside few rows, which are done long before, it is the walk of one block that decides, and splits of a few
+// tokens and heads are quicker: beside 64 rows 8 tokens of 320 to 960 keys of one key/value head 18.4, 22.1, of four 18.8, 22.3, of eight 21.3, 21.8, 15 of one 18.9, 22.2, of four 21.8,
+// 22.5, of eight 25.7, 23.4, 33 of two of 64 17.3, 18.2, of four 29.7, 24.3.  The lines are where a recorded step, which has its portion filled up to 128 rows, its single tokens to eights and the positions to 512 or 1024,
 // falls on the same side as the step as it comes.
-extern "C" int qe_attention_prefill_takes_single(int n_dec, int max_position, int rows, int max_keys) {
-    if (n_dec <= 0 || rows <= 0 || max_keys > qe_attention_prefill_uncut_keys()) return 0;
-    return max_position < 512 || (max_position < 1024 && (rows > 128 || n_dec >= 8));
+extern "C" int qe_attention_prefill_takes_single(int n_dec, int max_position, int rows, int max_keys, int Hkv) {
+    if (n_dec <= 0 || rows <= 0 || Hkv <= 0 || max_keys > qe_attention_prefill_uncut_keys()) return 0;
+    const long filled = n_dec <= 8 ? n_dec : (n_dec + 7) / 8 * 8;      // (a recorded step's single tokens)
+    return max_position < 512 || (max_position < 1024 && (rows > 128 || filled * Hkv >= 100));
 }
 
 // rows of a tile for these head counts

@@ -69,7 +69,7 @@ def load_library():
         "qe_attention_f32_fused_run": [vp, vp, vp, vp, i32, i32, vp, vp, vp, i32, vp, vp, vp, f32, vp, i32, i32, i32, i32, f32, i32, vp],
         "qe_attention_prefill_plan_segments": [i32, i32, i32],
         "qe_attention_prefill_tiles_run": [vp, i32, i32, vp, i32, i32, vp],
-        "qe_attention_prefill_takes_single": [i32, i32, i32, i32],
+        "qe_attention_prefill_takes_single": [i32, i32, i32, i32, i32],
         "qe_attention_prefill_workspace_bytes_for": [i32, i32, i32, i32, i32],
         "qe_attention_prefill_plan": [i32, i32, i32, i32],
         "qe_attention_prefill_plan_uncut_keys": [],
@@ -822,10 +822,10 @@ def prefill_tile_rows(num_heads: int, num_kv_heads: int) -> int:
     return load_library().qe_attention_prefill_rows(num_heads, num_kv_heads)
 
 
-def prefill_takes_single(n_dec: int, max_position: int, rows: int, max_keys: int) -> bool:
+def prefill_takes_single(n_dec: int, max_position: int, rows: int, max_keys: int, num_kv_heads: int = 8) -> bool:
     """True if ``n_dec`` single new tokens at positions up to ``max_position`` are best computed by the prefill attention kernel, together
     with ``rows`` rows of portions that see at most ``max_keys`` keys."""
-    return bool(load_library().qe_attention_prefill_takes_single(int(n_dec), int(max_position), int(rows), int(max_keys)))
+    return bool(load_library().qe_attention_prefill_takes_single(int(n_dec), int(max_position), int(rows), int(max_keys), int(num_kv_heads)))
 
 
 def prefill_tiles_on_device(portions: torch.Tensor, rows_per_tile: int, max_groups: int, singles: int = 0) -> torch.Tensor:

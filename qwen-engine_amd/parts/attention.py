@@ -129,7 +129,7 @@ class PagedAttention:
         if dec is None or other is None or not dec.shape[0] or not other.shape[0] or not ops.attention_prefill_supported(q, cache):
             return None
         max_keys = ops.prefill_uncut_keys() + 1 if ex.get("other_keys_row") is not None else ex.get("max_other_keys", 0)
-        if not ops.prefill_takes_single(dec.shape[0], ex["max_dec_position"], other.shape[0], max_keys):
+        if not ops.prefill_takes_single(dec.shape[0], ex["max_dec_position"], other.shape[0], max_keys, self.hkv):
             return None
         rows_per_tile = ops.prefill_tile_rows(self.hq, self.hkv)
         key = ("paged_attention.all_tiles", rows_per_tile)

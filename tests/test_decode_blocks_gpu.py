@@ -177,13 +177,23 @@ def test_recorded_steps_choose_as_steps_that_run_as_they_come(ops):
     from qwen_engine_amd.engine import ModelRunner
     from qwen_engine_amd.parts.attention import PagedAttention
     step = ModelRunner.MIXED_GRAPH_STEP
-    for n in (1, 2, 7, 8, 9, 15, 33, 70):
+    for n in (1, 2, 7, 8, 9, 15, 33, 50, 70, 97, 101):
         for last in (0, 300, 511, 512, 700, 1023, 1024, 1500):
             end = PagedAttention.graph_key(last) * ops.DECODE_SPLIT_KEYS - 1
             for rows in (2, 100, 127, 128, 129, 200, 255, 256, 257, 500):
                 for keys in (rows, 1024, 1025, 3000):
-                    comes = ops.prefill_takes_single(n, last, rows, keys)
-                    assert comes == ops.prefill_takes_single(ModelRunner.graph_rows(n), end, -(-rows // step) * step, keys), (n, last, rows, keys)
+                    for heads in (1, 2, 4, 8, 16):
+                        comes = ops.prefill_takes_single(n, last, rows, keys, heads)
+                        then = ops.prefill_takes_single(ModelRunner.graph_rows(n), end, -(-rows // step) * step, keys, heads)
+                        assert comes == then, (n, last, rows, keys, heads)
+
+
+def test_few_walks_beside_few_rows_go_apart(ops):
+    """Beyond 512 positions one block's walk decides, which was up to a fifth slower than splits and the portion by itself."""
+    for n, heads in ((8, 1), (8, 4), (8, 8), (15, 1), (15, 4), (33, 2)):
+        assert not ops.prefill_takes_single(n, 960, 64, 64, heads) and ops.prefill_takes_single(n, 960, 400, 400, heads)
+        assert ops.prefill_takes_single(n, 500, 64, 64, heads)
+    assert ops.prefill_takes_single(15, 960, 64, 64, 8) and ops.prefill_takes_single(33, 960, 64, 64, 4) and not ops.prefill_takes_single(15, 1024, 64, 64, 8)
 
 
 def test_where_the_step_before_goes_inside(ops):
