@@ -537,14 +537,14 @@ static bool by_lines(int M, int N, int K) {
 // the residual sum and the norm in front.  K in whole steps of 16.
 extern int g_qe_matrix_f32;      // (switched off: the vector units' kernels do it all, one by one)
 bool qe_gemm_f32_silu_ok(int M, int N, int K) { return g_qe_matrix_f32 && M <= 16 && N % 64 == 0 && K % FK == 0 && !by_lines(M, N, K); }
-// Whether silu * up is best done in the product's launch.  That form has 32 rows of w a block and asks for half as much at once: up to 128 blocks leave
+// Whether silu * up is best done in the product's launch (-1: it cannot be).  That form has 32 rows of w a block and asks for half as much at once: up to 128 blocks leave
 // the units idle that four, eight or sixteen rows a block give work, beyond 256 their second turn is thin, but where the product by itself would have the same
 // blocks.  (us, product and silu * up, then in one; two rows: 4096 x 512 6.5, 6.1, x 1536 10.9, 11.2, x 2048 10.9, 13.7, x 4096 18.8, 27.7; 2048 x 4096 12.3, 21.8;
 // 4608 x 2048 15.4, 16.2, 6144 x 1024 9.7, 9.9, x 1536 17.5, 13.8, x 4096 28.6, 31.3 (behind the norm 35.3, 39.3), 8192 x 1024 11.3, 11.1, x 3072 25.2, 26.1; 9216 x 1024 12.1, 17.8; 24576 x 256 8.7,
 // 8.2, x 512 12.5, 14.7, x 1536 43.7, 37.2, x 4096 77.7, 127; eight rows: 12288 x 2560 45.4, 43.4, 24576 x 2048 48.4, 57.7, x 4096 138, 127.  A launch less is some
 // 12 us of the host's for a step that is not recorded.)
 extern "C" int qe_gemm_f32_silu_inside(int M, int N, int K) {
-    if (!qe_gemm_f32_silu_ok(M, N, K)) return 0;
+    if (!qe_gemm_f32_silu_ok(M, N, K)) return -1;
     if (N <= 4096) return K <= 1536;
     if (N <= 8192) return M > 4 || K <= 3072;
     const bool chunks = K % chunk_len(K) == 0 && chunk_len(K) % 64 == 0 && chunk_len(K) <= 128;

@@ -569,8 +569,8 @@ def gemm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor] = None,
         raise KernelError("gemm: 32-bit activations need 32-bit weights")
     if bias is not None:
         _need(bias, "bias", torch.float32, (w.shape[0],), x.device)
-    if (epilogue == EPI_SILU_MUL_IL and x.dtype == w.dtype == (out_dtype or x.dtype) == torch.float32 and gemm_silu_supported(x, w) and
-            not lib.qe_gemm_f32_silu_inside(M, w.shape[0], K)):        # (quicker by itself; the same bits)
+    if (epilogue == EPI_SILU_MUL_IL and x.dtype == w.dtype == (out_dtype or x.dtype) == torch.float32 and
+            lib.qe_gemm_f32_silu_inside(M, w.shape[0], K) == 0):       # (quicker by itself; the same bits)
         return silu_mul(gemm(x, w, bias, algo=algo, norm_weight=norm_weight, norm_eps=norm_eps, delta=delta, stream_out=stream_out), out, interleaved=True)
     if epilogue == EPI_RESIDUAL:
         if out is None:

@@ -119,7 +119,8 @@ class Runtime:
 def is_replaced(part, written) -> bool:
     """True if a program, or a class derived from the part's, has put something else in the place of the method ``written`` (a trace, a
     change of its own): what would pass it by calls it then."""
-    return written.__name__ in vars(part) or getattr(type(part), written.__name__) is not written
+    name = written.__name__
+    return name in part.__dict__ or getattr(part.__class__, name) is not written
 
 
 class Stream:

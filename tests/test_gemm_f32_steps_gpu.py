@@ -128,9 +128,10 @@ def test_silu_in_the_products_launch(ops):
     """Only where that is not slower: two rows against 24576 x 4096 took 127 us in it, 78 apart."""
     inside = ops.load_library().qe_gemm_f32_silu_inside
     for taken in ((2, 6144, 1024), (16, 1024, 512), (2, 24576, 256), (2, 24576, 1536), (8, 24576, 4096), (8, 8192, 4096)):
-        assert inside(*taken), taken
-    for apart in ((2, 24576, 4096), (2, 2048, 4096), (16, 512, 2048), (8, 24576, 2048), (1, 12288, 1024), (2, 24576, 1024), (2, 6144, 4096), (17, 6144, 1024)):
-        assert not inside(*apart), apart
+        assert inside(*taken) == 1, taken
+    for apart in ((2, 24576, 4096), (2, 2048, 4096), (16, 512, 2048), (8, 24576, 2048), (1, 12288, 1024), (2, 6144, 4096)):
+        assert inside(*apart) == 0, apart
+    assert inside(17, 6144, 1024) == inside(2, 6144, 1000) == inside(2, 24576, 1024) == -1
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 2000, 1024), (16, 1376, 256), (3, 34, 496)])
